@@ -12,7 +12,9 @@ Before the W warm-up steps the same step runs untimed for ``--settle-seconds``
 (default 0.3 s) so that the shader clock has left its idle state; the timed
 region is exactly K steps between two synchronisations (``ms_per_step``,
 ``value``).  After it, forward, backward, the step and the step through autograd
-(``LinearAttention.apply`` + ``torch.autograd.grad``) are each timed once more
+(``LinearAttention.apply`` + ``torch.autograd.grad``; that operator chooses its
+evaluation by shape, chunk-wise at the larger workloads, where ``value`` is the
+quadratic kernels whatever the shape) are each timed once more
 with one HIP event pair per iteration; ``config.median_ms`` holds the medians.
 
 Prints ONE JSON line.  ``value`` is causal-counted algorithmic TFLOP/s of the
@@ -326,7 +328,7 @@ def _other_extension(torch, name, algo, dev, steps):
         linear_attention_normalised_fwd(q, k, v, 1e-5, chunked, want_state=chunked)
         linear_attention_normalised_bwd(do, q, k, v, out, denom, chunked, state)
 
-    def recipe_step():  # README.md:27-30 of the reference around the quadratic operator, through autograd
+    def recipe_step():  # README.md:27-30 of the reference around the product operator (evaluation by shape), through autograd
         qr, kr, vr = (t.detach().requires_grad_(True) for t in (q, k, v))
         num = (LinearAttentionSmallVHD if w.small_v else LinearAttention).apply(qr, kr, vr)
         (num / ((qr * kr.cumsum(-2)).sum(dim=-1, keepdim=True) + 1e-5)).backward(do)

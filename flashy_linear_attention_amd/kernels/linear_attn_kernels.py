@@ -23,14 +23,20 @@ def _block_sq(hd: int) -> int:
     return 64 if next_power_of_2(hd) <= 128 else 32
 
 
-def linear_flash_wrapper_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-    """O = tril(Q K^T) V for (batch, heads, seq, head_dim) tensors."""
+def check_operands(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
+    """The reference's assertions on a forward call (linear_attn_kernels.py:322-325)."""
     batch, nh, sq, hd = q.shape
     BLOCK_SQ = _block_sq(hd)
 
     assert hd <= 256, "Only head_dims <= 256 are supported."
     assert sq % BLOCK_SQ == 0, f"Number of elements in sequence must be a multiple of {BLOCK_SQ}, {sq, BLOCK_SQ}"
     assert k.shape == q.shape and v.shape == q.shape, "q, k and v must have the same shape"
+
+
+def linear_flash_wrapper_fwd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+    """O = tril(Q K^T) V for (batch, heads, seq, head_dim) tensors."""
+    batch, nh, sq, hd = q.shape
+    check_operands(q, k, v)
 
     q, k, v = prepare(q, k, v)
     out = torch.empty_like(q, memory_format=torch.contiguous_format)

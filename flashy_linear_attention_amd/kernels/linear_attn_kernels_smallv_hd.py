@@ -16,8 +16,8 @@ from .. import _lib
 from ._common import call, device_guard, dtype_code, next_power_of_2, prepare, stream_handle
 
 
-def linear_flash_wrapper_fwd_smallv_hd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-    """O = tril(Q K^T) V with q, k of width hd_qk and v, O of width hd_v."""
+def check_operands(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> None:
+    """The reference's assertions on a forward call (linear_attn_kernels_smallv_hd.py:320)."""
     batch, nh, sq, hd_qk = q.shape
     batch, nh, sq, hd_v = v.shape
 
@@ -30,6 +30,13 @@ def linear_flash_wrapper_fwd_smallv_hd(q: torch.Tensor, k: torch.Tensor, v: torc
     assert hd_qk <= 256, "Only head_dims <= 256 are supported."
     assert sq % BLOCK_SQ == 0, f"Number of elements in sequence must be a multiple of {BLOCK_SQ}, {sq, BLOCK_SQ}"
     assert k.shape == q.shape and v.shape[:3] == q.shape[:3], "q, k, v must agree in batch, heads and sequence"
+
+
+def linear_flash_wrapper_fwd_smallv_hd(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
+    """O = tril(Q K^T) V with q, k of width hd_qk and v, O of width hd_v."""
+    check_operands(q, k, v)
+    batch, nh, sq, hd_qk = q.shape
+    hd_v = v.shape[3]
 
     q, k, v = prepare(q, k, v)
     out = torch.empty_like(v, memory_format=torch.contiguous_format)

@@ -10,20 +10,22 @@ from typing import Any, Tuple
 import torch
 from torch.autograd import Function
 
-from .kernels import linear_flash_wrapper_bwd_smallv_hd, linear_flash_wrapper_fwd_smallv_hd
+from .auto import evaluate_bwd, evaluate_fwd, prefers_chunked
+from .kernels.linear_attn_kernels_smallv_hd import check_operands
 
 
 class LinearAttentionSmallVHD(Function):
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
-        out = linear_flash_wrapper_fwd_smallv_hd(q, k, v)
-        ctx.save_for_backward(q, k, v)
-        return out
+        check_operands(q, k, v)
+        # (bf16 and D_v up to 128 only: see LinearAttention.  The quadratic backward wants
+        # N a multiple of 64 where forward takes 32, so such a sequence stays with it)
+        chunked = (q.dtype == torch.bfloat16 and q.shape[2] % 64 == 0 and v.shape[-1] <= 128
+                   and prefers_chunked(q, v))
+        return evaluate_fwd(ctx, q, k, v, chunked, False)
 
     @staticmethod
     @torch.amp.custom_bwd(device_type="cuda")
     def backward(ctx: Any, grad_output: torch.Tensor) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-        query, key, value = ctx.saved_tensors
-        gradq, gradk, gradv = linear_flash_wrapper_bwd_smallv_hd(grad_output, query, key, value)
-        return gradq, gradk, gradv
+        return evaluate_bwd(ctx, grad_output)
