@@ -16,7 +16,7 @@ from typing import Any, Tuple
 import torch
 from torch.autograd import Function
 
-from . import _lib
+from . import _lib, _native
 from .chunked import linear_attention_chunked_bwd, linear_attention_chunked_fwd
 from .kernels import (
     linear_flash_wrapper_bwd,
@@ -61,6 +61,14 @@ def evaluate_bwd(ctx: Any, grad_output: torch.Tensor) -> Tuple[torch.Tensor, tor
 
 
 class LinearAttentionAuto(Function):
+    @classmethod
+    def apply(cls, *args):
+        if cls is LinearAttentionAuto and len(args) == 3:
+            out = _native.product(2, *args)
+            if out is not None:
+                return out
+        return super().apply(*args)
+
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:

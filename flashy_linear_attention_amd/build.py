@@ -2,7 +2,8 @@
 
 Run as ``python -m flashy_linear_attention_amd.build``.  hipcc cross-compiles
 without a GPU.  One object per (dtype, DC, DO) kernel instantiation, compiled in
-parallel, then linked with the C ABI into the package directory.
+parallel, then linked with the C ABI into the package directory; ``_fla_torch.so`` beside it
+is the operators' host path against PyTorch (no kernels in it).
 """
 
 from __future__ import annotations
@@ -12,6 +13,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from typing import List
 
 PKG_DIR = os.path.dirname(os.path.abspath(__file__))
@@ -21,6 +23,7 @@ INCLUDE = os.path.join(REPO_ROOT, "include")
 OBJ_DIR = os.path.join(PKG_DIR, "csrc", "_obj")
 LIB_NAME = "libfla_gfx950.so"
 LIB_PATH = os.path.join(PKG_DIR, LIB_NAME)
+BINDING_PATH = os.path.join(PKG_DIR, "_fla_torch.so")
 
 DIMS = (32, 64, 128, 256)
 HIPCC_FLAGS = [
@@ -81,29 +84,63 @@ def _compile_inst(args) -> str:
     return obj
 
 
+def _compile_walk(args) -> str:
+    dtype, part = args
+    obj = os.path.join(OBJ_DIR, f"walk_t{dtype}_p{part}.o")
+    report = _run([_hipcc(), *HIPCC_FLAGS, "-Rpass-analysis=kernel-resource-usage", f"-DFLA_WALK_DTYPE={dtype}",
+                   f"-DFLA_WALK_PART={part}", "-c", os.path.join(CSRC, "fla_walk_inst.hip"), "-o", obj])
+    if part == 1:
+        _check_no_scratch(report, "walk_bwd_rev_kernel")
+        _check_no_scratch(report, "walk_bwd_rev_wide_kernel")
+    return obj
+
+
+def _compile_other(name: str) -> str:
+    obj = os.path.join(OBJ_DIR, f"{name}.o")
+    # (the pair kernels without the VGPR form of MFMA: see that file's header)
+    flags = [f for f in HIPCC_FLAGS if name != "fla_pair_inst" or f not in ("-mllvm", "-amdgpu-mfma-vgpr-form")]
+    _run([_hipcc(), *flags, "-c", os.path.join(CSRC, f"{name}.hip"), "-o", obj])
+    return obj
+
+
+def _compile_torch(_=None) -> str:
+    """The operators' host path against this PyTorch (host code only)."""
+    import torch
+    from torch.utils.cpp_extension import include_paths
+
+    obj = os.path.join(OBJ_DIR, "fla_torch.o")
+    _run(["g++", "-O2", "-std=c++17", "-fPIC", "-fvisibility=hidden", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+          f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I" + INCLUDE,
+          *(flag for path in include_paths() for flag in ("-isystem", path)), "-isystem", "/opt/rocm/include",
+          "-isystem", sysconfig.get_paths()["include"], "-c", os.path.join(CSRC, "fla_torch.cc"), "-o", obj])
+    return obj
+
+
 def build(jobs: int | None = None, verbose: bool = True) -> str:
-    """Compile every kernel instantiation and link the shared library.  Always recompiles."""
+    """Compile every kernel instantiation and link the shared library, and the extension module that binds it
+    to PyTorch.  Always recompiles."""
+    import torch
+
     os.makedirs(OBJ_DIR, exist_ok=True)
     jobs = jobs or min(8, os.cpu_count() or 1)
-    work = [(t, dc, do) for t in (0, 1) for dc in DIMS for do in DIMS]
+    # (the slowest first)
+    work = [(_compile_walk, (t, part)) for part in (1, 0) for t in (0, 1)]
+    work += [(_compile_torch, None), (_compile_other, "fla_capi"), (_compile_other, "fla_pair_inst")]
+    work += [(_compile_inst, (t, dc, do)) for dc in DIMS for do in DIMS for t in (0, 1)]
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
-        objs = list(pool.map(_compile_inst, work))
-    capi = os.path.join(OBJ_DIR, "fla_capi.o")
-    _run([_hipcc(), *HIPCC_FLAGS, "-c", os.path.join(CSRC, "fla_capi.hip"), "-o", capi])
-    walk = os.path.join(OBJ_DIR, "fla_walk_inst.o")
-    report = _run([_hipcc(), *HIPCC_FLAGS, "-Rpass-analysis=kernel-resource-usage", "-c",
-                   os.path.join(CSRC, "fla_walk_inst.hip"), "-o", walk])
-    _check_no_scratch(report, "walk_bwd_rev_kernel")
-    _check_no_scratch(report, "walk_bwd_rev_wide_kernel")
-    # (this one without the VGPR form of MFMA: see the file's header)
-    pair = os.path.join(OBJ_DIR, "fla_pair_inst.o")
-    pair_flags = [f for f in HIPCC_FLAGS if f not in ("-mllvm", "-amdgpu-mfma-vgpr-form")]
-    _run([_hipcc(), *pair_flags, "-c", os.path.join(CSRC, "fla_pair_inst.hip"), "-o", pair])
+        objs = list(pool.map(lambda w: w[0](w[1]), work))
+    binding = next(o for o in objs if o.endswith("fla_torch.o"))
+    objs.remove(binding)
     tmp = LIB_PATH + ".tmp"
-    _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-o", tmp, capi, walk, pair, *objs])
+    _run([_hipcc(), "--offload-arch=gfx950", "-shared", "-fPIC", "-Wl,-soname," + LIB_NAME, "-o", tmp, *objs])
     os.replace(tmp, LIB_PATH)
+    torch_lib = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = BINDING_PATH + ".tmp"
+    _run(["g++", "-shared", "-o", tmp, binding, LIB_PATH, "-L" + torch_lib, "-lc10", "-lc10_hip", "-ltorch", "-ltorch_cpu",
+          "-ltorch_python", "-Wl,-rpath,$ORIGIN"])
+    os.replace(tmp, BINDING_PATH)
     if verbose:
-        print(f"built {LIB_PATH} ({os.path.getsize(LIB_PATH) / 1e6:.1f} MB, {len(objs)} kernel objects)")
+        print(f"built {LIB_PATH} ({os.path.getsize(LIB_PATH) / 1e6:.1f} MB, {len(objs)} objects) and {BINDING_PATH}")
     return LIB_PATH
 
 
@@ -128,8 +165,9 @@ def build_trace(jobs: int | None = None) -> str:
     work = [("fla_inst.hip", f"inst_t{t}_c{dc}_o{do}.o",
              [f"-DFLA_INST_DTYPE={t}", f"-DFLA_INST_DC={dc}", f"-DFLA_INST_DO={do}"])
             for t in (0, 1) for dc in DIMS for do in DIMS]
-    work += [("fla_capi.hip", "fla_capi.o", []), ("fla_walk_inst.hip", "fla_walk_inst.o", []),
-             ("fla_pair_inst.hip", "fla_pair_inst.o", []),
+    work += [("fla_walk_inst.hip", f"walk_t{t}_p{part}.o", [f"-DFLA_WALK_DTYPE={t}", f"-DFLA_WALK_PART={part}"])
+             for t in (0, 1) for part in (0, 1)]
+    work += [("fla_capi.hip", "fla_capi.o", []), ("fla_pair_inst.hip", "fla_pair_inst.o", []),
              ("fla_trace.cc", "fla_trace.o", ["-x", "c++"])]
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
         objs = list(pool.map(one, work))

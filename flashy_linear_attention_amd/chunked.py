@@ -16,7 +16,7 @@ from typing import Any, Tuple
 import torch
 from torch.autograd import Function
 
-from . import _lib
+from . import _lib, _native
 from .kernels._common import device_guard, dtype_code, prepare, stream_handle
 
 
@@ -106,6 +106,14 @@ def linear_attention_chunked_bwd(
 
 
 class LinearAttentionChunked(Function):
+    @classmethod
+    def apply(cls, *args):
+        if cls is LinearAttentionChunked and len(args) == 3:
+            out = _native.product(3, *args)
+            if out is not None:
+                return out
+        return super().apply(*args)
+
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:

@@ -50,14 +50,34 @@ FLA_DECLARE_PAIR(32) FLA_DECLARE_PAIR(64) FLA_DECLARE_PAIR(128)
 #undef FLA_DECLARE_PAIR
 // walk kernels (fla_chunk_walk.h), dtype 0 bf16 / 1 f16, padded head dim D = 32, 64 or 128
 // (walk_bwd: 32 and 64; walk_dkdv, walk_bwd_rev: 128)
-hipError_t walk_totals(int dtype, int D, const WalkTotalsParams &p, hipStream_t stream);
-hipError_t walk_fwd(int dtype, int D, const WalkParams &p, hipStream_t stream);
-hipError_t walk_fwd_wide(int dtype, const WalkParams &p, hipStream_t stream);  // (q, k of 129 .. 256 columns)
-hipError_t walk_bwd_rev_wide(int dtype, const WalkParams &p, hipStream_t stream);  // (... and v of at most 64)
-hipError_t walk_bwd_rev(int dtype, int D, const WalkParams &p, hipStream_t stream);
-hipError_t walk_bwd(int dtype, int D, const WalkParams &p, hipStream_t stream);
-hipError_t walk_dkdv(int dtype, int D, const WalkParams &p, hipStream_t stream);
-hipError_t walk_vec_sums(int dtype, int D, const WalkVecParams &p, int64_t BH, hipStream_t stream);
+#define FLA_WALK_NAME_(fn, t) fn##_t##t
+#define FLA_WALK_NAME(fn, t) FLA_WALK_NAME_(fn, t)
+#define FLA_DECLARE_WALK_D(fn, P)                                                                    \
+    hipError_t FLA_WALK_NAME(fn, 0)(int D, const P &p, hipStream_t stream);                          \
+    hipError_t FLA_WALK_NAME(fn, 1)(int D, const P &p, hipStream_t stream);                          \
+    inline hipError_t fn(int dtype, int D, const P &p, hipStream_t stream) {                         \
+        return dtype == 0 ? FLA_WALK_NAME(fn, 0)(D, p, stream) : FLA_WALK_NAME(fn, 1)(D, p, stream); \
+    }
+#define FLA_DECLARE_WALK_WIDE(fn)                                                                    \
+    hipError_t FLA_WALK_NAME(fn, 0)(const WalkParams &p, hipStream_t stream);                        \
+    hipError_t FLA_WALK_NAME(fn, 1)(const WalkParams &p, hipStream_t stream);                        \
+    inline hipError_t fn(int dtype, const WalkParams &p, hipStream_t stream) {                       \
+        return dtype == 0 ? FLA_WALK_NAME(fn, 0)(p, stream) : FLA_WALK_NAME(fn, 1)(p, stream);       \
+    }
+FLA_DECLARE_WALK_D(walk_totals, WalkTotalsParams)
+FLA_DECLARE_WALK_D(walk_fwd, WalkParams)
+FLA_DECLARE_WALK_D(walk_bwd_rev, WalkParams)
+FLA_DECLARE_WALK_D(walk_bwd, WalkParams)
+FLA_DECLARE_WALK_D(walk_dkdv, WalkParams)
+FLA_DECLARE_WALK_WIDE(walk_fwd_wide)      // (q, k of 129 .. 256 columns)
+FLA_DECLARE_WALK_WIDE(walk_bwd_rev_wide)  // (... and v of at most 64)
+#undef FLA_DECLARE_WALK_D
+#undef FLA_DECLARE_WALK_WIDE
+hipError_t walk_vec_sums_t0(int D, const WalkVecParams &p, int64_t BH, hipStream_t stream);
+hipError_t walk_vec_sums_t1(int D, const WalkVecParams &p, int64_t BH, hipStream_t stream);
+inline hipError_t walk_vec_sums(int dtype, int D, const WalkVecParams &p, int64_t BH, hipStream_t stream) {
+    return dtype == 0 ? walk_vec_sums_t0(D, p, BH, stream) : walk_vec_sums_t1(D, p, BH, stream);
+}
 hipError_t walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, int reverse, hipStream_t stream);
 hipError_t walk_scan(const float *totals, float *entry, int64_t BH, int n_seg, int D, int cols, int reverse,
                      hipStream_t stream, const float *totals_b = nullptr, float *entry_b = nullptr);

@@ -1,0 +1,433 @@
+// The operators' host path between PyTorch and the C ABI (fla.h), natively: argument tests, output and
+// workspace allocation, the call, and the autograd node whose backward runs without the interpreter.
+//
+// A small problem is bound by this path, not by its kernels (forward + backward of B 1, H 2, N 256,
+// D 64: 5 + 7 us of kernels).  With the same steps in Python (torch.autograd.Function, ctypes) the pair
+// took 55 us on one host and 113 us on a slower one, of which most is interpreter work on two threads that
+// hand the interpreter lock to each other.
+//
+// Every entry point returns None where a call is not the plain case (tensor types and shapes that
+// the operator refuses or converts, wrapped tensors, a status other than FLA_OK): the Python class then runs
+// its own forward, which raises what there is to raise.
+#include <Python.h>
+#include <torch/csrc/autograd/custom_function.h>
+#include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/Exceptions.h>
+#include <torch/types.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/DeviceGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <tuple>
+
+#include "fla.h"
+
+namespace {
+
+using at::Tensor;
+using torch::autograd::AutogradContext;
+using torch::autograd::Function;
+using torch::autograd::variable_list;
+
+struct Refused : std::runtime_error {  // the library returned a status: the Python path reports it
+    explicit Refused(int status) : std::runtime_error(fla_strerror(status)) {}
+};
+
+void must(int status) {
+    if (status != FLA_OK) throw Refused(status);
+}
+
+int dtype_code(at::ScalarType t) {
+    return t == at::kBFloat16 ? FLA_DTYPE_BF16 : t == at::kHalf ? FLA_DTYPE_F16 : -1;
+}
+
+// Calls in flight on a device: its guard, the current stream and uninitialised tensors on it.
+struct Call {
+    c10::DeviceGuard guard;
+    at::TensorOptions like;
+    void *stream;
+    int64_t b, h, n, dqk, dv;
+    int dtype;
+    Call(const Tensor &q, const Tensor &v)
+        : guard(q.device()), like(q.options().requires_grad(false)),
+          stream(c10::hip::getCurrentHIPStream(q.device().index()).stream()), b(q.size(0)), h(q.size(1)), n(q.size(2)),
+          dqk(q.size(3)), dv(v.size(3)), dtype(dtype_code(q.scalar_type())) {}
+    Tensor rows(int64_t width) const { return at::empty({b, h, n, width}, like); }
+    Tensor row_floats() const { return at::empty({b, h, n}, like.dtype(at::kFloat)); }
+    Tensor bytes(int64_t count) const { return count ? at::empty({count}, like.dtype(at::kByte)) : Tensor(); }
+};
+
+void *ptr(const Tensor &t) { return t.defined() ? t.data_ptr() : nullptr; }
+const int64_t *str(const Tensor &t) { return t.strides().data(); }
+int64_t size_of(const Tensor &t) { return t.defined() ? t.numel() : 0; }
+
+// (the innermost dimension dense: what the library asks of every operand)
+Tensor dense(const Tensor &t) { return t.stride(3) != 1 && t.size(3) > 1 ? t.contiguous() : t; }
+
+// ---- tests of a call's tensors
+
+bool plain(const Tensor &t) {
+    using K = c10::DispatchKey;
+    static const c10::DispatchKeySet odd({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper,
+                                          K::Functionalize, K::Conjugate, K::Negative, K::ZeroTensor});
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.dim() == 4 && !t.key_set().has_any(odd);
+}
+
+// q, k: (B, H, N, D_qk), v: (B, H, N, D_v), one device; `cast`: autocast turns any floating type into bf16
+bool agree(const Tensor &q, const Tensor &k, const Tensor &v, bool cast) {
+    if (!plain(q) || !plain(k) || !plain(v) || k.device() != q.device() || v.device() != q.device()) return false;
+    if (q.sizes() != k.sizes() || v.size(0) != q.size(0) || v.size(1) != q.size(1) || v.size(2) != q.size(2)) return false;
+    if (q.size(3) < 1 || v.size(3) < 1 || q.numel() == 0) return false;
+    auto castable = [](at::ScalarType t) { return t == at::kFloat || t == at::kBFloat16 || t == at::kHalf; };
+    if (cast) return castable(q.scalar_type()) && castable(k.scalar_type()) && castable(v.scalar_type());
+    return dtype_code(q.scalar_type()) >= 0 && k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type();
+}
+
+Tensor cast_to(const Tensor &t, bool cast) { return cast ? t.to(at::kBFloat16) : t; }
+
+bool wants_grad(const Tensor &q, const Tensor &k, const Tensor &v) {
+    return at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
+}
+
+// ---- tril(Q K^T) V
+
+enum Evaluation { kEqual = 0, kSmallV = 1, kChunked = 2 };
+
+std::tuple<Tensor, Tensor> product_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, int ev, bool want_state) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor q = dense(q_), k = dense(k_), v = dense(v_);
+    const Call c(q, v);
+    Tensor o = c.rows(c.dv), state;
+    if (ev == kEqual) {
+        must(fla_linear_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(o), c.b, c.h, c.n, c.dqk, str(q), str(k), str(v), str(o), c.dtype,
+                                 c.stream));
+    } else if (ev == kSmallV) {
+        must(fla_linear_attn_smallv_fwd(ptr(q), ptr(k), ptr(v), ptr(o), c.b, c.h, c.n, c.dqk, c.dv, str(q), str(k), str(v),
+                                        str(o), c.dtype, c.stream));
+    } else {
+        if (want_state) state = c.bytes(fla_linear_attn_chunked_state_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        int32_t valid = 0;
+        must(fla_linear_attn_chunked_fwd(ptr(q), ptr(k), ptr(v), ptr(o), c.b, c.h, c.n, c.dqk, c.dv, str(q), str(k), str(v),
+                                         str(o), c.dtype, ptr(state), &valid, ptr(work), size_of(work), c.stream));
+        if (!valid) state = Tensor();
+    }
+    return {o, state};
+}
+
+variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &state, int ev) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor go = dense(go_), q = dense(q_), k = dense(k_), v = dense(v_);
+    const Call c(q, v);
+    Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
+    if (ev == kEqual) {
+        must(fla_linear_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, str(go),
+                                 str(q), str(k), str(v), str(dq), str(dk), str(dv), c.dtype, c.stream));
+    } else if (ev == kSmallV) {
+        must(fla_linear_attn_smallv_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
+                                        str(go), str(q), str(k), str(v), str(dq), str(dk), str(dv), c.dtype, c.stream));
+    } else {
+        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        must(fla_linear_attn_chunked_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
+                                         str(go), str(q), str(k), str(v), str(dq), str(dk), str(dv), c.dtype, ptr(state),
+                                         ptr(work), size_of(work), c.stream));
+    }
+    return {dq, dk, dv};
+}
+
+struct Product : Function<Product> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, int64_t ev, bool cast) {
+        const Tensor q = cast_to(q_, cast), k = cast_to(k_, cast), v = cast_to(v_, cast);
+        auto [o, state] = product_fwd(q, k, v, (int)ev, true);
+        ctx->saved_data["ev"] = ev;
+        if (state.defined())
+            ctx->save_for_backward({q, k, v, state});
+        else
+            ctx->save_for_backward({q, k, v});
+        return o;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list go) {
+        const variable_list s = ctx->get_saved_variables();
+        variable_list g = product_bwd(go[0], s[0], s[1], s[2], s.size() > 3 ? s[3] : Tensor(), (int)ctx->saved_data["ev"].toInt());
+        g.resize(5);
+        return g;
+    }
+};
+
+// ---- the normalised operator, without and with a feature map; the feature map alone
+
+struct Options {
+    int fmap;  // 0: none
+    bool normalise, chunked;
+    double eps;
+    int64_t code() const { return fmap | (normalise ? 16 : 0) | (chunked ? 32 : 0); }
+    static Options of(int64_t code) { return {(int)(code & 15), (code & 16) != 0, (code & 32) != 0, 0.0}; }
+};
+
+struct MappedResult {
+    Tensor o, q, k, denom, state;  // q, k: phi(xq), phi(xk) with a feature map
+};
+
+MappedResult mapped_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Options &opt, bool want_state) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor q = dense(q_), k = dense(k_), v = dense(v_);
+    const Call c(q, v);
+    MappedResult r;
+    r.o = c.rows(c.dv);
+    if (opt.fmap) r.q = c.rows(c.dqk), r.k = c.rows(c.dqk);
+    if (want_state && opt.chunked) r.state = c.bytes(fla_linear_attn_chunked_state_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+    int32_t valid = 0;
+    if (opt.normalise) {
+        r.denom = c.row_floats();
+        const Tensor work = c.bytes(fla_normalised_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv, opt.chunked));
+        if (opt.fmap)
+            must(fla_feature_attn_normalised_fwd(ptr(q), ptr(k), ptr(v), ptr(r.o), ptr(r.q), ptr(r.k), r.denom.data_ptr<float>(),
+                                                 c.b, c.h, c.n, c.dqk, c.dv, str(q), str(k), str(v), str(r.o), str(r.q),
+                                                 str(r.k), opt.fmap, (float)opt.eps, c.dtype, opt.chunked, ptr(r.state), &valid,
+                                                 ptr(work), size_of(work), c.stream));
+        else
+            must(fla_linear_attn_normalised_fwd(ptr(q), ptr(k), ptr(v), ptr(r.o), r.denom.data_ptr<float>(), c.b, c.h, c.n,
+                                                c.dqk, c.dv, str(q), str(k), str(v), str(r.o), (float)opt.eps, c.dtype,
+                                                opt.chunked, ptr(r.state), &valid, ptr(work), size_of(work), c.stream));
+    } else {
+        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        must(fla_feature_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(r.o), ptr(r.q), ptr(r.k), c.b, c.h, c.n, c.dqk, c.dv, str(q),
+                                  str(k), str(v), str(r.o), str(r.q), str(r.k), opt.fmap, c.dtype, ptr(r.state), &valid,
+                                  ptr(work), size_of(work), c.stream));
+    }
+    if (!valid) r.state = Tensor();
+    return r;
+}
+
+variable_list mapped_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &o,
+                         const Tensor &denom, const Tensor &state, const Options &opt) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor go = dense(go_), q = dense(q_), k = dense(k_), v = dense(v_);
+    const Call c(q, v);
+    Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
+    if (opt.normalise) {
+        const Tensor work = c.bytes(fla_normalised_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv, opt.chunked));
+        const float *n = denom.data_ptr<float>();
+        if (opt.fmap)
+            must(fla_feature_attn_normalised_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h,
+                                                 c.n, c.dqk, c.dv, str(go), str(q), str(k), str(v), str(o), str(dq), str(dk),
+                                                 str(dv), opt.fmap, c.dtype, opt.chunked, ptr(state), ptr(work), size_of(work),
+                                                 c.stream));
+        else
+            must(fla_linear_attn_normalised_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h,
+                                                c.n, c.dqk, c.dv, str(go), str(q), str(k), str(v), str(o), str(dq), str(dk),
+                                                str(dv), c.dtype, opt.chunked, ptr(state), ptr(work), size_of(work), c.stream));
+    } else {
+        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        must(fla_feature_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go),
+                                  str(q), str(k), str(v), str(dq), str(dk), str(dv), opt.fmap, c.dtype, ptr(state), ptr(work),
+                                  size_of(work), c.stream));
+    }
+    return {dq, dk, dv};
+}
+
+struct Mapped : Function<Mapped> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, int64_t code, double eps,
+                          bool cast) {
+        Options opt = Options::of(code);
+        opt.eps = eps;
+        const Tensor q = cast_to(q_, cast), k = cast_to(k_, cast), v = cast_to(v_, cast);
+        MappedResult r = mapped_fwd(q, k, v, opt, true);
+        ctx->saved_data["opt"] = code;
+        variable_list s = {opt.fmap ? r.q : q, opt.fmap ? r.k : k, v};
+        if (opt.normalise) s.push_back(r.o), s.push_back(r.denom);
+        if (r.state.defined()) s.push_back(r.state);
+        ctx->save_for_backward(std::move(s));
+        return r.o;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list go) {
+        const Options opt = Options::of(ctx->saved_data["opt"].toInt());
+        const variable_list s = ctx->get_saved_variables();
+        const size_t base = opt.normalise ? 5 : 3;
+        variable_list g = mapped_bwd(go[0], s[0], s[1], s[2], opt.normalise ? s[3] : Tensor(), opt.normalise ? s[4] : Tensor(),
+                                     s.size() > base ? s[base] : Tensor(), opt);
+        g.resize(6);
+        return g;
+    }
+};
+
+// ---- the polynomial score map
+
+struct Poly {
+    float c[3];
+    bool normalise;
+    float eps;
+};
+
+std::tuple<Tensor, Tensor> poly_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Poly &p) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor q = dense(q_), k = dense(k_), v = dense(v_);
+    const Call c(q, v);
+    Tensor o = c.rows(c.dv), denom;
+    if (p.normalise) denom = c.row_floats();
+    must(fla_poly_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(o), static_cast<float *>(ptr(denom)), c.b, c.h, c.n, c.dqk, c.dv, str(q),
+                           str(k), str(v), str(o), p.c, p.eps, c.dtype, c.stream));
+    return {o, denom};
+}
+
+variable_list poly_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &o,
+                       const Tensor &denom, const Poly &p) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    const Tensor go = dense(go_), q = dense(q_), k = dense(k_), v = dense(v_);
+    const Call c(q, v);
+    Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
+    const Tensor work = c.bytes(fla_poly_attn_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+    must(fla_poly_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), static_cast<const float *>(ptr(denom)), ptr(dq), ptr(dk),
+                           ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go), str(q), str(k), str(v),
+                           o.defined() ? str(o) : nullptr, str(dq), str(dk), str(dv), p.c, c.dtype, ptr(work), size_of(work),
+                           c.stream));
+    return {dq, dk, dv};
+}
+
+struct Polynomial : Function<Polynomial> {
+    static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, double c0, double c1,
+                          double c2, bool normalise, double eps, bool cast) {
+        const Tensor q = cast_to(q_, cast), k = cast_to(k_, cast), v = cast_to(v_, cast);
+        auto [o, denom] = poly_fwd(q, k, v, Poly{{(float)c0, (float)c1, (float)c2}, normalise, (float)eps});
+        ctx->saved_data["c0"] = c0, ctx->saved_data["c1"] = c1, ctx->saved_data["c2"] = c2;
+        if (normalise)
+            ctx->save_for_backward({q, k, v, o, denom});
+        else
+            ctx->save_for_backward({q, k, v});
+        return o;
+    }
+    static variable_list backward(AutogradContext *ctx, variable_list go) {
+        const variable_list s = ctx->get_saved_variables();
+        const bool normalise = s.size() > 3;
+        auto c = [&](const char *key) { return (float)ctx->saved_data[key].toDouble(); };
+        variable_list g = poly_bwd(go[0], s[0], s[1], s[2], normalise ? s[3] : Tensor(), normalise ? s[4] : Tensor(),
+                                   Poly{{c("c0"), c("c1"), c("c2")}, normalise, 0.f});
+        g.resize(9);
+        return g;
+    }
+};
+
+// ---- Python entry points: each takes q, k, v and plain numbers, and returns a tensor or None
+
+struct Operands {
+    Tensor q, k, v;
+    bool cast = false, ok = false;
+};
+
+Operands operands(PyObject *const *args) {
+    Operands a;
+    if (!THPVariable_Check(args[0]) || !THPVariable_Check(args[1]) || !THPVariable_Check(args[2])) return a;
+    a.q = THPVariable_Unpack(args[0]), a.k = THPVariable_Unpack(args[1]), a.v = THPVariable_Unpack(args[2]);
+    a.cast = at::autocast::is_autocast_enabled(at::kCUDA);
+    a.ok = agree(a.q, a.k, a.v, a.cast);
+    return a;
+}
+
+template <typename Run>
+PyObject *released(Run &&run) {  // (allocation and launches without the interpreter lock)
+    Tensor out;
+    {
+        PyThreadState *ts = PyEval_SaveThread();
+        try {
+            out = run();
+        } catch (const Refused &) {  // (out stays undefined)
+        } catch (...) {
+            PyEval_RestoreThread(ts);
+            throw;
+        }
+        PyEval_RestoreThread(ts);
+    }
+    if (!out.defined()) Py_RETURN_NONE;
+    return THPVariable_Wrap(std::move(out));
+}
+
+bool pow2(int64_t x) { return (x & (x - 1)) == 0; }
+int64_t next_pow2(int64_t x) {
+    int64_t p = 1;
+    while (p < x) p <<= 1;
+    return p;
+}
+
+// product(kind, q, k, v): kind 0 LinearAttention, 1 LinearAttentionSmallVHD, 2 LinearAttentionAuto, 3 LinearAttentionChunked
+PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 4) Py_RETURN_NONE;
+    const long kind = PyLong_AsLong(args[0]);
+    const Operands a = operands(args + 1);
+    if (!a.ok) Py_RETURN_NONE;
+    const int64_t rows = a.q.size(2), dqk = a.q.size(3), dv = a.v.size(3);
+    if (dqk > 256 || dv > 256) Py_RETURN_NONE;
+    const bool bf16 = a.cast || a.q.scalar_type() == at::kBFloat16, equal = dqk == dv;
+    auto prefers = [&] { return fla_linear_attn_prefers_chunked(a.q.size(0), a.q.size(1), rows, dqk, dv) != 0; };
+    int ev = equal ? kEqual : kSmallV;
+    if (kind == 0) {  // (the shapes its forward takes, and its choice: linear_attn.py)
+        if (!equal || rows % (dqk > 128 ? 32 : 64) != 0) Py_RETURN_NONE;
+        if (bf16 && dqk <= 128 && prefers()) ev = kChunked;
+    } else if (kind == 1) {  // (linear_attn_smallv_hd.py)
+        if (!pow2(dv) || dv > next_pow2(dqk) || rows % 64 != 0) Py_RETURN_NONE;
+        ev = bf16 && dv <= 128 && prefers() ? kChunked : kSmallV;
+    } else if (kind == 2) {  // (auto.py)
+        if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || prefers()) ev = kChunked;
+    } else {
+        ev = kChunked;
+    }
+    return released([&]() -> Tensor {
+        if (wants_grad(a.q, a.k, a.v)) return Product::apply(a.q, a.k, a.v, (int64_t)ev, a.cast);
+        return std::get<0>(product_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast), ev, false));
+    });
+    END_HANDLE_TH_ERRORS
+}
+
+// mapped(q, k, v, feature map code, normalise, eps, chunked)
+PyObject *py_mapped(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 7) Py_RETURN_NONE;
+    const Operands a = operands(args);
+    if (!a.ok || a.q.size(3) > 256 || a.v.size(3) > 256) Py_RETURN_NONE;
+    Options opt;
+    opt.fmap = (int)PyLong_AsLong(args[3]);
+    opt.normalise = PyObject_IsTrue(args[4]) == 1, opt.eps = PyFloat_AsDouble(args[5]), opt.chunked = PyObject_IsTrue(args[6]) == 1;
+    if (PyErr_Occurred()) {  // (not numbers: the Python path says so)
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    return released([&]() -> Tensor {
+        if (wants_grad(a.q, a.k, a.v)) return Mapped::apply(a.q, a.k, a.v, opt.code(), opt.eps, a.cast);
+        return mapped_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast), opt, false).o;
+    });
+    END_HANDLE_TH_ERRORS
+}
+
+// polynomial(xq, xk, v, c0, c1, c2, normalise, eps)
+PyObject *py_polynomial(PyObject *, PyObject *const *args, Py_ssize_t n) {
+    HANDLE_TH_ERRORS
+    if (n != 8) Py_RETURN_NONE;
+    const Operands a = operands(args);
+    if (!a.ok || a.q.size(3) > 32 || a.q.size(3) % 8 != 0 || a.v.size(3) > 128 || a.v.size(3) % 8 != 0) Py_RETURN_NONE;
+    double c[3];
+    for (int i = 0; i < 3; ++i) c[i] = PyFloat_AsDouble(args[3 + i]);
+    const bool normalise = PyObject_IsTrue(args[6]) == 1;
+    const double eps = PyFloat_AsDouble(args[7]);
+    if (PyErr_Occurred()) {
+        PyErr_Clear();
+        Py_RETURN_NONE;
+    }
+    return released([&]() -> Tensor {
+        if (wants_grad(a.q, a.k, a.v)) return Polynomial::apply(a.q, a.k, a.v, c[0], c[1], c[2], normalise, eps, a.cast);
+        return std::get<0>(poly_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast),
+                                    Poly{{(float)c[0], (float)c[1], (float)c[2]}, normalise, (float)eps}));
+    });
+    END_HANDLE_TH_ERRORS
+}
+
+PyMethodDef methods[] = {
+    {"product", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_product)), METH_FASTCALL, nullptr},
+    {"mapped", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_mapped)), METH_FASTCALL, nullptr},
+    {"polynomial", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(py_polynomial)), METH_FASTCALL, nullptr},
+    {nullptr, nullptr, 0, nullptr}};
+
+PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fla_torch", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
+
+}  // namespace
+
+PyMODINIT_FUNC PyInit__fla_torch() { return PyModule_Create(&module); }

@@ -25,7 +25,7 @@ from typing import Any, Optional, Tuple
 import torch
 from torch.autograd import Function
 
-from . import _lib
+from . import _lib, _native
 from .kernels._common import device_guard, dtype_code, prepare, stream_handle
 
 FEATURE_MAPS = {"elu1": 1, "softplus": 2}  # enum fla_feature_map
@@ -175,6 +175,17 @@ def feature_attention_normalised_bwd(grad_output: torch.Tensor, q: torch.Tensor,
 
 
 class FeatureMapLinearAttention(Function):
+    @classmethod
+    def apply(cls, *args):
+        if cls is FeatureMapLinearAttention and 3 <= len(args) <= 7:
+            feature, normalise, eps, chunked = (*args[3:], *("elu1", False, 1e-5, True)[len(args) - 3:])
+            code = FEATURE_MAPS.get(feature)
+            if code is not None and (normalise or chunked):
+                out = _native.mapped(*args[:3], code, normalise, eps, chunked)
+                if out is not None:
+                    return out
+        return super().apply(*args)
+
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx: Any, xq: torch.Tensor, xk: torch.Tensor, v: torch.Tensor, feature: str = "elu1",

@@ -20,7 +20,7 @@ import ctypes
 import torch
 from torch.autograd import Function
 
-from . import _lib
+from . import _lib, _native
 from .kernels._common import device_guard, dtype_code, prepare, stream_handle
 
 
@@ -100,6 +100,15 @@ def linear_attention_normalised_bwd(
 
 
 class LinearAttentionNormalised(Function):
+    @classmethod
+    def apply(cls, *args):
+        if cls is LinearAttentionNormalised and 3 <= len(args) <= 5:
+            eps, chunked = (*args[3:], *(1e-5, False)[len(args) - 3:])
+            out = _native.mapped(*args[:3], 0, True, eps, chunked)
+            if out is not None:
+                return out
+        return super().apply(*args)
+
     @staticmethod
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, eps: float = 1e-5,
