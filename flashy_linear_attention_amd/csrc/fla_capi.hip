@@ -9,6 +9,7 @@
 
 #include "fla_dispatch.h"
 #include "fla_norm.h"
+#include "fla_pack.h"
 
 // Scratch of fla_linear_attn_chunked_fwd_static: one copy per GPU, at its own address on each.
 // Host code never uses the array's name as an address; it asks the runtime for the device
@@ -1161,6 +1162,118 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                                                                                                    : FLA_ERR_LAUNCH;
 }
 
+// ---- widths that are no multiples of 8: the plain chunk-wise operator on copies with aligned rows (fla_pack.h).
+// The copies' columns beyond the true width are zeros, so sums and results are the same.  Forward leaves its copies of q, k, v in the state
+// buffer, behind the state, and backward takes them from there.
+struct PackPlan {
+    bool ok;
+    int64_t wq, wv;                     // rounded widths
+    int64_t q_bytes, v_bytes;           // one copy of width wq / wv (0: that side's rows are taken as they are)
+    int64_t inner_state, inner_work;    // of the rounded problem
+};
+
+PackPlan pack_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
+    PackPlan p{};
+    if ((dqk % 8 == 0 && dv % 8 == 0) || dqk < 1 || dv < 1 || B <= 0 || H <= 0 || N <= 0) return p;
+    if (B * H > 0x7fffffffLL / N) return p;  // (the copy kernel counts rows in 32 bits)
+    p.wq = (dqk + 7) / 8 * 8, p.wv = (dv + 7) / 8 * 8;
+    p.ok = true;
+    auto up = [](int64_t bytes) { return (bytes + 255) / 256 * 256; };
+    p.q_bytes = dqk % 8 ? up(B * H * N * p.wq * 2) : 0, p.v_bytes = dv % 8 ? up(B * H * N * p.wv * 2) : 0;
+    p.inner_state = up(shared_state_bytes(B, H, N, p.wq, p.wv));
+    p.inner_work = up(chunked_op_workspace_bytes(B, H, N, p.wq, p.wv));
+    return p;
+}
+
+int64_t packed_state_bytes(const PackPlan &p) { return p.inner_state + 2 * p.q_bytes + p.v_bytes; }
+// (backward without forward's copies is the larger: q, k, dQ, dK on one side, v, dO, dV on the other)
+int64_t packed_work_bytes(const PackPlan &p) { return p.inner_work + 4 * p.q_bytes + 3 * p.v_bytes; }
+
+// Row-packed stand-ins of a call's operands: views of copies carved from a buffer, and the launch that fills
+// them (or, for results, copies them back).
+struct Packed {
+    fla::PackParams pp{};
+    int count = 0;
+    int64_t B, H, N;
+    Packed(int64_t b, int64_t h, int64_t n) : B(b), H(h), N(n) {
+        pp.H = (int32_t)h, pp.N = (int32_t)n, pp.rows = (int32_t)(b * h * n);
+    }
+    void in(const View &from, const View &to, int64_t width, int64_t wp) { add(from, to, width, wp); }
+    void out(const View &from, const View &to, int64_t width) { add(from, to, width, width); }
+    void add(const View &from, const View &to, int64_t width, int64_t wp) {
+        fla::PackItem &t = pp.item[count++];
+        t.src = from.ptr, t.dst = const_cast<void *>(to.ptr);
+        t.ss_b = from.strides[0], t.ss_h = from.strides[1], t.ss_n = from.strides[2];
+        t.ds_b = to.strides[0], t.ds_h = to.strides[1], t.ds_n = to.strides[2];
+        t.width = (int32_t)width, t.wp = (int32_t)wp;
+    }
+    int launch(void *stream) {
+        if (!count) return FLA_OK;
+        return fla::launch_pack_rows(pp, count, static_cast<hipStream_t>(stream)) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
+    }
+};
+
+int packed_forward(const PackPlan &p, const View &q, const View &k, const View &v, const View &o, int64_t B, int64_t H,
+                   int64_t N, int64_t dqk, int64_t dv, int dtype, void *state_out, int32_t *state_valid, void *workspace,
+                   int64_t workspace_bytes, void *stream) {
+    if (state_valid) *state_valid = 0;
+    const View all[] = {q, k, v, o};
+    for (const View &t : all)
+        if (int rc = check_view(t)) return rc;
+    if (int rc = check_alias_fwd(q, k, v, o, B, H, N, dqk, dv)) return rc;
+    if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < packed_work_bytes(p))
+        return FLA_ERR_WORKSPACE;
+    if (state_out && reinterpret_cast<uintptr_t>(state_out) % 16 != 0) return FLA_ERR_WORKSPACE;
+    const int64_t qs[4] = {H * N * p.wq, N * p.wq, p.wq, 1}, vs[4] = {H * N * p.wv, N * p.wv, p.wv, 1};
+    char *copies = state_out ? static_cast<char *>(state_out) + p.inner_state : static_cast<char *>(workspace) + p.inner_work;
+    char *results = static_cast<char *>(workspace) + p.inner_work + 2 * p.q_bytes + p.v_bytes;
+    const View qp = p.q_bytes ? View{copies, qs} : q, kp = p.q_bytes ? View{copies + p.q_bytes, qs} : k;
+    const View vp = p.v_bytes ? View{copies + 2 * p.q_bytes, vs} : v, op = p.v_bytes ? View{results, vs} : o;
+    Packed in(B, H, N), out(B, H, N);
+    if (p.q_bytes) in.in(q, qp, dqk, p.wq), in.in(k, kp, dqk, p.wq);
+    if (p.v_bytes) in.in(v, vp, dv, p.wv), out.out(op, o, dv);
+    if (int rc = in.launch(stream)) return rc;
+    if (int rc = chunked_forward(qp, kp, vp, op, B, H, N, p.wq, p.wv, dtype, state_out, state_valid, workspace, p.inner_work,
+                                 stream))
+        return rc;
+    return out.launch(stream);
+}
+
+int packed_backward(const PackPlan &p, const View &go, const View &q, const View &k, const View &v, const View &dq,
+                    const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
+                    const void *state_in, void *workspace, int64_t workspace_bytes, void *stream) {
+    const View all[] = {go, q, k, v, dq, dk, dvv};
+    for (const View &t : all)
+        if (int rc = check_view(t)) return rc;
+    if (int rc = check_alias_bwd(go, q, k, v, nullptr, dq, dk, dvv, B, H, N, dqk, dv)) return rc;
+    if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < packed_work_bytes(p))
+        return FLA_ERR_WORKSPACE;
+    if (state_in && reinterpret_cast<uintptr_t>(state_in) % 16 != 0) return FLA_ERR_WORKSPACE;
+    const int64_t qs[4] = {H * N * p.wq, N * p.wq, p.wq, 1}, vs[4] = {H * N * p.wv, N * p.wv, p.wv, 1};
+    char *work = static_cast<char *>(workspace) + p.inner_work;
+    char *copies = state_in ? const_cast<char *>(static_cast<const char *>(state_in)) + p.inner_state : work;
+    char *more = work + 2 * p.q_bytes + p.v_bytes;  // (dQ, dK, dO, dV)
+    const View qp = p.q_bytes ? View{copies, qs} : q, kp = p.q_bytes ? View{copies + p.q_bytes, qs} : k;
+    const View vp = p.v_bytes ? View{copies + 2 * p.q_bytes, vs} : v;
+    const View dqp = p.q_bytes ? View{more, qs} : dq, dkp = p.q_bytes ? View{more + p.q_bytes, qs} : dk;
+    const View gop = p.v_bytes ? View{more + 2 * p.q_bytes, vs} : go;
+    const View dvp = p.v_bytes ? View{more + 2 * p.q_bytes + p.v_bytes, vs} : dvv;
+    Packed in(B, H, N), out(B, H, N);
+    if (p.q_bytes) {
+        if (!state_in) in.in(q, qp, dqk, p.wq), in.in(k, kp, dqk, p.wq);
+        out.out(dqp, dq, dqk), out.out(dkp, dk, dqk);
+    }
+    if (p.v_bytes) {
+        if (!state_in) in.in(v, vp, dv, p.wv);
+        in.in(go, gop, dv, p.wv), out.out(dvp, dvv, dv);
+    }
+    if (int rc = in.launch(stream)) return rc;
+    if (int rc = chunked_backward(gop, qp, kp, vp, dqp, dkp, dvp, B, H, N, p.wq, p.wv, dtype, state_in, workspace, p.inner_work,
+                                  stream))
+        return rc;
+    return out.launch(stream);
+}
+
 // O = tril(phi(xq) phi(xk)^T) v with mapped = {phi(xq), phi(xk)} as further outputs.  Chunk-wise
 // (chunked != 0): the kernels map on load where they can (the state kernel xk, the main kernel its
 // rows of xq); any other shape or layout, and the quadratic kernels, get one element-wise pass
@@ -1724,6 +1837,10 @@ int fla_linear_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_q
     if (B < 1 || H < 1 || N < 1 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
     const double w = (double)B * (double)H * (double)N * (double)N * (double)padded(D_qk > D_v ? D_qk : D_v);
     const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v, true);
+    // Widths that are no multiples of 8: the quadratic operator runs the bounds-checked kernel, the chunk-wise one the
+    // fast kernels of either kind on copies with aligned rows, 1.4 to 12 times faster (forward + backward) over
+    // B H = 2 ... 128, N = 256 ... 2048 and widths 36, 91/64, 100, 153/64.
+    if (pack_plan(B, H, N, D_qk, D_v).ok) return 1;
     // (padded widths that differ: the quadratic side is the small-V operator, whose wide products are two launches)
     if (wp.ok && pad_index(D_qk) != pad_index(D_v)) return w >= (wp.D <= 64 ? 1e9 : 5e8);
     if (wp.ok) return w >= (wp.D <= 64 ? 4e9 : 8e9);                              // equal padded head dims up to 128
@@ -1734,12 +1851,16 @@ int fla_linear_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_q
 
 int64_t fla_linear_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v) {
     if (B < 0 || H < 0 || N < 0 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
-    return shared_state_bytes(B, H, N, D_qk, D_v);
+    const int64_t plain = shared_state_bytes(B, H, N, D_qk, D_v);  // (the normalised operator's, whatever the widths)
+    const PackPlan p = pack_plan(B, H, N, D_qk, D_v);
+    return p.ok && packed_state_bytes(p) > plain ? packed_state_bytes(p) : plain;
 }
 
 int64_t fla_linear_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v) {
     if (B < 0 || H < 0 || N < 0 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
-    return chunked_op_workspace_bytes(B, H, N, D_qk, D_v);
+    const int64_t plain = chunked_op_workspace_bytes(B, H, N, D_qk, D_v);  // (the feature-map operator's, whatever the widths)
+    const PackPlan p = pack_plan(B, H, N, D_qk, D_v);
+    return p.ok && packed_work_bytes(p) > plain ? packed_work_bytes(p) : plain;
 }
 
 int fla_linear_attn_chunked_fwd(const void *q, const void *k, const void *v, void *o, int64_t B, int64_t H, int64_t N,
@@ -1750,6 +1871,9 @@ int fla_linear_attn_chunked_fwd(const void *q, const void *k, const void *v, voi
     if (int rc = check_common(B, H, N, dtype)) return rc;
     if (D_qk < 1 || D_qk > 256) return FLA_ERR_HEAD_DIM;
     if (D_v < 1 || D_v > 256) return FLA_ERR_V_HEAD_DIM;
+    if (const PackPlan p = pack_plan(B, H, N, D_qk, D_v); p.ok)
+        return packed_forward(p, {q, q_strides}, {k, k_strides}, {v, v_strides}, {o, o_strides}, B, H, N, D_qk, D_v, dtype,
+                              state_out, state_valid, workspace, workspace_bytes, stream);
     return chunked_forward({q, q_strides}, {k, k_strides}, {v, v_strides}, {o, o_strides}, B, H, N, D_qk, D_v, dtype,
                            state_out, state_valid, workspace, workspace_bytes, stream);
 }
@@ -1819,6 +1943,10 @@ int fla_linear_attn_chunked_bwd(const void *grad_out, const void *q, const void 
     if (int rc = check_common(B, H, N, dtype)) return rc;
     if (D_qk < 1 || D_qk > 256) return FLA_ERR_HEAD_DIM;
     if (D_v < 1 || D_v > 256) return FLA_ERR_V_HEAD_DIM;
+    if (const PackPlan p = pack_plan(B, H, N, D_qk, D_v); p.ok)
+        return packed_backward(p, {grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides}, {dq, dq_strides},
+                               {dk, dk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v, dtype, state_in, workspace,
+                               workspace_bytes, stream);
     return chunked_backward({grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides}, {dq, dq_strides},
                             {dk, dk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v, dtype, state_in, workspace,
                             workspace_bytes, stream);

@@ -8,6 +8,7 @@
 #include "fla_chunk_state.h"
 #include "fla_chunk_walk.h"
 #include "fla_norm.h"
+#include "fla_pack.h"
 #include "fla_tri_kernel.h"
 #include "fla_tri_pair.h"
 
@@ -84,6 +85,11 @@ FLA_FIELD(zs_n) FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(dc) FLA_FIELD(
 FLA_FIELD(map_y) FLA_FIELD(ymap_out) FLA_FIELD(yo_b) FLA_FIELD(yo_h) FLA_FIELD(yo_n)
 FLA_FIELDS_END
 
+FLA_FIELDS_BEGIN(PackItem)
+FLA_FIELD(src) FLA_FIELD(dst) FLA_FIELD(ss_b) FLA_FIELD(ss_h) FLA_FIELD(ss_n) FLA_FIELD(ds_b) FLA_FIELD(ds_h) FLA_FIELD(ds_n)
+FLA_FIELD(width) FLA_FIELD(wp)
+FLA_FIELDS_END
+
 #undef FLA_FIELDS_BEGIN
 #undef FLA_FIELD
 #undef FLA_FIELDS_END
@@ -95,6 +101,10 @@ inline void trace_describe(trace::Record &r, int arg, const WalkParams &p) { tra
 inline void trace_describe(trace::Record &r, int arg, const WalkTotalsParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const WalkVecParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const ChunkStateParams &p) { trace_fields(r, arg, "", p); }
+inline void trace_describe(trace::Record &r, int arg, const PackParams &p) {
+    for (int i = 0; i < 4; ++i) trace_fields(r, arg, "t" + std::to_string(i) + ".", p.item[i]);
+    r.field(arg, "H", p.H), r.field(arg, "N", p.N), r.field(arg, "rows", p.rows);
+}
 inline void trace_describe(trace::Record &r, int arg, const TriBatch &b) {
     for (int i = 0; i < 3; ++i) trace_fields(r, arg, "p" + std::to_string(i) + ".", b.p[i]);
 }

@@ -192,6 +192,8 @@ int fla_tri_xyt_z_chunked(const void *x, const void *y, const void *z, void *out
  * backward: `state_in` is that buffer, written by the forward call on the same q, k, v, or NULL
  *           (the state is then recomputed by another evaluation: two walks instead of one at
  *           padded head dims above 64, chunk states in memory below).
+ * Widths that are no multiples of 8 run on copies with aligned rows, which the workspace and the
+ * state buffer have room for.
  * `workspace`: fla_linear_attn_chunked_workspace_bytes() bytes of scratch, 16-byte aligned.
  * No counterpart in the reference (quadratic kernels only, linear_attn_kernels.py:63, 166-171). */
 int64_t fla_linear_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v);

@@ -1,0 +1,30 @@
+"""Widths that are no multiples of 8 through the chunk-wise operator (copies with aligned rows): the copy kernel's edges --
+a row's last partial chunk, one row, one column, rows of other strides -- and plans of every kind behind it, against
+the fp32 oracle (``-m gpu``)."""
+
+import pytest
+import torch
+
+from flashy_linear_attention_amd.chunked import linear_attention_chunked_bwd, linear_attention_chunked_fwd
+
+from helpers import assert_close, gpu_fp32_reference, reference_style_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("b,h,n,dqk,dv", [
+    (1, 1, 1, 1, 1), (1, 2, 65, 7, 9), (2, 3, 300, 33, 31), (1, 2, 700, 100, 100), (1, 3, 1000, 91, 64), (2, 1, 520, 153, 64),
+    (1, 2, 330, 64, 57), (1, 2, 390, 255, 255), (1, 1, 600, 129, 127), (1, 2, 640, 100, 250),
+])
+@pytest.mark.parametrize("dtype,transposed", [(torch.bfloat16, False), (torch.bfloat16, True), (torch.float16, True)])
+def test_widths_off_the_eights(b, h, n, dqk, dv, dtype, transposed, gpu_device):
+    q, k, v, do = (t.to(gpu_device) for t in reference_style_inputs(b, h, n, dqk, dv, dtype, seed=n + dqk))
+    want_o, want_g = gpu_fp32_reference(q, k, v, do, True)
+    if transposed:  # (B, N, H, D) storage
+        q, k, v, do = (t.transpose(1, 2).contiguous().transpose(1, 2) for t in (q, k, v, do))
+    out, state = linear_attention_chunked_fwd(q, k, v, want_state=True)
+    assert_close("O", out, want_o)
+    assert torch.equal(out, linear_attention_chunked_fwd(q, k, v))
+    for st in (state, None):  # (forward's copies, and copies of backward's own)
+        for name, got, want in zip(("dQ", "dK", "dV"), linear_attention_chunked_bwd(do, q, k, v, st), want_g):
+            assert_close(f"{name}, state {st is not None}", got, want)
