@@ -125,7 +125,8 @@ def build(jobs: int | None = None, verbose: bool = True) -> str:
     jobs = jobs or min(8, os.cpu_count() or 1)
     # (the slowest first)
     work = [(_compile_walk, (t, part)) for part in (1, 0) for t in (0, 1)]
-    work += [(_compile_torch, None), (_compile_other, "fla_capi"), (_compile_other, "fla_pair_inst")]
+    work += [(_compile_torch, None), (_compile_other, "fla_capi"), (_compile_other, "fla_pair_inst"),
+             (_compile_other, "fla_poly_inst")]
     work += [(_compile_inst, (t, dc, do)) for dc in DIMS for do in DIMS for t in (0, 1)]
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
         objs = list(pool.map(lambda w: w[0](w[1]), work))
@@ -168,6 +169,7 @@ def build_trace(jobs: int | None = None) -> str:
     work += [("fla_walk_inst.hip", f"walk_t{t}_p{part}.o", [f"-DFLA_WALK_DTYPE={t}", f"-DFLA_WALK_PART={part}"])
              for t in (0, 1) for part in (0, 1)]
     work += [("fla_capi.hip", "fla_capi.o", []), ("fla_pair_inst.hip", "fla_pair_inst.o", []),
+             ("fla_poly_inst.hip", "fla_poly_inst.o", []),
              ("fla_trace.cc", "fla_trace.o", ["-x", "c++"])]
     with concurrent.futures.ThreadPoolExecutor(max_workers=jobs) as pool:
         objs = list(pool.map(one, work))

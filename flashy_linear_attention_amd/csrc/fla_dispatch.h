@@ -81,4 +81,9 @@ inline hipError_t walk_vec_sums(int dtype, int D, const WalkVecParams &p, int64_
 hipError_t walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, int reverse, hipStream_t stream);
 hipError_t walk_scan(const float *totals, float *entry, int64_t BH, int n_seg, int D, int cols, int reverse,
                      hipStream_t stream, const float *totals_b = nullptr, float *entry_b = nullptr);
+// the polynomial score map chunk-wise (fla_poly_walk.h), bf16
+struct PolyWalkParams;
+hipError_t poly_totals(const PolyWalkParams &p, bool bwd, hipStream_t stream);
+hipError_t poly_walk(const PolyWalkParams &p, bool bwd, hipStream_t stream);
+hipError_t poly_scan(float *totals, int64_t BH, int n_seg, int reverse, hipStream_t stream);
 }  // namespace fla

@@ -1,0 +1,1042 @@
+// Chunk-wise evaluation of the polynomial score map, O = tril(f(Xq Xk^T)) V with f(u) = c0 + c1 u + c2 u^2, for rows of
+// at most 16 columns over values of at most 64: the quadratic kernels' work grows with N^2, this one's with N.
+//
+// f(x . y) is the product of feature rows phi_w(x) . phi(y) of F = 209 entries (the order of PolyFeatures below): the
+// quadratic terms x_r x_r2 with r2 in the same or an earlier block of eight columns than r (an earlier one counts
+// twice), the columns themselves and a one.  With the running sums of phi(k_j) [v_j, 1]^T over the rows before a chunk
+// (T), and of phi(q_i) [g_i, dn_i]^T over the rows after it (U),
+//
+//   O_i   = f-scores of the chunk . V + phi_w(q_i) T                      n_i the same with the column of ones
+//   dV_j  = f-scores^T of the chunk . g + phi_w(k_j) U
+//   dq_i  = ((M f'(u)) of the chunk) k   + the gradient of phi_w(q) (T [g_i, dn_i]) at q_i        M_ij = g_i . v_j + dn_i
+//   dk_j  = ((M f'(u))^T of the chunk) q + the gradient of phi_w(k) (U [v_j, 1]) at k_j
+//
+// (g = dO / n, dn_i = -(dO_i . O_i) / n_i formed here from dO, O and n; without the normaliser g = dO and no dn).
+// Nothing of width F goes to memory but the states at the ends of a walk's segments: feature rows are
+// formed from the 16-wide rows, the ones that are MFMA operands along the row in registers, the ones whose
+// contraction runs down the rows as an LDS tile.
+//
+// What bounds it: the matrix instructions and the multiplications and roundings that form feature rows (one fragment
+// of eight features costs twelve VALU instructions and serves one or two MFMAs); HBM is far away (40 KiB per
+// 128-row chunk).  Hence eight waves, two per SIMD, so that one wave's VALU work runs under the other's MFMAs: wave w owns
+// rows 32 (w % 4) .. of the chunk, and of their work one half: half of the features and of the score blocks (forward),
+// dq and the rows after the chunk in dV against dk and the chunk's own rows in dV (backward); the two waves of a row
+// block exchange one half of the sums through LDS.  (Halves of the output columns instead formed every feature row and
+// every score twice: VALU instructions were 63 % of the forward walk's time.)  A workgroup takes a CU's LDS; the next chunk's rows are fetched into registers a chunk ahead.  The split
+// into segments and the forms of their entry states are the walk kernels' (fla_chunk_walk.h), and as there the backward
+// walk gets T going backwards, by subtracting every chunk's sums from the state at its segment's end.
+// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 200 us this way (kernels
+// 21 totals, 58 forward, 28 totals, 125 backward; the VALU issues on half of the forward walk's cycles, the matrix
+// unit is busy on a third).
+#pragma once
+
+#include <hip/hip_runtime.h>
+#include <stdint.h>
+
+#include "fla_chunk_walk.h"
+
+namespace fla {
+
+struct PolyWalkParams {
+    const void *q, *k, *v, *go, *o;  // rows of width r (q, k) and dv (v, go: dO, o: forward's result, read by backward)
+    void *out, *dq, *dk, *dv;        // forward: out; backward: dq, dk, dv
+    int64_t qs_b, qs_h, qs_n, ks_b, ks_h, ks_n, vs_b, vs_h, vs_n, gs_b, gs_h, gs_n, os_b, os_h, os_n;
+    int64_t us_b, us_h, us_n;  // out
+    int64_t dqs_b, dqs_h, dqs_n, dks_b, dks_h, dks_n, dvs_b, dvs_h, dvs_n;
+    int32_t H, N, BH, r, wv, n_chunks, seg_chunks, n_seg;
+    float c0, c1, c2, eps;
+    float *denom;  // fp32 [BH][N], or null: not normalised.  Forward writes it, backward reads it
+    // states [BH][n_seg][PolyFeatures::kState] in fp32
+    float *totals;       // totals kernel: receives the segments' sums; walks: those (sum_entries) or the entry states, of
+                         // T (forward) / U (backward); null with a single segment
+    int32_t sum_entries;
+    float *ends;         // T after every segment: written by forward (null: nowhere), read by backward
+};
+
+// Feature order: groups of eight.  Groups 0 .. 7: x_r x_(0..7) for r = 0 .. 7; groups 8 .. 23: x_r x_(8h .. 8h+7) for
+// r = 8 .. 15, h = 0, 1; groups 24, 25: the row itself; group 26: a one and zeros; group 27: zeros.
+struct PolyFeatures {
+    static constexpr int kGroups = 28, kBlocks = 7, kF = 224;  // blocks of 32 features
+    static constexpr int kSteps = kGroups / 2;                 // 16-wide k steps of a contraction over the features
+    static constexpr int kV = 64;                              // value columns of a state
+    static constexpr int kState = kF * kV + kF;                // [feature][value column], then the column of ones / dn
+};
+
+struct PolyLds {  // byte offsets
+    // dn of a chunk: in fp32, rounded, and 256 bytes of zeros
+    static constexpr int DN = 128 * 4 + 256 + 256;
+    static constexpr int C = 128, XT = C * 32, VT = C * 128, PHI = C * 256, ST = 2 * 64 * 256, XTR = 16 * 272, EX = 8 * 4096;
+    // totals: the x tile, the v tile, two feature tiles, dn
+    static constexpr int tX = 0, tV = tX + XT, tPhi = tV + VT, tDn = tPhi + 2 * PHI, tTotal = tDn + DN;
+    // forward
+    static constexpr int fQ = 0, fK = fQ + XT, fV = fK + XT, fS = fV + VT, fPhi = fS + ST, fZ = fPhi + 2 * PHI,
+                         fSum = fZ + PolyFeatures::kF * 4, fEx = fSum + 2 * C * 4, fTotal = fEx + EX;
+    // backward (the second feature tile and T's copy share their place)
+    static constexpr int bQ = 0, bK = bQ + XT, bQt = bK + XT, bKt = bQt + XTR, bV = bKt + XTR, bG = bV + VT, bU = bG + VT,
+                         bPhi = bU + ST, bT = bPhi + PHI, bZ = bT + PHI, bY = bZ + PolyFeatures::kF * 4,
+                         bDn = bY + PolyFeatures::kF * 4, bTotal = bDn + DN;
+    static_assert(PHI == ST && EX == ST && fTotal <= 160 * 1024 && bTotal <= 160 * 1024, "a CU's LDS");
+};
+
+// (a select of two values: written between two elements of an array it would become one load with a computed index, and
+// the array would go to scratch memory)
+__device__ __forceinline__ float poly_pick(int g, float one, float zero) { return g ? one : zero; }
+
+// rounded pairs: eight floats to an operand fragment
+template <typename T>
+__device__ __forceinline__ typename Mma<T>::V8 poly_round8(const float (&f)[8]) {
+    typename Mma<T>::V8 r;
+#pragma unroll
+    for (int j = 0; j < 8; ++j) r[j] = static_cast<T>(f[j]);
+    return r;
+}
+
+// the sixteen columns of one row of an x tile, in fp32
+template <typename T>
+__device__ __forceinline__ void poly_row(const unsigned char *xt, int row, float (&x)[16]) {
+    using V8 = typename Mma<T>::V8;
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+        const V8 e = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4 *>(xt + row * 32 + h * 16));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) x[8 * h + j] = static_cast<float>(e[j]);
+    }
+}
+
+// this lane's eight columns of a row of an x tile: an MFMA operand with k along the row
+template <typename T>
+__device__ __forceinline__ typename Mma<T>::V8 poly_row_frag(const unsigned char *xt, int row, int g) {
+    return __builtin_bit_cast(typename Mma<T>::V8, *reinterpret_cast<const u32x4 *>(xt + row * 32 + g * 16));
+}
+
+// column r of an x tile from its transposed copy, rows R0 + {4g .., 8 + 4g ..}: the k order of a rounded score
+template <typename T>
+__device__ __forceinline__ typename Mma<T>::V8 poly_col_frag(const unsigned char *xtr, int r, int R0, int g) {
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    const u32x2 lo = *reinterpret_cast<const u32x2 *>(xtr + r * 272 + (R0 + 4 * g) * 2);
+    const u32x2 hi = *reinterpret_cast<const u32x2 *>(xtr + r * 272 + (R0 + 8 + 4 * g) * 2);
+    return __builtin_bit_cast(typename Mma<T>::V8, u32x4{lo[0], lo[1], hi[0], hi[1]});
+}
+
+// ---- operand fragments of the walk kernels' tile layouts (walk_row_frag, walk_col_frag, walk_col_frag_perm), with their
+// addresses split into what depends on the lane, computed once per chunk, an XOR that picks a chunk of a row or a column
+// block, and a constant offset -- the swizzle of a row depends on the row modulo 16 only.  (As one expression per
+// fragment the addresses took a third of the kernels' VALU instructions.)
+struct PolyPair {
+    uint32_t lo, hi;
+};
+// rows {4g .., 8 + 4g ..}, plain column mapping, column block cb
+template <int RB>
+__device__ __forceinline__ PolyPair poly_col_base(int lane, int cb) {
+    const int lam = lane & 15, g = lane >> 5, beta = (lane >> 4) & 1;
+    const int row = 4 * g + (lam >> 2), ch = 4 * cb + 2 * beta + ((lam & 3) >> 1), sub = 8 * (lam & 1);
+    return {(uint32_t)(row * RB + ((ch ^ walk_swizzle<RB / 16>(row)) << 4) + sub),
+            (uint32_t)((row + 8) * RB + ((ch ^ walk_swizzle<RB / 16>(row + 8)) << 4) + sub)};
+}
+// permuted column mapping, column block 0 (block cb: XOR cb << 6); CONS: rows 8g .. 8g + 7, else {4g .., 8 + 4g ..}
+template <int RB, bool CONS>
+__device__ __forceinline__ PolyPair poly_perm_base(int lane) {
+    const int lam = lane & 15, g = lane >> 5, beta = (lane >> 4) & 1, zc = lam & 3;
+    const int lo = (CONS ? 8 : 4) * g + (lam >> 2), hi = lo + (CONS ? 4 : 8), ch = 2 * (zc & 1) + beta, byte = 8 * (zc >> 1);
+    return {(uint32_t)(lo * RB + ((ch ^ walk_swizzle<RB / 16>(lo)) << 4) + byte),
+            (uint32_t)(hi * RB + ((ch ^ walk_swizzle<RB / 16>(hi)) << 4) + byte)};
+}
+// chunk g of row `row` (k chunk kc: XOR kc << 5)
+template <int RB>
+__device__ __forceinline__ uint32_t poly_row_base(int row, int g) {
+    return (uint32_t)(row * RB + ((g ^ walk_swizzle<RB / 16>(row)) << 4));
+}
+template <typename T>
+__device__ __forceinline__ typename Mma<T>::V8 poly_tr(const unsigned char *tile, PolyPair at, uint32_t flip = 0) {
+    const s16x4 lo = walk_tr_read(tile + (at.lo ^ flip)), hi = walk_tr_read(tile + (at.hi ^ flip));
+    return __builtin_bit_cast(typename Mma<T>::V8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+}
+template <typename T>
+__device__ __forceinline__ typename Mma<T>::V8 poly_rd(const unsigned char *tile, uint32_t at) {
+    return __builtin_bit_cast(typename Mma<T>::V8, *reinterpret_cast<const u32x4 *>(tile + at));
+}
+
+// The mask of a 32 x 32 block on the diagonal for a lane's score i (Y row 8 (i / 4) + 4g + i % 4 against X row l32) as
+// bits to AND with
+template <bool UPPER>
+__device__ __forceinline__ uint32_t poly_mask(int i, int l32, int g) {
+    const int jl = 8 * (i / 4) + 4 * g + (i % 4);
+    return (UPPER ? jl >= l32 : l32 >= jl) ? ~0u : 0u;
+}
+// sixteen values rounded to two fragments and masked as pairs (all: ~0 off the diagonal)
+template <typename T, bool UPPER>
+__device__ __forceinline__ void poly_round_masked(const float (&d)[16], uint32_t all, int l32, int g, typename Mma<T>::V8 (&out)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        float e[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) e[j] = d[8 * t + j];
+        u32x4 w = __builtin_bit_cast(u32x4, poly_round8<T>(e));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const uint32_t m = (poly_mask<UPPER>(8 * t + 2 * k, l32, g) & 0xffffu) | (poly_mask<UPPER>(8 * t + 2 * k + 1, l32, g) & 0xffff0000u);
+            w[k] &= m | all;
+        }
+        out[t] = __builtin_bit_cast(typename Mma<T>::V8, w);
+    }
+}
+
+// Feature fragment KS (features 16 KS + 8 g ..) of a row, weighted for the phi_w side; `raw` receives it in fp32.
+// xs: the row's columns 8 g .. 8 g + 7.
+template <typename T, int KS>
+__device__ __forceinline__ typename Mma<T>::V8 poly_feature_frag(const float (&x)[16], const float (&xs)[8], int g, float c0,
+                                                                 float c1, float c2, float (&raw)[8]) {
+    if constexpr (KS < 4) {
+        const float s = c2 * poly_pick(g, x[2 * KS + 1], x[2 * KS]);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) raw[j] = s * x[j];
+    } else if constexpr (KS < 12) {
+        const float s = (g ? c2 : 2.f * c2) * x[8 + KS - 4];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) raw[j] = s * xs[j];
+    } else if constexpr (KS == 12) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) raw[j] = c1 * xs[j];
+    } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) raw[j] = j == 0 && g == 0 ? c0 : 0.f;
+    }
+    return poly_round8<T>(raw);
+}
+
+// The feature rows of an x tile, written as two tiles of 128 features (the walk kernels' D = 128 tile layout, 128 rows):
+// groups 0 .. 15 to phi0, 16 .. 27 to phi1.  Thread t takes row t % 128, a quarter of the groups.  Rows past the
+// sequence are zeros, their one included.
+template <typename T>
+__device__ __forceinline__ void poly_gen_phi(const unsigned char *xt, unsigned char *phi0, unsigned char *phi1, int row0, int N,
+                                             int tid) {
+    const int row = tid & 127, part = __builtin_amdgcn_readfirstlane(tid >> 7);
+    float x[16];
+    poly_row<T>(xt, row, x);
+    auto put = [&](unsigned char *tile, int pos, typename Mma<T>::V8 v) {
+        *reinterpret_cast<u32x4 *>(tile + row * 256 + ((pos ^ walk_swizzle<16>(row)) << 4)) = __builtin_bit_cast(u32x4, v);
+    };
+    auto product = [&](int r, int h) {
+        float f[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = x[r] * x[8 * h + j];
+        return poly_round8<T>(f);
+    };
+    // (The assembler comments keep the branches' last stores apart.  Merged into one behind the branches, the store had
+    // the address of the last branch computed on one of the two ways into it only: its zeros went over the x tile.)
+    if (part == 0) {
+#pragma unroll
+        for (int r = 0; r < 8; ++r) put(phi0, r, product(r, 0));
+        asm volatile("; groups 0 .. 7" ::: "memory");
+    } else if (part == 1) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) put(phi0, 8 + i, product(8 + i / 2, i % 2));
+        asm volatile("; groups 8 .. 15" ::: "memory");
+    } else if (part == 2) {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) put(phi1, i, product(12 + i / 2, i % 2));
+        asm volatile("; groups 16 .. 23" ::: "memory");
+    } else {
+        float f[8];
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+#pragma unroll
+            for (int j = 0; j < 8; ++j) f[j] = x[8 * h + j];
+            put(phi1, 8 + h, poly_round8<T>(f));
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = j == 0 && row0 + row < N ? 1.f : 0.f;
+        put(phi1, 10, poly_round8<T>(f));
+#pragma unroll
+        for (int j = 0; j < 8; ++j) f[j] = 0.f;
+        put(phi1, 11, poly_round8<T>(f));
+        asm volatile("; groups 24 .. 27" ::: "memory");
+    }
+}
+
+// A state's blocks of this wave: columns 32 eb .., feature blocks p and p + 4 (p + 4 < 7), and -- NORM -- the column of
+// ones (of dn) for one of the two: lanes with l32 == 0 hold it.
+struct PolyState {
+    f32x16 st[2], ex;
+    int eb, p, fx;  // fx: the feature block of ex (7: none)
+    __device__ __forceinline__ void clear(int wave) {
+        eb = wave & 1, p = wave >> 1, fx = eb == 0 ? p : p + 4;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) st[0][v] = st[1][v] = ex[v] = 0.f;
+    }
+    __device__ __forceinline__ bool valid(int i) const { return p + 4 * i < PolyFeatures::kBlocks; }
+    // += the state at `s` in memory
+    template <bool NORM>
+    __device__ __forceinline__ void add(const float *s, int l32, int g) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (valid(i)) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    st[i][v] += s[(32 * (p + 4 * i) + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * eb + l32];
+            }
+        if (NORM && fx < PolyFeatures::kBlocks && l32 == 0) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                ex[v] += s[PolyFeatures::kF * PolyFeatures::kV + 32 * fx + 8 * (v / 4) + 4 * g + (v % 4)];
+        }
+    }
+    template <bool NORM>
+    __device__ __forceinline__ void store(float *s, int l32, int g) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (valid(i)) {
+#pragma unroll
+                for (int v = 0; v < 16; ++v)
+                    s[(32 * (p + 4 * i) + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * eb + l32] = st[i][v];
+            }
+        if (NORM && fx < PolyFeatures::kBlocks && l32 == 0) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                s[PolyFeatures::kF * PolyFeatures::kV + 32 * fx + 8 * (v / 4) + 4 * g + (v % 4)] = ex[v];
+        }
+    }
+    // rounded to the storage type as rows of value columns, features 0 .. 127 and 128 .. in two tiles; ex in fp32 to z
+    template <typename T, bool NORM>
+    __device__ __forceinline__ void to_lds(unsigned char *tile, float *z, int l32, int g) const {
+        typedef T t4 __attribute__((ext_vector_type(4)));
+        const int row = 32 * eb + l32;
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            if (valid(i)) {
+                unsigned char *t = tile + i * 64 * 256;  // (block p + 4 i: block p of tile i)
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    t4 w;
+#pragma unroll
+                    for (int b = 0; b < 4; ++b) w[b] = static_cast<T>(st[i][4 * a + b]);
+                    *reinterpret_cast<t4 *>(t + row * 256 + (((4 * p + a) ^ walk_swizzle<16>(row)) << 4) + 8 * g) = w;
+                }
+            }
+        if (NORM && fx < PolyFeatures::kBlocks && l32 == 0) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                *reinterpret_cast<f32x4 *>(z + 32 * fx + 8 * a + 4 * g) = f32x4{ex[4 * a], ex[4 * a + 1], ex[4 * a + 2], ex[4 * a + 3]};
+        }
+    }
+    // += (NEG: -=) phi^T [z tile, extra column] over the chunk's 128 rows.  extra: that column as 128 values of the storage
+    // type in LDS, 256 bytes of zeros behind them (null: ones) -- lanes other than l32 == 0 read the zeros, so that
+    // no VALU instruction is spent on the fragment.
+    template <typename T, bool NORM, bool NEG>
+    __device__ __forceinline__ void update(const unsigned char *phi0, const unsigned char *phi1, const unsigned char *zt,
+                                           const unsigned char *extra, int lane) {
+        using M = Mma<T>;
+        using V8 = typename M::V8;
+        const int l32 = lane & 31, g = lane >> 5;
+        auto signed_frag = [&](V8 z) {
+            if constexpr (NEG) {
+                u32x4 raw = __builtin_bit_cast(u32x4, z);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) raw[e] ^= 0x80008000u;
+                z = __builtin_bit_cast(V8, raw);
+            }
+            return z;
+        };
+        // (no branch in the loop: the wave whose second block does not exist multiplies block p of the first tile twice)
+        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+        const unsigned char *column = extra + (l32 == 0 ? 0 : 256) + 8 * g;
+        float one[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) one[j] = l32 == 0 ? (NEG ? -1.f : 1.f) : 0.f;
+        const V8 ones = poly_round8<T>(one);
+        const unsigned char *second = valid(1) ? phi1 : phi0;
+        const PolyPair za = poly_col_base<128>(lane, eb), ya = poly_col_base<256>(lane, p);
+        V8 zf = {}, y0 = {};
+        walk_pipe<8 * 3, 6, V8>(
+            [&](auto j) {
+                constexpr int ks = decltype(j)::value / 3, r = decltype(j)::value % 3;
+                if constexpr (r == 0)
+                    return signed_frag(poly_tr<T>(zt + 16 * 128 * ks, za));
+                else
+                    return poly_tr<T>((r == 1 ? phi0 : second) + 16 * 256 * ks, ya);
+            },
+            [&](auto j, V8 f) {
+                constexpr int ks = decltype(j)::value / 3, r = decltype(j)::value % 3;
+                if constexpr (r == 0) {
+                    zf = f;
+                } else if constexpr (r == 1) {
+                    y0 = f;
+                    st[0] = M::mma(f, zf, st[0]);
+                } else {
+                    st[1] = M::mma(f, zf, st[1]);
+                    if constexpr (NORM) {
+                        V8 ef = ones;
+                        if (extra) {
+                            const u32x2 lo = *reinterpret_cast<const u32x2 *>(column + 32 * ks);
+                            const u32x2 hi = *reinterpret_cast<const u32x2 *>(column + 32 * ks + 16);
+                            ef = signed_frag(__builtin_bit_cast(V8, u32x4{lo[0], lo[1], hi[0], hi[1]}));
+                        }
+                        const u32x4 a = __builtin_bit_cast(u32x4, y0), c = __builtin_bit_cast(u32x4, f);
+                        const u32x4 y = eb == 0 ? a : c;
+                        ex = M::mma(__builtin_bit_cast(V8, y), ef, ex);
+                    }
+                }
+            });
+    }
+};
+
+// The lane's number as a value the compiler cannot follow out of the chunk loop: LDS addresses that depend on the lane alone
+// would all be computed ahead of it and held in registers (dozens of them, to the point of spilling).
+__device__ __forceinline__ int poly_opaque(int lane) {
+    asm volatile("" : "+v"(lane));
+    return lane;
+}
+
+struct PolySlice {
+    int bh, seg, c_lo, c_hi;
+    bool valid;
+};
+__device__ __forceinline__ PolySlice poly_slice(const PolyWalkParams &p) {  // (walk_slice's map)
+    const int wg = blockIdx.x, xcd = wg & 7, slot = wg >> 3;
+    const int hl = slot / p.n_seg, seg = slot - hl * p.n_seg;
+    PolySlice s;
+    s.bh = hl * 8 + xcd, s.seg = seg;
+    s.c_lo = seg * p.seg_chunks;
+    s.c_hi = s.c_lo + p.seg_chunks < p.n_chunks ? s.c_lo + p.seg_chunks : p.n_chunks;
+    s.valid = s.bh < p.BH && s.c_lo < p.n_chunks;
+    return s;
+}
+
+// A chunk's rows on their way to LDS, in registers: an x operand (two of them: threads 0 .. 255 and 256 .. 511 take one
+// each), tiles of 64 columns, and -- for dO -- forward's result and n.
+template <typename T>
+__device__ __forceinline__ u32x4 poly_fetch_x(const T *base, int64_t stride, int row0, int N, int r, int tid) {
+    const int row = row0 + (tid & 127), half = (tid >> 7) & 1;
+    u32x4 v = {0u, 0u, 0u, 0u};
+    if (row < N && 8 * half < r) v = *reinterpret_cast<const u32x4 *>(base + (int64_t)row * stride + 8 * half);
+    return v;
+}
+__device__ __forceinline__ void poly_put_x(unsigned char *xt, u32x4 v, int tid) {
+    *reinterpret_cast<u32x4 *>(xt + (tid & 127) * 32 + ((tid >> 7) & 1) * 16) = v;
+}
+__device__ __forceinline__ void poly_put_xt(unsigned char *xtr, u32x4 v, int tid) {  // the transposed copy
+    const int row = tid & 127, half = (tid >> 7) & 1;
+#pragma unroll
+    for (int j = 0; j < 8; ++j)
+        *reinterpret_cast<uint16_t *>(xtr + (8 * half + j) * 272 + row * 2) = (uint16_t)(v[j / 2] >> (16 * (j & 1)));
+}
+template <typename T>
+struct PolyTile {
+    u32x4 v[2];
+    __device__ __forceinline__ void fetch(const T *base, int64_t stride, int row0, int N, int width, int tid) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int u = tid + 512 * i, row = row0 + (u >> 3), ch = u & 7;
+            v[i] = u32x4{0u, 0u, 0u, 0u};
+            if (row < N && ch * 8 < width) v[i] = *reinterpret_cast<const u32x4 *>(base + (int64_t)row * stride + ch * 8);
+        }
+    }
+    __device__ __forceinline__ void put(unsigned char *tile, int tid) const {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int u = tid + 512 * i, row = u >> 3, ch = u & 7;
+            *reinterpret_cast<u32x4 *>(tile + row * 128 + ((ch ^ walk_swizzle<8>(row)) << 4)) = v[i];
+        }
+    }
+};
+// dO, with the normaliser forward's result and n beside it: put() writes g = dO / n and dn = -(dO . O) / n
+template <typename T, bool NORM>
+struct PolyGrad {
+    PolyTile<T> g, o;
+    float n[2];
+    __device__ __forceinline__ void fetch(const T *go, int64_t gstride, const T *out, int64_t ostride, const float *denom, int row0,
+                                          int N, int width, int tid) {
+        g.fetch(go, gstride, row0, N, width, tid);
+        if constexpr (NORM) {
+            o.fetch(out, ostride, row0, N, width, tid);
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = row0 + ((tid + 512 * i) >> 3);
+                n[i] = row < N ? denom[row] : 1.f;
+            }
+        }
+    }
+    // (dn: in fp32, and rounded behind that: PolyLds::DN)
+    __device__ __forceinline__ void put(unsigned char *tile, float *dn, int tid) {
+        using V8 = typename Mma<T>::V8;
+        if constexpr (NORM) {
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const V8 a = __builtin_bit_cast(V8, g.v[i]), b = __builtin_bit_cast(V8, o.v[i]);
+                const float inv = 1.0f / n[i];
+                float dot = 0.f, f[8];
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    dot += static_cast<float>(a[j]) * static_cast<float>(b[j]);
+                    f[j] = static_cast<float>(a[j]) * inv;
+                }
+                g.v[i] = __builtin_bit_cast(u32x4, poly_round8<T>(f));
+                dot += __shfl_xor(dot, 1, 64);
+                dot += __shfl_xor(dot, 2, 64);
+                dot += __shfl_xor(dot, 4, 64);
+                if ((tid & 7) == 0) {
+                    // (one rounded value for every use, as the quadratic evaluation's bias column holds it)
+                    const T r = static_cast<T>(-dot * inv);
+                    dn[(tid + 512 * i) >> 3] = static_cast<float>(r);
+                    reinterpret_cast<T *>(dn + PolyLds::C)[(tid + 512 * i) >> 3] = r;
+                }
+            }
+        }
+        g.put(tile, tid);
+    }
+};
+
+// one accumulator block per wave through LDS: 4 KiB each, written and read in lane order
+__device__ __forceinline__ void poly_put_acc(unsigned char *ex, int wave, int lane, const f32x16 &v) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+        *reinterpret_cast<f32x4 *>(ex + (wave * 4 + a) * 1024 + lane * 16) = f32x4{v[4 * a], v[4 * a + 1], v[4 * a + 2], v[4 * a + 3]};
+}
+__device__ __forceinline__ void poly_get_acc(const unsigned char *ex, int wave, int lane, f32x16 &v) {
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        const f32x4 t = *reinterpret_cast<const f32x4 *>(ex + (wave * 4 + a) * 1024 + lane * 16);
+#pragma unroll
+        for (int b = 0; b < 4; ++b) v[4 * a + b] = t[b];
+    }
+}
+
+// sixteen consecutive columns (from column `col`) of a row, rounded and stored as two chunks
+template <typename T>
+__device__ __forceinline__ void poly_store16(T *dst, const float (&f)[16], int col, int width) {
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+        if (col + 8 * h < width) {
+            float e[8];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) e[j] = f[8 * h + j];
+            *reinterpret_cast<u32x4 *>(dst + col + 8 * h) = __builtin_bit_cast(u32x4, poly_round8<T>(e));
+        }
+}
+
+// ---- sums of phi(k) [v, 1]^T (BWD: phi(q) [g, dn]^T) over every segment but the last (the first)
+template <typename T, bool NORM, bool BWD>
+__global__ __launch_bounds__(512, 2) void poly_totals_kernel(const PolyWalkParams p) {
+#if defined(__gfx950__)
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    using L = PolyLds;
+    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const PolySlice sl = poly_slice(p);
+    if (!sl.valid || sl.seg == (BWD ? 0 : p.n_seg - 1)) return;
+    const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
+    const T *X = BWD ? static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h : static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
+    const int64_t xs = BWD ? p.qs_n : p.ks_n;
+    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
+    const T *G = BWD ? static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h : nullptr;
+    const T *O = BWD && NORM ? static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h : nullptr;
+    const float *n = NORM && BWD ? p.denom + (int64_t)sl.bh * N : nullptr;
+    float *dn = reinterpret_cast<float *>(smem + L::tDn);
+    PolyState s;
+    s.clear(wave);
+    u32x4 x = {0u, 0u, 0u, 0u};
+    PolyTile<T> v;
+    PolyGrad<T, NORM> go;
+    auto fetch = [&](int c) {
+        const int row0 = c * L::C;
+        if (tid < 256) x = poly_fetch_x<T>(X, xs, row0, N, p.r, tid);
+        if constexpr (BWD)
+            go.fetch(G, p.gs_n, O, p.os_n, n, row0, N, p.wv, tid);
+        else
+            v.fetch(V, p.vs_n, row0, N, p.wv, tid);
+    };
+    if (BWD && tid < 64) reinterpret_cast<uint32_t *>(smem + L::tDn + L::C * 6)[tid] = 0u;
+    fetch(sl.c_lo);
+#pragma unroll 1
+    for (int c = sl.c_lo; c < sl.c_hi; ++c) {
+        __syncthreads();
+        if (tid < 256) poly_put_x(smem + L::tX, x, tid);
+        if constexpr (BWD)
+            go.put(smem + L::tV, dn, tid);
+        else
+            v.put(smem + L::tV, tid);
+        if (c + 1 < sl.c_hi) fetch(c + 1);
+        __syncthreads();
+        poly_gen_phi<T>(smem + L::tX, smem + L::tPhi, smem + L::tPhi + L::PHI, c * L::C, N, tid);
+        __syncthreads();
+        s.template update<T, NORM, false>(smem + L::tPhi, smem + L::tPhi + L::PHI, smem + L::tV,
+                                             BWD ? smem + L::tDn + L::C * 4 : nullptr, lane);
+    }
+    s.template store<NORM>(p.totals + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, l32, g);
+#else
+    (void)p;
+#endif
+}
+
+// entry states from totals, in place: entry[s] = sum over f < s (reverse: f > s); the loads of eight segments together
+// (a template only so that the header can be included by several translation units)
+template <int kUnused = 0>
+__global__ __launch_bounds__(256) void poly_scan_kernel(float *totals, int n_seg, int64_t total, int reverse) {
+    const int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total) return;
+    const int64_t bh = i / PolyFeatures::kState, e = i - bh * PolyFeatures::kState;
+    float *at = totals + (bh * n_seg + (reverse ? n_seg - 1 : 0)) * PolyFeatures::kState + e;
+    const int64_t step = reverse ? -(int64_t)PolyFeatures::kState : (int64_t)PolyFeatures::kState;
+    float run = 0.f;
+    for (int s = 0; s < n_seg; s += 8) {
+        float t[8];
+#pragma unroll
+        for (int u = 0; u < 8; ++u) t[u] = s + u < n_seg - 1 ? at[(s + u) * step] : 0.f;  // (the last one's is not needed)
+#pragma unroll
+        for (int u = 0; u < 8; ++u)
+            if (s + u < n_seg) {
+                at[(s + u) * step] = run;
+                run += t[u];
+            }
+    }
+}
+
+// the entry state of a segment: zeros, one state in memory, or the sum of the totals before (after) it
+template <bool NORM>
+__device__ __forceinline__ void poly_entry(const PolyWalkParams &p, const PolySlice &sl, bool reverse, int l32, int g, PolyState &s) {
+    if (!p.totals) return;
+    const float *base = p.totals + (int64_t)sl.bh * p.n_seg * PolyFeatures::kState;
+    if (!p.sum_entries) {
+        s.template add<NORM>(base + (int64_t)sl.seg * PolyFeatures::kState, l32, g);
+        return;
+    }
+    const int lo = reverse ? sl.seg + 1 : 0, hi = reverse ? p.n_seg : sl.seg;
+#pragma unroll 1
+    for (int f = lo; f < hi; ++f) s.template add<NORM>(base + (int64_t)f * PolyFeatures::kState, l32, g);
+}
+
+template <typename T, bool NORM>
+__global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkParams p) {
+#if defined(__gfx950__)
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    using L = PolyLds;
+    using M = Mma<T>;
+    using V8 = typename M::V8;
+    const int tid0 = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6), rb = wave & 3, kh = wave >> 2;
+    const PolySlice sl = poly_slice(p);
+    if (!sl.valid) return;
+    const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
+    const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
+    const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
+    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
+    T *O = static_cast<T *>(p.out) + b * p.us_b + h * p.us_h;
+    const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
+    unsigned char *tq = smem + L::fQ, *tk = smem + L::fK, *tv = smem + L::fV, *ts = smem + L::fS, *phi0 = smem + L::fPhi,
+                  *phi1 = phi0 + L::PHI;
+    float *z = reinterpret_cast<float *>(smem + L::fZ), *sums = reinterpret_cast<float *>(smem + L::fSum);
+    unsigned char *exch = smem + L::fEx;
+    PolyState s;
+    s.clear(wave);
+    poly_entry<NORM>(p, sl, false, tid0 & 31, (tid0 & 63) >> 5, s);
+    u32x4 x;
+    PolyTile<T> v;
+    auto fetch = [&](int c, int tid) {
+        const int row0 = c * L::C;
+        x = tid < 256 ? poly_fetch_x<T>(Q, p.qs_n, row0, N, p.r, tid) : poly_fetch_x<T>(K, p.ks_n, row0, N, p.r, tid);
+        v.fetch(V, p.vs_n, row0, N, p.wv, tid);
+    };
+    fetch(sl.c_lo, tid0);
+#pragma unroll 1
+    for (int c = sl.c_lo; c < sl.c_hi; ++c) {
+        const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+        __syncthreads();
+        poly_put_x(tid < 256 ? tq : tk, x, tid);
+        v.put(tv, tid);
+        s.template to_lds<T, NORM>(ts, z, l32, g);
+        if (c + 1 < sl.c_hi) fetch(c + 1, tid);
+        __syncthreads();
+        poly_gen_phi<T>(tk, phi0, phi1, c * L::C, N, tid);
+
+        const int trow = 32 * rb + l32, row = c * L::C + trow;
+        f32x16 acc[2];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
+        float rsum = 0.f;
+        if (c > 0) {  // phi_w(q) T, this half of the features
+            float xr[16], xs[8];
+            poly_row<T>(tq, trow, xr);
+#pragma unroll
+            for (int j = 0; j < 8; ++j) xs[j] = poly_pick(g, xr[8 + j], xr[j]);
+            const uint32_t sa = poly_row_base<256>(walk_e_lane(l32), g);
+            auto step = [&](auto ksc) {
+                constexpr int KS = decltype(ksc)::value;
+                float raw[8];
+                const V8 f = poly_feature_frag<T, KS>(xr, xs, g, c0, c1, c2, raw);
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    acc[e] = M::mma(poly_rd<T>(ts + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5)), f, acc[e]);
+                if constexpr (NORM) {
+#pragma unroll
+                    for (int a = 0; a < 2; ++a) {
+                        const f32x4 zz = *reinterpret_cast<const f32x4 *>(z + 16 * KS + 8 * g + 4 * a);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) rsum += raw[4 * a + j] * zz[j];
+                    }
+                }
+            };
+            constexpr int H = PolyFeatures::kSteps / 2;
+            if (kh == 0) {
+                static_for<0, H>(step);
+                asm volatile("; first half of the features");
+            } else {
+                static_for<H, 2 * H>(step);
+                asm volatile("; second half of the features");
+            }
+        }
+        const V8 xq = poly_row_frag<T>(tq, trow, g);
+        const PolyPair va = poly_perm_base<128, false>(lane);
+#pragma unroll 1
+        for (int sb = kh; sb <= rb; sb += 2) {  // every other block of the chunk's scores
+            // (the mask as bits, not a branch: see fla_tri_pair.h on scores and branches)
+            const uint32_t all = sb < rb ? ~0u : 0u;
+            f32x16 sc;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) sc[i] = 0.f;
+            sc = M::mma(poly_row_frag<T>(tk, 32 * sb + l32, g), xq, sc);
+            float u[16];
+            V8 pf[2];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const float t = c0 + sc[i] * (c1 + c2 * sc[i]);
+                if constexpr (NORM) {
+                    u[i] = __builtin_bit_cast(float, __builtin_bit_cast(uint32_t, t) & (poly_mask<false>(i, l32, g) | all));
+                    rsum += u[i];
+                } else {
+                    u[i] = t;
+                }
+            }
+            poly_round_masked<T, false>(u, NORM ? ~0u : all, l32, g, pf);
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    acc[e] = M::mma(poly_tr<T>(tv + 128 * (32 * sb + 16 * t), va, e << 6), pf[t], acc[e]);
+        }
+        // each of the two waves of these rows finishes one half of the columns: the other half's sums go to the other wave
+        {
+            f32x16 mine;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mine[i] = poly_pick(kh, acc[0][i], acc[1][i]);
+            poly_put_acc(exch, wave, lane, mine);
+        }
+        if constexpr (NORM) {
+            rsum += __shfl_xor(rsum, 32, 64);
+            if (g == 0) sums[kh * L::C + trow] = rsum;
+        }
+        __syncthreads();
+        if (c + 1 < sl.c_hi || p.ends) s.template update<T, NORM, false>(phi0, phi1, tv, nullptr, lane);
+        f32x16 other;
+        poly_get_acc(exch, wave ^ 4, lane, other);
+        float f[16], inv = 1.f;
+        if constexpr (NORM) {
+            const float n = sums[trow] + sums[L::C + trow] + p.eps;
+            inv = 1.0f / n;
+            if (kh == 0 && g == 0 && row < N) p.denom[(int64_t)sl.bh * N + row] = n;
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) f[i] = (poly_pick(kh, acc[1][i], acc[0][i]) + other[i]) * inv;
+        if (row < N) poly_store16<T>(O + (int64_t)row * p.us_n, f, 32 * kh + 16 * g, p.wv);
+    }
+    if (p.ends) s.template store<NORM>(p.ends + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
+#else
+    (void)p;
+#endif
+}
+
+// dx += the gradient at x of phi_w(x) . (S [g, extra]): H = S g for the row's 224 features, contracted with the row.
+// S: the rounded state's tiles; gf: the row's g (v) as operands; z, extra: the state's last column and its factor.
+// Returns this lane's part of it (the other part is in the lane of the other g) in dx.
+template <typename T, bool NORM>
+__device__ __forceinline__ void poly_contract(const unsigned char *S, const float *z, float extra, const typename Mma<T>::V8 (&gf)[4],
+                                              const float (&x)[16], int lane, float c1, float c2, float (&quad)[16]) {
+    using M = Mma<T>;
+    const int g = lane >> 5;
+    const PolyPair sa = poly_perm_base<256, true>(lane);
+    static_for<0, PolyFeatures::kBlocks>([&](auto fbc) {
+        constexpr int FB = decltype(fbc)::value;
+        f32x16 hh;
+#pragma unroll
+        for (int a = 0; a < 4; ++a) {
+            f32x4 zz = {0.f, 0.f, 0.f, 0.f};
+            if constexpr (NORM) zz = *reinterpret_cast<const f32x4 *>(z + 32 * FB + 16 * g + 4 * a);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) hh[4 * a + j] = NORM ? zz[j] * extra : 0.f;
+        }
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc)
+            hh = M::mma(poly_tr<T>(S + (FB >> 2) * 64 * 256 + 16 * 256 * kc, sa, (FB & 3) << 6), gf[kc], hh);
+        // hh[v]: feature 32 FB + 16 g + v
+        if constexpr (FB < 2) {  // two groups x_r x_(0..7), r = 4 FB + 2 g and the next
+            float t[2] = {0.f, 0.f};
+#pragma unroll
+            for (int e = 0; e < 2; ++e)
+#pragma unroll
+                for (int j = 0; j < 8; ++j) t[e] += hh[8 * e + j] * x[j];
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                quad[4 * FB + e] += poly_pick(g, 0.f, t[e]);
+                quad[4 * FB + 2 + e] += poly_pick(g, t[e], 0.f);
+            }
+        } else if constexpr (FB < 6) {  // x_r x_(0..15), r = 8 + 2 (FB - 2) + g
+            constexpr int R = 8 + 2 * (FB - 2);
+            float t = 0.f;
+            const float xr = poly_pick(g, x[R + 1], x[R]);
+#pragma unroll
+            for (int j = 0; j < 16; ++j) t += hh[j] * x[j];
+#pragma unroll
+            for (int j = 0; j < 8; ++j) quad[j] += hh[j] * xr;
+            quad[R] += poly_pick(g, 0.f, t);
+            quad[R + 1] += poly_pick(g, t, 0.f);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 16; ++j) quad[j] = 2.f * c2 * quad[j] + poly_pick(g, 0.f, c1 * hh[j]);
+        }
+        if constexpr (FB % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // (two blocks at a time: registers)
+    });
+}
+
+template <typename T, bool NORM>
+__global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkParams p) {
+#if defined(__gfx950__)
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    using L = PolyLds;
+    using M = Mma<T>;
+    using V8 = typename M::V8;
+    const int tid0 = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6), rb = wave & 3, half = wave >> 2;
+    const PolySlice sl = poly_slice(p);
+    if (!sl.valid) return;
+    const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
+    const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
+    const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
+    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
+    const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
+    const T *O = NORM ? static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h : nullptr;
+    const float *den = NORM ? p.denom + (int64_t)sl.bh * N : nullptr;
+    T *dQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h;
+    T *dK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h;
+    T *dV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
+    const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
+    unsigned char *tq = smem + L::bQ, *tk = smem + L::bK, *tqt = smem + L::bQt, *tkt = smem + L::bKt, *tv = smem + L::bV,
+                  *tg = smem + L::bG, *us = smem + L::bU, *phi0 = smem + L::bPhi, *ts = smem + L::bT;
+    float *z = reinterpret_cast<float *>(smem + L::bZ), *y = reinterpret_cast<float *>(smem + L::bY),
+          *dn = reinterpret_cast<float *>(smem + L::bDn);
+    PolyState st, su;
+    st.clear(wave), su.clear(wave);
+    st.template add<NORM>(p.ends + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
+    poly_entry<NORM>(p, sl, true, tid0 & 31, (tid0 & 63) >> 5, su);
+    u32x4 x;
+    PolyTile<T> v;
+    PolyGrad<T, NORM> go;
+    auto fetch = [&](int c, int tid) {
+        const int row0 = c * L::C;
+        x = tid < 256 ? poly_fetch_x<T>(Q, p.qs_n, row0, N, p.r, tid) : poly_fetch_x<T>(K, p.ks_n, row0, N, p.r, tid);
+        v.fetch(V, p.vs_n, row0, N, p.wv, tid);
+        go.fetch(G, p.gs_n, O, p.os_n, den, row0, N, p.wv, tid);
+    };
+    if (tid0 < 64) reinterpret_cast<uint32_t *>(smem + L::bDn + L::C * 6)[tid0] = 0u;
+    fetch(sl.c_hi - 1, tid0);
+#pragma unroll 1
+    for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
+        const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+        const bool before = c > 0, after = c + 1 < p.n_chunks;  // (T, U of this chunk hold anything)
+        __syncthreads();
+        poly_put_x(tid < 256 ? tq : tk, x, tid);
+        poly_put_xt(tid < 256 ? tqt : tkt, x, tid);
+        v.put(tv, tid);
+        go.put(tg, dn, tid);
+        if (after) su.template to_lds<T, NORM>(us, y, l32, g);
+        if (c > sl.c_lo) fetch(c - 1, tid);
+        __syncthreads();
+        if (before) {  // T <- T - this chunk's phi(k) [v, 1]^T
+            poly_gen_phi<T>(tk, phi0, ts, c * L::C, N, tid);
+            __syncthreads();
+            st.template update<T, NORM, true>(phi0, ts, tv, nullptr, lane);
+            __syncthreads();
+            st.template to_lds<T, NORM>(ts, z, l32, g);
+            __syncthreads();
+        }
+
+        const int trow = 32 * rb + l32, row = c * L::C + trow;
+        const V8 xk = poly_row_frag<T>(tk, trow, g);
+        const uint32_t ra = poly_row_base<128>(l32, g);
+        const int rc = walk_e_lane(l32) & 15;  // (columns 16 .. of the 32-wide blocks of dq, dk are not used)
+        float dxs[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dxs[i] = 0.f;
+        f32x16 dx;
+        if (half == 0) {  // dq
+            V8 gf[4];
+#pragma unroll
+            for (int kc = 0; kc < 4; ++kc) gf[kc] = poly_rd<T>(tg + 32 * 128 * rb, ra ^ (kc << 5));
+            const V8 xq = poly_row_frag<T>(tq, trow, g);
+            const float dni = NORM ? dn[trow] : 0.f;
+            if (before) {
+                float xr[16];
+                poly_row<T>(tq, trow, xr);
+                poly_contract<T, NORM>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dx[i] = 0.f;
+#pragma unroll 1
+            for (int sb = 0; sb <= rb; ++sb) {
+                const uint32_t all = sb < rb ? ~0u : 0u;
+                f32x16 m, u;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) m[i] = dni, u[i] = 0.f;
+                u = M::mma(poly_row_frag<T>(tk, 32 * sb + l32, g), xq, u);
+#pragma unroll
+                for (int kc = 0; kc < 4; ++kc) m = M::mma(poly_rd<T>(tv + 32 * 128 * sb, ra ^ (kc << 5)), gf[kc], m);
+                V8 df[2];
+                float d[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) d[i] = m[i] * (c1 + 2.f * c2 * u[i]);
+                poly_round_masked<T, false>(d, all, l32, g, df);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(tkt, rc, 32 * sb + 16 * t, g), df[t], dx);
+            }
+        } else {  // dk
+            V8 vf[4];
+#pragma unroll
+            for (int kc = 0; kc < 4; ++kc) vf[kc] = poly_rd<T>(tv + 32 * 128 * rb, ra ^ (kc << 5));
+            if (after) {
+                float xr[16];
+                poly_row<T>(tk, trow, xr);
+                poly_contract<T, NORM>(us, y, 1.f, vf, xr, lane, c1, c2, dxs);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dx[i] = 0.f;
+#pragma unroll 1
+            for (int sb = rb; sb < 4; ++sb) {
+                const uint32_t all = sb > rb ? ~0u : 0u;
+                f32x16 m, u;
+#pragma unroll
+                for (int a = 0; a < 4; ++a) {
+                    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+                    if constexpr (NORM) d = *reinterpret_cast<const f32x4 *>(dn + 32 * sb + 8 * a + 4 * g);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) m[4 * a + j] = d[j], u[4 * a + j] = 0.f;
+                }
+                u = M::mma(poly_row_frag<T>(tq, 32 * sb + l32, g), xk, u);
+#pragma unroll
+                for (int kc = 0; kc < 4; ++kc) m = M::mma(poly_rd<T>(tg + 32 * 128 * sb, ra ^ (kc << 5)), vf[kc], m);
+                V8 df[2];
+                float d[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) d[i] = m[i] * (c1 + 2.f * c2 * u[i]);
+                poly_round_masked<T, true>(d, all, l32, g, df);
+#pragma unroll
+                for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(tqt, rc, 32 * sb + 16 * t, g), df[t], dx);
+            }
+        }
+        {
+            float f[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                f[i] = dxs[i] + __shfl_xor(dxs[i], 32, 64) + dx[i];  // (lanes of g = 0 hold the block's columns 0 .. 15)
+            }
+            T *to = half == 0 ? dQ + (int64_t)row * p.dqs_n : dK + (int64_t)row * p.dks_n;
+            if (row < N && g == 0) poly_store16<T>(to, f, 0, p.r);
+        }
+        // dV: the dq waves form phi_w(k) U, the dk waves the chunk's own part; each finishes one half of the columns
+        f32x16 acc[2];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
+        if (half == 0) {
+            if (after) {
+                float xr[16], xs[8];
+                poly_row<T>(tk, trow, xr);
+#pragma unroll
+                for (int j = 0; j < 8; ++j) xs[j] = poly_pick(g, xr[8 + j], xr[j]);
+                const uint32_t sa = poly_row_base<256>(walk_e_lane(l32), g);
+                static_for<0, PolyFeatures::kSteps>([&](auto ksc) {
+                    constexpr int KS = decltype(ksc)::value;
+                    float raw[8];
+                    const V8 f = poly_feature_frag<T, KS>(xr, xs, g, c0, c1, c2, raw);
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        acc[e] = M::mma(poly_rd<T>(us + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5)), f, acc[e]);
+                });
+            }
+            asm volatile("; dV, the rows after");
+        } else {
+            const PolyPair ga = poly_perm_base<128, false>(lane);
+#pragma unroll 1
+            for (int sb = rb; sb < 4; ++sb) {
+                const uint32_t all = sb > rb ? ~0u : 0u;
+                f32x16 u;
+#pragma unroll
+                for (int i = 0; i < 16; ++i) u[i] = 0.f;
+                u = M::mma(poly_row_frag<T>(tq, 32 * sb + l32, g), xk, u);
+                V8 pf[2];
+                float f[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) f[i] = c0 + u[i] * (c1 + c2 * u[i]);
+                poly_round_masked<T, true>(f, all, l32, g, pf);
+#pragma unroll
+                for (int t = 0; t < 2; ++t)
+#pragma unroll
+                    for (int e = 0; e < 2; ++e)
+                        acc[e] = M::mma(poly_tr<T>(tg + 128 * (32 * sb + 16 * t), ga, e << 6), pf[t], acc[e]);
+            }
+            asm volatile("; dV, the chunk's own rows");
+        }
+        __syncthreads();
+        {
+            f32x16 mine;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) mine[i] = poly_pick(half, acc[0][i], acc[1][i]);
+            poly_put_acc(us, wave, lane, mine);  // (U's copy has been read)
+        }
+        if (c > sl.c_lo) poly_gen_phi<T>(tq, phi0, ts, c * L::C, N, tid);
+        __syncthreads();
+        {
+            f32x16 other;
+            poly_get_acc(us, wave ^ 4, lane, other);
+            float f[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) f[i] = poly_pick(half, acc[1][i], acc[0][i]) + other[i];
+            if (row < N) poly_store16<T>(dV + (int64_t)row * p.dvs_n, f, 32 * half + 16 * g, p.wv);
+        }
+        // U <- U + this chunk's phi(q) [g, dn]^T
+        if (c > sl.c_lo) su.template update<T, NORM, false>(phi0, ts, tg, smem + L::bDn + L::C * 4, lane);
+    }
+#else
+    (void)p;
+#endif
+}
+
+template <auto kern>
+hipError_t launch_poly_kernel(const PolyWalkParams &p, int smem, hipStream_t stream) {
+    const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
+    if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+    if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
+    return launch_kernel<kern>(dim3((unsigned)grid), dim3(512), smem, stream, p);
+}
+
+template <typename T>
+hipError_t launch_poly_totals(const PolyWalkParams &p, bool bwd, hipStream_t stream) {
+    if (bwd)
+        return p.denom ? launch_poly_kernel<poly_totals_kernel<T, true, true>>(p, PolyLds::tTotal, stream)
+                       : launch_poly_kernel<poly_totals_kernel<T, false, true>>(p, PolyLds::tTotal, stream);
+    return p.denom ? launch_poly_kernel<poly_totals_kernel<T, true, false>>(p, PolyLds::tTotal, stream)
+                   : launch_poly_kernel<poly_totals_kernel<T, false, false>>(p, PolyLds::tTotal, stream);
+}
+
+template <typename T>
+hipError_t launch_poly_walk(const PolyWalkParams &p, bool bwd, hipStream_t stream) {
+    if (bwd)
+        return p.denom ? launch_poly_kernel<poly_walk_bwd_kernel<T, true>>(p, PolyLds::bTotal, stream)
+                       : launch_poly_kernel<poly_walk_bwd_kernel<T, false>>(p, PolyLds::bTotal, stream);
+    return p.denom ? launch_poly_kernel<poly_walk_fwd_kernel<T, true>>(p, PolyLds::fTotal, stream)
+                   : launch_poly_kernel<poly_walk_fwd_kernel<T, false>>(p, PolyLds::fTotal, stream);
+}
+
+inline hipError_t launch_poly_scan(float *totals, int64_t BH, int n_seg, int reverse, hipStream_t stream) {
+    const int64_t total = BH * PolyFeatures::kState;
+    return launch_kernel<poly_scan_kernel<0>>(dim3((unsigned)((total + 255) / 256)), dim3(256), 0, stream, totals, n_seg, total,
+                                              reverse);
+}
+
+}  // namespace fla

@@ -259,28 +259,49 @@ struct Poly {
     float eps;
 };
 
-std::tuple<Tensor, Tensor> poly_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Poly &p) {
+struct PolyResult {
+    Tensor o, denom, state;  // state: of the chunk-wise evaluation, for its backward
+};
+
+PolyResult poly_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, const Poly &p, bool want_state) {
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor q = dense(q_), k = dense(k_), v = dense(v_);
     const Call c(q, v);
-    Tensor o = c.rows(c.dv), denom;
-    if (p.normalise) denom = c.row_floats();
-    must(fla_poly_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(o), static_cast<float *>(ptr(denom)), c.b, c.h, c.n, c.dqk, c.dv, str(q),
-                           str(k), str(v), str(o), p.c, p.eps, c.dtype, c.stream));
-    return {o, denom};
+    PolyResult r;
+    r.o = c.rows(c.dv);
+    if (p.normalise) r.denom = c.row_floats();
+    float *n = static_cast<float *>(ptr(r.denom));
+    if (fla_poly_attn_prefers_chunked(c.b, c.h, c.n, c.dqk, c.dv, c.dtype, want_state)) {
+        if (want_state) r.state = c.bytes(fla_poly_attn_chunked_state_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        const Tensor work = c.bytes(fla_poly_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        must(fla_poly_attn_chunked_fwd(ptr(q), ptr(k), ptr(v), ptr(r.o), n, c.b, c.h, c.n, c.dqk, c.dv, str(q), str(k), str(v),
+                                       str(r.o), p.c, p.eps, c.dtype, ptr(r.state), ptr(work), size_of(work), c.stream));
+    } else {
+        must(fla_poly_attn_fwd(ptr(q), ptr(k), ptr(v), ptr(r.o), n, c.b, c.h, c.n, c.dqk, c.dv, str(q), str(k), str(v), str(r.o),
+                               p.c, p.eps, c.dtype, c.stream));
+    }
+    return r;
 }
 
 variable_list poly_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &o,
-                       const Tensor &denom, const Poly &p) {
+                       const Tensor &denom, const Tensor &state, const Poly &p) {
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor go = dense(go_), q = dense(q_), k = dense(k_), v = dense(v_);
     const Call c(q, v);
     Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
-    const Tensor work = c.bytes(fla_poly_attn_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-    must(fla_poly_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), static_cast<const float *>(ptr(denom)), ptr(dq), ptr(dk),
-                           ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go), str(q), str(k), str(v),
-                           o.defined() ? str(o) : nullptr, str(dq), str(dk), str(dv), p.c, c.dtype, ptr(work), size_of(work),
-                           c.stream));
+    const float *n = static_cast<const float *>(ptr(denom));
+    const int64_t *os = o.defined() ? str(o) : nullptr;
+    if (state.defined()) {
+        const Tensor work = c.bytes(fla_poly_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        must(fla_poly_attn_chunked_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n,
+                                       c.dqk, c.dv, str(go), str(q), str(k), str(v), os, str(dq), str(dk), str(dv), p.c, c.dtype,
+                                       ptr(state), ptr(work), size_of(work), c.stream));
+    } else {
+        const Tensor work = c.bytes(fla_poly_attn_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        must(fla_poly_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
+                               str(go), str(q), str(k), str(v), os, str(dq), str(dk), str(dv), p.c, c.dtype, ptr(work),
+                               size_of(work), c.stream));
+    }
     return {dq, dk, dv};
 }
 
@@ -288,20 +309,21 @@ struct Polynomial : Function<Polynomial> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, double c0, double c1,
                           double c2, bool normalise, double eps, bool cast) {
         const Tensor q = cast_to(q_, cast), k = cast_to(k_, cast), v = cast_to(v_, cast);
-        auto [o, denom] = poly_fwd(q, k, v, Poly{{(float)c0, (float)c1, (float)c2}, normalise, (float)eps});
-        ctx->saved_data["c0"] = c0, ctx->saved_data["c1"] = c1, ctx->saved_data["c2"] = c2;
-        if (normalise)
-            ctx->save_for_backward({q, k, v, o, denom});
-        else
-            ctx->save_for_backward({q, k, v});
-        return o;
+        PolyResult r = poly_fwd(q, k, v, Poly{{(float)c0, (float)c1, (float)c2}, normalise, (float)eps}, true);
+        ctx->saved_data["c0"] = c0, ctx->saved_data["c1"] = c1, ctx->saved_data["c2"] = c2, ctx->saved_data["n"] = normalise;
+        variable_list s = {q, k, v};
+        if (normalise) s.push_back(r.o), s.push_back(r.denom);
+        if (r.state.defined()) s.push_back(r.state);
+        ctx->save_for_backward(std::move(s));
+        return r.o;
     }
     static variable_list backward(AutogradContext *ctx, variable_list go) {
         const variable_list s = ctx->get_saved_variables();
-        const bool normalise = s.size() > 3;
+        const bool normalise = ctx->saved_data["n"].toBool();
+        const size_t base = normalise ? 5 : 3;
         auto c = [&](const char *key) { return (float)ctx->saved_data[key].toDouble(); };
         variable_list g = poly_bwd(go[0], s[0], s[1], s[2], normalise ? s[3] : Tensor(), normalise ? s[4] : Tensor(),
-                                   Poly{{c("c0"), c("c1"), c("c2")}, normalise, 0.f});
+                                   s.size() > base ? s[base] : Tensor(), Poly{{c("c0"), c("c1"), c("c2")}, normalise, 0.f});
         g.resize(9);
         return g;
     }
@@ -414,8 +436,8 @@ PyObject *py_polynomial(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
     return released([&]() -> Tensor {
         if (wants_grad(a.q, a.k, a.v)) return Polynomial::apply(a.q, a.k, a.v, c[0], c[1], c[2], normalise, eps, a.cast);
-        return std::get<0>(poly_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast),
-                                    Poly{{(float)c[0], (float)c[1], (float)c[2]}, normalise, (float)eps}));
+        return poly_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast),
+                        Poly{{(float)c[0], (float)c[1], (float)c[2]}, normalise, (float)eps}, false).o;
     });
     END_HANDLE_TH_ERRORS
 }

@@ -9,6 +9,7 @@
 #include "fla_chunk_walk.h"
 #include "fla_norm.h"
 #include "fla_pack.h"
+#include "fla_poly_walk.h"
 #include "fla_tri_kernel.h"
 #include "fla_tri_pair.h"
 
@@ -90,6 +91,12 @@ FLA_FIELD(src) FLA_FIELD(dst) FLA_FIELD(ss_b) FLA_FIELD(ss_h) FLA_FIELD(ss_n) FL
 FLA_FIELD(width) FLA_FIELD(wp)
 FLA_FIELDS_END
 
+FLA_FIELDS_BEGIN(PolyWalkParams)
+FLA_FIELD(q) FLA_FIELD(k) FLA_FIELD(v) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(out) FLA_FIELD(dq) FLA_FIELD(dk) FLA_FIELD(dv)
+FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(r) FLA_FIELD(wv) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks) FLA_FIELD(n_seg)
+FLA_FIELD(denom) FLA_FIELD(totals) FLA_FIELD(sum_entries) FLA_FIELD(ends)
+FLA_FIELDS_END
+
 #undef FLA_FIELDS_BEGIN
 #undef FLA_FIELD
 #undef FLA_FIELDS_END
@@ -101,6 +108,7 @@ inline void trace_describe(trace::Record &r, int arg, const WalkParams &p) { tra
 inline void trace_describe(trace::Record &r, int arg, const WalkTotalsParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const WalkVecParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const ChunkStateParams &p) { trace_fields(r, arg, "", p); }
+inline void trace_describe(trace::Record &r, int arg, const PolyWalkParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const PackParams &p) {
     for (int i = 0; i < 4; ++i) trace_fields(r, arg, "t" + std::to_string(i) + ".", p.item[i]);
     r.field(arg, "H", p.H), r.field(arg, "N", p.N), r.field(arg, "rows", p.rows);

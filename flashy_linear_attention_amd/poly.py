@@ -96,6 +96,71 @@ def poly_attention_bwd(
     return dxq, dxk, dvv
 
 
+def poly_attention_chunked_fwd(
+    xq: torch.Tensor, xk: torch.Tensor, v: torch.Tensor, coef: Tuple[float, float, float],
+    normalise: bool = False, eps: float = 1e-5,
+) -> Tuple[torch.Tensor, Optional[torch.Tensor], torch.Tensor]:
+    """(out, denom, state) by the chunk-wise evaluation (bf16, R <= 16, D_v <= 64), O(N);
+    ``PolynomialLinearAttention`` takes it where it is the faster one."""
+    _check(xq, xk, v)
+    xq, xk, v = prepare(xq, xk, v)
+    b, h, n, r = xq.shape
+    dv = v.shape[-1]
+    out = torch.empty_like(v, memory_format=torch.contiguous_format)
+    denom = torch.empty(b, h, n, dtype=torch.float32, device=xq.device) if normalise else None
+    lib = _lib.load()
+    with device_guard(xq.device):
+        state = torch.empty(_lib.query("fla_poly_attn_chunked_state_bytes", b, h, n, r, dv), dtype=torch.uint8, device=xq.device)
+        nbytes = _lib.query("fla_poly_attn_chunked_workspace_bytes", b, h, n, r, dv)
+        work = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=xq.device)
+        _lib.check(
+            "fla_poly_attn_chunked_fwd",
+            lib.fla_poly_attn_chunked_fwd(
+                xq.data_ptr(), xk.data_ptr(), v.data_ptr(), out.data_ptr(),
+                denom.data_ptr() if denom is not None else None, b, h, n, r, dv,
+                _lib.strides_arg(xq), _lib.strides_arg(xk), _lib.strides_arg(v), _lib.strides_arg(out),
+                _coef(*coef), float(eps), dtype_code(xq), state.data_ptr(), work.data_ptr(), nbytes, stream_handle(xq.device),
+            ),
+        )
+    return out, denom, state
+
+
+def poly_attention_chunked_bwd(
+    grad_output: torch.Tensor, xq: torch.Tensor, xk: torch.Tensor, v: torch.Tensor, coef: Tuple[float, float, float],
+    state: torch.Tensor, out: Optional[torch.Tensor] = None, denom: Optional[torch.Tensor] = None,
+) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+    """(dXq, dXk, dV) from what :func:`poly_attention_chunked_fwd` returned (out and denom when normalised)."""
+    _check(xq, xk, v)
+    assert (out is None) == (denom is None)
+    grad_output, xq, xk, v = prepare(grad_output, xq, xk, v)
+    if out is not None:
+        (out,) = prepare(out)
+        assert denom.dtype == torch.float32 and denom.is_contiguous() and denom.shape == xq.shape[:3]
+    b, h, n, r = xq.shape
+    dv = v.shape[-1]
+    assert state.numel() == _lib.query("fla_poly_attn_chunked_state_bytes", b, h, n, r, dv), "state of another shape"
+    dxq = torch.empty_like(xq, memory_format=torch.contiguous_format)
+    dxk = torch.empty_like(xk, memory_format=torch.contiguous_format)
+    dvv = torch.empty_like(v, memory_format=torch.contiguous_format)
+    lib = _lib.load()
+    with device_guard(xq.device):
+        nbytes = _lib.query("fla_poly_attn_chunked_workspace_bytes", b, h, n, r, dv)
+        work = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=xq.device)
+        _lib.check(
+            "fla_poly_attn_chunked_bwd",
+            lib.fla_poly_attn_chunked_bwd(
+                grad_output.data_ptr(), xq.data_ptr(), xk.data_ptr(), v.data_ptr(),
+                out.data_ptr() if out is not None else None, denom.data_ptr() if denom is not None else None,
+                dxq.data_ptr(), dxk.data_ptr(), dvv.data_ptr(), b, h, n, r, dv,
+                _lib.strides_arg(grad_output), _lib.strides_arg(xq), _lib.strides_arg(xk), _lib.strides_arg(v),
+                _lib.strides_arg(out) if out is not None else None,
+                _lib.strides_arg(dxq), _lib.strides_arg(dxk), _lib.strides_arg(dvv),
+                _coef(*coef), dtype_code(xq), state.data_ptr(), work.data_ptr(), nbytes, stream_handle(xq.device),
+            ),
+        )
+    return dxq, dxk, dvv
+
+
 class PolynomialLinearAttention(Function):
     @classmethod
     def apply(cls, *args):

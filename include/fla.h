@@ -343,6 +343,33 @@ int fla_poly_attn_bwd(const void *grad_out, const void *xq, const void *xk, cons
                       const int64_t *dv_strides,
                       const float *coef, int dtype, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* The same operator evaluated chunk-wise (O(N): running sums of Taylor features formed inside the kernels, nothing
+ * feature-wide in memory but the states at segment ends).  FLA_DTYPE_BF16 and R <= 16, D_v <= 64 only
+ * (FLA_ERR_UNSUPPORTED otherwise, as for operands that are not 16-byte aligned).  fla_poly_attn_prefers_chunked(): 1 where
+ * it is the faster evaluation (of a forward + backward pair, or with backward == 0 of forward alone; host arithmetic,
+ * measured thresholds), 0 elsewhere and where it does not exist.
+ * `workspace`: fla_poly_attn_chunked_workspace_bytes() bytes; `state_out` / `state_in`:
+ * fla_poly_attn_chunked_state_bytes() bytes, written by forward (NULL: no backward will follow) and read by
+ * backward; both 16-byte aligned, both may be 0 bytes. */
+int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward);
+int64_t fla_poly_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v);
+int64_t fla_poly_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v);
+int fla_poly_attn_chunked_fwd(const void *xq, const void *xk, const void *v, void *o, float *denom,
+                              int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v,
+                              const int64_t *xq_strides, const int64_t *xk_strides,
+                              const int64_t *v_strides, const int64_t *o_strides,
+                              const float *coef, float eps, int dtype, void *state_out,
+                              void *workspace, int64_t workspace_bytes, void *stream);
+int fla_poly_attn_chunked_bwd(const void *grad_out, const void *xq, const void *xk, const void *v,
+                              const void *o, const float *denom,
+                              void *dxq, void *dxk, void *dv,
+                              int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v,
+                              const int64_t *go_strides, const int64_t *xq_strides,
+                              const int64_t *xk_strides, const int64_t *v_strides, const int64_t *o_strides,
+                              const int64_t *dxq_strides, const int64_t *dxk_strides,
+                              const int64_t *dv_strides, const float *coef, int dtype, const void *state_in,
+                              void *workspace, int64_t workspace_bytes, void *stream);
+
 /* Normalised causal linear attention, the full operator a caller of the reference assembles
  * in PyTorch around LinearAttention.apply (README.md:27-30 of the reference):
  *
