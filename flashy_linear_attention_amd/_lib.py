@@ -25,6 +25,8 @@ _strides = ctypes.POINTER(ctypes.c_int64)
 SIGNATURES = {
     "fla_abi_version": ([], ctypes.c_int),
     "fla_strerror": ([ctypes.c_int], ctypes.c_char_p),
+    "fla_convert": ([ctypes.POINTER(_ptr), ctypes.POINTER(_ptr), _strides, ctypes.c_int, ctypes.c_int, ctypes.c_int, _ptr],
+                    ctypes.c_int),
     "fla_linear_attn_fwd": ([_ptr] * 4 + [_i64] * 4 + [_strides] * 4 + [ctypes.c_int, _ptr], ctypes.c_int),
     "fla_linear_attn_bwd": ([_ptr] * 7 + [_i64] * 4 + [_strides] * 7 + [ctypes.c_int, _ptr], ctypes.c_int),
     "fla_linear_attn_smallv_fwd": ([_ptr] * 4 + [_i64] * 5 + [_strides] * 4 + [ctypes.c_int, _ptr], ctypes.c_int),

@@ -8,6 +8,7 @@
 #include <atomic>
 
 #include "fla_dispatch.h"
+#include "fla_convert.h"
 #include "fla_norm.h"
 #include "fla_pack.h"
 #include "fla_poly_walk.h"
@@ -393,6 +394,11 @@ struct WalkPlan {
 // are padded with zeros as they land in LDS, and at D = 128 the kernels built for at most 64 true columns on one side
 // leave the padding's MFMAs out.  The plain operator only (the normaliser's and the feature maps' variants of the
 // kernels are built for equal padded widths).
+// D = 128: up to this many segments per (b, h) the walks add up the segments' totals themselves, beyond it a scan kernel
+// does.  Measured per forward + backward, scan against sums on load: B H 32, N 4096 (8 segments) 146 / 137 us; B H 24, N
+// 1500 (8) 80 / 77; B H 20, N 4096 (11) 145 / 141; B H 16, N 4096 (16) 101 / 104; B H 8, N 4096 (32) 79 / 109.
+constexpr int kSumOnLoadMost = 12;
+
 WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false) {
     WalkPlan w{};
     if (B <= 0 || H <= 0 || N <= 0) return w;  // (an empty problem has no plan; the callers return before any launch)
@@ -874,9 +880,9 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         // them to state_out (the totals themselves are computed there, and no workspace is used);
         // the normalised operator at padded head dims up to 64 hands over the 16-bit state of every chunk instead
         const bool in_state = state_out && (wp.split || !nx);
-        // D = 128, a few segments more than two: the totals go to the workspace, the walk adds them up itself as it starts
+        // D = 128, a few segments more than two (kSumOnLoadMost): the totals go to the workspace, the walk adds them up itself as it starts
         // and writes the entry states it formed to state_out -- no scan launch (B H 64, N 4096: see wide_forward)
-        const bool sum_on_load = wp.split && !fmap && !nx && wp.n_seg >= 3 && wp.n_seg <= 7;
+        const bool sum_on_load = wp.split && !fmap && !nx && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
         if (need_totals && (!in_state || sum_on_load) &&
             (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < wp.work_bytes))
             return FLA_ERR_WORKSPACE;
@@ -1026,7 +1032,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         // with forward's states at hand (and without the normaliser): one reverse walk
         const bool one_walk = state_in && !nx;
         // (... which adds up the totals of the segments after its own itself, as forward does)
-        const bool rev_sums_on_load = one_walk && wp.n_seg >= 3 && wp.n_seg <= 7;
+        const bool rev_sums_on_load = one_walk && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
         if (wp.n_seg > 1) {
             if (!state_in) {
                 const float *fwd_entry = nullptr;
@@ -1823,6 +1829,23 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
 extern "C" {
 
 int fla_abi_version(void) { return FLA_ABI_VERSION; }
+
+int fla_convert(const void *const *src, void *const *dst, const int64_t *counts, int n, int widen, int dtype, void *stream) {
+    if (dtype != FLA_DTYPE_BF16 && dtype != FLA_DTYPE_F16) return FLA_ERR_DTYPE;
+    if (n < 0 || n > 4 || !src || !dst || !counts) return n == 0 ? FLA_OK : FLA_ERR_SHAPE;
+    fla::ConvertParams p{};
+    for (int i = 0; i < n; ++i) {
+        if (counts[i] < 0) return FLA_ERR_SHAPE;
+        if (counts[i] && (!src[i] || !dst[i])) return FLA_ERR_NULL_POINTER;
+        // (the 16-byte side in 16-byte accesses, the fp32 side in 32-byte ones that the compiler splits)
+        if (reinterpret_cast<uintptr_t>(src[i]) % 16 || reinterpret_cast<uintptr_t>(dst[i]) % 16) return FLA_ERR_UNSUPPORTED;
+        p.src[i] = src[i], p.dst[i] = dst[i], p.count[i] = counts[i];
+    }
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const hipError_t e = dtype == FLA_DTYPE_BF16 ? fla::launch_convert<__bf16>(p, n, widen != 0, s)
+                                                 : fla::launch_convert<_Float16>(p, n, widen != 0, s);
+    return e == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
+}
 
 const char *fla_strerror(int status) {
     switch (status) {

@@ -83,7 +83,56 @@ bool agree(const Tensor &q, const Tensor &k, const Tensor &v, bool cast) {
     return dtype_code(q.scalar_type()) >= 0 && k.scalar_type() == q.scalar_type() && v.scalar_type() == q.scalar_type();
 }
 
-Tensor cast_to(const Tensor &t, bool cast) { return cast ? t.to(at::kBFloat16) : t; }
+// Operands as the kernels take them.  `cast` (autocast): in bf16, the fp32 ones in one launch; `widened` remembers which
+// came in fp32, so that their gradients leave in fp32 from one launch too (the engine would convert them one by one).
+struct Casts {
+    Tensor q, k, v;
+    int64_t widened = 0;
+    Casts(const Tensor &q_, const Tensor &k_, const Tensor &v_, bool cast) : q(q_), k(k_), v(v_) {
+        if (!cast) return;
+        at::AutoDispatchBelowADInplaceOrView below;
+        Tensor *all[3] = {&q, &k, &v}, out[3];
+        const void *src[3];
+        void *dst[3];
+        int64_t count[3];
+        int n = 0;
+        for (int i = 0; i < 3; ++i) {
+            const Tensor &t = *all[i];
+            if (t.scalar_type() == at::kFloat) widened |= 1 << i;
+            if (t.scalar_type() == at::kFloat && t.is_non_overlapping_and_dense() && (uintptr_t)t.data_ptr() % 16 == 0) {
+                out[i] = at::empty_strided(t.sizes(), t.strides(), t.options().dtype(at::kBFloat16));
+                src[n] = t.data_ptr(), dst[n] = out[i].data_ptr(), count[n++] = t.numel();
+            } else {
+                out[i] = t.to(at::kBFloat16);
+            }
+        }
+        if (n) {
+            const c10::DeviceGuard guard(q.device());
+            must(fla_convert(src, dst, count, n, 0, FLA_DTYPE_BF16, c10::hip::getCurrentHIPStream(q.device().index()).stream()));
+        }
+        q = out[0], k = out[1], v = out[2];
+    }
+};
+
+// gradients of the inputs that came in fp32, in fp32
+void widen(variable_list &g, int64_t which) {
+    if (!which) return;
+    at::AutoDispatchBelowADInplaceOrView below;
+    const void *src[3];
+    void *dst[3];
+    int64_t count[3];
+    int n = 0;
+    const c10::DeviceGuard guard(g[0].device());
+    variable_list out = g;
+    for (int i = 0; i < 3; ++i)
+        if (which >> i & 1) {
+            out[i] = at::empty(g[i].sizes(), g[i].options().dtype(at::kFloat));
+            src[n] = g[i].data_ptr(), dst[n] = out[i].data_ptr(), count[n++] = g[i].numel();
+        }
+    must(fla_convert(src, dst, count, n, 1, dtype_code(g[0].scalar_type()),
+                     c10::hip::getCurrentHIPStream(g[0].device().index()).stream()));
+    g = std::move(out);
+}
 
 bool wants_grad(const Tensor &q, const Tensor &k, const Tensor &v) {
     return at::GradMode::is_enabled() && (q.requires_grad() || k.requires_grad() || v.requires_grad());
@@ -137,7 +186,9 @@ variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_,
 
 struct Product : Function<Product> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, int64_t ev, bool cast) {
-        const Tensor q = cast_to(q_, cast), k = cast_to(k_, cast), v = cast_to(v_, cast);
+        const Casts in(q_, k_, v_, cast);
+        const Tensor &q = in.q, &k = in.k, &v = in.v;
+        ctx->saved_data["widened"] = in.widened;
         auto [o, state] = product_fwd(q, k, v, (int)ev, true);
         ctx->saved_data["ev"] = ev;
         if (state.defined())
@@ -149,6 +200,7 @@ struct Product : Function<Product> {
     static variable_list backward(AutogradContext *ctx, variable_list go) {
         const variable_list s = ctx->get_saved_variables();
         variable_list g = product_bwd(go[0], s[0], s[1], s[2], s.size() > 3 ? s[3] : Tensor(), (int)ctx->saved_data["ev"].toInt());
+        widen(g, ctx->saved_data["widened"].toInt());
         g.resize(5);
         return g;
     }
@@ -231,7 +283,9 @@ struct Mapped : Function<Mapped> {
                           bool cast) {
         Options opt = Options::of(code);
         opt.eps = eps;
-        const Tensor q = cast_to(q_, cast), k = cast_to(k_, cast), v = cast_to(v_, cast);
+        const Casts in(q_, k_, v_, cast);
+        const Tensor &q = in.q, &k = in.k, &v = in.v;
+        ctx->saved_data["widened"] = in.widened;
         MappedResult r = mapped_fwd(q, k, v, opt, true);
         ctx->saved_data["opt"] = code;
         variable_list s = {opt.fmap ? r.q : q, opt.fmap ? r.k : k, v};
@@ -246,6 +300,7 @@ struct Mapped : Function<Mapped> {
         const size_t base = opt.normalise ? 5 : 3;
         variable_list g = mapped_bwd(go[0], s[0], s[1], s[2], opt.normalise ? s[3] : Tensor(), opt.normalise ? s[4] : Tensor(),
                                      s.size() > base ? s[base] : Tensor(), opt);
+        widen(g, ctx->saved_data["widened"].toInt());
         g.resize(6);
         return g;
     }
@@ -308,7 +363,9 @@ variable_list poly_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, co
 struct Polynomial : Function<Polynomial> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, double c0, double c1,
                           double c2, bool normalise, double eps, bool cast) {
-        const Tensor q = cast_to(q_, cast), k = cast_to(k_, cast), v = cast_to(v_, cast);
+        const Casts in(q_, k_, v_, cast);
+        const Tensor &q = in.q, &k = in.k, &v = in.v;
+        ctx->saved_data["widened"] = in.widened;
         PolyResult r = poly_fwd(q, k, v, Poly{{(float)c0, (float)c1, (float)c2}, normalise, (float)eps}, true);
         ctx->saved_data["c0"] = c0, ctx->saved_data["c1"] = c1, ctx->saved_data["c2"] = c2, ctx->saved_data["n"] = normalise;
         variable_list s = {q, k, v};
@@ -324,6 +381,7 @@ struct Polynomial : Function<Polynomial> {
         auto c = [&](const char *key) { return (float)ctx->saved_data[key].toDouble(); };
         variable_list g = poly_bwd(go[0], s[0], s[1], s[2], normalise ? s[3] : Tensor(), normalise ? s[4] : Tensor(),
                                    s.size() > base ? s[base] : Tensor(), Poly{{c("c0"), c("c1"), c("c2")}, normalise, 0.f});
+        widen(g, ctx->saved_data["widened"].toInt());
         g.resize(9);
         return g;
     }
@@ -395,7 +453,8 @@ PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
     return released([&]() -> Tensor {
         if (wants_grad(a.q, a.k, a.v)) return Product::apply(a.q, a.k, a.v, (int64_t)ev, a.cast);
-        return std::get<0>(product_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast), ev, false));
+        const Casts in(a.q, a.k, a.v, a.cast);
+        return std::get<0>(product_fwd(in.q, in.k, in.v, ev, false));
     });
     END_HANDLE_TH_ERRORS
 }
@@ -415,7 +474,8 @@ PyObject *py_mapped(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
     return released([&]() -> Tensor {
         if (wants_grad(a.q, a.k, a.v)) return Mapped::apply(a.q, a.k, a.v, opt.code(), opt.eps, a.cast);
-        return mapped_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast), opt, false).o;
+        const Casts in(a.q, a.k, a.v, a.cast);
+        return mapped_fwd(in.q, in.k, in.v, opt, false).o;
     });
     END_HANDLE_TH_ERRORS
 }
@@ -436,7 +496,8 @@ PyObject *py_polynomial(PyObject *, PyObject *const *args, Py_ssize_t n) {
     }
     return released([&]() -> Tensor {
         if (wants_grad(a.q, a.k, a.v)) return Polynomial::apply(a.q, a.k, a.v, c[0], c[1], c[2], normalise, eps, a.cast);
-        return poly_fwd(cast_to(a.q, a.cast), cast_to(a.k, a.cast), cast_to(a.v, a.cast),
+        const Casts in(a.q, a.k, a.v, a.cast);
+        return poly_fwd(in.q, in.k, in.v,
                         Poly{{(float)c[0], (float)c[1], (float)c[2]}, normalise, (float)eps}, false).o;
     });
     END_HANDLE_TH_ERRORS

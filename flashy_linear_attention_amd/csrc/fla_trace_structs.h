@@ -7,6 +7,7 @@
 
 #include "fla_chunk_state.h"
 #include "fla_chunk_walk.h"
+#include "fla_convert.h"
 #include "fla_norm.h"
 #include "fla_pack.h"
 #include "fla_poly_walk.h"
@@ -109,6 +110,12 @@ inline void trace_describe(trace::Record &r, int arg, const WalkTotalsParams &p)
 inline void trace_describe(trace::Record &r, int arg, const WalkVecParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const ChunkStateParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const PolyWalkParams &p) { trace_fields(r, arg, "", p); }
+inline void trace_describe(trace::Record &r, int arg, const ConvertParams &p) {
+    for (int i = 0; i < 4; ++i) {
+        const std::string at = std::to_string(i);
+        r.field(arg, ("src" + at).c_str(), p.src[i]), r.field(arg, ("dst" + at).c_str(), p.dst[i]);
+    }
+}
 inline void trace_describe(trace::Record &r, int arg, const PackParams &p) {
     for (int i = 0; i < 4; ++i) trace_fields(r, arg, "t" + std::to_string(i) + ".", p.item[i]);
     r.field(arg, "H", p.H), r.field(arg, "N", p.N), r.field(arg, "rows", p.rows);

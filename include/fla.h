@@ -67,6 +67,9 @@ enum fla_status {
 
 /* ABI revision of the loaded library (== FLA_ABI_VERSION it was built with). */
 int fla_abi_version(void);
+/* dst[i][0 .. counts[i]) = src[i][0 .. counts[i]), i < n <= 4, from fp32 to the 16-bit type (widen: the other way), in one
+ * launch: the copies autocast makes of an operator's operands and gradients.  Dense, 16-byte aligned buffers. */
+int fla_convert(const void *const *src, void *const *dst, const int64_t *counts, int n, int widen, int dtype, void *stream);
 
 /* Static, human-readable text for a status code. */
 const char *fla_strerror(int status);
