@@ -399,7 +399,8 @@ struct WalkPlan {
 // 1500 (8) 80 / 77; B H 20, N 4096 (11) 145 / 141; B H 16, N 4096 (16) 101 / 104; B H 8, N 4096 (32) 79 / 109.
 constexpr int kSumOnLoadMost = 12;
 
-WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false) {
+// `parts`: workgroups per segment (a launch that does several column halves at a time).
+WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false, int64_t parts = 1) {
     WalkPlan w{};
     if (B <= 0 || H <= 0 || N <= 0) return w;  // (an empty problem has no plan; the callers return before any launch)
     const int64_t wider = padded(dqk) > padded(dv) ? padded(dqk) : padded(dv);
@@ -419,7 +420,7 @@ WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, boo
     // (totals over finer segments than the walk's, 2 or 4 per walk segment, would put more workgroups on the
     // totals kernel; measured at D = 128 over B H = 8 ... 256, N = 1024 ... 32768, one total per walk segment
     // is the fastest everywhere, by 3 to 27 % of a forward + backward step)
-    const int64_t resident = w.split ? 256 : 512;
+    const int64_t resident = (w.split ? 256 : 512) / parts;
     int64_t segs = resident / (B * H) > 1 ? resident / (B * H) : 1;
     if (segs > w.n_chunks) segs = w.n_chunks;
     w.seg_chunks = (w.n_chunks + segs - 1) / segs;
@@ -448,8 +449,9 @@ struct EntryHalf {
 int walk_entry_states(const WalkPlan &w, const View &y, const View &z, int64_t B, int64_t H, int64_t N, int64_t dy,
                       int64_t dz, int dtype, int reverse, void *work, float *entry, const float **where, hipStream_t s,
                       int map_y = 0, const View *ymap_out = nullptr, const EntryHalf *second = nullptr,
-                      bool totals_only = false) {
+                      bool totals_only = false, bool z_narrow = false) {
     fla::WalkTotalsParams tp{};
+    tp.z_narrow = z_narrow;
     if (map_y) {
         tp.map_y = map_y, tp.ymap_out = const_cast<void *>(ymap_out->ptr);
         tp.yo_b = ymap_out->strides[0], tp.yo_h = ymap_out->strides[1], tp.yo_n = ymap_out->strides[2];
@@ -483,7 +485,7 @@ int walk_entry_states(const WalkPlan &w, const View &y, const View &z, int64_t B
     if (fla::walk_totals(dtype, w.D, tp, s) != hipSuccess) return FLA_ERR_LAUNCH;
     *where = entry;
     if (no_scan) return FLA_OK;
-    return fla::walk_scan(totals, entry, B * H, (int)w.n_seg, w.D, fla::walk_totals_cols(w.D, (int)dy, (int)dz), reverse,
+    return fla::walk_scan(totals, entry, B * H, (int)w.n_seg, w.D, z_narrow ? 64 : fla::walk_totals_cols(w.D, (int)dy, (int)dz), reverse,
                           s, totals2, entry2) == hipSuccess
                ? FLA_OK
                : FLA_ERR_LAUNCH;
@@ -492,15 +494,17 @@ int walk_entry_states(const WalkPlan &w, const View &y, const View &z, int64_t B
 // Entry states of both 128-column halves of a wide q / k (Y = the halves of `y`, against the same Z):
 // one totals launch and one scan for the two when both halves take the same kernel variant, else
 // one after the other.  work[h], entry[h] (null: over work[h]) and where[h] per half.
+// `z_narrow`: dz <= 64, and the walks behind leave columns 64 .. of the states out whatever the second half's width
+// (walk_fwd_wide_kernel, walk_bwd_rev_wide_kernel): one launch for any D_qk.
 int wide_entry_states(const WalkPlan &wp, const View &y, const View &z, int64_t B, int64_t H, int64_t N, int64_t dy_all,
                       int64_t dz, int dtype, int reverse, void *const (&work)[2], float *const (&entry)[2],
-                      const float *(&where)[2], hipStream_t s, bool totals_only = false) {
+                      const float *(&where)[2], hipStream_t s, bool totals_only = false, bool z_narrow = false) {
     const View y1{static_cast<const char *>(y.ptr) + 128 * 2, y.strides};
     const int64_t dy1 = dy_all - 128;
-    if (fla::walk_totals_cols(wp.D, 128, (int)dz) == fla::walk_totals_cols(wp.D, (int)dy1, (int)dz)) {
+    if (z_narrow || fla::walk_totals_cols(wp.D, 128, (int)dz) == fla::walk_totals_cols(wp.D, (int)dy1, (int)dz)) {
         const EntryHalf other{y1.ptr, dy1, work[1], entry[1], &where[1]};
         return walk_entry_states(wp, y, z, B, H, N, 128, dz, dtype, reverse, work[0], entry[0], &where[0], s, 0, nullptr,
-                                 &other, totals_only);
+                                 &other, totals_only, z_narrow);
     }
     if (int rc = walk_entry_states(wp, y, z, B, H, N, 128, dz, dtype, reverse, work[0], entry[0], &where[0], s, 0, nullptr,
                                    nullptr, totals_only))
@@ -668,6 +672,24 @@ fla::WalkParams lower_walk_params(const WalkPlan &wp, const View &x, const View 
     return w;
 }
 
+// the reverse walk that computes dQ, dK and dV
+fla::WalkParams reverse_walk_params(const WalkPlan &wp, const View &go, const View &q, const View &k, const View &v, const View &dq,
+                                    const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t wqk, int64_t wv) {
+    fla::WalkParams r{};
+    r.q = q.ptr, r.k = k.ptr, r.v = v.ptr, r.go = go.ptr;
+    r.dq = const_cast<void *>(dq.ptr), r.dk = const_cast<void *>(dk.ptr), r.dv = const_cast<void *>(dvv.ptr);
+    r.qs_b = q.strides[0], r.qs_h = q.strides[1], r.qs_n = q.strides[2];
+    r.ks_b = k.strides[0], r.ks_h = k.strides[1], r.ks_n = k.strides[2];
+    r.vs_b = v.strides[0], r.vs_h = v.strides[1], r.vs_n = v.strides[2];
+    r.gs_b = go.strides[0], r.gs_h = go.strides[1], r.gs_n = go.strides[2];
+    r.dqs_b = dq.strides[0], r.dqs_h = dq.strides[1], r.dqs_n = dq.strides[2];
+    r.dks_b = dk.strides[0], r.dks_h = dk.strides[1], r.dks_n = dk.strides[2];
+    r.dvs_b = dvv.strides[0], r.dvs_h = dvv.strides[1], r.dvs_n = dvv.strides[2];
+    r.H = (int32_t)H, r.N = (int32_t)N, r.BH = (int32_t)(B * H), r.wqk = (int32_t)wqk, r.wv = (int32_t)wv;
+    r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
+    return r;
+}
+
 bool wide_fast_path(const View &q, const View &k, const View &v, const View &o, int64_t B, int64_t H, int64_t N,
                     int64_t dqk, int64_t dv) {
     return fla::fast_path_ok(make_params(q, k, v, o, B, H, N, 128, dv, 0)) &&
@@ -696,7 +718,7 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
         }
         float *const none[2] = {nullptr, nullptr};
         if (int rc = wide_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0, work, sum_on_load ? none : keep, entry, s,
-                                       sum_on_load))
+                                       sum_on_load, dv <= 64))
             return rc;
     }
     // one walk over both halves (the second one's columns start 128 elements into q's and k's rows)
@@ -717,6 +739,7 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
     char *ws = static_cast<char *>(workspace);
     const int64_t temp_strides[4] = {H * N * dv, N * dv, dv, 1};
     const View temp{ws, temp_strides};
+    const bool one_walk = state_in && dv <= 64;  // forward's states at hand, narrow v: one reverse walk over both halves
     // entry states of both halves up front: Q_h^T dO over the segments after, and -- when forward's are not
     // at hand -- K_h^T V over the segments before
     const float *fwd_entries[2] = {nullptr, nullptr}, *entries[2] = {nullptr, nullptr};
@@ -733,23 +756,13 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
             if (int rc = wide_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0, work, none, fwd_entries, s)) return rc;
         }
         void *const work[2] = {base, base + wp.work_bytes};
-        if (int rc = wide_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, work, none, entries, s, rev_sums_on_load))
+        if (int rc = wide_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, work, none, entries, s, rev_sums_on_load,
+                                       one_walk))
             return rc;
     }
-    if (state_in && dv <= 64) {  // forward's states at hand, narrow v: one reverse walk over both halves
-        fla::WalkParams r{};
-        r.q = q.ptr, r.k = k.ptr, r.v = v.ptr, r.go = go.ptr;
-        r.dq = const_cast<void *>(dq.ptr), r.dk = const_cast<void *>(dk.ptr), r.dv = const_cast<void *>(dvv.ptr);
-        r.qs_b = q.strides[0], r.qs_h = q.strides[1], r.qs_n = q.strides[2];
-        r.ks_b = k.strides[0], r.ks_h = k.strides[1], r.ks_n = k.strides[2];
-        r.vs_b = v.strides[0], r.vs_h = v.strides[1], r.vs_n = v.strides[2];
-        r.gs_b = go.strides[0], r.gs_h = go.strides[1], r.gs_n = go.strides[2];
-        r.dqs_b = dq.strides[0], r.dqs_h = dq.strides[1], r.dqs_n = dq.strides[2];
-        r.dks_b = dk.strides[0], r.dks_h = dk.strides[1], r.dks_n = dk.strides[2];
-        r.dvs_b = dvv.strides[0], r.dvs_h = dvv.strides[1], r.dvs_n = dvv.strides[2];
-        r.H = (int32_t)H, r.N = (int32_t)N, r.BH = (int32_t)(B * H), r.wqk = 128, r.wqk2 = (int32_t)(dqk - 128);
-        r.wv = (int32_t)dv;
-        r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
+    if (one_walk) {
+        fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, 128, dv);
+        r.wqk2 = (int32_t)(dqk - 128);
         r.init = entries[0], r.init2 = entries[1], r.init_is_totals = rev_sums_on_load;
         const char *half0 = static_cast<const char *>(state_in), *half1 = half0 + wp.saved_bytes;
         r.xinit = reinterpret_cast<const float *>(half0), r.xinit2 = reinterpret_cast<const float *>(half1);
@@ -763,19 +776,8 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
         const float *fwd_entry = fwd_entries[h], *entry = entries[h];
         const View &dvh = h == 0 ? dvv : temp;
         if (state_in) {  // forward's states at hand: dQ_h, dK_h and this half's part of dV in one reverse walk
-            fla::WalkParams r{};
-            r.q = qh.ptr, r.k = kh.ptr, r.v = v.ptr, r.go = go.ptr;
-            r.dq = const_cast<void *>(dqh.ptr), r.dk = const_cast<void *>(dkh.ptr), r.dv = const_cast<void *>(dvv.ptr);
+            fla::WalkParams r = reverse_walk_params(wp, go, qh, kh, v, dqh, dkh, dvv, B, H, N, wqk, dv);
             r.accumulate = h;  // (the second half's walk adds its part of dV to the first one's)
-            r.qs_b = qh.strides[0], r.qs_h = qh.strides[1], r.qs_n = qh.strides[2];
-            r.ks_b = kh.strides[0], r.ks_h = kh.strides[1], r.ks_n = kh.strides[2];
-            r.vs_b = v.strides[0], r.vs_h = v.strides[1], r.vs_n = v.strides[2];
-            r.gs_b = go.strides[0], r.gs_h = go.strides[1], r.gs_n = go.strides[2];
-            r.dqs_b = dqh.strides[0], r.dqs_h = dqh.strides[1], r.dqs_n = dqh.strides[2];
-            r.dks_b = dkh.strides[0], r.dks_h = dkh.strides[1], r.dks_n = dkh.strides[2];
-            r.dvs_b = dvv.strides[0], r.dvs_h = dvv.strides[1], r.dvs_n = dvv.strides[2];
-            r.H = (int32_t)H, r.N = (int32_t)N, r.BH = (int32_t)(B * H), r.wqk = (int32_t)wqk, r.wv = (int32_t)dv;
-            r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
             r.init = entry, r.init_is_totals = rev_sums_on_load;
             const char *half = static_cast<const char *>(state_in) + h * wp.saved_bytes;
             r.xinit = reinterpret_cast<const float *>(half);
@@ -803,6 +805,77 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
         if (fla::walk_dkdv(dtype, wp.D, r, s) != hipSuccess) return FLA_ERR_LAUNCH;
     }
     return state_in ? FLA_OK : launch_feature_pass(3, 0, temp, dvv, B, H, N, dv, dtype, s);
+}
+
+// ---- D_qk and D_v in (128, 256]: two column halves of q / k and two of v, four pairs with a state each.  One launch
+// works on two pairs (grid y), so a plan has half as many segments as the two walks after each other that it
+// replaces: half the totals and entry states to move, which at B H = 16 outweigh the operands.
+//   forward   one walk over both halves of q / k per half of v: O's halves are columns of their own
+//   backward  dQ and dK are sums over v's halves, dV over q / k's: first the pairs (0, 0) and (1, 1), whose results are
+//             different columns of all three, then (1, 0) and (0, 1), which add theirs in the walks' epilogues
+// Five launches per step, and no scratch tensors.  256 / 256, forward + backward, halves of v after each other -> this:
+// B H 16, N 4096: 408 -> 245 us.
+WalkPlan quad_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
+    if (dqk <= 128 || dqk > 256 || dv <= 128 || dv > 256) return WalkPlan{};
+    return walk_plan(B, H, N, 128, 128, false, 2);
+}
+
+// four sets of entry states in one buffer, and in `state` four final states behind them
+float *quad_finals(const WalkPlan &wp, const void *state) {
+    return reinterpret_cast<float *>(static_cast<char *>(const_cast<void *>(state)) + 4 * wp.entry_bytes);
+}
+
+bool quad_sums_on_load(const WalkPlan &wp) { return wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost; }
+
+// the four pairs' segment totals of Y^T Z to `entries`, and the entry states over them where the walk does not add up
+int quad_entry_states(const WalkPlan &wp, const View &y, const View &z, int64_t B, int64_t H, int64_t N, int64_t dy, int64_t dz,
+                      int dtype, int reverse, float *entries, hipStream_t s) {
+    fla::WalkTotalsParams tp{};
+    tp.y = y.ptr, tp.y2 = column_half(y, 1).ptr, tp.z = z.ptr;
+    tp.totals = entries, tp.totals2 = entries + wp.entry_bytes / 4;
+    tp.ys_b = y.strides[0], tp.ys_h = y.strides[1], tp.ys_n = y.strides[2];
+    tp.zs_b = z.strides[0], tp.zs_h = z.strides[1], tp.zs_n = z.strides[2];
+    tp.H = (int32_t)H, tp.N = (int32_t)N, tp.BH = (int32_t)(B * H);
+    tp.dy = tp.dz = 128, tp.dy2 = (int32_t)(dy - 128), tp.dz2 = (int32_t)(dz - 128);
+    tp.n_chunks = (int32_t)wp.n_chunks, tp.seg_chunks = (int32_t)wp.seg_chunks, tp.n_seg = (int32_t)wp.n_seg;
+    tp.direct = wp.n_seg == 2;
+    tp.seg_lo = reverse ? 1 : 0, tp.seg_hi = (int32_t)(reverse ? wp.n_seg : wp.n_seg - 1);
+    if (fla::walk_totals(dtype, wp.D, tp, s) != hipSuccess) return FLA_ERR_LAUNCH;
+    if (tp.direct || quad_sums_on_load(wp)) return FLA_OK;
+    return fla::walk_scan(entries, entries, 4 * B * H, (int)wp.n_seg, wp.D, wp.D, reverse, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
+}
+
+int quad_forward(const WalkPlan &wp, const View &q, const View &k, const View &v, const View &o, int64_t B, int64_t H, int64_t N,
+                 int64_t dqk, int64_t dv, int dtype, void *state_out, void *workspace, hipStream_t s) {
+    const bool sum_on_load = quad_sums_on_load(wp);
+    const int64_t pair = wp.entry_bytes / 4;  // floats
+    float *const kept = static_cast<float *>(state_out);
+    float *const entries = kept && !sum_on_load ? kept : static_cast<float *>(workspace);
+    if (wp.n_seg > 1)
+        if (int rc = quad_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0, entries, s)) return rc;
+    fla::WalkParams w = lower_walk_params(wp, q, k, v, o, B, H, N, 128, 128, entries);
+    w.quad = 1, w.wqk2 = (int32_t)(dqk - 128), w.wv2 = (int32_t)(dv - 128);
+    w.init2 = w.init ? w.init + pair : nullptr;
+    if (sum_on_load) w.init_is_totals = 1, w.entry_out = kept, w.entry_out2 = kept ? kept + pair : nullptr;
+    if (kept) w.total_out = quad_finals(wp, kept), w.total_out2 = w.total_out + B * H * wp.D * wp.D;
+    return fla::walk_fwd_wide(dtype, w, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
+}
+
+int quad_backward(const WalkPlan &wp, const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
+                  const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype, const void *state_in,
+                  void *workspace, hipStream_t s) {
+    float *const entries = static_cast<float *>(workspace);
+    if (wp.n_seg > 1)
+        if (int rc = quad_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, entries, s)) return rc;
+    fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, 128, 128);
+    r.wqk2 = (int32_t)(dqk - 128), r.wv2 = (int32_t)(dv - 128);
+    r.init = wp.n_seg > 1 ? entries : nullptr, r.init_is_totals = quad_sums_on_load(wp);
+    r.xinit = static_cast<const float *>(state_in), r.xtotal = quad_finals(wp, state_in);
+    for (int pass = 0; pass < 2; ++pass) {
+        r.quad = 2 + pass, r.accumulate = 2 * pass;
+        if (fla::walk_bwd_rev(dtype, wp.D, r, s) != hipSuccess) return FLA_ERR_LAUNCH;
+    }
+    return FLA_OK;
 }
 
 // both column halves of (x4, o4) = (v, O) / (dO, dV) with (a, b) = (q, k) / (dQ, dK) qualify for their plans' kernels
@@ -848,6 +921,13 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
                 workspace_bytes < vsplit_inner_bytes(vs, B, H, N, dqk))
                 return FLA_ERR_WORKSPACE;
             if (state_out && reinterpret_cast<uintptr_t>(state_out) % 16 != 0) return FLA_ERR_WORKSPACE;
+            if (const WalkPlan quad = quad_plan(B, H, N, dqk, dv); quad.ok) {  // (fits: half the segments of vs's plans)
+                if (int rc = quad_forward(quad, q, k, v, o, B, H, N, dqk, dv, dtype, state_out, workspace,
+                                          static_cast<hipStream_t>(stream)))
+                    return rc;
+                if (state_out && state_valid) *state_valid = 1;
+                return FLA_OK;
+            }
             int32_t valid[2] = {0, 0};
             for (int j = 0; j < 2; ++j) {
                 void *st = state_out ? static_cast<char *>(state_out) + j * vs.state0 : nullptr;
@@ -976,6 +1056,10 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
             if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < inner + 2 * vs.temp_bytes)
                 return FLA_ERR_WORKSPACE;
             if (state_in && reinterpret_cast<uintptr_t>(state_in) % 16 != 0) return FLA_ERR_WORKSPACE;
+            // (without forward's states the halves of v go one after the other: each needs them again, and a walk of its own for dQ)
+            if (const WalkPlan quad = quad_plan(B, H, N, dqk, dv); quad.ok && state_in)
+                return quad_backward(quad, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace,
+                                     static_cast<hipStream_t>(stream));
             const int64_t temp_strides[4] = {H * N * dqk, N * dqk, dqk, 1};
             const View tq{static_cast<char *>(workspace) + inner, temp_strides};
             const View tk{static_cast<char *>(workspace) + inner + vs.temp_bytes, temp_strides};
@@ -1054,18 +1138,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
             else if (int rc = walk_chunk_vectors(wp, k, dqk, nullptr, 0, zc, B, H, N, dtype, s)) return rc;
         }
         if (one_walk) {
-            fla::WalkParams r{};
-            r.q = q.ptr, r.k = k.ptr, r.v = v.ptr, r.go = go.ptr;
-            r.dq = const_cast<void *>(dq.ptr), r.dk = const_cast<void *>(dk.ptr), r.dv = const_cast<void *>(dvv.ptr);
-            r.qs_b = q.strides[0], r.qs_h = q.strides[1], r.qs_n = q.strides[2];
-            r.ks_b = k.strides[0], r.ks_h = k.strides[1], r.ks_n = k.strides[2];
-            r.vs_b = v.strides[0], r.vs_h = v.strides[1], r.vs_n = v.strides[2];
-            r.gs_b = go.strides[0], r.gs_h = go.strides[1], r.gs_n = go.strides[2];
-            r.dqs_b = dq.strides[0], r.dqs_h = dq.strides[1], r.dqs_n = dq.strides[2];
-            r.dks_b = dk.strides[0], r.dks_h = dk.strides[1], r.dks_n = dk.strides[2];
-            r.dvs_b = dvv.strides[0], r.dvs_h = dvv.strides[1], r.dvs_n = dvv.strides[2];
-            r.H = (int32_t)H, r.N = (int32_t)N, r.BH = (int32_t)(B * H), r.wqk = (int32_t)dqk, r.wv = (int32_t)dv;
-            r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
+            fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv);
             r.init = entry, r.fmap = fmap;  // (dQ, dK: the slopes from phi(xq), phi(xk) in the Q and K tiles)
             r.init_is_totals = rev_sums_on_load;
             r.xinit = static_cast<const float *>(state_in);

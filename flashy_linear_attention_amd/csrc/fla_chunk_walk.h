@@ -119,8 +119,8 @@ struct WalkParams {
     // states (xinit, the layout of `init`, not transposed; may be null with a single segment).
     float *total_out;
     const float *xinit, *xtotal;
-    // D = 128, plain: the result (forward: o; walk_bwd_rev_kernel: dv) is added to what its place in
-    // memory holds already -- the second of two walks whose results sum up (halves of a wide q / k)
+    // D = 128, plain: the result (forward: o; walk_bwd_rev_kernel: dv, with 2 dq and dk as well) is added to what its
+    // place in memory holds already -- the second of two walks whose results sum up (halves of a wide q / k, of v)
     int32_t accumulate;
     // The wide walks (walk_fwd_wide_kernel, walk_bwd_rev_wide_kernel): q and k (dq and dk) have 129 .. 256
     // columns.  Columns 128 .. are the second half, of true width wqk2 (wqk = 128 is the first half's), with
@@ -136,6 +136,11 @@ struct WalkParams {
     // state they formed to entry_out / entry_out2 (the layout of init; null: nowhere), for the backward walk.
     int32_t init_is_totals;
     float *entry_out, *entry_out2;
+    // A v of 129 .. 256 columns beside a wide q / k: its columns 128 .. are a second half of true width wv2, and grid y
+    // picks a part of the work.  0: none.  1 (walk_fwd_wide_kernel): half y of v.  2, 3 (walk_bwd_rev_kernel): half y of
+    // q / k with half y (2) or half 1 - y (3) of v, so that the two parts of a launch write different columns.
+    // The states of (q / k half i, v half j) are matrices (2 j + i) BH .. of every state buffer.
+    int32_t quad, wv2;
 };
 
 template <int D>
@@ -1103,22 +1108,25 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
     const int rb = wave % W::NRB, db0 = OB::db0(wave);
     const WalkSlice sl = walk_slice(p);
     if (!sl.valid) return;
+    const int vh = p.quad ? (int)blockIdx.y : 0, wv = vh ? p.wv2 : p.wv;  // (the half of v that this workgroup takes)
+    WalkSlice ss = sl;  // (as sl, for the states)
+    ss.bh += 2 * vh * p.BH;
     const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
     const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
-    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
-    T *O = static_cast<T *>(p.o) + b * p.os_b + h * p.os_h;
+    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h + vh * D;
+    T *O = static_cast<T *>(p.o) + b * p.os_b + h * p.os_h + vh * D;
     const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2, os2 = (int)p.os_n * 2;
     const u32x4 rq0 = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
     const u32x4 rk0 = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
     const u32x4 rq1 = make_rsrc(Q + D, (uint32_t)((N - 1) * qs2 + p.wqk2 * 2));
     const u32x4 rk1 = make_rsrc(K + D, (uint32_t)((N - 1) * ks2 + p.wqk2 * 2));
-    const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
-    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(O, 0, (N - 1) * os2 + p.wv * 2, 0x00020000);
+    const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + wv * 2));
+    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(O, 0, (N - 1) * os2 + wv * 2, 0x00020000);
 
     f32x16 st0[W::NBW], st1[W::NBW];
     if (p.init_is_totals) {
-        const int64_t at = (int64_t)sl.bh * p.n_seg * (D * D);
+        const int64_t at = (int64_t)ss.bh * p.n_seg * (D * D);
         if constexpr (NV == 2) {  // (both halves' loads in flight together; with four blocks per wave and state, one half's)
             walk_sum_two<D, B>(p.init + at, p.init2 + at, 0, sl.seg, wave, lane, st0, st1);
         } else {
@@ -1130,8 +1138,8 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
             walk_write_state<D, B>(p.entry_out2 + at + (int64_t)sl.seg * (D * D), wave, lane, st1);
         }
     } else {
-        walk_load_init_from<D, B>(p.init, p, sl, wave, lane, st0, false);
-        walk_load_init_from<D, B>(p.init2, p, sl, wave, lane, st1, false);
+        walk_load_init_from<D, B>(p.init, p, ss, wave, lane, st0, false);
+        walk_load_init_from<D, B>(p.init2, p, ss, wave, lane, st1, false);
     }
     walk_state_to_lds<T, D, B>(tl, wave, lane, st0);
 
@@ -1142,7 +1150,7 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
         walk_load_tile<D>(HF ? rk1 : rk0, base + W::TILE, c * W::C, ks2, HF ? p.wqk2 : p.wqk, wave, lane);
     };
     auto v_slot = [&](int c) { return 4 + ((c - sl.c_lo) & 1); };
-    auto load_v = [&](int c) { walk_load_tile<D>(rv, lds0 + v_slot(c) * W::TILE, c * W::C, vs2, p.wv, wave, lane); };
+    auto load_v = [&](int c) { walk_load_tile<D>(rv, lds0 + v_slot(c) * W::TILE, c * W::C, vs2, wv, wave, lane); };
     auto sync = [&]() {  // this wave's LDS accesses are done; then every wave's
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0xc07f);
@@ -1179,14 +1187,14 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
         }
         sync();  // the tiles have landed, S_1 is in LDS
         walk_product<T, D, false, 0, B::KQ, NV, true>(tq1, tk1, tv, wave, lane, c > 0, sfrag, acc);
-        walk_store<T, D, OB::PER>(ro, os2, p.wv, row, g, db0, acc);
+        walk_store<T, D, OB::PER>(ro, os2, wv, row, g, db0, acc);
         walk_update<T, D, B>(tk1, tv, wave, lane, st1);
         sync();  // every wave has read S_1, this half's tiles and V
         walk_state_to_lds<T, D, B>(tl, wave, lane, st0);
     }
     if (p.total_out && sl.c_hi == p.n_chunks) {  // the states after the last chunk, for the backward walk
-        walk_write_state<D, B>(p.total_out + (int64_t)sl.bh * (D * D), wave, lane, st0);
-        walk_write_state<D, B>(p.total_out2 + (int64_t)sl.bh * (D * D), wave, lane, st1);
+        walk_write_state<D, B>(p.total_out + (int64_t)ss.bh * (D * D), wave, lane, st0);
+        walk_write_state<D, B>(p.total_out2 + (int64_t)ss.bh * (D * D), wave, lane, st1);
         // (NV = 2: the v blocks beyond stay unwritten -- walk_bwd_rev_wide_kernel, the reader, is built for the same extent)
     }
 #else
@@ -1472,7 +1480,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 // The one 16-bit state in LDS holds R for dV and dK, then X for dQ.  q, k, v, dO are read once and
 // nothing but the results is written, where the walk for dQ followed by walk_dkdv_kernel reads
 // dO, v, k twice.
-template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool ACCUM = false, bool FM = false>
+template <typename T, int D, int NQ = D / 32, int NV = D / 32, int ACCUM = 0, bool FM = false>
 __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1488,39 +1496,44 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
     const int rb = W::NCH == 1 ? wave : wave % W::NRB;
     const WalkSlice sl = walk_slice(p);
     if (!sl.valid) return;
+    // the column halves that this workgroup takes (WalkParams::quad)
+    const int qh = p.quad ? (int)blockIdx.y : 0, vh = p.quad == 3 ? 1 - qh : qh;
+    const int wqk = qh ? p.wqk2 : p.wqk, wv = vh ? p.wv2 : p.wv;
+    WalkSlice ss = sl;  // (as sl, for the states)
+    ss.bh += (2 * vh + qh) * p.BH;
     // FM: q and k hold y = phi(x); dQ and dK leave multiplied by the slope of phi, computed from the tiles
     const int fmap = FM ? p.fmap : 0;
     const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
-    const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
-    const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
-    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
-    const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
-    T *DQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h;
-    T *DK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h;
-    T *DV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
+    const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h + qh * D;
+    const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h + qh * D;
+    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h + vh * D;
+    const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h + vh * D;
+    T *DQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h + qh * D;
+    T *DK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h + qh * D;
+    T *DV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h + vh * D;
     const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2, gs2 = (int)p.gs_n * 2;
     const int dqs2 = (int)p.dqs_n * 2, dks2 = (int)p.dks_n * 2, dvs2 = (int)p.dvs_n * 2;
-    const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
-    const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
-    const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
-    const u32x4 rg = make_rsrc(G, (uint32_t)((N - 1) * gs2 + p.wv * 2));
-    const __amdgpu_buffer_rsrc_t rdq = __builtin_amdgcn_make_buffer_rsrc(DQ, 0, (N - 1) * dqs2 + p.wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdk = __builtin_amdgcn_make_buffer_rsrc(DK, 0, (N - 1) * dks2 + p.wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdv = __builtin_amdgcn_make_buffer_rsrc(DV, 0, (N - 1) * dvs2 + p.wv * 2, 0x00020000);
+    const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + wqk * 2));
+    const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + wqk * 2));
+    const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + wv * 2));
+    const u32x4 rg = make_rsrc(G, (uint32_t)((N - 1) * gs2 + wv * 2));
+    const __amdgpu_buffer_rsrc_t rdq = __builtin_amdgcn_make_buffer_rsrc(DQ, 0, (N - 1) * dqs2 + wqk * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rdk = __builtin_amdgcn_make_buffer_rsrc(DK, 0, (N - 1) * dks2 + wqk * 2, 0x00020000);
+    const __amdgpu_buffer_rsrc_t rdv = __builtin_amdgcn_make_buffer_rsrc(DV, 0, (N - 1) * dvs2 + wv * 2, 0x00020000);
 
     f32x16 st[W::NBW];  // R [q/k index][v index]
     f32x16 xs[W::NBW];  // X [q/k index][v index]
-    walk_load_init<D, B>(p, sl, wave, lane, st, true);
-    walk_load_end_state<D, B>(p, sl, wave, lane, xs);
+    walk_load_init<D, B>(p, ss, wave, lane, st, true);
+    walk_load_end_state<D, B>(p, ss, wave, lane, xs);
     walk_state_to_lds<T, D, B>(tl, wave, lane, st);
 
     auto load_chunk = [&](int c, int buf) {
         const uint32_t base = lds0 + buf * 4 * W::TILE;
         const int row0 = c * W::C;
-        walk_load_tile<D>(rq, base, row0, qs2, p.wqk, wave, lane);
-        walk_load_tile<D>(rk, base + W::TILE, row0, ks2, p.wqk, wave, lane);
-        walk_load_tile<D>(rv, base + 2 * W::TILE, row0, vs2, p.wv, wave, lane);
-        walk_load_tile<D>(rg, base + 3 * W::TILE, row0, gs2, p.wv, wave, lane);
+        walk_load_tile<D>(rq, base, row0, qs2, wqk, wave, lane);
+        walk_load_tile<D>(rk, base + W::TILE, row0, ks2, wqk, wave, lane);
+        walk_load_tile<D>(rv, base + 2 * W::TILE, row0, vs2, wv, wave, lane);
+        walk_load_tile<D>(rg, base + 3 * W::TILE, row0, gs2, wv, wave, lane);
     };
     auto sync = [&]() {  // this wave's LDS accesses are done; then every wave's
         asm volatile("" ::: "memory");
@@ -1528,8 +1541,9 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    // ACCUM: dV is added to what dv holds (in fp32, before the one rounding)
+    // ACCUM 1, 2: dV, 2: dK and dQ too are added to what their places hold (in fp32, before the one rounding)
     WalkPrev<T, D, OV::PER> prev;
+    WalkPrev<T, D, OQ::PER> prev_qk;
     load_chunk(sl.c_hi - 1, 0);
 #pragma unroll 1
     for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
@@ -1546,25 +1560,29 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
         sync();  // the tiles have landed, R is in LDS
         const int row = c * W::C + 32 * rb + l32;
         const bool later = c + 1 < p.n_chunks;  // chunks after this one exist: R is not identically zero
-        if constexpr (ACCUM) prev.request(rdv, dvs2, p.wv, row, g, OV::db0(wave));
+        if constexpr (ACCUM) prev.request(rdv, dvs2, wv, row, g, OV::db0(wave));
         walk_update<T, D, B, true, true>(tk, tv, wave, lane, xs);  // X: now the sum over the chunks before this one
         f32x16 acc[W::DBW];
         // dV = upper(K Q^T) dO + K R: A operand R^T[v index][q/k index] = the LDS copy as it is
         walk_product<T, D, true, 0, B::KQ, NV>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
         }, acc);
-        f32x16 held[W::DBW];  // ACCUM: dV waits for the end of the chunk (see WalkPrev)
-        if constexpr (ACCUM) {
+        // ACCUM 1: dV waits for the end of the chunk (see WalkPrev).  (2: no registers left for that)
+        f32x16 held[W::DBW];
+        if constexpr (ACCUM == 1) {
 #pragma unroll
             for (int i = 0; i < OV::PER; ++i) held[i] = acc[i];
         } else {
-            walk_store<T, D, OV::PER>(rdv, dvs2, p.wv, row, g, OV::db0(wave), acc);
+            if constexpr (ACCUM == 2) prev.add_to(acc);
+            walk_store<T, D, OV::PER>(rdv, dvs2, wv, row, g, OV::db0(wave), acc);
         }
+        if constexpr (ACCUM == 2) prev_qk.request(rdk, dks2, wqk, row, g, OQ::db0(wave));
         // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
         walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
-        walk_store<T, D, OQ::PER>(rdk, dks2, p.wqk, row, g, OQ::db0(wave), acc, fmap, tk, 32 * rb + l32);
+        if constexpr (ACCUM == 2) prev_qk.add_to(acc);
+        walk_store<T, D, OQ::PER>(rdk, dks2, wqk, row, g, OQ::db0(wave), acc, fmap, tk, 32 * rb + l32);
         // R += Q^T dO touches registers and tiles only, so it can sit on either side of the barriers: the waves of
         // the last row block, with one score block in dV and dK against two, take it here, the others after dQ,
         // where they have one score block against two
@@ -1580,14 +1598,16 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
             asm volatile("" : "+a"(xs[0]), "+a"(xs[1]));
         walk_state_to_lds<T, D, B>(tl, wave, lane, xs);
         sync();  // X is in LDS
+        if constexpr (ACCUM == 2) prev_qk.request(rdq, dqs2, wqk, row, g, OQ::db0(wave));
         // dQ = lower(dO V^T) K + dO X^T: A operand X[q/k index][v index], read transposed like R for dK
         walk_product<T, D, false, 0, B::KV, NQ>(tg, tv, tk, wave, lane, c > 0, [&](int db, int kc) -> V8 {
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
-        walk_store<T, D, OQ::PER>(rdq, dqs2, p.wqk, row, g, OQ::db0(wave), acc, fmap, tq, 32 * rb + l32);
-        if constexpr (ACCUM) {
+        if constexpr (ACCUM == 2) prev_qk.add_to(acc);
+        walk_store<T, D, OQ::PER>(rdq, dqs2, wqk, row, g, OQ::db0(wave), acc, fmap, tq, 32 * rb + l32);
+        if constexpr (ACCUM == 1) {
             prev.add_to(held);
-            walk_store<T, D, OV::PER>(rdv, dvs2, p.wv, row, g, OV::db0(wave), held);
+            walk_store<T, D, OV::PER>(rdv, dvs2, wv, row, g, OV::db0(wave), held);
         }
         if (!(kSplitUpdate && rb == 1)) walk_update<T, D, B, false, true>(tq, tg, wave, lane, st);
         sync();  // every wave has read X and is done with the tiles
@@ -1758,17 +1778,23 @@ struct WalkTotalsParams {
     const void *y2;
     int32_t dy2;
     float *totals2;
+    // walk_totals_quad_kernel: true width of Z's second half (its columns 128 ..), 0: Z has one half.  The totals of
+    // (Y half i, Z half j) are matrices (2 j + i) BH n_seg .. of `totals` (totals2 = totals + BH n_seg D D).
+    int32_t dz2;
+    // nobody reads the totals' columns 64 .. (every walk behind them leaves a narrow z's padding out): they may stay
+    // unwritten for a narrow y as well
+    int32_t z_narrow;
 };
 
 constexpr int walk_totals_sets(int D) { return D == 128 ? 4 : 2; }  // sets of (Y, Z) tiles in LDS
 
 // BOTH (D = 128, NV = 2): the launch's two Y operands (WalkTotalsParams::y2) in ONE workgroup -- three sets of
 // (Y, Y2, Z) tiles, a state per operand -- so that Z is loaded once for the two; otherwise grid y picks the operand.
-template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool BOTH = false>
-__global__ __launch_bounds__(256, BOTH ? 1 : 2) void walk_totals_kernel(const WalkTotalsParams p) {
-#if defined(__HIP_DEVICE_COMPILE__)
+template <typename T, int D, int NQ, int NV, bool BOTH>
+__device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     using W = WalkCfg<D>;
-    static_assert(!BOTH || (D == 128 && NV == 2), "two states per wave: built for the narrow v side of D = 128");
+    static_assert(!BOTH || D == 128, "halves of 128 columns");
+    const int zh = BOTH && p.dz2 ? (int)blockIdx.y : 0, dz = zh ? p.dz2 : p.dz;  // (the half of Z: walk_totals_quad_kernel)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
@@ -1801,6 +1827,7 @@ __global__ __launch_bounds__(256, BOTH ? 1 : 2) void walk_totals_kernel(const Wa
         c_lo = seg * p.seg_chunks;
         c_hi = c_lo + p.seg_chunks < p.n_chunks ? c_lo + p.seg_chunks : p.n_chunks;
     }
+    out_at += (int64_t)2 * zh * p.BH * p.n_seg * (D * D);
     float *const out = (second ? p.totals2 : p.totals) + out_at;
     float *const out2 = BOTH ? p.totals2 + out_at : nullptr;
     if (c_lo >= c_hi) {  // nothing to add up (a segment beyond the end of the sequence, the second half of one chunk)
@@ -1814,11 +1841,11 @@ __global__ __launch_bounds__(256, BOTH ? 1 : 2) void walk_totals_kernel(const Wa
     const int b = bh / p.H, h = bh - b * p.H, N = p.N;
     const T *Y = static_cast<const T *>(second ? p.y2 : p.y) + b * p.ys_b + h * p.ys_h;
     const T *Y2 = static_cast<const T *>(BOTH ? p.y2 : p.y) + b * p.ys_b + h * p.ys_h;
-    const T *Z = static_cast<const T *>(p.z) + b * p.zs_b + h * p.zs_h;
+    const T *Z = static_cast<const T *>(p.z) + b * p.zs_b + h * p.zs_h + zh * D;
     const int ys2 = (int)p.ys_n * 2, zs2 = (int)p.zs_n * 2;
     const u32x4 ry = make_rsrc(Y, (uint32_t)((N - 1) * ys2 + dy * 2));
     const u32x4 ry2 = make_rsrc(Y2, (uint32_t)((N - 1) * ys2 + (BOTH ? p.dy2 : dy) * 2));
-    const u32x4 rz = make_rsrc(Z, (uint32_t)((N - 1) * zs2 + p.dz * 2));
+    const u32x4 rz = make_rsrc(Z, (uint32_t)((N - 1) * zs2 + dz * 2));
     using B = WalkExt<D, NQ, NV>;  // (blocks outside it stay unwritten: no walk of the same extent reads them)
     f32x16 st[W::NBW], st2[W::NBW];
 #pragma unroll
@@ -1833,7 +1860,7 @@ __global__ __launch_bounds__(256, BOTH ? 1 : 2) void walk_totals_kernel(const Wa
         const uint32_t base = lds0 + set * TPS * W::TILE;
         walk_load_tile<D>(ry, base, c * W::C, ys2, dy, wave, lane);
         if constexpr (BOTH) walk_load_tile<D>(ry2, base + W::TILE, c * W::C, ys2, p.dy2, wave, lane);
-        walk_load_tile<D>(rz, base + (TPS - 1) * W::TILE, c * W::C, zs2, p.dz, wave, lane);
+        walk_load_tile<D>(rz, base + (TPS - 1) * W::TILE, c * W::C, zs2, dz, wave, lane);
     };
     auto map_tile = [&](unsigned char *ty, int c) {
         walk_map_tile<T, D>(ty, p.map_y, c * W::C, N, dy, static_cast<T *>(p.ymap_out) + b * p.yo_b + h * p.yo_h,
@@ -1903,6 +1930,23 @@ __global__ __launch_bounds__(256, BOTH ? 1 : 2) void walk_totals_kernel(const Wa
                 if constexpr (BOTH) out2[at] = st2[i][v];
             }
         }
+}
+
+template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool BOTH = false>
+__global__ __launch_bounds__(256, BOTH ? 1 : 2) void walk_totals_kernel(const WalkTotalsParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    walk_totals_body<T, D, NQ, NV, BOTH>(p);
+#else
+    (void)p;
+#endif
+}
+
+// All four pairs of 128-column halves of Y and Z (a v wider than 128 columns beside a wide q / k) in one launch: a
+// workgroup takes both halves of Y, grid y picks the half of Z.
+template <typename T>
+__global__ __launch_bounds__(256, 1) void walk_totals_quad_kernel(const WalkTotalsParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    walk_totals_body<T, 128, 4, 4, true>(p);
 #else
     (void)p;
 #endif
@@ -2063,17 +2107,29 @@ hipError_t launch_walk_totals(const WalkTotalsParams &p, hipStream_t stream) {
     constexpr int smem = walk_totals_sets(D) * 2 * WalkCfg<D>::TILE;
     if (p.direct && (p.n_seg != 2 || p.seg_lo < 0 || p.seg_lo > 1)) return hipErrorInvalidValue;
     // (a second operand runs the same kernel variant: the caller pairs operands of one kind only)
-    if (p.y2 && (p.map_y || !p.totals2 || walk_totals_cols(D, p.dy2, p.dz) != walk_totals_cols(D, p.dy, p.dz)))
+    if (p.y2 && (p.map_y || !p.totals2 ||
+                 (!p.z_narrow && walk_totals_cols(D, p.dy2, p.dz) != walk_totals_cols(D, p.dy, p.dz))))
         return hipErrorInvalidValue;
+    if (p.dz2 || p.z_narrow) {
+        if (D != 128 || (p.dz2 && (!p.y2 || p.dy != 128 || p.dz != 128 || p.dz2 < 1 || p.dz2 > 128 || p.z_narrow)) ||
+            (p.z_narrow && p.dz > 64))
+            return hipErrorInvalidValue;
+    }
     const dim3 g((unsigned)grid, p.y2 ? 2u : 1u);
     if constexpr (D == 128) {
-        if (p.y2 && walk_totals_cols(D, p.dy, p.dz) == 64) {  // ... and both operands in one workgroup: z loaded once
+        constexpr int smem_both = 3 * 3 * WalkCfg<D>::TILE;
+        if (p.dz2) {
+            constexpr auto kern = walk_totals_quad_kernel<T>;
+            if (hipError_t e = ensure_dynamic_lds<kern>(smem_both)) return e;
+            return launch_kernel<kern>(dim3((unsigned)grid, 2u), dim3(256), smem_both, stream, p);
+        }
+        const bool narrow = p.z_narrow || walk_totals_cols(D, p.dy, p.dz) == 64;
+        if (p.y2 && narrow) {  // ... and both operands in one workgroup: z loaded once
             constexpr auto kern = walk_totals_kernel<T, D, 4, 2, true>;
-            constexpr int smem_both = 3 * 3 * WalkCfg<D>::TILE;
             if (hipError_t e = ensure_dynamic_lds<kern>(smem_both)) return e;
             return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_both, stream, p);
         }
-        if (walk_totals_cols(D, p.dy, p.dz) == 64) {  // z of at most 64 true columns: the state's other v blocks hold zeros
+        if (narrow) {  // z of at most 64 true columns: the state's other v blocks hold zeros
             constexpr auto kern = walk_totals_kernel<T, D, 4, 2>;
             if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
             return launch_kernel<kern>(g, dim3(256), smem, stream, p);
@@ -2096,9 +2152,9 @@ inline hipError_t launch_walk_scan(const float *totals, float *entry, int64_t BH
 }
 
 template <auto kern>
-hipError_t launch_walk_kernel(int64_t grid, int smem, const WalkParams &p, hipStream_t stream) {
+hipError_t launch_walk_kernel(int64_t grid, int smem, const WalkParams &p, hipStream_t stream, int parts = 1) {
     if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
-    return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
+    return launch_kernel<kern>(dim3((unsigned)grid, (unsigned)parts), dim3(256), smem, stream, p);
 }
 
 template <typename T, int D>
@@ -2147,6 +2203,10 @@ hipError_t launch_walk_fwd_wide(const WalkParams &p, hipStream_t stream) {
         (p.entry_out != nullptr) != (p.entry_out2 != nullptr) || (p.entry_out && !p.init_is_totals))
         return hipErrorInvalidValue;
     constexpr int smem = 6 * W::TILE + W::STATE;  // two sets of (Q_h, K_h), two V tiles, one state
+    if (p.quad) {
+        if (p.quad != 1 || p.wv != 128 || p.wv2 < 1 || p.wv2 > 128) return hipErrorInvalidValue;
+        return launch_walk_kernel<walk_fwd_wide_kernel<T, 4>>(grid, smem, p, stream, 2);
+    }
     if (p.wv <= 64) return launch_walk_kernel<walk_fwd_wide_kernel<T, 2>>(grid, smem, p, stream);
     return launch_walk_kernel<walk_fwd_wide_kernel<T, 4>>(grid, smem, p, stream);
 }
@@ -2202,16 +2262,23 @@ hipError_t launch_walk_bwd_rev(const WalkParams &p, hipStream_t stream) {
     if (p.entry_out || (p.init_is_totals && (p.n_seg < 3 || !p.init))) return hipErrorInvalidValue;
     constexpr int smem = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     static_assert(smem <= 160 * 1024, "two sets of tiles and the state must fit the LDS of a CU");
+    if (p.quad) {
+        if ((p.quad != 2 && p.quad != 3) || p.wqk != 128 || p.wv != 128 || p.wqk2 < 1 || p.wqk2 > 128 || p.wv2 < 1 ||
+            p.wv2 > 128 || p.fmap || p.accumulate == 1)
+            return hipErrorInvalidValue;
+        return p.accumulate ? launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, 2>>(grid, smem, p, stream, 2)
+                            : launch_walk_kernel<walk_bwd_rev_kernel<T, D>>(grid, smem, p, stream, 2);
+    }
     if constexpr (D == 128) {  // a half of a wide q / k against a narrow v: without the blocks of padding
         if (!p.fmap && p.wqk > 64 && p.wv <= 64)
-            return p.accumulate ? launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2, true>>(grid, smem, p, stream)
+            return p.accumulate ? launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2, 1>>(grid, smem, p, stream)
                                 : launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2>>(grid, smem, p, stream);
     }
     if (p.fmap) {
         if (p.accumulate) return hipErrorNotSupported;
-        return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, false, true>>(grid, smem, p, stream);
+        return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, 0, true>>(grid, smem, p, stream);
     }
-    if (p.accumulate) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, true>>(grid, smem, p, stream);
+    if (p.accumulate) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, 1>>(grid, smem, p, stream);
     return launch_walk_kernel<walk_bwd_rev_kernel<T, D>>(grid, smem, p, stream);
 }
 
