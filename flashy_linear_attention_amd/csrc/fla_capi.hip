@@ -449,8 +449,9 @@ struct EntryHalf {
 int walk_entry_states(const WalkPlan &w, const View &y, const View &z, int64_t B, int64_t H, int64_t N, int64_t dy,
                       int64_t dz, int dtype, int reverse, void *work, float *entry, const float **where, hipStream_t s,
                       int map_y = 0, const View *ymap_out = nullptr, const EntryHalf *second = nullptr,
-                      bool totals_only = false, bool z_narrow = false) {
+                      bool totals_only = false, bool z_narrow = false, float *vsum = nullptr) {
     fla::WalkTotalsParams tp{};
+    tp.vsum = vsum;
     tp.z_narrow = z_narrow;
     if (map_y) {
         tp.map_y = map_y, tp.ymap_out = const_cast<void *>(ymap_out->ptr);
@@ -973,7 +974,8 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
             if (int rc = walk_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0,
                                            in_state && !sum_on_load ? state_out : workspace,
                                            in_state && !sum_on_load ? static_cast<float *>(state_out) : nullptr, &entry, s,
-                                           fmap, fmap ? &mapped[1] : nullptr, nullptr, sum_on_load))
+                                           fmap, fmap ? &mapped[1] : nullptr, nullptr, sum_on_load, false,
+                                           nx ? static_cast<float *>(nx->vec) : nullptr))
                 return rc;
         const View &kk = fmap ? mapped[1] : k;
         fla::WalkParams w{};
@@ -991,12 +993,10 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         w.init = wp.n_seg > 1 ? entry : nullptr, w.saved = in_state ? nullptr : state_out;
         if (sum_on_load) w.init_is_totals = 1, w.entry_out = in_state ? static_cast<float *>(state_out) : nullptr;
         if (in_state) w.total_out = reinterpret_cast<float *>(static_cast<char *>(state_out) + wp.entry_bytes);
-        if (nx) {  // the normaliser inside the walk: zc = running sum of k at the entry of every chunk
-            // (kept behind the state, when there is one, for backward)
-            float *zc = state_out ? reinterpret_cast<float *>(static_cast<char *>(state_out) + state_core_bytes(B, H, N, dqk, dv))
-                                  : static_cast<float *>(nx->vec);
-            if (int rc = walk_chunk_vectors(wp, kk, dqk, nullptr, 0, zc, B, H, N, dtype, s)) return rc;
-            w.denom = nx->denom, w.eps = nx->eps, w.zc = zc;
+        if (nx) {  // the normaliser inside the walk, which carries the running sum of k from the segments' totals of it
+            // (kept for backward, at the entry of every chunk, behind the state when there is one)
+            w.denom = nx->denom, w.eps = nx->eps, w.vsum = wp.n_seg > 1 ? static_cast<const float *>(nx->vec) : nullptr;
+            if (state_out) w.zc_out = reinterpret_cast<float *>(static_cast<char *>(state_out) + state_core_bytes(B, H, N, dqk, dv));
             nx->fused = true;
         }
         if (fla::walk_fwd(dtype, wp.D, w, s) != hipSuccess) return FLA_ERR_LAUNCH;

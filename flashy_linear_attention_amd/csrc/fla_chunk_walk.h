@@ -105,13 +105,16 @@ struct WalkParams {
     const void *slope_y;
     int64_t sy_b, sy_h, sy_n;
     // The normaliser n_i = q_i . (k_0 + ... + k_i) + eps fused into the walks (null pointers: off).
-    // Forward (denom, zc): n_i = sum of row i's masked scores + q_i . zc_c; the result is divided by
-    // n_i and n goes to denom.  Backward, with dn_i = -(g_i . out_i) / n_i and dO = g / n prepared by
+    // Forward (denom): n_i = sum of row i's masked scores + q_i . zc_c, with zc_c carried by the walk beside the
+    // state (walk_col_sums; vsum: the segments' totals of k from the totals kernel, null with a single segment) and
+    // written to zc_out (null: nowhere) for backward; the result is divided by n_i and n goes to denom.  Backward, with dn_i = -(g_i . out_i) / n_i and dO = g / n prepared by
     // the caller: dQ's scores get + dn_i and its result + dn_i zc_c (dn, zc); dK's scores get + dn_i
     // (i: the dO row) and its result + rc_c (dn, rc).
     float *denom;     // fp32 [BH][N]
     float eps;
-    const float *zc;  // fp32 [BH][n_chunks][D]: sum of k over the rows before chunk c
+    const float *zc;  // fp32 [BH][n_chunks][D]: sum of k over the rows before chunk c (backward)
+    const float *vsum;  // fp32 [BH][n_seg][D], slots as those of `init` (two segments: partial sums in both)
+    float *zc_out;      // as zc
     const float *dn;  // fp32 [BH][N]
     const float *rc;  // fp32 [BH][n_chunks][D]: sum of dn_i q_i over the rows after chunk c
     // Forward, D = 128: where the state after the last chunk of every (b, h) goes, fp32 [BH][D][D]
@@ -653,6 +656,42 @@ __device__ __forceinline__ void walk_update(const unsigned char *yt, const unsig
     }
 }
 
+// acc += column sums of the tile's rows (all of them, or this wave's part: with fewer than four 32-column blocks the
+// waves of a block share the rows), by MFMAs against a fragment of ones: exact products, fp32 sums, four MFMAs per wave
+// and chunk.  Every lane column holds the same sums: acc[v] of column 32 (wave % DB) + 8(v/4) + 4g + v%4.
+template <typename T, int D>
+__device__ __forceinline__ void walk_col_sums(const unsigned char *yt, int wave, int lane, f32x16 &acc) {
+    using W = WalkCfg<D>;
+    using V8 = typename Mma<T>::V8;
+    constexpr int KS = W::C / 16 / (4 / W::DB);  // 16-row steps per wave
+    V8 ones;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) ones[e] = static_cast<T>(1.0f);
+    static_for<0, KS>([&](auto j) {
+        const int ks = (wave / W::DB) * KS + decltype(j)::value;
+        acc = Mma<T>::mma(walk_col_frag<T, D>(yt, 16 * ks, wave % W::DB, lane), ones, acc);
+    });
+}
+// ... to LDS: part[wave / DB][column], 4 / DB parts of D floats
+template <int D>
+__device__ __forceinline__ void walk_col_sums_to_lds(float *part, int wave, int lane, const f32x16 &acc) {
+    constexpr int DB = D / 32;
+    typedef float f32x4_ __attribute__((ext_vector_type(4)));
+    if ((lane & 31) == 0) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+            *reinterpret_cast<f32x4_ *>(part + (wave / DB) * D + 32 * (wave % DB) + 8 * a + 4 * (lane >> 5)) =
+                f32x4_{acc[4 * a], acc[4 * a + 1], acc[4 * a + 2], acc[4 * a + 3]};
+    }
+}
+template <int D>
+__device__ __forceinline__ float walk_col_sum_of(const float *part, int col) {
+    float t = 0.f;
+#pragma unroll
+    for (int u = 0; u < 4 / (D / 32); ++u) t += part[u * D + col];
+    return t;
+}
+
 // the state rounded to 16 bit into LDS as T[v index][q/k index] (row = 32 eb + l32, four consecutive
 // columns per register group), in the tile layout
 template <typename T, int D, typename B = WalkExt<D>>
@@ -916,7 +955,8 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
     unsigned char *tl = smem + SETS * 3 * W::TILE;
-    unsigned char *xv = tl + W::STATE;  // per set: zc, (unused), dn of the chunk
+    unsigned char *xv = tl + W::STATE;  // NORM 2: per set: zc, (unused), dn of the chunk
+    float *zv = reinterpret_cast<float *>(xv), *zpart = zv + 256;  // NORM 1: zc; the waves' column sums
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int rb = W::NCH == 1 ? wave : wave % W::NRB, db0 = OB::db0(wave);
@@ -942,6 +982,29 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
             walk_write_state<D, B>(p.entry_out + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D), wave, lane, st);
     }
     walk_state_to_lds<T, D, B>(tl, wave, lane, st);
+    // NORM 1: zc at the segment's entry from the segments' totals, thread groups of D taking every (256 / D)-th segment
+    float zrun = 0.f;  // (of column tid, tid < D)
+    auto zc_publish = [&](int c) {
+        zv[tid] = zrun;
+        if (p.zc_out) p.zc_out[((int64_t)sl.bh * p.n_chunks + c) * D + tid] = zrun;
+    };
+    if constexpr (NORM == 1) {
+        constexpr int G = 256 / D;
+        float t = 0.f;
+        if (p.vsum) {
+            const float *vs = p.vsum + (int64_t)sl.bh * p.n_seg * D + tid % D;
+            const int before = p.n_seg == 2 ? (sl.seg ? 2 : 0) : sl.seg;
+#pragma unroll 8
+            for (int f = tid / D; f < before; f += G) t += vs[(int64_t)f * D];
+        }
+        zpart[tid] = t;
+        __syncthreads();
+        if (tid < D) {
+#pragma unroll
+            for (int u = 0; u < G; ++u) zrun += zpart[u * D + tid];
+            zc_publish(sl.c_lo);
+        }
+    }
 
     auto load_chunk = [&](int c, int buf) {
         const uint32_t base = lds0 + buf * 3 * W::TILE;
@@ -949,12 +1012,12 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         walk_load_tile<D>(rk, base + W::TILE, c * W::C, ks2, p.wqk, wave, lane);
         walk_load_tile<D>(rv, base + 2 * W::TILE, c * W::C, vs2, p.wv, wave, lane);
         const uint32_t xbase = lds0 + SETS * 3 * W::TILE + W::STATE + buf * W::VEC;
-        if constexpr (NORM) {
+        if constexpr (NORM == 2) {
             walk_load_vec<D>(p.zc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase, lane);
-            if constexpr (NORM == 2) walk_load_rows<D>(p.dn + (int64_t)sl.bh * N, c * W::C, N, xbase + 2048, lane);
+            walk_load_rows<D>(p.dn + (int64_t)sl.bh * N, c * W::C, N, xbase + 2048, lane);
         }
     };
-    constexpr int n_extra = NORM == 0 ? 0 : NORM == 1 ? 1 : 1 + W::NID;  // loads per chunk and wave beyond the tiles
+    constexpr int n_extra = NORM == 2 ? 1 + W::NID : 0;  // loads per chunk and wave beyond the tiles
     // ACCUM: the result is added to what o holds (in fp32, before the one rounding)
     WalkPrev<T, D, OB::PER> prev;
     if constexpr (DOUBLE) load_chunk(sl.c_lo, 0);
@@ -1009,7 +1072,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         }
         if constexpr (ACCUM) prev.request(ro, os2, p.wv, row, g, db0);
         f32x16 acc[W::DBW];
-        const float *vz = reinterpret_cast<const float *>(xv + buf * W::VEC);
+        const float *vz = reinterpret_cast<const float *>(xv + (NORM == 1 ? 0 : buf * W::VEC));
         const float *vd = reinterpret_cast<const float *>(xv + buf * W::VEC + 2048);
         auto sfrag = [&](int db, int kc) -> V8 { return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g); };
         if constexpr (NORM == 1) {  // forward with the normaliser: n = masked row sum + q . zc + eps
@@ -1051,6 +1114,13 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                 }
         }
         walk_update<T, D, B>(tk, tv, wave, lane, st);
+        if constexpr (NORM == 1) {
+            f32x16 zs;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) zs[v] = 0.f;
+            walk_col_sums<T, D>(tk, wave, lane, zs);
+            walk_col_sums_to_lds<D>(zpart, wave, lane, zs);
+        }
         if constexpr (DOUBLE) {
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_waitcnt(0xc07f);  // this wave's LDS reads of the tiles and of the state are done
@@ -1060,6 +1130,12 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
             __syncthreads();  // every wave is done with the tiles and with the old state
         }
         walk_state_to_lds<T, D, B>(tl, wave, lane, st);
+        if constexpr (NORM == 1) {
+            if (tid < D && c + 1 < sl.c_hi) {
+                zrun += walk_col_sum_of<D>(zpart, tid);
+                zc_publish(c + 1);
+            }
+        }
     }
     if (p.total_out && sl.c_hi == p.n_chunks) {  // the state after the last chunk, for the backward walks
         float *out = p.total_out + (int64_t)sl.bh * (D * D);
@@ -1781,6 +1857,9 @@ struct WalkTotalsParams {
     // walk_totals_quad_kernel: true width of Z's second half (its columns 128 ..), 0: Z has one half.  The totals of
     // (Y half i, Z half j) are matrices (2 j + i) BH n_seg .. of `totals` (totals2 = totals + BH n_seg D D).
     int32_t dz2;
+    // The totals of Y's rows, fp32 [BH][n_seg][D], in the slots of `totals` -- the normaliser's running sum of k at the
+    // segments' entries (WalkParams::vsum); null: not formed.  One operand only.
+    float *vsum;
     // nobody reads the totals' columns 64 .. (every walk behind them leaves a narrow z's padding out): they may stay
     // unwritten for a narrow y as well
     int32_t z_narrow;
@@ -1835,6 +1914,7 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
             out[i] = 0.f;
             if constexpr (BOTH) out2[i] = 0.f;
         }
+        if (p.vsum && tid < D) p.vsum[out_at / D + tid] = 0.f;
         return;
     }
     const bool discard = p.direct && p.map_y && seg != p.seg_lo;  // (visited for the map only)
@@ -1847,7 +1927,9 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     const u32x4 ry2 = make_rsrc(Y2, (uint32_t)((N - 1) * ys2 + (BOTH ? p.dy2 : dy) * 2));
     const u32x4 rz = make_rsrc(Z, (uint32_t)((N - 1) * zs2 + dz * 2));
     using B = WalkExt<D, NQ, NV>;  // (blocks outside it stay unwritten: no walk of the same extent reads them)
-    f32x16 st[W::NBW], st2[W::NBW];
+    f32x16 st[W::NBW], st2[W::NBW], zs;  // (zs: the column sums of Y, with vsum)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) zs[v] = 0.f;
 #pragma unroll
     for (int i = 0; i < W::NBW; ++i)
 #pragma unroll
@@ -1887,6 +1969,7 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
             asm volatile("" ::: "memory");
             if (p.map_y) map_tile(ty, c);
             walk_update<T, D, B>(ty, tz, wave, lane, st);
+            if (p.vsum) walk_col_sums<T, D>(ty, wave, lane, zs);
             asm volatile("" ::: "memory");
             __builtin_amdgcn_s_waitcnt(0xc07f);  // this wave's LDS reads of the set are done
             __builtin_amdgcn_s_barrier();
@@ -1916,6 +1999,8 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
             if (p.map_y) map_tile(ty, c);
             walk_update<T, D, B>(ty, tz, wave, lane, st);
             if constexpr (BOTH) walk_update<T, D, B>(ty + W::TILE, tz, wave, lane, st2);
+            if constexpr (!BOTH && NV == W::DB)
+                if (p.vsum) walk_col_sums<T, D>(ty, wave, lane, zs);
             asm volatile("" ::: "memory");
             set = (set + 1) % SETS;
         }
@@ -1930,6 +2015,13 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
                 if constexpr (BOTH) out2[at] = st2[i][v];
             }
         }
+    if (p.vsum) {  // (no loads into LDS are in flight any more)
+        float *part = reinterpret_cast<float *>(smem);
+        __syncthreads();
+        walk_col_sums_to_lds<D>(part, wave, lane, zs);
+        __syncthreads();
+        if (tid < D) p.vsum[out_at / D + tid] = discard ? 0.f : walk_col_sum_of<D>(part, tid);
+    }
 }
 
 template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool BOTH = false>
@@ -2110,6 +2202,7 @@ hipError_t launch_walk_totals(const WalkTotalsParams &p, hipStream_t stream) {
     if (p.y2 && (p.map_y || !p.totals2 ||
                  (!p.z_narrow && walk_totals_cols(D, p.dy2, p.dz) != walk_totals_cols(D, p.dy, p.dz))))
         return hipErrorInvalidValue;
+    if (p.vsum && (p.y2 || p.dz2 || (D == 128 && walk_totals_cols(D, p.dy, p.dz) == 64))) return hipErrorInvalidValue;
     if (p.dz2 || p.z_narrow) {
         if (D != 128 || (p.dz2 && (!p.y2 || p.dy != 128 || p.dz != 128 || p.dz2 < 1 || p.dz2 > 128 || p.z_narrow)) ||
             (p.z_narrow && p.dz > 64))
@@ -2168,7 +2261,7 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     if (p.init_is_totals && (D != 128 || p.n_seg < 3 || !p.init)) return hipErrorInvalidValue;
     if (p.entry_out && (!p.init_is_totals || fm || p.denom || p.dn)) return hipErrorInvalidValue;
     if (p.denom || p.dn) {  // the normaliser's terms: its vectors live behind the state
-        if (!p.zc || p.accumulate) return hipErrorInvalidValue;
+        if ((p.dn && !p.zc) || (p.denom && p.n_seg > 1 && !p.vsum) || p.accumulate) return hipErrorInvalidValue;
         constexpr int smem_n = smem + (kDouble ? 2 : 1) * WalkCfg<D>::VEC;
         if (p.denom)
             return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 1, true>>(grid, smem_n, p, stream)

@@ -65,7 +65,7 @@ FLA_FIELD(qo_b) FLA_FIELD(qo_h) FLA_FIELD(qo_n) FLA_FIELD(slope_y) FLA_FIELD(sy_
 FLA_FIELD(denom) FLA_FIELD(eps) FLA_FIELD(zc) FLA_FIELD(dn) FLA_FIELD(rc) FLA_FIELD(total_out) FLA_FIELD(xinit)
 FLA_FIELD(xtotal) FLA_FIELD(accumulate)
     FLA_FIELD(wqk2) FLA_FIELD(init2) FLA_FIELD(total_out2) FLA_FIELD(xinit2) FLA_FIELD(xtotal2)
-    FLA_FIELD(init_is_totals) FLA_FIELD(entry_out) FLA_FIELD(entry_out2) FLA_FIELD(quad) FLA_FIELD(wv2)
+    FLA_FIELD(init_is_totals) FLA_FIELD(entry_out) FLA_FIELD(entry_out2) FLA_FIELD(quad) FLA_FIELD(wv2) FLA_FIELD(vsum) FLA_FIELD(zc_out)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(WalkTotalsParams)
@@ -73,7 +73,7 @@ FLA_FIELD(y) FLA_FIELD(z) FLA_FIELD(ys_b) FLA_FIELD(ys_h) FLA_FIELD(ys_n) FLA_FI
 FLA_FIELD(zs_n) FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(dy) FLA_FIELD(dz) FLA_FIELD(n_chunks)
 FLA_FIELD(seg_chunks) FLA_FIELD(n_seg) FLA_FIELD(seg_lo) FLA_FIELD(seg_hi) FLA_FIELD(totals) FLA_FIELD(direct)
 FLA_FIELD(map_y) FLA_FIELD(ymap_out) FLA_FIELD(yo_b) FLA_FIELD(yo_h) FLA_FIELD(yo_n) FLA_FIELD(y2) FLA_FIELD(dy2)
-FLA_FIELD(totals2) FLA_FIELD(dz2) FLA_FIELD(z_narrow)
+FLA_FIELD(totals2) FLA_FIELD(dz2) FLA_FIELD(z_narrow) FLA_FIELD(vsum)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(WalkVecParams)
