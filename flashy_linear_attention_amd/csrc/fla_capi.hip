@@ -2206,6 +2206,19 @@ int fla_poly_attn_bwd(const void *grad_out, const void *xq, const void *xk, cons
                          R, D_v, coef, dtype, workspace, workspace_bytes, stream);
 }
 
+// Measured (bf16, quadratic time over chunk-wise time, widths 32, 64, 128, B H 2 ... 192, N 256 ... 4096).  Forward alone: N =
+// 2048 1.3 to 1.9, N = 4096 2.1 to 3.8; at N = 1024 1.06 to 1.5 up to 64 columns, but 0.8 to 1.3 at 128.  Forward + backward
+// (the host's time hides much below 80 us): W = B H N^2 D from 4e9 0.97 to 3.7, N = 4096 1.1 to 3.7, below 0.83 to 0.94.
+// Errors against fp64 are the smaller ones everywhere (0.72 to 0.97 of the quadratic evaluation's, N 512 ... 6000).
+// fp16 keeps the quadratic kernels: the chunk-wise running state has fp16's range.
+int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype, int backward) {
+    if (dtype != FLA_DTYPE_BF16 || D_qk < 1 || D_v < 1 || D_qk % 8 != 0 || D_v % 8 != 0) return 0;
+    const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v);
+    if (!wp.ok) return 0;
+    const double w = (double)B * (double)H * (double)N * (double)N * (double)wp.D;
+    if (backward) return N >= 4096 || w >= (wp.D <= 64 ? 4e9 : 8e9);
+    return N >= 2048 || (N >= 1024 && wp.D <= 64) || w >= 1.2e10;
+}
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward) {
     if (dtype != FLA_DTYPE_BF16 || !poly_plan(B, H, N, R, D_v).ok) return 0;
     // Measured over B H = 2 ... 256, N = 128 ... 2048, R / D_v = 16 / 64 and 8 / 32, with and without the normaliser: the

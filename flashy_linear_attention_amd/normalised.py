@@ -4,9 +4,9 @@ normaliser to the caller, README.md:27-30 of the reference):
     out = LinearAttention.apply(q, k, v) / ((q * k.cumsum(-2)).sum(-1, keepdim=True) + eps)
 
 ``LinearAttentionNormalised.apply(q, k, v, eps, chunked=False)`` returns the same tensor
-(``chunked=True``: the product is evaluated chunk-wise, O(N), for long sequences).  The product runs on
-the kernels of ``LinearAttention``; the cumulative sum, the dot with q, eps and the division
-are one fused pass in fp32 (``fla_linear_attn_normalised_fwd``), and backward adds the
+(``chunked=True``: the product is evaluated chunk-wise, O(N), whatever the shape; by default where that
+is faster, ``fla_normalised_prefers_chunked``).  The product runs on the kernels of ``LinearAttention``;
+the cumulative sum, the dot with q, eps and the division are one fused pass in fp32 (``fla_linear_attn_normalised_fwd``), and backward adds the
 normaliser's own gradient terms with two more fused passes instead of an autograd graph of
 elementwise kernels (``fla_linear_attn_normalised_bwd``).
 """
@@ -33,6 +33,12 @@ def _workspace(lib, b: int, h: int, n: int, dqk: int, dv: int, chunked: bool,
 def _state_buffer(lib, b: int, h: int, n: int, dqk: int, dv: int, want: bool, device: torch.device):
     sbytes = _lib.query("fla_linear_attn_chunked_state_bytes", b, h, n, dqk, dv) if want else 0
     return torch.empty(sbytes, dtype=torch.uint8, device=device) if sbytes else None
+
+
+def _prefers_chunked(q: torch.Tensor, v: torch.Tensor, grad: bool) -> bool:
+    if q.dim() != 4 or v.dim() != 4 or not q.is_cuda or q.dtype != torch.bfloat16:
+        return False  # (what is no call of the operator is refused by its forward)
+    return bool(_lib.query("fla_normalised_prefers_chunked", *q.shape, v.shape[-1], dtype_code(q), int(grad)))
 
 
 def linear_attention_normalised_fwd(
@@ -113,7 +119,9 @@ class LinearAttentionNormalised(Function):
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, eps: float = 1e-5,
                 chunked: bool = False) -> torch.Tensor:
-        want = bool(chunked) and any(ctx.needs_input_grad[:3])
+        grad = any(ctx.needs_input_grad[:3])
+        chunked = bool(chunked) or _prefers_chunked(q, v, grad)
+        want = chunked and grad
         out, denom, state = linear_attention_normalised_fwd(q, k, v, eps, chunked, want_state=True) if want else (
             *linear_attention_normalised_fwd(q, k, v, eps, chunked), None)
         ctx.has_state = state is not None

@@ -346,6 +346,10 @@ int fla_poly_attn_bwd(const void *grad_out, const void *xq, const void *xk, cons
                       const int64_t *dv_strides,
                       const float *coef, int dtype, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* 1 where the chunk-wise evaluation of the normalised operator (chunked != 0 below) is the faster one (of a forward +
+ * backward pair, or with backward == 0 of forward alone; host arithmetic, measured thresholds), 0 elsewhere. */
+int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype, int backward);
+
 /* The same operator evaluated chunk-wise (O(N): running sums of Taylor features formed inside the kernels, nothing
  * feature-wide in memory but the states at segment ends).  FLA_DTYPE_BF16 and R <= 16, D_v <= 64 only
  * (FLA_ERR_UNSUPPORTED otherwise, as for operands that are not 16-byte aligned).  fla_poly_attn_prefers_chunked(): 1 where
