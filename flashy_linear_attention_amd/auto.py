@@ -32,6 +32,16 @@ def prefers_chunked(q: torch.Tensor, v: torch.Tensor) -> bool:
     return bool(_lib.query("fla_linear_attn_prefers_chunked", b, h, n, dqk, v.shape[-1]))
 
 
+def chunked_keeps_range(q: torch.Tensor, v: torch.Tensor, grad: bool) -> bool:
+    """Whether the chunk-wise evaluation takes whatever the quadratic one does.  bf16: yes.  fp16: a state element may
+    exceed 65504 where no score and no result does; the forward walk (head dims up to 128, multiples of 8, more than
+    256 rows) scales its state's fp16 copy, the backward walks do not."""
+    if q.dtype == torch.bfloat16:
+        return True
+    dqk, dv = q.shape[-1], v.shape[-1]
+    return not grad and max(dqk, dv) <= 128 and dqk % 8 == 0 and dv % 8 == 0 and q.shape[2] > 256
+
+
 def evaluate_fwd(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, chunked: bool, equal: bool) -> torch.Tensor:
     """Forward of an autograd Function by the evaluation `chunked` names; keeps what :func:`evaluate_bwd` needs."""
     ctx.chunked, ctx.equal = chunked, equal

@@ -812,8 +812,9 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
 // works on two pairs (grid y), so a plan has half as many segments as the two walks after each other that it
 // replaces: half the totals and entry states to move, which at B H = 16 outweigh the operands.
 //   forward   one walk over both halves of q / k per half of v: O's halves are columns of their own
-//   backward  dQ and dK are sums over v's halves, dV over q / k's: first the pairs (0, 0) and (1, 1), whose results are
-//             different columns of all three, then (1, 0) and (0, 1), which add theirs in the walks' epilogues
+//   backward  dQ and dK are sums over v's halves, dV over q / k's: first the pairs (0, 1) and (1, 0), whose results are
+//             different columns of all three, then (0, 0) and (1, 1), which add theirs in the walks' epilogues (in this
+//             order what is rounded in between is, for most columns, the smaller part: that of a narrow second half)
 // Five launches per step, and no scratch tensors.  256 / 256, forward + backward, halves of v after each other -> this:
 // B H 16, N 4096: 408 -> 245 us.
 WalkPlan quad_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
@@ -873,7 +874,7 @@ int quad_backward(const WalkPlan &wp, const View &go, const View &q, const View 
     r.init = wp.n_seg > 1 ? entries : nullptr, r.init_is_totals = quad_sums_on_load(wp);
     r.xinit = static_cast<const float *>(state_in), r.xtotal = quad_finals(wp, state_in);
     for (int pass = 0; pass < 2; ++pass) {
-        r.quad = 2 + pass, r.accumulate = 2 * pass;
+        r.quad = 3 - pass, r.accumulate = 2 * pass;
         if (fla::walk_bwd_rev(dtype, wp.D, r, s) != hipSuccess) return FLA_ERR_LAUNCH;
     }
     return FLA_OK;

@@ -66,6 +66,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "fla_launch.h"
 #include "fla_tri_fast.h"
 
@@ -361,13 +363,14 @@ __device__ __forceinline__ void walk_pipe(Read &&read, Use &&use) {
 }
 
 // KCL: 16-wide k chunks of the contraction X Y^T that hold anything; NOB: output blocks that do.
-// KEEP: the product is added to what acc holds.
+// KEEP: the product is added to what acc holds.  SCALED: the state's part is multiplied by sback (walk_state_scale).
 template <typename T, int D, bool UPPER, int EX = 0, int KCL = WalkCfg<D>::KC, int NOB = WalkCfg<D>::DB, bool KEEP = false,
-          typename SFrag, typename YRows = WalkNoRows>
+          bool SCALED = false, typename SFrag, typename YRows = WalkNoRows>
 __device__ __forceinline__ void walk_product(const unsigned char *xt, const unsigned char *yt, const unsigned char *zt,
                                              int wave, int lane, bool has_state, SFrag &&sfrag,
                                              f32x16 (&acc)[WalkCfg<D>::DBW], float *ex = nullptr,
-                                             const float *exv = nullptr, YRows &&yrows = WalkNoRows{}) {
+                                             const float *exv = nullptr, YRows &&yrows = WalkNoRows{}, float sback = 1.f) {
+    static_assert(!SCALED || !KEEP, "what acc held would be scaled too");
     using W = WalkCfg<D>;
     using M = Mma<T>;
     using V8 = typename M::V8;
@@ -424,6 +427,12 @@ __device__ __forceinline__ void walk_product(const unsigned char *xt, const unsi
             },
             [&](auto j, V8 f) {
                 constexpr int J = decltype(j)::value;
+                if constexpr (SCALED && ST && J == NA + NB) {  // (the state product is complete)
+#pragma unroll
+                    for (int i = 0; i < PER; ++i)
+#pragma unroll
+                        for (int v = 0; v < 16; ++v) acc[i][v] *= sback;
+                }
                 if constexpr (J == CONV) {  // normaliser's terms, mask, rounding
                     if constexpr (EX == 2) {
 #pragma unroll
@@ -483,6 +492,12 @@ __device__ __forceinline__ void walk_product(const unsigned char *xt, const unsi
                                             constexpr int I = decltype(j)::value % PER, KC_ = decltype(j)::value / PER;
                                             acc[I] = M::mma(f, xf[KC_], acc[I]);
                                         });
+            if constexpr (SCALED) {
+#pragma unroll
+                for (int i = 0; i < PER; ++i)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) acc[i][v] *= sback;
+            }
         }
 #pragma unroll 1
         for (int s = s_lo; s <= s_hi; ++s) block(s, std::false_type{});
@@ -696,7 +711,7 @@ __device__ __forceinline__ float walk_col_sum_of(const float *part, int col) {
 // columns per register group), in the tile layout
 template <typename T, int D, typename B = WalkExt<D>>
 __device__ __forceinline__ void walk_state_to_lds(unsigned char *tl, int wave, int lane,
-                                                  const f32x16 (&st)[WalkCfg<D>::NBW]) {
+                                                  const f32x16 (&st)[WalkCfg<D>::NBW], float scale = 1.f) {
     using W = WalkCfg<D>;
     typedef T t4 __attribute__((ext_vector_type(4)));
     const int l32 = lane & 31, g = lane >> 5, row = 32 * B::eb(wave) + l32;
@@ -708,10 +723,35 @@ __device__ __forceinline__ void walk_state_to_lds(unsigned char *tl, int wave, i
         for (int a = 0; a < 4; ++a) {
             t4 w;
 #pragma unroll
-            for (int b = 0; b < 4; ++b) w[b] = static_cast<T>(st[i][4 * a + b]);
+            for (int b = 0; b < 4; ++b) w[b] = static_cast<T>(scale * st[i][4 * a + b]);
             *reinterpret_cast<t4 *>(tl + row * W::RB + (((4 * dbk + a) ^ walk_swizzle<W::CR>(row)) << 4) + 8 * g) = w;
         }
     }
+}
+
+// fp16: the sums of a long sequence leave its range where results of the operator do not, so the state's 16-bit copy is
+// scaled by a power of two that puts its largest element at 2^14 (exact; what is 2^28 times smaller than that becomes
+// subnormal).  Every wave leaves its largest |element| in smax[wave]; behind a barrier walk_state_scale gives
+// the factor of the copy and, in `back`, its inverse for the product (1 for a zero or a non-finite state).
+template <int D, typename B>
+__device__ __forceinline__ void walk_state_max(float *smax, int wave, int lane, const f32x16 (&st)[WalkCfg<D>::NBW]) {
+    float m = 0.f;
+#pragma unroll
+    for (int i = 0; i < B::SLOTS; ++i)
+        if (B::valid(wave, i)) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) m = fmaxf(m, fabsf(st[i][v]));
+        }
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    if (lane == 0) smax[wave] = m;
+}
+__device__ __forceinline__ float walk_state_scale(const float *smax, float &back) {
+    const float m = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
+    const int e = (int)(__builtin_bit_cast(uint32_t, m) >> 23);  // biased exponent: m < 2^(e - 126)
+    const int k = m > 0.f && e < 255 ? (e < 40 ? 40 : e) - 141 : 0;
+    back = __builtin_bit_cast(float, (uint32_t)(127 + k) << 23);
+    return __builtin_bit_cast(float, (uint32_t)(127 - k) << 23);
 }
 
 struct WalkSlice {
@@ -942,6 +982,10 @@ __device__ __forceinline__ void walk_write_state(float *out, int wave, int lane,
 // FM: the instantiations that know of feature maps (WalkParams::fmap, slope_y); the others ignore both.
 // NQ, NV: blocks of the state [q/k index][v index] that hold anything (WalkExt).
 // ACCUM: the result is added to what o holds already (WalkParams::accumulate, WalkPrev).
+// the plain fp16 forward: walk_state_scale
+template <typename T, int NORM, bool FM>
+constexpr bool walk_fwd_scaled = std::is_same<T, _Float16>::value && NORM == 0 && !FM;
+
 template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool ACCUM = false>
 __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -952,6 +996,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     static_assert(NORM == 0 || (NQ == W::DB && NV == W::DB), "the normaliser's variants are built for full widths");
     static_assert(!ACCUM || (DOUBLE && NORM == 0 && !FM), "adding to the result: the plain D = 128 walk only");
     constexpr int SETS = DOUBLE ? 2 : 1;
+    constexpr bool SCALED = walk_fwd_scaled<T, NORM, FM>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
     unsigned char *tl = smem + SETS * 3 * W::TILE;
@@ -981,7 +1026,21 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         if (p.init_is_totals && p.entry_out && sl.seg > 0)
             walk_write_state<D, B>(p.entry_out + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D), wave, lane, st);
     }
-    walk_state_to_lds<T, D, B>(tl, wave, lane, st);
+    // the state's copy in LDS for the next chunk (SCALED: every wave has passed a barrier since its walk_state_max)
+    float sback = 1.f, *smax = reinterpret_cast<float *>(xv);
+    auto publish_state = [&]() {
+        if constexpr (SCALED) {
+            const float scale = walk_state_scale(smax, sback);
+            walk_state_to_lds<T, D, B>(tl, wave, lane, st, scale);
+        } else {
+            walk_state_to_lds<T, D, B>(tl, wave, lane, st);
+        }
+    };
+    if constexpr (SCALED) {
+        walk_state_max<D, B>(smax, wave, lane, st);
+        __syncthreads();
+    }
+    publish_state();
     // NORM 1: zc at the segment's entry from the segments' totals, thread groups of D taking every (256 / D)-th segment
     float zrun = 0.f;  // (of column tid, tid < D)
     auto zc_publish = [&](int c) {
@@ -1089,7 +1148,8 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
             walk_product<T, D, false, 2, B::KQ, NV>(tq, tk, tv, wave, lane, c > 0, sfrag, acc, &ax);
             walk_add_vec<D>(acc, ax, vz, db0, g);
         } else {
-            walk_product<T, D, false, 0, B::KQ, NV>(tq, tk, tv, wave, lane, c > 0, sfrag, acc);
+            walk_product<T, D, false, 0, B::KQ, NV, false, SCALED>(tq, tk, tv, wave, lane, c > 0, sfrag, acc, nullptr, nullptr,
+                                                                   WalkNoRows{}, sback);
         }
         if (slope_y) {
             feature_dispatch(fmap, [&](auto map) {
@@ -1114,6 +1174,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                 }
         }
         walk_update<T, D, B>(tk, tv, wave, lane, st);
+        if constexpr (SCALED) walk_state_max<D, B>(smax, wave, lane, st);
         if constexpr (NORM == 1) {
             f32x16 zs;
 #pragma unroll
@@ -1129,7 +1190,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         } else {
             __syncthreads();  // every wave is done with the tiles and with the old state
         }
-        walk_state_to_lds<T, D, B>(tl, wave, lane, st);
+        publish_state();
         if constexpr (NORM == 1) {
             if (tid < D && c + 1 < sl.c_hi) {
                 zrun += walk_col_sum_of<D>(zpart, tid);
@@ -2255,7 +2316,8 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr bool kDouble = D > 64;  // (the plan's workgroup count must match: one per CU when double)
-    constexpr int smem = (kDouble ? 6 : 3) * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
+    // (walk_fwd_scaled: the waves' largest elements behind the state)
+    constexpr int smem = (kDouble ? 6 : 3) * WalkCfg<D>::TILE + WalkCfg<D>::STATE + (walk_fwd_scaled<T, 0, false> ? 16 : 0);
     const bool fm = p.fmap || p.slope_y;
     // (segment totals in place of entry states: the D = 128 walks, by the flag; below that by the number of segments)
     if (p.init_is_totals && (D != 128 || p.n_seg < 3 || !p.init)) return hipErrorInvalidValue;

@@ -439,13 +439,15 @@ PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
     if (dqk > 256 || dv > 256) Py_RETURN_NONE;
     const bool bf16 = a.cast || a.q.scalar_type() == at::kBFloat16, equal = dqk == dv;
     auto prefers = [&] { return fla_linear_attn_prefers_chunked(a.q.size(0), a.q.size(1), rows, dqk, dv) != 0; };
+    // (fp16: auto.py, chunked_keeps_range)
+    const bool range = bf16 || (!wants_grad(a.q, a.k, a.v) && dqk <= 128 && dv <= 128 && dqk % 8 == 0 && dv % 8 == 0 && rows > 256);
     int ev = equal ? kEqual : kSmallV;
     if (kind == 0) {  // (the shapes its forward takes, and its choice: linear_attn.py)
         if (!equal || rows % (dqk > 128 ? 32 : 64) != 0) Py_RETURN_NONE;
-        if (bf16 && dqk <= 128 && prefers()) ev = kChunked;
+        if (range && dqk <= 128 && prefers()) ev = kChunked;
     } else if (kind == 1) {  // (linear_attn_smallv_hd.py)
         if (!pow2(dv) || dv > next_pow2(dqk) || rows % 64 != 0) Py_RETURN_NONE;
-        ev = bf16 && dv <= 128 && prefers() ? kChunked : kSmallV;
+        ev = range && dv <= 128 && prefers() ? kChunked : kSmallV;
     } else if (kind == 2) {  // (auto.py)
         if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || prefers()) ev = kChunked;
     } else {

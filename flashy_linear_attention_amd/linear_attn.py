@@ -12,7 +12,7 @@ import torch
 from torch.autograd import Function
 
 from . import _native
-from .auto import evaluate_bwd, evaluate_fwd, prefers_chunked
+from .auto import chunked_keeps_range, evaluate_bwd, evaluate_fwd, prefers_chunked
 from .kernels.linear_attn_kernels import check_operands
 
 
@@ -30,10 +30,9 @@ class LinearAttention(Function):
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         check_operands(q, k, v)
         # The chunk-wise kernels where the measured thresholds say so, up to 27 times faster on long sequences.
-        # bf16 only: the chunk-wise running state is kept in the storage type too, and in fp16 its range
-        # would narrow what may be passed in (a state element may exceed 65504 where no score and no result does).
         # Head dims up to 128: beyond, dQ and dK are sums over v's column halves, each half rounded.
-        chunked = q.dtype == torch.bfloat16 and q.shape[-1] <= 128 and prefers_chunked(q, v)
+        chunked = (q.shape[-1] <= 128 and chunked_keeps_range(q, v, any(ctx.needs_input_grad))
+                   and prefers_chunked(q, v))
         return evaluate_fwd(ctx, q, k, v, chunked, True)
 
     @staticmethod

@@ -11,7 +11,7 @@ import torch
 from torch.autograd import Function
 
 from . import _native
-from .auto import evaluate_bwd, evaluate_fwd, prefers_chunked
+from .auto import chunked_keeps_range, evaluate_bwd, evaluate_fwd, prefers_chunked
 from .kernels.linear_attn_kernels_smallv_hd import check_operands
 
 
@@ -28,10 +28,10 @@ class LinearAttentionSmallVHD(Function):
     @torch.amp.custom_fwd(device_type="cuda", cast_inputs=torch.bfloat16)
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor) -> torch.Tensor:
         check_operands(q, k, v)
-        # (bf16 and D_v up to 128 only: see LinearAttention.  The quadratic backward wants
+        # (D_v up to 128 only: see LinearAttention.  The quadratic backward wants
         # N a multiple of 64 where forward takes 32, so such a sequence stays with it)
-        chunked = (q.dtype == torch.bfloat16 and q.shape[2] % 64 == 0 and v.shape[-1] <= 128
-                   and prefers_chunked(q, v))
+        chunked = (q.shape[2] % 64 == 0 and v.shape[-1] <= 128
+                   and chunked_keeps_range(q, v, any(ctx.needs_input_grad)) and prefers_chunked(q, v))
         return evaluate_fwd(ctx, q, k, v, chunked, False)
 
     @staticmethod
