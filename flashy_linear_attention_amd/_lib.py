@@ -39,6 +39,7 @@ SIGNATURES = {
     "fla_linear_attn_chunked_state_bytes": ([_i64] * 5, ctypes.c_int64),
     "fla_linear_attn_chunked_workspace_bytes": ([_i64] * 5, ctypes.c_int64),
     "fla_linear_attn_prefers_chunked": ([_i64] * 5, ctypes.c_int),
+    "fla_linear_attn_forward_prefers_chunked": ([_i64] * 5, ctypes.c_int),
     "fla_linear_attn_chunked_fwd": ([_ptr] * 4 + [_i64] * 5 + [_strides] * 4
                                     + [ctypes.c_int, _ptr, ctypes.POINTER(ctypes.c_int32), _ptr, _i64, _ptr], ctypes.c_int),
     "fla_feature_attn_fwd": ([_ptr] * 6 + [_i64] * 5 + [_strides] * 6
@@ -59,7 +60,7 @@ SIGNATURES = {
                           + [ctypes.POINTER(ctypes.c_float), ctypes.c_float, ctypes.c_int, _ptr], ctypes.c_int),
     "fla_poly_attn_bwd": ([_ptr] * 9 + [_i64] * 5 + [_strides] * 8
                           + [ctypes.POINTER(ctypes.c_float), ctypes.c_int, _ptr, _i64, _ptr], ctypes.c_int),
-    "fla_normalised_prefers_chunked": ([_i64] * 5 + [ctypes.c_int] * 2, ctypes.c_int),
+    "fla_normalised_forward_prefers_chunked": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int),
     "fla_poly_attn_prefers_chunked": ([_i64] * 5 + [ctypes.c_int] * 2, ctypes.c_int),
     "fla_poly_attn_chunked_state_bytes": ([_i64] * 5, ctypes.c_int64),
     "fla_poly_attn_chunked_workspace_bytes": ([_i64] * 5, ctypes.c_int64),

@@ -26,10 +26,11 @@ from .kernels import (
 )
 
 
-def prefers_chunked(q: torch.Tensor, v: torch.Tensor) -> bool:
-    """Whether the chunk-wise kernels are the faster choice for (B, H, N, D_qk) q and (B, H, N, D_v) v."""
+def prefers_chunked(q: torch.Tensor, v: torch.Tensor, grad: bool = True) -> bool:
+    """Whether the chunk-wise kernels are the faster choice for (B, H, N, D_qk) q and (B, H, N, D_v) v, for forward +
+    backward or (``grad`` false) forward alone."""
     b, h, n, dqk = q.shape
-    return bool(_lib.query("fla_linear_attn_prefers_chunked", b, h, n, dqk, v.shape[-1]))
+    return bool(_lib.query("fla_linear_attn_prefers_chunked" if grad else "fla_linear_attn_forward_prefers_chunked", b, h, n, dqk, v.shape[-1]))
 
 
 def chunked_keeps_range(q: torch.Tensor, v: torch.Tensor, grad: bool) -> bool:
@@ -88,7 +89,7 @@ class LinearAttentionAuto(Function):
         dqk, dv = q.shape[-1], v.shape[-1]
         equal = dqk == dv
         refused = q.shape[2] % 64 != 0 or (not equal and (dv > dqk or dv & (dv - 1)))
-        return evaluate_fwd(ctx, q, k, v, prefers_chunked(q, v) or refused, equal)
+        return evaluate_fwd(ctx, q, k, v, prefers_chunked(q, v, any(ctx.needs_input_grad)) or refused, equal)
 
     @staticmethod
     @torch.amp.custom_bwd(device_type="cuda")

@@ -1898,6 +1898,30 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
     return fla::poly_walk(w, true, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 
+// Which evaluation is faster on MI355X (bench.py --crossover): the quadratic kernels' time grows with W = B H N^2 D (D: the
+// larger padded head dim) above the time of one workgroup's longest row tile, which grows with N; the chunk-wise kernels'
+// with B H N D above a floor of launches.  Measured quadratic time over chunk-wise time, widths 32 ... 128 and 64/32, 128/64, 128/32, B H 1 ...
+// 192, N 512 ... 8192.  Forward + backward, equal widths: from W = B H N^2 D = 4e9 (8e9 at 128) 1.08 to 4.9 with few heads
+// or many; few heads and long: N = 4096 1.8 to 2.9, N = 2048 1.25 to 1.7 at 64 and 128 columns, 0.84 to 1.1 at 32; N = 1024
+// 0.67 to 1.2.  Widths that differ (small-V operator): N = 1024 1.4 to 1.9.  Forward alone: N = 2048 1.17 to 1.9 (0.92 to
+// 0.99 at 32 columns), W from 1.2e10 1.1 to 2; N = 512 and 1024 below that 0.65 to 1.15.
+int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, bool backward) {
+    if (B < 1 || H < 1 || N < 1 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
+    const double w = (double)B * (double)H * (double)N * (double)N * (double)padded(D_qk > D_v ? D_qk : D_v);
+    const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v, true);
+    // Widths that are no multiples of 8: the quadratic operator runs the bounds-checked kernel, the chunk-wise one the
+    // fast kernels of either kind on copies with aligned rows, 1.4 to 12 times faster (forward + backward) over
+    // B H = 2 ... 128, N = 256 ... 2048 and widths 36, 91/64, 100, 153/64.
+    if (pack_plan(B, H, N, D_qk, D_v).ok) return 1;
+    // (padded widths that differ: the quadratic side is the small-V operator, whose wide products are two launches)
+    if (wp.ok && !backward) return wp.D <= 32 ? N >= 4096 || w >= 5e9 : N >= 2048 || w >= 1.2e10;
+    if (wp.ok && pad_index(D_qk) != pad_index(D_v)) return N >= 1024 || w >= (wp.D <= 64 ? 1e9 : 5e8);
+    if (wp.ok) return N >= (wp.D <= 32 ? 4096 : 2048) || w >= (wp.D <= 64 ? 4e9 : 8e9);  // equal padded head dims up to 128
+    if (wide_plan(B, H, N, D_qk, D_v).ok) return w >= (D_v <= 64 ? 1e9 : 1.5e10);  // D_qk in (128, 256], D_v <= 128
+    if (vsplit_plan(B, H, N, D_qk, D_v).ok) return w >= 3e10;  // D_v in (128, 256] as two column halves of v
+    return N >= 4096;  // chunk states in memory, a launch per product and state (measured at 256 / 256)
+}
+
 }  // namespace
 
 extern "C" {
@@ -2025,25 +2049,11 @@ int fla_tri_xyt_z_chunked(const void *x, const void *y, const void *z, void *out
     return run_tri_chunked(vx, vy, vz, vo, B, H, N, D_c, D_o, upper, dtype, workspace, workspace_bytes, stream);
 }
 
-// Which evaluation of forward + backward is faster on MI355X, from timings of both over grids of
-// (head dims, B H, N) (bench.py --crossover): the quadratic kernels' time grows with
-// W = B H N^2 D (D: the larger padded head dim), the chunk-wise kernels' with B H N D above a floor
-// of launches (four to six for the walk kernels, also for a wide q / k against a narrow v), so each
-// of these classes of shapes has one threshold on W.
 int fla_linear_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v) {
-    if (B < 1 || H < 1 || N < 1 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
-    const double w = (double)B * (double)H * (double)N * (double)N * (double)padded(D_qk > D_v ? D_qk : D_v);
-    const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v, true);
-    // Widths that are no multiples of 8: the quadratic operator runs the bounds-checked kernel, the chunk-wise one the
-    // fast kernels of either kind on copies with aligned rows, 1.4 to 12 times faster (forward + backward) over
-    // B H = 2 ... 128, N = 256 ... 2048 and widths 36, 91/64, 100, 153/64.
-    if (pack_plan(B, H, N, D_qk, D_v).ok) return 1;
-    // (padded widths that differ: the quadratic side is the small-V operator, whose wide products are two launches)
-    if (wp.ok && pad_index(D_qk) != pad_index(D_v)) return w >= (wp.D <= 64 ? 1e9 : 5e8);
-    if (wp.ok) return w >= (wp.D <= 64 ? 4e9 : 8e9);                              // equal padded head dims up to 128
-    if (wide_plan(B, H, N, D_qk, D_v).ok) return w >= (D_v <= 64 ? 1e9 : 1.5e10);  // D_qk in (128, 256], D_v <= 128
-    if (vsplit_plan(B, H, N, D_qk, D_v).ok) return w >= 3e10;  // D_v in (128, 256] as two column halves of v
-    return N >= 4096;  // chunk states in memory, a launch per product and state (measured at 256 / 256)
+    return prefers_chunked(B, H, N, D_qk, D_v, true);
+}
+int fla_linear_attn_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v) {
+    return prefers_chunked(B, H, N, D_qk, D_v, false);
 }
 
 int64_t fla_linear_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v) {
@@ -2207,17 +2217,17 @@ int fla_poly_attn_bwd(const void *grad_out, const void *xq, const void *xk, cons
                          R, D_v, coef, dtype, workspace, workspace_bytes, stream);
 }
 
-// Measured (bf16, quadratic time over chunk-wise time, widths 32, 64, 128, B H 2 ... 192, N 256 ... 4096).  Forward alone: N =
-// 2048 1.3 to 1.9, N = 4096 2.1 to 3.8; at N = 1024 1.06 to 1.5 up to 64 columns, but 0.8 to 1.3 at 128.  Forward + backward
-// (the host's time hides much below 80 us): W = B H N^2 D from 4e9 0.97 to 3.7, N = 4096 1.1 to 3.7, below 0.83 to 0.94.
-// Errors against fp64 are the smaller ones everywhere (0.72 to 0.97 of the quadratic evaluation's, N 512 ... 6000).
-// fp16 keeps the quadratic kernels: the chunk-wise running state has fp16's range.
-int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype, int backward) {
+// Forward alone, measured (bf16, quadratic time over chunk-wise time, widths 32, 64, 128, B H 2 ... 192, N 256 ... 4096): N = 2048
+// 1.3 to 1.9, N = 4096 2.1 to 3.8; at N = 1024 1.06 to 1.5 up to 64 columns, but 0.8 to 1.3 at 128.  Errors against fp64 are the
+// smaller ones (0.86 to 0.97 of the quadratic evaluation's).  A call whose gradients are wanted keeps the quadratic
+// kernels: they add the normaliser's part of dQ to the rounded rest, the walks before rounding, and where the two cancel
+// (early rows) single elements of dQ come out up to 1.2 of its root mean square apart.  So does fp16: the normalised walks
+// do not scale their state.
+int fla_normalised_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype) {
     if (dtype != FLA_DTYPE_BF16 || D_qk < 1 || D_v < 1 || D_qk % 8 != 0 || D_v % 8 != 0) return 0;
     const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v);
     if (!wp.ok) return 0;
     const double w = (double)B * (double)H * (double)N * (double)N * (double)wp.D;
-    if (backward) return N >= 4096 || w >= (wp.D <= 64 ? 4e9 : 8e9);
     return N >= 2048 || (N >= 1024 && wp.D <= 64) || w >= 1.2e10;
 }
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward) {

@@ -438,9 +438,13 @@ PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const int64_t rows = a.q.size(2), dqk = a.q.size(3), dv = a.v.size(3);
     if (dqk > 256 || dv > 256) Py_RETURN_NONE;
     const bool bf16 = a.cast || a.q.scalar_type() == at::kBFloat16, equal = dqk == dv;
-    auto prefers = [&] { return fla_linear_attn_prefers_chunked(a.q.size(0), a.q.size(1), rows, dqk, dv) != 0; };
+    const bool grad = wants_grad(a.q, a.k, a.v);
+    auto prefers = [&] {
+        return (grad ? fla_linear_attn_prefers_chunked : fla_linear_attn_forward_prefers_chunked)(a.q.size(0), a.q.size(1), rows,
+                                                                                                  dqk, dv) != 0;
+    };
     // (fp16: auto.py, chunked_keeps_range)
-    const bool range = bf16 || (!wants_grad(a.q, a.k, a.v) && dqk <= 128 && dv <= 128 && dqk % 8 == 0 && dv % 8 == 0 && rows > 256);
+    const bool range = bf16 || (!grad && dqk <= 128 && dv <= 128 && dqk % 8 == 0 && dv % 8 == 0 && rows > 256);
     int ev = equal ? kEqual : kSmallV;
     if (kind == 0) {  // (the shapes its forward takes, and its choice: linear_attn.py)
         if (!equal || rows % (dqk > 128 ? 32 : 64) != 0) Py_RETURN_NONE;
@@ -474,10 +478,10 @@ PyObject *py_mapped(PyObject *, PyObject *const *args, Py_ssize_t n) {
         PyErr_Clear();
         Py_RETURN_NONE;
     }
-    if (!opt.fmap && opt.normalise && !opt.chunked) {  // (normalised.py: the evaluation chosen by shape)
+    if (!opt.fmap && opt.normalise && !opt.chunked && !wants_grad(a.q, a.k, a.v)) {  // (normalised.py)
         const int dtype = a.cast ? FLA_DTYPE_BF16 : dtype_code(a.q.scalar_type());
-        opt.chunked = fla_normalised_prefers_chunked(a.q.size(0), a.q.size(1), a.q.size(2), a.q.size(3), a.v.size(3), dtype,
-                                                     wants_grad(a.q, a.k, a.v)) != 0;
+        opt.chunked = fla_normalised_forward_prefers_chunked(a.q.size(0), a.q.size(1), a.q.size(2), a.q.size(3), a.v.size(3),
+                                                             dtype) != 0;
     }
     return released([&]() -> Tensor {
         if (wants_grad(a.q, a.k, a.v)) return Mapped::apply(a.q, a.k, a.v, opt.code(), opt.eps, a.cast);

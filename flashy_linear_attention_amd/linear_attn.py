@@ -31,8 +31,8 @@ class LinearAttention(Function):
         check_operands(q, k, v)
         # The chunk-wise kernels where the measured thresholds say so, up to 27 times faster on long sequences.
         # Head dims up to 128: beyond, dQ and dK are sums over v's column halves, each half rounded.
-        chunked = (q.shape[-1] <= 128 and chunked_keeps_range(q, v, any(ctx.needs_input_grad))
-                   and prefers_chunked(q, v))
+        grad = any(ctx.needs_input_grad)
+        chunked = q.shape[-1] <= 128 and chunked_keeps_range(q, v, grad) and prefers_chunked(q, v, grad)
         return evaluate_fwd(ctx, q, k, v, chunked, True)
 
     @staticmethod

@@ -30,8 +30,9 @@ class LinearAttentionSmallVHD(Function):
         check_operands(q, k, v)
         # (D_v up to 128 only: see LinearAttention.  The quadratic backward wants
         # N a multiple of 64 where forward takes 32, so such a sequence stays with it)
-        chunked = (q.shape[2] % 64 == 0 and v.shape[-1] <= 128
-                   and chunked_keeps_range(q, v, any(ctx.needs_input_grad)) and prefers_chunked(q, v))
+        grad = any(ctx.needs_input_grad)
+        chunked = (q.shape[2] % 64 == 0 and v.shape[-1] <= 128 and chunked_keeps_range(q, v, grad)
+                   and prefers_chunked(q, v, grad))
         return evaluate_fwd(ctx, q, k, v, chunked, False)
 
     @staticmethod

@@ -204,6 +204,8 @@ int64_t fla_linear_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int
  * quadratic fla_linear_attn(_smallv)_fwd + bwd are: a table of measured thresholds (host arithmetic,
  * no device call) in place of the autotuning the reference lists as a to-do (README.md:68). */
 int fla_linear_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v);
+/* The same question for forward alone. */
+int fla_linear_attn_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v);
 int64_t fla_linear_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v);
 int fla_linear_attn_chunked_fwd(const void *q, const void *k, const void *v, void *o,
                                 int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v,
@@ -346,9 +348,9 @@ int fla_poly_attn_bwd(const void *grad_out, const void *xq, const void *xk, cons
                       const int64_t *dv_strides,
                       const float *coef, int dtype, void *workspace, int64_t workspace_bytes, void *stream);
 
-/* 1 where the chunk-wise evaluation of the normalised operator (chunked != 0 below) is the faster one (of a forward +
- * backward pair, or with backward == 0 of forward alone; host arithmetic, measured thresholds), 0 elsewhere. */
-int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype, int backward);
+/* 1 where the chunk-wise evaluation (chunked != 0) of the normalised operator's forward alone is the faster one (host
+ * arithmetic, measured thresholds), 0 elsewhere. */
+int fla_normalised_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype);
 
 /* The same operator evaluated chunk-wise (O(N): running sums of Taylor features formed inside the kernels, nothing
  * feature-wide in memory but the states at segment ends).  FLA_DTYPE_BF16 and R <= 16, D_v <= 64 only

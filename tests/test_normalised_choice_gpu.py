@@ -1,11 +1,11 @@
-"""LinearAttentionNormalised chooses the evaluation by shape when not told: both sides of the thresholds, with and without
-gradients, natively and through the Python forward, against the fp64 recipe (``-m gpu``)."""
+"""LinearAttentionNormalised chooses the evaluation of forward alone by shape when not told: both sides of the thresholds, with
+and without gradients, natively and through the Python forward, against the fp64 recipe (``-m gpu``)."""
 
 import pytest
 import torch
 
 from flashy_linear_attention_amd import LinearAttentionNormalised, _lib
-from flashy_linear_attention_amd.normalised import _prefers_chunked
+from flashy_linear_attention_amd.normalised import _forward_prefers_chunked
 
 from helpers import assert_close
 
@@ -19,20 +19,22 @@ def _recipe(q, k, v, g):
     return (out, *torch.autograd.grad(out, (q, k, v), g.double()))
 
 
-# (B, H, N, D, chunk-wise with gradients, chunk-wise without): below and from each threshold, ragged lengths
-@pytest.mark.parametrize("b,h,n,d,with_grad,without", [
-    (1, 2, 1023, 64, False, False), (1, 2, 1024, 64, False, True), (1, 1, 1500, 128, False, False), (1, 1, 2049, 72, False, True),
-    (2, 2, 4096, 32, True, True), (1, 30, 1500, 64, True, True), (1, 2, 257, 128, False, False),
-    (1, 8, 2900, 128, True, True), (1, 1, 2100, 100, False, False),
+# (B, H, N, D, chunk-wise without gradients): below and from each threshold, ragged lengths
+@pytest.mark.parametrize("b,h,n,d,chunked", [
+    (1, 2, 1023, 64, False), (1, 2, 1024, 64, True), (1, 1, 1500, 128, False), (1, 1, 2049, 72, True), (2, 2, 4096, 32, True),
+    (1, 30, 1500, 64, True), (1, 2, 257, 128, False), (1, 8, 2900, 128, True), (1, 1, 2100, 100, False),
 ])
-def test_choice_and_results(b, h, n, d, with_grad, without, gpu_device):
+def test_choice_and_results(b, h, n, d, chunked, gpu_device):
     gen = torch.Generator().manual_seed(n + d)
     q, k = (torch.nn.functional.softplus(torch.randn(b, h, n, d, generator=gen)).to(gpu_device).bfloat16() for _ in range(2))
     v, g = (torch.randn(b, h, n, d, generator=gen).to(gpu_device).bfloat16() for _ in range(2))
-    assert (_prefers_chunked(q, v, True), _prefers_chunked(q, v, False)) == (with_grad, without)
-    assert not _lib.query("fla_normalised_prefers_chunked", b, h, n, d, d, 1, 0)  # fp16
+    assert _forward_prefers_chunked(q, v) == chunked
+    assert not _lib.query("fla_normalised_forward_prefers_chunked", b, h, n, d, d, 1)  # fp16
     want = _recipe(q, k, v, g)
-    assert_close("out, no gradients", LinearAttentionNormalised.apply(q, k, v, EPS), want[0].float())
+    with torch.no_grad():
+        out = LinearAttentionNormalised.apply(q, k, v, EPS)
+    assert_close("out, no gradients", out, want[0].float())
+    assert torch.equal(out, LinearAttentionNormalised.apply(q, k, v, EPS, chunked))
     leaves = [t.requires_grad_(True) for t in (q, k, v)]
     for apply in (LinearAttentionNormalised.apply, super(LinearAttentionNormalised, LinearAttentionNormalised).apply):
         out = apply(*leaves, EPS)
