@@ -1917,7 +1917,13 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
     if (wp.ok && !backward) return wp.D <= 32 ? N >= 4096 || w >= 5e9 : N >= 2048 || w >= 1.2e10;
     if (wp.ok && pad_index(D_qk) != pad_index(D_v)) return N >= 1024 || w >= (wp.D <= 64 ? 1e9 : 5e8);
     if (wp.ok) return N >= (wp.D <= 32 ? 4096 : 2048) || w >= (wp.D <= 64 ? 4e9 : 8e9);  // equal padded head dims up to 128
-    if (wide_plan(B, H, N, D_qk, D_v).ok) return w >= (D_v <= 64 ? 1e9 : 1.5e10);  // D_qk in (128, 256], D_v <= 128
+    // D_qk in (128, 256].  D_v <= 64: pairs 1.8 to 5 from N = 1024 or W = 1e9 on, forward alone 1.13 to 2.9 from N = 1024 (N = 512
+    // 0.82 to 1.1).  D_v in (64, 128]: pairs 1.26 to 2.1 from N = 2048, 1.2 from W = 2.5e10 (0.95 at 1.5e10, N = 1024); forward
+    // alone 1.14 to 1.55 from N = 4096, at N = 2048 1.1 to 1.4 with B H <= 4 and 0.93 with 16.
+    if (wide_plan(B, H, N, D_qk, D_v).ok) {
+        if (D_v <= 64) return N >= 1024 || (backward && w >= 1e9);
+        return backward ? N >= 2048 || w >= 2.5e10 : N >= 4096 || (N >= 2048 && B * H <= 4) || w >= 5e10;
+    }
     if (vsplit_plan(B, H, N, D_qk, D_v).ok) return w >= 3e10;  // D_v in (128, 256] as two column halves of v
     return N >= 4096;  // chunk states in memory, a launch per product and state (measured at 256 / 256)
 }
