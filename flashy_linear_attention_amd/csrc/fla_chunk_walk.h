@@ -1910,8 +1910,7 @@ struct WalkTotalsParams {
     void *ymap_out;
     int64_t yo_b, yo_h, yo_n;
     // A second Y operand of the same layout against the same Z, in the same launch: the other 128-column half
-    // of a wide q / k, whose totals go to `totals2`.  Null: none.  (Without a feature map.)  Grid y = 1 takes
-    // it, or -- the kernel variant with BOTH -- every workgroup takes both operands.
+    // of a wide q / k, whose totals go to `totals2`.  Null: none.  (Without a feature map.)  Every workgroup takes both.
     const void *y2;
     int32_t dy2;
     float *totals2;
@@ -1928,8 +1927,9 @@ struct WalkTotalsParams {
 
 constexpr int walk_totals_sets(int D) { return D == 128 ? 4 : 2; }  // sets of (Y, Z) tiles in LDS
 
-// BOTH (D = 128, NV = 2): the launch's two Y operands (WalkTotalsParams::y2) in ONE workgroup -- three sets of
-// (Y, Y2, Z) tiles, a state per operand -- so that Z is loaded once for the two; otherwise grid y picks the operand.
+// BOTH (D = 128): the launch's two Y operands (WalkTotalsParams::y2) in ONE workgroup -- three sets of (Y, Y2, Z) tiles, a
+// state per operand -- so that Z is loaded once for the two.  256 / 128, forward + backward, a workgroup per operand -> this:
+// B H 64, N 4096 430 -> 420 us; B H 32, N 2048 178 -> 168 us.
 template <typename T, int D, int NQ, int NV, bool BOTH>
 __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     using W = WalkCfg<D>;
@@ -1943,8 +1943,7 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     const int hl = slot / p.n_seg, bh = hl * 8 + xcd;
     int seg = slot - hl * p.n_seg;
     if (bh >= p.BH) return;
-    const bool second = !BOTH && blockIdx.y != 0;  // (the launch's second Y operand: see WalkTotalsParams::y2)
-    const int dy = second ? p.dy2 : p.dy;
+    const int dy = p.dy;
     int64_t out_at;
     int c_lo, c_hi;
     if (p.direct) {
@@ -1968,7 +1967,7 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
         c_hi = c_lo + p.seg_chunks < p.n_chunks ? c_lo + p.seg_chunks : p.n_chunks;
     }
     out_at += (int64_t)2 * zh * p.BH * p.n_seg * (D * D);
-    float *const out = (second ? p.totals2 : p.totals) + out_at;
+    float *const out = p.totals + out_at;
     float *const out2 = BOTH ? p.totals2 + out_at : nullptr;
     if (c_lo >= c_hi) {  // nothing to add up (a segment beyond the end of the sequence, the second half of one chunk)
         for (int i = tid; i < D * D; i += 256) {
@@ -1980,7 +1979,7 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     }
     const bool discard = p.direct && p.map_y && seg != p.seg_lo;  // (visited for the map only)
     const int b = bh / p.H, h = bh - b * p.H, N = p.N;
-    const T *Y = static_cast<const T *>(second ? p.y2 : p.y) + b * p.ys_b + h * p.ys_h;
+    const T *Y = static_cast<const T *>(p.y) + b * p.ys_b + h * p.ys_h;
     const T *Y2 = static_cast<const T *>(BOTH ? p.y2 : p.y) + b * p.ys_b + h * p.ys_h;
     const T *Z = static_cast<const T *>(p.z) + b * p.zs_b + h * p.zs_h + zh * D;
     const int ys2 = (int)p.ys_n * 2, zs2 = (int)p.zs_n * 2;
@@ -2094,8 +2093,8 @@ __global__ __launch_bounds__(256, BOTH ? 1 : 2) void walk_totals_kernel(const Wa
 #endif
 }
 
-// All four pairs of 128-column halves of Y and Z (a v wider than 128 columns beside a wide q / k) in one launch: a
-// workgroup takes both halves of Y, grid y picks the half of Z.
+// Both 128-column halves of Y against a Z of more than 64 columns: a workgroup takes both halves of Y; of a Z wider than 128
+// columns grid y picks the half (all four pairs in one launch).
 template <typename T>
 __global__ __launch_bounds__(256, 1) void walk_totals_quad_kernel(const WalkTotalsParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -2264,20 +2263,20 @@ hipError_t launch_walk_totals(const WalkTotalsParams &p, hipStream_t stream) {
                  (!p.z_narrow && walk_totals_cols(D, p.dy2, p.dz) != walk_totals_cols(D, p.dy, p.dz))))
         return hipErrorInvalidValue;
     if (p.vsum && (p.y2 || p.dz2 || (D == 128 && walk_totals_cols(D, p.dy, p.dz) == 64))) return hipErrorInvalidValue;
-    if (p.dz2 || p.z_narrow) {
+    if (p.y2 || p.dz2 || p.z_narrow) {
         if (D != 128 || (p.dz2 && (!p.y2 || p.dy != 128 || p.dz != 128 || p.dz2 < 1 || p.dz2 > 128 || p.z_narrow)) ||
             (p.z_narrow && p.dz > 64))
             return hipErrorInvalidValue;
     }
-    const dim3 g((unsigned)grid, p.y2 ? 2u : 1u);
+    const dim3 g((unsigned)grid);
     if constexpr (D == 128) {
         constexpr int smem_both = 3 * 3 * WalkCfg<D>::TILE;
-        if (p.dz2) {
+        const bool narrow = p.z_narrow || walk_totals_cols(D, p.dy, p.dz) == 64;
+        if (p.dz2 || (p.y2 && !narrow)) {
             constexpr auto kern = walk_totals_quad_kernel<T>;
             if (hipError_t e = ensure_dynamic_lds<kern>(smem_both)) return e;
-            return launch_kernel<kern>(dim3((unsigned)grid, 2u), dim3(256), smem_both, stream, p);
+            return launch_kernel<kern>(dim3((unsigned)grid, p.dz2 ? 2u : 1u), dim3(256), smem_both, stream, p);
         }
-        const bool narrow = p.z_narrow || walk_totals_cols(D, p.dy, p.dz) == 64;
         if (p.y2 && narrow) {  // ... and both operands in one workgroup: z loaded once
             constexpr auto kern = walk_totals_kernel<T, D, 4, 2, true>;
             if (hipError_t e = ensure_dynamic_lds<kern>(smem_both)) return e;
