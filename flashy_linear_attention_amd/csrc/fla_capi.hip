@@ -827,6 +827,8 @@ float *quad_finals(const WalkPlan &wp, const void *state) {
     return reinterpret_cast<float *>(static_cast<char *>(const_cast<void *>(state)) + 4 * wp.entry_bytes);
 }
 
+// (forward + backward at 256 / 256, scan against sums on load: B H 16, N 4096, 8 segments 258 / 234 us; B H 12, 10 segments 319 /
+// 313; B H 32, N 2048, 4 segments 250 / 229)
 bool quad_sums_on_load(const WalkPlan &wp) { return wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost; }
 
 // the four pairs' segment totals of Y^T Z to `entries`, and the entry states over them where the walk does not add up
