@@ -828,12 +828,14 @@ __device__ __forceinline__ void walk_load_state(const float *init, bool transpos
 //     wrote them, and a walk adds up the totals of the segments before it (after it, walking in reverse)
 //     as it starts -- a few states of D x D read from L2 per workgroup instead of a scan kernel between
 //     the totals kernel and the walk, whose launch costs more than it computes on plans this small
-//     (B H = 16, N = 1024, D = 64, forward + backward: 40.7 -> 32.8 us, bound by its six -> four launches);
+//     (B H = 16, N = 1024, D = 64, forward + backward: 40.7 -> 32.8 us, bound by its six -> four launches).  D = 64, scan
+//     against sums on load: 8 to 16 segments, N 4096: B H 40 77 / 68 us, B H 32 69 / 64, forward alone 26.7 / 22.3; 21 segments
+//     equal; 32 and more: forward alone 20.7 / 21.7 (B H 16, N 4096), 21.7 / 28.8 (64 segments), B H 16 N 32768 212 / 215;
 //   * more segments: the slots hold the entry states themselves (walk_scan_kernel).
 // Padded head dims up to 64 only.  At D = 128 a workgroup has its CU to itself and nothing hides the
 // latency of those reads at its start: with four segments the forward walk gained 10 us and the reverse
 // walk, which starts from two such sums, lost 60 (B 4, H 16, N 4096, D_qk 256 as two halves: 0.333 -> 0.384 ms).
-__host__ __device__ constexpr int walk_sum_on_load_max(int D) { return D <= 64 ? 8 : 0; }
+__host__ __device__ constexpr int walk_sum_on_load_max(int D) { return D <= 64 ? 16 : 0; }
 __host__ __device__ constexpr bool walk_entries_are_totals(int D, int n_seg) {
     return n_seg >= 3 && n_seg <= walk_sum_on_load_max(D);
 }
