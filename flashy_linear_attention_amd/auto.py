@@ -4,9 +4,10 @@
 ``LinearAttentionSmallVHD`` (flashlinear/linear_attn.py:11-31, linear_attn_smallv_hd.py:14-36) and
 returns the same ``tril(Q K^T) V``; it runs the quadratic kernels where they are faster (short
 sequences, few heads) and the chunk-wise ones elsewhere, by the library's table of measured
-thresholds (``fla_linear_attn_prefers_chunked``) -- the reference lists autotuning as a to-do
-(README.md:68).  The two reference-named Functions choose the same way within the reference's
-limits on shapes; ``kernels.linear_flash_wrapper_*`` are the quadratic kernels whatever the shape.
+thresholds (``fla_linear_attn_prefers_chunked``) and where that narrows no range
+(:func:`chunked_keeps_range`) -- the reference lists autotuning as a to-do (README.md:68).  The
+two reference-named Functions choose the same way within the reference's limits on shapes;
+``kernels.linear_flash_wrapper_*`` are the quadratic kernels whatever the shape.
 """
 
 from __future__ import annotations
@@ -89,7 +90,9 @@ class LinearAttentionAuto(Function):
         dqk, dv = q.shape[-1], v.shape[-1]
         equal = dqk == dv
         refused = q.shape[2] % 64 != 0 or (not equal and (dv > dqk or dv & (dv - 1)))
-        return evaluate_fwd(ctx, q, k, v, prefers_chunked(q, v, any(ctx.needs_input_grad)) or refused, equal)
+        grad = any(ctx.needs_input_grad)
+        chunked = refused or (chunked_keeps_range(q, v, grad) and prefers_chunked(q, v, grad))
+        return evaluate_fwd(ctx, q, k, v, chunked, equal)
 
     @staticmethod
     @torch.amp.custom_bwd(device_type="cuda")

@@ -453,7 +453,7 @@ PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
         if (!pow2(dv) || dv > next_pow2(dqk) || rows % 64 != 0) Py_RETURN_NONE;
         ev = range && dv <= 128 && prefers() ? kChunked : kSmallV;
     } else if (kind == 2) {  // (auto.py)
-        if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || prefers()) ev = kChunked;
+        if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || (range && prefers())) ev = kChunked;
     } else {
         ev = kChunked;
     }
