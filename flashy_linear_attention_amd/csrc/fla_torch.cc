@@ -7,8 +7,8 @@
 // hand the interpreter lock to each other.
 //
 // Every entry point returns None where a call is not the plain case (tensor types and shapes that
-// the operator refuses or converts, wrapped tensors, a status other than FLA_OK): the Python class then runs
-// its own forward, which raises what there is to raise.
+// the operator refuses or converts, wrapped tensors, forward-mode tangents, a status other than FLA_OK): the Python
+// class then runs its own forward, which raises what there is to raise.
 #include <Python.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
@@ -70,7 +70,9 @@ bool plain(const Tensor &t) {
     using K = c10::DispatchKey;
     static const c10::DispatchKeySet odd({K::Python, K::PythonTLSSnapshot, K::FuncTorchBatched, K::FuncTorchGradWrapper,
                                           K::Functionalize, K::Conjugate, K::Negative, K::ZeroTensor});
-    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.dim() == 4 && !t.key_set().has_any(odd);
+    // (a forward-mode tangent: the operators have no formula for it, and the Python class says so)
+    return t.defined() && t.is_cuda() && t.layout() == at::kStrided && t.dim() == 4 && !t.key_set().has_any(odd) &&
+           !t._fw_grad(/*level=*/0).defined();
 }
 
 // q, k: (B, H, N, D_qk), v: (B, H, N, D_v), one device; `cast`: autocast turns any floating type into bf16
