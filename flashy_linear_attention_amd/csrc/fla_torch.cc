@@ -7,12 +7,13 @@
 // hand the interpreter lock to each other.
 //
 // Every entry point returns None where a call is not the plain case (tensor types and shapes that
-// the operator refuses or converts, wrapped tensors, forward-mode tangents, a status other than FLA_OK): the Python
-// class then runs its own forward, which raises what there is to raise.
+// the operator refuses or converts, wrapped tensors, forward-mode tangents, torch.jit.trace, a status other
+// than FLA_OK): the Python class then runs its own forward, which raises what there is to raise.
 #include <Python.h>
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/Exceptions.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/types.h>
 #include <ATen/autocast_mode.h>
 #include <c10/core/DeviceGuard.h>
@@ -398,6 +399,8 @@ struct Operands {
 
 Operands operands(PyObject *const *args) {
     Operands a;
+    // (torch.jit.trace records the Python Function as a whole; of the calls made here it would see the allocations alone)
+    if (torch::jit::tracer::isTracing()) return a;
     if (!THPVariable_Check(args[0]) || !THPVariable_Check(args[1]) || !THPVariable_Check(args[2])) return a;
     a.q = THPVariable_Unpack(args[0]), a.k = THPVariable_Unpack(args[1]), a.v = THPVariable_Unpack(args[2]);
     a.cast = at::autocast::is_autocast_enabled(at::kCUDA);

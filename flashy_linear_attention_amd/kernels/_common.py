@@ -13,7 +13,7 @@ _DTYPES = {torch.bfloat16: _lib.FLA_DTYPE_BF16, torch.float16: _lib.FLA_DTYPE_F1
 
 
 def next_power_of_2(x: int) -> int:
-    return 1 if x <= 1 else 1 << (x - 1).bit_length()
+    return 1 if x <= 1 else 1 << (int(x) - 1).bit_length()  # (under torch.jit.trace a size is a tensor)
 
 
 def dtype_code(t: torch.Tensor) -> int:

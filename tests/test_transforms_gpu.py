@@ -1,4 +1,5 @@
-"""The operators under forward-mode AD, which they refuse (``-m gpu``)."""
+"""The operators under forward-mode AD, which they refuse, and under ``torch.jit.trace``, which records them as the
+Python function (``-m gpu``)."""
 
 import pytest
 import torch
@@ -40,3 +41,13 @@ def test_forward_mode_is_refused(name, which, gpu_device):
         args[which] = torch.autograd.forward_ad.make_dual(args[which], torch.ones_like(args[which]))
         with pytest.raises((NotImplementedError, RuntimeError)):
             op(*args)
+
+
+@pytest.mark.parametrize("grad", [False, True], ids=["inference", "training"])
+@pytest.mark.parametrize("name", OPERATORS)
+def test_a_traced_call_computes(name, grad, gpu_device):
+    op, dqk, dv = OPERATORS[name]
+    first = tuple(t.requires_grad_(grad) for t in _inputs(dqk, dv, gpu_device))
+    traced = torch.jit.trace(lambda q, k, v: op(q, k, v), first, check_trace=False)
+    other = _inputs(dqk, dv, gpu_device, seed=1)
+    assert torch.equal(traced(*other), op(*other))
