@@ -1912,9 +1912,16 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
     const double w = (double)B * (double)H * (double)N * (double)N * (double)padded(D_qk > D_v ? D_qk : D_v);
     const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v, true);
     // Widths that are no multiples of 8: the quadratic operator runs the bounds-checked kernel, the chunk-wise one the
-    // fast kernels of either kind on copies with aligned rows, 1.4 to 12 times faster (forward + backward) over
-    // B H = 2 ... 128, N = 256 ... 2048 and widths 36, 91/64, 100, 153/64.
-    if (pack_plan(B, H, N, D_qk, D_v).ok) return 1;
+    // fast kernels of either kind on copies with aligned rows, at the cost of two copy launches.  Quadratic time over
+    // chunk-wise time, B H = 1 ... 64, at the last N below and the first N from the line on -- forward alone: 20 columns
+    // 0.95 to 1.06 at 512, 1.3 to 1.8 at 1024; 36 columns 0.80 to 0.86 at 128, 1.12 to 1.18 at 256; 91/64 and 100 0.91 to
+    // 1.1 at 64, 1.17 to 1.4 at 128; wider (153/64, 153/128, 250) 1.15 to 2.8 from 64 to 256.  Forward + backward: 20 columns
+    // 0.80 to 0.87 at 128, 1.12 to 1.21 at 256; 36 columns 0.92 to 0.97 at 64, 1.24 to 1.27 at 128; wider 1.1 to 3.3.
+    if (pack_plan(B, H, N, D_qk, D_v).ok) {
+        const int64_t d = padded(D_qk > D_v ? D_qk : D_v);
+        if (backward) return d <= 32 ? N >= 256 : d <= 64 ? N >= 128 : 1;
+        return d <= 32 ? N > 512 : d <= 64 ? N >= 256 : d <= 128 ? N >= 128 : 1;
+    }
     // (padded widths that differ: the quadratic side is the small-V operator, whose wide products are two launches)
     if (wp.ok && !backward) return wp.D <= 32 ? N >= 4096 || w >= 5e9 : N >= 2048 || w >= 1.2e10;
     if (wp.ok && pad_index(D_qk) != pad_index(D_v)) return N >= 1024 || w >= (wp.D <= 64 ? 1e9 : 5e8);
