@@ -376,8 +376,7 @@ int run_tri_chunked(const View &x, const View &y, const View &z, const View &out
 //            one backward kernel computes dQ, dV and dK of a chunk from one set of tiles;
 //   D = 128 (`split`): one workgroup per CU with two sets of tiles.  A per-chunk state would cost as
 //            much traffic as an operand, so forward hands over its segments' fp32 entry states
-//            only; backward is a forward-direction walk for dQ (from those entry states,
-//            transposed) and a reverse walk for dK and dV.  The totals kernel visits a part of the
+//            only (backward: chunked_backward).  The totals kernel visits a part of the
 //            sequence only (the last segment's total is never needed).
 struct WalkPlan {
     bool ok, split;
@@ -385,9 +384,9 @@ struct WalkPlan {
     int64_t n_chunks, seg_chunks, n_seg;  // the walks' segments
     int64_t entry_bytes;                  // fp32 entry states of the walk segments (formed in place over their totals)
     int64_t work_bytes;                   // workspace of one direction: the same
-    int64_t saved_bytes;                  // what forward hands to backward: the entry states and, behind them, the state
-                                          // after the last chunk of every (b, h); with the normaliser at padded head dims
-                                          // up to 64, the 16-bit state of every chunk (room for the larger of the two)
+    int64_t saved_bytes;                  // what forward hands to backward -- D = 128: the entry states and, behind them, the
+                                          // state after the last chunk of every (b, h); up to 64: the 16-bit state at the
+                                          // entry of every chunk
 };
 
 // `mixed`: also for head dims whose padded widths differ (128 / 64, 64 / 32, 64 / 128 ...), at the larger one: the tiles
@@ -427,8 +426,10 @@ WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, boo
     w.n_seg = (w.n_chunks + w.seg_chunks - 1) / w.seg_chunks;
     w.entry_bytes = B * H * w.n_seg * w.D * w.D * 4;
     w.work_bytes = w.entry_bytes;  // (a single segment needs them only with a feature map)
-    // (padded head dims up to 64: the per-chunk states of the normalised operator are the larger of the two)
-    const int64_t states = w.entry_bytes + B * H * w.D * w.D * 4, per_chunk = B * H * w.n_chunks * w.D * w.D * 2;
+    // (up to 64 with few chunks per segment: the size that held the segments' fp32 states, which callers of the C ABI may
+    // have set aside, stays the larger)
+    const int64_t states = w.entry_bytes + B * H * w.D * w.D * 4;
+    const int64_t per_chunk = B * H * w.n_chunks * w.D * w.D * 2;
     w.saved_bytes = w.split || states > per_chunk ? states : per_chunk;
     return w;
 }
@@ -960,10 +961,10 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         // the segments' entry states; with a feature map the same kernel maps xk as it loads it and
         // writes phi(xk), which the walk then reads (so it runs for a single segment as well)
         const bool need_totals = wp.n_seg > 1 || fmap;
-        // the entry states (and the state after the last chunk) are what backward gets, so the scan writes
+        // D = 128: the entry states (and the state after the last chunk) are what backward gets, so the scan writes
         // them to state_out (the totals themselves are computed there, and no workspace is used);
-        // the normalised operator at padded head dims up to 64 hands over the 16-bit state of every chunk instead
-        const bool in_state = state_out && (wp.split || !nx);
+        // padded head dims up to 64 hand over the 16-bit state of every chunk instead
+        const bool in_state = state_out && wp.split;
         // D = 128, a few segments more than two (kSumOnLoadMost): the totals go to the workspace, the walk adds them up itself as it starts
         // and writes the entry states it formed to state_out -- no scan launch (B H 64, N 4096: see wide_forward)
         const bool sum_on_load = wp.split && !fmap && !nx && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
@@ -1203,12 +1204,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         w.H = (int32_t)H, w.N = (int32_t)N, w.BH = (int32_t)(B * H), w.wqk = (int32_t)dqk, w.wv = (int32_t)dv;
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = entry;
-        if (nx) {
-            w.saved = const_cast<void *>(state_in);
-        } else {  // forward's entry states and, behind them, its state after the last chunk
-            w.xinit = static_cast<const float *>(state_in);
-            w.xtotal = reinterpret_cast<const float *>(static_cast<const char *>(state_in) + wp.entry_bytes);
-        }
+        w.saved = const_cast<void *>(state_in);
         if (nx) {
             const int64_t vb = walk_vec_bytes(B, H, N, dqk, dv);
             float *zc = static_cast<float *>(nx->vec), *rcv = reinterpret_cast<float *>(static_cast<char *>(nx->vec) + vb);

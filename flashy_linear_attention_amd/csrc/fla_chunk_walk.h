@@ -25,11 +25,9 @@
 //
 //   D <= 64: 128-row chunks, two workgroups per CU.  ONE backward kernel (walk_bwd_kernel)
 //            computes dQ, dV and dK of a chunk from one set of tiles; dQ's state -- the sum of
-//            K^T V over the chunks BEFORE -- is obtained going backwards, by subtracting every
-//            chunk's K^T V from the forward state at the segment's end, so forward hands over
-//            only its segments' fp32 entry states and the state after the last chunk.  (With
-//            the normaliser, whose vectors take the LDS a second state copy would need, forward
-//            saves the 16-bit state at the entry of every chunk instead.)
+//            K^T V over the chunks BEFORE -- is the 16-bit copy that forward multiplied q by, saved at
+//            the entry of every chunk (half the bytes of one operand at D = 64).  Nothing of a row
+//            reaches the dQ of the chunks before it.
 //   D = 128: tiles and state must share the 160 KiB of LDS: 64-row chunks, one workgroup per CU
 //            with two sets of tiles (the next chunk's loads are in flight while this one is
 //            multiplied).  A saved per-chunk state would cost as much traffic as an operand, so
@@ -90,8 +88,8 @@ struct WalkParams {
     // transposed matrices ([v index][q/k index]).
     const float *init;
     int32_t init_transposed;
-    // forward: where the 16-bit state at the entry of every chunk goes, [BH][n_chunks][D][D]
-    // ([q/k index][v index]), or null; backward: the same buffer, read for dQ
+    // forward, D <= 64: where the 16-bit state at the entry of every chunk goes, [BH][n_chunks][D][D], or null; backward:
+    // the same buffer, read for dQ.  Laid out as its copy in LDS (unscaled); with the normaliser [q/k index][v index].
     void *saved;
     // Feature map (fla_feature.h), 0: none.  Forward: q holds the argument xq of the map phi; the Q
     // tile is mapped in LDS as it lands and phi(xq) is written to qmap_out (q's shape, element
@@ -729,6 +727,18 @@ __device__ __forceinline__ void walk_state_to_lds(unsigned char *tl, int wave, i
     }
 }
 
+// a chunk's saved copy (WalkParams::saved) HBM -> LDS, as it lay there
+template <int D>
+__device__ __forceinline__ void walk_load_state_copy(const void *src, uint32_t lds_dst, int wave, int lane) {
+    constexpr int LOADS = WalkCfg<D>::STATE / 1024;  // of a wave each
+    const u32x4 rs = walk_uniform_rsrc(src, WalkCfg<D>::STATE);
+    const uint32_t base = (uint32_t)__builtin_amdgcn_readfirstlane((int)(lds_dst + wave * 1024));
+    static_for<0, (LOADS + 3) / 4>([&](auto u) {
+        constexpr int U = decltype(u)::value;
+        if (4 * U + wave < LOADS) dma_16B_per_lane<U * 4096>(rs, base, (uint32_t)(wave * 1024 + lane * 16), U * 4096);
+    });
+}
+
 // fp16: the sums of a long sequence leave its range where results of the operator do not, so the state's 16-bit copy is
 // scaled by a power of two that puts its largest element at 2^14 (exact; what is 2^28 times smaller than that becomes
 // subnormal).  Every wave leaves its largest |element| in smax[wave]; behind a barrier walk_state_scale gives
@@ -921,7 +931,7 @@ __device__ __forceinline__ void walk_load_init_from(const float *buf, const Walk
             walk_sum_states<D, B>(buf + (int64_t)sl.bh * p.n_seg * (D * D), reverse ? sl.seg + 1 : 0,
                                   reverse ? p.n_seg : sl.seg, p.init_transposed != 0, wave, lane, st);
             return;
-        } else {
+        } else if (sl.seg != (reverse ? p.n_seg - 1 : 0)) {  // (the first one in walking order starts from zero)
             init = buf + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D);
         }
     }
@@ -1131,6 +1141,19 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                 __syncthreads();
             }
         }
+        if constexpr (!DOUBLE && NORM == 0) {
+            if (p.saved && c > 0) {  // the state's copy for backward's dQ (at the first chunk it is zero and not read)
+                unsigned char *sv = static_cast<unsigned char *>(p.saved) + ((int64_t)sl.bh * p.n_chunks + c) * W::STATE;
+                for (int i = tid * 16; i < W::STATE; i += 4096) {
+                    V8 copy = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4 *>(tl + i));
+                    if constexpr (SCALED) {
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) copy[e] = static_cast<T>(static_cast<float>(copy[e]) * sback);
+                    }
+                    *reinterpret_cast<u32x4 *>(sv + i) = __builtin_bit_cast(u32x4, copy);
+                }
+            }
+        }
         if constexpr (ACCUM) prev.request(ro, os2, p.wv, row, g, db0);
         f32x16 acc[W::DBW];
         const float *vz = reinterpret_cast<const float *>(xv + (NORM == 1 ? 0 : buf * W::VEC));
@@ -1164,7 +1187,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         }
         if constexpr (ACCUM) prev.add_to(acc);
         walk_store<T, D, OB::PER>(ro, os2, p.wv, row, g, db0, acc);
-        if (!DOUBLE && p.saved) {  // the state at the entry of this chunk, [q/k index][v index], for backward's dQ
+        if (!DOUBLE && NORM == 1 && p.saved) {  // the state at the entry of this chunk, [q/k index][v index], for backward's dQ
             T *sv = static_cast<T *>(p.saved) + ((int64_t)sl.bh * p.n_chunks + c) * (D * D);
 #pragma unroll
             for (int i = 0; i < B::SLOTS; ++i)
@@ -1342,12 +1365,12 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
 }
 
 // ---- backward: dQ, dV, dK of a chunk from one set of tiles; R += Q_c^T dO_c, chunks descending.
-// dQ's state, the sum of K^T V over the chunks before:
-//   NORM (the normaliser's terms): the 16-bit state forward saved at the entry of every chunk
-//   (WalkParams::saved), fragments straight from memory;
-//   otherwise obtained backwards as in walk_bwd_rev_kernel: X starts as the forward state at the
-//   segment's end (xinit / xtotal) and every chunk's K^T V is subtracted when the walk reaches it;
-//   X has a 16-bit copy of its own in LDS beside R's.  Forward then saves no per-chunk states.
+// dQ's state, the sum of K^T V over the chunks before: the 16-bit copy forward saved at the entry of every chunk
+// (WalkParams::saved), brought to LDS with the chunk's tiles; NORM (the normaliser's terms, whose vectors take that
+// place in LDS): fragments straight from memory.
+// (Obtained backwards instead -- from the state at the segment's end, subtracting every chunk's K^T V when the walk reaches
+// it -- one late row that is infinite, NaN or merely huge spoiled the dQ of every chunk before it.  Forward + backward
+// at B H 16, N 32768, D 64 that way 222 us, this way 234.)
 template <typename T, int D, bool NORM>
 __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1358,7 +1381,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
     unsigned char *tq = smem, *tk = smem + W::TILE, *tv = smem + 2 * W::TILE, *tg = smem + 3 * W::TILE,
                   *tl = smem + 4 * W::TILE;
-    unsigned char *tx = tl + W::STATE;  // (!NORM) X's copy; (NORM) the chunk's vectors
+    unsigned char *tx = tl + W::STATE;  // (!NORM) dQ's state; (NORM) the chunk's vectors
     const float *vz = reinterpret_cast<const float *>(tl + W::STATE), *vr = vz + 256, *vd = vz + 512;
     const uint32_t xbase = lds0 + 4 * W::TILE + W::STATE;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
@@ -1386,13 +1409,11 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
     f32x16 st[W::NBW];  // R[q/k index][v index]
     walk_load_init<D>(p, sl, wave, lane, st, true);
     walk_state_to_lds<T, D>(tl, wave, lane, st);
-    f32x16 xs[W::NBW];  // X[q/k index][v index]
-    if constexpr (!NORM)
-        walk_load_end_state<D>(p, sl, wave, lane, xs);
 
 #pragma unroll 1
     for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
         const int row0 = c * W::C;
+        const int64_t at = (int64_t)sl.bh * p.n_chunks + c;
         walk_load_tile<D>(rq, lds0, row0, qs2, p.wqk, wave, lane);
         walk_load_tile<D>(rk, lds0 + W::TILE, row0, ks2, p.wqk, wave, lane);
         walk_load_tile<D>(rv, lds0 + 2 * W::TILE, row0, vs2, p.wv, wave, lane);
@@ -1401,13 +1422,15 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
             walk_load_vec<D>(p.zc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase, lane);
             walk_load_vec<D>(p.rc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase + 1024, lane);
             walk_load_rows<D>(p.dn + (int64_t)sl.bh * N, row0, N, xbase + 2048, lane);
+        } else if (c > 0) {
+            walk_load_state_copy<D>(static_cast<const unsigned char *>(p.saved) + at * W::STATE, xbase, wave, lane);
         }
         // NORM: dQ's state, S_c[q/k index][v index] as saved by forward: A-operand fragments straight from
         // memory (row = output column of dQ, eight consecutive v indices)
         V8 sfq[NORM ? W::DB : 1][NORM ? W::KC : 1];
         if constexpr (NORM) {
             const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                static_cast<T *>(p.saved) + ((int64_t)sl.bh * p.n_chunks + c) * (D * D), 0, D * D * 2, 0x00020000);
+                static_cast<T *>(p.saved) + at * (D * D), 0, D * D * 2, 0x00020000);
             if (c > 0) {
 #pragma unroll
                 for (int db = 0; db < W::DB; ++db)
@@ -1429,9 +1452,6 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
                                          acc, &ax);
             walk_add_vec<D>(acc, ax, vz, 0, g);
             walk_store<T, D>(rdq, dqs2, p.wqk, row, g, 0, acc, p.fmap, tq, 32 * wave + l32);
-        } else {
-            walk_update<T, D, WalkExt<D>, true>(tk, tv, wave, lane, xs);  // X: now the sum over the chunks before this one
-            walk_state_to_lds<T, D>(tx, wave, lane, xs);
         }
         // dV = upper(K Q^T) dO + K R: A operand R^T[v index][q/k index] = the LDS copy as it is
         walk_product<T, D, true>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
@@ -1454,8 +1474,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
         }
         walk_store<T, D>(rdk, dks2, p.wqk, row, g, 0, acc, p.fmap, tk, 32 * wave + l32);
         if constexpr (!NORM) {
-            __syncthreads();  // every wave's part of X is in LDS
-            // dQ = lower(dO V^T) K + dO X^T: A operand X[q/k index][v index], its LDS copy read transposed
+            // dQ = lower(dO V^T) K + dO S_c^T: A operand S_c[q/k index][v index], its LDS copy read transposed
             walk_product<T, D, false>(tg, tv, tk, wave, lane, c > 0, [&](int db, int kc) -> V8 {
                 return walk_col_frag_perm<T, D>(tx, 16 * kc, db, lane, true);
             }, acc);
@@ -2379,9 +2398,9 @@ hipError_t launch_walk_bwd(const WalkParams &p, hipStream_t stream) {
         if (hipError_t e = ensure_dynamic_lds<kern>(smem_n)) return e;
         return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_n, stream, p);
     }
-    if (!p.xtotal || (p.n_seg > 1 && !p.xinit)) return hipErrorInvalidValue;
+    if (!p.saved) return hipErrorInvalidValue;
     constexpr auto kern = walk_bwd_kernel<T, D, false>;
-    constexpr int smem_x = smem + WalkCfg<D>::STATE;  // X's copy beside R's
+    constexpr int smem_x = smem + WalkCfg<D>::STATE;  // dQ's state beside R
     if (hipError_t e = ensure_dynamic_lds<kern>(smem_x)) return e;
     return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_x, stream, p);
 }
