@@ -552,15 +552,14 @@ bool states_shareable(int64_t dqk, int64_t dv, int64_t N) {
 // the two 128-column halves of q and k and everything is linear in them:
 //     O  = tril(Q_0 K_0^T) V + tril(Q_1 K_1^T) V        dV = the same sum of the halves' dV
 //     dQ_h = tril(dO V^T) K_h                           dK_h = triu(V dO^T) Q_h
-// so each half runs the D = 128 walk kernels on column views of q, k, dq, dk (v and dO are padded
-// with zeros in LDS, never in memory); the second half's walk adds its O (its part of dV) to what the
-// first one wrote.  Forward hands over both halves' entry and final states, and backward of a half
-// is then one reverse walk; without them it is the forward-direction walk for dQ_h and the dK / dV
-// walk, whose second dV goes to a scratch tensor that one element-wise pass adds.
+// so each half is a D = 128 walk on column views of q, k, dq, dk (v and dO are padded with zeros in
+// LDS, never in memory), and one launch walks both halves of a chunk, O and dV in fp32 from the first
+// half to the second.  Forward hands over both halves' entry and final states.  Backward is one reverse
+// walk with them and a v of at most 64 columns (wide_backward says when); otherwise a reverse walk for dK
+// and dV and a forward-direction walk per half for dQ_h.
 struct WidePlan {
     bool ok;
-    WalkPlan wp;         // the plan of a 128 / 128 problem of the same B, H, N
-    int64_t temp_bytes;  // the second half's dV in backward without forward's states, contiguous (B, H, N, D_v)
+    WalkPlan wp;  // the plan of a 128 / 128 problem of the same B, H, N
 };
 
 WidePlan wide_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
@@ -568,7 +567,6 @@ WidePlan wide_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
     if (dqk <= 128 || dqk > 256 || dv > 128) return w;
     w.wp = walk_plan(B, H, N, 128, 128);
     w.ok = w.wp.ok;
-    w.temp_bytes = (B * H * N * dv * 2 + 255) / 256 * 256;
     return w;
 }
 
@@ -630,9 +628,9 @@ int64_t shared_state_bytes(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t
     return core ? core + walk_vec_bytes(B, H, N, dqk, dv) : 0;
 }
 
-// workspace of the two-halves evaluation: the scratch tensor for dV, then totals and entry states of both
-// halves (two sets of them in backward: Q^T dO, and K^T V when forward's entry states are not given)
-int64_t wide_workspace_bytes(const WidePlan &w) { return w.temp_bytes + 4 * w.wp.work_bytes; }
+// workspace of the two-halves evaluation: totals and entry states of both halves (two sets of them in
+// backward: Q^T dO, and K^T V when forward's entry states are not given)
+int64_t wide_workspace_bytes(const WidePlan &w) { return 4 * w.wp.work_bytes; }
 
 int64_t chunked_op_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
     const int64_t shared = shared_state_bytes(B, H, N, dqk, dv);
@@ -711,12 +709,12 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
     float *keep[2] = {nullptr, nullptr};
     if (wp.n_seg > 1) {
         // (kept for backward when there is a state buffer: each half's entry states, its final state behind them;
-        // otherwise, and the totals that the walk adds up, in the workspace behind the scratch tensor)
+        // otherwise, and the totals that the walk adds up, in the workspace)
         void *work[2];
         for (int h = 0; h < 2; ++h) {
             if (state_out) keep[h] = reinterpret_cast<float *>(static_cast<char *>(state_out) + h * wp.saved_bytes);
             work[h] = keep[h] && !sum_on_load ? static_cast<void *>(keep[h])
-                                              : static_cast<void *>(ws + wide.temp_bytes + h * wp.work_bytes);
+                                              : static_cast<void *>(ws + h * wp.work_bytes);
         }
         float *const none[2] = {nullptr, nullptr};
         if (int rc = wide_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0, work, sum_on_load ? none : keep, entry, s,
@@ -734,79 +732,54 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
     return fla::walk_fwd_wide(dtype, w, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 
+// With forward's states at hand and a narrow v: one reverse walk over both halves, dQ included, whose state goes
+// backwards by subtraction from the state at the segment's end (walk_bwd_rev_wide_kernel).  A wider v or no states: dQ_h
+// by forward-direction walks.  Backward at B 4, H 16, N 4096, 256 / 128: 297 us as a reverse walk per half, the second
+// adding to the first one's dV in memory, 279 us this way.
 int wide_backward(const WidePlan &wide, const View &go, const View &q, const View &k, const View &v, const View &dq,
                   const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                   const void *state_in, void *workspace, hipStream_t s) {
     const WalkPlan &wp = wide.wp;
     char *ws = static_cast<char *>(workspace);
-    const int64_t temp_strides[4] = {H * N * dv, N * dv, dv, 1};
-    const View temp{ws, temp_strides};
-    const bool one_walk = state_in && dv <= 64;  // forward's states at hand, narrow v: one reverse walk over both halves
+    const bool one_walk = state_in && dv <= 64;
     // entry states of both halves up front: Q_h^T dO over the segments after, and -- when forward's are not
     // at hand -- K_h^T V over the segments before
     const float *fwd_entries[2] = {nullptr, nullptr}, *entries[2] = {nullptr, nullptr};
-    // (the reverse walks add up the totals of the segments after their own themselves, as forward does)
-    const bool rev_sums_on_load = state_in && wp.n_seg >= 3 && wp.n_seg <= 7;
+    // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
+    const bool rev_sums_on_load = wp.n_seg >= 3 && wp.n_seg <= 7;
     if (wp.n_seg > 1) {
         float *const none[2] = {nullptr, nullptr};
-        char *base = ws + wide.temp_bytes;
         if (state_in) {
             for (int h = 0; h < 2; ++h)
                 fwd_entries[h] = reinterpret_cast<const float *>(static_cast<const char *>(state_in) + h * wp.saved_bytes);
         } else {
-            void *const work[2] = {base + 2 * wp.work_bytes, base + 3 * wp.work_bytes};
-            if (int rc = wide_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0, work, none, fwd_entries, s)) return rc;
+            void *const work[2] = {ws + 2 * wp.work_bytes, ws + 3 * wp.work_bytes};
+            if (int rc = wide_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0, work, none, fwd_entries, s, false, dv <= 64))
+                return rc;
         }
-        void *const work[2] = {base, base + wp.work_bytes};
-        if (int rc = wide_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, work, none, entries, s, rev_sums_on_load,
-                                       one_walk))
+        void *const work[2] = {ws, ws + wp.work_bytes};
+        if (int rc = wide_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, work, none, entries, s, rev_sums_on_load, dv <= 64))
             return rc;
     }
+    fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, 128, dv);
+    r.wqk2 = (int32_t)(dqk - 128);
+    r.init = entries[0], r.init2 = entries[1], r.init_is_totals = rev_sums_on_load;
     if (one_walk) {
-        fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, 128, dv);
-        r.wqk2 = (int32_t)(dqk - 128);
-        r.init = entries[0], r.init2 = entries[1], r.init_is_totals = rev_sums_on_load;
         const char *half0 = static_cast<const char *>(state_in), *half1 = half0 + wp.saved_bytes;
         r.xinit = reinterpret_cast<const float *>(half0), r.xinit2 = reinterpret_cast<const float *>(half1);
         r.xtotal = reinterpret_cast<const float *>(half0 + wp.entry_bytes);
         r.xtotal2 = reinterpret_cast<const float *>(half1 + wp.entry_bytes);
         return fla::walk_bwd_rev_wide(dtype, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
+    // dQ_h = lower(dO V^T) K_h + dO S_h^T: the forward walk over (dO, V, K_h)
     for (int h = 0; h < 2; ++h) {
-        const View qh = column_half(q, h), kh = column_half(k, h), dqh = column_half(dq, h), dkh = column_half(dk, h);
-        const int64_t wqk = h == 0 ? 128 : dqk - 128;
-        const float *fwd_entry = fwd_entries[h], *entry = entries[h];
-        const View &dvh = h == 0 ? dvv : temp;
-        if (state_in) {  // forward's states at hand: dQ_h, dK_h and this half's part of dV in one reverse walk
-            fla::WalkParams r = reverse_walk_params(wp, go, qh, kh, v, dqh, dkh, dvv, B, H, N, wqk, dv);
-            r.accumulate = h;  // (the second half's walk adds its part of dV to the first one's)
-            r.init = entry, r.init_is_totals = rev_sums_on_load;
-            const char *half = static_cast<const char *>(state_in) + h * wp.saved_bytes;
-            r.xinit = reinterpret_cast<const float *>(half);
-            r.xtotal = reinterpret_cast<const float *>(half + wp.entry_bytes);
-            if (fla::walk_bwd_rev(dtype, wp.D, r, s) != hipSuccess) return FLA_ERR_LAUNCH;
-            continue;
-        }
-        // dQ_h = lower(dO V^T) K_h + dO S_h^T: the forward walk over (dO, V, K_h)
-        fla::WalkParams w = lower_walk_params(wp, go, v, kh, dqh, B, H, N, dv, wqk, fwd_entry);
+        fla::WalkParams w = lower_walk_params(wp, go, v, column_half(k, h), column_half(dq, h), B, H, N, dv, h ? dqk - 128 : 128,
+                                              fwd_entries[h]);
         w.init_transposed = 1;
         if (fla::walk_fwd(dtype, wp.D, w, s) != hipSuccess) return FLA_ERR_LAUNCH;
-        // dV (this half's part) and dK_h: the reverse walk
-        fla::WalkParams r{};
-        r.q = qh.ptr, r.k = kh.ptr, r.v = v.ptr, r.go = go.ptr;
-        r.dk = const_cast<void *>(dkh.ptr), r.dv = const_cast<void *>(dvh.ptr);
-        r.qs_b = qh.strides[0], r.qs_h = qh.strides[1], r.qs_n = qh.strides[2];
-        r.ks_b = kh.strides[0], r.ks_h = kh.strides[1], r.ks_n = kh.strides[2];
-        r.vs_b = v.strides[0], r.vs_h = v.strides[1], r.vs_n = v.strides[2];
-        r.gs_b = go.strides[0], r.gs_h = go.strides[1], r.gs_n = go.strides[2];
-        r.dks_b = dkh.strides[0], r.dks_h = dkh.strides[1], r.dks_n = dkh.strides[2];
-        r.dvs_b = dvh.strides[0], r.dvs_h = dvh.strides[1], r.dvs_n = dvh.strides[2];
-        r.H = (int32_t)H, r.N = (int32_t)N, r.BH = (int32_t)(B * H), r.wqk = (int32_t)wqk, r.wv = (int32_t)dv;
-        r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
-        r.init = entry;
-        if (fla::walk_dkdv(dtype, wp.D, r, s) != hipSuccess) return FLA_ERR_LAUNCH;
     }
-    return state_in ? FLA_OK : launch_feature_pass(3, 0, temp, dvv, B, H, N, dv, dtype, s);
+    r.dq = nullptr;
+    return fla::walk_bwd_rev_wide(dtype, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 
 // ---- D_qk and D_v in (128, 256]: two column halves of q / k and two of v, four pairs with a state each.  One launch
@@ -877,7 +850,7 @@ int quad_backward(const WalkPlan &wp, const View &go, const View &q, const View 
     r.init = wp.n_seg > 1 ? entries : nullptr, r.init_is_totals = quad_sums_on_load(wp);
     r.xinit = static_cast<const float *>(state_in), r.xtotal = quad_finals(wp, state_in);
     for (int pass = 0; pass < 2; ++pass) {
-        r.quad = 3 - pass, r.accumulate = 2 * pass;
+        r.quad = 3 - pass, r.accumulate = pass;
         if (fla::walk_bwd_rev(dtype, wp.D, r, s) != hipSuccess) return FLA_ERR_LAUNCH;
     }
     return FLA_OK;
@@ -1119,7 +1092,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         const float *entry = nullptr;
         // with forward's states at hand (and without the normaliser): one reverse walk
         const bool one_walk = state_in && !nx;
-        // (... which adds up the totals of the segments after its own itself, as forward does)
+        // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
         const bool rev_sums_on_load = one_walk && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
         if (wp.n_seg > 1) {
             if (!state_in) {
@@ -1348,7 +1321,7 @@ int packed_backward(const PackPlan &p, const View &go, const View &q, const View
     }
     if (int rc = in.launch(stream)) return rc;
     if (int rc = chunked_backward(gop, qp, kp, vp, dqp, dkp, dvp, B, H, N, p.wq, p.wv, dtype, state_in, workspace, p.inner_work,
-                                  stream))
+                                  stream, 0, nullptr))
         return rc;
     return out.launch(stream);
 }

@@ -122,8 +122,8 @@ struct WalkParams {
     // states (xinit, the layout of `init`, not transposed; may be null with a single segment).
     float *total_out;
     const float *xinit, *xtotal;
-    // D = 128, plain: the result (forward: o; walk_bwd_rev_kernel: dv, with 2 dq and dk as well) is added to what its
-    // place in memory holds already -- the second of two walks whose results sum up (halves of a wide q / k, of v)
+    // walk_bwd_rev_kernel with `quad`: the results are added to what their places in memory hold already -- the second of
+    // two walks whose results sum up
     int32_t accumulate;
     // The wide walks (walk_fwd_wide_kernel, walk_bwd_rev_wide_kernel): q and k (dq and dk) have 129 .. 256
     // columns.  Columns 128 .. are the second half, of true width wqk2 (wqk = 128 is the first half's), with
@@ -993,12 +993,11 @@ __device__ __forceinline__ void walk_write_state(float *out, int wave, int lane,
 // NORM: the instantiations that take the normaliser's terms: 1 forward (WalkParams::denom), 2 dQ (dn).
 // FM: the instantiations that know of feature maps (WalkParams::fmap, slope_y); the others ignore both.
 // NQ, NV: blocks of the state [q/k index][v index] that hold anything (WalkExt).
-// ACCUM: the result is added to what o holds already (WalkParams::accumulate, WalkPrev).
 // the plain fp16 forward: walk_state_scale
 template <typename T, int NORM, bool FM>
 constexpr bool walk_fwd_scaled = std::is_same<T, _Float16>::value && NORM == 0 && !FM;
 
-template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool ACCUM = false>
+template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32>
 __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1006,7 +1005,6 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     using B = WalkExt<D, NQ, NV>;
     using OB = WalkOut<D, NV>;  // the result is as wide as v
     static_assert(NORM == 0 || (NQ == W::DB && NV == W::DB), "the normaliser's variants are built for full widths");
-    static_assert(!ACCUM || (DOUBLE && NORM == 0 && !FM), "adding to the result: the plain D = 128 walk only");
     constexpr int SETS = DOUBLE ? 2 : 1;
     constexpr bool SCALED = walk_fwd_scaled<T, NORM, FM>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -1089,8 +1087,6 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         }
     };
     constexpr int n_extra = NORM == 2 ? 1 + W::NID : 0;  // loads per chunk and wave beyond the tiles
-    // ACCUM: the result is added to what o holds (in fp32, before the one rounding)
-    WalkPrev<T, D, OB::PER> prev;
     if constexpr (DOUBLE) load_chunk(sl.c_lo, 0);
 #pragma unroll 1
     for (int c = sl.c_lo; c < sl.c_hi; ++c) {
@@ -1154,7 +1150,6 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                 }
             }
         }
-        if constexpr (ACCUM) prev.request(ro, os2, p.wv, row, g, db0);
         f32x16 acc[W::DBW];
         const float *vz = reinterpret_cast<const float *>(xv + (NORM == 1 ? 0 : buf * W::VEC));
         const float *vd = reinterpret_cast<const float *>(xv + buf * W::VEC + 2048);
@@ -1185,7 +1180,6 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                         acc[i][v] *= feature_slope_c<decltype(map)::value>(static_cast<float>(ys[i][v / 8][v % 8]));
             });
         }
-        if constexpr (ACCUM) prev.add_to(acc);
         walk_store<T, D, OB::PER>(ro, os2, p.wv, row, g, db0, acc);
         if (!DOUBLE && NORM == 1 && p.saved) {  // the state at the entry of this chunk, [q/k index][v index], for backward's dQ
             T *sv = static_cast<T *>(p.saved) + ((int64_t)sl.bh * p.n_chunks + c) * (D * D);
@@ -1638,7 +1632,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 // The one 16-bit state in LDS holds R for dV and dK, then X for dQ.  q, k, v, dO are read once and
 // nothing but the results is written, where the walk for dQ followed by walk_dkdv_kernel reads
 // dO, v, k twice.
-template <typename T, int D, int NQ = D / 32, int NV = D / 32, int ACCUM = 0, bool FM = false>
+template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool ACCUM = false, bool FM = false>
 __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1699,7 +1693,7 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
-    // ACCUM 1, 2: dV, 2: dK and dQ too are added to what their places hold (in fp32, before the one rounding)
+    // ACCUM: the results are added to what their places hold (in fp32, before the one rounding)
     WalkPrev<T, D, OV::PER> prev;
     WalkPrev<T, D, OQ::PER> prev_qk;
     load_chunk(sl.c_hi - 1, 0);
@@ -1725,21 +1719,14 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
         walk_product<T, D, true, 0, B::KQ, NV>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
         }, acc);
-        // ACCUM 1: dV waits for the end of the chunk (see WalkPrev).  (2: no registers left for that)
-        f32x16 held[W::DBW];
-        if constexpr (ACCUM == 1) {
-#pragma unroll
-            for (int i = 0; i < OV::PER; ++i) held[i] = acc[i];
-        } else {
-            if constexpr (ACCUM == 2) prev.add_to(acc);
-            walk_store<T, D, OV::PER>(rdv, dvs2, wv, row, g, OV::db0(wave), acc);
-        }
-        if constexpr (ACCUM == 2) prev_qk.request(rdk, dks2, wqk, row, g, OQ::db0(wave));
+        if constexpr (ACCUM) prev.add_to(acc);
+        walk_store<T, D, OV::PER>(rdv, dvs2, wv, row, g, OV::db0(wave), acc);
+        if constexpr (ACCUM) prev_qk.request(rdk, dks2, wqk, row, g, OQ::db0(wave));
         // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
         walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
-        if constexpr (ACCUM == 2) prev_qk.add_to(acc);
+        if constexpr (ACCUM) prev_qk.add_to(acc);
         walk_store<T, D, OQ::PER>(rdk, dks2, wqk, row, g, OQ::db0(wave), acc, fmap, tk, 32 * rb + l32);
         // R += Q^T dO touches registers and tiles only, so it can sit on either side of the barriers: the waves of
         // the last row block, with one score block in dV and dK against two, take it here, the others after dQ,
@@ -1756,17 +1743,13 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
             asm volatile("" : "+a"(xs[0]), "+a"(xs[1]));
         walk_state_to_lds<T, D, B>(tl, wave, lane, xs);
         sync();  // X is in LDS
-        if constexpr (ACCUM == 2) prev_qk.request(rdq, dqs2, wqk, row, g, OQ::db0(wave));
+        if constexpr (ACCUM) prev_qk.request(rdq, dqs2, wqk, row, g, OQ::db0(wave));
         // dQ = lower(dO V^T) K + dO X^T: A operand X[q/k index][v index], read transposed like R for dK
         walk_product<T, D, false, 0, B::KV, NQ>(tg, tv, tk, wave, lane, c > 0, [&](int db, int kc) -> V8 {
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
-        if constexpr (ACCUM == 2) prev_qk.add_to(acc);
+        if constexpr (ACCUM) prev_qk.add_to(acc);
         walk_store<T, D, OQ::PER>(rdq, dqs2, wqk, row, g, OQ::db0(wave), acc, fmap, tq, 32 * rb + l32);
-        if constexpr (ACCUM == 1) {
-            prev.add_to(held);
-            walk_store<T, D, OV::PER>(rdv, dvs2, wv, row, g, OV::db0(wave), held);
-        }
         if (!(kSplitUpdate && rb == 1)) walk_update<T, D, B, false, true>(tq, tg, wave, lane, st);
         sync();  // every wave has read X and is done with the tiles
         walk_state_to_lds<T, D, B>(tl, wave, lane, st);
@@ -1776,20 +1759,21 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
 #endif
 }
 
-// ---- walk_bwd_rev_kernel for q and k of 129 .. 256 columns against a v of at most 64: one reverse walk over
+// ---- the reverse walk for q and k of 129 .. 256 columns against a v of at most 128: one walk over
 // both 128-column halves.  Per chunk and half h, with R_h and X_h the states of walk_bwd_rev_kernel for the half:
 //   dV  += upper(K_h Q_h^T) dO + K_h R_h        (fp32 accumulators from the first half to the second, stored once)
-//   dK_h = upper(V dO^T) Q_h + V R_h^T          dQ_h = lower(dO V^T) K_h + dO X_h^T
-// V and dO are loaded once per chunk, where two walks of walk_bwd_rev_kernel, the second adding its part of dV to
-// the first one's, load them twice, write dV twice and read it back once.
+//   dK_h = upper(V dO^T) Q_h + V R_h^T
+//   WITH_DQ: dQ_h = lower(dO V^T) K_h + dO X_h^T     (otherwise dQ_h is a walk_fwd_kernel launch of its own)
+// V and dO are loaded once per chunk.  (A walk per half, the second adding its part of dV to the first one's in memory,
+// loaded them twice and rounded that part of dV once more.)
 // LDS as in walk_fwd_wide_kernel: a set of (Q_h, K_h) tiles per half, two (V, dO) pairs by chunk parity, and ONE
 // 16-bit state that holds R_h, then X_h, of the half at work; at the end of a half-chunk the other half's R (in
-// registers throughout) is rounded into it.  Four states in registers: built for v blocks NV = 2 only.
-template <typename T, int NV>
+// registers throughout) is rounded into it.  With dQ four states in registers: built for v blocks NV = 2 only.
+template <typename T, int NV, bool WITH_DQ>
 __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int D = 128, NQ = D / 32;
-    static_assert(NV == 2, "R and X of both halves live in registers: two blocks per wave and state");
+    static_assert(!WITH_DQ || NV == 2, "R and X of both halves live in registers: two blocks per wave and state");
     using W = WalkCfg<D>;
     using V8 = typename Mma<T>::V8;
     using B = WalkExt<D, NQ, NV>;   // R, X [q/k index][v index]
@@ -1829,13 +1813,20 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
     f32x16 xs0[W::NBW], xs1[W::NBW];  // X_0, X_1
     if (p.init_is_totals) {
         const int64_t at = (int64_t)sl.bh * p.n_seg * (D * D);
-        walk_sum_two<D, B>(p.init + at, p.init2 + at, sl.seg + 1, p.n_seg, wave, lane, st0, st1);
+        if constexpr (NV == 2) {
+            walk_sum_two<D, B>(p.init + at, p.init2 + at, sl.seg + 1, p.n_seg, wave, lane, st0, st1);
+        } else {
+            walk_sum_states<D, B>(p.init + at, sl.seg + 1, p.n_seg, false, wave, lane, st0);
+            walk_sum_states<D, B>(p.init2 + at, sl.seg + 1, p.n_seg, false, wave, lane, st1);
+        }
     } else {
         walk_load_init_from<D, B>(p.init, p, sl, wave, lane, st0, true);
         walk_load_init_from<D, B>(p.init2, p, sl, wave, lane, st1, true);
     }
-    walk_load_end_state_from<D, B>(p.xinit, p.xtotal, p, sl, wave, lane, xs0);
-    walk_load_end_state_from<D, B>(p.xinit2, p.xtotal2, p, sl, wave, lane, xs1);
+    if constexpr (WITH_DQ) {
+        walk_load_end_state_from<D, B>(p.xinit, p.xtotal, p, sl, wave, lane, xs0);
+        walk_load_end_state_from<D, B>(p.xinit2, p.xtotal2, p, sl, wave, lane, xs1);
+    }
     walk_state_to_lds<T, D, B>(tl, wave, lane, st0);
 
     auto load_half = [&](int c, auto half) {  // Q_h, K_h of chunk c to set h
@@ -1887,22 +1878,24 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
                 }
             }
             sync();  // the tiles have landed, R_h is in LDS
-            walk_update<T, D, B, true, true>(tk, tv, wave, lane, xs);  // X_h: now the sum over the chunks before this one
+            if constexpr (WITH_DQ) walk_update<T, D, B, true, true>(tk, tv, wave, lane, xs);  // X_h: now the sum over the chunks before this one
             walk_product<T, D, true, 0, B::KQ, NV, HF != 0>(tk, tq, tg, wave, lane, later, rows_of_state, dvacc);
             f32x16 acc[W::DBW];
             walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, cols_of_state, acc);
             walk_store<T, D, OQ::PER>(HF ? rdk1 : rdk0, dks2, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc);
-            sync();  // every wave has read R_h
-            // (X stays in its accumulation registers up to here: without this the copies that the rounding
-            // below reads are made right after the update and occupy registers through both products)
-            asm volatile("" : "+a"(xs[0]), "+a"(xs[1]));
-            walk_state_to_lds<T, D, B>(tl, wave, lane, xs);
-            sync();  // X_h is in LDS
-            walk_product<T, D, false, 0, B::KV, NQ>(tg, tv, tk, wave, lane, c > 0, cols_of_state, acc);
-            walk_store<T, D, OQ::PER>(HF ? rdq1 : rdq0, dqs2, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc);
+            if constexpr (WITH_DQ) {
+                sync();  // every wave has read R_h
+                // (X stays in its accumulation registers up to here: without this the copies that the rounding
+                // below reads are made right after the update and occupy registers through both products)
+                asm volatile("" : "+a"(xs[0]), "+a"(xs[1]));
+                walk_state_to_lds<T, D, B>(tl, wave, lane, xs);
+                sync();  // X_h is in LDS
+                walk_product<T, D, false, 0, B::KV, NQ>(tg, tv, tk, wave, lane, c > 0, cols_of_state, acc);
+                walk_store<T, D, OQ::PER>(HF ? rdq1 : rdq0, dqs2, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc);
+            }
             if constexpr (HF != 0) walk_store<T, D, OV::PER>(rdv, dvs2, p.wv, row, g, OV::db0(wave), dvacc);
             walk_update<T, D, B, false, true>(tq, tg, wave, lane, st);  // R_h += Q_h^T dO
-            sync();  // every wave has read X_h and is done with this half's tiles
+            sync();  // every wave has read the state's copy and is done with this half's tiles
             walk_state_to_lds<T, D, B>(tl, wave, lane, st_next);
         };
         half_chunk(std::integral_constant<int, 0>{}, st0, xs0, st1);
@@ -2343,7 +2336,7 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     if (p.init_is_totals && (D != 128 || p.n_seg < 3 || !p.init)) return hipErrorInvalidValue;
     if (p.entry_out && (!p.init_is_totals || fm || p.denom || p.dn)) return hipErrorInvalidValue;
     if (p.denom || p.dn) {  // the normaliser's terms: its vectors live behind the state
-        if ((p.dn && !p.zc) || (p.denom && p.n_seg > 1 && !p.vsum) || p.accumulate) return hipErrorInvalidValue;
+        if ((p.dn && !p.zc) || (p.denom && p.n_seg > 1 && !p.vsum)) return hipErrorInvalidValue;
         constexpr int smem_n = smem + (kDouble ? 2 : 1) * WalkCfg<D>::VEC;
         if (p.denom)
             return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 1, true>>(grid, smem_n, p, stream)
@@ -2351,19 +2344,14 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
         return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, true>>(grid, smem_n, p, stream)
                   : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, false>>(grid, smem_n, p, stream);
     }
-    if (fm) return p.accumulate ? hipErrorNotSupported : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true>>(grid, smem, p, stream);
+    if (fm) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true>>(grid, smem, p, stream);
     if constexpr (D == 128) {
-        // operands of at most 64 true columns on one side (the halves of a wide q / k against a narrow v):
-        // the kernels that leave out the blocks of padding
-        if (p.wqk > 64 && p.wv <= 64)
-            return p.accumulate ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2, true>>(grid, smem, p, stream)
-                                : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2>>(grid, smem, p, stream);
-        if (p.wqk <= 64 && p.wv > 64)
-            return p.accumulate ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4, true>>(grid, smem, p, stream)
-                                : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4>>(grid, smem, p, stream);
-        if (p.accumulate) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 4, true>>(grid, smem, p, stream);
+        // operands of at most 64 true columns on a side (the halves of a wide q / k, a narrow v): the kernels that
+        // leave out the blocks of padding, which the states in memory may not hold either
+        if (p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2>>(grid, smem, p, stream);
+        if (p.wqk <= 64 && p.wv > 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4>>(grid, smem, p, stream);
+        if (p.wqk <= 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 2>>(grid, smem, p, stream);
     }
-    if (p.accumulate) return hipErrorNotSupported;
     return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false>>(grid, smem, p, stream);
 }
 
@@ -2434,26 +2422,20 @@ hipError_t launch_walk_bwd_rev(const WalkParams &p, hipStream_t stream) {
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     if (!p.xtotal || (p.n_seg > 1 && !p.xinit)) return hipErrorInvalidValue;
-    if (p.entry_out || (p.init_is_totals && (p.n_seg < 3 || !p.init))) return hipErrorInvalidValue;
+    if (p.entry_out || (p.accumulate && !p.quad) || (p.init_is_totals && (p.n_seg < 3 || !p.init))) return hipErrorInvalidValue;
     constexpr int smem = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     static_assert(smem <= 160 * 1024, "two sets of tiles and the state must fit the LDS of a CU");
     if (p.quad) {
         if ((p.quad != 2 && p.quad != 3) || p.wqk != 128 || p.wv != 128 || p.wqk2 < 1 || p.wqk2 > 128 || p.wv2 < 1 ||
-            p.wv2 > 128 || p.fmap || p.accumulate == 1)
+            p.wv2 > 128 || p.fmap)
             return hipErrorInvalidValue;
-        return p.accumulate ? launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, 2>>(grid, smem, p, stream, 2)
+        return p.accumulate ? launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, true>>(grid, smem, p, stream, 2)
                             : launch_walk_kernel<walk_bwd_rev_kernel<T, D>>(grid, smem, p, stream, 2);
     }
     if constexpr (D == 128) {  // a half of a wide q / k against a narrow v: without the blocks of padding
-        if (!p.fmap && p.wqk > 64 && p.wv <= 64)
-            return p.accumulate ? launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2, 1>>(grid, smem, p, stream)
-                                : launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2>>(grid, smem, p, stream);
+        if (!p.fmap && p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2>>(grid, smem, p, stream);
     }
-    if (p.fmap) {
-        if (p.accumulate) return hipErrorNotSupported;
-        return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, 0, true>>(grid, smem, p, stream);
-    }
-    if (p.accumulate) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, 1>>(grid, smem, p, stream);
+    if (p.fmap) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, false, true>>(grid, smem, p, stream);
     return launch_walk_kernel<walk_bwd_rev_kernel<T, D>>(grid, smem, p, stream);
 }
 
@@ -2462,14 +2444,18 @@ hipError_t launch_walk_bwd_rev_wide(const WalkParams &p, hipStream_t stream) {
     using W = WalkCfg<128>;
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
-    if (p.wqk != 128 || p.wqk2 < 1 || p.wqk2 > 128 || p.wv < 1 || p.wv > 64) return hipErrorNotSupported;
-    if (p.fmap || p.dn || p.accumulate || p.init_transposed || !p.xtotal || !p.xtotal2 || p.entry_out || p.entry_out2 ||
-        (p.n_seg > 1 && (!p.init || !p.init2 || !p.xinit || !p.xinit2)) || (p.init_is_totals && p.n_seg < 3))
+    if (p.wqk != 128 || p.wqk2 < 1 || p.wqk2 > 128 || p.wv < 1 || p.wv > (p.dq ? 64 : 128)) return hipErrorNotSupported;
+    if (p.fmap || p.dn || p.accumulate || p.init_transposed || p.entry_out || p.entry_out2 ||
+        (p.n_seg > 1 && (!p.init || !p.init2)) || (p.init_is_totals && p.n_seg < 3))
         return hipErrorInvalidValue;
     constexpr int smem = 8 * W::TILE + W::STATE;  // two sets of (Q_h, K_h), two of (V, dO), one state
     static_assert(smem <= 160 * 1024, "the tiles and the state must fit the LDS of a CU");
-    return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2>>(grid, smem, p, stream);
+    if (p.dq) {
+        if (!p.xtotal || !p.xtotal2 || (p.n_seg > 1 && (!p.xinit || !p.xinit2))) return hipErrorInvalidValue;
+        return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, true>>(grid, smem, p, stream);
+    }
+    return p.wv <= 64 ? launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, false>>(grid, smem, p, stream)
+                      : launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 4, false>>(grid, smem, p, stream);
 }
-
 
 }  // namespace fla

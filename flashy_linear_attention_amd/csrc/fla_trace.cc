@@ -20,7 +20,9 @@ const char *fla_trace_symbol(const void *kernel, const char *fallback) {
     if (!dladdr(kernel, &info) || !info.dli_sname) return fallback;
     int status = 0;
     char *text = abi::__cxa_demangle(info.dli_sname, nullptr, nullptr, &status);
-    return status == 0 && text ? text : strdup(info.dli_sname);  // (kept for the life of the process)
+    // (libstdc++ takes __bf16, DF16b, for a fixed-point "_Accum" where the arguments behind it happen to fit)
+    const bool read = status == 0 && text && !strstr(text, "_Accum");
+    return read ? text : strdup(info.dli_sname);  // (kept for the life of the process)
 }
 
 void fla_trace_append(const char *line) {

@@ -1,0 +1,48 @@
+"""The error against fp64 of the evaluation chosen by shape is that of the quadratic kernels (``-m gpu``)."""
+
+import pytest
+import torch
+
+from flashy_linear_attention_amd import LinearAttention, LinearAttentionSmallVHD
+from flashy_linear_attention_amd import kernels
+
+pytestmark = pytest.mark.gpu
+
+# Both round one factor of every product to bf16 (the scores; within a chunk the scores, beyond it the running state), sum in
+# fp32 and round the result, so the errors are alike: at worst the state's rounding is averaged over D terms where the
+# scores' are averaged over N, 1 + 1 / D of the squared error for data of one sign (1.016 at D = 32).  The rest of the 3 %
+# is the sampling of the two norms.
+NO_LARGER = 1.03
+
+
+def _exact(q, k, v, do):
+    q, k, v, do = (t.double() for t in (q, k, v, do))
+    a, m = (torch.matmul(x, y.transpose(-2, -1).contiguous()).tril() for x, y in ((q, k), (do, v)))
+    return (torch.matmul(a, v), torch.matmul(m, k), torch.matmul(m.transpose(-2, -1).contiguous(), q),
+            torch.matmul(a.transpose(-2, -1).contiguous(), do))
+
+
+def _compare(chosen, other, want):
+    for name, got, ref, w in zip(("O", "dQ", "dK", "dV"), chosen, other, want):
+        err, bound = (float(torch.linalg.norm(t.double() - w) / torch.linalg.norm(w)) for t in (got, ref))
+        assert err <= NO_LARGER * bound, f"{name}: {err:.3e} against {bound:.3e}"
+
+
+@pytest.mark.parametrize("positive", [False, True], ids=["signed", "positive"])
+@pytest.mark.parametrize("h,n,dqk,dv", [
+    (4, 2048, 64, 64), (4, 4096, 32, 32), (4, 2048, 128, 128), (4, 2048, 128, 64), (4, 2048, 256, 64), (4, 2048, 256, 128),
+    (4, 2048, 192, 128), (4, 2048, 153, 64), (4, 2048, 136, 128),
+])
+def test_no_larger_than_the_quadratic_kernels(h, n, dqk, dv, positive, gpu_device):
+    gen = torch.Generator().manual_seed(dqk + dv)
+    q, k, v, do = (torch.randn(1, h, n, d, generator=gen) for d in (dqk, dqk, dv, dv))
+    q, k, v, do = ((t.abs() if positive else t).bfloat16().to(gpu_device) for t in (q, k, v, do))
+    args = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    out = (LinearAttention if dqk == dv else LinearAttentionSmallVHD).apply(*args)
+    chosen = (out.detach(), *torch.autograd.grad(out, args, do))
+    if dqk == dv:
+        other = (kernels.linear_flash_wrapper_fwd(q, k, v), *kernels.linear_flash_wrapper_bwd(do, q, k, v))
+    else:
+        other = (kernels.linear_flash_wrapper_fwd_smallv_hd(q, k, v), *kernels.linear_flash_wrapper_bwd_smallv_hd(do, q, k, v))
+    assert any(not torch.equal(a, b) for a, b in zip(chosen, other))  # (chunk-wise, at these sizes)
+    _compare(chosen, other, _exact(q, k, v, do))
