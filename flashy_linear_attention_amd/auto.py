@@ -66,7 +66,8 @@ def evaluate_bwd(ctx: Any, grad_output: torch.Tensor) -> Tuple[torch.Tensor, tor
     else:
         (q, k, v), state = ctx.saved_tensors, None
     if ctx.chunked:
-        return linear_attention_chunked_bwd(grad_output, q, k, v, state)
+        # (what later rows hold must not reach dQ, as in the quadratic evaluation)
+        return linear_attention_chunked_bwd(grad_output, q, k, v, state, causal=True)
     if ctx.equal:
         return linear_flash_wrapper_bwd(grad_output, q, k, v)
     return linear_flash_wrapper_bwd_smallv_hd(grad_output, q, k, v)

@@ -5,7 +5,9 @@ the quadratic kernels, flashlinear/kernels/linear_attn_kernels.py:63,166-171).
 gradients as ``LinearAttention`` / ``LinearAttentionSmallVHD``, but through per-chunk KV states
 (``fla_tri_xyt_z_chunked``): O(N) instead of O(N^2) work, meant for long sequences.  Results
 agree with the quadratic path up to rounding (the running state is rounded once to the storage
-dtype before it multiplies the queries).
+dtype before it multiplies the queries).  Head dims above 64: dQ's state is taken backwards from
+the end of a segment, by subtraction, so infinite, NaN or far larger late rows of k and v spoil the
+dQ of rows before them; ``LinearAttentionAuto`` and the two reference-named operators do not.
 """
 
 from __future__ import annotations
@@ -76,9 +78,11 @@ def linear_attention_chunked_fwd(
 
 
 def linear_attention_chunked_bwd(
-    grad_output: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor = None
+    grad_output: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, state: torch.Tensor = None,
+    causal: bool = False,
 ) -> Tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
-    """(dQ, dK, dV) chunk-wise; ``state`` is what the forward call returned (or None)."""
+    """(dQ, dK, dV) chunk-wise; ``state`` is what the forward call returned (or None).  ``causal``: no dQ from a state
+    that later rows are part of (``fla_linear_attn_chunked_bwd_causal``)."""
     grad_output, q, k, v = prepare(grad_output, q, k, v)
     b, h, n, dqk = q.shape
     dv = v.shape[-1]
@@ -91,9 +95,10 @@ def linear_attention_chunked_bwd(
             assert state.numel() == _lib.query("fla_linear_attn_chunked_state_bytes", b, h, n, dqk, dv), "state of another shape"
         wbytes = _lib.query("fla_linear_attn_chunked_workspace_bytes", b, h, n, dqk, dv)
         work = torch.empty(max(wbytes, 16), dtype=torch.uint8, device=q.device)
+        name = "fla_linear_attn_chunked_bwd_causal" if causal else "fla_linear_attn_chunked_bwd"
         _lib.check(
-            "fla_linear_attn_chunked_bwd",
-            lib.fla_linear_attn_chunked_bwd(
+            name,
+            getattr(lib, name)(
                 grad_output.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(),
                 dq.data_ptr(), dk.data_ptr(), dvv.data_ptr(), b, h, n, dqk, dv,
                 _lib.strides_arg(grad_output), _lib.strides_arg(q), _lib.strides_arg(k), _lib.strides_arg(v),

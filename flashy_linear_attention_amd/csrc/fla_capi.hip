@@ -733,15 +733,15 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
 }
 
 // With forward's states at hand and a narrow v: one reverse walk over both halves, dQ included, whose state goes
-// backwards by subtraction from the state at the segment's end (walk_bwd_rev_wide_kernel).  A wider v or no states: dQ_h
-// by forward-direction walks.  Backward at B 4, H 16, N 4096, 256 / 128: 297 us as a reverse walk per half, the second
-// adding to the first one's dV in memory, 279 us this way.
+// backwards by subtraction from the state at the segment's end (walk_bwd_rev_wide_kernel).  `causal`, a wider v or no states:
+// dQ_h by forward-direction walks.  Backward at B 4, H 16, N 4096: 256 / 64 176 us in one walk, 199 in three; 256 / 128 297 us
+// as a reverse walk per half, the second adding to the first one's dV in memory, 279 us in three walks.
 int wide_backward(const WidePlan &wide, const View &go, const View &q, const View &k, const View &v, const View &dq,
                   const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
-                  const void *state_in, void *workspace, hipStream_t s) {
+                  const void *state_in, void *workspace, hipStream_t s, bool causal) {
     const WalkPlan &wp = wide.wp;
     char *ws = static_cast<char *>(workspace);
-    const bool one_walk = state_in && dv <= 64;
+    const bool one_walk = state_in && dv <= 64 && !causal;
     // entry states of both halves up front: Q_h^T dO over the segments after, and -- when forward's are not
     // at hand -- K_h^T V over the segments before
     const float *fwd_entries[2] = {nullptr, nullptr}, *entries[2] = {nullptr, nullptr};
@@ -874,7 +874,8 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
                     int64_t workspace_bytes, void *stream, int fmap, const View *mapped, bool *mapped_done, WalkNorm *nx);
 int chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
-                     const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap, WalkNorm *nx);
+                     const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap, WalkNorm *nx,
+                     bool causal);
 
 // fmap != 0 (feature_forward below): q and k hold the arguments xq, xk of the feature map phi, and
 // `mapped` = {phi(xq), phi(xk)} are outputs: the state kernel maps xk as it loads it and writes
@@ -1009,10 +1010,14 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
     return FLA_OK;
 }
 
+// `causal` (D_v up to 128): with forward's states at hand, too, dQ comes from a walk in forward direction (and dK, dV from
+// one in reverse), never by subtraction from a later state: nothing of a row reaches the dQ of the chunks before it.
+// Backward at D = 128, one reverse walk against two walks: B H 128, N 4096 274 / 292 us; B H 16, N 4096 53 / 58; B H 256, N 1024
+// 124 / 128; B H 4, N 8192 66 / 73; 128 / 64, B H 64, N 4096 98 / 113.
 int chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                      const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap = 0,
-                     WalkNorm *nx = nullptr) {
+                     WalkNorm *nx = nullptr, bool causal = false) {
     if (nx) nx->fused = nx->dk_pending = false;
     const View all[] = {go, q, k, v, dq, dk, dvv};
     for (const View &t : all)
@@ -1044,7 +1049,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                 const void *st = state_in ? static_cast<const char *>(state_in) + j * vs.state0 : nullptr;
                 if (int rc = chunked_backward(v_half(go, j), q, k, v_half(v, j), j == 0 ? dq : tq, j == 0 ? dk : tk,
                                               v_half(dvv, j), B, H, N, dqk, j == 0 ? 128 : vs.dv1, dtype, st, workspace, inner,
-                                              stream, 0, nullptr))
+                                              stream, 0, nullptr, causal))
                     return rc;
             }
             if (int rc = launch_feature_pass(3, 0, tq, dq, B, H, N, dqk, dtype, stream)) return rc;
@@ -1056,7 +1061,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                 return FLA_ERR_WORKSPACE;
             if (state_in && reinterpret_cast<uintptr_t>(state_in) % 16 != 0) return FLA_ERR_WORKSPACE;
             return wide_backward(wide, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace,
-                                 static_cast<hipStream_t>(stream));
+                                 static_cast<hipStream_t>(stream), causal);
         }
     }
     // (with the normaliser's terms still to be added by the caller, so is the slope)
@@ -1091,9 +1096,9 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         hipStream_t s = static_cast<hipStream_t>(stream);
         const float *entry = nullptr;
         // with forward's states at hand (and without the normaliser): one reverse walk
-        const bool one_walk = state_in && !nx;
+        const bool one_walk = state_in && !nx && !causal;
         // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
-        const bool rev_sums_on_load = one_walk && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
+        const bool rev_sums_on_load = (one_walk || causal) && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
         if (wp.n_seg > 1) {
             if (!state_in) {
                 const float *fwd_entry = nullptr;
@@ -1151,6 +1156,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         r.H = (int32_t)H, r.N = (int32_t)N, r.BH = (int32_t)(B * H), r.wqk = (int32_t)dqk, r.wv = (int32_t)dv;
         r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
         r.init = entry, r.fmap = fmap;  // (dK: the slope from phi(xk) in the K tile)
+        r.init_is_totals = rev_sums_on_load;
         if (nx) r.dn = nx->dn, r.rc = rcv;  // dK's terms
         return fla::walk_dkdv(dtype, wp.D, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
@@ -1293,7 +1299,7 @@ int packed_forward(const PackPlan &p, const View &q, const View &k, const View &
 
 int packed_backward(const PackPlan &p, const View &go, const View &q, const View &k, const View &v, const View &dq,
                     const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
-                    const void *state_in, void *workspace, int64_t workspace_bytes, void *stream) {
+                    const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, bool causal) {
     const View all[] = {go, q, k, v, dq, dk, dvv};
     for (const View &t : all)
         if (int rc = check_view(t)) return rc;
@@ -1321,9 +1327,22 @@ int packed_backward(const PackPlan &p, const View &go, const View &q, const View
     }
     if (int rc = in.launch(stream)) return rc;
     if (int rc = chunked_backward(gop, qp, kp, vp, dqp, dkp, dvp, B, H, N, p.wq, p.wv, dtype, state_in, workspace, p.inner_work,
-                                  stream, 0, nullptr))
+                                  stream, 0, nullptr, causal))
         return rc;
     return out.launch(stream);
+}
+
+int plain_chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
+                           const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
+                           const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, bool causal) {
+    if (int rc = check_common(B, H, N, dtype)) return rc;
+    if (dqk < 1 || dqk > 256) return FLA_ERR_HEAD_DIM;
+    if (dv < 1 || dv > 256) return FLA_ERR_V_HEAD_DIM;
+    if (const PackPlan p = pack_plan(B, H, N, dqk, dv); p.ok)
+        return packed_backward(p, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace, workspace_bytes,
+                               stream, causal);
+    return chunked_backward(go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace, workspace_bytes, stream, 0,
+                            nullptr, causal);
 }
 
 // O = tril(phi(xq) phi(xk)^T) v with mapped = {phi(xq), phi(xk)} as further outputs.  Chunk-wise
@@ -2131,16 +2150,20 @@ int fla_linear_attn_chunked_bwd(const void *grad_out, const void *q, const void 
                                 const int64_t *v_strides, const int64_t *dq_strides, const int64_t *dk_strides,
                                 const int64_t *dv_strides, int dtype, const void *state_in, void *workspace,
                                 int64_t workspace_bytes, void *stream) {
-    if (int rc = check_common(B, H, N, dtype)) return rc;
-    if (D_qk < 1 || D_qk > 256) return FLA_ERR_HEAD_DIM;
-    if (D_v < 1 || D_v > 256) return FLA_ERR_V_HEAD_DIM;
-    if (const PackPlan p = pack_plan(B, H, N, D_qk, D_v); p.ok)
-        return packed_backward(p, {grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides}, {dq, dq_strides},
-                               {dk, dk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v, dtype, state_in, workspace,
-                               workspace_bytes, stream);
-    return chunked_backward({grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides}, {dq, dq_strides},
-                            {dk, dk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v, dtype, state_in, workspace,
-                            workspace_bytes, stream);
+    return plain_chunked_backward({grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides}, {dq, dq_strides},
+                                  {dk, dk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v, dtype, state_in, workspace,
+                                  workspace_bytes, stream, false);
+}
+
+int fla_linear_attn_chunked_bwd_causal(const void *grad_out, const void *q, const void *k, const void *v, void *dq, void *dk,
+                                       void *dv, int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v,
+                                       const int64_t *go_strides, const int64_t *q_strides, const int64_t *k_strides,
+                                       const int64_t *v_strides, const int64_t *dq_strides, const int64_t *dk_strides,
+                                       const int64_t *dv_strides, int dtype, const void *state_in, void *workspace,
+                                       int64_t workspace_bytes, void *stream) {
+    return plain_chunked_backward({grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides}, {dq, dq_strides},
+                                  {dk, dk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v, dtype, state_in, workspace,
+                                  workspace_bytes, stream, true);
 }
 
 int fla_feature_attn_normalised_fwd(const void *xq, const void *xk, const void *v, void *o, void *q_out, void *k_out,

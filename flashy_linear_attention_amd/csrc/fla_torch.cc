@@ -143,7 +143,8 @@ bool wants_grad(const Tensor &q, const Tensor &k, const Tensor &v) {
 
 // ---- tril(Q K^T) V
 
-enum Evaluation { kEqual = 0, kSmallV = 1, kChunked = 2 };
+// (kChosen: chunk-wise because the shape says so, with the quadratic evaluation's causality of dQ)
+enum Evaluation { kEqual = 0, kSmallV = 1, kChunked = 2, kChosen = 3 };
 
 std::tuple<Tensor, Tensor> product_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, int ev, bool want_state) {
     at::AutoDispatchBelowADInplaceOrView below;
@@ -180,9 +181,9 @@ variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_,
                                         str(go), str(q), str(k), str(v), str(dq), str(dk), str(dv), c.dtype, c.stream));
     } else {
         const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        must(fla_linear_attn_chunked_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
-                                         str(go), str(q), str(k), str(v), str(dq), str(dk), str(dv), c.dtype, ptr(state),
-                                         ptr(work), size_of(work), c.stream));
+        must((ev == kChosen ? fla_linear_attn_chunked_bwd_causal : fla_linear_attn_chunked_bwd)(
+            ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go), str(q), str(k),
+            str(v), str(dq), str(dk), str(dv), c.dtype, ptr(state), ptr(work), size_of(work), c.stream));
     }
     return {dq, dk, dv};
 }
@@ -453,12 +454,12 @@ PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
     int ev = equal ? kEqual : kSmallV;
     if (kind == 0) {  // (the shapes its forward takes, and its choice: linear_attn.py)
         if (!equal || rows % (dqk > 128 ? 32 : 64) != 0) Py_RETURN_NONE;
-        if (range && dqk <= 128 && prefers()) ev = kChunked;
+        if (range && dqk <= 128 && prefers()) ev = kChosen;
     } else if (kind == 1) {  // (linear_attn_smallv_hd.py)
         if (!pow2(dv) || dv > next_pow2(dqk) || rows % 64 != 0) Py_RETURN_NONE;
-        ev = range && dv <= 128 && prefers() ? kChunked : kSmallV;
+        ev = range && dv <= 128 && prefers() ? kChosen : kSmallV;
     } else if (kind == 2) {  // (auto.py)
-        if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || (range && prefers())) ev = kChunked;
+        if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || (range && prefers())) ev = kChosen;
     } else {
         ev = kChunked;
     }

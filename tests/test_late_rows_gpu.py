@@ -23,6 +23,12 @@ def _step(op, q, k, v, do):
 @pytest.mark.parametrize("op,b,h,n,dqk,dv", [
     ("linear", 4, 160, 512, 64, 64), ("linear", 4, 64, 1024, 64, 64), ("linear", 1, 16, 8192, 32, 32), ("linear", 1, 4, 16384, 64, 64),
     ("smallv", 1, 48, 1024, 64, 32), ("auto", 1, 30, 2200, 40, 40), ("auto", 2, 2, 2500, 36, 36),
+    # D = 128: one, two, several and many segments; unequal widths; copies with aligned rows
+    ("linear", 8, 40, 512, 128, 128), ("linear", 4, 32, 2048, 128, 128), ("linear", 1, 32, 4096, 96, 96), ("linear", 1, 4, 8192, 128, 128),
+    ("smallv", 2, 16, 2048, 128, 64), ("auto", 2, 10, 1500, 72, 72), ("auto", 1, 6, 2100, 100, 100), ("smallv", 1, 12, 1024, 91, 64),
+    # q and k of more than 128 columns
+    ("smallv", 4, 64, 512, 256, 64), ("smallv", 4, 16, 2048, 256, 64), ("smallv", 1, 8, 2048, 160, 32), ("smallv", 1, 20, 2048, 192, 128),
+    ("smallv", 2, 3, 4096, 136, 128), ("smallv", 1, 16, 2048, 153, 64),
 ])
 def test_late_rows_do_not_reach_earlier_ones(op, b, h, n, dqk, dv, late, gpu_device):
     gen = torch.Generator().manual_seed(n + dqk + dv)
