@@ -12,22 +12,25 @@
 //   dk_j  = ((M f'(u))^T of the chunk) q + the gradient of phi_w(k) (U [v_j, 1]) at k_j
 //
 // (g = dO / n, dn_i = -(dO_i . O_i) / n_i formed here from dO, O and n; without the normaliser g = dO and no dn).
-// Nothing of width F goes to memory but the states at the ends of a walk's segments: feature rows are
-// formed from the 16-wide rows, the ones that are MFMA operands along the row in registers, the ones whose
-// contraction runs down the rows as an LDS tile.
+// Nothing of width F goes to memory but the states at the ends of a walk's segments, and no feature row to LDS: MFMA
+// operands of features are formed in registers, along the row from a row of the x tile (phi_w) and down the rows
+// from two rows of its transposed copy (the state's update).  Feature values stay what fp32 gives, as two bf16 numbers
+// each (poly_split8), and what is rounded to bf16 is what the quadratic evaluation rounds -- the scores of the chunk -- and
+// the running sums once per chunk: errors against fp64 0.87 to 1.01 times the quadratic kernels', the normaliser's 1e-7.
 //
-// What bounds it: the matrix instructions and the multiplications and roundings that form feature rows (one fragment
-// of eight features costs twelve VALU instructions and serves one or two MFMAs); HBM is far away (40 KiB per
-// 128-row chunk).  Hence eight waves, two per SIMD, so that one wave's VALU work runs under the other's MFMAs: wave w owns
+// What bounds it: the matrix instructions and the VALU work that forms features together (an update's fragment of eight
+// features costs about 50 VALU instructions and serves four MFMAs, one along the row 28 and four); HBM is far away
+// (40 KiB per 128-row chunk).  Hence eight waves, two per SIMD, so that one wave's VALU work runs under the other's MFMAs: wave w owns
 // rows 32 (w % 4) .. of the chunk, and of their work one half: half of the features and of the score blocks (forward),
 // dq and the rows after the chunk in dV against dk and the chunk's own rows in dV (backward); the two waves of a row
 // block exchange one half of the sums through LDS.  (Halves of the output columns instead formed every feature row and
-// every score twice: VALU instructions were 63 % of the forward walk's time.)  A workgroup takes a CU's LDS; the next chunk's rows are fetched into registers a chunk ahead.  The split
-// into segments and the forms of their entry states are the walk kernels' (fla_chunk_walk.h), and as there the backward
+// every score twice.)  Of a state a wave owns one of the seven blocks of 32 features, over all value columns, so that every feature is
+// formed once.  A workgroup has a CU to itself; the next chunk's rows are fetched into registers a chunk ahead.  The split
+// into segments and the forms of their entry states are the walk kernels' (fla_chunk_walk.h); the backward
 // walk gets T going backwards, by subtracting every chunk's sums from the state at its segment's end.
-// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 200 us this way (kernels
-// 21 totals, 58 forward, 28 totals, 125 backward; the VALU issues on half of the forward walk's cycles, the matrix
-// unit is busy on a third).
+// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 228 us this way.  (With
+// feature rows rounded to one bf16 number on both sides, from tiles of them in LDS: 200 us, and errors 1.2 times the
+// quadratic kernels'.)
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -63,19 +66,18 @@ struct PolyFeatures {
 };
 
 struct PolyLds {  // byte offsets
-    // dn of a chunk: in fp32, rounded, and 256 bytes of zeros
-    static constexpr int DN = 128 * 4 + 256 + 256;
-    static constexpr int C = 128, XT = C * 32, VT = C * 128, PHI = C * 256, ST = 2 * 64 * 256, XTR = 16 * 272, EX = 8 * 4096;
-    // totals: the x tile, the v tile, two feature tiles, dn
-    static constexpr int tX = 0, tV = tX + XT, tPhi = tV + VT, tDn = tPhi + 2 * PHI, tTotal = tDn + DN;
+    // XTR: an x tile transposed (rows of 272 bytes: the sixteen columns, a one per row of the sequence, zeros)
+    static constexpr int C = 128, XT = C * 32, VT = C * 128, ST = 2 * 64 * 256, XTR = 18 * 272, EX = 8 * 4096;
+    static constexpr int Z = PolyFeatures::kF * 4, DN = C * 4;
+    // totals: the x tile transposed, the v tile, dn
+    static constexpr int tX = 0, tV = tX + XTR, tDn = tV + VT, tTotal = tDn + DN;
     // forward
-    static constexpr int fQ = 0, fK = fQ + XT, fV = fK + XT, fS = fV + VT, fPhi = fS + ST, fZ = fPhi + 2 * PHI,
-                         fSum = fZ + PolyFeatures::kF * 4, fEx = fSum + 2 * C * 4, fTotal = fEx + EX;
-    // backward (the second feature tile and T's copy share their place)
+    static constexpr int fQ = 0, fK = fQ + XT, fKt = fK + XT, fV = fKt + XTR, fS = fV + VT, fEx = fS + ST, fZ = fEx + EX,
+                         fSum = fZ + Z, fTotal = fSum + 2 * C * 4;
+    // backward
     static constexpr int bQ = 0, bK = bQ + XT, bQt = bK + XT, bKt = bQt + XTR, bV = bKt + XTR, bG = bV + VT, bU = bG + VT,
-                         bPhi = bU + ST, bT = bPhi + PHI, bZ = bT + PHI, bY = bZ + PolyFeatures::kF * 4,
-                         bDn = bY + PolyFeatures::kF * 4, bTotal = bDn + DN;
-    static_assert(PHI == ST && EX == ST && fTotal <= 160 * 1024 && bTotal <= 160 * 1024, "a CU's LDS");
+                         bT = bU + ST, bZ = bT + ST, bY = bZ + Z, bDn = bY + Z, bTotal = bDn + DN;
+    static_assert(EX == ST && XTR % 16 == 0 && fTotal <= 160 * 1024 && bTotal <= 160 * 1024, "a CU's LDS");
 };
 
 // (a select of two values: written between two elements of an array it would become one load with a computed index, and
@@ -125,13 +127,13 @@ __device__ __forceinline__ typename Mma<T>::V8 poly_col_frag(const unsigned char
 struct PolyPair {
     uint32_t lo, hi;
 };
-// rows {4g .., 8 + 4g ..}, plain column mapping, column block cb
+// rows 8g .. 8g + 7, plain column mapping, column block 0 (block cb: XOR cb << 6)
 template <int RB>
-__device__ __forceinline__ PolyPair poly_col_base(int lane, int cb) {
+__device__ __forceinline__ PolyPair poly_col_base(int lane) {
     const int lam = lane & 15, g = lane >> 5, beta = (lane >> 4) & 1;
-    const int row = 4 * g + (lam >> 2), ch = 4 * cb + 2 * beta + ((lam & 3) >> 1), sub = 8 * (lam & 1);
+    const int row = 8 * g + (lam >> 2), ch = 2 * beta + ((lam & 3) >> 1), sub = 8 * (lam & 1);
     return {(uint32_t)(row * RB + ((ch ^ walk_swizzle<RB / 16>(row)) << 4) + sub),
-            (uint32_t)((row + 8) * RB + ((ch ^ walk_swizzle<RB / 16>(row + 8)) << 4) + sub)};
+            (uint32_t)((row + 4) * RB + ((ch ^ walk_swizzle<RB / 16>(row + 4)) << 4) + sub)};
 }
 // permuted column mapping, column block 0 (block cb: XOR cb << 6); CONS: rows 8g .. 8g + 7, else {4g .., 8 + 4g ..}
 template <int RB, bool CONS>
@@ -181,11 +183,41 @@ __device__ __forceinline__ void poly_round_masked(const float (&d)[16], uint32_t
     }
 }
 
+// Eight fp32 numbers as sums of two bf16 ones each: the upper half of the bits, and what is left, rounded (EXACT: of a
+// product of two bf16 numbers, whose sixteen significant bits both halves hold without rounding: the upper half as well)
+struct PolyTwo {
+    Mma<__bf16>::V8 hi, lo;
+};
+template <bool EXACT>
+__device__ __forceinline__ PolyTwo poly_split8(const float (&f)[8]) {
+    PolyTwo t;
+    u32x4 hi, lo;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        uint32_t bits[2];
+        float rest[2];
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+            bits[e] = __builtin_bit_cast(uint32_t, f[2 * k + e]);
+            rest[e] = f[2 * k + e] - __builtin_bit_cast(float, bits[e] & 0xffff0000u);
+        }
+        hi[k] = __builtin_amdgcn_perm(bits[1], bits[0], 0x07060302u);
+        if constexpr (EXACT) {
+            lo[k] = __builtin_amdgcn_perm(__builtin_bit_cast(uint32_t, rest[1]), __builtin_bit_cast(uint32_t, rest[0]), 0x07060302u);
+        } else {
+            typedef __bf16 t2 __attribute__((ext_vector_type(2)));
+            lo[k] = __builtin_bit_cast(uint32_t, t2{static_cast<__bf16>(rest[0]), static_cast<__bf16>(rest[1])});
+        }
+    }
+    t.hi = __builtin_bit_cast(Mma<__bf16>::V8, hi), t.lo = __builtin_bit_cast(Mma<__bf16>::V8, lo);
+    return t;
+}
+
 // Feature fragment KS (features 16 KS + 8 g ..) of a row, weighted for the phi_w side; `raw` receives it in fp32.
 // xs: the row's columns 8 g .. 8 g + 7.
-template <typename T, int KS>
-__device__ __forceinline__ typename Mma<T>::V8 poly_feature_frag(const float (&x)[16], const float (&xs)[8], int g, float c0,
-                                                                 float c1, float c2, float (&raw)[8]) {
+template <int KS>
+__device__ __forceinline__ PolyTwo poly_feature_frag(const float (&x)[16], const float (&xs)[8], int g, float c0, float c1,
+                                                     float c2, float (&raw)[8]) {
     if constexpr (KS < 4) {
         const float s = c2 * poly_pick(g, x[2 * KS + 1], x[2 * KS]);
 #pragma unroll
@@ -201,182 +233,130 @@ __device__ __forceinline__ typename Mma<T>::V8 poly_feature_frag(const float (&x
 #pragma unroll
         for (int j = 0; j < 8; ++j) raw[j] = j == 0 && g == 0 ? c0 : 0.f;
     }
-    return poly_round8<T>(raw);
+    return poly_split8<false>(raw);
 }
 
-// The feature rows of an x tile, written as two tiles of 128 features (the walk kernels' D = 128 tile layout, 128 rows):
-// groups 0 .. 15 to phi0, 16 .. 27 to phi1.  Thread t takes row t % 128, a quarter of the groups.  Rows past the
-// sequence are zeros, their one included.
-template <typename T>
-__device__ __forceinline__ void poly_gen_phi(const unsigned char *xt, unsigned char *phi0, unsigned char *phi1, int row0, int N,
-                                             int tid) {
-    const int row = tid & 127, part = __builtin_amdgcn_readfirstlane(tid >> 7);
-    float x[16];
-    poly_row<T>(xt, row, x);
-    auto put = [&](unsigned char *tile, int pos, typename Mma<T>::V8 v) {
-        *reinterpret_cast<u32x4 *>(tile + row * 256 + ((pos ^ walk_swizzle<16>(row)) << 4)) = __builtin_bit_cast(u32x4, v);
-    };
-    auto product = [&](int r, int h) {
-        float f[8];
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = x[r] * x[8 * h + j];
-        return poly_round8<T>(f);
-    };
-    // (The assembler comments keep the branches' last stores apart.  Merged into one behind the branches, the store had
-    // the address of the last branch computed on one of the two ways into it only: its zeros went over the x tile.)
-    if (part == 0) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) put(phi0, r, product(r, 0));
-        asm volatile("; groups 0 .. 7" ::: "memory");
-    } else if (part == 1) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) put(phi0, 8 + i, product(8 + i / 2, i % 2));
-        asm volatile("; groups 8 .. 15" ::: "memory");
-    } else if (part == 2) {
-#pragma unroll
-        for (int i = 0; i < 8; ++i) put(phi1, i, product(12 + i / 2, i % 2));
-        asm volatile("; groups 16 .. 23" ::: "memory");
-    } else {
-        float f[8];
-#pragma unroll
-        for (int h = 0; h < 2; ++h) {
-#pragma unroll
-            for (int j = 0; j < 8; ++j) f[j] = x[8 * h + j];
-            put(phi1, 8 + h, poly_round8<T>(f));
-        }
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = j == 0 && row0 + row < N ? 1.f : 0.f;
-        put(phi1, 10, poly_round8<T>(f));
-#pragma unroll
-        for (int j = 0; j < 8; ++j) f[j] = 0.f;
-        put(phi1, 11, poly_round8<T>(f));
-        asm volatile("; groups 24 .. 27" ::: "memory");
+// The two rows of a transposed x tile whose product is feature f, as byte offsets
+struct PolyFactors {
+    uint32_t a, b;
+};
+__device__ __forceinline__ PolyFactors poly_factors(int f) {
+    const int group = f >> 3, j = f & 7;
+    int a, b;
+    if (group < 24) {
+        a = group < 8 ? group : 4 + (group >> 1), b = group < 8 ? j : 8 * (group & 1) + j;
+    } else {  // the row itself; a one and zeros; zeros
+        a = group < 27 ? 16 : 17, b = group < 26 ? 8 * (group & 1) + j : group == 26 && j == 0 ? 16 : 17;
     }
+    return {(uint32_t)(a * 272), (uint32_t)(b * 272)};
 }
 
-// A state's blocks of this wave: columns 32 eb .., feature blocks p and p + 4 (p + 4 < 7), and -- NORM -- the column of
-// ones (of dn) for one of the two: lanes with l32 == 0 hold it.
+// A state's blocks of this wave: feature block `wave` (wave 7: none) over both 32-column blocks of the values, and -- NORM --
+// the column of ones (of dn): lane l32 of either half holds its part of feature 32 wave + l32.
 struct PolyState {
-    f32x16 st[2], ex;
-    int eb, p, fx;  // fx: the feature block of ex (7: none)
-    __device__ __forceinline__ void clear(int wave) {
-        eb = wave & 1, p = wave >> 1, fx = eb == 0 ? p : p + 4;
+    f32x16 st[2];
+    float ex;
+    int wave;
+    __device__ __forceinline__ void clear(int w) {
+        wave = w, ex = 0.f;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) st[0][v] = st[1][v] = ex[v] = 0.f;
+        for (int v = 0; v < 16; ++v) st[0][v] = st[1][v] = 0.f;
     }
-    __device__ __forceinline__ bool valid(int i) const { return p + 4 * i < PolyFeatures::kBlocks; }
+    __device__ __forceinline__ bool valid() const { return wave < PolyFeatures::kBlocks; }
     // += the state at `s` in memory
     template <bool NORM>
     __device__ __forceinline__ void add(const float *s, int l32, int g) {
+        if (!valid()) return;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            if (valid(i)) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    st[i][v] += s[(32 * (p + 4 * i) + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * eb + l32];
-            }
-        if (NORM && fx < PolyFeatures::kBlocks && l32 == 0) {
 #pragma unroll
             for (int v = 0; v < 16; ++v)
-                ex[v] += s[PolyFeatures::kF * PolyFeatures::kV + 32 * fx + 8 * (v / 4) + 4 * g + (v % 4)];
-        }
+                st[i][v] += s[(32 * wave + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * i + l32];
+        if (NORM && g == 0) ex += s[PolyFeatures::kF * PolyFeatures::kV + 32 * wave + l32];
     }
     template <bool NORM>
     __device__ __forceinline__ void store(float *s, int l32, int g) const {
+        if (!valid()) return;
 #pragma unroll
         for (int i = 0; i < 2; ++i)
-            if (valid(i)) {
-#pragma unroll
-                for (int v = 0; v < 16; ++v)
-                    s[(32 * (p + 4 * i) + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * eb + l32] = st[i][v];
-            }
-        if (NORM && fx < PolyFeatures::kBlocks && l32 == 0) {
 #pragma unroll
             for (int v = 0; v < 16; ++v)
-                s[PolyFeatures::kF * PolyFeatures::kV + 32 * fx + 8 * (v / 4) + 4 * g + (v % 4)] = ex[v];
+                s[(32 * wave + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * i + l32] = st[i][v];
+        if (NORM) {
+            const float t = ex + __shfl_xor(ex, 32, 64);
+            if (g == 0) s[PolyFeatures::kF * PolyFeatures::kV + 32 * wave + l32] = t;
         }
     }
     // rounded to the storage type as rows of value columns, features 0 .. 127 and 128 .. in two tiles; ex in fp32 to z
     template <typename T, bool NORM>
     __device__ __forceinline__ void to_lds(unsigned char *tile, float *z, int l32, int g) const {
         typedef T t4 __attribute__((ext_vector_type(4)));
-        const int row = 32 * eb + l32;
+        if (!valid()) return;
+        unsigned char *t = tile + (wave >> 2) * 64 * 256;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
-            if (valid(i)) {
-                unsigned char *t = tile + i * 64 * 256;  // (block p + 4 i: block p of tile i)
+        for (int i = 0; i < 2; ++i) {
+            const int row = 32 * i + l32;
 #pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    t4 w;
+            for (int a = 0; a < 4; ++a) {
+                t4 w;
 #pragma unroll
-                    for (int b = 0; b < 4; ++b) w[b] = static_cast<T>(st[i][4 * a + b]);
-                    *reinterpret_cast<t4 *>(t + row * 256 + (((4 * p + a) ^ walk_swizzle<16>(row)) << 4) + 8 * g) = w;
-                }
+                for (int b = 0; b < 4; ++b) w[b] = static_cast<T>(st[i][4 * a + b]);
+                *reinterpret_cast<t4 *>(t + row * 256 + (((4 * (wave & 3) + a) ^ walk_swizzle<16>(row)) << 4) + 8 * g) = w;
             }
-        if (NORM && fx < PolyFeatures::kBlocks && l32 == 0) {
-#pragma unroll
-            for (int a = 0; a < 4; ++a)
-                *reinterpret_cast<f32x4 *>(z + 32 * fx + 8 * a + 4 * g) = f32x4{ex[4 * a], ex[4 * a + 1], ex[4 * a + 2], ex[4 * a + 3]};
+        }
+        if (NORM) {
+            const float sum = ex + __shfl_xor(ex, 32, 64);
+            if (g == 0) z[32 * wave + l32] = sum;
         }
     }
-    // += (NEG: -=) phi^T [z tile, extra column] over the chunk's 128 rows.  extra: that column as 128 values of the storage
-    // type in LDS, 256 bytes of zeros behind them (null: ones) -- lanes other than l32 == 0 read the zeros, so that
-    // no VALU instruction is spent on the fragment.
+    // += (NEG: -=) phi^T [z tile, extra column] over the chunk's 128 rows.  Feature rows are formed here, as products of two
+    // rows of the transposed x tile: a lane's eight rows of one feature, exactly, in two bf16 numbers each.
+    // extra: the extra column, 128 floats in LDS (null: ones).
+    // (Rounded to one bf16 number, from a tile of feature rows, they and the weighted ones along the rows made the errors of
+    // O, dq, dk and dv 1.2 times the quadratic kernels', and those of the normaliser 1e-3 in place of 1e-7.)
     template <typename T, bool NORM, bool NEG>
-    __device__ __forceinline__ void update(const unsigned char *phi0, const unsigned char *phi1, const unsigned char *zt,
-                                           const unsigned char *extra, int lane) {
+    __device__ __forceinline__ void update(const unsigned char *xtr, const unsigned char *zt, const float *extra, int lane) {
         using M = Mma<T>;
         using V8 = typename M::V8;
+        if (!valid()) return;
         const int l32 = lane & 31, g = lane >> 5;
-        auto signed_frag = [&](V8 z) {
-            if constexpr (NEG) {
-                u32x4 raw = __builtin_bit_cast(u32x4, z);
+        const PolyFactors at = poly_factors(32 * wave + l32);
+        const unsigned char *fa = xtr + at.a + 16 * g, *fb = xtr + at.b + 16 * g;
+        const PolyPair za = poly_col_base<128>(lane);
+        auto step = [&](auto ksc) {
+            constexpr int ks = decltype(ksc)::value;
+            const V8 z0 = poly_tr<T>(zt + 16 * 128 * ks, za), z1 = poly_tr<T>(zt + 16 * 128 * ks, za, 1 << 6);
+            const u32x4 a = *reinterpret_cast<const u32x4 *>(fa + 32 * ks), b = *reinterpret_cast<const u32x4 *>(fb + 32 * ks);
+            float f[8];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) raw[e] ^= 0x80008000u;
-                z = __builtin_bit_cast(V8, raw);
+            for (int k = 0; k < 4; ++k) {
+                f[2 * k] = __builtin_bit_cast(float, a[k] << 16) * __builtin_bit_cast(float, b[k] << 16);
+                f[2 * k + 1] = __builtin_bit_cast(float, a[k] & 0xffff0000u) * __builtin_bit_cast(float, b[k] & 0xffff0000u);
             }
-            return z;
-        };
-        // (no branch in the loop: the wave whose second block does not exist multiplies block p of the first tile twice)
-        typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-        const unsigned char *column = extra + (l32 == 0 ? 0 : 256) + 8 * g;
-        float one[8];
+            if constexpr (NEG) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) one[j] = l32 == 0 ? (NEG ? -1.f : 1.f) : 0.f;
-        const V8 ones = poly_round8<T>(one);
-        const unsigned char *second = valid(1) ? phi1 : phi0;
-        const PolyPair za = poly_col_base<128>(lane, eb), ya = poly_col_base<256>(lane, p);
-        V8 zf = {}, y0 = {};
-        walk_pipe<8 * 3, 6, V8>(
-            [&](auto j) {
-                constexpr int ks = decltype(j)::value / 3, r = decltype(j)::value % 3;
-                if constexpr (r == 0)
-                    return signed_frag(poly_tr<T>(zt + 16 * 128 * ks, za));
-                else
-                    return poly_tr<T>((r == 1 ? phi0 : second) + 16 * 256 * ks, ya);
-            },
-            [&](auto j, V8 f) {
-                constexpr int ks = decltype(j)::value / 3, r = decltype(j)::value % 3;
-                if constexpr (r == 0) {
-                    zf = f;
-                } else if constexpr (r == 1) {
-                    y0 = f;
-                    st[0] = M::mma(f, zf, st[0]);
-                } else {
-                    st[1] = M::mma(f, zf, st[1]);
-                    if constexpr (NORM) {
-                        V8 ef = ones;
-                        if (extra) {
-                            const u32x2 lo = *reinterpret_cast<const u32x2 *>(column + 32 * ks);
-                            const u32x2 hi = *reinterpret_cast<const u32x2 *>(column + 32 * ks + 16);
-                            ef = signed_frag(__builtin_bit_cast(V8, u32x4{lo[0], lo[1], hi[0], hi[1]}));
-                        }
-                        const u32x4 a = __builtin_bit_cast(u32x4, y0), c = __builtin_bit_cast(u32x4, f);
-                        const u32x4 y = eb == 0 ? a : c;
-                        ex = M::mma(__builtin_bit_cast(V8, y), ef, ex);
+                for (int j = 0; j < 8; ++j) f[j] = -f[j];
+            }
+            if constexpr (NORM) {
+                if (extra) {
+#pragma unroll
+                    for (int h = 0; h < 2; ++h) {
+                        const f32x4 e = *reinterpret_cast<const f32x4 *>(extra + 16 * ks + 8 * g + 4 * h);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) ex += f[4 * h + j] * e[j];
                     }
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) ex += f[j];
                 }
-            });
+            }
+            const PolyTwo y = poly_split8<true>(f);
+            st[0] = M::mma(y.hi, z0, st[0]);
+            st[1] = M::mma(y.hi, z1, st[1]);
+            st[0] = M::mma(y.lo, z0, st[0]);
+            st[1] = M::mma(y.lo, z1, st[1]);
+        };
+        static_for<0, PolyLds::C / 16>(step);
     }
 };
 
@@ -420,6 +400,12 @@ __device__ __forceinline__ void poly_put_xt(unsigned char *xtr, u32x4 v, int tid
     for (int j = 0; j < 8; ++j)
         *reinterpret_cast<uint16_t *>(xtr + (8 * half + j) * 272 + row * 2) = (uint16_t)(v[j / 2] >> (16 * (j & 1)));
 }
+// ... its rows of ones (zeros past the sequence's last row) and of zeros, by the same threads
+template <typename T>
+__device__ __forceinline__ void poly_put_ones(unsigned char *xtr, int row0, int N, int tid) {
+    const int row = tid & 127, half = (tid >> 7) & 1;
+    *reinterpret_cast<T *>(xtr + (16 + half) * 272 + row * 2) = static_cast<T>(half == 0 && row0 + row < N ? 1.f : 0.f);
+}
 template <typename T>
 struct PolyTile {
     u32x4 v[2];
@@ -456,7 +442,6 @@ struct PolyGrad {
             }
         }
     }
-    // (dn: in fp32, and rounded behind that: PolyLds::DN)
     __device__ __forceinline__ void put(unsigned char *tile, float *dn, int tid) {
         using V8 = typename Mma<T>::V8;
         if constexpr (NORM) {
@@ -474,12 +459,8 @@ struct PolyGrad {
                 dot += __shfl_xor(dot, 1, 64);
                 dot += __shfl_xor(dot, 2, 64);
                 dot += __shfl_xor(dot, 4, 64);
-                if ((tid & 7) == 0) {
-                    // (one rounded value for every use, as the quadratic evaluation's bias column holds it)
-                    const T r = static_cast<T>(-dot * inv);
-                    dn[(tid + 512 * i) >> 3] = static_cast<float>(r);
-                    reinterpret_cast<T *>(dn + PolyLds::C)[(tid + 512 * i) >> 3] = r;
-                }
+                // (rounded once for every use, as the quadratic evaluation's bias column holds it)
+                if ((tid & 7) == 0) dn[(tid + 512 * i) >> 3] = static_cast<float>(static_cast<T>(-dot * inv));
             }
         }
         g.put(tile, tid);
@@ -545,22 +526,18 @@ __global__ __launch_bounds__(512, 2) void poly_totals_kernel(const PolyWalkParam
         else
             v.fetch(V, p.vs_n, row0, N, p.wv, tid);
     };
-    if (BWD && tid < 64) reinterpret_cast<uint32_t *>(smem + L::tDn + L::C * 6)[tid] = 0u;
     fetch(sl.c_lo);
 #pragma unroll 1
     for (int c = sl.c_lo; c < sl.c_hi; ++c) {
         __syncthreads();
-        if (tid < 256) poly_put_x(smem + L::tX, x, tid);
+        if (tid < 256) poly_put_xt(smem + L::tX, x, tid), poly_put_ones<T>(smem + L::tX, c * L::C, N, tid);
         if constexpr (BWD)
             go.put(smem + L::tV, dn, tid);
         else
             v.put(smem + L::tV, tid);
         if (c + 1 < sl.c_hi) fetch(c + 1);
         __syncthreads();
-        poly_gen_phi<T>(smem + L::tX, smem + L::tPhi, smem + L::tPhi + L::PHI, c * L::C, N, tid);
-        __syncthreads();
-        s.template update<T, NORM, false>(smem + L::tPhi, smem + L::tPhi + L::PHI, smem + L::tV,
-                                             BWD ? smem + L::tDn + L::C * 4 : nullptr, lane);
+        s.template update<T, NORM, false>(smem + L::tX, smem + L::tV, BWD ? dn : nullptr, lane);
     }
     s.template store<NORM>(p.totals + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, l32, g);
 #else
@@ -622,8 +599,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
     const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
     T *O = static_cast<T *>(p.out) + b * p.us_b + h * p.us_h;
     const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
-    unsigned char *tq = smem + L::fQ, *tk = smem + L::fK, *tv = smem + L::fV, *ts = smem + L::fS, *phi0 = smem + L::fPhi,
-                  *phi1 = phi0 + L::PHI;
+    unsigned char *tq = smem + L::fQ, *tk = smem + L::fK, *tkt = smem + L::fKt, *tv = smem + L::fV, *ts = smem + L::fS;
     float *z = reinterpret_cast<float *>(smem + L::fZ), *sums = reinterpret_cast<float *>(smem + L::fSum);
     unsigned char *exch = smem + L::fEx;
     PolyState s;
@@ -642,11 +618,11 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
         const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
         __syncthreads();
         poly_put_x(tid < 256 ? tq : tk, x, tid);
+        if (tid >= 256) poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
         v.put(tv, tid);
         s.template to_lds<T, NORM>(ts, z, l32, g);
         if (c + 1 < sl.c_hi) fetch(c + 1, tid);
         __syncthreads();
-        poly_gen_phi<T>(tk, phi0, phi1, c * L::C, N, tid);
 
         const int trow = 32 * rb + l32, row = c * L::C + trow;
         f32x16 acc[2];
@@ -662,10 +638,13 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
             auto step = [&](auto ksc) {
                 constexpr int KS = decltype(ksc)::value;
                 float raw[8];
-                const V8 f = poly_feature_frag<T, KS>(xr, xs, g, c0, c1, c2, raw);
+                const PolyTwo f = poly_feature_frag<KS>(xr, xs, g, c0, c1, c2, raw);
 #pragma unroll
-                for (int e = 0; e < 2; ++e)
-                    acc[e] = M::mma(poly_rd<T>(ts + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5)), f, acc[e]);
+                for (int e = 0; e < 2; ++e) {
+                    const V8 sf = poly_rd<T>(ts + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5));
+                    acc[e] = M::mma(sf, f.hi, acc[e]);
+                    acc[e] = M::mma(sf, f.lo, acc[e]);
+                }
                 if constexpr (NORM) {
 #pragma unroll
                     for (int a = 0; a < 2; ++a) {
@@ -676,13 +655,10 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
                 }
             };
             constexpr int H = PolyFeatures::kSteps / 2;
-            if (kh == 0) {
+            if (kh == 0)
                 static_for<0, H>(step);
-                asm volatile("; first half of the features");
-            } else {
+            else
                 static_for<H, 2 * H>(step);
-                asm volatile("; second half of the features");
-            }
         }
         const V8 xq = poly_row_frag<T>(tq, trow, g);
         const PolyPair va = poly_perm_base<128, false>(lane);
@@ -725,7 +701,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
             if (g == 0) sums[kh * L::C + trow] = rsum;
         }
         __syncthreads();
-        if (c + 1 < sl.c_hi || p.ends) s.template update<T, NORM, false>(phi0, phi1, tv, nullptr, lane);
+        if (c + 1 < sl.c_hi || p.ends) s.template update<T, NORM, false>(tkt, tv, nullptr, lane);
         f32x16 other;
         poly_get_acc(exch, wave ^ 4, lane, other);
         float f[16], inv = 1.f;
@@ -819,7 +795,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
     T *dV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
     const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
     unsigned char *tq = smem + L::bQ, *tk = smem + L::bK, *tqt = smem + L::bQt, *tkt = smem + L::bKt, *tv = smem + L::bV,
-                  *tg = smem + L::bG, *us = smem + L::bU, *phi0 = smem + L::bPhi, *ts = smem + L::bT;
+                  *tg = smem + L::bG, *us = smem + L::bU, *ts = smem + L::bT;
     float *z = reinterpret_cast<float *>(smem + L::bZ), *y = reinterpret_cast<float *>(smem + L::bY),
           *dn = reinterpret_cast<float *>(smem + L::bDn);
     PolyState st, su;
@@ -835,7 +811,6 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
         v.fetch(V, p.vs_n, row0, N, p.wv, tid);
         go.fetch(G, p.gs_n, O, p.os_n, den, row0, N, p.wv, tid);
     };
-    if (tid0 < 64) reinterpret_cast<uint32_t *>(smem + L::bDn + L::C * 6)[tid0] = 0u;
     fetch(sl.c_hi - 1, tid0);
 #pragma unroll 1
     for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
@@ -844,16 +819,14 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
         __syncthreads();
         poly_put_x(tid < 256 ? tq : tk, x, tid);
         poly_put_xt(tid < 256 ? tqt : tkt, x, tid);
+        poly_put_ones<T>(tid < 256 ? tqt : tkt, c * L::C, N, tid);
         v.put(tv, tid);
         go.put(tg, dn, tid);
         if (after) su.template to_lds<T, NORM>(us, y, l32, g);
         if (c > sl.c_lo) fetch(c - 1, tid);
         __syncthreads();
         if (before) {  // T <- T - this chunk's phi(k) [v, 1]^T
-            poly_gen_phi<T>(tk, phi0, ts, c * L::C, N, tid);
-            __syncthreads();
-            st.template update<T, NORM, true>(phi0, ts, tv, nullptr, lane);
-            __syncthreads();
+            st.template update<T, NORM, true>(tkt, tv, nullptr, lane);
             st.template to_lds<T, NORM>(ts, z, l32, g);
             __syncthreads();
         }
@@ -953,13 +926,15 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
                 static_for<0, PolyFeatures::kSteps>([&](auto ksc) {
                     constexpr int KS = decltype(ksc)::value;
                     float raw[8];
-                    const V8 f = poly_feature_frag<T, KS>(xr, xs, g, c0, c1, c2, raw);
+                    const PolyTwo f = poly_feature_frag<KS>(xr, xs, g, c0, c1, c2, raw);
 #pragma unroll
-                    for (int e = 0; e < 2; ++e)
-                        acc[e] = M::mma(poly_rd<T>(us + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5)), f, acc[e]);
+                    for (int e = 0; e < 2; ++e) {
+                        const V8 uf = poly_rd<T>(us + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5));
+                        acc[e] = M::mma(uf, f.hi, acc[e]);
+                        acc[e] = M::mma(uf, f.lo, acc[e]);
+                    }
                 });
             }
-            asm volatile("; dV, the rows after");
         } else {
             const PolyPair ga = poly_perm_base<128, false>(lane);
 #pragma unroll 1
@@ -980,7 +955,6 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
                     for (int e = 0; e < 2; ++e)
                         acc[e] = M::mma(poly_tr<T>(tg + 128 * (32 * sb + 16 * t), ga, e << 6), pf[t], acc[e]);
             }
-            asm volatile("; dV, the chunk's own rows");
         }
         __syncthreads();
         {
@@ -989,7 +963,6 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
             for (int i = 0; i < 16; ++i) mine[i] = poly_pick(half, acc[0][i], acc[1][i]);
             poly_put_acc(us, wave, lane, mine);  // (U's copy has been read)
         }
-        if (c > sl.c_lo) poly_gen_phi<T>(tq, phi0, ts, c * L::C, N, tid);
         __syncthreads();
         {
             f32x16 other;
@@ -1000,7 +973,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
             if (row < N) poly_store16<T>(dV + (int64_t)row * p.dvs_n, f, 32 * half + 16 * g, p.wv);
         }
         // U <- U + this chunk's phi(q) [g, dn]^T
-        if (c > sl.c_lo) su.template update<T, NORM, false>(phi0, ts, tg, smem + L::bDn + L::C * 4, lane);
+        if (c > sl.c_lo) su.template update<T, NORM, false>(tqt, tg, dn, lane);
     }
 #else
     (void)p;

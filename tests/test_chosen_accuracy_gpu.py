@@ -3,8 +3,9 @@
 import pytest
 import torch
 
-from flashy_linear_attention_amd import LinearAttention, LinearAttentionSmallVHD
+from flashy_linear_attention_amd import LinearAttention, LinearAttentionSmallVHD, PolynomialLinearAttention
 from flashy_linear_attention_amd import kernels
+from flashy_linear_attention_amd.poly import poly_attention_bwd, poly_attention_chunked_fwd, poly_attention_fwd
 
 pytestmark = pytest.mark.gpu
 
@@ -46,3 +47,30 @@ def test_no_larger_than_the_quadratic_kernels(h, n, dqk, dv, positive, gpu_devic
         other = (kernels.linear_flash_wrapper_fwd_smallv_hd(q, k, v), *kernels.linear_flash_wrapper_bwd_smallv_hd(do, q, k, v))
     assert any(not torch.equal(a, b) for a, b in zip(chosen, other))  # (chunk-wise, at these sizes)
     _compare(chosen, other, _exact(q, k, v, do))
+
+
+# (0.1 and 0.3 are no bf16 numbers; the second-order part alone; a leading constant)
+@pytest.mark.parametrize("normalise", [False, True], ids=["plain", "normalised"])
+@pytest.mark.parametrize("coef", [(1.0, 1.0, 0.5), (0.0, 0.0, 0.5), (0.1, 0.3, 0.7)], ids=str)
+@pytest.mark.parametrize("h,n,r,dv,scale", [(4, 2048, 16, 64, 1.0), (4, 2048, 16, 64, 0.5), (4, 4096, 8, 32, 1.0), (4, 512, 16, 64, 1.0), (3, 1111, 16, 40, 1.0)])
+def test_polynomial_no_larger_than_the_quadratic_kernels(h, n, r, dv, scale, coef, normalise, gpu_device):
+    gen = torch.Generator().manual_seed(n + r + dv)
+    xq, xk, v, do = ((s * torch.randn(1, h, n, d, generator=gen)).bfloat16().to(gpu_device)
+                     for d, s in ((r, scale), (r, scale), (dv, 1.0), (dv, 1.0)))
+    args = [t.clone().requires_grad_(True) for t in (xq, xk, v)]
+    out = PolynomialLinearAttention.apply(*args, *coef, normalise, 1e-5)
+    chosen = (out.detach(), *torch.autograd.grad(out, args, do))
+    o, denom = poly_attention_fwd(xq, xk, v, coef, normalise, 1e-5)
+    other = (o, *poly_attention_bwd(do, xq, xk, v, coef, *((o, denom) if normalise else ())))
+    assert any(not torch.equal(a, b) for a, b in zip(chosen, other))
+    exact = [t.double().requires_grad_(True) for t in (xq, xk, v)]
+    u = torch.matmul(exact[0], exact[1].transpose(-2, -1).contiguous())
+    scores = (coef[0] + coef[1] * u + coef[2] * u * u).tril()
+    want = torch.matmul(scores, exact[2])
+    n_want = scores.sum(-1) + 1e-5
+    if normalise:
+        want = want / n_want[..., None]
+        # (sums of fp32 scores, as the quadratic kernels' normaliser: a few 1e-7 where nothing cancels)
+        got = poly_attention_chunked_fwd(xq, xk, v, coef, True, 1e-5)[1]
+        assert float(torch.linalg.norm(got.double() - n_want.detach()) / torch.linalg.norm(n_want.detach())) <= 1e-6
+    _compare(chosen, other, (want.detach(), *torch.autograd.grad(want, exact, do.double())))
