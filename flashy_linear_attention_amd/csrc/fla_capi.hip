@@ -1805,8 +1805,8 @@ PolyPlan poly_plan(int64_t B, int64_t H, int64_t N, int64_t r, int64_t dv) {
     if (segs > p.n_chunks) segs = p.n_chunks;
     p.seg_chunks = (p.n_chunks + segs - 1) / segs;
     p.n_seg = (p.n_chunks + p.seg_chunks - 1) / p.seg_chunks;
-    p.state_bytes = B * H * p.n_seg * fla::PolyFeatures::kState * 4;
-    p.work_bytes = p.n_seg > 1 ? p.state_bytes : 0;
+    p.work_bytes = p.n_seg > 1 ? B * H * p.n_seg * fla::PolyFeatures::kState * 4 : 0;
+    p.state_bytes = p.n_seg > 1 ? p.work_bytes : 16;  // (a single segment per (b, h) hands nothing over: a token)
     return p;
 }
 
@@ -1851,7 +1851,7 @@ int poly_chunked_forward(const View &xq, const View &xk, const View &v, const Vi
     fla::PolyWalkParams w{};
     poly_common(w, pl, xq, xk, v, B, H, N, r, dv, coef);
     w.out = const_cast<void *>(o.ptr), w.us_b = o.strides[0], w.us_h = o.strides[1], w.us_n = o.strides[2];
-    w.eps = eps, w.denom = denom, w.ends = static_cast<float *>(state_out);
+    w.eps = eps, w.denom = denom, w.entries = pl.n_seg > 1 ? static_cast<float *>(state_out) : nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (int rc = poly_entries(pl, w, false, workspace, s)) return rc;
     return fla::poly_walk(w, false, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
@@ -1882,7 +1882,7 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
     w.dq = const_cast<void *>(dxq.ptr), w.dqs_b = dxq.strides[0], w.dqs_h = dxq.strides[1], w.dqs_n = dxq.strides[2];
     w.dk = const_cast<void *>(dxk.ptr), w.dks_b = dxk.strides[0], w.dks_h = dxk.strides[1], w.dks_n = dxk.strides[2];
     w.dv = const_cast<void *>(dvv.ptr), w.dvs_b = dvv.strides[0], w.dvs_h = dvv.strides[1], w.dvs_n = dvv.strides[2];
-    w.denom = const_cast<float *>(denom), w.ends = static_cast<float *>(const_cast<void *>(state_in));
+    w.denom = const_cast<float *>(denom), w.entries = pl.n_seg > 1 ? static_cast<float *>(const_cast<void *>(state_in)) : nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
     if (int rc = poly_entries(pl, w, true, workspace, s)) return rc;
     return fla::poly_walk(w, true, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
@@ -2239,9 +2239,13 @@ int fla_normalised_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int6
 }
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward) {
     if (dtype != FLA_DTYPE_BF16 || !poly_plan(B, H, N, R, D_v).ok) return 0;
-    // Measured over B H = 2 ... 256, N = 128 ... 2048, R / D_v = 16 / 64 and 8 / 32, with and without the normaliser: the
-    // pair is faster everywhere (1.14 to 2.8 times), forward alone from N = 2048 (at 1024, B H = 64: 35 us against 26).
-    return backward || N >= 2048;
+    // Quadratic time over chunk-wise time, R 8 and 16, with and without the normaliser, B H 1 ... 1024, N 100 ... 4096.  Pairs,
+    // D_v 64: 1.0 to 4.8 (0.91 to 0.99 at a few N of 200).  D_v 32, up to 256 heads: 0.94 to 4.2 (0.88 at B H 128, N 512); 512
+    // and 1024 heads: N 128 1.07 to 1.6, N 200 to 512 0.59 to 1.06, N 1024 0.85 to 1.18, N 2048 1.34 to 1.7.  Forward
+    // alone: N 4096 1.07 to 2.6; N 2048 1.1 to 1.5 with at most four heads, 0.62 to 1.09 with more; below 0.36 to 1.0.
+    const bool few = B * H <= 256;
+    if (backward) return D_v > 32 || few || N <= 128 || N >= 2048;
+    return N >= 4096 || (N >= 2048 && B * H <= 4);
 }
 
 int64_t fla_poly_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v) {

@@ -21,16 +21,18 @@
 // What bounds it: the matrix instructions and the VALU work that forms features together (an update's fragment of eight
 // features costs about 50 VALU instructions and serves four MFMAs, one along the row 28 and four); HBM is far away
 // (40 KiB per 128-row chunk).  Hence eight waves, two per SIMD, so that one wave's VALU work runs under the other's MFMAs: wave w owns
-// rows 32 (w % 4) .. of the chunk, and of their work one half: half of the features and of the score blocks (forward),
-// dq and the rows after the chunk in dV against dk and the chunk's own rows in dV (backward); the two waves of a row
+// rows 32 (w % 4) .. of the chunk, and of their work one half: half of the features and of the score blocks (forward
+// and dq), the rows after the chunk in dV against dk and the chunk's own rows in dV; the two waves of a row
 // block exchange one half of the sums through LDS.  (Halves of the output columns instead formed every feature row and
 // every score twice.)  Of a state a wave owns one of the seven blocks of 32 features, over all value columns, so that every feature is
 // formed once.  A workgroup has a CU to itself; the next chunk's rows are fetched into registers a chunk ahead.  The split
-// into segments and the forms of their entry states are the walk kernels' (fla_chunk_walk.h); the backward
-// walk gets T going backwards, by subtracting every chunk's sums from the state at its segment's end.
-// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 228 us this way.  (With
-// feature rows rounded to one bf16 number on both sides, from tiles of them in LDS: 200 us, and errors 1.2 times the
-// quadratic kernels'.)
+// into segments and the forms of their entry states are the walk kernels' (fla_chunk_walk.h).  Backward is a walk in
+// forward direction for dq, from the entry states forward formed, and one in reverse for dk and dv, so that nothing of a
+// row reaches the dq of the chunks before it.
+// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 239 us this way (kernels
+// 26 totals, 66 forward, 34 totals, 62 dq, 94 dk and dv).  With T for dq going backwards, by subtraction, in the reverse walk
+// 228 us, but a late row that is infinite, NaN or huge spoiled dq before it; with feature rows rounded to one bf16 number on
+// both sides as well, from tiles of them in LDS, 200 us, and errors up to 1.28 times the quadratic kernels'.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -53,7 +55,7 @@ struct PolyWalkParams {
     float *totals;       // totals kernel: receives the segments' sums; walks: those (sum_entries) or the entry states, of
                          // T (forward) / U (backward); null with a single segment
     int32_t sum_entries;
-    float *ends;         // T after every segment: written by forward (null: nowhere), read by backward
+    float *entries;      // T before every segment but the first: written by forward (null: nowhere), read by dq's walk
 };
 
 // Feature order: groups of eight.  Groups 0 .. 7: x_r x_(0..7) for r = 0 .. 7; groups 8 .. 23: x_r x_(8h .. 8h+7) for
@@ -74,10 +76,13 @@ struct PolyLds {  // byte offsets
     // forward
     static constexpr int fQ = 0, fK = fQ + XT, fKt = fK + XT, fV = fKt + XTR, fS = fV + VT, fEx = fS + ST, fZ = fEx + EX,
                          fSum = fZ + Z, fTotal = fSum + 2 * C * 4;
-    // backward
-    static constexpr int bQ = 0, bK = bQ + XT, bQt = bK + XT, bKt = bQt + XTR, bV = bKt + XTR, bG = bV + VT, bU = bG + VT,
-                         bT = bU + ST, bZ = bT + ST, bY = bZ + Z, bDn = bY + Z, bTotal = bDn + DN;
-    static_assert(EX == ST && XTR % 16 == 0 && fTotal <= 160 * 1024 && bTotal <= 160 * 1024, "a CU's LDS");
+    // dq (the exchange: sixteen floats a row)
+    static constexpr int qQ = 0, qK = qQ + XT, qKt = qK + XT, qV = qKt + XTR, qG = qV + VT, qS = qG + VT, qEx = qS + ST,
+                         qZ = qEx + C * 64, qDn = qZ + Z, qTotal = qDn + DN;
+    // dk, dv (the exchange over U's copy)
+    static constexpr int kQ = 0, kQt = kQ + XT, kK = kQt + XTR, kV = kK + XT, kG = kV + VT, kU = kG + VT, kY = kU + ST,
+                         kDn = kY + Z, kTotal = kDn + DN;
+    static_assert(EX == ST && XTR % 16 == 0 && fTotal <= 160 * 1024 && qTotal <= 160 * 1024 && kTotal <= 160 * 1024, "a CU's LDS");
 };
 
 // (a select of two values: written between two elements of an array it would become one load with a computed index, and
@@ -309,12 +314,12 @@ struct PolyState {
             if (g == 0) z[32 * wave + l32] = sum;
         }
     }
-    // += (NEG: -=) phi^T [z tile, extra column] over the chunk's 128 rows.  Feature rows are formed here, as products of two
+    // += phi^T [z tile, extra column] over the chunk's 128 rows.  Feature rows are formed here, as products of two
     // rows of the transposed x tile: a lane's eight rows of one feature, exactly, in two bf16 numbers each.
     // extra: the extra column, 128 floats in LDS (null: ones).
     // (Rounded to one bf16 number, from a tile of feature rows, they and the weighted ones along the rows made the errors of
     // O, dq, dk and dv 1.2 times the quadratic kernels', and those of the normaliser 1e-3 in place of 1e-7.)
-    template <typename T, bool NORM, bool NEG>
+    template <typename T, bool NORM>
     __device__ __forceinline__ void update(const unsigned char *xtr, const unsigned char *zt, const float *extra, int lane) {
         using M = Mma<T>;
         using V8 = typename M::V8;
@@ -332,10 +337,6 @@ struct PolyState {
             for (int k = 0; k < 4; ++k) {
                 f[2 * k] = __builtin_bit_cast(float, a[k] << 16) * __builtin_bit_cast(float, b[k] << 16);
                 f[2 * k + 1] = __builtin_bit_cast(float, a[k] & 0xffff0000u) * __builtin_bit_cast(float, b[k] & 0xffff0000u);
-            }
-            if constexpr (NEG) {
-#pragma unroll
-                for (int j = 0; j < 8; ++j) f[j] = -f[j];
             }
             if constexpr (NORM) {
                 if (extra) {
@@ -537,7 +538,7 @@ __global__ __launch_bounds__(512, 2) void poly_totals_kernel(const PolyWalkParam
             v.put(smem + L::tV, tid);
         if (c + 1 < sl.c_hi) fetch(c + 1);
         __syncthreads();
-        s.template update<T, NORM, false>(smem + L::tX, smem + L::tV, BWD ? dn : nullptr, lane);
+        s.template update<T, NORM>(smem + L::tX, smem + L::tV, BWD ? dn : nullptr, lane);
     }
     s.template store<NORM>(p.totals + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, l32, g);
 #else
@@ -605,6 +606,8 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
     PolyState s;
     s.clear(wave);
     poly_entry<NORM>(p, sl, false, tid0 & 31, (tid0 & 63) >> 5, s);
+    if (p.entries && sl.seg > 0)
+        s.template store<NORM>(p.entries + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
     u32x4 x;
     PolyTile<T> v;
     auto fetch = [&](int c, int tid) {
@@ -701,7 +704,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
             if (g == 0) sums[kh * L::C + trow] = rsum;
         }
         __syncthreads();
-        if (c + 1 < sl.c_hi || p.ends) s.template update<T, NORM, false>(tkt, tv, nullptr, lane);
+        if (c + 1 < sl.c_hi) s.template update<T, NORM>(tkt, tv, nullptr, lane);
         f32x16 other;
         poly_get_acc(exch, wave ^ 4, lane, other);
         float f[16], inv = 1.f;
@@ -714,22 +717,22 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
         for (int i = 0; i < 16; ++i) f[i] = (poly_pick(kh, acc[1][i], acc[0][i]) + other[i]) * inv;
         if (row < N) poly_store16<T>(O + (int64_t)row * p.us_n, f, 32 * kh + 16 * g, p.wv);
     }
-    if (p.ends) s.template store<NORM>(p.ends + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
 #else
     (void)p;
 #endif
 }
 
-// dx += the gradient at x of phi_w(x) . (S [g, extra]): H = S g for the row's 224 features, contracted with the row.
+// dx += the gradient at x of phi_w(x) . (S [g, extra]): H = S g for the row's feature blocks FB0 .. FB1 - 1, contracted with
+// the row.
 // S: the rounded state's tiles; gf: the row's g (v) as operands; z, extra: the state's last column and its factor.
 // Returns this lane's part of it (the other part is in the lane of the other g) in dx.
-template <typename T, bool NORM>
+template <typename T, bool NORM, int FB0, int FB1>
 __device__ __forceinline__ void poly_contract(const unsigned char *S, const float *z, float extra, const typename Mma<T>::V8 (&gf)[4],
                                               const float (&x)[16], int lane, float c1, float c2, float (&quad)[16]) {
     using M = Mma<T>;
     const int g = lane >> 5;
     const PolyPair sa = poly_perm_base<256, true>(lane);
-    static_for<0, PolyFeatures::kBlocks>([&](auto fbc) {
+    static_for<FB0, FB1>([&](auto fbc) {
         constexpr int FB = decltype(fbc)::value;
         f32x16 hh;
 #pragma unroll
@@ -770,10 +773,130 @@ __device__ __forceinline__ void poly_contract(const unsigned char *S, const floa
         }
         if constexpr (FB % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // (two blocks at a time: registers)
     });
+    if constexpr (FB1 < PolyFeatures::kBlocks) {
+#pragma unroll
+        for (int j = 0; j < 16; ++j) quad[j] *= 2.f * c2;
+    }
 }
 
+// dq: chunks ascending, T += phi(k) [v, 1]^T as in forward.  Each of the two waves of a row block takes a part of the feature
+// blocks and every other score block.
 template <typename T, bool NORM>
-__global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkParams p) {
+__global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkParams p) {
+#if defined(__gfx950__)
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    using L = PolyLds;
+    using M = Mma<T>;
+    using V8 = typename M::V8;
+    const int tid0 = threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid0 >> 6), rb = wave & 3, kh = wave >> 2;
+    const PolySlice sl = poly_slice(p);
+    if (!sl.valid) return;
+    const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
+    const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
+    const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
+    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
+    const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
+    const T *O = NORM ? static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h : nullptr;
+    const float *den = NORM ? p.denom + (int64_t)sl.bh * N : nullptr;
+    T *dQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h;
+    const float c1 = p.c1, c2 = p.c2;
+    unsigned char *tq = smem + L::qQ, *tk = smem + L::qK, *tkt = smem + L::qKt, *tv = smem + L::qV, *tg = smem + L::qG,
+                  *ts = smem + L::qS, *exch = smem + L::qEx;
+    float *z = reinterpret_cast<float *>(smem + L::qZ), *dn = reinterpret_cast<float *>(smem + L::qDn);
+    PolyState s;
+    s.clear(wave);
+    if (sl.seg > 0)
+        s.template add<NORM>(p.entries + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
+    u32x4 x;
+    PolyTile<T> v;
+    PolyGrad<T, NORM> go;
+    auto fetch = [&](int c, int tid) {
+        const int row0 = c * L::C;
+        x = tid < 256 ? poly_fetch_x<T>(Q, p.qs_n, row0, N, p.r, tid) : poly_fetch_x<T>(K, p.ks_n, row0, N, p.r, tid);
+        v.fetch(V, p.vs_n, row0, N, p.wv, tid);
+        go.fetch(G, p.gs_n, O, p.os_n, den, row0, N, p.wv, tid);
+    };
+    fetch(sl.c_lo, tid0);
+#pragma unroll 1
+    for (int c = sl.c_lo; c < sl.c_hi; ++c) {
+        const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+        __syncthreads();
+        poly_put_x(tid < 256 ? tq : tk, x, tid);
+        if (tid >= 256) poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
+        v.put(tv, tid);
+        go.put(tg, dn, tid);
+        s.template to_lds<T, NORM>(ts, z, l32, g);
+        if (c + 1 < sl.c_hi) fetch(c + 1, tid);
+        __syncthreads();
+
+        const int trow = 32 * rb + l32, row = c * L::C + trow;
+        const uint32_t ra = poly_row_base<128>(l32, g);
+        V8 gf[4];
+#pragma unroll
+        for (int kc = 0; kc < 4; ++kc) gf[kc] = poly_rd<T>(tg + 32 * 128 * rb, ra ^ (kc << 5));
+        const float dni = NORM ? dn[trow] : 0.f;
+        float dxs[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dxs[i] = 0.f;
+        if (c > 0) {
+            float xr[16];
+            poly_row<T>(tq, trow, xr);
+            if (kh == 0)
+                poly_contract<T, NORM, 0, 3>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
+            else
+                poly_contract<T, NORM, 3, PolyFeatures::kBlocks>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
+        }
+        const V8 xq = poly_row_frag<T>(tq, trow, g);
+        const int rc = walk_e_lane(l32) & 15;  // (columns 16 .. of the 32-wide block of dq are not used)
+        f32x16 dx;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) dx[i] = 0.f;
+#pragma unroll 1
+        for (int sb = kh; sb <= rb; sb += 2) {
+            const uint32_t all = sb < rb ? ~0u : 0u;
+            f32x16 m, u;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) m[i] = dni, u[i] = 0.f;
+            u = M::mma(poly_row_frag<T>(tk, 32 * sb + l32, g), xq, u);
+#pragma unroll
+            for (int kc = 0; kc < 4; ++kc) m = M::mma(poly_rd<T>(tv + 32 * 128 * sb, ra ^ (kc << 5)), gf[kc], m);
+            V8 df[2];
+            float d[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) d[i] = m[i] * (c1 + 2.f * c2 * u[i]);
+            poly_round_masked<T, false>(d, all, l32, g, df);
+#pragma unroll
+            for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(tkt, rc, 32 * sb + 16 * t, g), df[t], dx);
+        }
+        float f[16];  // (lanes of g = 0 hold the block's columns 0 .. 15)
+#pragma unroll
+        for (int i = 0; i < 16; ++i) f[i] = dxs[i] + __shfl_xor(dxs[i], 32, 64) + dx[i];
+        if (kh == 1 && g == 0) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                *reinterpret_cast<f32x4 *>(exch + (a * L::C + trow) * 16) = f32x4{f[4 * a], f[4 * a + 1], f[4 * a + 2], f[4 * a + 3]};
+        }
+        if (c + 1 < sl.c_hi) s.template update<T, NORM>(tkt, tv, nullptr, lane);
+        __syncthreads();
+        if (kh == 0 && g == 0) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f32x4 t = *reinterpret_cast<const f32x4 *>(exch + (a * L::C + trow) * 16);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) f[4 * a + j] += t[j];
+            }
+            if (row < N) poly_store16<T>(dQ + (int64_t)row * p.dqs_n, f, 0, p.r);
+        }
+    }
+#else
+    (void)p;
+#endif
+}
+
+// dk and dV: chunks descending, U += phi(q) [g, dn]^T
+template <typename T, bool NORM>
+__global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkParams p) {
 #if defined(__gfx950__)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     using L = PolyLds;
@@ -790,17 +913,14 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
     const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
     const T *O = NORM ? static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h : nullptr;
     const float *den = NORM ? p.denom + (int64_t)sl.bh * N : nullptr;
-    T *dQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h;
     T *dK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h;
     T *dV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
     const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
-    unsigned char *tq = smem + L::bQ, *tk = smem + L::bK, *tqt = smem + L::bQt, *tkt = smem + L::bKt, *tv = smem + L::bV,
-                  *tg = smem + L::bG, *us = smem + L::bU, *ts = smem + L::bT;
-    float *z = reinterpret_cast<float *>(smem + L::bZ), *y = reinterpret_cast<float *>(smem + L::bY),
-          *dn = reinterpret_cast<float *>(smem + L::bDn);
-    PolyState st, su;
-    st.clear(wave), su.clear(wave);
-    st.template add<NORM>(p.ends + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
+    unsigned char *tq = smem + L::kQ, *tqt = smem + L::kQt, *tk = smem + L::kK, *tv = smem + L::kV, *tg = smem + L::kG,
+                  *us = smem + L::kU;
+    float *y = reinterpret_cast<float *>(smem + L::kY), *dn = reinterpret_cast<float *>(smem + L::kDn);
+    PolyState su;
+    su.clear(wave);
     poly_entry<NORM>(p, sl, true, tid0 & 31, (tid0 & 63) >> 5, su);
     u32x4 x;
     PolyTile<T> v;
@@ -815,104 +935,19 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
 #pragma unroll 1
     for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
         const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-        const bool before = c > 0, after = c + 1 < p.n_chunks;  // (T, U of this chunk hold anything)
+        const bool after = c + 1 < p.n_chunks;  // (U of this chunk holds anything)
         __syncthreads();
         poly_put_x(tid < 256 ? tq : tk, x, tid);
-        poly_put_xt(tid < 256 ? tqt : tkt, x, tid);
-        poly_put_ones<T>(tid < 256 ? tqt : tkt, c * L::C, N, tid);
+        if (tid < 256) poly_put_xt(tqt, x, tid), poly_put_ones<T>(tqt, c * L::C, N, tid);
         v.put(tv, tid);
         go.put(tg, dn, tid);
         if (after) su.template to_lds<T, NORM>(us, y, l32, g);
         if (c > sl.c_lo) fetch(c - 1, tid);
         __syncthreads();
-        if (before) {  // T <- T - this chunk's phi(k) [v, 1]^T
-            st.template update<T, NORM, true>(tkt, tv, nullptr, lane);
-            st.template to_lds<T, NORM>(ts, z, l32, g);
-            __syncthreads();
-        }
 
         const int trow = 32 * rb + l32, row = c * L::C + trow;
-        const V8 xk = poly_row_frag<T>(tk, trow, g);
-        const uint32_t ra = poly_row_base<128>(l32, g);
-        const int rc = walk_e_lane(l32) & 15;  // (columns 16 .. of the 32-wide blocks of dq, dk are not used)
-        float dxs[16];
-#pragma unroll
-        for (int i = 0; i < 16; ++i) dxs[i] = 0.f;
-        f32x16 dx;
-        if (half == 0) {  // dq
-            V8 gf[4];
-#pragma unroll
-            for (int kc = 0; kc < 4; ++kc) gf[kc] = poly_rd<T>(tg + 32 * 128 * rb, ra ^ (kc << 5));
-            const V8 xq = poly_row_frag<T>(tq, trow, g);
-            const float dni = NORM ? dn[trow] : 0.f;
-            if (before) {
-                float xr[16];
-                poly_row<T>(tq, trow, xr);
-                poly_contract<T, NORM>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) dx[i] = 0.f;
-#pragma unroll 1
-            for (int sb = 0; sb <= rb; ++sb) {
-                const uint32_t all = sb < rb ? ~0u : 0u;
-                f32x16 m, u;
-#pragma unroll
-                for (int i = 0; i < 16; ++i) m[i] = dni, u[i] = 0.f;
-                u = M::mma(poly_row_frag<T>(tk, 32 * sb + l32, g), xq, u);
-#pragma unroll
-                for (int kc = 0; kc < 4; ++kc) m = M::mma(poly_rd<T>(tv + 32 * 128 * sb, ra ^ (kc << 5)), gf[kc], m);
-                V8 df[2];
-                float d[16];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) d[i] = m[i] * (c1 + 2.f * c2 * u[i]);
-                poly_round_masked<T, false>(d, all, l32, g, df);
-#pragma unroll
-                for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(tkt, rc, 32 * sb + 16 * t, g), df[t], dx);
-            }
-        } else {  // dk
-            V8 vf[4];
-#pragma unroll
-            for (int kc = 0; kc < 4; ++kc) vf[kc] = poly_rd<T>(tv + 32 * 128 * rb, ra ^ (kc << 5));
-            if (after) {
-                float xr[16];
-                poly_row<T>(tk, trow, xr);
-                poly_contract<T, NORM>(us, y, 1.f, vf, xr, lane, c1, c2, dxs);
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) dx[i] = 0.f;
-#pragma unroll 1
-            for (int sb = rb; sb < 4; ++sb) {
-                const uint32_t all = sb > rb ? ~0u : 0u;
-                f32x16 m, u;
-#pragma unroll
-                for (int a = 0; a < 4; ++a) {
-                    f32x4 d = {0.f, 0.f, 0.f, 0.f};
-                    if constexpr (NORM) d = *reinterpret_cast<const f32x4 *>(dn + 32 * sb + 8 * a + 4 * g);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) m[4 * a + j] = d[j], u[4 * a + j] = 0.f;
-                }
-                u = M::mma(poly_row_frag<T>(tq, 32 * sb + l32, g), xk, u);
-#pragma unroll
-                for (int kc = 0; kc < 4; ++kc) m = M::mma(poly_rd<T>(tg + 32 * 128 * sb, ra ^ (kc << 5)), vf[kc], m);
-                V8 df[2];
-                float d[16];
-#pragma unroll
-                for (int i = 0; i < 16; ++i) d[i] = m[i] * (c1 + 2.f * c2 * u[i]);
-                poly_round_masked<T, true>(d, all, l32, g, df);
-#pragma unroll
-                for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(tqt, rc, 32 * sb + 16 * t, g), df[t], dx);
-            }
-        }
-        {
-            float f[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                f[i] = dxs[i] + __shfl_xor(dxs[i], 32, 64) + dx[i];  // (lanes of g = 0 hold the block's columns 0 .. 15)
-            }
-            T *to = half == 0 ? dQ + (int64_t)row * p.dqs_n : dK + (int64_t)row * p.dks_n;
-            if (row < N && g == 0) poly_store16<T>(to, f, 0, p.r);
-        }
-        // dV: the dq waves form phi_w(k) U, the dk waves the chunk's own part; each finishes one half of the columns
+        // dV: the waves of half 0 form phi_w(k) U, those of half 1 -- after dk -- the chunk's own part; each finishes one
+        // half of the columns
         f32x16 acc[2];
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
@@ -936,25 +971,56 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
                 });
             }
         } else {
+            const V8 xk = poly_row_frag<T>(tk, trow, g);
+            const uint32_t ra = poly_row_base<128>(l32, g);
+            const int rc = walk_e_lane(l32) & 15;  // (columns 16 .. of the 32-wide block of dk are not used)
             const PolyPair ga = poly_perm_base<128, false>(lane);
+            V8 vf[4];
+#pragma unroll
+            for (int kc = 0; kc < 4; ++kc) vf[kc] = poly_rd<T>(tv + 32 * 128 * rb, ra ^ (kc << 5));
+            float dxs[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dxs[i] = 0.f;
+            if (after) {
+                float xr[16];
+                poly_row<T>(tk, trow, xr);
+                poly_contract<T, NORM, 0, PolyFeatures::kBlocks>(us, y, 1.f, vf, xr, lane, c1, c2, dxs);
+            }
+            f32x16 dx;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) dx[i] = 0.f;
 #pragma unroll 1
             for (int sb = rb; sb < 4; ++sb) {
                 const uint32_t all = sb > rb ? ~0u : 0u;
-                f32x16 u;
+                f32x16 m, u;
 #pragma unroll
-                for (int i = 0; i < 16; ++i) u[i] = 0.f;
+                for (int a = 0; a < 4; ++a) {
+                    f32x4 d = {0.f, 0.f, 0.f, 0.f};
+                    if constexpr (NORM) d = *reinterpret_cast<const f32x4 *>(dn + 32 * sb + 8 * a + 4 * g);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) m[4 * a + j] = d[j], u[4 * a + j] = 0.f;
+                }
                 u = M::mma(poly_row_frag<T>(tq, 32 * sb + l32, g), xk, u);
-                V8 pf[2];
-                float f[16];
 #pragma unroll
-                for (int i = 0; i < 16; ++i) f[i] = c0 + u[i] * (c1 + c2 * u[i]);
+                for (int kc = 0; kc < 4; ++kc) m = M::mma(poly_rd<T>(tg + 32 * 128 * sb, ra ^ (kc << 5)), vf[kc], m);
+                V8 df[2], pf[2];
+                float d[16], f[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) d[i] = m[i] * (c1 + 2.f * c2 * u[i]), f[i] = c0 + u[i] * (c1 + c2 * u[i]);
+                poly_round_masked<T, true>(d, all, l32, g, df);
                 poly_round_masked<T, true>(f, all, l32, g, pf);
 #pragma unroll
-                for (int t = 0; t < 2; ++t)
+                for (int t = 0; t < 2; ++t) {
+                    dx = M::mma(poly_col_frag<T>(tqt, rc, 32 * sb + 16 * t, g), df[t], dx);
 #pragma unroll
                     for (int e = 0; e < 2; ++e)
                         acc[e] = M::mma(poly_tr<T>(tg + 128 * (32 * sb + 16 * t), ga, e << 6), pf[t], acc[e]);
+                }
             }
+            float f[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) f[i] = dxs[i] + __shfl_xor(dxs[i], 32, 64) + dx[i];
+            if (row < N && g == 0) poly_store16<T>(dK + (int64_t)row * p.dks_n, f, 0, p.r);
         }
         __syncthreads();
         {
@@ -963,6 +1029,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
             for (int i = 0; i < 16; ++i) mine[i] = poly_pick(half, acc[0][i], acc[1][i]);
             poly_put_acc(us, wave, lane, mine);  // (U's copy has been read)
         }
+        if (c > sl.c_lo) su.template update<T, NORM>(tqt, tg, dn, lane);
         __syncthreads();
         {
             f32x16 other;
@@ -972,8 +1039,6 @@ __global__ __launch_bounds__(512, 2) void poly_walk_bwd_kernel(const PolyWalkPar
             for (int i = 0; i < 16; ++i) f[i] = poly_pick(half, acc[1][i], acc[0][i]) + other[i];
             if (row < N) poly_store16<T>(dV + (int64_t)row * p.dvs_n, f, 32 * half + 16 * g, p.wv);
         }
-        // U <- U + this chunk's phi(q) [g, dn]^T
-        if (c > sl.c_lo) su.template update<T, NORM, false>(tqt, tg, dn, lane);
     }
 #else
     (void)p;
@@ -999,9 +1064,14 @@ hipError_t launch_poly_totals(const PolyWalkParams &p, bool bwd, hipStream_t str
 
 template <typename T>
 hipError_t launch_poly_walk(const PolyWalkParams &p, bool bwd, hipStream_t stream) {
-    if (bwd)
-        return p.denom ? launch_poly_kernel<poly_walk_bwd_kernel<T, true>>(p, PolyLds::bTotal, stream)
-                       : launch_poly_kernel<poly_walk_bwd_kernel<T, false>>(p, PolyLds::bTotal, stream);
+    if (bwd) {
+        if (p.n_seg > 1 && !p.entries) return hipErrorInvalidValue;
+        if (hipError_t e = p.denom ? launch_poly_kernel<poly_walk_dq_kernel<T, true>>(p, PolyLds::qTotal, stream)
+                                   : launch_poly_kernel<poly_walk_dq_kernel<T, false>>(p, PolyLds::qTotal, stream))
+            return e;
+        return p.denom ? launch_poly_kernel<poly_walk_dkdv_kernel<T, true>>(p, PolyLds::kTotal, stream)
+                       : launch_poly_kernel<poly_walk_dkdv_kernel<T, false>>(p, PolyLds::kTotal, stream);
+    }
     return p.denom ? launch_poly_kernel<poly_walk_fwd_kernel<T, true>>(p, PolyLds::fTotal, stream)
                    : launch_poly_kernel<poly_walk_fwd_kernel<T, false>>(p, PolyLds::fTotal, stream);
 }

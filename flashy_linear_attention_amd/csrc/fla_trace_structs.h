@@ -95,7 +95,7 @@ FLA_FIELDS_END
 FLA_FIELDS_BEGIN(PolyWalkParams)
 FLA_FIELD(q) FLA_FIELD(k) FLA_FIELD(v) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(out) FLA_FIELD(dq) FLA_FIELD(dk) FLA_FIELD(dv)
 FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(r) FLA_FIELD(wv) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks) FLA_FIELD(n_seg)
-FLA_FIELD(denom) FLA_FIELD(totals) FLA_FIELD(sum_entries) FLA_FIELD(ends)
+FLA_FIELD(denom) FLA_FIELD(totals) FLA_FIELD(sum_entries) FLA_FIELD(entries)
 FLA_FIELDS_END
 
 #undef FLA_FIELDS_BEGIN

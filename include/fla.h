@@ -372,8 +372,8 @@ int fla_normalised_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int6
  * it is the faster evaluation (of a forward + backward pair, or with backward == 0 of forward alone; host arithmetic,
  * measured thresholds), 0 elsewhere and where it does not exist.
  * `workspace`: fla_poly_attn_chunked_workspace_bytes() bytes; `state_out` / `state_in`:
- * fla_poly_attn_chunked_state_bytes() bytes, written by forward (NULL: no backward will follow) and read by
- * backward; both 16-byte aligned, both may be 0 bytes. */
+ * fla_poly_attn_chunked_state_bytes() bytes (58 KiB per segment; a single segment per (b, h) needs none: 16),
+ * written by forward (NULL: no backward will follow) and read by backward; both 16-byte aligned. */
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward);
 int64_t fla_poly_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v);
 int64_t fla_poly_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v);

@@ -1,5 +1,6 @@
-"""Which evaluation the library names for widths that are no multiples of 8 (host arithmetic, no GPU): the chunk-wise one from
-the sequence length on from which it was measured to be the faster one, later for forward alone than for a pair."""
+"""Which evaluation the library names (host arithmetic, no GPU) for widths that are no multiples of 8 and for the polynomial
+map: the chunk-wise one where it was measured to be the faster one, later for forward alone than for a pair; and the
+polynomial map's state."""
 
 import pytest
 
@@ -16,3 +17,21 @@ def test_widths_that_are_no_multiples_of_8(bh, dqk, dv, pair_from, forward_from)
             assert _lib.query(name, 1, bh, first - 1, dqk, dv) == 0
         assert _lib.query(name, 1, bh, first, dqk, dv) == 1
         assert _lib.query(name, 1, bh, 4096, dqk, dv) == 1
+
+
+def test_polynomial_state_is_for_several_segments_alone():
+    """One state of 224 features over 64 columns, and their column of ones, per segment; nothing where a (b, h) is one segment
+    (256 workgroups at a time, 128 rows a chunk), however many heads there are."""
+    nbytes = lambda *shape: _lib.query("fla_poly_attn_chunked_state_bytes", *shape)  # noqa: E731
+    assert nbytes(16, 256, 128, 16, 64) == nbytes(4, 100, 4096, 16, 64) == nbytes(1, 1, 100, 8, 32) == 16
+    assert nbytes(4, 16, 4096, 16, 64) == 64 * 4 * 224 * 65 * 4
+
+
+@pytest.mark.parametrize("bh,n,dv,pair,forward", [
+    (1, 128, 64, 1, 0), (64, 1024, 64, 1, 0), (1024, 512, 64, 1, 0), (4, 2048, 64, 1, 1), (8, 2048, 64, 1, 0), (64, 4096, 64, 1, 1),
+    (256, 512, 32, 1, 0), (512, 512, 32, 0, 0), (512, 128, 32, 1, 0), (512, 2048, 32, 1, 0), (1024, 4096, 32, 1, 1),
+    (64, 1024, 72, 0, 0),
+])
+def test_polynomial(bh, n, dv, pair, forward):
+    for dtype, backward, want in ((0, 1, pair), (0, 0, forward), (1, 1, 0), (1, 0, 0)):
+        assert _lib.query("fla_poly_attn_prefers_chunked", 1, bh, n, 16, dv, dtype, backward) == want

@@ -4,7 +4,7 @@ of a call without them, bit for bit, in the operators that choose their evaluati
 import pytest
 import torch
 
-from flashy_linear_attention_amd import LinearAttention, LinearAttentionAuto, LinearAttentionSmallVHD
+from flashy_linear_attention_amd import LinearAttention, LinearAttentionAuto, LinearAttentionSmallVHD, PolynomialLinearAttention
 
 pytestmark = pytest.mark.gpu
 
@@ -39,4 +39,24 @@ def test_late_rows_do_not_reach_earlier_ones(op, b, h, n, dqk, dv, late, gpu_dev
     got = _step(op, q, k, v, do)
     rows = first // 32 * 32  # (the score blocks on the diagonal are 32 rows: a masked score times a late row)
     for name, a, w in zip(("O", "dQ"), got, want):
+        assert torch.equal(a[:, :, :rows], w[:, :, :rows]), name
+
+
+@pytest.mark.parametrize("normalise", [False, True], ids=["plain", "normalised"])
+@pytest.mark.parametrize("late", [float("nan"), float("inf"), 1e9], ids=["nan", "inf", "huge"])
+@pytest.mark.parametrize("b,h,n,r,dv", [(4, 70, 512, 16, 64), (4, 32, 1024, 8, 32), (1, 6, 1700, 16, 64), (1, 1, 4096, 16, 48)])
+def test_late_rows_do_not_reach_earlier_ones_of_the_polynomial(b, h, n, r, dv, late, normalise, gpu_device):
+    gen = torch.Generator().manual_seed(n + r + dv)
+    q, k, v, do = (torch.randn(b, h, n, d, generator=gen).bfloat16().to(gpu_device) for d in (r, r, dv, dv))
+
+    def step():
+        args = [t.clone().requires_grad_(True) for t in (q, k, v)]
+        out = PolynomialLinearAttention.apply(*args, 1.0, 1.0, 0.5, normalise, 1e-5)
+        return out.detach(), torch.autograd.grad(out, args, do)[0]
+
+    want = step()
+    first = n - 40
+    k[:, :, first:], v[:, :, first:] = late, late
+    rows = first // 32 * 32
+    for name, a, w in zip(("O", "dXq"), step(), want):
         assert torch.equal(a[:, :, :rows], w[:, :, :rows]), name
