@@ -53,6 +53,8 @@ SIGNATURES = {
     "fla_feature_attn_normalised_bwd": ([_ptr] * 9 + [_i64] * 5 + [_strides] * 8
                                         + [ctypes.c_int, ctypes.c_int, ctypes.c_int, _ptr, _ptr, _i64, _ptr], ctypes.c_int),
     "fla_linear_attn_chunked_fwd_static": ([_ptr] * 4 + [_i64] * 5 + [_strides] * 4 + [ctypes.c_int, _ptr], ctypes.c_int),
+    "fla_linear_attn_chunked_fwd_workspace_bytes": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int64),
+    "fla_linear_attn_chunked_state_operands": ([_i64] * 5 + [ctypes.POINTER(ctypes.c_int64)] * 2, ctypes.c_int),
     "fla_linear_attn_chunked_bwd": ([_ptr] * 7 + [_i64] * 5 + [_strides] * 7 + [ctypes.c_int, _ptr, _ptr, _i64, _ptr],
                                     ctypes.c_int),
     "fla_linear_attn_chunked_bwd_causal": ([_ptr] * 7 + [_i64] * 5 + [_strides] * 7 + [ctypes.c_int, _ptr, _ptr, _i64, _ptr],

@@ -60,7 +60,7 @@ def linear_attention_chunked_fwd(
     with device_guard(q.device):
         sbytes = _lib.query("fla_linear_attn_chunked_state_bytes", b, h, n, dqk, dv) if want_state else 0
         state = torch.empty(sbytes, dtype=torch.uint8, device=q.device) if sbytes else None
-        wbytes = _lib.query("fla_linear_attn_chunked_workspace_bytes", b, h, n, dqk, dv)
+        wbytes = _lib.query("fla_linear_attn_chunked_fwd_workspace_bytes", b, h, n, dqk, dv, int(state is not None))
         work = torch.empty(max(wbytes, 16), dtype=torch.uint8, device=q.device)
         valid = ctypes.c_int32(0)
         _lib.check(

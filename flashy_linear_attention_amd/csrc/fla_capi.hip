@@ -1246,6 +1246,10 @@ PackPlan pack_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
 int64_t packed_state_bytes(const PackPlan &p) { return p.inner_state + 2 * p.q_bytes + p.v_bytes; }
 // (backward without forward's copies is the larger: q, k, dQ, dK on one side, v, dO, dV on the other)
 int64_t packed_work_bytes(const PackPlan &p) { return p.inner_work + 4 * p.q_bytes + 3 * p.v_bytes; }
+// (forward: the copies of q, k, v, unless a state buffer takes them, and of O)
+int64_t packed_fwd_work_bytes(const PackPlan &p, bool with_state) {
+    return p.inner_work + (with_state ? 0 : 2 * p.q_bytes + p.v_bytes) + p.v_bytes;
+}
 
 // Row-packed stand-ins of a call's operands: views of copies carved from a buffer, and the launch that fills
 // them (or, for results, copies them back).
@@ -1279,12 +1283,12 @@ int packed_forward(const PackPlan &p, const View &q, const View &k, const View &
     for (const View &t : all)
         if (int rc = check_view(t)) return rc;
     if (int rc = check_alias_fwd(q, k, v, o, B, H, N, dqk, dv)) return rc;
-    if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < packed_work_bytes(p))
-        return FLA_ERR_WORKSPACE;
+    const int64_t need = packed_fwd_work_bytes(p, state_out != nullptr);
+    if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < need) return FLA_ERR_WORKSPACE;
     if (state_out && reinterpret_cast<uintptr_t>(state_out) % 16 != 0) return FLA_ERR_WORKSPACE;
     const int64_t qs[4] = {H * N * p.wq, N * p.wq, p.wq, 1}, vs[4] = {H * N * p.wv, N * p.wv, p.wv, 1};
     char *copies = state_out ? static_cast<char *>(state_out) + p.inner_state : static_cast<char *>(workspace) + p.inner_work;
-    char *results = static_cast<char *>(workspace) + p.inner_work + 2 * p.q_bytes + p.v_bytes;
+    char *results = static_cast<char *>(workspace) + need - p.v_bytes;
     const View qp = p.q_bytes ? View{copies, qs} : q, kp = p.q_bytes ? View{copies + p.q_bytes, qs} : k;
     const View vp = p.v_bytes ? View{copies + 2 * p.q_bytes, vs} : v, op = p.v_bytes ? View{results, vs} : o;
     Packed in(B, H, N), out(B, H, N);
@@ -2071,6 +2075,24 @@ int64_t fla_linear_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N,
     const int64_t plain = chunked_op_workspace_bytes(B, H, N, D_qk, D_v);  // (the feature-map operator's, whatever the widths)
     const PackPlan p = pack_plan(B, H, N, D_qk, D_v);
     return p.ok && packed_work_bytes(p) > plain ? packed_work_bytes(p) : plain;
+}
+
+int64_t fla_linear_attn_chunked_fwd_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int with_state) {
+    if (B < 0 || H < 0 || N < 0 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
+    if (const PackPlan p = pack_plan(B, H, N, D_qk, D_v); p.ok) return packed_fwd_work_bytes(p, with_state != 0);
+    return chunked_op_workspace_bytes(B, H, N, D_qk, D_v);
+}
+
+int fla_linear_attn_chunked_state_operands(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int64_t *offsets,
+                                           int64_t *pitches) {
+    if (B < 0 || H < 0 || N < 0 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256 || !offsets || !pitches) return 0;
+    const PackPlan p = pack_plan(B, H, N, D_qk, D_v);
+    if (!p.ok) return 0;
+    for (int i = 0; i < 3; ++i) {
+        const bool copied = i < 2 ? p.q_bytes != 0 : p.v_bytes != 0;
+        offsets[i] = copied ? p.inner_state + i * p.q_bytes : -1, pitches[i] = i < 2 ? p.wq : p.wv;
+    }
+    return 1;
 }
 
 int fla_linear_attn_chunked_fwd(const void *q, const void *k, const void *v, void *o, int64_t B, int64_t H, int64_t N,

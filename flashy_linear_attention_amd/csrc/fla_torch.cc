@@ -159,7 +159,7 @@ std::tuple<Tensor, Tensor> product_fwd(const Tensor &q_, const Tensor &k_, const
                                         str(o), c.dtype, c.stream));
     } else {
         if (want_state) state = c.bytes(fla_linear_attn_chunked_state_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        const Tensor work = c.bytes(fla_linear_attn_chunked_fwd_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv, state.defined()));
         int32_t valid = 0;
         must(fla_linear_attn_chunked_fwd(ptr(q), ptr(k), ptr(v), ptr(o), c.b, c.h, c.n, c.dqk, c.dv, str(q), str(k), str(v),
                                          str(o), c.dtype, ptr(state), &valid, ptr(work), size_of(work), c.stream));
@@ -195,10 +195,21 @@ struct Product : Function<Product> {
         ctx->saved_data["widened"] = in.widened;
         auto [o, state] = product_fwd(q, k, v, (int)ev, true);
         ctx->saved_data["ev"] = ev;
-        if (state.defined())
-            ctx->save_for_backward({q, k, v, state});
-        else
-            ctx->save_for_backward({q, k, v});
+        variable_list s = {q, k, v};
+        if (state.defined()) {
+            // (copies with aligned rows in the state buffer are what backward reads: kept in place of the operands)
+            int64_t at[3], pitch[3];
+            const int64_t b = q.size(0), h = q.size(1), n = q.size(2);
+            if (fla_linear_attn_chunked_state_operands(b, h, n, q.size(3), v.size(3), at, pitch)) {
+                at::AutoDispatchBelowADInplaceOrView below;
+                for (int i = 0; i < 3; ++i)
+                    if (at[i] >= 0)
+                        s[i] = state.narrow(0, at[i], 2 * b * h * n * pitch[i]).view(q.scalar_type()).view({b, h, n, pitch[i]})
+                                   .narrow(3, 0, s[i].size(3));
+            }
+            s.push_back(state);
+        }
+        ctx->save_for_backward(std::move(s));
         return o;
     }
     static variable_list backward(AutogradContext *ctx, variable_list go) {

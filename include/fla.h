@@ -206,6 +206,15 @@ int fla_linear_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_q
 /* The same question for forward alone. */
 int fla_linear_attn_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v);
 int64_t fla_linear_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v);
+/* What the forward call alone needs of it (less only for widths that are no multiples of 8); `with_state`: with a
+ * state buffer, which then takes the copies of q, k and v. */
+int64_t fla_linear_attn_chunked_fwd_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int with_state);
+/* 1 when forward leaves copies of operands in the state buffer and backward, given that buffer, reads those: byte offsets of
+ * the copies of q, k, v (-1: that operand is read where the caller has it) and their row pitches in elements, heads and batches
+ * following densely.  A caller that keeps the buffer for backward may pass such a copy as the operand itself and let its own
+ * go.  0: none. */
+int fla_linear_attn_chunked_state_operands(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int64_t *offsets,
+                                           int64_t *pitches);
 int fla_linear_attn_chunked_fwd(const void *q, const void *k, const void *v, void *o,
                                 int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v,
                                 const int64_t *q_strides, const int64_t *k_strides,

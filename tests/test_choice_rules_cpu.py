@@ -35,3 +35,14 @@ def test_polynomial_state_is_for_several_segments_alone():
 def test_polynomial(bh, n, dv, pair, forward):
     for dtype, backward, want in ((0, 1, pair), (0, 0, forward), (1, 1, 0), (1, 0, 0)):
         assert _lib.query("fla_poly_attn_prefers_chunked", 1, bh, n, 16, dv, dtype, backward) == want
+
+
+def test_forward_workspace_of_copied_operands():
+    """Forward asks for the copies it makes: of O, and of q, k, v where no state buffer takes them (rows of 160 and 64 elements)."""
+    shape = (2, 16, 2048, 153, 64)
+    full = _lib.query("fla_linear_attn_chunked_workspace_bytes", *shape)
+    with_state, without = (_lib.query("fla_linear_attn_chunked_fwd_workspace_bytes", *shape, s) for s in (1, 0))
+    copy = 2 * 16 * 2048 * 160 * 2
+    assert without - with_state == 2 * copy and full - with_state == 4 * copy
+    assert _lib.query("fla_linear_attn_chunked_fwd_workspace_bytes", 2, 16, 2048, 160, 64, 1) == _lib.query(
+        "fla_linear_attn_chunked_workspace_bytes", 2, 16, 2048, 160, 64) == with_state

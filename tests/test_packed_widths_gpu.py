@@ -28,3 +28,27 @@ def test_widths_off_the_eights(b, h, n, dqk, dv, dtype, transposed, gpu_device):
     for st in (state, None):  # (forward's copies, and copies of backward's own)
         for name, got, want in zip(("dQ", "dK", "dV"), linear_attention_chunked_bwd(do, q, k, v, st), want_g):
             assert_close(f"{name}, state {st is not None}", got, want)
+
+
+def test_copies_are_kept_in_place_of_the_operands(gpu_device):
+    """What a training step holds on to between forward and backward: the copies, and not q, k, v beside them."""
+    from flashy_linear_attention_amd import LinearAttentionSmallVHD, _lib
+
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in reference_style_inputs(1, 8, 2048, 153, 64, torch.bfloat16, seed=3)[:3]]
+    torch.cuda.synchronize()
+    q, k, v = (t * 1.0 for t in leaves)  # (a product with a number keeps neither factor)
+    base = torch.cuda.memory_allocated() - sum(t.numel() * 2 for t in (q, k, v))
+    out = LinearAttentionSmallVHD.apply(q, k, v)
+    size = q.numel() * 2
+    del q, k
+    state = _lib.query("fla_linear_attn_chunked_state_bytes", 1, 8, 2048, 153, 64)
+    # (v, the output and the state buffer with the copies; allocations are rounded up to 2 MiB at most)
+    held = torch.cuda.memory_allocated() - base
+    assert held <= v.numel() * 2 + out.numel() * 2 + state + 3 * (2 << 20) < held + 2 * size
+    out.backward(torch.ones_like(out))
+    grads = [t.grad.clone() for t in leaves]
+    for t in leaves:
+        t.grad = None
+    qc, kc, vc = leaves
+    LinearAttentionSmallVHD.apply(qc, kc, vc).backward(torch.ones_like(out))
+    assert all(torch.equal(a, t.grad) for a, t in zip(grads, leaves))
