@@ -1342,7 +1342,9 @@ int plain_chunked_backward(const View &go, const View &q, const View &k, const V
     if (int rc = check_common(B, H, N, dtype)) return rc;
     if (dqk < 1 || dqk > 256) return FLA_ERR_HEAD_DIM;
     if (dv < 1 || dv > 256) return FLA_ERR_V_HEAD_DIM;
-    if (const PackPlan p = pack_plan(B, H, N, dqk, dv); p.ok)
+    // (causal, D_v above 128: product by product with the states of 256-row chunks in memory, each sum rounded once and no state
+    // by subtraction, where the copies would run as column halves of v)
+    if (const PackPlan p = pack_plan(B, H, N, dqk, dv); p.ok && !(causal && dv > 128))
         return packed_backward(p, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace, workspace_bytes,
                                stream, causal);
     return chunked_backward(go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace, workspace_bytes, stream, 0,
@@ -1907,9 +1909,10 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
     // fast kernels of either kind on copies with aligned rows, at the cost of two copy launches.  Quadratic time over
     // chunk-wise time, B H = 1 ... 64, at the last N below and the first N from the line on -- forward alone: 20 columns
     // 0.95 to 1.06 at 512, 1.3 to 1.8 at 1024; 36 columns 0.80 to 0.86 at 128, 1.12 to 1.18 at 256; 91/64 and 100 0.91 to
-    // 1.1 at 64, 1.17 to 1.4 at 128; wider (153/64, 153/128, 250) 1.15 to 2.8 from 64 to 256.  Forward + backward: 20 columns
+    // 1.1 at 64, 1.17 to 1.4 at 128; wider (153/64, 153/128) 1.15 to 2.1 from 64 to 256.  Forward + backward: 20 columns
     // 0.80 to 0.87 at 128, 1.12 to 1.21 at 256; 36 columns 0.92 to 0.97 at 64, 1.24 to 1.27 at 128; wider 1.1 to 3.3.
-    if (pack_plan(B, H, N, D_qk, D_v).ok) {
+    // (A v wider than 128 columns: the rule of multiples of 8 below -- dQ and dK would be rounded once per half of v.)
+    if (D_v <= 128 && pack_plan(B, H, N, D_qk, D_v).ok) {
         const int64_t d = padded(D_qk > D_v ? D_qk : D_v);
         if (backward) return d <= 32 ? N >= 256 : d <= 64 ? N >= 128 : 1;
         return d <= 32 ? N > 512 : d <= 64 ? N >= 256 : d <= 128 ? N >= 128 : 1;

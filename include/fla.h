@@ -235,7 +235,8 @@ int fla_linear_attn_chunked_bwd(const void *grad_out, const void *q, const void 
  * head dims above 64 and with `state_in`, the call above walks once, in reverse, and gets dQ's running state
  * by subtracting from the one at the end of a segment: late rows that are infinite, NaN or far larger than
  * the rest spoil the dQ of the rows before them.  This one takes a walk in forward direction for dQ, as the
- * call without `state_in` does (with D_v above 128 it is the same as the call above).  Same arguments. */
+ * call without `state_in` does (with D_v above 128 and widths that are multiples of 8 it is the same as the call
+ * above).  Same arguments. */
 int fla_linear_attn_chunked_bwd_causal(const void *grad_out, const void *q, const void *k, const void *v,
                                        void *dq, void *dk, void *dv,
                                        int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v,

@@ -8,7 +8,7 @@ from flashy_linear_attention_amd import _lib
 
 
 @pytest.mark.parametrize("dqk,dv,pair_from,forward_from", [
-    (20, 20, 256, 513), (31, 7, 256, 513), (36, 36, 128, 256), (100, 100, 1, 128), (91, 64, 1, 128), (153, 64, 1, 1), (250, 250, 1, 1),
+    (20, 20, 256, 513), (31, 7, 256, 513), (36, 36, 128, 256), (100, 100, 1, 128), (91, 64, 1, 128), (153, 64, 1, 1),
 ])
 @pytest.mark.parametrize("bh", [1, 64])
 def test_widths_that_are_no_multiples_of_8(bh, dqk, dv, pair_from, forward_from):
@@ -46,3 +46,10 @@ def test_forward_workspace_of_copied_operands():
     assert without - with_state == 2 * copy and full - with_state == 4 * copy
     assert _lib.query("fla_linear_attn_chunked_fwd_workspace_bytes", 2, 16, 2048, 160, 64, 1) == _lib.query(
         "fla_linear_attn_chunked_workspace_bytes", 2, 16, 2048, 160, 64) == with_state
+
+
+@pytest.mark.parametrize("name", ["fla_linear_attn_prefers_chunked", "fla_linear_attn_forward_prefers_chunked"])
+def test_a_wide_v_has_one_rule(name):
+    """A v of more than 128 columns: the same line whatever the widths (W = B H N^2 256 from 3e10 on)."""
+    for width in (250, 255, 256):
+        assert _lib.query(name, 1, 16, 2048, width, width) == 0 and _lib.query(name, 1, 16, 4096, width, width) == 1

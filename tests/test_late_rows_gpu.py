@@ -28,7 +28,7 @@ def _step(op, q, k, v, do):
     ("smallv", 2, 16, 2048, 128, 64), ("auto", 2, 10, 1500, 72, 72), ("auto", 1, 6, 2100, 100, 100), ("smallv", 1, 12, 1024, 91, 64),
     # q and k of more than 128 columns
     ("smallv", 4, 64, 512, 256, 64), ("smallv", 4, 16, 2048, 256, 64), ("smallv", 1, 8, 2048, 160, 32), ("smallv", 1, 20, 2048, 192, 128),
-    ("smallv", 2, 3, 4096, 136, 128), ("smallv", 1, 16, 2048, 153, 64),
+    ("smallv", 2, 3, 4096, 136, 128), ("smallv", 1, 16, 2048, 153, 64), ("auto", 1, 4, 1100, 250, 250),
 ])
 def test_late_rows_do_not_reach_earlier_ones(op, b, h, n, dqk, dv, late, gpu_device):
     gen = torch.Generator().manual_seed(n + dqk + dv)
