@@ -55,7 +55,7 @@ PROFILED_TRAFFIC = {
     # chunk-wise: all kernels of a step
     ("C3", "chunked"): (1.847e9, "profiles/chunked_C3_C5_kernel_trace_pmc.md"),
     ("C4", "chunked"): (1.310e9, "profiles/chunked_C4_kernel_trace_pmc.md"),
-    ("C5", "chunked"): (1.074e9, "profiles/chunked_C3_C5_kernel_trace_pmc.md"),
+    ("C5", "chunked"): (1.132e9, "profiles/chunked_C3_C5_kernel_trace_pmc.md"),
 }
 # MFMA operations the dominant kernel issues over those of its product-units (rocprofv3
 # SQ_INSTS_VALU_MFMA_MOPS_BF16 x 512 FLOPs; the excess is the 32 x 32 blocks on the diagonal)

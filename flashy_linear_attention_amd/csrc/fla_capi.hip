@@ -393,10 +393,14 @@ struct WalkPlan {
 // are padded with zeros as they land in LDS, and at D = 128 the kernels built for at most 64 true columns on one side
 // leave the padding's MFMAs out.  The plain operator only (the normaliser's and the feature maps' variants of the
 // kernels are built for equal padded widths).
-// D = 128: up to this many segments per (b, h) the walks add up the segments' totals themselves, beyond it a scan kernel
-// does.  Measured per forward + backward, scan against sums on load: B H 32, N 4096 (8 segments) 146 / 137 us; B H 24, N
-// 1500 (8) 80 / 77; B H 20, N 4096 (11) 145 / 141; B H 16, N 4096 (16) 101 / 104; B H 8, N 4096 (32) 79 / 109.
-constexpr int kSumOnLoadMost = 12;
+// From three segments per (b, h) up to this many the walks add up the segments' totals themselves, beyond it a scan kernel
+// does (padded head dims up to 64: fla::walk_sum_on_load_max, which the kernels know).
+//   D = 128.  Forward + backward, scan against sums on load: B H 32, N 4096 (8 segments) 146 / 137 us; B H 24, N 1500 (8)
+//   80 / 77; B H 20, N 4096 (11) 145 / 141; B H 16, N 4096 (16) 101 / 104; B H 8, N 4096 (32) 79 / 109.  Four pairs of column
+//   halves at a time (256 / 256) the same: B H 16, N 4096 (8) 258 / 234; B H 12 (10) 319 / 313; B H 32, N 2048 (4) 250 / 229.
+//   A wide q / k against a v of up to 128: two states to add up.  256 / 64, B H 64, N 4096 (4): 273 / 264.
+//   The polynomial map, of 58 KiB a state: where adding them up costs more than a launch.
+constexpr int kSumOnLoadMost = 12, kSumOnLoadWide = 7, kSumOnLoadPoly = 8;
 
 // `parts`: workgroups per segment (a launch that does several column halves at a time).
 WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false, int64_t parts = 1) {
@@ -433,6 +437,8 @@ WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, boo
     w.saved_bytes = w.split || states > per_chunk ? states : per_chunk;
     return w;
 }
+
+bool sums_on_load(const WalkPlan &w, int most = kSumOnLoadMost) { return w.n_seg >= 3 && w.n_seg <= most; }
 
 // totals of Y^T Z over the walk's segments into `work`, then the segments' entry states: their sums
 // over the segments before (reverse == 0) or after (reverse != 0), written to `entry` (null: over
@@ -705,7 +711,7 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
     // starts (three of each half in flight together) and writes the entry state it formed for backward
     // (B 4, H 16, N 4096, D_qk 256, D_v 64, four segments: 0.273 -> 0.267 ms per forward + backward, and 0.264 with
     // the reverse walk doing the same).
-    const bool sum_on_load = wp.n_seg >= 3 && wp.n_seg <= 7;
+    const bool sum_on_load = sums_on_load(wp, kSumOnLoadWide);
     float *keep[2] = {nullptr, nullptr};
     if (wp.n_seg > 1) {
         // (kept for backward when there is a state buffer: each half's entry states, its final state behind them;
@@ -746,7 +752,7 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
     // at hand -- K_h^T V over the segments before
     const float *fwd_entries[2] = {nullptr, nullptr}, *entries[2] = {nullptr, nullptr};
     // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
-    const bool rev_sums_on_load = wp.n_seg >= 3 && wp.n_seg <= 7;
+    const bool rev_sums_on_load = sums_on_load(wp, kSumOnLoadWide);
     if (wp.n_seg > 1) {
         float *const none[2] = {nullptr, nullptr};
         if (state_in) {
@@ -801,10 +807,6 @@ float *quad_finals(const WalkPlan &wp, const void *state) {
     return reinterpret_cast<float *>(static_cast<char *>(const_cast<void *>(state)) + 4 * wp.entry_bytes);
 }
 
-// (forward + backward at 256 / 256, scan against sums on load: B H 16, N 4096, 8 segments 258 / 234 us; B H 12, 10 segments 319 /
-// 313; B H 32, N 2048, 4 segments 250 / 229)
-bool quad_sums_on_load(const WalkPlan &wp) { return wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost; }
-
 // the four pairs' segment totals of Y^T Z to `entries`, and the entry states over them where the walk does not add up
 int quad_entry_states(const WalkPlan &wp, const View &y, const View &z, int64_t B, int64_t H, int64_t N, int64_t dy, int64_t dz,
                       int dtype, int reverse, float *entries, hipStream_t s) {
@@ -819,13 +821,13 @@ int quad_entry_states(const WalkPlan &wp, const View &y, const View &z, int64_t 
     tp.direct = wp.n_seg == 2;
     tp.seg_lo = reverse ? 1 : 0, tp.seg_hi = (int32_t)(reverse ? wp.n_seg : wp.n_seg - 1);
     if (fla::walk_totals(dtype, wp.D, tp, s) != hipSuccess) return FLA_ERR_LAUNCH;
-    if (tp.direct || quad_sums_on_load(wp)) return FLA_OK;
+    if (tp.direct || sums_on_load(wp)) return FLA_OK;
     return fla::walk_scan(entries, entries, 4 * B * H, (int)wp.n_seg, wp.D, wp.D, reverse, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 
 int quad_forward(const WalkPlan &wp, const View &q, const View &k, const View &v, const View &o, int64_t B, int64_t H, int64_t N,
                  int64_t dqk, int64_t dv, int dtype, void *state_out, void *workspace, hipStream_t s) {
-    const bool sum_on_load = quad_sums_on_load(wp);
+    const bool sum_on_load = sums_on_load(wp);
     const int64_t pair = wp.entry_bytes / 4;  // floats
     float *const kept = static_cast<float *>(state_out);
     float *const entries = kept && !sum_on_load ? kept : static_cast<float *>(workspace);
@@ -847,7 +849,7 @@ int quad_backward(const WalkPlan &wp, const View &go, const View &q, const View 
         if (int rc = quad_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, entries, s)) return rc;
     fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, 128, 128);
     r.wqk2 = (int32_t)(dqk - 128), r.wv2 = (int32_t)(dv - 128);
-    r.init = wp.n_seg > 1 ? entries : nullptr, r.init_is_totals = quad_sums_on_load(wp);
+    r.init = wp.n_seg > 1 ? entries : nullptr, r.init_is_totals = sums_on_load(wp);
     r.xinit = static_cast<const float *>(state_in), r.xtotal = quad_finals(wp, state_in);
     for (int pass = 0; pass < 2; ++pass) {
         r.quad = 3 - pass, r.accumulate = pass;
@@ -939,9 +941,9 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         // them to state_out (the totals themselves are computed there, and no workspace is used);
         // padded head dims up to 64 hand over the 16-bit state of every chunk instead
         const bool in_state = state_out && wp.split;
-        // D = 128, a few segments more than two (kSumOnLoadMost): the totals go to the workspace, the walk adds them up itself as it starts
-        // and writes the entry states it formed to state_out -- no scan launch (B H 64, N 4096: see wide_forward)
-        const bool sum_on_load = wp.split && !fmap && !nx && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
+        // D = 128, a few segments more than two: the totals go to the workspace, the walk adds them up itself as it starts
+        // and writes the entry states it formed to state_out -- no scan launch
+        const bool sum_on_load = wp.split && !fmap && !nx && sums_on_load(wp);
         if (need_totals && (!in_state || sum_on_load) &&
             (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < wp.work_bytes))
             return FLA_ERR_WORKSPACE;
@@ -1098,7 +1100,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         // with forward's states at hand (and without the normaliser): one reverse walk
         const bool one_walk = state_in && !nx && !causal;
         // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
-        const bool rev_sums_on_load = (one_walk || causal) && wp.n_seg >= 3 && wp.n_seg <= kSumOnLoadMost;
+        const bool rev_sums_on_load = (one_walk || causal) && sums_on_load(wp);
         if (wp.n_seg > 1) {
             if (!state_in) {
                 const float *fwd_entry = nullptr;
@@ -1823,12 +1825,12 @@ int check_poly_chunked(const PolyPlan &pl, int dtype, int64_t workspace_bytes, c
     return reinterpret_cast<uintptr_t>(state) % 16 != 0 ? FLA_ERR_WORKSPACE : FLA_OK;
 }
 
-// totals over the segments and -- beyond eight of them, where adding them up on load costs more than a launch -- their scan
+// totals over the segments and -- beyond kSumOnLoadPoly of them -- their scan
 int poly_entries(const PolyPlan &pl, fla::PolyWalkParams &w, bool bwd, void *workspace, hipStream_t s) {
     if (pl.n_seg == 1) return FLA_OK;
     w.totals = static_cast<float *>(workspace);
     if (fla::poly_totals(w, bwd, s) != hipSuccess) return FLA_ERR_LAUNCH;
-    w.sum_entries = pl.n_seg <= 8;
+    w.sum_entries = pl.n_seg <= kSumOnLoadPoly;
     if (w.sum_entries) return FLA_OK;
     return fla::poly_scan(w.totals, w.BH, w.n_seg, bwd ? 1 : 0, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
@@ -1897,9 +1899,10 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
 // Which evaluation is faster on MI355X (bench.py --crossover): the quadratic kernels' time grows with W = B H N^2 D (D: the
 // larger padded head dim) above the time of one workgroup's longest row tile, which grows with N; the chunk-wise kernels'
 // with B H N D above a floor of launches.  Measured quadratic time over chunk-wise time, widths 32 ... 128 and 64/32, 128/64, 128/32, B H 1 ...
-// 192, N 512 ... 8192.  Forward + backward, equal widths: from W = B H N^2 D = 4e9 (8e9 at 128) 1.08 to 4.9 with few heads
-// or many; few heads and long: N = 4096 1.8 to 2.9, N = 2048 1.25 to 1.7 at 64 and 128 columns, 0.84 to 1.1 at 32; N = 1024
-// 0.67 to 1.2.  Widths that differ (small-V operator): N = 1024 1.4 to 1.9.  Forward alone: N = 2048 1.17 to 1.9 (0.92 to
+// 192, N 256 ... 8192.  Forward + backward (dQ by its own walk, see chunked_backward), equal widths: from W = B H N^2 D = 4e9
+// (8e9 at 128) 1.17 to 4.8 with few heads or many (0.90 at 32 columns, B H 16, N 3072); few heads and long: N = 4096 1.5 to
+// 3.1, N = 2048 1.42 to 2.0 at 64 and 128 columns, 0.88 to 1.19 at 32; N = 1024 0.67 to 1.2.  Widths that differ (small-V
+// operator): N = 1024 1.38 to 2.1, from W = 5e8 (1e9 below 128) 1.08 to 1.6.  Forward alone: N = 2048 1.17 to 1.9 (0.92 to
 // 0.99 at 32 columns), W from 1.2e10 1.1 to 2; N = 512 and 1024 below that 0.65 to 1.15.
 int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, bool backward) {
     if (B < 1 || H < 1 || N < 1 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
@@ -1921,8 +1924,8 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
     if (wp.ok && !backward) return wp.D <= 32 ? N >= 4096 || w >= 5e9 : N >= 2048 || w >= 1.2e10;
     if (wp.ok && pad_index(D_qk) != pad_index(D_v)) return N >= 1024 || w >= (wp.D <= 64 ? 1e9 : 5e8);
     if (wp.ok) return N >= (wp.D <= 32 ? 4096 : 2048) || w >= (wp.D <= 64 ? 4e9 : 8e9);  // equal padded head dims up to 128
-    // D_qk in (128, 256].  D_v <= 64: pairs 1.8 to 5 from N = 1024 or W = 1e9 on, forward alone 1.13 to 2.9 from N = 1024 (N = 512
-    // 0.82 to 1.1).  D_v in (64, 128]: pairs 1.26 to 2.1 from N = 2048, 1.2 from W = 2.5e10 (0.95 at 1.5e10, N = 1024); forward
+    // D_qk in (128, 256].  D_v <= 64: pairs 1.13 to 5 from N = 1024 or W = 1e9 on, forward alone 1.13 to 2.9 from N = 1024 (N = 512
+    // 0.82 to 1.1).  D_v in (64, 128]: pairs 1.35 to 3.1 from N = 2048, 1.3 from W = 2.5e10 (1.0 at 1.7e10, N = 1024); forward
     // alone 1.14 to 1.55 from N = 4096, at N = 2048 1.1 to 1.4 with B H <= 4 and 0.93 with 16.
     if (wide_plan(B, H, N, D_qk, D_v).ok) {
         if (D_v <= 64) return N >= 1024 || (backward && w >= 1e9);

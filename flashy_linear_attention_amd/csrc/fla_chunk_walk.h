@@ -41,9 +41,9 @@
 // Options of the walks: an element-wise feature map applied to q, k as they are loaded, with its
 // slope multiplied into dQ, dK (WalkParams::fmap); the normaliser of linear attention and its
 // gradient terms as rank-one additions to the products (WalkParams::denom ...); at D = 128,
-// operands of at most 64 true columns on one side without the MFMAs on their padding (WalkExt), and
-// a result added to what its place in memory holds (WalkParams::accumulate) -- both for a wide
-// q / k evaluated as two 128-column halves.
+// operands of at most 64 true columns on a side without the MFMAs on their padding (WalkExt), and
+// results added to what their place in memory holds (WalkParams::accumulate) -- the second of two passes
+// over a q / k and a v that are both wider than 128 columns.
 //
 // Scheduling.  With one wave per SIMD nothing hides the latency of an LDS read but the wave's own
 // instruction order, and the compiler, short of registers, moves every operand read down to the
@@ -831,11 +831,11 @@ __device__ __forceinline__ void walk_load_state(const float *init, bool transpos
 }
 
 // Entry states in memory, fp32 [D][D] per segment, [bh][seg], in one of three forms that host and
-// kernels tell apart by the number of segments alone:
+// kernels tell apart by the number of segments and, at D = 128, WalkParams::init_is_totals:
 //   * two segments per (b, h): the first segment in walking order starts from zero and the other one
 //     from the one total the totals kernel forms; its two workgroups of a (b, h) add up half of that
 //     segment each, and the two slots hold their partial sums;
-//   * three to walk_sum_on_load_max(D) segments: the slots hold the segments' TOTALS as the totals kernel
+//   * three to walk_sum_on_load_max(D) segments, or with that flag: the slots hold the segments' TOTALS as the totals kernel
 //     wrote them, and a walk adds up the totals of the segments before it (after it, walking in reverse)
 //     as it starts -- a few states of D x D read from L2 per workgroup instead of a scan kernel between
 //     the totals kernel and the walk, whose launch costs more than it computes on plans this small
@@ -843,9 +843,7 @@ __device__ __forceinline__ void walk_load_state(const float *init, bool transpos
 //     against sums on load: 8 to 16 segments, N 4096: B H 40 77 / 68 us, B H 32 69 / 64, forward alone 26.7 / 22.3; 21 segments
 //     equal; 32 and more: forward alone 20.7 / 21.7 (B H 16, N 4096), 21.7 / 28.8 (64 segments), B H 16 N 32768 212 / 215;
 //   * more segments: the slots hold the entry states themselves (walk_scan_kernel).
-// Padded head dims up to 64 only.  At D = 128 a workgroup has its CU to itself and nothing hides the
-// latency of those reads at its start: with four segments the forward walk gained 10 us and the reverse
-// walk, which starts from two such sums, lost 60 (B 4, H 16, N 4096, D_qk 256 as two halves: 0.333 -> 0.384 ms).
+// (At D = 128 a forward walk then writes the entry states it formed, for backward.)
 __host__ __device__ constexpr int walk_sum_on_load_max(int D) { return D <= 64 ? 16 : 0; }
 __host__ __device__ constexpr bool walk_entries_are_totals(int D, int n_seg) {
     return n_seg >= 3 && n_seg <= walk_sum_on_load_max(D);
@@ -1628,8 +1626,9 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 //   X = sum of K^T V over the chunks before it, obtained backwards: X starts as the forward state at
 //   the end of the segment (the next segment's entry state, or the state after the last chunk) and
 //   every chunk's K^T V is subtracted when the walk reaches it.  (In fp32: the difference carries
-//   the rounding of the sums it is taken from, about 1e-7 of the largest state -- far below the
-//   16-bit rounding the state gets before it multiplies dO.)
+//   the rounding of the sums it is taken from, about 1e-7 of the segment's largest state -- below the
+//   16-bit rounding the state gets before it multiplies dO unless the rows so far are some 1e4 times smaller
+//   than later ones; and a late row that is infinite or NaN leaves nothing of it.)
 // The one 16-bit state in LDS holds R for dV and dK, then X for dQ.  q, k, v, dO are read once and
 // nothing but the results is written, where the walk for dQ followed by walk_dkdv_kernel reads
 // dO, v, k twice.

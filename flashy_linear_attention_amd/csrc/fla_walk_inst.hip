@@ -1,7 +1,7 @@
 // Instantiations of the walk kernels (fla_chunk_walk.h) for one storage type (FLA_WALK_DTYPE: 0 bf16, 1 fp16) and one
 // group of kernels (FLA_WALK_PART: 0 totals and forward walks, 1 backward walks), padded head dims 32, 64 and 128
-// (128: backward is one reverse walk when forward handed its states over; otherwise, and with a feature map or
-// the normaliser, dQ is a forward-direction walk and dK, dV a kernel of their own).
+// (128: backward is a forward-direction walk for dQ and a kernel for dK and dV, or one reverse walk where
+// a caller asks for it and forward handed its states over).
 #include "fla_dispatch.h"
 
 namespace fla {
