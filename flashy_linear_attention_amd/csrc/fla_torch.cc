@@ -16,10 +16,13 @@
 #include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/types.h>
 #include <ATen/autocast_mode.h>
+#include <torch/custom_class.h>
 #include <c10/core/DeviceGuard.h>
 #include <c10/hip/HIPStream.h>
 
 #include <tuple>
+#include <utility>
+#include <vector>
 
 #include "fla.h"
 
@@ -188,6 +191,21 @@ variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_,
     return {dq, dk, dv};
 }
 
+// Operands that a node does not keep: backward is refused all the same once one of them was written to in place
+struct Unkept : torch::CustomClassHolder {
+    std::vector<std::pair<c10::VariableVersion, uint32_t>> seen;
+    void add(const Tensor &t) {
+        const c10::VariableVersion &version = t.unsafeGetTensorImpl()->version_counter();
+        if (version.enabled()) seen.emplace_back(version, version.current_version());
+    }
+    void check() const {
+        for (const auto &[version, then] : seen)
+            TORCH_CHECK(version.current_version() == then, "one of the variables needed for gradient computation has been "
+                        "modified by an inplace operation: it is at version ", version.current_version(),
+                        "; expected version ", then, " instead");
+    }
+};
+
 struct Product : Function<Product> {
     static Tensor forward(AutogradContext *ctx, const Tensor &q_, const Tensor &k_, const Tensor &v_, int64_t ev, bool cast) {
         const Casts in(q_, k_, v_, cast);
@@ -202,10 +220,14 @@ struct Product : Function<Product> {
             const int64_t b = q.size(0), h = q.size(1), n = q.size(2);
             if (fla_linear_attn_chunked_state_operands(b, h, n, q.size(3), v.size(3), at, pitch)) {
                 at::AutoDispatchBelowADInplaceOrView below;
+                auto unkept = c10::make_intrusive<Unkept>();
                 for (int i = 0; i < 3; ++i)
-                    if (at[i] >= 0)
+                    if (at[i] >= 0) {
+                        unkept->add(s[i]);
                         s[i] = state.narrow(0, at[i], 2 * b * h * n * pitch[i]).view(q.scalar_type()).view({b, h, n, pitch[i]})
                                    .narrow(3, 0, s[i].size(3));
+                    }
+                ctx->saved_data["unkept"] = c10::IValue::make_capsule(std::move(unkept));
             }
             s.push_back(state);
         }
@@ -214,6 +236,8 @@ struct Product : Function<Product> {
     }
     static variable_list backward(AutogradContext *ctx, variable_list go) {
         const variable_list s = ctx->get_saved_variables();
+        if (const auto unkept = ctx->saved_data.find("unkept"); unkept != ctx->saved_data.end())
+            c10::static_intrusive_pointer_cast<Unkept>(unkept->second.toCapsule())->check();
         variable_list g = product_bwd(go[0], s[0], s[1], s[2], s.size() > 3 ? s[3] : Tensor(), (int)ctx->saved_data["ev"].toInt());
         widen(g, ctx->saved_data["widened"].toInt());
         g.resize(5);

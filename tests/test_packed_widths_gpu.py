@@ -52,3 +52,27 @@ def test_copies_are_kept_in_place_of_the_operands(gpu_device):
     qc, kc, vc = leaves
     LinearAttentionSmallVHD.apply(qc, kc, vc).backward(torch.ones_like(out))
     assert all(torch.equal(a, t.grad) for a, t in zip(grads, leaves))
+
+
+@pytest.mark.parametrize("which", range(3), ids=["q", "k", "v"])
+def test_an_operand_written_to_in_place_is_refused(which, gpu_device):
+    """... as autograd refuses it for an operand that a node keeps, copied or not."""
+    from flashy_linear_attention_amd import LinearAttentionSmallVHD
+
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in reference_style_inputs(1, 2, 1024, 91, 64, torch.bfloat16, seed=5)[:3]]
+    args = [t * 1.0 for t in leaves]
+    out = LinearAttentionSmallVHD.apply(*args)
+    args[which].add_(1.0)
+    with pytest.raises(RuntimeError, match="modified by an inplace operation"):
+        out.sum().backward()
+
+
+def test_saved_tensor_hooks_see_the_copies(gpu_device):
+    from flashy_linear_attention_amd import LinearAttentionSmallVHD
+
+    leaves = [t.to(gpu_device).requires_grad_(True) for t in reference_style_inputs(1, 2, 1024, 91, 64, torch.bfloat16, seed=6)[:3]]
+    want = torch.autograd.grad(LinearAttentionSmallVHD.apply(*leaves).sum(), leaves)
+    with torch.autograd.graph.save_on_cpu():
+        out = LinearAttentionSmallVHD.apply(*leaves)
+    for a, b in zip(torch.autograd.grad(out.sum(), leaves), want):
+        assert torch.equal(a, b)
