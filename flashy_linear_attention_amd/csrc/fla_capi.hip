@@ -525,8 +525,13 @@ int wide_entry_states(const WalkPlan &wp, const View &y, const View &z, int64_t 
 struct WalkNorm {
     float *denom;     // forward: receives n
     float eps;
-    const float *dn;  // backward: dn_i = -(g_i . out_i) / n_i (and the grad_out operand holds g / n)
-    void *vec;        // scratch, 2 * walk_vec_bytes(): zc, rc
+    float *dn;        // backward: dn_i = -(g_i . out_i) / n_i (and the grad_out operand holds g / n)
+    void *vec;        // scratch, 2 * walk_vec_bytes(): the segments' totals of k (forward), zc without a saved one; rc
+    // backward: g, out and n, from which the kernel in front of the walks forms dO and dn beside the segments' totals (where
+    // norm_walks_backward() says that the walks take the call: otherwise they have been formed before it)
+    const View *go, *out;
+    const float *n;
+    bool vec16;       // g and out allow 16-byte loads
     bool fused;       // out: the kernels took the terms (false: the caller runs the passes of fla_norm.h)
     bool dk_pending;  // out: ... all but dK's sum over later rows (and dK's slope, with a feature map)
 };
@@ -536,15 +541,36 @@ int64_t walk_vec_bytes(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv)
     return w.ok ? B * H * w.n_chunks * w.D * 4 : 0;
 }
 
-// out[bh][c] = sum over the rows before (reverse: after) chunk c of w[row] y[row] (w null: y[row])
-int walk_chunk_vectors(const WalkPlan &wp, const View &y, int64_t width, const float *w, int reverse, float *out,
-                       int64_t B, int64_t H, int64_t N, int dtype, hipStream_t s) {
+// zc, the running sum of k at the entry of every chunk, where forward's is not at hand (D = 128)
+int walk_chunk_vectors(const WalkPlan &wp, const View &k, int64_t width, float *out, int64_t B, int64_t H, int64_t N, int dtype,
+                       hipStream_t s) {
     fla::WalkVecParams vp{};
-    vp.y = y.ptr, vp.ys_b = y.strides[0], vp.ys_h = y.strides[1], vp.ys_n = y.strides[2];
-    vp.w = w, vp.H = (int32_t)H, vp.N = (int32_t)N, vp.width = (int32_t)width, vp.n_chunks = (int32_t)wp.n_chunks;
+    vp.y = k.ptr, vp.ys_b = k.strides[0], vp.ys_h = k.strides[1], vp.ys_n = k.strides[2];
+    vp.H = (int32_t)H, vp.N = (int32_t)N, vp.width = (int32_t)width, vp.n_chunks = (int32_t)wp.n_chunks;
     vp.out = out;
-    if (fla::walk_vec_sums(dtype, wp.D, vp, B * H, s) != hipSuccess) return FLA_ERR_LAUNCH;
-    return fla::walk_vec_scan(out, B * H, (int)wp.n_chunks, wp.D, reverse, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
+    if (fla::walk_vec_sums(dtype, vp, B * H, s) != hipSuccess) return FLA_ERR_LAUNCH;
+    return fla::walk_vec_scan(out, B * H, (int)wp.n_chunks, wp.D, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
+}
+
+// dO and dn of the normalised backward with the segments' totals of Q^T dO (to `work`) and of dn_i q_i (to `rc`), and the
+// entry states of the reverse walk from the former where it does not add them up itself (`totals_only`, or by its number of
+// segments).  Returns where the entry states are.
+int walk_grad_entry_states(const WalkPlan &w, const View &q, const View &dout, const WalkNorm &nx, int64_t B, int64_t H, int64_t N,
+                           int64_t dqk, int64_t dv, int dtype, void *work, float *rc_totals, const float **where, bool totals_only,
+                           hipStream_t s) {
+    fla::WalkGradParams gp{};
+    gp.q = q.ptr, gp.qs_b = q.strides[0], gp.qs_h = q.strides[1], gp.qs_n = q.strides[2];
+    gp.go = nx.go->ptr, gp.gs_b = nx.go->strides[0], gp.gs_h = nx.go->strides[1], gp.gs_n = nx.go->strides[2];
+    gp.o = nx.out->ptr, gp.os_b = nx.out->strides[0], gp.os_h = nx.out->strides[1], gp.os_n = nx.out->strides[2];
+    gp.denom = nx.n, gp.dout = const_cast<void *>(dout.ptr), gp.dn = nx.dn, gp.vec = nx.vec16;
+    gp.H = (int32_t)H, gp.N = (int32_t)N, gp.BH = (int32_t)(B * H), gp.wqk = (int32_t)dqk, gp.wv = (int32_t)dv;
+    gp.n_chunks = (int32_t)w.n_chunks, gp.seg_chunks = (int32_t)w.seg_chunks, gp.n_seg = (int32_t)w.n_seg;
+    const bool several = w.n_seg > 1;
+    gp.totals = several ? static_cast<float *>(work) : nullptr, gp.rsum = several ? rc_totals : nullptr;
+    *where = gp.totals;
+    if (fla::walk_grad_totals(dtype, w.D, gp, s) != hipSuccess) return FLA_ERR_LAUNCH;
+    if (w.n_seg <= 2 || totals_only || fla::walk_entries_are_totals(w.D, (int)w.n_seg)) return FLA_OK;
+    return fla::walk_scan(gp.totals, gp.totals, B * H, (int)w.n_seg, w.D, w.D, 1, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 
 bool states_shareable(int64_t dqk, int64_t dv, int64_t N) {
@@ -943,10 +969,10 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         const bool in_state = state_out && wp.split;
         // D = 128, a few segments more than two: the totals go to the workspace, the walk adds them up itself as it starts
         // and writes the entry states it formed to state_out -- no scan launch
-        const bool sum_on_load = wp.split && !fmap && !nx && sums_on_load(wp);
-        if (need_totals && (!in_state || sum_on_load) &&
-            (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < wp.work_bytes))
-            return FLA_ERR_WORKSPACE;
+        // (with a feature map or the normaliser a caller may have brought a state buffer and no workspace: then a scan in the former)
+        const bool has_work = workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= wp.work_bytes;
+        const bool sum_on_load = wp.split && sums_on_load(wp) && ((!fmap && !nx) || !in_state || has_work);
+        if (need_totals && (!in_state || sum_on_load) && !has_work) return FLA_ERR_WORKSPACE;
         if (state_out && reinterpret_cast<uintptr_t>(state_out) % 16 != 0) return FLA_ERR_WORKSPACE;
         hipStream_t s = static_cast<hipStream_t>(stream);
         const float *entry = nullptr;
@@ -1012,6 +1038,15 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
     return FLA_OK;
 }
 
+// whether the walk kernels take the normalised backward of these operands
+bool norm_walks_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
+                         const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, const void *state_in) {
+    const WalkPlan wp = walk_plan(B, H, N, dqk, dv);
+    return wp.ok && (state_in || wp.split) && states_shareable(dqk, dv, N) && fla::fast_path_ok(make_params(go, v, k, dq, B, H, N, dv, dqk, 0)) &&
+           fla::fast_path_ok(make_params(k, q, go, dvv, B, H, N, dqk, dv, 1)) &&
+           fla::fast_path_ok(make_params(v, go, q, dk, B, H, N, dv, dqk, 1));
+}
+
 // `causal` (D_v up to 128): with forward's states at hand, too, dQ comes from a walk in forward direction (and dK, dV from
 // one in reverse), never by subtraction from a later state: nothing of a row reaches the dQ of the chunks before it.
 // Backward at D = 128, one reverse walk against two walks: B H 128, N 4096 274 / 292 us; B H 16, N 4096 53 / 58; B H 256, N 1024
@@ -1070,7 +1105,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
     const int fmap_late = nx ? 0 : fmap;
     const WalkPlan wp = walk_plan(B, H, N, dqk, dv, !fmap && !nx);
     // (what forward saved is in the walks' format; at D = 128 the entry states are cheap to recompute)
-    const bool walk = wp.ok && (state_in || wp.split);
+    const bool walk = wp.ok && (state_in || wp.split);  // (norm_walks_backward: the same)
     // (padded widths that differ: the walks or product by product -- the 256-row chunks share states between equal ones only)
     const bool mixed_walk = walk && pad_index(dqk) != pad_index(dv);
     if ((!states_shareable(dqk, dv, N) && !mixed_walk) || !fla::fast_path_ok(pq) || !fla::fast_path_ok(pv) ||
@@ -1100,7 +1135,8 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         // with forward's states at hand (and without the normaliser): one reverse walk
         const bool one_walk = state_in && !nx && !causal;
         // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
-        const bool rev_sums_on_load = (one_walk || causal) && sums_on_load(wp);
+        const bool rev_sums_on_load = (one_walk || causal || nx) && sums_on_load(wp);
+        float *const rcv = nx ? reinterpret_cast<float *>(static_cast<char *>(nx->vec) + walk_vec_bytes(B, H, N, dqk, dv)) : nullptr;
         if (wp.n_seg > 1) {
             if (!state_in) {
                 const float *fwd_entry = nullptr;
@@ -1109,17 +1145,19 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                     return rc;
                 state_in = fwd_entry;
             }
-            if (int rc = walk_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, workspace, nullptr, &entry, s, 0, nullptr,
-                                           nullptr, rev_sums_on_load))
-                return rc;
+            if (!nx)
+                if (int rc = walk_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, workspace, nullptr, &entry, s, 0, nullptr,
+                                               nullptr, rev_sums_on_load))
+                    return rc;
         }
-        float *zc = nullptr, *rcv = nullptr;
-        if (nx) {  // zc: running sum of k at the entry of every chunk; rc: sum of dn_i q_i over the rows after it
-            zc = static_cast<float *>(nx->vec);
-            rcv = reinterpret_cast<float *>(static_cast<char *>(nx->vec) + walk_vec_bytes(B, H, N, dqk, dv));
-            if (int rc = walk_chunk_vectors(wp, q, dqk, nx->dn, 1, rcv, B, H, N, dtype, s)) return rc;
-            if (zc_saved) zc = const_cast<float *>(zc_saved);
-            else if (int rc = walk_chunk_vectors(wp, k, dqk, nullptr, 0, zc, B, H, N, dtype, s)) return rc;
+        const float *zc = zc_saved;  // (running sum of k at the entry of every chunk)
+        if (nx) {
+            if (int rc = walk_grad_entry_states(wp, q, go, *nx, B, H, N, dqk, dv, dtype, workspace, rcv, &entry, rev_sums_on_load, s))
+                return rc;
+            if (!zc) {
+                if (int rc = walk_chunk_vectors(wp, k, dqk, static_cast<float *>(nx->vec), B, H, N, dtype, s)) return rc;
+                zc = static_cast<const float *>(nx->vec);
+            }
         }
         if (one_walk) {
             fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv);
@@ -1159,7 +1197,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
         r.init = entry, r.fmap = fmap;  // (dK: the slope from phi(xk) in the K tile)
         r.init_is_totals = rev_sums_on_load;
-        if (nx) r.dn = nx->dn, r.rc = rcv;  // dK's terms
+        if (nx) r.dn = nx->dn, r.rc = wp.n_seg > 1 ? rcv : nullptr;  // dK's terms
         return fla::walk_dkdv(dtype, wp.D, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
     if (walk) {  // (the states forward saved are per 128-row chunk: only this path reads them)
@@ -1169,9 +1207,15 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         if (reinterpret_cast<uintptr_t>(state_in) % 16 != 0) return FLA_ERR_WORKSPACE;
         hipStream_t s = static_cast<hipStream_t>(stream);
         const float *entry = nullptr;
-        if (wp.n_seg > 1)
+        if (wp.n_seg > 1 && !nx)
             if (int rc = walk_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, workspace, nullptr, &entry, s)) return rc;
         fla::WalkParams w{};
+        if (nx) {
+            float *const rcv = reinterpret_cast<float *>(static_cast<char *>(nx->vec) + walk_vec_bytes(B, H, N, dqk, dv));
+            if (int rc = walk_grad_entry_states(wp, q, go, *nx, B, H, N, dqk, dv, dtype, workspace, rcv, &entry, false, s)) return rc;
+            w.dn = nx->dn, w.zc = zc_saved, w.rc = wp.n_seg > 1 ? rcv : nullptr;
+            nx->fused = true;
+        }
         w.fmap = fmap;  // q, k hold phi(x): the slopes come from the LDS tiles
         w.q = q.ptr, w.k = k.ptr, w.v = v.ptr, w.go = go.ptr;
         w.dq = const_cast<void *>(dq.ptr), w.dk = const_cast<void *>(dk.ptr), w.dv = const_cast<void *>(dvv.ptr);
@@ -1186,15 +1230,6 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = entry;
         w.saved = const_cast<void *>(state_in);
-        if (nx) {
-            const int64_t vb = walk_vec_bytes(B, H, N, dqk, dv);
-            float *zc = static_cast<float *>(nx->vec), *rcv = reinterpret_cast<float *>(static_cast<char *>(nx->vec) + vb);
-            if (zc_saved) zc = const_cast<float *>(zc_saved);
-            else if (int rc = walk_chunk_vectors(wp, k, dqk, nullptr, 0, zc, B, H, N, dtype, s)) return rc;
-            if (int rc = walk_chunk_vectors(wp, q, dqk, nx->dn, 1, rcv, B, H, N, dtype, s)) return rc;
-            w.dn = nx->dn, w.zc = zc, w.rc = rcv;
-            nx->fused = true;
-        }
         return fla::walk_bwd(dtype, wp.D, w, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
     if (wp.ok) state_in = nullptr;  // not in the 256-row chunks' format: recomputed below
@@ -1552,7 +1587,8 @@ int normalised_forward(const View &q0, const View &k0, const View &v, const View
     }
     // chunk-wise walk kernels compute n and divide by it themselves
     WalkNorm nx{denom, eps, nullptr,
-                workspace ? static_cast<char *>(workspace) + l.do_bytes + l.dn_bytes + 2 * l.sums_bytes : nullptr, false, false};
+                workspace ? static_cast<char *>(workspace) + l.do_bytes + l.dn_bytes + 2 * l.sums_bytes : nullptr,
+                nullptr, nullptr, nullptr, false, false, false};
     const View &q = fmap ? mapped[0] : q0, &k = fmap ? mapped[1] : k0;
     if (!chunked) {
         const int rc = fused_normalised_forward(q, k, v, o, denom, B, H, N, dqk, dv, eps, dtype, stream);
@@ -1610,13 +1646,14 @@ int normalised_backward(const View &go, const View &q, const View &k, const View
     fla::NormParams p;
     norm_common(p, q, k, B, H, N, dqk, dv, l);
     p.denom = const_cast<float *>(denom), p.dn = dn, p.ksum = ksum, p.wsum = wsum;
-    // dO = g / n, dn = -(g . out) / n
+    // dO = g / n, dn = -(g . out) / n: by the first kernel of the walks where they take the call, else by a pass of its own
     p.a = go.ptr, p.as_b = go.strides[0], p.as_h = go.strides[1], p.as_n = go.strides[2], p.vec_a = vec_ok(go, dv);
     p.b = o.ptr, p.bs_b = o.strides[0], p.bs_h = o.strides[1], p.bs_n = o.strides[2], p.vec_b = vec_ok(o, dv);
     p.out = dO, p.os_b = do_strides[0], p.os_h = do_strides[1], p.os_n = do_strides[2], p.vec_out = vec_ok(dOv, dv);
-    if (norm_launch(1, dtype, l.lpr, p, stream) != hipSuccess) return FLA_ERR_LAUNCH;
+    const bool walks = chunked && norm_walks_backward(dOv, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, state_in);
+    if (!walks && norm_launch(1, dtype, l.lpr, p, stream) != hipSuccess) return FLA_ERR_LAUNCH;
     // gradients of the unnormalised product
-    WalkNorm nx{nullptr, 0.f, dn, ws + l.do_bytes + l.dn_bytes + 2 * l.sums_bytes, false, false};
+    WalkNorm nx{nullptr, 0.f, dn, ws + l.do_bytes + l.dn_bytes + 2 * l.sums_bytes, &go, &o, denom, p.vec_a && p.vec_b, false, false};
     if (chunked) {
         // the walk kernels add the normaliser's terms (and apply the slope of a feature map) themselves
         if (int rc = chunked_backward(dOv, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, ws + l.norm_bytes,

@@ -90,7 +90,7 @@ struct WalkParams {
     const float *init;
     int32_t init_transposed;
     // forward, D <= 64: where the 16-bit state at the entry of every chunk goes, [BH][n_chunks][D][D], or null; backward:
-    // the same buffer, read for dQ.  Laid out as its copy in LDS (unscaled); with the normaliser [q/k index][v index].
+    // the same buffer, read for dQ.  Laid out as its copy in LDS (unscaled).
     void *saved;
     // Feature map (fla_feature.h), 0: none.  Forward: q holds the argument xq of the map phi; the Q
     // tile is mapped in LDS as it lands and phi(xq) is written to qmap_out (q's shape, element
@@ -108,16 +108,17 @@ struct WalkParams {
     // The normaliser n_i = q_i . (k_0 + ... + k_i) + eps fused into the walks (null pointers: off).
     // Forward (denom): n_i = sum of row i's masked scores + q_i . zc_c, with zc_c carried by the walk beside the
     // state (walk_col_sums; vsum: the segments' totals of k from the totals kernel, null with a single segment) and
-    // written to zc_out (null: nowhere) for backward; the result is divided by n_i and n goes to denom.  Backward, with dn_i = -(g_i . out_i) / n_i and dO = g / n prepared by
-    // the caller: dQ's scores get + dn_i and its result + dn_i zc_c (dn, zc); dK's scores get + dn_i
-    // (i: the dO row) and its result + rc_c (dn, rc).
+    // written to zc_out (null: nowhere) for backward; the result is divided by n_i and n goes to denom.  Backward, with
+    // dn_i = -(g_i . out_i) / n_i and dO = g / n from walk_grad_totals_kernel: dQ's scores get + dn_i and its result
+    // + dn_i zc_c (dn, zc); dK's scores get + dn_i (i: the dO row) and its result + rc_c, the sum of dn_i q_i over the rows
+    // after chunk c, carried by the walk beside R (rc: the segments' totals of dn_i q_i, null with a single one).
     float *denom;     // fp32 [BH][N]
     float eps;
     const float *zc;  // fp32 [BH][n_chunks][D]: sum of k over the rows before chunk c (backward)
     const float *vsum;  // fp32 [BH][n_seg][D], slots as those of `init` (two segments: partial sums in both)
     float *zc_out;      // as zc
     const float *dn;  // fp32 [BH][N]
-    const float *rc;  // fp32 [BH][n_chunks][D]: sum of dn_i q_i over the rows after chunk c
+    const float *rc;  // fp32 [BH][n_seg][D], slots as those of `init`
     // Forward, D = 128: where the state after the last chunk of every (b, h) goes, fp32 [BH][D][D]
     // ([q/k index][v index]), or null.  walk_bwd_rev_kernel: that buffer (xtotal) and forward's entry
     // states (xinit, the layout of `init`, not transposed; may be null with a single segment).
@@ -136,7 +137,7 @@ struct WalkParams {
     // init_is_totals (every D = 128 walk; three segments or more): init (and init2) hold the segments' TOTALS as the
     // totals kernel wrote them, and a workgroup adds up those of the segments before its own (after it, walking in
     // reverse) as it starts, several loads in flight together -- no scan launch between the totals kernel and the
-    // walk.  The forward walks (walk_fwd_kernel's plain D = 128 variant, walk_fwd_wide_kernel) then write the entry
+    // walk.  The forward walks (walk_fwd_kernel at D = 128, walk_fwd_wide_kernel) then write the entry
     // state they formed to entry_out / entry_out2 (the layout of init; null: nowhere), for the backward walk.
     int32_t init_is_totals;
     float *entry_out, *entry_out2;
@@ -158,7 +159,7 @@ struct WalkCfg {
     static constexpr int RPI = 1024 / RB;   // rows covered by one wave-level 1 KiB load
     static constexpr int NI = TILE / 4096;  // such loads per wave and tile
     static constexpr int STATE = D * RB;    // the 16-bit state in LDS
-    static constexpr int VEC = 3 * 1024;    // per set of tiles: zc, rc, dn of the chunk (fp32, 1 KiB each)
+    static constexpr int VEC = 3 * 1024;    // per set of tiles: zc, rc (walk_bwd_kernel), dn of the chunk (fp32, 1 KiB each)
     static constexpr int NID = C / 64;      // wave-level 256-byte loads of a chunk's dn
     static constexpr int NBLK = DB * DB;    // 32 x 32 blocks of the state: block b belongs to wave b % 4
     static constexpr int NBW = (NBLK + 3) / 4;  // state blocks per wave
@@ -706,6 +707,52 @@ __device__ __forceinline__ float walk_col_sum_of(const float *part, int col) {
     return t;
 }
 
+// this lane's part of the column sums of the tile's rows times w (fp32 in LDS, one value per row): the rows
+// R0 + {4g .., 8 + 4g ..} of the steps ks of this wave, of column 32 (wave % DB) + l32.  In fp32 throughout: the fragments
+// are the ones an MFMA would take, but w would have to be rounded for it.
+template <typename T, int D>
+__device__ __forceinline__ float walk_weighted_sums(const unsigned char *yt, const float *w, int wave, int lane) {
+    using W = WalkCfg<D>;
+    using V8 = typename Mma<T>::V8;
+    constexpr int KS = W::C / 16 / (4 / W::DB);  // 16-row steps per wave
+    const int g = lane >> 5;
+    float sum = 0.f;
+    static_for<0, KS>([&](auto j) {
+        const int ks = (wave / W::DB) * KS + decltype(j)::value;
+        const V8 y = walk_col_frag<T, D>(yt, 16 * ks, wave % W::DB, lane);
+#pragma unroll
+        for (int a = 0; a < 2; ++a) {
+            const f32x4 wv = *reinterpret_cast<const f32x4 *>(w + 16 * ks + 8 * a + 4 * g);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) sum += wv[b] * static_cast<float>(y[4 * a + b]);
+        }
+    });
+    return sum;
+}
+// ... to LDS, in the layout of walk_col_sums_to_lds
+template <int D>
+__device__ __forceinline__ void walk_weighted_sums_to_lds(float *part, int wave, int lane, float sum) {
+    constexpr int DB = D / 32;
+    sum += __shfl_xor(sum, 32, 64);
+    if (lane < 32) part[(wave / DB) * D + 32 * (wave % DB) + lane] = sum;
+}
+
+// x as the sum of three bf16 numbers (its 24 significant bits; what is not finite in the first alone), in the k slots 0 .. 2 of
+// an MFMA's A operand whose row is this lane's l32; walk_ones3 is the B operand that adds them up.  One MFMA then adds x to
+// a row of an accumulator, where handing it round within the wave takes a ds_bpermute per register.
+__device__ __forceinline__ Mma<__bf16>::V8 walk_split3(float x, int g) {
+    uint32_t hi = __builtin_bit_cast(uint32_t, x) & 0xffff0000u;
+    if (x != x) hi = 0x7fc00000u;
+    const float r1 = (hi & 0x7f800000u) == 0x7f800000u ? 0.f : x - __builtin_bit_cast(float, hi);
+    const uint32_t mid = __builtin_bit_cast(uint32_t, r1) & 0xffff0000u;
+    const float r2 = r1 - __builtin_bit_cast(float, mid);
+    const u32x4 w = {g ? 0u : (hi >> 16) | mid, g ? 0u : __builtin_bit_cast(uint32_t, r2) >> 16, 0u, 0u};
+    return __builtin_bit_cast(Mma<__bf16>::V8, w);
+}
+__device__ __forceinline__ Mma<__bf16>::V8 walk_ones3(int g) {
+    return __builtin_bit_cast(Mma<__bf16>::V8, u32x4{g ? 0u : 0x3f803f80u, g ? 0u : 0x3f80u, 0u, 0u});
+}
+
 // the state rounded to 16 bit into LDS as T[v index][q/k index] (row = 32 eb + l32, four consecutive
 // columns per register group), in the tile layout
 template <typename T, int D, typename B = WalkExt<D>>
@@ -1031,7 +1078,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
 
     f32x16 st[W::NBW];
     walk_load_init<D, B>(p, sl, wave, lane, st, false);
-    if constexpr (DOUBLE && NORM == 0 && !FM) {  // (the entry state this walk formed from the segments' totals, for backward)
+    if constexpr (DOUBLE && NORM <= 1) {  // (the entry state this walk formed from the segments' totals, for backward)
         if (p.init_is_totals && p.entry_out && sl.seg > 0)
             walk_write_state<D, B>(p.entry_out + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D), wave, lane, st);
     }
@@ -1136,7 +1183,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                 __syncthreads();
             }
         }
-        if constexpr (!DOUBLE && NORM == 0) {
+        if constexpr (!DOUBLE && NORM <= 1) {
             if (p.saved && c > 0) {  // the state's copy for backward's dQ (at the first chunk it is zero and not read)
                 unsigned char *sv = static_cast<unsigned char *>(p.saved) + ((int64_t)sl.bh * p.n_chunks + c) * W::STATE;
                 for (int i = tid * 16; i < W::STATE; i += 4096) {
@@ -1180,17 +1227,6 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
             });
         }
         walk_store<T, D, OB::PER>(ro, os2, p.wv, row, g, db0, acc);
-        if (!DOUBLE && NORM == 1 && p.saved) {  // the state at the entry of this chunk, [q/k index][v index], for backward's dQ
-            T *sv = static_cast<T *>(p.saved) + ((int64_t)sl.bh * p.n_chunks + c) * (D * D);
-#pragma unroll
-            for (int i = 0; i < B::SLOTS; ++i)
-                if (B::valid(wave, i)) {
-#pragma unroll
-                    for (int v = 0; v < 16; ++v)
-                        sv[(32 * B::dbk(wave, i) + 8 * (v / 4) + 4 * g + (v % 4)) * D + 32 * B::eb(wave) + l32] =
-                            static_cast<T>(st[i][v]);
-                }
-        }
         walk_update<T, D, B>(tk, tv, wave, lane, st);
         if constexpr (SCALED) walk_state_max<D, B>(smax, wave, lane, st);
         if constexpr (NORM == 1) {
@@ -1359,8 +1395,9 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
 
 // ---- backward: dQ, dV, dK of a chunk from one set of tiles; R += Q_c^T dO_c, chunks descending.
 // dQ's state, the sum of K^T V over the chunks before: the 16-bit copy forward saved at the entry of every chunk
-// (WalkParams::saved), brought to LDS with the chunk's tiles; NORM (the normaliser's terms, whose vectors take that
-// place in LDS): fragments straight from memory.
+// (WalkParams::saved), brought to LDS with the chunk's tiles.  With the normaliser's terms (NORM), whose vectors leave room for
+// one state: dQ first, then R in its place, for two barriers more.  (dQ's state as fragments straight from memory, which
+// forward then wrote element by element, spilled 64 bytes a lane: B H 64, N 4096, D 64 71 us, this way 59.)
 // (Obtained backwards instead -- from the state at the segment's end, subtracting every chunk's K^T V when the walk reaches
 // it -- one late row that is infinite, NaN or merely huge spoiled the dQ of every chunk before it.  Forward + backward
 // at B H 16, N 32768, D 64 that way 222 us, this way 234.)
@@ -1375,7 +1412,9 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
     unsigned char *tq = smem, *tk = smem + W::TILE, *tv = smem + 2 * W::TILE, *tg = smem + 3 * W::TILE,
                   *tl = smem + 4 * W::TILE;
     unsigned char *tx = tl + W::STATE;  // (!NORM) dQ's state; (NORM) the chunk's vectors
-    const float *vz = reinterpret_cast<const float *>(tl + W::STATE), *vr = vz + 256, *vd = vz + 512;
+    // (NORM: zc, rc, dn of the chunk, and the waves' parts of rc's next term)
+    const float *vz = reinterpret_cast<const float *>(tl + W::STATE), *vd = vz + 512;
+    float *vr = reinterpret_cast<float *>(tl + W::STATE) + 256, *rpart = vr + 512;
     const uint32_t xbase = lds0 + 4 * W::TILE + W::STATE;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1401,7 +1440,25 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 
     f32x16 st[W::NBW];  // R[q/k index][v index]
     walk_load_init<D>(p, sl, wave, lane, st, true);
-    walk_state_to_lds<T, D>(tl, wave, lane, st);
+    if constexpr (!NORM) walk_state_to_lds<T, D>(tl, wave, lane, st);
+    float rrun = 0.f;  // NORM: rc (of column tid, tid < D); at the segment's entry from the segments' totals, as zc in forward
+    if constexpr (NORM) {
+        constexpr int G = 256 / D;
+        float t = 0.f;
+        if (p.rc) {
+            const float *rs = p.rc + (int64_t)sl.bh * p.n_seg * D + tid % D;
+            const int lo = p.n_seg == 2 ? (sl.seg ? 2 : 0) : sl.seg + 1;
+#pragma unroll 8
+            for (int f = lo + tid / D; f < p.n_seg; f += G) t += rs[(int64_t)f * D];
+        }
+        rpart[tid] = t;
+        __syncthreads();
+        if (tid < D) {
+#pragma unroll
+            for (int u = 0; u < G; ++u) rrun += rpart[u * D + tid];
+            vr[tid] = rrun;
+        }
+    }
 
 #pragma unroll 1
     for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
@@ -1411,28 +1468,13 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
         walk_load_tile<D>(rk, lds0 + W::TILE, row0, ks2, p.wqk, wave, lane);
         walk_load_tile<D>(rv, lds0 + 2 * W::TILE, row0, vs2, p.wv, wave, lane);
         walk_load_tile<D>(rg, lds0 + 3 * W::TILE, row0, gs2, p.wv, wave, lane);
-        if constexpr (NORM) {  // the normaliser's terms: zc, rc of this chunk and its rows of dn
+        if constexpr (NORM) {  // the normaliser's terms: zc of this chunk and its rows of dn
             walk_load_vec<D>(p.zc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase, lane);
-            walk_load_vec<D>(p.rc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase + 1024, lane);
             walk_load_rows<D>(p.dn + (int64_t)sl.bh * N, row0, N, xbase + 2048, lane);
-        } else if (c > 0) {
-            walk_load_state_copy<D>(static_cast<const unsigned char *>(p.saved) + at * W::STATE, xbase, wave, lane);
         }
-        // NORM: dQ's state, S_c[q/k index][v index] as saved by forward: A-operand fragments straight from
-        // memory (row = output column of dQ, eight consecutive v indices)
-        V8 sfq[NORM ? W::DB : 1][NORM ? W::KC : 1];
-        if constexpr (NORM) {
-            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
-                static_cast<T *>(p.saved) + at * (D * D), 0, D * D * 2, 0x00020000);
-            if (c > 0) {
-#pragma unroll
-                for (int db = 0; db < W::DB; ++db)
-#pragma unroll
-                    for (int kc = 0; kc < W::KC; ++kc)
-                        sfq[db][kc] = __builtin_bit_cast(V8, __builtin_amdgcn_raw_buffer_load_b128(
-                                                                 rs, (uint32_t)(((32 * db + walk_e_lane(l32)) * D + 16 * kc + 8 * g) * 2), 0, 0));
-            }
-        }
+        if (c > 0)
+            walk_load_state_copy<D>(static_cast<const unsigned char *>(p.saved) + at * W::STATE, NORM ? lds0 + 4 * W::TILE : xbase, wave,
+                                    lane);
         wait_vm<0>();
         __syncthreads();
         const int row = row0 + 32 * wave + l32;
@@ -1441,10 +1483,14 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
         if constexpr (NORM) {
             // dQ = lower(dO V^T) K + dO S_c^T  (normaliser: scores + dn_i, result + dn_i zc)
             float ax = vd[32 * wave + l32];
-            walk_product<T, D, false, 2>(tg, tv, tk, wave, lane, c > 0, [&](int db, int kc) -> V8 { return sfq[db][kc]; },
-                                         acc, &ax);
+            walk_product<T, D, false, 2>(tg, tv, tk, wave, lane, c > 0, [&](int db, int kc) -> V8 {
+                return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
+            }, acc, &ax);
             walk_add_vec<D>(acc, ax, vz, 0, g);
             walk_store<T, D>(rdq, dqs2, p.wqk, row, g, 0, acc, p.fmap, tq, 32 * wave + l32);
+            __syncthreads();  // every wave has read dQ's state
+            walk_state_to_lds<T, D>(tl, wave, lane, st);
+            __syncthreads();
         }
         // dV = upper(K Q^T) dO + K R: A operand R^T[v index][q/k index] = the LDS copy as it is
         walk_product<T, D, true>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
@@ -1474,8 +1520,16 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
             walk_store<T, D>(rdq, dqs2, p.wqk, row, g, 0, acc, p.fmap, tq, 32 * wave + l32);
         }
         walk_update<T, D>(tq, tg, wave, lane, st);
+        if constexpr (NORM) walk_weighted_sums_to_lds<D>(rpart, wave, lane, walk_weighted_sums<T, D>(tq, vd, wave, lane));
         __syncthreads();
-        walk_state_to_lds<T, D>(tl, wave, lane, st);
+        if constexpr (!NORM) {
+            walk_state_to_lds<T, D>(tl, wave, lane, st);
+        } else {
+            if (tid < D) {
+                rrun += walk_col_sum_of<D>(rpart, tid);
+                vr[tid] = rrun;
+            }
+        }
     }
 #else
     (void)p;
@@ -1485,11 +1539,10 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 // ---- backward without saved per-chunk states, dV and dK: chunks descending, R += Q_c^T dO_c.  One
 // workgroup per CU with two sets of tiles: the loads of the next chunk are in flight while this
 // one is multiplied.  (dQ is a walk_fwd_kernel launch over dO, V, K.)
-// NORM: dK with the normaliser's terms (scores + dn_i, i the dO row; result + rc).  Tiles and state
-// fill the LDS at D = 128, so the chunk's dn and this wave's columns of rc travel in registers: a
-// lane loads one value of each, a chunk ahead, and the values are handed round within the wave
-// (ds_bpermute: 64 per chunk, about 30 clocks each -- 28 us of a 207 us launch at B H = 128,
-// N = 4096) when the chunk's turn comes.
+// NORM: dK with the normaliser's terms (scores + dn_i, i the dO row; result + rc).  Tiles and state fill the LDS at
+// D = 128, so the chunk's dn comes as ordinary loads, a chunk ahead, in the order in which the scores' registers take it, and
+// rc is carried in registers: a wave adds up its own output columns, in the order of an MFMA's A rows, and one MFMA
+// per 32 columns adds rc to the result (walk_split3).
 template <typename T, int D, bool NORM, int NQ = D / 32, int NV = D / 32>
 __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1541,18 +1594,33 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
     // in front of the first use is one for every outstanding load and store (it cannot count past
     // stores), and at that point nothing is in flight that the walk would not wait for anyway but the
     // previous chunk's stores, issued two products earlier.
-    float nxt_dn = 0.f, nxt_rc = 0.f;
-    // (rows past the end read as zero; without the normaliser the two descriptors are never used)
-    const __amdgpu_buffer_rsrc_t rs_dn =
-        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(NORM ? p.dn + (int64_t)sl.bh * N : nullptr), 0, NORM ? N * 4 : 0, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rs_rc = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<float *>(NORM ? p.rc + (int64_t)sl.bh * p.n_chunks * D : nullptr), 0, NORM ? p.n_chunks * D * 4 : 0, 0x00020000);
-    auto load_vecs = [&](int c) {  // lane l: dn of row l of chunk c, rc of column 32 db0 + l
+    f32x4 nxt_dn[8];
+    // (whole groups of four rows: up to three values past the sequence's end, of the next head or of the scratch behind dn, are
+    // read and dropped below; groups past the end read as zero.  Without the normaliser the descriptor is never used)
+    const __amdgpu_buffer_rsrc_t rs_dn = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<float *>(NORM ? p.dn + (int64_t)sl.bh * N : nullptr), 0, NORM ? (N + 3) / 4 * 16 : 0, 0x00020000);
+    auto load_vecs = [&](int c) {  // dn of rows 8 a + 4 g .. of chunk c
         if constexpr (NORM) {
-            nxt_dn = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_dn, (c * W::C + lane) * 4, 0, 0));
-            nxt_rc = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rs_rc, (c * D + 32 * db0 + lane) * 4, 0, 0));
+#pragma unroll
+            for (int a = 0; a < 8; ++a)
+                nxt_dn[a] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rs_dn, (c * W::C + 8 * a + 4 * g) * 4, 0, 0));
         }
     };
+    // rc of column 32 (db0 + i) + walk_e_lane(l32), at the segment's entry from the segments' totals: the part of every other
+    // row (g) or segment that this lane adds up -- the lane of the other g holds the rest
+    float rrun[W::DBW];
+#pragma unroll
+    for (int i = 0; i < W::DBW; ++i) rrun[i] = 0.f;
+    if constexpr (NORM) {
+        if (p.rc) {
+            const float *rs = p.rc + (int64_t)sl.bh * p.n_seg * D + 32 * db0 + walk_e_lane(l32);
+            const int lo = p.n_seg == 2 ? (sl.seg ? 2 : 0) : sl.seg + 1;
+#pragma unroll 4
+            for (int f = lo + g; f < p.n_seg; f += 2)
+#pragma unroll
+                for (int i = 0; i < W::DBW; ++i) rrun[i] += rs[(int64_t)f * D + 32 * i];
+        }
+    }
     load_chunk(sl.c_hi - 1, 0);
     load_vecs(sl.c_hi - 1);
 #pragma unroll 1
@@ -1560,20 +1628,19 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         const int buf = (sl.c_hi - 1 - c) & 1;
         unsigned char *tq = smem + buf * 4 * W::TILE, *tk = tq + W::TILE, *tv = tq + 2 * W::TILE, *tg = tq + 3 * W::TILE;
         const bool more = c > sl.c_lo;
-        // this chunk's vectors, from the lanes that loaded them: dnv[a][b] = dn of tile row 8 a + 4 g + b,
-        // rcv[i][v] = rc of column 32 (db0 + i) + 16 g + v
-        f32x4 dnv[8];
-        f32x16 rcv[W::DBW];
+        f32x4 dnv[8];  // dn of tile rows 8 a + 4 g ..
         if constexpr (NORM) {
 #pragma unroll
-            for (int a8 = 0; a8 < 8; ++a8)
+            for (int a = 0; a < 8; ++a) {
+                dnv[a] = nxt_dn[a];
+                asm volatile("" : "+v"(dnv[a])::"memory");  // (awaited before the tile loads below)
+            }
+            if ((c + 1) * W::C > N) {
 #pragma unroll
-                for (int b4 = 0; b4 < 4; ++b4) dnv[a8][b4] = __shfl(nxt_dn, 8 * a8 + 4 * g + b4, 64);
+                for (int a = 0; a < 8; ++a)
 #pragma unroll
-            for (int i = 0; i < W::DBW; ++i)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) rcv[i][v] = __shfl(nxt_rc, 32 * i + 16 * g + v, 64);
-            asm volatile("" ::"v"(dnv[7]), "v"(rcv[W::DBW - 1]) : "memory");  // (handed round before the tile loads below)
+                    for (int b4 = 0; b4 < 4; ++b4) dnv[a][b4] = c * W::C + 8 * a + 4 * g + b4 < N ? dnv[a][b4] : 0.f;
+            }
         }
         if (more) load_chunk(c - 1, buf ^ 1);  // (every wave has left the barrier that ended the reads of that set)
         // this wave's loads of chunk c have landed when at most the loads issued after them are
@@ -1601,8 +1668,10 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
             walk_product<T, D, true, 3>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
                 return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
             }, acc, nullptr, nullptr, [&](int s, int a4) -> f32x4 { return s == 0 ? dnv[a4] : dnv[4 + a4]; });
+            const Mma<__bf16>::V8 ones = walk_ones3(g);
 #pragma unroll
-            for (int i = 0; i < W::DBW; ++i) acc[i] += rcv[i];
+            for (int i = 0; i < W::DBW; ++i)
+                acc[i] = Mma<__bf16>::mma(walk_split3(rrun[i] + __shfl_xor(rrun[i], 32, 64), g), ones, acc[i]);
         } else {
             walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
                 return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
@@ -1610,6 +1679,17 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         }
         walk_store<T, D, OQ::PER>(rdk, dks2, p.wqk, row, g, db0, acc, p.fmap, tk, 32 * rb + l32);
         walk_update<T, D, B>(tq, tg, wave, lane, st);
+        if constexpr (NORM) {  // rc += this chunk's dn_i q_i
+            static_for<0, W::C / 16>([&](auto j) {
+                constexpr int ks = decltype(j)::value;
+#pragma unroll
+                for (int i = 0; i < W::DBW; ++i) {
+                    const V8 y = walk_col_frag_perm<T, D>(tq, 16 * ks, db0 + i, lane, false);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) rrun[i] += dnv[2 * ks + e / 4][e % 4] * static_cast<float>(y[e]);
+                }
+            });
+        }
         asm volatile("" ::: "memory");
         __builtin_amdgcn_s_waitcnt(0xc07f);  // this wave's LDS reads of the tiles and of the state are done
         __builtin_amdgcn_s_barrier();
@@ -2164,13 +2244,11 @@ __global__ __launch_bounds__(256) void walk_scan_kernel(const float *totals, flo
     *reinterpret_cast<f32x2 *>(pe) = run;  // the last segment in walking order: its own total is not needed
 }
 
-// ---- per-chunk column sums for the normaliser's running vectors: out[bh][c][col] = sum over the
-// rows of chunk c of w[row] y[row][col] (w null: plain sums); fp32.  A scan over the chunks
-// (walk_vec_scan_kernel) then gives zc (y = k, prefix) or rc (y = q, w = dn, suffix).
+// ---- per-chunk column sums: out[bh][c][col] = sum over the rows of chunk c of y[row][col]; fp32.  A scan over the chunks
+// (walk_vec_scan_kernel) then gives zc where forward's is not at hand (a backward at D = 128 without forward's state).
 struct WalkVecParams {
     const void *y;
     int64_t ys_b, ys_h, ys_n;
-    const float *w;  // [BH][N] or null
     int32_t H, N, width, n_chunks;
     float *out;      // [BH][n_chunks][D]
 };
@@ -2193,9 +2271,8 @@ __global__ __launch_bounds__(256) void walk_vec_sums_kernel(const WalkVecParams 
             const int row = c * W::C + r;
             if (row < p.N) {
                 const V8 y = __builtin_bit_cast(V8, *reinterpret_cast<const u32x4 *>(Y + (int64_t)row * p.ys_n + pos * 8));
-                const float w = p.w ? p.w[(int64_t)bh * p.N + row] : 1.0f;
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[e] += w * static_cast<float>(y[e]);
+                for (int e = 0; e < 8; ++e) acc[e] += static_cast<float>(y[e]);
             }
         }
     }
@@ -2210,26 +2287,24 @@ __global__ __launch_bounds__(256) void walk_vec_sums_kernel(const WalkVecParams 
     }
 }
 
-// ---- exclusive prefix (reverse: suffix) sums over the chunks of the vectors above, in place:
-// v[bh][c][col] <- sum of v[bh][c'][col] over c' < c (c' > c).  There are few columns and many
+// ---- exclusive prefix sums over the chunks of the vectors above, in place: v[bh][c][col] <- sum of v[bh][c'][col] over
+// c' < c.  There are few columns and many
 // chunks, so the chunks of a (b, h) are split over sixteen thread groups: each adds up its range,
 // the ranges' sums are scanned in LDS, and each group writes its range's running sums.
 // (a template only so that the header can be included by several translation units)
 template <int kUnused = 0>
-__global__ __launch_bounds__(256) void walk_vec_scan_kernel(float *v, int n_chunks, int D, int reverse) {
+__global__ __launch_bounds__(256) void walk_vec_scan_kernel(float *v, int n_chunks, int D) {
     __shared__ float part[16][16];
     const int j = threadIdx.x & 15, grp = threadIdx.x >> 4;  // column within the block's 16, range of chunks
     const int bh = blockIdx.y, col = blockIdx.x * 16 + j;
     const int per = (n_chunks + 15) / 16;
     float *base = v + (int64_t)bh * n_chunks * D + col;
-    // walking order: position t = 0 .. n_chunks - 1 is chunk t, or chunk n_chunks - 1 - t in reverse
     const int t0 = grp * per, t1 = t0 + per < n_chunks ? t0 + per : n_chunks;
-    auto chunk_of = [&](int t) { return reverse ? n_chunks - 1 - t : t; };
     float sum = 0.f;
     for (int t = t0; t < t1; t += 8) {
         float x[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = t + u < t1 ? base[(int64_t)chunk_of(t + u) * D] : 0.f;
+        for (int u = 0; u < 8; ++u) x[u] = t + u < t1 ? base[(int64_t)(t + u) * D] : 0.f;
 #pragma unroll
         for (int u = 0; u < 8; ++u) sum += x[u];
     }
@@ -2240,26 +2315,200 @@ __global__ __launch_bounds__(256) void walk_vec_scan_kernel(float *v, int n_chun
     for (int t = t0; t < t1; t += 8) {
         float x[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) x[u] = t + u < t1 ? base[(int64_t)chunk_of(t + u) * D] : 0.f;
+        for (int u = 0; u < 8; ++u) x[u] = t + u < t1 ? base[(int64_t)(t + u) * D] : 0.f;
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             if (t + u < t1) {
-                base[(int64_t)chunk_of(t + u) * D] = run;
+                base[(int64_t)(t + u) * D] = run;
                 run += x[u];
             }
     }
 }
 
-inline hipError_t launch_walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, int reverse, hipStream_t stream) {
+inline hipError_t launch_walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, hipStream_t stream) {
     if (BH > 65535 || D % 16 != 0) return hipErrorInvalidConfiguration;
     return launch_kernel<walk_vec_scan_kernel<0>>(dim3((unsigned)(D / 16), (unsigned)BH), dim3(256), 0, stream, v, n_chunks,
-                         D, reverse);
+                         D);
 }
 
 template <typename T, int D>
 hipError_t launch_walk_vec_sums(const WalkVecParams &p, int64_t BH, hipStream_t stream) {
     if (BH > 65535) return hipErrorInvalidConfiguration;
     return launch_kernel<walk_vec_sums_kernel<T, D>>(dim3((unsigned)p.n_chunks, (unsigned)BH), dim3(256), 0, stream, p);
+}
+
+// ---- the normalised backward's first pass: dO = g / n and dn = -(g . out) / n (contiguous, for the walks behind it), and from
+// them, while they are in LDS, every segment's totals of Q^T dO -- walk_totals_kernel's -- and of dn_i q_i.
+// Bound by memory: g, out and dO once each and the needed segments' q.  As passes of their own (dO and dn, totals, per-chunk
+// vectors and their scan, each reading q or dO again) B H 64, N 4096, D 64 took 42 us, this way 25 (134 MB: 5.4 TB/s); B H 16,
+// N 8192, D 128 48 -> 33 us.
+struct WalkGradParams {
+    const void *q, *go, *o;
+    int64_t qs_b, qs_h, qs_n, gs_b, gs_h, gs_n, os_b, os_h, os_n;
+    const float *denom;        // n, fp32 [BH][N]
+    void *dout;                // dO: contiguous rows of wv elements
+    float *dn;                 // fp32 [BH][N]
+    int32_t H, N, BH, wqk, wv;
+    int32_t vec;               // g and out allow 16-byte loads
+    int32_t n_chunks, seg_chunks, n_seg;
+    float *totals, *rsum;      // [BH][n_seg] states and vectors in the slots the walks read (two segments: partial sums of the
+                               // second one's in both; the first one's stay unwritten otherwise); null with a single segment
+};
+
+// Steps on their way: what a step needs is requested DEPTH steps ahead -- one where two workgroups share a CU, two at D = 128,
+// where one workgroup has it (one there: 36 us in place of 33 at B H 16, N 8192).
+// VEC: g and out allow 16-byte loads.
+constexpr int walk_grad_depth(int D) { return D == 128 ? 2 : 1; }
+
+template <typename T, int D, bool VEC>
+__global__ __launch_bounds__(256, D == 128 ? 1 : 2) void walk_grad_totals_kernel(const WalkGradParams p) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    using W = WalkCfg<D>;
+    using V8 = typename Mma<T>::V8;
+    constexpr int PIECES = W::C * W::CR / 256;  // 16-byte pieces of a tile per thread
+    constexpr int DEPTH = walk_grad_depth(D), QT = DEPTH + 1;
+    extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
+    const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
+    float *vd = reinterpret_cast<float *>(smem + (QT + 2) * W::TILE);  // QT tiles of Q, two of dO, two of dn
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wg = blockIdx.x, xcd = wg & 7, slot = wg >> 3;
+    const int hl = slot / p.n_seg, bh = hl * 8 + xcd, seg = slot - hl * p.n_seg;
+    if (bh >= p.BH) return;
+    // the chunks whose sums are wanted, [a_lo, a_hi), and those that are visited for dO and dn alone, from b_lo on.  Two
+    // segments: both workgroups of a (b, h) take one half of either segment
+    int a_lo = seg * p.seg_chunks, a_hi = a_lo + p.seg_chunks < p.n_chunks ? a_lo + p.seg_chunks : p.n_chunks;
+    int b_lo = a_lo, b_hi = a_lo;
+    if (p.n_seg == 2) {
+        const int first = p.seg_chunks, mid = first + (p.n_chunks - first + 1) / 2;
+        a_lo = seg ? mid : first, a_hi = seg ? p.n_chunks : mid;
+        b_lo = seg ? (first + 1) / 2 : 0, b_hi = seg ? first : (first + 1) / 2;
+    } else if (seg == 0) {
+        b_hi = a_hi, a_hi = a_lo;
+    }
+    const int n_a = a_hi - a_lo, n_all = n_a + b_hi - b_lo;
+    auto chunk_of = [&](int i) { return i < n_a ? a_lo + i : b_lo + i - n_a; };
+    const int b = bh / p.H, h = bh - b * p.H, N = p.N;
+    const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
+    const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
+    const T *O = static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h;
+    const float *den = p.denom + (int64_t)bh * N;
+    T *dO = static_cast<T *>(p.dout) + (int64_t)bh * N * p.wv;
+    float *dn = p.dn + (int64_t)bh * N;
+    const int qs2 = (int)p.qs_n * 2;
+    const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
+    f32x16 st[W::NBW];
+    float zs = 0.f;
+#pragma unroll
+    for (int i = 0; i < W::NBW; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) st[i][v] = 0.f;
+    const int col = 8 * (tid % W::CR), r0 = tid / W::CR;  // of piece u: row r0 + u 256 / CR of the chunk
+    u32x4 gw[DEPTH][PIECES], ow[DEPTH][PIECES];
+    float nw[DEPTH][PIECES];
+    int q_next = 0;  // the Q tile of the next request
+    auto request = [&](int i, auto set) {  // step i: q to its tile, the other operands to registers (rows past the end: the last one)
+        constexpr int S = decltype(set)::value;
+        const int row0 = chunk_of(i) * W::C;
+        if (i < n_a) walk_load_tile<D>(rq, lds0 + q_next * W::TILE, row0, qs2, p.wqk, wave, lane);
+        q_next = q_next + 1 == QT ? 0 : q_next + 1;
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int row = row0 + r0 + u * (256 / W::CR), at = row < N ? row : N - 1;
+            gw[S][u] = load8(G + (int64_t)at * p.gs_n, true, col, p.wv, VEC);
+            ow[S][u] = load8(O + (int64_t)at * p.os_n, true, col, p.wv, VEC);
+            nw[S][u] = den[at];
+        }
+    };
+    static_for<0, DEPTH>([&](auto set) {
+        if (decltype(set)::value < n_all) request(decltype(set)::value, set);
+    });
+    int q_at = 0;
+    auto step = [&](int i, auto set) {
+        constexpr int S = decltype(set)::value;
+        const int row0 = chunk_of(i) * W::C;
+        unsigned char *tq = smem + q_at * W::TILE, *tg = smem + (QT + (i & 1)) * W::TILE;
+        q_at = q_at + 1 == QT ? 0 : q_at + 1;
+        float *vdn = vd + (i & 1) * W::C;
+        // what was requested for this step has arrived: at most the next step's requests, which follow the stores of the step
+        // before, are out
+        if constexpr (DEPTH == 1) {
+            wait_vm<0>();
+        } else {
+            if (i + 1 < n_a)
+                wait_vm<W::NI + 3 * PIECES>();
+            else if (i + 1 < n_all)
+                wait_vm<3 * PIECES>();
+            else
+                wait_vm<0>();
+        }
+#pragma unroll
+        for (int u = 0; u < PIECES; ++u) {
+            const int r = r0 + u * (256 / W::CR), row = row0 + r;
+            const bool ok = row < N;
+            const V8 a = __builtin_bit_cast(V8, gw[S][u]), o8 = __builtin_bit_cast(V8, ow[S][u]);
+            const float inv = 1.0f / nw[S][u];
+            float dot = 0.f;
+            V8 d8;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                dot += static_cast<float>(a[e]) * static_cast<float>(o8[e]);
+                d8[e] = static_cast<T>(static_cast<float>(a[e]) * inv);
+            }
+#pragma unroll
+            for (int d = 1; d < W::CR; d <<= 1) dot += __shfl_xor(dot, d, 64);
+            u32x4 w = __builtin_bit_cast(u32x4, d8);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) w[e] = ok ? w[e] : 0u;
+            *reinterpret_cast<u32x4 *>(tg + r * W::RB + (((tid % W::CR) ^ walk_swizzle<W::CR>(r)) << 4)) = w;
+            if (tid % W::CR == 0) vdn[r] = ok ? -dot * inv : 0.f;
+            if (ok) {
+                if (col < p.wv) *reinterpret_cast<u32x4 *>(dO + (int64_t)row * p.wv + col) = w;
+                if (tid % W::CR == 0) dn[row] = -dot * inv;
+            }
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0): this wave's part of dO and dn is in LDS, its reads of the step before are done
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (i + DEPTH < n_all) request(i + DEPTH, set);
+        if (i < n_a) {
+            walk_update<T, D>(tq, tg, wave, lane, st);
+            zs += walk_weighted_sums<T, D>(tq, vdn, wave, lane);
+        }
+    };
+#pragma unroll 1
+    for (int i = 0; i < n_all; i += DEPTH)
+        static_for<0, DEPTH>([&](auto set) {
+            if (i + decltype(set)::value < n_all) step(i + decltype(set)::value, set);
+        });
+    if (p.n_seg == 1 || (p.n_seg > 2 && seg == 0)) return;
+    const int64_t at = (int64_t)bh * p.n_seg + seg;
+    walk_write_state<D, WalkExt<D>>(p.totals + at * (D * D), wave, lane, st);
+    float *part = reinterpret_cast<float *>(smem);
+    __syncthreads();
+    walk_weighted_sums_to_lds<D>(part, wave, lane, zs);
+    __syncthreads();
+    if (tid < D) p.rsum[at * D + tid] = walk_col_sum_of<D>(part, tid);
+#else
+    (void)p;
+#endif
+}
+
+template <typename T, int D>
+hipError_t launch_walk_grad_totals(const WalkGradParams &p, hipStream_t stream) {
+    const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
+    if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+    if (p.n_seg > 1 && (!p.totals || !p.rsum)) return hipErrorInvalidValue;
+    constexpr int smem = (walk_grad_depth(D) + 3) * WalkCfg<D>::TILE + 2 * WalkCfg<D>::C * 4;
+    if (p.vec) {
+        constexpr auto kern = walk_grad_totals_kernel<T, D, true>;
+        if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
+        return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
+    }
+    constexpr auto kern = walk_grad_totals_kernel<T, D, false>;
+    if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
+    return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
 }
 
 // columns of the D x D totals that walk_totals_kernel writes for operands of true widths dy, dz (the
@@ -2334,7 +2583,7 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     const bool fm = p.fmap || p.slope_y;
     // (segment totals in place of entry states: the D = 128 walks, by the flag; below that by the number of segments)
     if (p.init_is_totals && (D != 128 || p.n_seg < 3 || !p.init)) return hipErrorInvalidValue;
-    if (p.entry_out && (!p.init_is_totals || fm || p.denom || p.dn)) return hipErrorInvalidValue;
+    if (p.entry_out && (!p.init_is_totals || p.dn || p.slope_y)) return hipErrorInvalidValue;
     if (p.denom || p.dn) {  // the normaliser's terms: its vectors live behind the state
         if ((p.dn && !p.zc) || (p.denom && p.n_seg > 1 && !p.vsum)) return hipErrorInvalidValue;
         constexpr int smem_n = smem + (kDouble ? 2 : 1) * WalkCfg<D>::VEC;
@@ -2380,9 +2629,9 @@ hipError_t launch_walk_bwd(const WalkParams &p, hipStream_t stream) {
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr int smem = 4 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     if (p.dn) {
-        if (!p.zc || !p.rc) return hipErrorInvalidValue;
+        if (!p.zc || !p.saved || (p.n_seg > 1 && !p.rc)) return hipErrorInvalidValue;
         constexpr auto kern = walk_bwd_kernel<T, D, true>;
-        constexpr int smem_n = smem + WalkCfg<D>::VEC;
+        constexpr int smem_n = smem + WalkCfg<D>::VEC + 1024;
         if (hipError_t e = ensure_dynamic_lds<kern>(smem_n)) return e;
         return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_n, stream, p);
     }
@@ -2400,7 +2649,7 @@ hipError_t launch_walk_dkdv(const WalkParams &p, hipStream_t stream) {
     constexpr int smem = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     static_assert(smem <= 160 * 1024, "two sets of tiles and the state must fit the LDS of a CU");
     if (p.dn) {
-        if (!p.rc) return hipErrorInvalidValue;
+        if (p.n_seg > 1 && !p.rc) return hipErrorInvalidValue;
         constexpr auto kern = walk_dkdv_kernel<T, D, true>;
         if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
         return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);

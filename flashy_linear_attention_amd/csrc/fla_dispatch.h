@@ -69,16 +69,17 @@ FLA_DECLARE_WALK_D(walk_fwd, WalkParams)
 FLA_DECLARE_WALK_D(walk_bwd_rev, WalkParams)
 FLA_DECLARE_WALK_D(walk_bwd, WalkParams)
 FLA_DECLARE_WALK_D(walk_dkdv, WalkParams)
+FLA_DECLARE_WALK_D(walk_grad_totals, WalkGradParams)
 FLA_DECLARE_WALK_WIDE(walk_fwd_wide)      // (q, k of 129 .. 256 columns)
 FLA_DECLARE_WALK_WIDE(walk_bwd_rev_wide)  // (... and v of at most 64)
 #undef FLA_DECLARE_WALK_D
 #undef FLA_DECLARE_WALK_WIDE
-hipError_t walk_vec_sums_t0(int D, const WalkVecParams &p, int64_t BH, hipStream_t stream);
-hipError_t walk_vec_sums_t1(int D, const WalkVecParams &p, int64_t BH, hipStream_t stream);
-inline hipError_t walk_vec_sums(int dtype, int D, const WalkVecParams &p, int64_t BH, hipStream_t stream) {
-    return dtype == 0 ? walk_vec_sums_t0(D, p, BH, stream) : walk_vec_sums_t1(D, p, BH, stream);
+hipError_t walk_vec_sums_t0(const WalkVecParams &p, int64_t BH, hipStream_t stream);  // (D = 128)
+hipError_t walk_vec_sums_t1(const WalkVecParams &p, int64_t BH, hipStream_t stream);
+inline hipError_t walk_vec_sums(int dtype, const WalkVecParams &p, int64_t BH, hipStream_t stream) {
+    return dtype == 0 ? walk_vec_sums_t0(p, BH, stream) : walk_vec_sums_t1(p, BH, stream);
 }
-hipError_t walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, int reverse, hipStream_t stream);
+hipError_t walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, hipStream_t stream);
 hipError_t walk_scan(const float *totals, float *entry, int64_t BH, int n_seg, int D, int cols, int reverse,
                      hipStream_t stream, const float *totals_b = nullptr, float *entry_b = nullptr);
 // the polynomial score map chunk-wise (fla_poly_walk.h), bf16

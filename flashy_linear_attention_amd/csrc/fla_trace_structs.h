@@ -77,8 +77,15 @@ FLA_FIELD(totals2) FLA_FIELD(dz2) FLA_FIELD(z_narrow) FLA_FIELD(vsum)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(WalkVecParams)
-FLA_FIELD(y) FLA_FIELD(ys_b) FLA_FIELD(ys_h) FLA_FIELD(ys_n) FLA_FIELD(w) FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(width)
-FLA_FIELD(n_chunks) FLA_FIELD(out)
+FLA_FIELD(y) FLA_FIELD(ys_b) FLA_FIELD(ys_h) FLA_FIELD(ys_n) FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(width) FLA_FIELD(n_chunks)
+FLA_FIELD(out)
+FLA_FIELDS_END
+
+FLA_FIELDS_BEGIN(WalkGradParams)
+FLA_FIELD(q) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(qs_b) FLA_FIELD(qs_h) FLA_FIELD(qs_n) FLA_FIELD(gs_b) FLA_FIELD(gs_h)
+FLA_FIELD(gs_n) FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n) FLA_FIELD(denom) FLA_FIELD(dout) FLA_FIELD(dn) FLA_FIELD(H)
+FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(wqk) FLA_FIELD(wv) FLA_FIELD(vec) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks)
+FLA_FIELD(n_seg) FLA_FIELD(totals) FLA_FIELD(rsum)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(ChunkStateParams)
@@ -108,6 +115,7 @@ inline void trace_describe(trace::Record &r, int arg, const NormParams &p) { tra
 inline void trace_describe(trace::Record &r, int arg, const WalkParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const WalkTotalsParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const WalkVecParams &p) { trace_fields(r, arg, "", p); }
+inline void trace_describe(trace::Record &r, int arg, const WalkGradParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const ChunkStateParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const PolyWalkParams &p) { trace_fields(r, arg, "", p); }
 inline void trace_describe(trace::Record &r, int arg, const ConvertParams &p) {

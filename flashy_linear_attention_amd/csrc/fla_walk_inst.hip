@@ -1,5 +1,5 @@
 // Instantiations of the walk kernels (fla_chunk_walk.h) for one storage type (FLA_WALK_DTYPE: 0 bf16, 1 fp16) and one
-// group of kernels (FLA_WALK_PART: 0 totals and forward walks, 1 backward walks), padded head dims 32, 64 and 128
+// group of kernels (FLA_WALK_PART: 0 totals and forward walks, 1 backward walks and the normalised backward's first pass), padded head dims 32, 64 and 128
 // (128: backward is a forward-direction walk for dQ and a kernel for dK and dV, or one reverse walk where
 // a caller asks for it and forward handed its states over).
 #include "fla_dispatch.h"
@@ -28,6 +28,9 @@ hipError_t FLA_WALK_FN(walk_dkdv)(int D, const WalkParams &p, hipStream_t stream
 hipError_t FLA_WALK_FN(walk_bwd_rev)(int D, const WalkParams &p, hipStream_t stream) {
     return D == 128 ? launch_walk_bwd_rev<WalkT, 128>(p, stream) : hipErrorNotSupported;
 }
+hipError_t FLA_WALK_FN(walk_grad_totals)(int D, const WalkGradParams &p, hipStream_t stream) {
+    FLA_WALK_DISPATCH3(launch_walk_grad_totals, p, stream);
+}
 hipError_t FLA_WALK_FN(walk_bwd_rev_wide)(const WalkParams &p, hipStream_t stream) {
     return launch_walk_bwd_rev_wide<WalkT>(p, stream);
 }
@@ -39,12 +42,12 @@ hipError_t FLA_WALK_FN(walk_fwd)(int D, const WalkParams &p, hipStream_t stream)
     FLA_WALK_DISPATCH3(launch_walk_fwd, p, stream);
 }
 hipError_t FLA_WALK_FN(walk_fwd_wide)(const WalkParams &p, hipStream_t stream) { return launch_walk_fwd_wide<WalkT>(p, stream); }
-hipError_t FLA_WALK_FN(walk_vec_sums)(int D, const WalkVecParams &p, int64_t BH, hipStream_t stream) {
-    FLA_WALK_DISPATCH3(launch_walk_vec_sums, p, BH, stream);
+hipError_t FLA_WALK_FN(walk_vec_sums)(const WalkVecParams &p, int64_t BH, hipStream_t stream) {
+    return launch_walk_vec_sums<WalkT, 128>(p, BH, stream);
 }
 #if FLA_WALK_DTYPE == 0  // (fp32 throughout: once)
-hipError_t walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, int reverse, hipStream_t stream) {
-    return launch_walk_vec_scan(v, BH, n_chunks, D, reverse, stream);
+hipError_t walk_vec_scan(float *v, int64_t BH, int n_chunks, int D, hipStream_t stream) {
+    return launch_walk_vec_scan(v, BH, n_chunks, D, stream);
 }
 hipError_t walk_scan(const float *totals, float *entry, int64_t BH, int n_seg, int D, int cols, int reverse,
                      hipStream_t stream, const float *totals_b, float *entry_b) {
