@@ -1851,7 +1851,7 @@ PolyPlan poly_plan(int64_t B, int64_t H, int64_t N, int64_t r, int64_t dv) {
     p.seg_chunks = (p.n_chunks + segs - 1) / segs;
     p.n_seg = (p.n_chunks + p.seg_chunks - 1) / p.seg_chunks;
     p.work_bytes = p.n_seg > 1 ? B * H * p.n_seg * fla::PolyFeatures::kState * 4 : 0;
-    p.state_bytes = p.n_seg > 1 ? p.work_bytes : 16;  // (a single segment per (b, h) hands nothing over: a token)
+    p.state_bytes = p.n_seg > 1 ? B * H * p.n_seg * fla::PolyFeatures::kStateRoom * 4 : 16;  // (a single segment per (b, h) hands nothing over: a token)
     return p;
 }
 

@@ -1,9 +1,8 @@
 // Chunk-wise evaluation of the polynomial score map, O = tril(f(Xq Xk^T)) V with f(u) = c0 + c1 u + c2 u^2, for rows of
 // at most 16 columns over values of at most 64: the quadratic kernels' work grows with N^2, this one's with N.
 //
-// f(x . y) is the product of feature rows phi_w(x) . phi(y) of F = 209 entries (the order of PolyFeatures below): the
-// quadratic terms x_r x_r2 with r2 in the same or an earlier block of eight columns than r (an earlier one counts
-// twice), the columns themselves and a one.  With the running sums of phi(k_j) [v_j, 1]^T over the rows before a chunk
+// f(x . y) is the product of feature rows phi_w(x) . phi(y) of F = 153 entries (the order of PolyFeatures below): the
+// quadratic terms x_a x_b, every pair of columns once (a pair of two counts twice), the columns themselves and a one.  With the running sums of phi(k_j) [v_j, 1]^T over the rows before a chunk
 // (T), and of phi(q_i) [g_i, dn_i]^T over the rows after it (U),
 //
 //   O_i   = f-scores of the chunk . V + phi_w(q_i) T                      n_i the same with the column of ones
@@ -19,18 +18,20 @@
 // the running sums once per chunk: errors against fp64 0.87 to 1.01 times the quadratic kernels', the normaliser's 1e-7.
 //
 // What bounds it: the matrix instructions and the VALU work that forms features together (an update's fragment of eight
-// features costs about 50 VALU instructions and serves four MFMAs, one along the row 28 and four); HBM is far away
+// features costs 48 VALU instructions and serves ten MFMAs of 16 x 16 x 32, one along the row 32 and four of 32 x 32 x 16): the VALU
+// issues two thirds of the walks' time, the matrix unit is busy a quarter; HBM is far away
 // (40 KiB per 128-row chunk).  Hence eight waves, two per SIMD, so that one wave's VALU work runs under the other's MFMAs: wave w owns
 // rows 32 (w % 4) .. of the chunk, and of their work one half: half of the features and of the score blocks (forward
 // and dq), the rows after the chunk in dV against dk and the chunk's own rows in dV; the two waves of a row
 // block exchange one half of the sums through LDS.  (Halves of the output columns instead formed every feature row and
-// every score twice.)  Of a state a wave owns one of the seven blocks of 32 features, over all value columns, so that every feature is
-// formed once.  A workgroup has a CU to itself; the next chunk's rows are fetched into registers a chunk ahead.  The split
+// every score twice.)  Of a state a wave owns one or two of the ten blocks of 16 features, over all value columns, so that every
+// feature is formed once.  A workgroup has a CU to itself; the next chunk's rows are fetched into registers a chunk ahead.  The split
 // into segments and the forms of their entry states are the walk kernels' (fla_chunk_walk.h).  Backward is a walk in
 // forward direction for dq, from the entry states forward formed, and one in reverse for dk and dv, so that nothing of a
 // row reaches the dq of the chunks before it.
-// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 239 us this way (kernels
-// 26 totals, 66 forward, 34 totals, 62 dq, 94 dk and dv).  With T for dq going backwards, by subtraction, in the reverse walk
+// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 208 us this way (kernels
+// under the profiler 21 totals, 53 forward, 29 totals, 53 dq, 74 dk and dv).  With the pairs taken by blocks of eight columns -- 209
+// features in seven blocks of 32 -- and a barrier more per chunk 239 us.  With T for dq going backwards, by subtraction, in the reverse walk
 // 228 us, but a late row that is infinite, NaN or huge spoiled dq before it; with feature rows rounded to one bf16 number on
 // both sides as well, from tiles of them in LDS, 200 us, and errors up to 1.28 times the quadratic kernels'.
 #pragma once
@@ -58,31 +59,35 @@ struct PolyWalkParams {
     float *entries;      // T before every segment but the first: written by forward (null: nowhere), read by dq's walk
 };
 
-// Feature order: groups of eight.  Groups 0 .. 7: x_r x_(0..7) for r = 0 .. 7; groups 8 .. 23: x_r x_(8h .. 8h+7) for
-// r = 8 .. 15, h = 0, 1; groups 24, 25: the row itself; group 26: a one and zeros; group 27: zeros.
+// Feature order: groups of eight.  Groups 0 .. 15: x_a x_b with a = 8h + j and b = (a + d) % 16 for d = 0 .. 7, h = 0, 1 (group
+// 2d + h, feature j of it); group 16: d = 8, a = 0 .. 7; groups 17, 18: the row itself; group 19: a one and zeros.  Going round
+// the columns by differences d every pair is there once (17 groups where pairs by blocks of eight columns took 24), and which
+// column a feature's factors are is the same for all features of a lane but for a rotation of the row by 8h.
 struct PolyFeatures {
-    static constexpr int kGroups = 28, kBlocks = 7, kF = 224;  // blocks of 32 features
+    static constexpr int kGroups = 20, kBlocks = 5, kF = 160;  // blocks of 32 features
     static constexpr int kSteps = kGroups / 2;                 // 16-wide k steps of a contraction over the features
+    static constexpr int kHalves = kF / 16;                    // blocks of 16 features: the units in which waves own a state
     static constexpr int kV = 64;                              // value columns of a state
     static constexpr int kState = kF * kV + kF;                // [feature][value column], then the column of ones / dn
+    static constexpr int kStateRoom = 224 * 65;                // floats per segment of a state buffer (what callers set aside)
 };
 
 struct PolyLds {  // byte offsets
     // XTR: an x tile transposed (rows of 272 bytes: the sixteen columns, a one per row of the sequence, zeros)
     static constexpr int C = 128, XT = C * 32, VT = C * 128, ST = 2 * 64 * 256, XTR = 18 * 272, EX = 8 * 4096;
     static constexpr int Z = PolyFeatures::kF * 4, DN = C * 4;
-    // totals: the x tile transposed, the v tile, dn
-    static constexpr int tX = 0, tV = tX + XTR, tDn = tV + VT, tTotal = tDn + DN;
+    // totals: two sets of the x tile transposed, the v tile, dn
+    static constexpr int tX = 0, tV = tX + XTR, tDn = tV + VT, tSet = tDn + DN, tTotal = 2 * tSet;
     // forward
     static constexpr int fQ = 0, fK = fQ + XT, fKt = fK + XT, fV = fKt + XTR, fS = fV + VT, fEx = fS + ST, fZ = fEx + EX,
                          fSum = fZ + Z, fTotal = fSum + 2 * C * 4;
     // dq (the exchange: sixteen floats a row)
     static constexpr int qQ = 0, qK = qQ + XT, qKt = qK + XT, qV = qKt + XTR, qG = qV + VT, qS = qG + VT, qEx = qS + ST,
                          qZ = qEx + C * 64, qDn = qZ + Z, qTotal = qDn + DN;
-    // dk, dv (the exchange over U's copy)
+    // dk, dv
     static constexpr int kQ = 0, kQt = kQ + XT, kK = kQt + XTR, kV = kK + XT, kG = kV + VT, kU = kG + VT, kY = kU + ST,
-                         kDn = kY + Z, kTotal = kDn + DN;
-    static_assert(EX == ST && XTR % 16 == 0 && fTotal <= 160 * 1024 && qTotal <= 160 * 1024 && kTotal <= 160 * 1024, "a CU's LDS");
+                         kDn = kY + Z, kEx = kDn + DN, kTotal = kEx + EX;
+    static_assert(XTR % 16 == 0 && tTotal >= 8 * 5 * 1024 && fTotal <= 160 * 1024 && qTotal <= 160 * 1024 && kTotal <= 160 * 1024, "a CU's LDS");
 };
 
 // (a select of two values: written between two elements of an array it would become one load with a computed index, and
@@ -218,25 +223,34 @@ __device__ __forceinline__ PolyTwo poly_split8(const float (&f)[8]) {
     return t;
 }
 
+// A row as the features along it take it: turned by 8 g columns, and its first half weighted for the phi_w side
+struct PolyTurned {
+    float x[16], w[8];  // x[(8g + i) % 16]; 2 c2 times the first eight
+};
+__device__ __forceinline__ PolyTurned poly_turn(const float (&x)[16], int g, float c2) {
+    PolyTurned t;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) t.x[i] = poly_pick(g, x[(i + 8) & 15], x[i]);
+#pragma unroll
+    for (int i = 0; i < 8; ++i) t.w[i] = 2.f * c2 * t.x[i];
+    return t;
+}
+
 // Feature fragment KS (features 16 KS + 8 g ..) of a row, weighted for the phi_w side; `raw` receives it in fp32.
-// xs: the row's columns 8 g .. 8 g + 7.
 template <int KS>
-__device__ __forceinline__ PolyTwo poly_feature_frag(const float (&x)[16], const float (&xs)[8], int g, float c0, float c1,
-                                                     float c2, float (&raw)[8]) {
-    if constexpr (KS < 4) {
-        const float s = c2 * poly_pick(g, x[2 * KS + 1], x[2 * KS]);
+__device__ __forceinline__ PolyTwo poly_feature_frag(const PolyTurned &t, int g, float c0, float c1, float (&raw)[8]) {
+    if constexpr (KS == 0) {  // squares count once
 #pragma unroll
-        for (int j = 0; j < 8; ++j) raw[j] = s * x[j];
-    } else if constexpr (KS < 12) {
-        const float s = (g ? c2 : 2.f * c2) * x[8 + KS - 4];
+        for (int j = 0; j < 8; ++j) raw[j] = 0.5f * t.w[j] * t.x[j];
+    } else if constexpr (KS < 8) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) raw[j] = s * xs[j];
-    } else if constexpr (KS == 12) {
+        for (int j = 0; j < 8; ++j) raw[j] = t.w[j] * t.x[j + KS];
+    } else if constexpr (KS == 8) {  // d = 8; the row's first half
 #pragma unroll
-        for (int j = 0; j < 8; ++j) raw[j] = c1 * xs[j];
-    } else {
+        for (int j = 0; j < 8; ++j) raw[j] = (g ? c1 : t.w[j]) * t.x[j + 8];
+    } else {  // its second half; the one
 #pragma unroll
-        for (int j = 0; j < 8; ++j) raw[j] = j == 0 && g == 0 ? c0 : 0.f;
+        for (int j = 0; j < 8; ++j) raw[j] = g ? (j == 0 ? c0 : 0.f) : c1 * t.x[j + 8];
     }
     return poly_split8<false>(raw);
 }
@@ -248,116 +262,161 @@ struct PolyFactors {
 __device__ __forceinline__ PolyFactors poly_factors(int f) {
     const int group = f >> 3, j = f & 7;
     int a, b;
-    if (group < 24) {
-        a = group < 8 ? group : 4 + (group >> 1), b = group < 8 ? j : 8 * (group & 1) + j;
-    } else {  // the row itself; a one and zeros; zeros
-        a = group < 27 ? 16 : 17, b = group < 26 ? 8 * (group & 1) + j : group == 26 && j == 0 ? 16 : 17;
+    if (group < 17) {
+        a = 8 * (group & 1) + j, b = (a + (group >> 1)) & 15;
+    } else {  // the row itself; a one and zeros
+        a = group < 19 ? 8 * (group - 17) + j : 16, b = group < 19 || j == 0 ? 16 : 17;
     }
     return {(uint32_t)(a * 272), (uint32_t)(b * 272)};
 }
 
-// A state's blocks of this wave: feature block `wave` (wave 7: none) over both 32-column blocks of the values, and -- NORM --
-// the column of ones (of dn): lane l32 of either half holds its part of feature 32 wave + l32.
+// A state's blocks of this wave: up to two blocks of 16 features (`first`, `second`, < 0: none) over the four 16-column blocks of
+// the values, and -- NORM -- the column of ones (of dn), the same in every lane column.  Register v of a block: feature
+// 4 (lane / 16) + v, value column lane % 16.
 struct PolyState {
-    f32x16 st[2];
-    float ex;
-    int wave;
-    __device__ __forceinline__ void clear(int w) {
-        wave = w, ex = 0.f;
+    f32x4 st[2][4], ex[2];
+    int own[2];
+    __device__ __forceinline__ void clear(int first, int second) {
+        own[0] = first, own[1] = second;
 #pragma unroll
-        for (int v = 0; v < 16; ++v) st[0][v] = st[1][v] = 0.f;
+        for (int u = 0; u < 2; ++u) {
+            ex[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) st[u][cb] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
     }
-    __device__ __forceinline__ bool valid() const { return wave < PolyFeatures::kBlocks; }
+    // ten blocks on eight waves, two waves to a SIMD: the waves of the row blocks with the least other work take two
+    __device__ __forceinline__ void clear_lower(int wave) { clear(wave, wave < 2 ? 8 + wave : -1); }
+    __device__ __forceinline__ void clear_upper(int wave) {
+        clear(wave < 4 ? 2 * wave : wave >= 6 ? wave + 2 : -1, wave < 4 ? 2 * wave + 1 : -1);
+    }
     // += the state at `s` in memory
     template <bool NORM>
-    __device__ __forceinline__ void add(const float *s, int l32, int g) {
-        if (!valid()) return;
+    __device__ __forceinline__ void add(const float *s, int lane) {
+        const int l16 = lane & 15, kq = lane >> 4;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int u = 0; u < 2; ++u)
+            if (own[u] >= 0) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-                st[i][v] += s[(32 * wave + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * i + l32];
-        if (NORM && g == 0) ex += s[PolyFeatures::kF * PolyFeatures::kV + 32 * wave + l32];
+                for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) st[u][cb][v] += s[(16 * own[u] + 4 * kq + v) * PolyFeatures::kV + 16 * cb + l16];
+                if (NORM) ex[u] += *reinterpret_cast<const f32x4 *>(s + PolyFeatures::kF * PolyFeatures::kV + 16 * own[u] + 4 * kq);
+            }
     }
     template <bool NORM>
-    __device__ __forceinline__ void store(float *s, int l32, int g) const {
-        if (!valid()) return;
+    __device__ __forceinline__ void store(float *s, int lane) const {
+        const int l16 = lane & 15, kq = lane >> 4;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+        for (int u = 0; u < 2; ++u)
+            if (own[u] >= 0) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-                s[(32 * wave + 8 * (v / 4) + 4 * g + (v % 4)) * PolyFeatures::kV + 32 * i + l32] = st[i][v];
-        if (NORM) {
-            const float t = ex + __shfl_xor(ex, 32, 64);
-            if (g == 0) s[PolyFeatures::kF * PolyFeatures::kV + 32 * wave + l32] = t;
-        }
+                for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+                    for (int v = 0; v < 4; ++v) s[(16 * own[u] + 4 * kq + v) * PolyFeatures::kV + 16 * cb + l16] = st[u][cb][v];
+                if (NORM && l16 == 0)
+                    *reinterpret_cast<f32x4 *>(s + PolyFeatures::kF * PolyFeatures::kV + 16 * own[u] + 4 * kq) = ex[u];
+            }
     }
     // rounded to the storage type as rows of value columns, features 0 .. 127 and 128 .. in two tiles; ex in fp32 to z
     template <typename T, bool NORM>
-    __device__ __forceinline__ void to_lds(unsigned char *tile, float *z, int l32, int g) const {
+    __device__ __forceinline__ void to_lds(unsigned char *tile, float *z, int lane) const {
         typedef T t4 __attribute__((ext_vector_type(4)));
-        if (!valid()) return;
-        unsigned char *t = tile + (wave >> 2) * 64 * 256;
+        const int l16 = lane & 15, kq = lane >> 4;
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int row = 32 * i + l32;
+        for (int u = 0; u < 2; ++u)
+            if (own[u] >= 0) {
+                unsigned char *t = tile + (own[u] >> 3) * 64 * 256;
+                const int ch = 2 * (own[u] & 7) + (kq >> 1);
 #pragma unroll
-            for (int a = 0; a < 4; ++a) {
-                t4 w;
+                for (int cb = 0; cb < 4; ++cb) {
+                    const int row = 16 * cb + l16;
+                    t4 w;
 #pragma unroll
-                for (int b = 0; b < 4; ++b) w[b] = static_cast<T>(st[i][4 * a + b]);
-                *reinterpret_cast<t4 *>(t + row * 256 + (((4 * (wave & 3) + a) ^ walk_swizzle<16>(row)) << 4) + 8 * g) = w;
+                    for (int v = 0; v < 4; ++v) w[v] = static_cast<T>(st[u][cb][v]);
+                    *reinterpret_cast<t4 *>(t + row * 256 + ((ch ^ walk_swizzle<16>(row)) << 4) + 8 * (kq & 1)) = w;
+                }
+                if (NORM && l16 == 0) *reinterpret_cast<f32x4 *>(z + 16 * own[u] + 4 * kq) = ex[u];
             }
+    }
+    // What a step of 32 rows reads; requested a step ahead of its use, block after block (both blocks in one loop of
+    // branches: the forward walk 53.6 us in place of 53.1, dk and dv 75.3 in place of 74.1).
+    struct Rows {
+        u32x4 a, b, e[2];
+        Mma<__bf16>::V8 z[4];
+    };
+    template <bool NORM>
+    __device__ __forceinline__ void request(Rows &r, const unsigned char *fa, const unsigned char *fb, const unsigned char *zt, PolyPair za,
+                                            const float *extra) const {
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) r.z[cb] = poly_tr<__bf16>(zt, za, cb << 5);
+        r.a = *reinterpret_cast<const u32x4 *>(fa), r.b = *reinterpret_cast<const u32x4 *>(fb);
+        if constexpr (NORM)
+            if (extra) r.e[0] = *reinterpret_cast<const u32x4 *>(extra), r.e[1] = *reinterpret_cast<const u32x4 *>(extra + 4);
+    }
+    template <bool NORM>
+    __device__ __forceinline__ void add_rows(const Rows &r, bool ones, f32x4 (&acc)[4], f32x4 &e) {
+        float f[8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            f[2 * k] = __builtin_bit_cast(float, r.a[k] << 16) * __builtin_bit_cast(float, r.b[k] << 16);
+            f[2 * k + 1] = __builtin_bit_cast(float, r.a[k] & 0xffff0000u) * __builtin_bit_cast(float, r.b[k] & 0xffff0000u);
         }
-        if (NORM) {
-            const float sum = ex + __shfl_xor(ex, 32, 64);
-            if (g == 0) z[32 * wave + l32] = sum;
+        const PolyTwo y = poly_split8<true>(f);
+        Mma<__bf16>::V8 ef;
+        if constexpr (NORM) {
+            u32x4 w = {0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u};
+            if (!ones) {
+#pragma unroll
+                for (int h = 0; h < 4; ++h)
+                    w[h] = __builtin_amdgcn_perm(r.e[h >> 1][2 * (h & 1) + 1], r.e[h >> 1][2 * (h & 1)], 0x07060302u);
+            }
+            ef = __builtin_bit_cast(Mma<__bf16>::V8, w);
         }
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y.hi, r.z[cb], acc[cb], 0, 0, 0);
+        if constexpr (NORM) e = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y.hi, ef, e, 0, 0, 0);
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) acc[cb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y.lo, r.z[cb], acc[cb], 0, 0, 0);
+        if constexpr (NORM) e = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y.lo, ef, e, 0, 0, 0);
     }
     // += phi^T [z tile, extra column] over the chunk's 128 rows.  Feature rows are formed here, as products of two
     // rows of the transposed x tile: a lane's eight rows of one feature, exactly, in two bf16 numbers each.
-    // extra: the extra column, 128 floats in LDS (null: ones).
+    // extra: the extra column, 128 floats in LDS that bf16 holds exactly (null: ones).
+    // ONE: of the second block the 32 rows of step `step` alone.
     // (Rounded to one bf16 number, from a tile of feature rows, they and the weighted ones along the rows made the errors of
     // O, dq, dk and dv 1.2 times the quadratic kernels', and those of the normaliser 1e-3 in place of 1e-7.)
-    template <typename T, bool NORM>
-    __device__ __forceinline__ void update(const unsigned char *xtr, const unsigned char *zt, const float *extra, int lane) {
-        using M = Mma<T>;
-        using V8 = typename M::V8;
-        if (!valid()) return;
-        const int l32 = lane & 31, g = lane >> 5;
-        const PolyFactors at = poly_factors(32 * wave + l32);
-        const unsigned char *fa = xtr + at.a + 16 * g, *fb = xtr + at.b + 16 * g;
-        const PolyPair za = poly_col_base<128>(lane);
-        auto step = [&](auto ksc) {
-            constexpr int ks = decltype(ksc)::value;
-            const V8 z0 = poly_tr<T>(zt + 16 * 128 * ks, za), z1 = poly_tr<T>(zt + 16 * 128 * ks, za, 1 << 6);
-            const u32x4 a = *reinterpret_cast<const u32x4 *>(fa + 32 * ks), b = *reinterpret_cast<const u32x4 *>(fb + 32 * ks);
-            float f[8];
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-                f[2 * k] = __builtin_bit_cast(float, a[k] << 16) * __builtin_bit_cast(float, b[k] << 16);
-                f[2 * k + 1] = __builtin_bit_cast(float, a[k] & 0xffff0000u) * __builtin_bit_cast(float, b[k] & 0xffff0000u);
-            }
-            if constexpr (NORM) {
-                if (extra) {
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        const f32x4 e = *reinterpret_cast<const f32x4 *>(extra + 16 * ks + 8 * g + 4 * h);
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) ex += f[4 * h + j] * e[j];
-                    }
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 8; ++j) ex += f[j];
-                }
-            }
-            const PolyTwo y = poly_split8<true>(f);
-            st[0] = M::mma(y.hi, z0, st[0]);
-            st[1] = M::mma(y.hi, z1, st[1]);
-            st[0] = M::mma(y.lo, z0, st[0]);
-            st[1] = M::mma(y.lo, z1, st[1]);
+    template <bool NORM, bool ONE = false>
+    __device__ __forceinline__ void update(const unsigned char *xtr, const unsigned char *zt, const float *extra, int lane, int step = 0) {
+        const int l16 = lane & 15, kq = lane >> 4;
+        const int row = 8 * kq + (l16 >> 2), ch = (l16 & 3) >> 1, sub = 8 * (l16 & 1);
+        const PolyPair za{(uint32_t)(row * 128 + ((ch ^ walk_swizzle<8>(row)) << 4) + sub),
+                          (uint32_t)((row + 4) * 128 + ((ch ^ walk_swizzle<8>(row + 4)) << 4) + sub)};
+        const float *ex_at = extra ? extra + 8 * kq : nullptr;
+        constexpr int STEPS = PolyLds::C / 32;
+        auto block = [&](auto uc, auto steps, int first) {
+            constexpr int U = decltype(uc)::value, NS = decltype(steps)::value;
+            const PolyFactors at = poly_factors(16 * own[U] + l16);
+            const unsigned char *fa = xtr + 16 * kq + at.a + 64 * first, *fb = xtr + 16 * kq + at.b + 64 * first;
+            const unsigned char *z0 = zt + 32 * 128 * first;
+            const float *e0 = extra ? ex_at + 32 * first : nullptr;
+            Rows r[2];
+            request<NORM>(r[0], fa, fb, z0, za, e0);
+            static_for<0, NS>([&](auto sc) {
+                constexpr int S = decltype(sc)::value;
+                if constexpr (S + 1 < NS)
+                    request<NORM>(r[(S + 1) & 1], fa + 64 * (S + 1), fb + 64 * (S + 1), z0 + 32 * 128 * (S + 1), za, extra ? e0 + 32 * (S + 1) : nullptr);
+                __builtin_amdgcn_sched_barrier(0);
+                add_rows<NORM>(r[S & 1], !extra, st[U], ex[U]);
+            });
         };
-        static_for<0, PolyLds::C / 16>(step);
+        using C4 = std::integral_constant<int, STEPS>;
+        if (own[0] >= 0) block(std::integral_constant<int, 0>{}, C4{}, 0);
+        if constexpr (ONE) {
+            block(std::integral_constant<int, 1>{}, std::integral_constant<int, 1>{}, step);
+        } else {
+            if (own[1] >= 0) block(std::integral_constant<int, 1>{}, C4{}, 0);
+        }
     }
 };
 
@@ -502,7 +561,7 @@ __global__ __launch_bounds__(512, 2) void poly_totals_kernel(const PolyWalkParam
 #if defined(__gfx950__)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     using L = PolyLds;
-    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const PolySlice sl = poly_slice(p);
     if (!sl.valid || sl.seg == (BWD ? 0 : p.n_seg - 1)) return;
@@ -513,34 +572,66 @@ __global__ __launch_bounds__(512, 2) void poly_totals_kernel(const PolyWalkParam
     const T *G = BWD ? static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h : nullptr;
     const T *O = BWD && NORM ? static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h : nullptr;
     const float *n = NORM && BWD ? p.denom + (int64_t)sl.bh * N : nullptr;
-    float *dn = reinterpret_cast<float *>(smem + L::tDn);
+    // Ten blocks of features on eight waves: a wave has one of its own and a quarter of the rows -- one step of every chunk --
+    // of one of the last two, whose four parts are added up at the end (B H 64, N 4096: 21.4 -> 20.8 us forward, 29.7 -> 28.6
+    // backward together with the second set of tiles; what is left is the chain load -> LDS -> features of two waves a SIMD)
     PolyState s;
-    s.clear(wave);
-    u32x4 x = {0u, 0u, 0u, 0u};
-    PolyTile<T> v;
-    PolyGrad<T, NORM> go;
-    auto fetch = [&](int c) {
+    s.clear(wave, 8 + (wave >> 2));
+    constexpr int SETS = 2;  // chunks on their way (registers and LDS)
+    u32x4 x[SETS];
+    PolyTile<T> v[SETS];
+    PolyGrad<T, NORM> go[SETS];
+    auto fetch = [&](int c, auto set) {
+        constexpr int S = decltype(set)::value;
         const int row0 = c * L::C;
-        if (tid < 256) x = poly_fetch_x<T>(X, xs, row0, N, p.r, tid);
+        if (tid < 256) x[S] = poly_fetch_x<T>(X, xs, row0, N, p.r, tid);
         if constexpr (BWD)
-            go.fetch(G, p.gs_n, O, p.os_n, n, row0, N, p.wv, tid);
+            go[S].fetch(G, p.gs_n, O, p.os_n, n, row0, N, p.wv, tid);
         else
-            v.fetch(V, p.vs_n, row0, N, p.wv, tid);
+            v[S].fetch(V, p.vs_n, row0, N, p.wv, tid);
     };
-    fetch(sl.c_lo);
-#pragma unroll 1
-    for (int c = sl.c_lo; c < sl.c_hi; ++c) {
-        __syncthreads();
-        if (tid < 256) poly_put_xt(smem + L::tX, x, tid), poly_put_ones<T>(smem + L::tX, c * L::C, N, tid);
+    static_for<0, SETS>([&](auto set) {
+        if (sl.c_lo + decltype(set)::value < sl.c_hi) fetch(sl.c_lo + decltype(set)::value, set);
+    });
+    auto chunk = [&](int c, auto set) {
+        constexpr int S = decltype(set)::value;
+        unsigned char *tile = smem + S * L::tSet;
+        float *dn = reinterpret_cast<float *>(tile + L::tDn);
+        // (every wave has passed the barrier below a chunk ago, behind its reads of this set)
+        if (tid < 256) poly_put_xt(tile + L::tX, x[S], tid), poly_put_ones<T>(tile + L::tX, c * L::C, N, tid);
         if constexpr (BWD)
-            go.put(smem + L::tV, dn, tid);
+            go[S].put(tile + L::tV, dn, tid);
         else
-            v.put(smem + L::tV, tid);
-        if (c + 1 < sl.c_hi) fetch(c + 1);
+            v[S].put(tile + L::tV, tid);
+        if (c + SETS < sl.c_hi) fetch(c + SETS, set);
         __syncthreads();
-        s.template update<T, NORM>(smem + L::tX, smem + L::tV, BWD ? dn : nullptr, lane);
+        s.template update<NORM, true>(tile + L::tX, tile + L::tV, BWD ? dn : nullptr, lane, wave & 3);
+    };
+#pragma unroll 1
+    for (int c = sl.c_lo; c < sl.c_hi; c += SETS)
+        static_for<0, SETS>([&](auto set) {
+            if (c + decltype(set)::value < sl.c_hi) chunk(c + decltype(set)::value, set);
+        });
+    // the last two blocks: waves 1 .. 3 and 5 .. 7 hand theirs to waves 0 and 4
+    __syncthreads();
+    f32x4 *part = reinterpret_cast<f32x4 *>(smem);  // [wave][5][lane]
+    if (wave & 3) {
+#pragma unroll
+        for (int cb = 0; cb < 4; ++cb) part[(wave * 5 + cb) * 64 + lane] = s.st[1][cb];
+        part[(wave * 5 + 4) * 64 + lane] = s.ex[1];
     }
-    s.template store<NORM>(p.totals + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, l32, g);
+    __syncthreads();
+    if (wave & 3) {
+        s.own[1] = -1;
+    } else {
+#pragma unroll
+        for (int u = 1; u < 4; ++u) {
+#pragma unroll
+            for (int cb = 0; cb < 4; ++cb) s.st[1][cb] += part[((wave + u) * 5 + cb) * 64 + lane];
+            s.ex[1] += part[((wave + u) * 5 + 4) * 64 + lane];
+        }
+    }
+    s.template store<NORM>(p.totals + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, lane);
 #else
     (void)p;
 #endif
@@ -571,16 +662,16 @@ __global__ __launch_bounds__(256) void poly_scan_kernel(float *totals, int n_seg
 
 // the entry state of a segment: zeros, one state in memory, or the sum of the totals before (after) it
 template <bool NORM>
-__device__ __forceinline__ void poly_entry(const PolyWalkParams &p, const PolySlice &sl, bool reverse, int l32, int g, PolyState &s) {
+__device__ __forceinline__ void poly_entry(const PolyWalkParams &p, const PolySlice &sl, bool reverse, int lane, PolyState &s) {
     if (!p.totals) return;
     const float *base = p.totals + (int64_t)sl.bh * p.n_seg * PolyFeatures::kState;
     if (!p.sum_entries) {
-        s.template add<NORM>(base + (int64_t)sl.seg * PolyFeatures::kState, l32, g);
+        s.template add<NORM>(base + (int64_t)sl.seg * PolyFeatures::kState, lane);
         return;
     }
     const int lo = reverse ? sl.seg + 1 : 0, hi = reverse ? p.n_seg : sl.seg;
 #pragma unroll 1
-    for (int f = lo; f < hi; ++f) s.template add<NORM>(base + (int64_t)f * PolyFeatures::kState, l32, g);
+    for (int f = lo; f < hi; ++f) s.template add<NORM>(base + (int64_t)f * PolyFeatures::kState, lane);
 }
 
 template <typename T, bool NORM>
@@ -604,10 +695,10 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
     float *z = reinterpret_cast<float *>(smem + L::fZ), *sums = reinterpret_cast<float *>(smem + L::fSum);
     unsigned char *exch = smem + L::fEx;
     PolyState s;
-    s.clear(wave);
-    poly_entry<NORM>(p, sl, false, tid0 & 31, (tid0 & 63) >> 5, s);
+    s.clear_lower(wave);
+    poly_entry<NORM>(p, sl, false, tid0 & 63, s);
     if (p.entries && sl.seg > 0)
-        s.template store<NORM>(p.entries + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
+        s.template store<NORM>(p.entries + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kStateRoom, tid0 & 63);
     u32x4 x;
     PolyTile<T> v;
     auto fetch = [&](int c, int tid) {
@@ -619,11 +710,11 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
 #pragma unroll 1
     for (int c = sl.c_lo; c < sl.c_hi; ++c) {
         const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-        __syncthreads();
+        // (every wave is past the barrier behind its last reads of the tiles and of the state's copy)
         poly_put_x(tid < 256 ? tq : tk, x, tid);
         if (tid >= 256) poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
         v.put(tv, tid);
-        s.template to_lds<T, NORM>(ts, z, l32, g);
+        s.template to_lds<T, NORM>(ts, z, lane);
         if (c + 1 < sl.c_hi) fetch(c + 1, tid);
         __syncthreads();
 
@@ -633,15 +724,14 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
         for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
         float rsum = 0.f;
         if (c > 0) {  // phi_w(q) T, this half of the features
-            float xr[16], xs[8];
+            float xr[16];
             poly_row<T>(tq, trow, xr);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) xs[j] = poly_pick(g, xr[8 + j], xr[j]);
+            const PolyTurned xt = poly_turn(xr, g, c2);
             const uint32_t sa = poly_row_base<256>(walk_e_lane(l32), g);
             auto step = [&](auto ksc) {
                 constexpr int KS = decltype(ksc)::value;
                 float raw[8];
-                const PolyTwo f = poly_feature_frag<KS>(xr, xs, g, c0, c1, c2, raw);
+                const PolyTwo f = poly_feature_frag<KS>(xt, g, c0, c1, raw);
 #pragma unroll
                 for (int e = 0; e < 2; ++e) {
                     const V8 sf = poly_rd<T>(ts + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5));
@@ -692,6 +782,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
                 for (int e = 0; e < 2; ++e)
                     acc[e] = M::mma(poly_tr<T>(tv + 128 * (32 * sb + 16 * t), va, e << 6), pf[t], acc[e]);
         }
+        if (c + 1 < sl.c_hi) s.template update<NORM>(tkt, tv, nullptr, lane);
         // each of the two waves of these rows finishes one half of the columns: the other half's sums go to the other wave
         {
             f32x16 mine;
@@ -704,7 +795,6 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
             if (g == 0) sums[kh * L::C + trow] = rsum;
         }
         __syncthreads();
-        if (c + 1 < sl.c_hi) s.template update<T, NORM>(tkt, tv, nullptr, lane);
         f32x16 other;
         poly_get_acc(exch, wave ^ 4, lane, other);
         float f[16], inv = 1.f;
@@ -728,10 +818,15 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
 // Returns this lane's part of it (the other part is in the lane of the other g) in dx.
 template <typename T, bool NORM, int FB0, int FB1>
 __device__ __forceinline__ void poly_contract(const unsigned char *S, const float *z, float extra, const typename Mma<T>::V8 (&gf)[4],
-                                              const float (&x)[16], int lane, float c1, float c2, float (&quad)[16]) {
+                                              const float (&x)[16], int lane, float c1, float c2, float (&dx)[16]) {
     using M = Mma<T>;
     const int g = lane >> 5;
     const PolyPair sa = poly_perm_base<256, true>(lane);
+    // of a block's feature v with the difference d = 2 FB + g: a = v, b = (v + 2 FB + g) % 16.  q1: sums of H x_b by a; q2: of
+    // H x_a by b - g; y: the row turned by g
+    float q1[16], q2[16], y[16], lin[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) q1[i] = q2[i] = lin[i] = 0.f, y[i] = poly_pick(g, x[(i + 1) & 15], x[i]);
     static_for<FB0, FB1>([&](auto fbc) {
         constexpr int FB = decltype(fbc)::value;
         f32x16 hh;
@@ -746,36 +841,28 @@ __device__ __forceinline__ void poly_contract(const unsigned char *S, const floa
         for (int kc = 0; kc < 4; ++kc)
             hh = M::mma(poly_tr<T>(S + (FB >> 2) * 64 * 256 + 16 * 256 * kc, sa, (FB & 3) << 6), gf[kc], hh);
         // hh[v]: feature 32 FB + 16 g + v
-        if constexpr (FB < 2) {  // two groups x_r x_(0..7), r = 4 FB + 2 g and the next
-            float t[2] = {0.f, 0.f};
+        if constexpr (FB < 4) {
+            const float once = FB == 0 ? (g ? 1.f : 0.5f) : 1.f;  // (d = 0: both sums meet in x_v)
 #pragma unroll
-            for (int e = 0; e < 2; ++e)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) t[e] += hh[8 * e + j] * x[j];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                quad[4 * FB + e] += poly_pick(g, 0.f, t[e]);
-                quad[4 * FB + 2 + e] += poly_pick(g, t[e], 0.f);
+            for (int v = 0; v < 16; ++v) {
+                const float t = FB == 0 ? hh[v] * once : hh[v];
+                q1[v] += t * y[(v + 2 * FB) & 15];
+                q2[(v + 2 * FB) & 15] += t * x[v];
             }
-        } else if constexpr (FB < 6) {  // x_r x_(0..15), r = 8 + 2 (FB - 2) + g
-            constexpr int R = 8 + 2 * (FB - 2);
-            float t = 0.f;
-            const float xr = poly_pick(g, x[R + 1], x[R]);
+        } else {  // g = 0: d = 8, the row's first half; g = 1: its second half, the one
 #pragma unroll
-            for (int j = 0; j < 16; ++j) t += hh[j] * x[j];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) quad[j] += hh[j] * xr;
-            quad[R] += poly_pick(g, 0.f, t);
-            quad[R + 1] += poly_pick(g, t, 0.f);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; ++j) quad[j] = 2.f * c2 * quad[j] + poly_pick(g, 0.f, c1 * hh[j]);
+            for (int j = 0; j < 8; ++j) {
+                const float t = poly_pick(g, 0.f, hh[j]);
+                q1[j] += t * x[j + 8], q1[j + 8] += t * x[j];
+                lin[j] = poly_pick(g, 0.f, hh[j + 8]), lin[j + 8] = poly_pick(g, hh[j], 0.f);
+            }
         }
         if constexpr (FB % 2 == 1) __builtin_amdgcn_sched_barrier(0);  // (two blocks at a time: registers)
     });
-    if constexpr (FB1 < PolyFeatures::kBlocks) {
 #pragma unroll
-        for (int j = 0; j < 16; ++j) quad[j] *= 2.f * c2;
+    for (int j = 0; j < 16; ++j) {
+        dx[j] = 2.f * c2 * (q1[j] + poly_pick(g, q2[(j + 15) & 15], q2[j]));
+        if constexpr (FB1 == PolyFeatures::kBlocks) dx[j] += c1 * lin[j];
     }
 }
 
@@ -805,9 +892,8 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
                   *ts = smem + L::qS, *exch = smem + L::qEx;
     float *z = reinterpret_cast<float *>(smem + L::qZ), *dn = reinterpret_cast<float *>(smem + L::qDn);
     PolyState s;
-    s.clear(wave);
-    if (sl.seg > 0)
-        s.template add<NORM>(p.entries + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 31, (tid0 & 63) >> 5);
+    s.clear_lower(wave);
+    if (sl.seg > 0) s.template add<NORM>(p.entries + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kStateRoom, tid0 & 63);
     u32x4 x;
     PolyTile<T> v;
     PolyGrad<T, NORM> go;
@@ -821,12 +907,12 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
 #pragma unroll 1
     for (int c = sl.c_lo; c < sl.c_hi; ++c) {
         const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
-        __syncthreads();
+        // (every wave is past the barrier behind its last reads of the tiles and of the state's copy)
         poly_put_x(tid < 256 ? tq : tk, x, tid);
         if (tid >= 256) poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
         v.put(tv, tid);
         go.put(tg, dn, tid);
-        s.template to_lds<T, NORM>(ts, z, l32, g);
+        s.template to_lds<T, NORM>(ts, z, lane);
         if (c + 1 < sl.c_hi) fetch(c + 1, tid);
         __syncthreads();
 
@@ -843,9 +929,9 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
             float xr[16];
             poly_row<T>(tq, trow, xr);
             if (kh == 0)
-                poly_contract<T, NORM, 0, 3>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
+                poly_contract<T, NORM, 0, 2>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
             else
-                poly_contract<T, NORM, 3, PolyFeatures::kBlocks>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
+                poly_contract<T, NORM, 2, PolyFeatures::kBlocks>(ts, z, dni, gf, xr, lane, c1, c2, dxs);
         }
         const V8 xq = poly_row_frag<T>(tq, trow, g);
         const int rc = walk_e_lane(l32) & 15;  // (columns 16 .. of the 32-wide block of dq are not used)
@@ -877,7 +963,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
             for (int a = 0; a < 4; ++a)
                 *reinterpret_cast<f32x4 *>(exch + (a * L::C + trow) * 16) = f32x4{f[4 * a], f[4 * a + 1], f[4 * a + 2], f[4 * a + 3]};
         }
-        if (c + 1 < sl.c_hi) s.template update<T, NORM>(tkt, tv, nullptr, lane);
+        if (c + 1 < sl.c_hi) s.template update<NORM>(tkt, tv, nullptr, lane);
         __syncthreads();
         if (kh == 0 && g == 0) {
 #pragma unroll
@@ -917,11 +1003,11 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
     T *dV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
     const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
     unsigned char *tq = smem + L::kQ, *tqt = smem + L::kQt, *tk = smem + L::kK, *tv = smem + L::kV, *tg = smem + L::kG,
-                  *us = smem + L::kU;
+                  *us = smem + L::kU, *exch = smem + L::kEx;
     float *y = reinterpret_cast<float *>(smem + L::kY), *dn = reinterpret_cast<float *>(smem + L::kDn);
     PolyState su;
-    su.clear(wave);
-    poly_entry<NORM>(p, sl, true, tid0 & 31, (tid0 & 63) >> 5, su);
+    su.clear_upper(wave);
+    poly_entry<NORM>(p, sl, true, tid0 & 63, su);
     u32x4 x;
     PolyTile<T> v;
     PolyGrad<T, NORM> go;
@@ -936,12 +1022,12 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
     for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
         const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
         const bool after = c + 1 < p.n_chunks;  // (U of this chunk holds anything)
-        __syncthreads();
+        // (every wave is past the barrier behind its last reads of the tiles and of the state's copy)
         poly_put_x(tid < 256 ? tq : tk, x, tid);
         if (tid < 256) poly_put_xt(tqt, x, tid), poly_put_ones<T>(tqt, c * L::C, N, tid);
         v.put(tv, tid);
         go.put(tg, dn, tid);
-        if (after) su.template to_lds<T, NORM>(us, y, l32, g);
+        if (after) su.template to_lds<T, NORM>(us, y, lane);
         if (c > sl.c_lo) fetch(c - 1, tid);
         __syncthreads();
 
@@ -953,15 +1039,14 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
         for (int i = 0; i < 16; ++i) acc[0][i] = acc[1][i] = 0.f;
         if (half == 0) {
             if (after) {
-                float xr[16], xs[8];
+                float xr[16];
                 poly_row<T>(tk, trow, xr);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) xs[j] = poly_pick(g, xr[8 + j], xr[j]);
+                const PolyTurned xt = poly_turn(xr, g, c2);
                 const uint32_t sa = poly_row_base<256>(walk_e_lane(l32), g);
                 static_for<0, PolyFeatures::kSteps>([&](auto ksc) {
                     constexpr int KS = decltype(ksc)::value;
                     float raw[8];
-                    const PolyTwo f = poly_feature_frag<KS>(xr, xs, g, c0, c1, c2, raw);
+                    const PolyTwo f = poly_feature_frag<KS>(xt, g, c0, c1, raw);
 #pragma unroll
                     for (int e = 0; e < 2; ++e) {
                         const V8 uf = poly_rd<T>(us + (KS >> 3) * 64 * 256 + 32 * 256 * e, sa ^ ((KS & 7) << 5));
@@ -1022,18 +1107,17 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
             for (int i = 0; i < 16; ++i) f[i] = dxs[i] + __shfl_xor(dxs[i], 32, 64) + dx[i];
             if (row < N && g == 0) poly_store16<T>(dK + (int64_t)row * p.dks_n, f, 0, p.r);
         }
-        __syncthreads();
+        if (c > sl.c_lo) su.template update<NORM>(tqt, tg, dn, lane);
         {
             f32x16 mine;
 #pragma unroll
             for (int i = 0; i < 16; ++i) mine[i] = poly_pick(half, acc[0][i], acc[1][i]);
-            poly_put_acc(us, wave, lane, mine);  // (U's copy has been read)
+            poly_put_acc(exch, wave, lane, mine);
         }
-        if (c > sl.c_lo) su.template update<T, NORM>(tqt, tg, dn, lane);
         __syncthreads();
         {
             f32x16 other;
-            poly_get_acc(us, wave ^ 4, lane, other);
+            poly_get_acc(exch, wave ^ 4, lane, other);
             float f[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) f[i] = poly_pick(half, acc[1][i], acc[0][i]) + other[i];
