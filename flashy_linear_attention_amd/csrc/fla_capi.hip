@@ -107,11 +107,11 @@ struct Span {
     uintptr_t lo, hi;
 };
 
-Span span_of(const View &t, int64_t B, int64_t H, int64_t N, int64_t width) {
+Span span_of(const View &t, int64_t B, int64_t H, int64_t N, int64_t width, int size = 2) {
     if (B <= 0 || H <= 0 || N <= 0 || !t.ptr || !t.strides) return {0, 0};
     const int64_t last = (B - 1) * t.strides[0] + (H - 1) * t.strides[1] + (N - 1) * t.strides[2] + width;
     const uintptr_t lo = reinterpret_cast<uintptr_t>(t.ptr);
-    return {lo, lo + (uintptr_t)last * 2};
+    return {lo, lo + (uintptr_t)last * size};
 }
 
 bool overlap(const Span &a, const Span &b) { return a.lo < b.hi && b.lo < a.hi; }
@@ -145,10 +145,12 @@ int check_alias_fwd(const View &x, const View &y, const View &z, const View &out
 // backward-shaped call: go, v (and the forward's output `o`, when given) of width dv, q, k of width
 // dqk in; dq, dk of width dqk and dv of width dv out
 int check_alias_bwd(const View &go, const View &q, const View &k, const View &v, const View *o, const View &dq,
-                    const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
+                    const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv,
+                    bool wide = false) {
+    const int size = wide ? 4 : 2;  // (FLA_GRADS_F32)
     const Span ins[] = {span_of(go, B, H, N, dv), span_of(q, B, H, N, dqk), span_of(k, B, H, N, dqk),
                         span_of(v, B, H, N, dv), o ? span_of(*o, B, H, N, dv) : Span{0, 0}};
-    const Span outs[] = {span_of(dq, B, H, N, dqk), span_of(dk, B, H, N, dqk), span_of(dvv, B, H, N, dv)};
+    const Span outs[] = {span_of(dq, B, H, N, dqk, size), span_of(dk, B, H, N, dqk, size), span_of(dvv, B, H, N, dv, size)};
     return check_alias(ins, 5, outs, 3);
 }
 
@@ -770,7 +772,7 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
 // as a reverse walk per half, the second adding to the first one's dV in memory, 279 us in three walks.
 int wide_backward(const WidePlan &wide, const View &go, const View &q, const View &k, const View &v, const View &dq,
                   const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
-                  const void *state_in, void *workspace, hipStream_t s, bool causal) {
+                  const void *state_in, void *workspace, hipStream_t s, bool causal, bool wide_out) {
     const WalkPlan &wp = wide.wp;
     char *ws = static_cast<char *>(workspace);
     const bool one_walk = state_in && dv <= 64 && !causal;
@@ -795,7 +797,7 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
     }
     fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, 128, dv);
     r.wqk2 = (int32_t)(dqk - 128);
-    r.init = entries[0], r.init2 = entries[1], r.init_is_totals = rev_sums_on_load;
+    r.init = entries[0], r.init2 = entries[1], r.init_is_totals = rev_sums_on_load, r.wide_out = wide_out;
     if (one_walk) {
         const char *half0 = static_cast<const char *>(state_in), *half1 = half0 + wp.saved_bytes;
         r.xinit = reinterpret_cast<const float *>(half0), r.xinit2 = reinterpret_cast<const float *>(half1);
@@ -805,9 +807,9 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
     }
     // dQ_h = lower(dO V^T) K_h + dO S_h^T: the forward walk over (dO, V, K_h)
     for (int h = 0; h < 2; ++h) {
-        fla::WalkParams w = lower_walk_params(wp, go, v, column_half(k, h), column_half(dq, h), B, H, N, dv, h ? dqk - 128 : 128,
-                                              fwd_entries[h]);
-        w.init_transposed = 1;
+        const View dq_h{static_cast<const char *>(dq.ptr) + h * 128 * (wide_out ? 4 : 2), dq.strides};
+        fla::WalkParams w = lower_walk_params(wp, go, v, column_half(k, h), dq_h, B, H, N, dv, h ? dqk - 128 : 128, fwd_entries[h]);
+        w.init_transposed = 1, w.wide_out = wide_out;
         if (fla::walk_fwd(dtype, wp.D, w, s) != hipSuccess) return FLA_ERR_LAUNCH;
     }
     r.dq = nullptr;
@@ -903,7 +905,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
 int chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                      const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap, WalkNorm *nx,
-                     bool causal);
+                     bool causal, bool wide_out);
 
 // fmap != 0 (feature_forward below): q and k hold the arguments xq, xk of the feature map phi, and
 // `mapped` = {phi(xq), phi(xk)} are outputs: the state kernel maps xk as it loads it and writes
@@ -1038,6 +1040,23 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
     return FLA_OK;
 }
 
+// whether walks that can store their results in fp32 (FLA_GRADS_F32) take a backward; `plain`: without feature map and normaliser
+bool wide_grads_walk(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk, const View &dvv,
+                     int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype, const void *state_in, bool plain) {
+    if (dtype != FLA_DTYPE_BF16) return false;
+    // (a (b, h) of a result stays within the 1 GiB that a descriptor's offsets reach, as 16-bit operands do)
+    for (const View *t : {&dq, &dk, &dvv})
+        if (N * t->strides[2] * 4 > fla::kMaxFastExtent) return false;
+    if (dqk > 128)
+        return plain && dv <= 64 && wide_plan(B, H, N, dqk, dv).ok && wide_fast_path(q, k, v, go, B, H, N, dqk, dv) &&
+               wide_fast_path(dq, dk, dvv, dvv, B, H, N, dqk, dv);
+    const WalkPlan wp = walk_plan(B, H, N, dqk, dv, plain);
+    if (!wp.ok || !(wp.split || state_in) || (!states_shareable(dqk, dv, N) && pad_index(dqk) == pad_index(dv))) return false;
+    return fla::fast_path_ok(make_params(go, v, k, dq, B, H, N, dv, dqk, 0)) &&
+           fla::fast_path_ok(make_params(k, q, go, dvv, B, H, N, dqk, dv, 1)) &&
+           fla::fast_path_ok(make_params(v, go, q, dk, B, H, N, dv, dqk, 1));
+}
+
 // whether the walk kernels take the normalised backward of these operands
 bool norm_walks_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                          const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, const void *state_in) {
@@ -1054,13 +1073,15 @@ bool norm_walks_backward(const View &go, const View &q, const View &k, const Vie
 int chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                      const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap = 0,
-                     WalkNorm *nx = nullptr, bool causal = false) {
+                     WalkNorm *nx = nullptr, bool causal = false, bool wide_out = false) {
     if (nx) nx->fused = nx->dk_pending = false;
     const View all[] = {go, q, k, v, dq, dk, dvv};
     for (const View &t : all)
         if (int rc = check_view(t)) return rc;
-    if (int rc = check_alias_bwd(go, q, k, v, nullptr, dq, dk, dvv, B, H, N, dqk, dv)) return rc;
+    if (int rc = check_alias_bwd(go, q, k, v, nullptr, dq, dk, dvv, B, H, N, dqk, dv, wide_out)) return rc;
     if (B == 0 || H == 0 || N == 0) return FLA_OK;
+    if (wide_out && !wide_grads_walk(go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, !fmap && !nx))
+        return FLA_ERR_UNSUPPORTED;
     // fmap != 0: q and k hold y = phi(x) (what the forward pass wrote), and the gradients leave as
     // gradients with respect to x: dQ and dK are multiplied by phi'(x), computed from y -- in the
     // kernels' epilogue on the fast path, by a pass of its own after the products otherwise.
@@ -1098,7 +1119,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                 return FLA_ERR_WORKSPACE;
             if (state_in && reinterpret_cast<uintptr_t>(state_in) % 16 != 0) return FLA_ERR_WORKSPACE;
             return wide_backward(wide, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace,
-                                 static_cast<hipStream_t>(stream), causal);
+                                 static_cast<hipStream_t>(stream), causal, wide_out);
         }
     }
     // (with the normaliser's terms still to be added by the caller, so is the slope)
@@ -1165,6 +1186,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
             r.init_is_totals = rev_sums_on_load;
             r.xinit = static_cast<const float *>(state_in);
             r.xtotal = reinterpret_cast<const float *>(static_cast<const char *>(state_in) + wp.entry_bytes);
+            r.wide_out = wide_out;
             return fla::walk_bwd_rev(dtype, wp.D, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
         }
         // dQ = lower(dO V^T) K + dO S^T: the forward walk over (dO, V, K), its states V^T K = S^T
@@ -1177,6 +1199,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         w.H = (int32_t)H, w.N = (int32_t)N, w.BH = (int32_t)(B * H), w.wqk = (int32_t)dv, w.wv = (int32_t)dqk;
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = wp.n_seg > 1 ? static_cast<const float *>(state_in) : nullptr, w.init_transposed = 1;
+        w.wide_out = wide_out;
         if (fmap) {  // q holds phi(xq): dQ leaves multiplied by the slope computed from it
             w.fmap = fmap, w.slope_y = q.ptr;
             w.sy_b = q.strides[0], w.sy_h = q.strides[1], w.sy_n = q.strides[2];
@@ -1196,7 +1219,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         r.H = (int32_t)H, r.N = (int32_t)N, r.BH = (int32_t)(B * H), r.wqk = (int32_t)dqk, r.wv = (int32_t)dv;
         r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
         r.init = entry, r.fmap = fmap;  // (dK: the slope from phi(xk) in the K tile)
-        r.init_is_totals = rev_sums_on_load;
+        r.init_is_totals = rev_sums_on_load, r.wide_out = wide_out;
         if (nx) r.dn = nx->dn, r.rc = wp.n_seg > 1 ? rcv : nullptr;  // dK's terms
         return fla::walk_dkdv(dtype, wp.D, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
@@ -1230,6 +1253,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = entry;
         w.saved = const_cast<void *>(state_in);
+        w.wide_out = wide_out;
         return fla::walk_bwd(dtype, wp.D, w, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
     if (wp.ok) state_in = nullptr;  // not in the 256-row chunks' format: recomputed below
@@ -1373,19 +1397,28 @@ int packed_backward(const PackPlan &p, const View &go, const View &q, const View
     return out.launch(stream);
 }
 
+// takes FLA_GRADS_F32 off a dtype
+bool take_wide_flag(int &dtype) {
+    const bool wide = (dtype & FLA_GRADS_F32) != 0;
+    dtype &= ~FLA_GRADS_F32;
+    return wide;
+}
+
 int plain_chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                            const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                            const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, bool causal) {
+    const bool wide_out = take_wide_flag(dtype);
     if (int rc = check_common(B, H, N, dtype)) return rc;
     if (dqk < 1 || dqk > 256) return FLA_ERR_HEAD_DIM;
     if (dv < 1 || dv > 256) return FLA_ERR_V_HEAD_DIM;
+    if (wide_out && (dv > 128 || dqk % 8 || dv % 8)) return FLA_ERR_UNSUPPORTED;
     // (causal, D_v above 128: product by product with the states of 256-row chunks in memory, each sum rounded once and no state
     // by subtraction, where the copies would run as column halves of v)
     if (const PackPlan p = pack_plan(B, H, N, dqk, dv); p.ok && !(causal && dv > 128))
         return packed_backward(p, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace, workspace_bytes,
                                stream, causal);
     return chunked_backward(go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace, workspace_bytes, stream, 0,
-                            nullptr, causal);
+                            nullptr, causal, wide_out);
 }
 
 // O = tril(phi(xq) phi(xk)^T) v with mapped = {phi(xq), phi(xk)} as further outputs.  Chunk-wise
@@ -1623,14 +1656,14 @@ int normalised_forward(const View &q0, const View &k0, const View &v, const View
 int normalised_backward(const View &go, const View &q, const View &k, const View &v, const View &o,
                         const float *denom, const View &dq, const View &dk, const View &dvv, int64_t B, int64_t H,
                         int64_t N, int64_t dqk, int64_t dv, int dtype, int chunked, void *workspace,
-                        int64_t workspace_bytes, void *stream, int fmap = 0, const void *state_in = nullptr) {
+                        int64_t workspace_bytes, void *stream, int fmap = 0, const void *state_in = nullptr, bool wide_out = false) {
     // fmap != 0: q, k hold phi(xq), phi(xk) and dq, dk leave as gradients with respect to xq, xk (the
     // slope is multiplied in by the last pass, after the normaliser's own terms have been added)
     const View all[] = {go, q, k, v, o, dq, dk, dvv};
     for (const View &t : all)
         if (int rc = check_view(t)) return rc;
     if (!denom) return FLA_ERR_NULL_POINTER;
-    if (int rc = check_alias_bwd(go, q, k, v, &o, dq, dk, dvv, B, H, N, dqk, dv)) return rc;
+    if (int rc = check_alias_bwd(go, q, k, v, &o, dq, dk, dvv, B, H, N, dqk, dv, wide_out)) return rc;
     if (B == 0 || H == 0 || N == 0) return FLA_OK;
     const NormLayout l = norm_layout(B, H, N, dqk, dv, chunked);
     if (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < l.norm_bytes + l.chunk_bytes)
@@ -1651,13 +1684,15 @@ int normalised_backward(const View &go, const View &q, const View &k, const View
     p.b = o.ptr, p.bs_b = o.strides[0], p.bs_h = o.strides[1], p.bs_n = o.strides[2], p.vec_b = vec_ok(o, dv);
     p.out = dO, p.os_b = do_strides[0], p.os_h = do_strides[1], p.os_n = do_strides[2], p.vec_out = vec_ok(dOv, dv);
     const bool walks = chunked && norm_walks_backward(dOv, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, state_in);
+    if (wide_out && !(walks && wide_grads_walk(dOv, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, false)))
+        return FLA_ERR_UNSUPPORTED;
     if (!walks && norm_launch(1, dtype, l.lpr, p, stream) != hipSuccess) return FLA_ERR_LAUNCH;
     // gradients of the unnormalised product
     WalkNorm nx{nullptr, 0.f, dn, ws + l.do_bytes + l.dn_bytes + 2 * l.sums_bytes, &go, &o, denom, p.vec_a && p.vec_b, false, false};
     if (chunked) {
         // the walk kernels add the normaliser's terms (and apply the slope of a feature map) themselves
         if (int rc = chunked_backward(dOv, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, ws + l.norm_bytes,
-                                      l.chunk_bytes, stream, fmap, &nx))
+                                      l.chunk_bytes, stream, fmap, &nx, false, wide_out))
             return rc;
         if (nx.fused && !nx.dk_pending) return FLA_OK;
     } else if (int rc = backward_products(dOv, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, stream)) {
@@ -1905,14 +1940,14 @@ int poly_chunked_forward(const View &xq, const View &xk, const View &v, const Vi
 int poly_chunked_backward(const View &go, const View &xq, const View &xk, const View &v, const View *o, const float *denom,
                           const View &dxq, const View &dxk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t r,
                           int64_t dv, const float *coef, int dtype, const void *state_in, void *workspace,
-                          int64_t workspace_bytes, void *stream) {
+                          int64_t workspace_bytes, void *stream, bool wide_out) {
     const View all[] = {go, xq, xk, v, dxq, dxk, dvv};
     for (const View &t : all)
         if (int rc = check_view(t)) return rc;
     if ((o == nullptr) != (denom == nullptr)) return FLA_ERR_NULL_POINTER;
     if (o)
         if (int rc = check_view(*o)) return rc;
-    if (int rc = check_alias_bwd(go, xq, xk, v, o, dxq, dxk, dvv, B, H, N, r, dv)) return rc;
+    if (int rc = check_alias_bwd(go, xq, xk, v, o, dxq, dxk, dvv, B, H, N, r, dv, wide_out)) return rc;
     if (B == 0 || H == 0 || N == 0) return FLA_OK;
     if (!state_in) return FLA_ERR_NULL_POINTER;
     const PolyPlan pl = poly_plan(B, H, N, r, dv);
@@ -1922,6 +1957,7 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
         return FLA_ERR_UNSUPPORTED;
     fla::PolyWalkParams w{};
     poly_common(w, pl, xq, xk, v, B, H, N, r, dv, coef);
+    w.wide_out = wide_out;
     w.go = go.ptr, w.gs_b = go.strides[0], w.gs_h = go.strides[1], w.gs_n = go.strides[2];
     if (o) w.o = o->ptr, w.os_b = o->strides[0], w.os_h = o->strides[1], w.os_n = o->strides[2];
     w.dq = const_cast<void *>(dxq.ptr), w.dqs_b = dxq.strides[0], w.dqs_h = dxq.strides[1], w.dqs_n = dxq.strides[2];
@@ -2200,13 +2236,14 @@ int fla_feature_attn_bwd(const void *grad_out, const void *xq, const void *xk, c
                          const int64_t *dv_strides, int feature_map, int dtype, const void *state_in, void *workspace,
                          int64_t workspace_bytes, void *stream) {
     // (xq, xk name the forward's q_out, k_out here: phi(xq), phi(xk))
+    const bool wide_out = take_wide_flag(dtype);
     if (int rc = check_common(B, H, N, dtype)) return rc;
     if (D_qk < 1 || D_qk > 256) return FLA_ERR_HEAD_DIM;
     if (D_v < 1 || D_v > 256) return FLA_ERR_V_HEAD_DIM;
     if (feature_map != FLA_MAP_ELU1 && feature_map != FLA_MAP_SOFTPLUS) return FLA_ERR_UNSUPPORTED;
     return chunked_backward({grad_out, go_strides}, {xq, xq_strides}, {xk, xk_strides}, {v, v_strides},
                             {dxq, dxq_strides}, {dxk, dxk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v, dtype,
-                            state_in, workspace, workspace_bytes, stream, feature_map);
+                            state_in, workspace, workspace_bytes, stream, feature_map, nullptr, false, wide_out);
 }
 
 int fla_linear_attn_chunked_bwd(const void *grad_out, const void *q, const void *k, const void *v, void *dq, void *dk,
@@ -2254,11 +2291,12 @@ int fla_feature_attn_normalised_bwd(const void *grad_out, const void *q, const v
                                     const int64_t *o_strides, const int64_t *dxq_strides, const int64_t *dxk_strides,
                                     const int64_t *dv_strides, int feature_map, int dtype, int chunked,
                                     const void *state_in, void *workspace, int64_t workspace_bytes, void *stream) {
+    const bool wide_out = take_wide_flag(dtype);
     if (int rc = check_norm_args(B, H, N, D_qk, D_v, dtype)) return rc;
     if (feature_map != FLA_MAP_ELU1 && feature_map != FLA_MAP_SOFTPLUS) return FLA_ERR_UNSUPPORTED;
     return normalised_backward({grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides}, {o, o_strides},
                                denom, {dxq, dxq_strides}, {dxk, dxk_strides}, {dv, dv_strides}, B, H, N, D_qk, D_v,
-                               dtype, chunked, workspace, workspace_bytes, stream, feature_map, state_in);
+                               dtype, chunked, workspace, workspace_bytes, stream, feature_map, state_in, wide_out);
 }
 
 int64_t fla_poly_attn_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v) {
@@ -2336,11 +2374,12 @@ int fla_poly_attn_chunked_bwd(const void *grad_out, const void *xq, const void *
                               const int64_t *v_strides, const int64_t *o_strides, const int64_t *dxq_strides,
                               const int64_t *dxk_strides, const int64_t *dv_strides, const float *coef, int dtype,
                               const void *state_in, void *workspace, int64_t workspace_bytes, void *stream) {
+    const bool wide_out = take_wide_flag(dtype);
     if (int rc = check_poly_args(B, H, N, R, D_v, dtype, coef)) return rc;
     const View ov{o, o_strides};
     return poly_chunked_backward({grad_out, go_strides}, {xq, xq_strides}, {xk, xk_strides}, {v, v_strides}, o ? &ov : nullptr,
                                  denom, {dxq, dxq_strides}, {dxk, dxk_strides}, {dv, dv_strides}, B, H, N, R, D_v, coef, dtype,
-                                 state_in, workspace, workspace_bytes, stream);
+                                 state_in, workspace, workspace_bytes, stream, wide_out);
 }
 
 int64_t fla_normalised_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int chunked) {
@@ -2368,10 +2407,11 @@ int fla_linear_attn_normalised_bwd(const void *grad_out, const void *q, const vo
                                    const int64_t *o_strides, const int64_t *dq_strides, const int64_t *dk_strides,
                                    const int64_t *dv_strides, int dtype, int chunked, const void *state_in,
                                    void *workspace, int64_t workspace_bytes, void *stream) {
+    const bool wide_out = take_wide_flag(dtype);
     if (int rc = check_norm_args(B, H, N, D_qk, D_v, dtype)) return rc;
     return normalised_backward({grad_out, go_strides}, {q, q_strides}, {k, k_strides}, {v, v_strides},
                                {o, o_strides}, denom, {dq, dq_strides}, {dk, dk_strides}, {dv, dv_strides}, B, H, N,
-                               D_qk, D_v, dtype, chunked, workspace, workspace_bytes, stream, 0, state_in);
+                               D_qk, D_v, dtype, chunked, workspace, workspace_bytes, stream, 0, state_in, wide_out);
 }
 
 }  // extern "C"

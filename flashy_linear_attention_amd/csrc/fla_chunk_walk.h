@@ -141,6 +141,11 @@ struct WalkParams {
     // state they formed to entry_out / entry_out2 (the layout of init; null: nowhere), for the backward walk.
     int32_t init_is_totals;
     float *entry_out, *entry_out2;
+    // walk_fwd_kernel as dQ's walk and the backward walks (but quad, and v wider than 64 beside a wide q / k), bf16: the results
+    // are stored in fp32 (o / dq, dk, dv then
+    // point to floats; what is stored is rounded to bf16 as always).  Kernels of their own (WIDE): as a branch in front of the
+    // stores it cost the others up to 3 %
+    int32_t wide_out;
     // A v of 129 .. 256 columns beside a wide q / k: its columns 128 .. are a second half of true width wv2, and grid y
     // picks a part of the work.  0: none.  1 (walk_fwd_wide_kernel): half y of v.  2, 3 (walk_bwd_rev_kernel): half y of
     // q / k with half y (2) or half 1 - y (3) of v, so that the two parts of a launch write different columns.
@@ -577,15 +582,50 @@ __device__ __forceinline__ void walk_store_packed(__amdgpu_buffer_rsrc_t rs, int
         }
 }
 
-// (PER: the blocks of acc that are this wave's -- the others belong to another wave or hold nothing)
+// ... the same values as fp32 (bf16: its bits with sixteen zeros behind them), four stores per block; stride_b: of a row, in bytes
+template <int D, int PER>
+__device__ __forceinline__ void walk_store_widened(__amdgpu_buffer_rsrc_t rs, int stride_b, int width, int row, int g, int db0,
+                                                   const u32x4 (&pk)[WalkCfg<D>::DBW][2]) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+#pragma unroll
+        for (int hq = 0; hq < 2; ++hq)
+#pragma unroll
+            for (int a = 0; a < 2; ++a) {
+                const int col = 32 * (db0 + i) + 16 * g + 8 * hq + 4 * a;
+                const uint32_t off = (uint32_t)(row * stride_b + col * 4) + (col < width ? 0u : kOobOffset);
+                const uint32_t lo = pk[i][hq][2 * a], hi = pk[i][hq][2 * a + 1];
+                __builtin_amdgcn_raw_buffer_store_b128(u32x4{lo << 16, lo & 0xffff0000u, hi << 16, hi & 0xffff0000u}, rs, off, 0, 0);
+            }
+}
+
+// (PER: the blocks of acc that are this wave's -- the others belong to another wave or hold nothing.  wide: WalkParams::wide_out,
+// stride2 then being a row of floats)
 template <typename T, int D, int PER = WalkCfg<D>::DBW>
 __device__ __forceinline__ void walk_store(__amdgpu_buffer_rsrc_t rs, int stride2, int width, int row, int g, int db0,
                                            const f32x16 (&acc)[WalkCfg<D>::DBW], int fmap = 0,
-                                           const unsigned char *ytile = nullptr, int trow = 0) {
+                                           const unsigned char *ytile = nullptr, int trow = 0, int wide = 0) {
     u32x4 pk[WalkCfg<D>::DBW][2];
     walk_pack<T, D, PER>(acc, g, db0, pk, fmap, ytile, trow);
+    if constexpr (std::is_same<T, __bf16>::value) {
+        if (wide) {
+            walk_store_widened<D, PER>(rs, stride2, width, row, g, db0, pk);
+            return;
+        }
+    }
     walk_store_packed<D, PER>(rs, stride2, width, row, g, db0, pk);
 }
+
+// Where a result of (b, h) starts and its rows' stride and descriptor, for 16-bit or fp32 storage
+struct WalkResult {
+    __amdgpu_buffer_rsrc_t rs;
+    int stride;  // bytes
+    __device__ __forceinline__ WalkResult(void *base, int64_t at, int64_t stride_n, int width, int N, int wide) {
+        const int size = wide ? 4 : 2;
+        stride = (int)stride_n * size;
+        rs = __builtin_amdgcn_make_buffer_rsrc(static_cast<char *>(base) + at * size, 0, (N - 1) * stride + width * size, 0x00020000);
+    }
+};
 
 // What a result's place in memory holds before the walk adds to it: this lane's 16-byte pieces of the
 // row it will store (the pieces of walk_store_packed).  Ordinary loads, requested once a chunk's tiles
@@ -1043,7 +1083,7 @@ __device__ __forceinline__ void walk_write_state(float *out, int wave, int lane,
 template <typename T, int NORM, bool FM>
 constexpr bool walk_fwd_scaled = std::is_same<T, _Float16>::value && NORM == 0 && !FM;
 
-template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32>
+template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool WIDE = false>
 __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1069,12 +1109,11 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
     const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
-    T *O = static_cast<T *>(p.o) + b * p.os_b + h * p.os_h;
-    const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2, os2 = (int)p.os_n * 2;
+    const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2;
     const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
     const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
     const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
-    const __amdgpu_buffer_rsrc_t ro = __builtin_amdgcn_make_buffer_rsrc(O, 0, (N - 1) * os2 + p.wv * 2, 0x00020000);
+    const WalkResult ro(p.o, b * p.os_b + h * p.os_h, p.os_n, p.wv, N, WIDE);
 
     f32x16 st[W::NBW];
     walk_load_init<D, B>(p, sl, wave, lane, st, false);
@@ -1226,7 +1265,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                         acc[i][v] *= feature_slope_c<decltype(map)::value>(static_cast<float>(ys[i][v / 8][v % 8]));
             });
         }
-        walk_store<T, D, OB::PER>(ro, os2, p.wv, row, g, db0, acc);
+        walk_store<T, D, OB::PER>(ro.rs, ro.stride, p.wv, row, g, db0, acc, 0, nullptr, 0, WIDE);
         walk_update<T, D, B>(tk, tv, wave, lane, st);
         if constexpr (SCALED) walk_state_max<D, B>(smax, wave, lane, st);
         if constexpr (NORM == 1) {
@@ -1401,7 +1440,7 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
 // (Obtained backwards instead -- from the state at the segment's end, subtracting every chunk's K^T V when the walk reaches
 // it -- one late row that is infinite, NaN or merely huge spoiled the dQ of every chunk before it.  Forward + backward
 // at B H 16, N 32768, D 64 that way 222 us, this way 234.)
-template <typename T, int D, bool NORM>
+template <typename T, int D, bool NORM, bool WIDE = false>
 __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1416,7 +1455,8 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
     const float *vz = reinterpret_cast<const float *>(tl + W::STATE), *vd = vz + 512;
     float *vr = reinterpret_cast<float *>(tl + W::STATE) + 256, *rpart = vr + 512;
     const uint32_t xbase = lds0 + 4 * W::TILE + W::STATE;
-    const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
+    const int tid = threadIdx.x;
+    int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const WalkSlice sl = walk_slice(p);
     if (!sl.valid) return;
@@ -1425,18 +1465,14 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
     const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
     const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
-    T *DQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h;
-    T *DK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h;
-    T *DV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
     const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2, gs2 = (int)p.gs_n * 2;
-    const int dqs2 = (int)p.dqs_n * 2, dks2 = (int)p.dks_n * 2, dvs2 = (int)p.dvs_n * 2;
     const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
     const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
     const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
     const u32x4 rg = make_rsrc(G, (uint32_t)((N - 1) * gs2 + p.wv * 2));
-    const __amdgpu_buffer_rsrc_t rdq = __builtin_amdgcn_make_buffer_rsrc(DQ, 0, (N - 1) * dqs2 + p.wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdk = __builtin_amdgcn_make_buffer_rsrc(DK, 0, (N - 1) * dks2 + p.wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdv = __builtin_amdgcn_make_buffer_rsrc(DV, 0, (N - 1) * dvs2 + p.wv * 2, 0x00020000);
+    const WalkResult rdq(p.dq, b * p.dqs_b + h * p.dqs_h, p.dqs_n, p.wqk, N, WIDE);
+    const WalkResult rdk(p.dk, b * p.dks_b + h * p.dks_h, p.dks_n, p.wqk, N, WIDE);
+    const WalkResult rdv(p.dv, b * p.dvs_b + h * p.dvs_h, p.dvs_n, p.wv, N, WIDE);
 
     f32x16 st[W::NBW];  // R[q/k index][v index]
     walk_load_init<D>(p, sl, wave, lane, st, true);
@@ -1462,6 +1498,10 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 
 #pragma unroll 1
     for (int c = sl.c_hi - 1; c >= sl.c_lo; --c) {
+        // (NORM, WIDE: LDS addresses that depend on the lane alone would be computed ahead of the loop and held in registers, to the
+        // point of spilling)
+        if constexpr (NORM && WIDE) asm volatile("" : "+v"(lane));
+        const int l32 = lane & 31, g = lane >> 5;
         const int row0 = c * W::C;
         const int64_t at = (int64_t)sl.bh * p.n_chunks + c;
         walk_load_tile<D>(rq, lds0, row0, qs2, p.wqk, wave, lane);
@@ -1487,7 +1527,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
                 return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
             }, acc, &ax);
             walk_add_vec<D>(acc, ax, vz, 0, g);
-            walk_store<T, D>(rdq, dqs2, p.wqk, row, g, 0, acc, p.fmap, tq, 32 * wave + l32);
+            walk_store<T, D>(rdq.rs, rdq.stride, p.wqk, row, g, 0, acc, p.fmap, tq, 32 * wave + l32, WIDE);
             __syncthreads();  // every wave has read dQ's state
             walk_state_to_lds<T, D>(tl, wave, lane, st);
             __syncthreads();
@@ -1496,7 +1536,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
         walk_product<T, D, true>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
         }, acc);
-        walk_store<T, D>(rdv, dvs2, p.wv, row, g, 0, acc);
+        walk_store<T, D>(rdv.rs, rdv.stride, p.wv, row, g, 0, acc, 0, nullptr, 0, WIDE);
         // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
         // (normaliser: scores + dn_i with i the dO row, result + rc)
         if constexpr (NORM) {
@@ -1511,13 +1551,13 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
                 return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
             }, acc);
         }
-        walk_store<T, D>(rdk, dks2, p.wqk, row, g, 0, acc, p.fmap, tk, 32 * wave + l32);
+        walk_store<T, D>(rdk.rs, rdk.stride, p.wqk, row, g, 0, acc, p.fmap, tk, 32 * wave + l32, WIDE);
         if constexpr (!NORM) {
             // dQ = lower(dO V^T) K + dO S_c^T: A operand S_c[q/k index][v index], its LDS copy read transposed
             walk_product<T, D, false>(tg, tv, tk, wave, lane, c > 0, [&](int db, int kc) -> V8 {
                 return walk_col_frag_perm<T, D>(tx, 16 * kc, db, lane, true);
             }, acc);
-            walk_store<T, D>(rdq, dqs2, p.wqk, row, g, 0, acc, p.fmap, tq, 32 * wave + l32);
+            walk_store<T, D>(rdq.rs, rdq.stride, p.wqk, row, g, 0, acc, p.fmap, tq, 32 * wave + l32, WIDE);
         }
         walk_update<T, D>(tq, tg, wave, lane, st);
         if constexpr (NORM) walk_weighted_sums_to_lds<D>(rpart, wave, lane, walk_weighted_sums<T, D>(tq, vd, wave, lane));
@@ -1543,7 +1583,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 // D = 128, so the chunk's dn comes as ordinary loads, a chunk ahead, in the order in which the scores' registers take it, and
 // rc is carried in registers: a wave adds up its own output columns, in the order of an MFMA's A rows, and one MFMA
 // per 32 columns adds rc to the result (walk_split3).
-template <typename T, int D, bool NORM, int NQ = D / 32, int NV = D / 32>
+template <typename T, int D, bool NORM, int NQ = D / 32, int NV = D / 32, bool WIDE = false>
 __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1565,16 +1605,13 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
     const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
     const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
-    T *DK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h;
-    T *DV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
     const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2, gs2 = (int)p.gs_n * 2;
-    const int dks2 = (int)p.dks_n * 2, dvs2 = (int)p.dvs_n * 2;
     const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
     const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
     const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
     const u32x4 rg = make_rsrc(G, (uint32_t)((N - 1) * gs2 + p.wv * 2));
-    const __amdgpu_buffer_rsrc_t rdk = __builtin_amdgcn_make_buffer_rsrc(DK, 0, (N - 1) * dks2 + p.wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdv = __builtin_amdgcn_make_buffer_rsrc(DV, 0, (N - 1) * dvs2 + p.wv * 2, 0x00020000);
+    const WalkResult rdk(p.dk, b * p.dks_b + h * p.dks_h, p.dks_n, p.wqk, N, WIDE);
+    const WalkResult rdv(p.dv, b * p.dvs_b + h * p.dvs_h, p.dvs_n, p.wv, N, WIDE);
 
     f32x16 st[W::NBW];  // R[q/k index][v index]
     walk_load_init<D, B>(p, sl, wave, lane, st, true);
@@ -1662,7 +1699,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         walk_product<T, D, true, 0, B::KQ, NV>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
         }, acc);
-        walk_store<T, D, OV::PER>(rdv, dvs2, p.wv, row, g, OV::db0(wave), acc);
+        walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, p.wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
         // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
         if constexpr (NORM) {
             walk_product<T, D, true, 3>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
@@ -1677,7 +1714,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
                 return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
             }, acc);
         }
-        walk_store<T, D, OQ::PER>(rdk, dks2, p.wqk, row, g, db0, acc, p.fmap, tk, 32 * rb + l32);
+        walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, p.wqk, row, g, db0, acc, p.fmap, tk, 32 * rb + l32, WIDE);
         walk_update<T, D, B>(tq, tg, wave, lane, st);
         if constexpr (NORM) {  // rc += this chunk's dn_i q_i
             static_for<0, W::C / 16>([&](auto j) {
@@ -1712,7 +1749,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 // The one 16-bit state in LDS holds R for dV and dK, then X for dQ.  q, k, v, dO are read once and
 // nothing but the results is written, where the walk for dQ followed by walk_dkdv_kernel reads
 // dO, v, k twice.
-template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool ACCUM = false, bool FM = false>
+template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool ACCUM = false, bool FM = false, bool WIDE = false>
 __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1740,18 +1777,15 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h + qh * D;
     const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h + vh * D;
     const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h + vh * D;
-    T *DQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h + qh * D;
-    T *DK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h + qh * D;
-    T *DV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h + vh * D;
     const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2, gs2 = (int)p.gs_n * 2;
-    const int dqs2 = (int)p.dqs_n * 2, dks2 = (int)p.dks_n * 2, dvs2 = (int)p.dvs_n * 2;
     const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + wqk * 2));
     const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + wqk * 2));
     const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + wv * 2));
     const u32x4 rg = make_rsrc(G, (uint32_t)((N - 1) * gs2 + wv * 2));
-    const __amdgpu_buffer_rsrc_t rdq = __builtin_amdgcn_make_buffer_rsrc(DQ, 0, (N - 1) * dqs2 + wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdk = __builtin_amdgcn_make_buffer_rsrc(DK, 0, (N - 1) * dks2 + wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdv = __builtin_amdgcn_make_buffer_rsrc(DV, 0, (N - 1) * dvs2 + wv * 2, 0x00020000);
+    static_assert(!WIDE || !ACCUM, "what is added to is 16-bit");
+    const WalkResult rdq(p.dq, b * p.dqs_b + h * p.dqs_h + qh * D, p.dqs_n, wqk, N, WIDE);
+    const WalkResult rdk(p.dk, b * p.dks_b + h * p.dks_h + qh * D, p.dks_n, wqk, N, WIDE);
+    const WalkResult rdv(p.dv, b * p.dvs_b + h * p.dvs_h + vh * D, p.dvs_n, wv, N, WIDE);
 
     f32x16 st[W::NBW];  // R [q/k index][v index]
     f32x16 xs[W::NBW];  // X [q/k index][v index]
@@ -1792,7 +1826,7 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
         sync();  // the tiles have landed, R is in LDS
         const int row = c * W::C + 32 * rb + l32;
         const bool later = c + 1 < p.n_chunks;  // chunks after this one exist: R is not identically zero
-        if constexpr (ACCUM) prev.request(rdv, dvs2, wv, row, g, OV::db0(wave));
+        if constexpr (ACCUM) prev.request(rdv.rs, rdv.stride, wv, row, g, OV::db0(wave));
         walk_update<T, D, B, true, true>(tk, tv, wave, lane, xs);  // X: now the sum over the chunks before this one
         f32x16 acc[W::DBW];
         // dV = upper(K Q^T) dO + K R: A operand R^T[v index][q/k index] = the LDS copy as it is
@@ -1800,14 +1834,14 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
             return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
         }, acc);
         if constexpr (ACCUM) prev.add_to(acc);
-        walk_store<T, D, OV::PER>(rdv, dvs2, wv, row, g, OV::db0(wave), acc);
-        if constexpr (ACCUM) prev_qk.request(rdk, dks2, wqk, row, g, OQ::db0(wave));
+        walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
+        if constexpr (ACCUM) prev_qk.request(rdk.rs, rdk.stride, wqk, row, g, OQ::db0(wave));
         // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
         walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
         if constexpr (ACCUM) prev_qk.add_to(acc);
-        walk_store<T, D, OQ::PER>(rdk, dks2, wqk, row, g, OQ::db0(wave), acc, fmap, tk, 32 * rb + l32);
+        walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, wqk, row, g, OQ::db0(wave), acc, fmap, tk, 32 * rb + l32, WIDE);
         // R += Q^T dO touches registers and tiles only, so it can sit on either side of the barriers: the waves of
         // the last row block, with one score block in dV and dK against two, take it here, the others after dQ,
         // where they have one score block against two
@@ -1823,13 +1857,13 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
             asm volatile("" : "+a"(xs[0]), "+a"(xs[1]));
         walk_state_to_lds<T, D, B>(tl, wave, lane, xs);
         sync();  // X is in LDS
-        if constexpr (ACCUM) prev_qk.request(rdq, dqs2, wqk, row, g, OQ::db0(wave));
+        if constexpr (ACCUM) prev_qk.request(rdq.rs, rdq.stride, wqk, row, g, OQ::db0(wave));
         // dQ = lower(dO V^T) K + dO X^T: A operand X[q/k index][v index], read transposed like R for dK
         walk_product<T, D, false, 0, B::KV, NQ>(tg, tv, tk, wave, lane, c > 0, [&](int db, int kc) -> V8 {
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
         if constexpr (ACCUM) prev_qk.add_to(acc);
-        walk_store<T, D, OQ::PER>(rdq, dqs2, wqk, row, g, OQ::db0(wave), acc, fmap, tq, 32 * rb + l32);
+        walk_store<T, D, OQ::PER>(rdq.rs, rdq.stride, wqk, row, g, OQ::db0(wave), acc, fmap, tq, 32 * rb + l32, WIDE);
         if (!(kSplitUpdate && rb == 1)) walk_update<T, D, B, false, true>(tq, tg, wave, lane, st);
         sync();  // every wave has read X and is done with the tiles
         walk_state_to_lds<T, D, B>(tl, wave, lane, st);
@@ -1849,7 +1883,7 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
 // LDS as in walk_fwd_wide_kernel: a set of (Q_h, K_h) tiles per half, two (V, dO) pairs by chunk parity, and ONE
 // 16-bit state that holds R_h, then X_h, of the half at work; at the end of a half-chunk the other half's R (in
 // registers throughout) is rounded into it.  With dQ four states in registers: built for v blocks NV = 2 only.
-template <typename T, int NV, bool WITH_DQ>
+template <typename T, int NV, bool WITH_DQ, bool WIDE = false>
 __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int D = 128, NQ = D / 32;
@@ -1872,22 +1906,17 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
     const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
     const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
-    T *DQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h;
-    T *DK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h;
-    T *DV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
     const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2, gs2 = (int)p.gs_n * 2;
-    const int dqs2 = (int)p.dqs_n * 2, dks2 = (int)p.dks_n * 2, dvs2 = (int)p.dvs_n * 2;
     const u32x4 rq0 = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
     const u32x4 rk0 = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
     const u32x4 rq1 = make_rsrc(Q + D, (uint32_t)((N - 1) * qs2 + p.wqk2 * 2));
     const u32x4 rk1 = make_rsrc(K + D, (uint32_t)((N - 1) * ks2 + p.wqk2 * 2));
     const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
     const u32x4 rg = make_rsrc(G, (uint32_t)((N - 1) * gs2 + p.wv * 2));
-    const __amdgpu_buffer_rsrc_t rdq0 = __builtin_amdgcn_make_buffer_rsrc(DQ, 0, (N - 1) * dqs2 + p.wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdk0 = __builtin_amdgcn_make_buffer_rsrc(DK, 0, (N - 1) * dks2 + p.wqk * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdq1 = __builtin_amdgcn_make_buffer_rsrc(DQ + D, 0, (N - 1) * dqs2 + p.wqk2 * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdk1 = __builtin_amdgcn_make_buffer_rsrc(DK + D, 0, (N - 1) * dks2 + p.wqk2 * 2, 0x00020000);
-    const __amdgpu_buffer_rsrc_t rdv = __builtin_amdgcn_make_buffer_rsrc(DV, 0, (N - 1) * dvs2 + p.wv * 2, 0x00020000);
+    const int64_t dq_at = b * p.dqs_b + h * p.dqs_h, dk_at = b * p.dks_b + h * p.dks_h;
+    const WalkResult rdq0(p.dq, dq_at, p.dqs_n, p.wqk, N, WIDE), rdq1(p.dq, dq_at + D, p.dqs_n, p.wqk2, N, WIDE);
+    const WalkResult rdk0(p.dk, dk_at, p.dks_n, p.wqk, N, WIDE), rdk1(p.dk, dk_at + D, p.dks_n, p.wqk2, N, WIDE);
+    const WalkResult rdv(p.dv, b * p.dvs_b + h * p.dvs_h, p.dvs_n, p.wv, N, WIDE);
 
     f32x16 st0[W::NBW], st1[W::NBW];  // R_0, R_1
     f32x16 xs0[W::NBW], xs1[W::NBW];  // X_0, X_1
@@ -1962,7 +1991,7 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
             walk_product<T, D, true, 0, B::KQ, NV, HF != 0>(tk, tq, tg, wave, lane, later, rows_of_state, dvacc);
             f32x16 acc[W::DBW];
             walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, cols_of_state, acc);
-            walk_store<T, D, OQ::PER>(HF ? rdk1 : rdk0, dks2, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc);
+            walk_store<T, D, OQ::PER>((HF ? rdk1 : rdk0).rs, rdk0.stride, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc, 0, nullptr, 0, WIDE);
             if constexpr (WITH_DQ) {
                 sync();  // every wave has read R_h
                 // (X stays in its accumulation registers up to here: without this the copies that the rounding
@@ -1971,9 +2000,9 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
                 walk_state_to_lds<T, D, B>(tl, wave, lane, xs);
                 sync();  // X_h is in LDS
                 walk_product<T, D, false, 0, B::KV, NQ>(tg, tv, tk, wave, lane, c > 0, cols_of_state, acc);
-                walk_store<T, D, OQ::PER>(HF ? rdq1 : rdq0, dqs2, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc);
+                walk_store<T, D, OQ::PER>((HF ? rdq1 : rdq0).rs, rdq0.stride, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc, 0, nullptr, 0, WIDE);
             }
-            if constexpr (HF != 0) walk_store<T, D, OV::PER>(rdv, dvs2, p.wv, row, g, OV::db0(wave), dvacc);
+            if constexpr (HF != 0) walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, p.wv, row, g, OV::db0(wave), dvacc, 0, nullptr, 0, WIDE);
             walk_update<T, D, B, false, true>(tq, tg, wave, lane, st);  // R_h += Q_h^T dO
             sync();  // every wave has read the state's copy and is done with this half's tiles
             walk_state_to_lds<T, D, B>(tl, wave, lane, st_next);
@@ -2573,8 +2602,15 @@ hipError_t launch_walk_kernel(int64_t grid, int smem, const WalkParams &p, hipSt
     return launch_kernel<kern>(dim3((unsigned)grid, (unsigned)parts), dim3(256), smem, stream, p);
 }
 
-template <typename T, int D>
+template <typename T, int D, bool WIDE = false>
 hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
+    if constexpr (!WIDE) {
+        if (p.wide_out) {  // (dQ's walk)
+            if constexpr (D == 128 && std::is_same<T, __bf16>::value) return launch_walk_fwd<T, D, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    }
+    constexpr int NB = D / 32;
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr bool kDouble = D > 64;  // (the plan's workgroup count must match: one per CU when double)
@@ -2584,24 +2620,26 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     // (segment totals in place of entry states: the D = 128 walks, by the flag; below that by the number of segments)
     if (p.init_is_totals && (D != 128 || p.n_seg < 3 || !p.init)) return hipErrorInvalidValue;
     if (p.entry_out && (!p.init_is_totals || p.dn || p.slope_y)) return hipErrorInvalidValue;
+    if (WIDE && p.denom) return hipErrorInvalidValue;
     if (p.denom || p.dn) {  // the normaliser's terms: its vectors live behind the state
         if ((p.dn && !p.zc) || (p.denom && p.n_seg > 1 && !p.vsum)) return hipErrorInvalidValue;
         constexpr int smem_n = smem + (kDouble ? 2 : 1) * WalkCfg<D>::VEC;
-        if (p.denom)
-            return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 1, true>>(grid, smem_n, p, stream)
-                      : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 1, false>>(grid, smem_n, p, stream);
-        return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, true>>(grid, smem_n, p, stream)
-                  : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, false>>(grid, smem_n, p, stream);
+        if constexpr (!WIDE)
+            if (p.denom)
+                return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 1, true>>(grid, smem_n, p, stream)
+                          : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 1, false>>(grid, smem_n, p, stream);
+        return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, true, NB, NB, WIDE>>(grid, smem_n, p, stream)
+                  : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, false, NB, NB, WIDE>>(grid, smem_n, p, stream);
     }
-    if (fm) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true>>(grid, smem, p, stream);
+    if (fm) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true, NB, NB, WIDE>>(grid, smem, p, stream);
     if constexpr (D == 128) {
         // operands of at most 64 true columns on a side (the halves of a wide q / k, a narrow v): the kernels that
         // leave out the blocks of padding, which the states in memory may not hold either
-        if (p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2>>(grid, smem, p, stream);
-        if (p.wqk <= 64 && p.wv > 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4>>(grid, smem, p, stream);
-        if (p.wqk <= 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 2>>(grid, smem, p, stream);
+        if (p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2, WIDE>>(grid, smem, p, stream);
+        if (p.wqk <= 64 && p.wv > 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4, WIDE>>(grid, smem, p, stream);
+        if (p.wqk <= 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 2, WIDE>>(grid, smem, p, stream);
     }
-    return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false>>(grid, smem, p, stream);
+    return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, NB, NB, WIDE>>(grid, smem, p, stream);
 }
 
 template <typename T>
@@ -2623,58 +2661,79 @@ hipError_t launch_walk_fwd_wide(const WalkParams &p, hipStream_t stream) {
     return launch_walk_kernel<walk_fwd_wide_kernel<T, 4>>(grid, smem, p, stream);
 }
 
-template <typename T, int D>
+template <typename T, int D, bool WIDE = false>
 hipError_t launch_walk_bwd(const WalkParams &p, hipStream_t stream) {
+    if constexpr (!WIDE) {
+        if (p.wide_out) {
+            if constexpr (std::is_same<T, __bf16>::value) return launch_walk_bwd<T, D, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    }
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr int smem = 4 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     if (p.dn) {
         if (!p.zc || !p.saved || (p.n_seg > 1 && !p.rc)) return hipErrorInvalidValue;
-        constexpr auto kern = walk_bwd_kernel<T, D, true>;
+        constexpr auto kern = walk_bwd_kernel<T, D, true, WIDE>;
         constexpr int smem_n = smem + WalkCfg<D>::VEC + 1024;
         if (hipError_t e = ensure_dynamic_lds<kern>(smem_n)) return e;
         return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_n, stream, p);
     }
     if (!p.saved) return hipErrorInvalidValue;
-    constexpr auto kern = walk_bwd_kernel<T, D, false>;
+    constexpr auto kern = walk_bwd_kernel<T, D, false, WIDE>;
     constexpr int smem_x = smem + WalkCfg<D>::STATE;  // dQ's state beside R
     if (hipError_t e = ensure_dynamic_lds<kern>(smem_x)) return e;
     return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_x, stream, p);
 }
 
-template <typename T, int D>
+template <typename T, int D, bool WIDE = false>
 hipError_t launch_walk_dkdv(const WalkParams &p, hipStream_t stream) {
+    if constexpr (!WIDE) {
+        if (p.wide_out) {
+            if constexpr (std::is_same<T, __bf16>::value) return launch_walk_dkdv<T, D, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    }
+    constexpr int NB = D / 32;
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr int smem = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     static_assert(smem <= 160 * 1024, "two sets of tiles and the state must fit the LDS of a CU");
     if (p.dn) {
         if (p.n_seg > 1 && !p.rc) return hipErrorInvalidValue;
-        constexpr auto kern = walk_dkdv_kernel<T, D, true>;
+        constexpr auto kern = walk_dkdv_kernel<T, D, true, NB, NB, WIDE>;
         if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
         return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
     }
     if constexpr (D == 128) {
         if (!p.fmap && p.wqk > 64 && p.wv <= 64) {
-            constexpr auto kern = walk_dkdv_kernel<T, D, false, 4, 2>;
+            constexpr auto kern = walk_dkdv_kernel<T, D, false, 4, 2, WIDE>;
             if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
             return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
         }
     }
-    constexpr auto kern = walk_dkdv_kernel<T, D, false>;
+    constexpr auto kern = walk_dkdv_kernel<T, D, false, NB, NB, WIDE>;
     if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
     return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
 }
 
-template <typename T, int D>
+template <typename T, int D, bool WIDE = false>
 hipError_t launch_walk_bwd_rev(const WalkParams &p, hipStream_t stream) {
+    if constexpr (!WIDE) {
+        if (p.wide_out) {
+            if constexpr (std::is_same<T, __bf16>::value) return launch_walk_bwd_rev<T, D, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    }
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     if (!p.xtotal || (p.n_seg > 1 && !p.xinit)) return hipErrorInvalidValue;
     if (p.entry_out || (p.accumulate && !p.quad) || (p.init_is_totals && (p.n_seg < 3 || !p.init))) return hipErrorInvalidValue;
     constexpr int smem = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     static_assert(smem <= 160 * 1024, "two sets of tiles and the state must fit the LDS of a CU");
+    constexpr int NB = D / 32;
     if (p.quad) {
+        if (WIDE) return hipErrorNotSupported;
         if ((p.quad != 2 && p.quad != 3) || p.wqk != 128 || p.wv != 128 || p.wqk2 < 1 || p.wqk2 > 128 || p.wv2 < 1 ||
             p.wv2 > 128 || p.fmap)
             return hipErrorInvalidValue;
@@ -2682,14 +2741,20 @@ hipError_t launch_walk_bwd_rev(const WalkParams &p, hipStream_t stream) {
                             : launch_walk_kernel<walk_bwd_rev_kernel<T, D>>(grid, smem, p, stream, 2);
     }
     if constexpr (D == 128) {  // a half of a wide q / k against a narrow v: without the blocks of padding
-        if (!p.fmap && p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2>>(grid, smem, p, stream);
+        if (!p.fmap && p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2, false, false, WIDE>>(grid, smem, p, stream);
     }
-    if (p.fmap) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, false, true>>(grid, smem, p, stream);
-    return launch_walk_kernel<walk_bwd_rev_kernel<T, D>>(grid, smem, p, stream);
+    if (p.fmap) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, NB, NB, false, true, WIDE>>(grid, smem, p, stream);
+    return launch_walk_kernel<walk_bwd_rev_kernel<T, D, NB, NB, false, false, WIDE>>(grid, smem, p, stream);
 }
 
-template <typename T>
+template <typename T, bool WIDE = false>
 hipError_t launch_walk_bwd_rev_wide(const WalkParams &p, hipStream_t stream) {
+    if constexpr (!WIDE) {
+        if (p.wide_out) {
+            if constexpr (std::is_same<T, __bf16>::value) return launch_walk_bwd_rev_wide<T, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    }
     using W = WalkCfg<128>;
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
@@ -2701,10 +2766,13 @@ hipError_t launch_walk_bwd_rev_wide(const WalkParams &p, hipStream_t stream) {
     static_assert(smem <= 160 * 1024, "the tiles and the state must fit the LDS of a CU");
     if (p.dq) {
         if (!p.xtotal || !p.xtotal2 || (p.n_seg > 1 && (!p.xinit || !p.xinit2))) return hipErrorInvalidValue;
-        return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, true>>(grid, smem, p, stream);
+        return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, true, WIDE>>(grid, smem, p, stream);
     }
-    return p.wv <= 64 ? launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, false>>(grid, smem, p, stream)
-                      : launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 4, false>>(grid, smem, p, stream);
+    if (p.wv <= 64) return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, false, WIDE>>(grid, smem, p, stream);
+    if constexpr (WIDE)  // (40 bytes of spills, which this kernel may not have)
+        return hipErrorNotSupported;
+    else
+        return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 4, false>>(grid, smem, p, stream);
 }
 
 }  // namespace fla

@@ -51,6 +51,7 @@ struct PolyWalkParams {
     int64_t dqs_b, dqs_h, dqs_n, dks_b, dks_h, dks_n, dvs_b, dvs_h, dvs_n;
     int32_t H, N, BH, r, wv, n_chunks, seg_chunks, n_seg;
     float c0, c1, c2, eps;
+    int32_t wide_out;  // dq, dk, dv are floats (and receive the bf16-rounded values)
     float *denom;  // fp32 [BH][N], or null: not normalised.  Forward writes it, backward reads it
     // states [BH][n_seg][PolyFeatures::kState] in fp32
     float *totals;       // totals kernel: receives the segments' sums; walks: those (sum_entries) or the entry states, of
@@ -542,16 +543,24 @@ __device__ __forceinline__ void poly_get_acc(const unsigned char *ex, int wave, 
     }
 }
 
-// sixteen consecutive columns (from column `col`) of a row, rounded and stored as two chunks
+// sixteen consecutive columns (from column `col`) of a row, rounded and stored as two chunks; wide: dst and at (of the row) in floats
 template <typename T>
-__device__ __forceinline__ void poly_store16(T *dst, const float (&f)[16], int col, int width) {
+__device__ __forceinline__ void poly_store16(void *dst, int64_t at, const float (&f)[16], int col, int width, int wide = 0) {
 #pragma unroll
     for (int h = 0; h < 2; ++h)
         if (col + 8 * h < width) {
             float e[8];
 #pragma unroll
             for (int j = 0; j < 8; ++j) e[j] = f[8 * h + j];
-            *reinterpret_cast<u32x4 *>(dst + col + 8 * h) = __builtin_bit_cast(u32x4, poly_round8<T>(e));
+            const u32x4 w = __builtin_bit_cast(u32x4, poly_round8<T>(e));
+            if (wide) {
+                u32x4 *to = reinterpret_cast<u32x4 *>(static_cast<float *>(dst) + at + col + 8 * h);
+#pragma unroll
+                for (int a = 0; a < 2; ++a)
+                    to[a] = u32x4{w[2 * a] << 16, w[2 * a] & 0xffff0000u, w[2 * a + 1] << 16, w[2 * a + 1] & 0xffff0000u};
+            } else {
+                *reinterpret_cast<u32x4 *>(static_cast<T *>(dst) + at + col + 8 * h) = w;
+            }
         }
 }
 
@@ -805,7 +814,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) f[i] = (poly_pick(kh, acc[1][i], acc[0][i]) + other[i]) * inv;
-        if (row < N) poly_store16<T>(O + (int64_t)row * p.us_n, f, 32 * kh + 16 * g, p.wv);
+        if (row < N) poly_store16<T>(O, (int64_t)row * p.us_n, f, 32 * kh + 16 * g, p.wv);
     }
 #else
     (void)p;
@@ -886,7 +895,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
     const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
     const T *O = NORM ? static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h : nullptr;
     const float *den = NORM ? p.denom + (int64_t)sl.bh * N : nullptr;
-    T *dQ = static_cast<T *>(p.dq) + b * p.dqs_b + h * p.dqs_h;
+    const int64_t dq_at = b * p.dqs_b + h * p.dqs_h;
     const float c1 = p.c1, c2 = p.c2;
     unsigned char *tq = smem + L::qQ, *tk = smem + L::qK, *tkt = smem + L::qKt, *tv = smem + L::qV, *tg = smem + L::qG,
                   *ts = smem + L::qS, *exch = smem + L::qEx;
@@ -972,7 +981,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
 #pragma unroll
                 for (int j = 0; j < 4; ++j) f[4 * a + j] += t[j];
             }
-            if (row < N) poly_store16<T>(dQ + (int64_t)row * p.dqs_n, f, 0, p.r);
+            if (row < N) poly_store16<T>(p.dq, dq_at + (int64_t)row * p.dqs_n, f, 0, p.r, p.wide_out);
         }
     }
 #else
@@ -999,8 +1008,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
     const T *G = static_cast<const T *>(p.go) + b * p.gs_b + h * p.gs_h;
     const T *O = NORM ? static_cast<const T *>(p.o) + b * p.os_b + h * p.os_h : nullptr;
     const float *den = NORM ? p.denom + (int64_t)sl.bh * N : nullptr;
-    T *dK = static_cast<T *>(p.dk) + b * p.dks_b + h * p.dks_h;
-    T *dV = static_cast<T *>(p.dv) + b * p.dvs_b + h * p.dvs_h;
+    const int64_t dk_at = b * p.dks_b + h * p.dks_h, dv_at = b * p.dvs_b + h * p.dvs_h;
     const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
     unsigned char *tq = smem + L::kQ, *tqt = smem + L::kQt, *tk = smem + L::kK, *tv = smem + L::kV, *tg = smem + L::kG,
                   *us = smem + L::kU, *exch = smem + L::kEx;
@@ -1105,7 +1113,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
             float f[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) f[i] = dxs[i] + __shfl_xor(dxs[i], 32, 64) + dx[i];
-            if (row < N && g == 0) poly_store16<T>(dK + (int64_t)row * p.dks_n, f, 0, p.r);
+            if (row < N && g == 0) poly_store16<T>(p.dk, dk_at + (int64_t)row * p.dks_n, f, 0, p.r, p.wide_out);
         }
         if (c > sl.c_lo) su.template update<NORM>(tqt, tg, dn, lane);
         {
@@ -1121,7 +1129,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
             float f[16];
 #pragma unroll
             for (int i = 0; i < 16; ++i) f[i] = poly_pick(half, acc[1][i], acc[0][i]) + other[i];
-            if (row < N) poly_store16<T>(dV + (int64_t)row * p.dvs_n, f, 32 * half + 16 * g, p.wv);
+            if (row < N) poly_store16<T>(p.dv, dv_at + (int64_t)row * p.dvs_n, f, 32 * half + 16 * g, p.wv, p.wide_out);
         }
     }
 #else

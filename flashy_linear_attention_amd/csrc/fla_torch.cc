@@ -120,9 +120,24 @@ struct Casts {
     }
 };
 
+// A chunk-wise backward: allocates the gradients and makes `call(dq, dk, dv, dtype)`.  For inputs that all came in fp32
+// (`widened` == 7) the gradients are stored in fp32 where the library's kernels can do so.
+template <typename Backward>
+variable_list chunked_gradients(const Call &c, int64_t widened, Backward &&call) {
+    for (bool wide = widened == 7 && c.dtype == FLA_DTYPE_BF16;; wide = false) {
+        const at::TensorOptions as = wide ? c.like.dtype(at::kFloat) : c.like;
+        const Tensor dq = at::empty({c.b, c.h, c.n, c.dqk}, as), dk = at::empty({c.b, c.h, c.n, c.dqk}, as),
+                     dv = at::empty({c.b, c.h, c.n, c.dv}, as);
+        const int status = call(dq, dk, dv, c.dtype | (wide ? FLA_GRADS_F32 : 0));
+        if (wide && status == FLA_ERR_UNSUPPORTED) continue;
+        must(status);
+        return {dq, dk, dv};
+    }
+}
+
 // gradients of the inputs that came in fp32, in fp32
 void widen(variable_list &g, int64_t which) {
-    if (!which) return;
+    if (!which || g[0].scalar_type() == at::kFloat) return;  // (already: FLA_GRADS_F32)
     at::AutoDispatchBelowADInplaceOrView below;
     const void *src[3];
     void *dst[3];
@@ -171,22 +186,28 @@ std::tuple<Tensor, Tensor> product_fwd(const Tensor &q_, const Tensor &k_, const
     return {o, state};
 }
 
-variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &state, int ev) {
+variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &state, int ev,
+                          int64_t widened) {
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor go = dense(go_), q = dense(q_), k = dense(k_), v = dense(v_);
     const Call c(q, v);
+    if (ev == kChunked || ev == kChosen) {
+        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+        // (what is refused whatever the operands is not tried)
+        const bool may = c.dv <= (c.dqk <= 128 ? 128 : 64) && c.dqk % 8 == 0 && c.dv % 8 == 0;
+        return chunked_gradients(c, may ? widened : 0, [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
+            return (ev == kChosen ? fla_linear_attn_chunked_bwd_causal : fla_linear_attn_chunked_bwd)(
+                ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go), str(q), str(k),
+                str(v), str(dq), str(dk), str(dv), dtype, ptr(state), ptr(work), size_of(work), c.stream);
+        });
+    }
     Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
     if (ev == kEqual) {
         must(fla_linear_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, str(go),
                                  str(q), str(k), str(v), str(dq), str(dk), str(dv), c.dtype, c.stream));
-    } else if (ev == kSmallV) {
+    } else {
         must(fla_linear_attn_smallv_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
                                         str(go), str(q), str(k), str(v), str(dq), str(dk), str(dv), c.dtype, c.stream));
-    } else {
-        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        must((ev == kChosen ? fla_linear_attn_chunked_bwd_causal : fla_linear_attn_chunked_bwd)(
-            ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go), str(q), str(k),
-            str(v), str(dq), str(dk), str(dv), c.dtype, ptr(state), ptr(work), size_of(work), c.stream));
     }
     return {dq, dk, dv};
 }
@@ -238,8 +259,10 @@ struct Product : Function<Product> {
         const variable_list s = ctx->get_saved_variables();
         if (const auto unkept = ctx->saved_data.find("unkept"); unkept != ctx->saved_data.end())
             c10::static_intrusive_pointer_cast<Unkept>(unkept->second.toCapsule())->check();
-        variable_list g = product_bwd(go[0], s[0], s[1], s[2], s.size() > 3 ? s[3] : Tensor(), (int)ctx->saved_data["ev"].toInt());
-        widen(g, ctx->saved_data["widened"].toInt());
+        const int64_t widened = ctx->saved_data["widened"].toInt();
+        variable_list g =
+            product_bwd(go[0], s[0], s[1], s[2], s.size() > 3 ? s[3] : Tensor(), (int)ctx->saved_data["ev"].toInt(), widened);
+        widen(g, widened);
         g.resize(5);
         return g;
     }
@@ -291,30 +314,29 @@ MappedResult mapped_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, co
 }
 
 variable_list mapped_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &o,
-                         const Tensor &denom, const Tensor &state, const Options &opt) {
+                         const Tensor &denom, const Tensor &state, const Options &opt, int64_t widened) {
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor go = dense(go_), q = dense(q_), k = dense(k_), v = dense(v_);
     const Call c(q, v);
-    Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
-    if (opt.normalise) {
-        const Tensor work = c.bytes(fla_normalised_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv, opt.chunked));
-        const float *n = denom.data_ptr<float>();
+    const float *n = opt.normalise ? denom.data_ptr<float>() : nullptr;
+    const Tensor work = c.bytes(opt.normalise ? fla_normalised_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv, opt.chunked)
+                                              : fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+    // (not chunk-wise: FLA_GRADS_F32 is refused before anything is launched)
+    return chunked_gradients(c, opt.chunked || !opt.normalise ? widened : 0,
+                             [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
+        if (!opt.normalise)
+            return fla_feature_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
+                                        str(go), str(q), str(k), str(v), str(dq), str(dk), str(dv), opt.fmap, dtype, ptr(state),
+                                        ptr(work), size_of(work), c.stream);
         if (opt.fmap)
-            must(fla_feature_attn_normalised_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h,
-                                                 c.n, c.dqk, c.dv, str(go), str(q), str(k), str(v), str(o), str(dq), str(dk),
-                                                 str(dv), opt.fmap, c.dtype, opt.chunked, ptr(state), ptr(work), size_of(work),
-                                                 c.stream));
-        else
-            must(fla_linear_attn_normalised_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h,
-                                                c.n, c.dqk, c.dv, str(go), str(q), str(k), str(v), str(o), str(dq), str(dk),
-                                                str(dv), c.dtype, opt.chunked, ptr(state), ptr(work), size_of(work), c.stream));
-    } else {
-        const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        must(fla_feature_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go),
-                                  str(q), str(k), str(v), str(dq), str(dk), str(dv), opt.fmap, c.dtype, ptr(state), ptr(work),
-                                  size_of(work), c.stream));
-    }
-    return {dq, dk, dv};
+            return fla_feature_attn_normalised_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h,
+                                                   c.n, c.dqk, c.dv, str(go), str(q), str(k), str(v), str(o), str(dq), str(dk),
+                                                   str(dv), opt.fmap, dtype, opt.chunked, ptr(state), ptr(work), size_of(work),
+                                                   c.stream);
+        return fla_linear_attn_normalised_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n,
+                                              c.dqk, c.dv, str(go), str(q), str(k), str(v), str(o), str(dq), str(dk), str(dv),
+                                              dtype, opt.chunked, ptr(state), ptr(work), size_of(work), c.stream);
+    });
 }
 
 struct Mapped : Function<Mapped> {
@@ -337,9 +359,10 @@ struct Mapped : Function<Mapped> {
         const Options opt = Options::of(ctx->saved_data["opt"].toInt());
         const variable_list s = ctx->get_saved_variables();
         const size_t base = opt.normalise ? 5 : 3;
+        const int64_t widened = ctx->saved_data["widened"].toInt();
         variable_list g = mapped_bwd(go[0], s[0], s[1], s[2], opt.normalise ? s[3] : Tensor(), opt.normalise ? s[4] : Tensor(),
-                                     s.size() > base ? s[base] : Tensor(), opt);
-        widen(g, ctx->saved_data["widened"].toInt());
+                                     s.size() > base ? s[base] : Tensor(), opt, widened);
+        widen(g, widened);
         g.resize(6);
         return g;
     }
@@ -378,24 +401,25 @@ PolyResult poly_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, const 
 }
 
 variable_list poly_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &o,
-                       const Tensor &denom, const Tensor &state, const Poly &p) {
+                       const Tensor &denom, const Tensor &state, const Poly &p, int64_t widened) {
     at::AutoDispatchBelowADInplaceOrView below;
     const Tensor go = dense(go_), q = dense(q_), k = dense(k_), v = dense(v_);
     const Call c(q, v);
-    Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
     const float *n = static_cast<const float *>(ptr(denom));
     const int64_t *os = o.defined() ? str(o) : nullptr;
     if (state.defined()) {
         const Tensor work = c.bytes(fla_poly_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        must(fla_poly_attn_chunked_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n,
-                                       c.dqk, c.dv, str(go), str(q), str(k), str(v), os, str(dq), str(dk), str(dv), p.c, c.dtype,
-                                       ptr(state), ptr(work), size_of(work), c.stream));
-    } else {
-        const Tensor work = c.bytes(fla_poly_attn_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        must(fla_poly_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
-                               str(go), str(q), str(k), str(v), os, str(dq), str(dk), str(dv), p.c, c.dtype, ptr(work),
-                               size_of(work), c.stream));
+        return chunked_gradients(c, widened, [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
+            return fla_poly_attn_chunked_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n,
+                                             c.dqk, c.dv, str(go), str(q), str(k), str(v), os, str(dq), str(dk), str(dv), p.c,
+                                             dtype, ptr(state), ptr(work), size_of(work), c.stream);
+        });
     }
+    Tensor dq = c.rows(c.dqk), dk = c.rows(c.dqk), dv = c.rows(c.dv);
+    const Tensor work = c.bytes(fla_poly_attn_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
+    must(fla_poly_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
+                           str(go), str(q), str(k), str(v), os, str(dq), str(dk), str(dv), p.c, c.dtype, ptr(work),
+                           size_of(work), c.stream));
     return {dq, dk, dv};
 }
 
@@ -418,9 +442,10 @@ struct Polynomial : Function<Polynomial> {
         const bool normalise = ctx->saved_data["n"].toBool();
         const size_t base = normalise ? 5 : 3;
         auto c = [&](const char *key) { return (float)ctx->saved_data[key].toDouble(); };
+        const int64_t widened = ctx->saved_data["widened"].toInt();
         variable_list g = poly_bwd(go[0], s[0], s[1], s[2], normalise ? s[3] : Tensor(), normalise ? s[4] : Tensor(),
-                                   s.size() > base ? s[base] : Tensor(), Poly{{c("c0"), c("c1"), c("c2")}, normalise, 0.f});
-        widen(g, ctx->saved_data["widened"].toInt());
+                                   s.size() > base ? s[base] : Tensor(), Poly{{c("c0"), c("c1"), c("c2")}, normalise, 0.f}, widened);
+        widen(g, widened);
         g.resize(9);
         return g;
     }

@@ -49,6 +49,10 @@ extern "C" {
 #define FLA_ABI_VERSION 4
 
 enum fla_dtype { FLA_DTYPE_BF16 = 0, FLA_DTYPE_F16 = 1 };
+/* or'ed to FLA_DTYPE_BF16 in the chunk-wise backward calls that say so: dQ, dK and dV are buffers of floats (strides in
+ * elements, 16-byte aligned rows) and receive the same bf16-rounded values -- what a caller that casts fp32 operands to bf16
+ * would convert them to in a pass of its own.  FLA_ERR_UNSUPPORTED, with nothing launched, where no kernel stores them so. */
+#define FLA_GRADS_F32 0x100
 
 enum fla_status {
     FLA_OK = 0,
@@ -236,7 +240,9 @@ int fla_linear_attn_chunked_bwd(const void *grad_out, const void *q, const void 
  * by subtracting from the one at the end of a segment: late rows that are infinite, NaN or far larger than
  * the rest spoil the dQ of the rows before them.  This one takes a walk in forward direction for dQ, as the
  * call without `state_in` does (with D_v above 128 and widths that are multiples of 8 it is the same as the call
- * above).  Same arguments. */
+ * above).  Same arguments.
+ * FLA_GRADS_F32 here and in the calls fla_linear_attn_chunked_bwd, fla_feature_attn_bwd, fla_linear_attn_normalised_bwd and
+ * fla_feature_attn_normalised_bwd (chunked != 0), fla_poly_attn_chunked_bwd. */
 int fla_linear_attn_chunked_bwd_causal(const void *grad_out, const void *q, const void *k, const void *v,
                                        void *dq, void *dk, void *dv,
                                        int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v,

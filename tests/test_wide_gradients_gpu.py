@@ -1,0 +1,80 @@
+"""fp32 operands under autocast whose gradients the chunk-wise kernels store in fp32 themselves (FLA_GRADS_F32): the values of a
+16-bit call, widened -- ragged lengths, one and several segments, heads of fewer columns than the padded width -- and what
+the flag is refused for (``-m gpu``)."""
+
+import pytest
+import torch
+
+from flashy_linear_attention_amd import (FeatureMapLinearAttention, LinearAttention, LinearAttentionAuto,
+                                         LinearAttentionChunked, LinearAttentionNormalised, LinearAttentionSmallVHD,
+                                         PolynomialLinearAttention, _lib)
+
+pytestmark = pytest.mark.gpu
+
+OPS = {
+    "auto": LinearAttentionAuto.apply,
+    "linear": LinearAttention.apply,
+    "smallv": LinearAttentionSmallVHD.apply,
+    "chunked": LinearAttentionChunked.apply,
+    "normalised": lambda *a: LinearAttentionNormalised.apply(*a, 1e-5, True),
+    "feature": lambda *a: FeatureMapLinearAttention.apply(*a, "elu1"),
+    "feature_normalised": lambda *a: FeatureMapLinearAttention.apply(*a, "softplus", True, 1e-5),
+    "poly": lambda *a: PolynomialLinearAttention.apply(*a, 1.0, 1.0, 0.5, True, 1e-5),
+}
+
+
+@pytest.mark.parametrize("op,b,h,n,dqk,dv", [
+    ("chunked", 2, 3, 333, 64, 64), ("chunked", 1, 2, 1100, 40, 40), ("auto", 2, 4, 3000, 80, 80), ("linear", 1, 64, 4096, 128, 128),
+    ("smallv", 1, 8, 4096, 128, 64), ("smallv", 1, 8, 4096, 256, 64), ("chunked", 1, 3, 700, 256, 64), ("chunked", 1, 3, 700, 200, 128), ("chunked", 1, 80, 700, 128, 128), ("chunked", 1, 2, 700, 72, 64), ("auto", 1, 2, 4096, 100, 100), ("normalised", 1, 5, 700, 64, 64),
+    ("normalised", 1, 130, 300, 96, 96), ("normalised", 2, 9, 1001, 128, 128), ("feature", 1, 3, 400, 32, 32), ("feature", 1, 3, 400, 128, 128),
+    ("feature_normalised", 1, 3, 515, 48, 48), ("feature_normalised", 1, 3, 515, 128, 128), ("poly", 1, 3, 515, 16, 40), ("poly", 1, 300, 200, 8, 64),
+    ("normalised", 1, 2, 300, 200, 64),
+])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_equals_widening_by_hand(op, b, h, n, dqk, dv, transposed, gpu_device):
+    gen = torch.Generator().manual_seed(n + dqk)
+    ins = [torch.rand(b, h, n, d, generator=gen).to(gpu_device) for d in (dqk, dqk, dv, dv)]
+    if transposed:
+        ins = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in ins]
+    do = ins[3].bfloat16()
+    wide = [t.clone().requires_grad_(True) for t in ins[:3]]
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        out = OPS[op](*wide)
+    grads = torch.autograd.grad(out, wide, do)
+    narrow = [t.bfloat16().requires_grad_(True) for t in ins[:3]]
+    want = OPS[op](*narrow)
+    want_grads = torch.autograd.grad(want, narrow, do)
+    assert torch.equal(out, want)
+    for got, w in zip(grads, want_grads):
+        assert got.dtype == torch.float32 and torch.equal(got, w.float())
+
+
+F32 = 0x100  # FLA_GRADS_F32
+
+
+@pytest.mark.parametrize("dtype,n,d,causal,status", [
+    (torch.bfloat16, 600, 64, True, 0), (torch.bfloat16, 600, 128, True, 0), (torch.float16, 600, 64, True, -8),
+    (torch.bfloat16, 600, 128, False, 0), (torch.bfloat16, 100, 64, True, -8), (torch.bfloat16, 600, 60, True, -8),
+    (torch.bfloat16, 600, 256, True, -8),
+])
+def test_what_the_flag_is_taken_for(dtype, n, d, causal, status, gpu_device):
+    lib = _lib.load()
+    q, k, v, go = (torch.rand(1, 2, n, d, device=gpu_device).to(dtype) for _ in range(4))
+    code = 0 if dtype is torch.bfloat16 else 1
+    out = torch.empty_like(v)
+    state = torch.empty(max(16, _lib.query("fla_linear_attn_chunked_state_bytes", 1, 2, n, d, d)), dtype=torch.uint8, device=gpu_device)
+    work = torch.empty(max(16, _lib.query("fla_linear_attn_chunked_workspace_bytes", 1, 2, n, d, d)), dtype=torch.uint8, device=gpu_device)
+    import ctypes
+    valid = ctypes.c_int32(0)
+    st = _lib.strides_arg
+    stream = torch.cuda.current_stream().cuda_stream
+    assert lib.fla_linear_attn_chunked_fwd(q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 1, 2, n, d, d, st(q), st(k), st(v),
+                                           st(out), code, state.data_ptr(), ctypes.byref(valid), work.data_ptr(), work.numel(), stream) == 0
+    grads = [torch.full((1, 2, n, d), 7.0, device=gpu_device) for _ in range(3)]
+    fn = lib.fla_linear_attn_chunked_bwd_causal if causal else lib.fla_linear_attn_chunked_bwd
+    got = fn(go.data_ptr(), q.data_ptr(), k.data_ptr(), v.data_ptr(), *(t.data_ptr() for t in grads), 1, 2, n, d, d, st(go), st(q),
+             st(k), st(v), *(st(t) for t in grads), code | F32, state.data_ptr() if valid.value else None, work.data_ptr(),
+             work.numel(), stream)
+    assert got == status
+    torch.cuda.synchronize()
+    assert all(bool((t == 7.0).all()) == (status != 0) for t in grads)
