@@ -397,12 +397,15 @@ struct WalkPlan {
 // kernels are built for equal padded widths).
 // From three segments per (b, h) up to this many the walks add up the segments' totals themselves, beyond it a scan kernel
 // does (padded head dims up to 64: fla::walk_sum_on_load_max, which the kernels know).
-//   D = 128.  Forward + backward, scan against sums on load: B H 32, N 4096 (8 segments) 146 / 137 us; B H 24, N 1500 (8)
-//   80 / 77; B H 20, N 4096 (11) 145 / 141; B H 16, N 4096 (16) 101 / 104; B H 8, N 4096 (32) 79 / 109.  Four pairs of column
-//   halves at a time (256 / 256) the same: B H 16, N 4096 (8) 258 / 234; B H 12 (10) 319 / 313; B H 32, N 2048 (4) 250 / 229.
-//   A wide q / k against a v of up to 128: two states to add up.  256 / 64, B H 64, N 4096 (4): 273 / 264.
+//   D = 128.  Forward + backward, scan against sums on load: B H 24, N 1500 (8 segments) 66.8 / 62.4 us; B H 20, N 2048 (11)
+//   89.6 / 83.6; B H 16, N 4096 (16) 92.0 / 87.5; B H 12, N 4096 (16) 83.8 / 82.0; B H 10, N 4096 (22) 106.0 / 107.6; B H 9
+//   (22) 101.9 / 105.7; B H 10, N 16384 (24) 248 / 251; B H 8, N 8192 (32) 91.4 / 99.4.  Four pairs of column
+//   halves at a time (256 / 256) the same: B H 8, N 4096 (16) 154.4 / 141.7; B H 6, N 8192 (19) 313 / 304; B H 5, N 4096 (22)
+//   182.9 / 190.1.
+//   A wide q / k against a v of up to 128: two states to add up, and the walks are held to seven.  256 / 64, B H 64, N 4096 (4)
+//   320 / 313 (kernels); it would pay up to fifteen: B H 32, N 2048 (8) 104.0 / 95.5, B H 20, N 4096 (11) 162.8 / 155.4.
 //   The polynomial map, of 58 KiB a state: where adding them up costs more than a launch.
-constexpr int kSumOnLoadMost = 12, kSumOnLoadWide = 7, kSumOnLoadPoly = 8;
+constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 7, kSumOnLoadPoly = 8;
 
 // `parts`: workgroups per segment (a launch that does several column halves at a time).
 WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false, int64_t parts = 1) {
@@ -475,7 +478,7 @@ int walk_entry_states(const WalkPlan &w, const View &y, const View &z, int64_t B
     const bool direct = w.n_seg == 2;
     const bool summed_on_load = fla::walk_entries_are_totals(w.D, (int)w.n_seg) || (totals_only && !direct);
     const bool no_scan = direct || summed_on_load;
-    tp.y = y.ptr, tp.z = z.ptr, tp.totals = no_scan ? entry : totals, tp.direct = direct;
+    tp.y = y.ptr, tp.z = z.ptr, tp.totals = no_scan ? entry : totals, tp.direct = direct, tp.frags = summed_on_load;
     tp.ys_b = y.strides[0], tp.ys_h = y.strides[1], tp.ys_n = y.strides[2];
     tp.zs_b = z.strides[0], tp.zs_h = z.strides[1], tp.zs_n = z.strides[2];
     tp.H = (int32_t)H, tp.N = (int32_t)N, tp.BH = (int32_t)(B * H), tp.dy = (int32_t)dy, tp.dz = (int32_t)dz;
@@ -569,9 +572,10 @@ int walk_grad_entry_states(const WalkPlan &w, const View &q, const View &dout, c
     gp.n_chunks = (int32_t)w.n_chunks, gp.seg_chunks = (int32_t)w.seg_chunks, gp.n_seg = (int32_t)w.n_seg;
     const bool several = w.n_seg > 1;
     gp.totals = several ? static_cast<float *>(work) : nullptr, gp.rsum = several ? rc_totals : nullptr;
+    gp.frags = w.n_seg > 2 && (totals_only || fla::walk_entries_are_totals(w.D, (int)w.n_seg));
     *where = gp.totals;
     if (fla::walk_grad_totals(dtype, w.D, gp, s) != hipSuccess) return FLA_ERR_LAUNCH;
-    if (w.n_seg <= 2 || totals_only || fla::walk_entries_are_totals(w.D, (int)w.n_seg)) return FLA_OK;
+    if (w.n_seg <= 2 || gp.frags) return FLA_OK;
     return fla::walk_scan(gp.totals, gp.totals, B * H, (int)w.n_seg, w.D, w.D, 1, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 
@@ -846,10 +850,10 @@ int quad_entry_states(const WalkPlan &wp, const View &y, const View &z, int64_t 
     tp.H = (int32_t)H, tp.N = (int32_t)N, tp.BH = (int32_t)(B * H);
     tp.dy = tp.dz = 128, tp.dy2 = (int32_t)(dy - 128), tp.dz2 = (int32_t)(dz - 128);
     tp.n_chunks = (int32_t)wp.n_chunks, tp.seg_chunks = (int32_t)wp.seg_chunks, tp.n_seg = (int32_t)wp.n_seg;
-    tp.direct = wp.n_seg == 2;
+    tp.direct = wp.n_seg == 2, tp.frags = sums_on_load(wp);
     tp.seg_lo = reverse ? 1 : 0, tp.seg_hi = (int32_t)(reverse ? wp.n_seg : wp.n_seg - 1);
     if (fla::walk_totals(dtype, wp.D, tp, s) != hipSuccess) return FLA_ERR_LAUNCH;
-    if (tp.direct || sums_on_load(wp)) return FLA_OK;
+    if (tp.direct || tp.frags) return FLA_OK;
     return fla::walk_scan(entries, entries, 4 * B * H, (int)wp.n_seg, wp.D, wp.D, reverse, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 

@@ -903,6 +903,38 @@ __device__ __forceinline__ void walk_read_state(const float *init, bool transpos
     }
 }
 
+// A state that is to be added up on load lies in memory by fragments: block (i, j) of 32 x 32 at float 1024 (i D / 32 + j), in it
+// the sixteen values that a lane holds, as four runs of four -- a wave moves 1 KiB of consecutive memory with each access.  Row by
+// row a lane's values are four bytes apart from the next lane's, and the 63 accesses that a wave may have in flight are one
+// D = 128 state: a memory latency per segment.  (Forward walk, D = 128: B H 32, N 2048, eight segments 24.2 -> 22.0 us, with the
+// scan's entry states 16.4; normalised, B H 16, N 4096, sixteen segments 53.6 -> 26.0 us, 20.4 behind a scan of 7.)
+template <int D, typename B>
+__device__ __forceinline__ void walk_read_frags(const float *buf, int wave, int lane, f32x16 (&st)[WalkCfg<D>::NBW]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int i = 0; i < B::SLOTS; ++i)
+        if (B::valid(wave, i)) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a) {
+                const f32x4 t = *reinterpret_cast<const f32x4 *>(buf + (B::dbk(wave, i) * (D / 32) + B::eb(wave)) * 1024 + a * 256 + lane * 4);
+#pragma unroll
+                for (int b = 0; b < 4; ++b) st[i][4 * a + b] = t[b];
+            }
+        }
+}
+template <int D, typename B>
+__device__ __forceinline__ void walk_write_frags(float *out, int wave, int lane, const f32x16 (&st)[WalkCfg<D>::NBW]) {
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+#pragma unroll
+    for (int i = 0; i < B::SLOTS; ++i)
+        if (B::valid(wave, i)) {
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+                *reinterpret_cast<f32x4 *>(out + (B::dbk(wave, i) * (D / 32) + B::eb(wave)) * 1024 + a * 256 + lane * 4) =
+                    f32x4{st[i][4 * a], st[i][4 * a + 1], st[i][4 * a + 2], st[i][4 * a + 3]};
+        }
+}
+
 // ... zeros for a null pointer; with `init2` the state is the sum of the two buffers
 template <int D, typename B = WalkExt<D>>
 __device__ __forceinline__ void walk_load_state(const float *init, bool transposed, int wave, int lane,
@@ -922,28 +954,35 @@ __device__ __forceinline__ void walk_load_state(const float *init, bool transpos
 //   * two segments per (b, h): the first segment in walking order starts from zero and the other one
 //     from the one total the totals kernel forms; its two workgroups of a (b, h) add up half of that
 //     segment each, and the two slots hold their partial sums;
-//   * three to walk_sum_on_load_max(D) segments, or with that flag: the slots hold the segments' TOTALS as the totals kernel
-//     wrote them, and a walk adds up the totals of the segments before it (after it, walking in reverse)
+//   * three to walk_sum_on_load_max(D) segments, or with that flag: the slots hold the segments' TOTALS, by fragments
+//     (walk_read_frags), and a walk adds up the totals of the segments before it (after it, walking in reverse)
 //     as it starts -- a few states of D x D read from L2 per workgroup instead of a scan kernel between
 //     the totals kernel and the walk, whose launch costs more than it computes on plans this small
 //     (B H = 16, N = 1024, D = 64, forward + backward: 40.7 -> 32.8 us, bound by its six -> four launches).  D = 64, scan
-//     against sums on load: 8 to 16 segments, N 4096: B H 40 77 / 68 us, B H 32 69 / 64, forward alone 26.7 / 22.3; 21 segments
-//     equal; 32 and more: forward alone 20.7 / 21.7 (B H 16, N 4096), 21.7 / 28.8 (64 segments), B H 16 N 32768 212 / 215;
+//     against sums on load: 32 segments B H 16 N 4096 84.7 / 77.1 us, N 32768 232.8 / 227.6, B H 12 N 8192 81.9 / 75.0, forward
+//     alone B H 12 N 4096 24.2 / 21.5, B H 10 N 8192 25.2 / 25.7; 64 segments (B H 8 N 8192) forward alone 23.3 / 24.9;
 //   * more segments: the slots hold the entry states themselves (walk_scan_kernel).
 // (At D = 128 a forward walk then writes the entry states it formed, for backward.)
-__host__ __device__ constexpr int walk_sum_on_load_max(int D) { return D <= 64 ? 16 : 0; }
+__host__ __device__ constexpr int walk_sum_on_load_max(int D) { return D <= 64 ? 40 : 0; }
 __host__ __device__ constexpr bool walk_entries_are_totals(int D, int n_seg) {
     return n_seg >= 3 && n_seg <= walk_sum_on_load_max(D);
 }
 
-// this wave's blocks of the sum of the states buf[f_lo .. f_hi - 1] (zeros for an empty range), added in
-// ascending order, the loads of up to four states (two of four blocks per wave) in flight together (one state at a time is a chain of
+// the loads above stay above their uses (short of registers the compiler moves every load down to its use otherwise, and two are in
+// flight at a time)
+__device__ __forceinline__ void walk_all_requested() {
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_sched_barrier(0);
+}
+
+// this wave's blocks of the sum of the states buf[f_lo .. f_hi - 1] (zeros for an empty range; by fragments), added in
+// ascending order, the loads of several states in flight together (one state at a time is a chain of
 // dependent loads: a memory latency per state at the start of every workgroup)
 template <int D, typename B>
-__device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int f_hi, bool transposed, int wave, int lane,
+__device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int f_hi, int wave, int lane,
                                                 f32x16 (&st)[WalkCfg<D>::NBW]) {
     using W = WalkCfg<D>;
-    constexpr int GROUP = B::SLOTS > 2 ? 2 : 4;  // (GROUP x SLOTS x 16 registers beside the sum)
+    constexpr int GROUP = B::SLOTS > 2 ? 3 : B::SLOTS > 1 ? 6 : 8;  // (GROUP x SLOTS x 16 registers beside the sum)
 #pragma unroll
     for (int i = 0; i < W::NBW; ++i)
 #pragma unroll
@@ -954,8 +993,9 @@ __device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int 
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
             const int f = f0 + u < f_hi ? f0 + u : f_hi - 1;  // (past the range: the last state once more, not added)
-            walk_read_state<D, B, false>(buf + (int64_t)f * (D * D), transposed, wave, lane, t[u]);
+            walk_read_frags<D, B>(buf + (int64_t)f * (D * D), wave, lane, t[u]);
         }
+        walk_all_requested();
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
             const float keep = f0 + u < f_hi ? 1.f : 0.f;
@@ -988,9 +1028,10 @@ __device__ __forceinline__ void walk_sum_two(const float *a, const float *b, int
         for (int u = 0; u < GROUP; ++u) {
             // (past the range: the last state once more, not added)
             const int f = f0 + u < f_hi ? f0 + u : f_hi - 1;
-            walk_read_state<D, B, false>(a + (int64_t)f * E, false, wave, lane, ta[u]);
-            walk_read_state<D, B, false>(b + (int64_t)f * E, false, wave, lane, tb[u]);
+            walk_read_frags<D, B>(a + (int64_t)f * E, wave, lane, ta[u]);
+            walk_read_frags<D, B>(b + (int64_t)f * E, wave, lane, tb[u]);
         }
+        walk_all_requested();
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
             const float keep = f0 + u < f_hi ? 1.f : 0.f;
@@ -1015,7 +1056,7 @@ __device__ __forceinline__ void walk_load_init_from(const float *buf, const Walk
             if (sl.seg != (reverse ? 1 : 0)) init = buf + (int64_t)sl.bh * 2 * (D * D), init2 = init + D * D;
         } else if (walk_entries_are_totals(D, p.n_seg) || p.init_is_totals) {
             walk_sum_states<D, B>(buf + (int64_t)sl.bh * p.n_seg * (D * D), reverse ? sl.seg + 1 : 0,
-                                  reverse ? p.n_seg : sl.seg, p.init_transposed != 0, wave, lane, st);
+                                  reverse ? p.n_seg : sl.seg, wave, lane, st);
             return;
         } else if (sl.seg != (reverse ? p.n_seg - 1 : 0)) {  // (the first one in walking order starts from zero)
             init = buf + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D);
@@ -1040,7 +1081,7 @@ __device__ __forceinline__ void walk_load_end_state_from(const float *xinit, con
         if (p.n_seg == 2) {
             x = xinit + (int64_t)sl.bh * 2 * (D * D), x2 = x + D * D;
         } else if (walk_entries_are_totals(D, p.n_seg)) {
-            walk_sum_states<D, B>(xinit + (int64_t)sl.bh * p.n_seg * (D * D), 0, sl.seg + 1, false, wave, lane, xs);
+            walk_sum_states<D, B>(xinit + (int64_t)sl.bh * p.n_seg * (D * D), 0, sl.seg + 1, wave, lane, xs);
             return;
         } else {
             x = xinit + ((int64_t)sl.bh * p.n_seg + sl.seg + 1) * (D * D);
@@ -1360,8 +1401,8 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
         if constexpr (NV == 2) {  // (both halves' loads in flight together; with four blocks per wave and state, one half's)
             walk_sum_two<D, B>(p.init + at, p.init2 + at, 0, sl.seg, wave, lane, st0, st1);
         } else {
-            walk_sum_states<D, B>(p.init + at, 0, sl.seg, false, wave, lane, st0);
-            walk_sum_states<D, B>(p.init2 + at, 0, sl.seg, false, wave, lane, st1);
+            walk_sum_states<D, B>(p.init + at, 0, sl.seg, wave, lane, st0);
+            walk_sum_states<D, B>(p.init2 + at, 0, sl.seg, wave, lane, st1);
         }
         if (p.entry_out && sl.seg > 0) {  // (the first segment's entry state, zero, is read by nobody)
             walk_write_state<D, B>(p.entry_out + at + (int64_t)sl.seg * (D * D), wave, lane, st0);
@@ -1925,8 +1966,8 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
         if constexpr (NV == 2) {
             walk_sum_two<D, B>(p.init + at, p.init2 + at, sl.seg + 1, p.n_seg, wave, lane, st0, st1);
         } else {
-            walk_sum_states<D, B>(p.init + at, sl.seg + 1, p.n_seg, false, wave, lane, st0);
-            walk_sum_states<D, B>(p.init2 + at, sl.seg + 1, p.n_seg, false, wave, lane, st1);
+            walk_sum_states<D, B>(p.init + at, sl.seg + 1, p.n_seg, wave, lane, st0);
+            walk_sum_states<D, B>(p.init2 + at, sl.seg + 1, p.n_seg, wave, lane, st1);
         }
     } else {
         walk_load_init_from<D, B>(p.init, p, sl, wave, lane, st0, true);
@@ -2043,6 +2084,8 @@ struct WalkTotalsParams {
     // The totals of Y's rows, fp32 [BH][n_seg][D], in the slots of `totals` -- the normaliser's running sum of k at the
     // segments' entries (WalkParams::vsum); null: not formed.  One operand only.
     float *vsum;
+    // the totals are written by fragments (walk_write_frags): the walks add them up as they start
+    int32_t frags;
     // nobody reads the totals' columns 64 .. (every walk behind them leaves a narrow z's padding out): they may stay
     // unwritten for a narrow y as well
     int32_t z_narrow;
@@ -2188,6 +2231,10 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
             set = (set + 1) % SETS;
         }
     }
+    if (p.frags) {
+        walk_write_frags<D, B>(out, wave, lane, st);
+        if constexpr (BOTH) walk_write_frags<D, B>(out2, wave, lane, st2);
+    } else
 #pragma unroll
     for (int i = 0; i < B::SLOTS; ++i)
         if (B::valid(wave, i)) {
@@ -2382,6 +2429,7 @@ struct WalkGradParams {
     int32_t n_chunks, seg_chunks, n_seg;
     float *totals, *rsum;      // [BH][n_seg] states and vectors in the slots the walks read (two segments: partial sums of the
                                // second one's in both; the first one's stay unwritten otherwise); null with a single segment
+    int32_t frags;             // WalkTotalsParams::frags
 };
 
 // Steps on their way: what a step needs is requested DEPTH steps ahead -- one where two workgroups share a CU, two at D = 128,
@@ -2513,7 +2561,10 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void walk_grad_totals_kernel
         });
     if (p.n_seg == 1 || (p.n_seg > 2 && seg == 0)) return;
     const int64_t at = (int64_t)bh * p.n_seg + seg;
-    walk_write_state<D, WalkExt<D>>(p.totals + at * (D * D), wave, lane, st);
+    if (p.frags)
+        walk_write_frags<D, WalkExt<D>>(p.totals + at * (D * D), wave, lane, st);
+    else
+        walk_write_state<D, WalkExt<D>>(p.totals + at * (D * D), wave, lane, st);
     float *part = reinterpret_cast<float *>(smem);
     __syncthreads();
     walk_weighted_sums_to_lds<D>(part, wave, lane, zs);
@@ -2549,7 +2600,7 @@ hipError_t launch_walk_totals(const WalkTotalsParams &p, hipStream_t stream) {
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr int smem = walk_totals_sets(D) * 2 * WalkCfg<D>::TILE;
-    if (p.direct && (p.n_seg != 2 || p.seg_lo < 0 || p.seg_lo > 1)) return hipErrorInvalidValue;
+    if (p.direct && (p.n_seg != 2 || p.seg_lo < 0 || p.seg_lo > 1 || p.frags)) return hipErrorInvalidValue;
     // (a second operand runs the same kernel variant: the caller pairs operands of one kind only)
     if (p.y2 && (p.map_y || !p.totals2 ||
                  (!p.z_narrow && walk_totals_cols(D, p.dy2, p.dz) != walk_totals_cols(D, p.dy, p.dz))))

@@ -1,0 +1,53 @@
+"""Plans whose walks add up the segments' totals as they start, around the numbers of segments where a scan takes over (20 at
+128 columns and with both sides above 128, 7 with a wide q / k alone, 40 up to 64): both passes, with forward's state and
+without, against the fp32 oracle (``-m gpu``)."""
+
+import pytest
+import torch
+
+from flashy_linear_attention_amd import LinearAttentionAuto, LinearAttentionSmallVHD
+from flashy_linear_attention_amd.chunked import linear_attention_chunked_bwd, linear_attention_chunked_fwd
+from flashy_linear_attention_amd.normalised import linear_attention_normalised_fwd
+
+from helpers import assert_close, gpu_fp32_reference, reference_style_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+# (heads, N, columns): the last segment ragged.  One chunk a segment (64 rows above 64 columns, 128 up to it) up to the rule
+# and one beyond it, and totals in groups of three (D = 128) and eight (64): 3, 4, 5, 9, 10 segments
+@pytest.mark.parametrize("h,n,dqk,dv,dtype", [
+    (12, 20 * 64 - 5, 128, 128, torch.bfloat16), (12, 21 * 64 - 5, 128, 128, torch.float16), (85, 9 * 64, 80, 80, torch.bfloat16),
+    (64, 1003, 96, 96, torch.float16), (50, 5 * 64 - 1, 128, 128, torch.bfloat16), (12, 1270, 128, 64, torch.bfloat16),
+    (6, 20 * 64 - 3, 256, 256, torch.bfloat16), (6, 21 * 64 - 3, 160, 256, torch.bfloat16), (32, 5 * 64, 256, 160, torch.float16),
+    (36, 7 * 64 - 7, 256, 64, torch.bfloat16), (32, 8 * 64 - 7, 256, 64, torch.bfloat16), (16, 900, 192, 128, torch.float16),
+    (12, 40 * 128 - 9, 64, 64, torch.bfloat16), (12, 41 * 128 - 9, 64, 64, torch.float16), (51, 9 * 128 + 1, 32, 32, torch.bfloat16),
+])
+def test_both_passes(h, n, dqk, dv, dtype, gpu_device):
+    q, k, v, do = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, dqk, dv, dtype, seed=n + dqk))
+    want_o, want_g = gpu_fp32_reference(q, k, v, do, True)
+    out, state = linear_attention_chunked_fwd(q, k, v, want_state=True)
+    assert_close("O", out, want_o)
+    for kept in (state, None):
+        for name, got, want in zip(("dQ", "dK", "dV"), linear_attention_chunked_bwd(do, q, k, v, kept), want_g):
+            assert_close(name, got, want)
+
+
+@pytest.mark.parametrize("h,n,dqk,dv", [(24, 1500, 80, 80), (36, 7 * 64, 256, 64), (36, 448, 153, 64), (32, 512, 256, 128)])
+def test_operators_that_keep_dq_causal(h, n, dqk, dv, gpu_device):
+    q, k, v, do = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, dqk, dv, torch.bfloat16, seed=n + dqk))
+    want_o, want_g = gpu_fp32_reference(q, k, v, do, True)
+    q, k, v = (t.requires_grad_() for t in (q, k, v))
+    op = LinearAttentionAuto if dqk == dv else LinearAttentionSmallVHD
+    out = op.apply(q, k, v)
+    assert_close("O", out, want_o)
+    for name, got, want in zip(("dQ", "dK", "dV"), torch.autograd.grad(out, (q, k, v), do), want_g):
+        assert_close(name, got, want)
+
+
+@pytest.mark.parametrize("h,n,d", [(12, 20 * 64 - 5, 128), (12, 21 * 64 - 5, 128), (16, 1000, 72), (12, 40 * 128, 64)])
+def test_normalised_forward(h, n, d, gpu_device):
+    q, k, v, _ = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, d, d, torch.bfloat16, seed=n + d))
+    qd, kd = q.double(), k.double()
+    want = (torch.tril(qd @ kd.transpose(-1, -2)) @ v.double()) / ((qd * kd.cumsum(-2)).sum(-1, keepdim=True) + 1e-5)
+    assert_close("out", linear_attention_normalised_fwd(q, k, v, 1e-5, True)[0], want.float())
