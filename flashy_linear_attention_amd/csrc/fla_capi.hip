@@ -585,6 +585,14 @@ bool states_shareable(int64_t dqk, int64_t dv, int64_t N) {
     return rows != 0 && N > rows;
 }
 
+// The caller's results of any alignment behind aligned stand-ins (packed_forward, packed_backward), of the true widths, for walks
+// that can store to them; `done`: they did, for all of the call's results
+struct AnyRows {
+    const View *o, *dq, *dk, *dv;
+    int64_t dqk, wv;
+    bool done;
+};
+
 // bytes of one rounded running state / of the scratch one state computation needs (fp32 chunk states)
 // ---- D_qk in (128, 256] with D_v <= 128 (the small-V operator's shapes).  The scores are a sum over
 // the two 128-column halves of q and k and everything is linear in them:
@@ -728,6 +736,17 @@ fla::WalkParams reverse_walk_params(const WalkPlan &wp, const View &go, const Vi
     return r;
 }
 
+fla::WalkRowsOut rows_out(const View &t, int64_t width) {
+    return {const_cast<void *>(t.ptr), t.strides[0], t.strides[1], t.strides[2], (int32_t)width};
+}
+// ... its results to the caller's rows
+void results_to_rows(fla::WalkParams &r, AnyRows &any) {
+    r.any_rows = 1, any.done = true;
+    if (r.dq) r.rows_dq = rows_out(*any.dq, any.dqk);
+    r.rows_dk = rows_out(*any.dk, any.dqk), r.rows_dv = rows_out(*any.dv, any.wv);
+    r.dq = r.dk = r.dv = nullptr;
+}
+
 bool wide_fast_path(const View &q, const View &k, const View &v, const View &o, int64_t B, int64_t H, int64_t N,
                     int64_t dqk, int64_t dv) {
     return fla::fast_path_ok(make_params(q, k, v, o, B, H, N, 128, dv, 0)) &&
@@ -776,7 +795,7 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
 // as a reverse walk per half, the second adding to the first one's dV in memory, 279 us in three walks.
 int wide_backward(const WidePlan &wide, const View &go, const View &q, const View &k, const View &v, const View &dq,
                   const View &dk, const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
-                  const void *state_in, void *workspace, hipStream_t s, bool causal, bool wide_out) {
+                  const void *state_in, void *workspace, hipStream_t s, bool causal, bool wide_out, AnyRows *any) {
     const WalkPlan &wp = wide.wp;
     char *ws = static_cast<char *>(workspace);
     const bool one_walk = state_in && dv <= 64 && !causal;
@@ -809,14 +828,19 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
         r.xtotal2 = reinterpret_cast<const float *>(half1 + wp.entry_bytes);
         return fla::walk_bwd_rev_wide(dtype, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
+    // (dQ, dK straight to the caller's rows; dV's are aligned)
+    if (any && dv <= 64 && any->wv == dv) any->done = true;
+    const bool rows = any && any->done;
     // dQ_h = lower(dO V^T) K_h + dO S_h^T: the forward walk over (dO, V, K_h)
     for (int h = 0; h < 2; ++h) {
         const View dq_h{static_cast<const char *>(dq.ptr) + h * 128 * (wide_out ? 4 : 2), dq.strides};
         fla::WalkParams w = lower_walk_params(wp, go, v, column_half(k, h), dq_h, B, H, N, dv, h ? dqk - 128 : 128, fwd_entries[h]);
         w.init_transposed = 1, w.wide_out = wide_out;
+        if (rows) w.any_rows = 1, w.rows_o = rows_out(column_half(*any->dq, h), h ? any->dqk - 128 : 128), w.o = nullptr;
         if (fla::walk_fwd(dtype, wp.D, w, s) != hipSuccess) return FLA_ERR_LAUNCH;
     }
     r.dq = nullptr;
+    if (rows) r.any_rows = 1, r.rows_dk = rows_out(*any->dk, any->dqk), r.dk = nullptr;
     return fla::walk_bwd_rev_wide(dtype, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 
@@ -905,11 +929,12 @@ bool vsplit_fast_path(const VSplit &vs, const View &a, const View &b, const View
 
 int chunked_forward(const View &q, const View &k, const View &v, const View &o, int64_t B, int64_t H, int64_t N,
                     int64_t dqk, int64_t dv, int dtype, void *state_out, int32_t *state_valid, void *workspace,
-                    int64_t workspace_bytes, void *stream, int fmap, const View *mapped, bool *mapped_done, WalkNorm *nx);
+                    int64_t workspace_bytes, void *stream, int fmap, const View *mapped, bool *mapped_done, WalkNorm *nx,
+                    AnyRows *any);
 int chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                      const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap, WalkNorm *nx,
-                     bool causal, bool wide_out);
+                     bool causal, bool wide_out, AnyRows *any);
 
 // fmap != 0 (feature_forward below): q and k hold the arguments xq, xk of the feature map phi, and
 // `mapped` = {phi(xq), phi(xk)} are outputs: the state kernel maps xk as it loads it and writes
@@ -918,7 +943,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
 int chunked_forward(const View &q, const View &k, const View &v, const View &o, int64_t B, int64_t H, int64_t N,
                     int64_t dqk, int64_t dv, int dtype, void *state_out, int32_t *state_valid, void *workspace,
                     int64_t workspace_bytes, void *stream, int fmap = 0, const View *mapped = nullptr,
-                    bool *mapped_done = nullptr, WalkNorm *nx = nullptr) {
+                    bool *mapped_done = nullptr, WalkNorm *nx = nullptr, AnyRows *any = nullptr) {
     if (state_valid) *state_valid = 0;
     if (nx) nx->fused = nx->dk_pending = false;
     const View all[] = {q, k, v, o};
@@ -1004,6 +1029,9 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = wp.n_seg > 1 ? entry : nullptr, w.saved = in_state ? nullptr : state_out;
         if (sum_on_load) w.init_is_totals = 1, w.entry_out = in_state ? static_cast<float *>(state_out) : nullptr;
+        if (any && wp.split) {
+            w.any_rows = 1, w.rows_o = rows_out(*any->o, any->wv), w.o = nullptr, any->done = true;
+        }
         if (in_state) w.total_out = reinterpret_cast<float *>(static_cast<char *>(state_out) + wp.entry_bytes);
         if (nx) {  // the normaliser inside the walk, which carries the running sum of k from the segments' totals of it
             // (kept for backward, at the entry of every chunk, behind the state when there is one)
@@ -1077,7 +1105,7 @@ bool norm_walks_backward(const View &go, const View &q, const View &k, const Vie
 int chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                      const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap = 0,
-                     WalkNorm *nx = nullptr, bool causal = false, bool wide_out = false) {
+                     WalkNorm *nx = nullptr, bool causal = false, bool wide_out = false, AnyRows *any = nullptr) {
     if (nx) nx->fused = nx->dk_pending = false;
     const View all[] = {go, q, k, v, dq, dk, dvv};
     for (const View &t : all)
@@ -1123,7 +1151,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                 return FLA_ERR_WORKSPACE;
             if (state_in && reinterpret_cast<uintptr_t>(state_in) % 16 != 0) return FLA_ERR_WORKSPACE;
             return wide_backward(wide, go, q, k, v, dq, dk, dvv, B, H, N, dqk, dv, dtype, state_in, workspace,
-                                 static_cast<hipStream_t>(stream), causal, wide_out);
+                                 static_cast<hipStream_t>(stream), causal, wide_out, any);
         }
     }
     // (with the normaliser's terms still to be added by the caller, so is the slope)
@@ -1191,6 +1219,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
             r.xinit = static_cast<const float *>(state_in);
             r.xtotal = reinterpret_cast<const float *>(static_cast<const char *>(state_in) + wp.entry_bytes);
             r.wide_out = wide_out;
+            if (any) results_to_rows(r, *any);
             return fla::walk_bwd_rev(dtype, wp.D, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
         }
         // dQ = lower(dO V^T) K + dO S^T: the forward walk over (dO, V, K), its states V^T K = S^T
@@ -1209,6 +1238,9 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
             w.sy_b = q.strides[0], w.sy_h = q.strides[1], w.sy_n = q.strides[2];
         }
         if (nx) w.dn = nx->dn, w.zc = zc, nx->fused = true;  // dQ's term of the normaliser inside its walk
+        if (any) {
+            w.any_rows = 1, w.rows_o = rows_out(*any->dq, any->dqk), w.o = nullptr;
+        }
         if (fla::walk_fwd(dtype, wp.D, w, s) != hipSuccess) return FLA_ERR_LAUNCH;
         // dV, dK: the reverse walk over the same segments
         fla::WalkParams r{};
@@ -1225,6 +1257,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         r.init = entry, r.fmap = fmap;  // (dK: the slope from phi(xk) in the K tile)
         r.init_is_totals = rev_sums_on_load, r.wide_out = wide_out;
         if (nx) r.dn = nx->dn, r.rc = wp.n_seg > 1 ? rcv : nullptr;  // dK's terms
+        if (any) results_to_rows(r, *any);
         return fla::walk_dkdv(dtype, wp.D, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }
     if (walk) {  // (the states forward saved are per 128-row chunk: only this path reads them)
@@ -1286,7 +1319,8 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
 }
 
 // ---- widths that are no multiples of 8: the plain chunk-wise operator on copies with aligned rows (fla_pack.h).
-// The copies' columns beyond the true width are zeros, so sums and results are the same.  Forward leaves its copies of q, k, v in the state
+// The copies' columns beyond the true width are zeros, so sums and results are the same.  The walks above 64 columns store results to
+// the caller's rows (AnyRows); other kernels to aligned ones, which a copy takes there.  Forward leaves its copies of q, k, v in the state
 // buffer, behind the state, and backward takes them from there.
 struct PackPlan {
     bool ok;
@@ -1360,10 +1394,11 @@ int packed_forward(const PackPlan &p, const View &q, const View &k, const View &
     if (p.q_bytes) in.in(q, qp, dqk, p.wq), in.in(k, kp, dqk, p.wq);
     if (p.v_bytes) in.in(v, vp, dv, p.wv), out.out(op, o, dv);
     if (int rc = in.launch(stream)) return rc;
+    AnyRows any{&o, nullptr, nullptr, nullptr, dqk, dv, false};
     if (int rc = chunked_forward(qp, kp, vp, op, B, H, N, p.wq, p.wv, dtype, state_out, state_valid, workspace, p.inner_work,
-                                 stream))
+                                 stream, 0, nullptr, nullptr, nullptr, p.v_bytes ? &any : nullptr))
         return rc;
-    return out.launch(stream);
+    return any.done ? FLA_OK : out.launch(stream);
 }
 
 int packed_backward(const PackPlan &p, const View &go, const View &q, const View &k, const View &v, const View &dq,
@@ -1395,10 +1430,11 @@ int packed_backward(const PackPlan &p, const View &go, const View &q, const View
         in.in(go, gop, dv, p.wv), out.out(dvp, dvv, dv);
     }
     if (int rc = in.launch(stream)) return rc;
+    AnyRows any{nullptr, &dq, &dk, &dvv, dqk, dv, false};
     if (int rc = chunked_backward(gop, qp, kp, vp, dqp, dkp, dvp, B, H, N, p.wq, p.wv, dtype, state_in, workspace, p.inner_work,
-                                  stream, 0, nullptr, causal))
+                                  stream, 0, nullptr, causal, false, &any))
         return rc;
-    return out.launch(stream);
+    return any.done ? FLA_OK : out.launch(stream);
 }
 
 // takes FLA_GRADS_F32 off a dtype

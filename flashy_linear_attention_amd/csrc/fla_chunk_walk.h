@@ -75,6 +75,13 @@ namespace fla {
 // rows per chunk of the walk kernels: 128, or 64 at D = 128 (tiles and state must share the LDS)
 constexpr int walk_rows(int D) { return D <= 64 ? 128 : 64; }
 
+// a result's place: pointer, element strides, true width
+struct WalkRowsOut {
+    void *ptr;
+    int64_t s_b, s_h, s_n;
+    int32_t width;
+};
+
 struct WalkParams {
     const void *q, *k, *v, *go;  // operands (go: backward only); (B, H, N, D)
     void *o, *dq, *dk, *dv;      // results (forward: o; backward: dq, dk, dv)
@@ -146,6 +153,11 @@ struct WalkParams {
     // point to floats; what is stored is rounded to bf16 as always).  Kernels of their own (WIDE): as a branch in front of the
     // stores it cost the others up to 3 %
     int32_t wide_out;
+    // walk_fwd_kernel (D = 128), walk_dkdv_kernel and walk_bwd_rev_kernel, plain, and walk_bwd_rev_wide_kernel with v of at most 64
+    // columns and without dQ (dk alone): the results go to rows of any alignment and width (WalkAnyRows), in place of o, dq, dk
+    // and dv.  Kernels of their own (ROWS)
+    int32_t any_rows;
+    WalkRowsOut rows_o, rows_dq, rows_dk, rows_dv;
     // A v of 129 .. 256 columns beside a wide q / k: its columns 128 .. are a second half of true width wv2, and grid y
     // picks a part of the work.  0: none.  1 (walk_fwd_wide_kernel): half y of v.  2, 3 (walk_bwd_rev_kernel): half y of
     // q / k with half y (2) or half 1 - y (3) of v, so that the two parts of a launch write different columns.
@@ -624,6 +636,40 @@ struct WalkResult {
         const int size = wide ? 4 : 2;
         stride = (int)stride_n * size;
         rs = __builtin_amdgcn_make_buffer_rsrc(static_cast<char *>(base) + at * size, 0, (N - 1) * stride + width * size, 0x00020000);
+    }
+};
+
+// A result whose rows start at any element: 16-byte stores at the rows' own alignment, what is left of a row element by
+// element.  Forward + backward with results in aligned rows that a copy took to the caller's -> this way: B H 32, N 2048, 153 over
+// 64 columns (306-byte rows) 139.5 -> 127.3 us; B H 32, N 4096, 100 columns 231 -> 177, by one reverse walk 218 -> 167; B H 128 736 -> 547.
+template <typename T>
+struct WalkAnyRows {
+    T *base;
+    int64_t stride;
+    int width, N;
+    __device__ __forceinline__ WalkAnyRows(const WalkRowsOut &o, int b, int h, int col0, int w, int n)
+        : base(static_cast<T *>(o.ptr) + b * o.s_b + h * o.s_h + col0), stride(o.s_n), width(w), N(n) {}
+    template <int D, int PER>
+    __device__ __forceinline__ void store(int row, int g, int db0, const f32x16 (&acc)[WalkCfg<D>::DBW]) const {
+        u32x4 pk[WalkCfg<D>::DBW][2];
+        walk_pack<T, D, PER>(acc, g, db0, pk);
+        if (row >= N) return;
+        T *r = base + row * stride;
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+#pragma unroll
+            for (int hq = 0; hq < 2; ++hq) {
+                const int col = 32 * (db0 + i) + 16 * g + 8 * hq;
+                if (col + 8 <= width) {
+                    __builtin_memcpy(r + col, &pk[i][hq], 16);
+                } else if (col < width) {
+#pragma unroll
+                    for (int e = 0; e < 7; ++e) {
+                        const uint16_t x = (uint16_t)(pk[i][hq][e / 2] >> (16 * (e & 1)));
+                        if (e < width % 8) __builtin_memcpy(r + col + e, &x, 2);  // (the same for all lanes)
+                    }
+                }
+            }
     }
 };
 
@@ -1124,7 +1170,7 @@ __device__ __forceinline__ void walk_write_state(float *out, int wave, int lane,
 template <typename T, int NORM, bool FM>
 constexpr bool walk_fwd_scaled = std::is_same<T, _Float16>::value && NORM == 0 && !FM;
 
-template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool WIDE = false>
+template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool WIDE = false, bool ROWS = false>
 __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1155,6 +1201,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
     const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
     const WalkResult ro(p.o, b * p.os_b + h * p.os_h, p.os_n, p.wv, N, WIDE);
+    const WalkAnyRows<T> ao(p.rows_o, b, h, 0, p.rows_o.width, N);
 
     f32x16 st[W::NBW];
     walk_load_init<D, B>(p, sl, wave, lane, st, false);
@@ -1306,7 +1353,10 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                         acc[i][v] *= feature_slope_c<decltype(map)::value>(static_cast<float>(ys[i][v / 8][v % 8]));
             });
         }
-        walk_store<T, D, OB::PER>(ro.rs, ro.stride, p.wv, row, g, db0, acc, 0, nullptr, 0, WIDE);
+        if constexpr (ROWS)
+            ao.template store<D, OB::PER>(row, g, db0, acc);
+        else
+            walk_store<T, D, OB::PER>(ro.rs, ro.stride, p.wv, row, g, db0, acc, 0, nullptr, 0, WIDE);
         walk_update<T, D, B>(tk, tv, wave, lane, st);
         if constexpr (SCALED) walk_state_max<D, B>(smax, wave, lane, st);
         if constexpr (NORM == 1) {
@@ -1624,7 +1674,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 // D = 128, so the chunk's dn comes as ordinary loads, a chunk ahead, in the order in which the scores' registers take it, and
 // rc is carried in registers: a wave adds up its own output columns, in the order of an MFMA's A rows, and one MFMA
 // per 32 columns adds rc to the result (walk_split3).
-template <typename T, int D, bool NORM, int NQ = D / 32, int NV = D / 32, bool WIDE = false>
+template <typename T, int D, bool NORM, int NQ = D / 32, int NV = D / 32, bool WIDE = false, bool ROWS = false>
 __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1653,6 +1703,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
     const u32x4 rg = make_rsrc(G, (uint32_t)((N - 1) * gs2 + p.wv * 2));
     const WalkResult rdk(p.dk, b * p.dks_b + h * p.dks_h, p.dks_n, p.wqk, N, WIDE);
     const WalkResult rdv(p.dv, b * p.dvs_b + h * p.dvs_h, p.dvs_n, p.wv, N, WIDE);
+    const WalkAnyRows<T> adk(p.rows_dk, b, h, 0, p.rows_dk.width, N), adv(p.rows_dv, b, h, 0, p.rows_dv.width, N);
 
     f32x16 st[W::NBW];  // R[q/k index][v index]
     walk_load_init<D, B>(p, sl, wave, lane, st, true);
@@ -1740,7 +1791,10 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         walk_product<T, D, true, 0, B::KQ, NV>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
         }, acc);
-        walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, p.wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
+        if constexpr (ROWS)
+            adv.template store<D, OV::PER>(row, g, OV::db0(wave), acc);
+        else
+            walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, p.wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
         // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
         if constexpr (NORM) {
             walk_product<T, D, true, 3>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
@@ -1755,7 +1809,10 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
                 return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
             }, acc);
         }
-        walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, p.wqk, row, g, db0, acc, p.fmap, tk, 32 * rb + l32, WIDE);
+        if constexpr (ROWS)
+            adk.template store<D, OQ::PER>(row, g, db0, acc);
+        else
+            walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, p.wqk, row, g, db0, acc, p.fmap, tk, 32 * rb + l32, WIDE);
         walk_update<T, D, B>(tq, tg, wave, lane, st);
         if constexpr (NORM) {  // rc += this chunk's dn_i q_i
             static_for<0, W::C / 16>([&](auto j) {
@@ -1790,7 +1847,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 // The one 16-bit state in LDS holds R for dV and dK, then X for dQ.  q, k, v, dO are read once and
 // nothing but the results is written, where the walk for dQ followed by walk_dkdv_kernel reads
 // dO, v, k twice.
-template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool ACCUM = false, bool FM = false, bool WIDE = false>
+template <typename T, int D, int NQ = D / 32, int NV = D / 32, bool ACCUM = false, bool FM = false, bool WIDE = false, bool ROWS = false>
 __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1827,6 +1884,8 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
     const WalkResult rdq(p.dq, b * p.dqs_b + h * p.dqs_h + qh * D, p.dqs_n, wqk, N, WIDE);
     const WalkResult rdk(p.dk, b * p.dks_b + h * p.dks_h + qh * D, p.dks_n, wqk, N, WIDE);
     const WalkResult rdv(p.dv, b * p.dvs_b + h * p.dvs_h + vh * D, p.dvs_n, wv, N, WIDE);
+    const WalkAnyRows<T> adq(p.rows_dq, b, h, 0, p.rows_dq.width, N), adk(p.rows_dk, b, h, 0, p.rows_dk.width, N),
+        adv(p.rows_dv, b, h, 0, p.rows_dv.width, N);
 
     f32x16 st[W::NBW];  // R [q/k index][v index]
     f32x16 xs[W::NBW];  // X [q/k index][v index]
@@ -1875,14 +1934,20 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
             return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
         }, acc);
         if constexpr (ACCUM) prev.add_to(acc);
-        walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
+        if constexpr (ROWS)
+            adv.template store<D, OV::PER>(row, g, OV::db0(wave), acc);
+        else
+            walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
         if constexpr (ACCUM) prev_qk.request(rdk.rs, rdk.stride, wqk, row, g, OQ::db0(wave));
         // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
         walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
         if constexpr (ACCUM) prev_qk.add_to(acc);
-        walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, wqk, row, g, OQ::db0(wave), acc, fmap, tk, 32 * rb + l32, WIDE);
+        if constexpr (ROWS)
+            adk.template store<D, OQ::PER>(row, g, OQ::db0(wave), acc);
+        else
+            walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, wqk, row, g, OQ::db0(wave), acc, fmap, tk, 32 * rb + l32, WIDE);
         // R += Q^T dO touches registers and tiles only, so it can sit on either side of the barriers: the waves of
         // the last row block, with one score block in dV and dK against two, take it here, the others after dQ,
         // where they have one score block against two
@@ -1904,7 +1969,10 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
             return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
         }, acc);
         if constexpr (ACCUM) prev_qk.add_to(acc);
-        walk_store<T, D, OQ::PER>(rdq.rs, rdq.stride, wqk, row, g, OQ::db0(wave), acc, fmap, tq, 32 * rb + l32, WIDE);
+        if constexpr (ROWS)
+            adq.template store<D, OQ::PER>(row, g, OQ::db0(wave), acc);
+        else
+            walk_store<T, D, OQ::PER>(rdq.rs, rdq.stride, wqk, row, g, OQ::db0(wave), acc, fmap, tq, 32 * rb + l32, WIDE);
         if (!(kSplitUpdate && rb == 1)) walk_update<T, D, B, false, true>(tq, tg, wave, lane, st);
         sync();  // every wave has read X and is done with the tiles
         walk_state_to_lds<T, D, B>(tl, wave, lane, st);
@@ -1924,7 +1992,7 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_kernel(const WalkParams p
 // LDS as in walk_fwd_wide_kernel: a set of (Q_h, K_h) tiles per half, two (V, dO) pairs by chunk parity, and ONE
 // 16-bit state that holds R_h, then X_h, of the half at work; at the end of a half-chunk the other half's R (in
 // registers throughout) is rounded into it.  With dQ four states in registers: built for v blocks NV = 2 only.
-template <typename T, int NV, bool WITH_DQ, bool WIDE = false>
+template <typename T, int NV, bool WITH_DQ, bool WIDE = false, bool ROWS = false>
 __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     constexpr int D = 128, NQ = D / 32;
@@ -1957,6 +2025,7 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
     const int64_t dq_at = b * p.dqs_b + h * p.dqs_h, dk_at = b * p.dks_b + h * p.dks_h;
     const WalkResult rdq0(p.dq, dq_at, p.dqs_n, p.wqk, N, WIDE), rdq1(p.dq, dq_at + D, p.dqs_n, p.wqk2, N, WIDE);
     const WalkResult rdk0(p.dk, dk_at, p.dks_n, p.wqk, N, WIDE), rdk1(p.dk, dk_at + D, p.dks_n, p.wqk2, N, WIDE);
+    const WalkAnyRows<T> adk0(p.rows_dk, b, h, 0, D, N), adk1(p.rows_dk, b, h, D, p.rows_dk.width - D, N);
     const WalkResult rdv(p.dv, b * p.dvs_b + h * p.dvs_h, p.dvs_n, p.wv, N, WIDE);
 
     f32x16 st0[W::NBW], st1[W::NBW];  // R_0, R_1
@@ -2032,7 +2101,10 @@ __global__ __launch_bounds__(256, 1) void walk_bwd_rev_wide_kernel(const WalkPar
             walk_product<T, D, true, 0, B::KQ, NV, HF != 0>(tk, tq, tg, wave, lane, later, rows_of_state, dvacc);
             f32x16 acc[W::DBW];
             walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, cols_of_state, acc);
-            walk_store<T, D, OQ::PER>((HF ? rdk1 : rdk0).rs, rdk0.stride, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc, 0, nullptr, 0, WIDE);
+            if constexpr (ROWS)
+                (HF ? adk1 : adk0).template store<D, OQ::PER>(row, g, OQ::db0(wave), acc);
+            else
+                walk_store<T, D, OQ::PER>((HF ? rdk1 : rdk0).rs, rdk0.stride, HF ? p.wqk2 : p.wqk, row, g, OQ::db0(wave), acc, 0, nullptr, 0, WIDE);
             if constexpr (WITH_DQ) {
                 sync();  // every wave has read R_h
                 // (X stays in its accumulation registers up to here: without this the copies that the rounding
@@ -2653,11 +2725,19 @@ hipError_t launch_walk_kernel(int64_t grid, int smem, const WalkParams &p, hipSt
     return launch_kernel<kern>(dim3((unsigned)grid, (unsigned)parts), dim3(256), smem, stream, p);
 }
 
-template <typename T, int D, bool WIDE = false>
+inline bool walk_rows_ok(const WalkRowsOut &o, int most) { return o.ptr && o.width >= 1 && o.width <= most; }
+
+template <typename T, int D, bool WIDE = false, bool ROWS = false>
 hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
+    if constexpr (!ROWS) {
+        if (p.any_rows) {
+            if constexpr (D == 128 && !WIDE) return launch_walk_fwd<T, D, false, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    }
     if constexpr (!WIDE) {
         if (p.wide_out) {  // (dQ's walk)
-            if constexpr (D == 128 && std::is_same<T, __bf16>::value) return launch_walk_fwd<T, D, true>(p, stream);
+            if constexpr (D == 128 && !ROWS && std::is_same<T, __bf16>::value) return launch_walk_fwd<T, D, true>(p, stream);
             return hipErrorNotSupported;
         }
     }
@@ -2672,7 +2752,9 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     if (p.init_is_totals && (D != 128 || p.n_seg < 3 || !p.init)) return hipErrorInvalidValue;
     if (p.entry_out && (!p.init_is_totals || p.dn || p.slope_y)) return hipErrorInvalidValue;
     if (WIDE && p.denom) return hipErrorInvalidValue;
-    if (p.denom || p.dn) {  // the normaliser's terms: its vectors live behind the state
+    if constexpr (ROWS) {
+        if (p.denom || p.dn || fm || !walk_rows_ok(p.rows_o, p.wv)) return hipErrorInvalidValue;
+    } else if (p.denom || p.dn) {  // the normaliser's terms: its vectors live behind the state
         if ((p.dn && !p.zc) || (p.denom && p.n_seg > 1 && !p.vsum)) return hipErrorInvalidValue;
         constexpr int smem_n = smem + (kDouble ? 2 : 1) * WalkCfg<D>::VEC;
         if constexpr (!WIDE)
@@ -2682,19 +2764,21 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
         return fm ? launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, true, NB, NB, WIDE>>(grid, smem_n, p, stream)
                   : launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 2, false, NB, NB, WIDE>>(grid, smem_n, p, stream);
     }
-    if (fm) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true, NB, NB, WIDE>>(grid, smem, p, stream);
+    if constexpr (!ROWS)
+        if (fm) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true, NB, NB, WIDE>>(grid, smem, p, stream);
     if constexpr (D == 128) {
         // operands of at most 64 true columns on a side (the halves of a wide q / k, a narrow v): the kernels that
         // leave out the blocks of padding, which the states in memory may not hold either
-        if (p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2, WIDE>>(grid, smem, p, stream);
-        if (p.wqk <= 64 && p.wv > 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4, WIDE>>(grid, smem, p, stream);
-        if (p.wqk <= 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 2, WIDE>>(grid, smem, p, stream);
+        if (p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2, WIDE, ROWS>>(grid, smem, p, stream);
+        if (p.wqk <= 64 && p.wv > 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4, WIDE, ROWS>>(grid, smem, p, stream);
+        if (p.wqk <= 64 && p.wv <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 2, WIDE, ROWS>>(grid, smem, p, stream);
     }
-    return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, NB, NB, WIDE>>(grid, smem, p, stream);
+    return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, NB, NB, WIDE, ROWS>>(grid, smem, p, stream);
 }
 
 template <typename T>
 hipError_t launch_walk_fwd_wide(const WalkParams &p, hipStream_t stream) {
+    if (p.any_rows) return hipErrorNotSupported;
     using W = WalkCfg<128>;
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
@@ -2714,6 +2798,7 @@ hipError_t launch_walk_fwd_wide(const WalkParams &p, hipStream_t stream) {
 
 template <typename T, int D, bool WIDE = false>
 hipError_t launch_walk_bwd(const WalkParams &p, hipStream_t stream) {
+    if (p.any_rows) return hipErrorNotSupported;
     if constexpr (!WIDE) {
         if (p.wide_out) {
             if constexpr (std::is_same<T, __bf16>::value) return launch_walk_bwd<T, D, true>(p, stream);
@@ -2737,11 +2822,17 @@ hipError_t launch_walk_bwd(const WalkParams &p, hipStream_t stream) {
     return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_x, stream, p);
 }
 
-template <typename T, int D, bool WIDE = false>
+template <typename T, int D, bool WIDE = false, bool ROWS = false>
 hipError_t launch_walk_dkdv(const WalkParams &p, hipStream_t stream) {
+    if constexpr (!ROWS) {
+        if (p.any_rows) {
+            if constexpr (!WIDE) return launch_walk_dkdv<T, D, false, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    }
     if constexpr (!WIDE) {
         if (p.wide_out) {
-            if constexpr (std::is_same<T, __bf16>::value) return launch_walk_dkdv<T, D, true>(p, stream);
+            if constexpr (!ROWS && std::is_same<T, __bf16>::value) return launch_walk_dkdv<T, D, true>(p, stream);
             return hipErrorNotSupported;
         }
     }
@@ -2750,7 +2841,9 @@ hipError_t launch_walk_dkdv(const WalkParams &p, hipStream_t stream) {
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr int smem = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
     static_assert(smem <= 160 * 1024, "two sets of tiles and the state must fit the LDS of a CU");
-    if (p.dn) {
+    if constexpr (ROWS) {
+        if (p.dn || p.fmap || !walk_rows_ok(p.rows_dk, p.wqk) || !walk_rows_ok(p.rows_dv, p.wv)) return hipErrorInvalidValue;
+    } else if (p.dn) {
         if (p.n_seg > 1 && !p.rc) return hipErrorInvalidValue;
         constexpr auto kern = walk_dkdv_kernel<T, D, true, NB, NB, WIDE>;
         if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
@@ -2758,19 +2851,27 @@ hipError_t launch_walk_dkdv(const WalkParams &p, hipStream_t stream) {
     }
     if constexpr (D == 128) {
         if (!p.fmap && p.wqk > 64 && p.wv <= 64) {
-            constexpr auto kern = walk_dkdv_kernel<T, D, false, 4, 2, WIDE>;
+            constexpr auto kern = walk_dkdv_kernel<T, D, false, 4, 2, WIDE, ROWS>;
             if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
             return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
         }
     }
-    constexpr auto kern = walk_dkdv_kernel<T, D, false, NB, NB, WIDE>;
+    constexpr auto kern = walk_dkdv_kernel<T, D, false, NB, NB, WIDE, ROWS>;
     if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
     return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
 }
 
-template <typename T, int D, bool WIDE = false>
+template <typename T, int D, bool WIDE = false, bool ROWS = false>
 hipError_t launch_walk_bwd_rev(const WalkParams &p, hipStream_t stream) {
-    if constexpr (!WIDE) {
+    if constexpr (!ROWS) {
+        if (p.any_rows) {
+            if constexpr (!WIDE) return launch_walk_bwd_rev<T, D, false, true>(p, stream);
+            return hipErrorNotSupported;
+        }
+    } else if (p.quad || p.fmap || !walk_rows_ok(p.rows_dq, p.wqk) || !walk_rows_ok(p.rows_dk, p.wqk) || !walk_rows_ok(p.rows_dv, p.wv)) {
+        return hipErrorInvalidValue;
+    }
+    if constexpr (!WIDE && !ROWS) {
         if (p.wide_out) {
             if constexpr (std::is_same<T, __bf16>::value) return launch_walk_bwd_rev<T, D, true>(p, stream);
             return hipErrorNotSupported;
@@ -2784,18 +2885,21 @@ hipError_t launch_walk_bwd_rev(const WalkParams &p, hipStream_t stream) {
     static_assert(smem <= 160 * 1024, "two sets of tiles and the state must fit the LDS of a CU");
     constexpr int NB = D / 32;
     if (p.quad) {
-        if (WIDE) return hipErrorNotSupported;
+        if constexpr (WIDE || ROWS) return hipErrorNotSupported;
+        else {
         if ((p.quad != 2 && p.quad != 3) || p.wqk != 128 || p.wv != 128 || p.wqk2 < 1 || p.wqk2 > 128 || p.wv2 < 1 ||
             p.wv2 > 128 || p.fmap)
             return hipErrorInvalidValue;
         return p.accumulate ? launch_walk_kernel<walk_bwd_rev_kernel<T, D, D / 32, D / 32, true>>(grid, smem, p, stream, 2)
                             : launch_walk_kernel<walk_bwd_rev_kernel<T, D>>(grid, smem, p, stream, 2);
+        }
     }
     if constexpr (D == 128) {  // a half of a wide q / k against a narrow v: without the blocks of padding
-        if (!p.fmap && p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2, false, false, WIDE>>(grid, smem, p, stream);
+        if (!p.fmap && p.wqk > 64 && p.wv <= 64) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, 4, 2, false, false, WIDE, ROWS>>(grid, smem, p, stream);
     }
-    if (p.fmap) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, NB, NB, false, true, WIDE>>(grid, smem, p, stream);
-    return launch_walk_kernel<walk_bwd_rev_kernel<T, D, NB, NB, false, false, WIDE>>(grid, smem, p, stream);
+    if constexpr (!ROWS)
+        if (p.fmap) return launch_walk_kernel<walk_bwd_rev_kernel<T, D, NB, NB, false, true, WIDE>>(grid, smem, p, stream);
+    return launch_walk_kernel<walk_bwd_rev_kernel<T, D, NB, NB, false, false, WIDE, ROWS>>(grid, smem, p, stream);
 }
 
 template <typename T, bool WIDE = false>
@@ -2816,8 +2920,13 @@ hipError_t launch_walk_bwd_rev_wide(const WalkParams &p, hipStream_t stream) {
     constexpr int smem = 8 * W::TILE + W::STATE;  // two sets of (Q_h, K_h), two of (V, dO), one state
     static_assert(smem <= 160 * 1024, "the tiles and the state must fit the LDS of a CU");
     if (p.dq) {
+        if (p.any_rows) return hipErrorNotSupported;
         if (!p.xtotal || !p.xtotal2 || (p.n_seg > 1 && (!p.xinit || !p.xinit2))) return hipErrorInvalidValue;
         return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, true, WIDE>>(grid, smem, p, stream);
+    }
+    if (p.any_rows) {
+        if (WIDE || p.wv > 64 || p.rows_dk.width <= 128 || !walk_rows_ok(p.rows_dk, 128 + p.wqk2)) return hipErrorInvalidValue;
+        return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, false, false, true>>(grid, smem, p, stream);
     }
     if (p.wv <= 64) return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 2, false, WIDE>>(grid, smem, p, stream);
     if constexpr (WIDE)  // (40 bytes of spills, which this kernel may not have)
