@@ -804,6 +804,10 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
     const float *fwd_entries[2] = {nullptr, nullptr}, *entries[2] = {nullptr, nullptr};
     // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
     const bool rev_sums_on_load = sums_on_load(wp, kSumOnLoadWide);
+    // dQ's walks add up their halves' totals of Q^T dO on their way (WalkParams::r_totals).  A totals kernel in front -> this: 256 / 64,
+    // B H 32, N 2048 104.5 -> 101.0 us, B H 64, N 4096 293 -> 288.  With a v above 64 columns a walk holds two full states: 256 / 128 eight
+    // segments or more 159.8 -> 155.5 (B H 32, N 2048), four 399 -> 403 (B H 64, N 4096), ten short ones 130.6 -> 130.4
+    const bool dq_walk_sums = !one_walk && (dv <= 64 || (dqk > 192 && wp.n_seg >= 8)) && wp.n_seg > 2 && dtype == FLA_DTYPE_BF16;
     if (wp.n_seg > 1) {
         float *const none[2] = {nullptr, nullptr};
         if (state_in) {
@@ -815,8 +819,11 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
                 return rc;
         }
         void *const work[2] = {ws, ws + wp.work_bytes};
-        if (int rc = wide_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, work, none, entries, s, rev_sums_on_load, dv <= 64))
+        if (dq_walk_sums) {
+            for (int h = 0; h < 2; ++h) entries[h] = static_cast<const float *>(work[h]);
+        } else if (int rc = wide_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, work, none, entries, s, rev_sums_on_load, dv <= 64)) {
             return rc;
+        }
     }
     fla::WalkParams r = reverse_walk_params(wp, go, q, k, v, dq, dk, dvv, B, H, N, 128, dv);
     r.wqk2 = (int32_t)(dqk - 128);
@@ -836,8 +843,16 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
         const View dq_h{static_cast<const char *>(dq.ptr) + h * 128 * (wide_out ? 4 : 2), dq.strides};
         fla::WalkParams w = lower_walk_params(wp, go, v, column_half(k, h), dq_h, B, H, N, dv, h ? dqk - 128 : 128, fwd_entries[h]);
         w.init_transposed = 1, w.wide_out = wide_out;
+        if (dq_walk_sums) {
+            w.r_q = column_half(q, h).ptr, w.rs_b = q.strides[0], w.rs_h = q.strides[1], w.rs_n = q.strides[2];
+            w.r_totals = const_cast<float *>(entries[h]), w.r_frags = rev_sums_on_load;
+        }
         if (rows) w.any_rows = 1, w.rows_o = rows_out(column_half(*any->dq, h), h ? any->dqk - 128 : 128), w.o = nullptr;
         if (fla::walk_fwd(dtype, wp.D, w, s) != hipSuccess) return FLA_ERR_LAUNCH;
+    }
+    if (dq_walk_sums && !rev_sums_on_load) {
+        float *const t0 = const_cast<float *>(entries[0]), *const t1 = const_cast<float *>(entries[1]);
+        if (fla::walk_scan(t0, t0, B * H, (int)wp.n_seg, wp.D, dv <= 64 ? 64 : 128, 1, s, t1, t1) != hipSuccess) return FLA_ERR_LAUNCH;
     }
     r.dq = nullptr;
     if (rows) r.any_rows = 1, r.rows_dk = rows_out(*any->dk, any->dqk), r.dk = nullptr;
@@ -1190,6 +1205,8 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
         const bool rev_sums_on_load = (one_walk || causal || nx) && sums_on_load(wp);
         float *const rcv = nx ? reinterpret_cast<float *>(static_cast<char *>(nx->vec) + walk_vec_bytes(B, H, N, dqk, dv)) : nullptr;
+        // dQ's walk adds up the segments' totals of Q^T dO on its way (WalkParams::r_totals, figures there)
+        const bool dq_walk_sums = !one_walk && !nx && !fmap && wp.n_seg > 2 && dtype == FLA_DTYPE_BF16 && dqk > 64;
         if (wp.n_seg > 1) {
             if (!state_in) {
                 const float *fwd_entry = nullptr;
@@ -1198,7 +1215,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                     return rc;
                 state_in = fwd_entry;
             }
-            if (!nx)
+            if (!nx && !dq_walk_sums)
                 if (int rc = walk_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, workspace, nullptr, &entry, s, 0, nullptr,
                                                nullptr, rev_sums_on_load))
                     return rc;
@@ -1241,7 +1258,16 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         if (any) {
             w.any_rows = 1, w.rows_o = rows_out(*any->dq, any->dqk), w.o = nullptr;
         }
+        if (dq_walk_sums) {
+            w.r_q = q.ptr, w.rs_b = q.strides[0], w.rs_h = q.strides[1], w.rs_n = q.strides[2];
+            w.r_totals = static_cast<float *>(workspace), w.r_frags = rev_sums_on_load;
+            entry = w.r_totals;
+        }
         if (fla::walk_fwd(dtype, wp.D, w, s) != hipSuccess) return FLA_ERR_LAUNCH;
+        if (dq_walk_sums && !rev_sums_on_load &&
+            fla::walk_scan(entry, static_cast<float *>(workspace), B * H, (int)wp.n_seg, wp.D, fla::walk_totals_cols(wp.D, (int)dqk, (int)dv), 1,
+                           s) != hipSuccess)
+            return FLA_ERR_LAUNCH;
         // dV, dK: the reverse walk over the same segments
         fla::WalkParams r{};
         r.q = q.ptr, r.k = k.ptr, r.v = v.ptr, r.go = go.ptr;

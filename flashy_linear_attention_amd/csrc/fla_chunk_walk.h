@@ -158,6 +158,15 @@ struct WalkParams {
     // and dv.  Kernels of their own (ROWS)
     int32_t any_rows;
     WalkRowsOut rows_o, rows_dq, rows_dk, rows_dv;
+    // walk_fwd_kernel as dQ's walk (D = 128, bf16, plain, q and k above 64 columns; kernels of their own: RSUM), three segments or more:
+    // beside dQ it adds up its segment's total of Q^T dO for the reverse walk -- dO is in LDS already -- and writes it to r_totals,
+    // as walk_totals_kernel would (r_frags: by fragments).  Null: not.  Forward + backward, a totals kernel in front -> this: D 128, B H
+    // 32, N 2048 83.0 -> 78.9 us; B H 64, N 4096 223.8 -> 213.7; B H 16, N 20000 295 -> 287; D 80, B H 24, N 1500 59.9 -> 57.6.  With two
+    // segments, where half of the workgroups have that work, B H 128, N 4096 422 -> 418, N 1024 111 -> 113
+    const void *r_q;
+    int64_t rs_b, rs_h, rs_n;
+    int32_t r_frags;
+    float *r_totals;
     // A v of 129 .. 256 columns beside a wide q / k: its columns 128 .. are a second half of true width wv2, and grid y
     // picks a part of the work.  0: none.  1 (walk_fwd_wide_kernel): half y of v.  2, 3 (walk_bwd_rev_kernel): half y of
     // q / k with half y (2) or half 1 - y (3) of v, so that the two parts of a launch write different columns.
@@ -1170,7 +1179,8 @@ __device__ __forceinline__ void walk_write_state(float *out, int wave, int lane,
 template <typename T, int NORM, bool FM>
 constexpr bool walk_fwd_scaled = std::is_same<T, _Float16>::value && NORM == 0 && !FM;
 
-template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool WIDE = false, bool ROWS = false>
+template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool WIDE = false, bool ROWS = false,
+          bool RSUM = false>
 __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1178,11 +1188,13 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     using B = WalkExt<D, NQ, NV>;
     using OB = WalkOut<D, NV>;  // the result is as wide as v
     static_assert(NORM == 0 || (NQ == W::DB && NV == W::DB), "the normaliser's variants are built for full widths");
-    constexpr int SETS = DOUBLE ? 2 : 1;
+    constexpr int SETS = DOUBLE ? 2 : 1, TPS = RSUM ? 4 : 3;  // (tiles per set)
+    static_assert(!RSUM || (DOUBLE && NORM == 0 && !FM), "the plain dQ walk");
+    using RB = WalkExt<D, D / 32, NQ>;  // (RSUM: the total's blocks -- q's columns are v's here, dO's are q's)
     constexpr bool SCALED = walk_fwd_scaled<T, NORM, FM>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
-    unsigned char *tl = smem + SETS * 3 * W::TILE;
+    unsigned char *tl = smem + SETS * TPS * W::TILE;
     unsigned char *xv = tl + W::STATE;  // NORM 2: per set: zc, (unused), dn of the chunk
     float *zv = reinterpret_cast<float *>(xv), *zpart = zv + 256;  // NORM 1: zc; the waves' column sums
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
@@ -1202,6 +1214,18 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
     const WalkResult ro(p.o, b * p.os_b + h * p.os_h, p.os_n, p.wv, N, WIDE);
     const WalkAnyRows<T> ao(p.rows_o, b, h, 0, p.rows_o.width, N);
+
+    // (RSUM: the first segment's total is under no sum of the reverse walk)
+    const bool rsum = RSUM && sl.seg > 0;
+    const int rs2 = RSUM ? (int)p.rs_n * 2 : 0;
+    const u32x4 rr = RSUM ? make_rsrc(static_cast<const T *>(p.r_q) + b * p.rs_b + h * p.rs_h, (uint32_t)((N - 1) * rs2 + p.wv * 2)) : rq;
+    f32x16 rt[W::NBW];
+    if constexpr (RSUM) {
+#pragma unroll
+        for (int i = 0; i < W::NBW; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) rt[i][v] = 0.f;
+    }
 
     f32x16 st[W::NBW];
     walk_load_init<D, B>(p, sl, wave, lane, st, false);
@@ -1249,10 +1273,12 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     }
 
     auto load_chunk = [&](int c, int buf) {
-        const uint32_t base = lds0 + buf * 3 * W::TILE;
+        const uint32_t base = lds0 + buf * TPS * W::TILE;
         walk_load_tile<D>(rq, base, c * W::C, qs2, p.wqk, wave, lane);
         walk_load_tile<D>(rk, base + W::TILE, c * W::C, ks2, p.wqk, wave, lane);
         walk_load_tile<D>(rv, base + 2 * W::TILE, c * W::C, vs2, p.wv, wave, lane);
+        if constexpr (RSUM)
+            if (rsum) walk_load_tile<D>(rr, base + 3 * W::TILE, c * W::C, rs2, p.wv, wave, lane);
         const uint32_t xbase = lds0 + SETS * 3 * W::TILE + W::STATE + buf * W::VEC;
         if constexpr (NORM == 2) {
             walk_load_vec<D>(p.zc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase, lane);
@@ -1264,7 +1290,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
 #pragma unroll 1
     for (int c = sl.c_lo; c < sl.c_hi; ++c) {
         const int row0 = c * W::C, buf = DOUBLE ? (c - sl.c_lo) & 1 : 0;
-        unsigned char *tq = smem + buf * 3 * W::TILE, *tk = tq + W::TILE, *tv = tq + 2 * W::TILE;
+        unsigned char *tq = smem + buf * TPS * W::TILE, *tk = tq + W::TILE, *tv = tq + 2 * W::TILE;
         const int row = row0 + 32 * rb + l32;
         // dQ walk with a feature map: this lane's values of phi(xq) under its accumulator registers,
         // requested before the tiles so that they have arrived with them
@@ -1286,7 +1312,9 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
             if (more) load_chunk(c + 1, buf ^ 1);  // (every wave has left the barrier that ended the reads of that set)
             // this wave's loads of chunk c have landed when at most the loads issued after them are
             // outstanding (the stores of the previous chunk were issued before those)
-            if (more)
+            if (more && rsum)
+                wait_vm<4 * W::NI>();
+            else if (more)
                 wait_vm<3 * W::NI + n_extra>();
             else
                 wait_vm<0>();
@@ -1358,6 +1386,8 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         else
             walk_store<T, D, OB::PER>(ro.rs, ro.stride, p.wv, row, g, db0, acc, 0, nullptr, 0, WIDE);
         walk_update<T, D, B>(tk, tv, wave, lane, st);
+        if constexpr (RSUM)
+            if (rsum) walk_update<T, D, RB>(tv + W::TILE, tq, wave, lane, rt);
         if constexpr (SCALED) walk_state_max<D, B>(smax, wave, lane, st);
         if constexpr (NORM == 1) {
             f32x16 zs;
@@ -1381,6 +1411,14 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                 zc_publish(c + 1);
             }
         }
+    }
+    if constexpr (RSUM) {
+        float *out = p.r_totals + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D);
+        if (rsum && p.r_frags)
+            walk_write_frags<D, RB>(out, wave, lane, rt);
+        else if (rsum)
+            walk_write_state<D, RB>(out, wave, lane, rt);
+        return;
     }
     if (p.total_out && sl.c_hi == p.n_chunks) {  // the state after the last chunk, for the backward walks
         float *out = p.total_out + (int64_t)sl.bh * (D * D);
@@ -2766,6 +2804,17 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     }
     if constexpr (!ROWS)
         if (fm) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true, NB, NB, WIDE>>(grid, smem, p, stream);
+    if (p.r_totals) {
+        if constexpr (D == 128 && std::is_same<T, __bf16>::value) {
+            constexpr int smem_r = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
+            static_assert(smem_r <= 160 * 1024, "two sets of four tiles and the state must fit the LDS of a CU");
+            if (!p.r_q || p.n_seg < 3 || p.total_out || p.entry_out || p.denom || p.dn || fm) return hipErrorInvalidValue;
+            if (p.wqk <= 64 && p.wv > 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 4, WIDE, ROWS, true>>(grid, smem_r, p, stream);
+            if (p.wqk <= 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 2, 2, WIDE, ROWS, true>>(grid, smem_r, p, stream);
+            if (p.wv > 64) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 4, WIDE, ROWS, true>>(grid, smem_r, p, stream);
+        }
+        return hipErrorNotSupported;
+    }
     if constexpr (D == 128) {
         // operands of at most 64 true columns on a side (the halves of a wide q / k, a narrow v): the kernels that
         // leave out the blocks of padding, which the states in memory may not hold either
