@@ -404,8 +404,9 @@ struct WalkPlan {
 //   182.9 / 190.1.
 //   A wide q / k against a v of up to 128: two states to add up, and the walks are held to seven.  256 / 64, B H 64, N 4096 (4)
 //   320 / 313 (kernels); it would pay up to fifteen: B H 32, N 2048 (8) 104.0 / 95.5, B H 20, N 4096 (11) 162.8 / 155.4.
-//   The polynomial map, of 58 KiB a state: where adding them up costs more than a launch.
-constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 7, kSumOnLoadPoly = 8;
+//   The polynomial map, 41 KiB a state, forward + backward (forward alone): B H 20, N 4096 (11 segments) 136.1 / 129.9 us (47.1 /
+//   43.7); B H 16, N 4096 (16) 84.1 / 83.3 (32.5 / 27.2); B H 10, N 2000 (16) 59.2 / 53.4; B H 8, N 8192 (32) 83.8 / 94.6.
+constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 7, kSumOnLoadPoly = 20;
 
 // `parts`: workgroups per segment (a launch that does several column halves at a time).
 WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false, int64_t parts = 1) {

@@ -305,6 +305,41 @@ struct PolyState {
                 if (NORM) ex[u] += *reinterpret_cast<const f32x4 *>(s + PolyFeatures::kF * PolyFeatures::kV + 16 * own[u] + 4 * kq);
             }
     }
+    // += the states `lo` .. `hi` - 1 at `s` in their order, the loads of three in flight together (one at a time is a memory latency
+    // per segment as a walk starts)
+    template <bool NORM>
+    __device__ __forceinline__ void add_range(const float *s, int lo, int hi, int lane) {
+        const int l16 = lane & 15, kq = lane >> 4;
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            if (own[u] < 0) continue;
+#pragma unroll 1
+            for (int f0 = lo; f0 < hi; f0 += 3) {
+                float t[3][4][4];
+                f32x4 e[3];
+#pragma unroll
+                for (int g = 0; g < 3; ++g) {
+                    // (past the range: the last state once more, not added)
+                    const float *sf = s + (int64_t)(f0 + g < hi ? f0 + g : hi - 1) * PolyFeatures::kState;
+#pragma unroll
+                    for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+                        for (int v = 0; v < 4; ++v) t[g][cb][v] = sf[(16 * own[u] + 4 * kq + v) * PolyFeatures::kV + 16 * cb + l16];
+                    if (NORM) e[g] = *reinterpret_cast<const f32x4 *>(sf + PolyFeatures::kF * PolyFeatures::kV + 16 * own[u] + 4 * kq);
+                }
+                walk_all_requested();
+#pragma unroll
+                for (int g = 0; g < 3; ++g)
+                    if (f0 + g < hi) {
+#pragma unroll
+                        for (int cb = 0; cb < 4; ++cb)
+#pragma unroll
+                            for (int v = 0; v < 4; ++v) st[u][cb][v] += t[g][cb][v];
+                        if (NORM) ex[u] += e[g];
+                    }
+            }
+        }
+    }
     template <bool NORM>
     __device__ __forceinline__ void store(float *s, int lane) const {
         const int l16 = lane & 15, kq = lane >> 4;
@@ -678,9 +713,7 @@ __device__ __forceinline__ void poly_entry(const PolyWalkParams &p, const PolySl
         s.template add<NORM>(base + (int64_t)sl.seg * PolyFeatures::kState, lane);
         return;
     }
-    const int lo = reverse ? sl.seg + 1 : 0, hi = reverse ? p.n_seg : sl.seg;
-#pragma unroll 1
-    for (int f = lo; f < hi; ++f) s.template add<NORM>(base + (int64_t)f * PolyFeatures::kState, lane);
+    s.template add_range<NORM>(base, reverse ? sl.seg + 1 : 0, reverse ? p.n_seg : sl.seg, lane);
 }
 
 template <typename T, bool NORM>

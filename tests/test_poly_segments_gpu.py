@@ -13,8 +13,9 @@ COEF, EPS = (0.25, -0.5, 0.75), 1e-5
 
 
 # (B H, N): 256 workgroups at a time, chunks of 128 rows -> segments x chunks
-@pytest.mark.parametrize("bh,n,r", [(64, 1536, 16), (100, 700, 16), (20, 3300, 8), (33, 1700, 16), (128, 500, 16)],
-                         ids=["4x3", "2x3", "9x3, scanned", "7x2", "2x2"])
+@pytest.mark.parametrize("bh,n,r", [(64, 1536, 16), (100, 700, 16), (20, 3300, 8), (33, 1700, 16), (128, 500, 16),
+                                     (12, 2500, 16), (10, 5500, 8)],
+                         ids=["4x3", "2x3", "9x3", "7x2", "2x2", "20x1", "22x2, scanned"])
 @pytest.mark.parametrize("normalise", [False, True])
 def test_segments_of_several_chunks(bh, n, r, normalise, gpu_device):
     gen = torch.Generator(device=gpu_device).manual_seed(n)
