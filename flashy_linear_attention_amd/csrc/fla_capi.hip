@@ -406,7 +406,7 @@ struct WalkPlan {
 //   320 / 313 (kernels); it would pay up to fifteen: B H 32, N 2048 (8) 104.0 / 95.5, B H 20, N 4096 (11) 162.8 / 155.4.
 //   The polynomial map, 41 KiB a state, forward + backward (forward alone): B H 20, N 4096 (11 segments) 136.1 / 129.9 us (47.1 /
 //   43.7); B H 16, N 4096 (16) 84.1 / 83.3 (32.5 / 27.2); B H 10, N 2000 (16) 59.2 / 53.4; B H 8, N 8192 (32) 83.8 / 94.6.
-constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 7, kSumOnLoadPoly = 20;
+constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 7, kSumOnLoadPoly = 20, kSumOnLoadWorkspace = 12;
 
 // `parts`: workgroups per segment (a launch that does several column halves at a time).
 WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false, int64_t parts = 1) {
@@ -1016,9 +1016,10 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         const bool in_state = state_out && wp.split;
         // D = 128, a few segments more than two: the totals go to the workspace, the walk adds them up itself as it starts
         // and writes the entry states it formed to state_out -- no scan launch
-        // (with a feature map or the normaliser a caller may have brought a state buffer and no workspace: then a scan in the former)
+        // (a caller may have brought a state buffer and no workspace: then a scan in the former -- but for the plain operator up to
+        // kSumOnLoadWorkspace segments, which asks for its workspace)
         const bool has_work = workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= wp.work_bytes;
-        const bool sum_on_load = wp.split && sums_on_load(wp) && ((!fmap && !nx) || !in_state || has_work);
+        const bool sum_on_load = wp.split && sums_on_load(wp) && (!in_state || has_work || (!fmap && !nx && wp.n_seg <= kSumOnLoadWorkspace));
         if (need_totals && (!in_state || sum_on_load) && !has_work) return FLA_ERR_WORKSPACE;
         if (state_out && reinterpret_cast<uintptr_t>(state_out) % 16 != 0) return FLA_ERR_WORKSPACE;
         hipStream_t s = static_cast<hipStream_t>(stream);

@@ -2,10 +2,12 @@
 128 columns and with both sides above 128, 7 with a wide q / k alone, 40 up to 64): both passes, with forward's state and
 without, against the fp32 oracle (``-m gpu``)."""
 
+import ctypes
+
 import pytest
 import torch
 
-from flashy_linear_attention_amd import LinearAttentionAuto, LinearAttentionSmallVHD
+from flashy_linear_attention_amd import LinearAttentionAuto, LinearAttentionSmallVHD, _lib
 from flashy_linear_attention_amd.chunked import linear_attention_chunked_bwd, linear_attention_chunked_fwd
 from flashy_linear_attention_amd.normalised import linear_attention_normalised_fwd
 
@@ -51,3 +53,19 @@ def test_normalised_forward(h, n, d, gpu_device):
     qd, kd = q.double(), k.double()
     want = (torch.tril(qd @ kd.transpose(-1, -2)) @ v.double()) / ((qd * kd.cumsum(-2)).sum(-1, keepdim=True) + 1e-5)
     assert_close("out", linear_attention_normalised_fwd(q, k, v, 1e-5, True)[0], want.float())
+
+
+@pytest.mark.parametrize("h,n,accepted", [(16, 16 * 64, True), (20, 12 * 64, False), (10, 24 * 64, True)])
+def test_a_state_buffer_and_no_workspace(h, n, accepted, gpu_device):
+    """From 13 segments on a forward with a state buffer needs no workspace: the entry states are scanned in the former."""
+    q, k, v, _ = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, 128, 128, torch.bfloat16, seed=n))
+    want, state = linear_attention_chunked_fwd(q, k, v, want_state=True)
+    out, mine, valid = torch.empty_like(want), torch.empty_like(state), ctypes.c_int32(0)
+    st = _lib.strides_arg
+    rc = _lib.load().fla_linear_attn_chunked_fwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), 1, h, n, 128, 128, st(q), st(k), st(v), st(out), _lib.FLA_DTYPE_BF16,
+        mine.data_ptr(), ctypes.byref(valid), None, 0, torch.cuda.current_stream().cuda_stream)
+    assert (rc == 0) == accepted
+    if accepted:
+        assert valid.value == 1
+        assert_close("O", out, want.float())
