@@ -1047,18 +1047,18 @@ __device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int 
         f32x16 t[GROUP][W::NBW];
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
-            const int f = f0 + u < f_hi ? f0 + u : f_hi - 1;  // (past the range: the last state once more, not added)
+            const int f = f0 + u < f_hi ? f0 + u : f_hi - 1;  // (past the range: the last state once more, not added -- nor times zero: it may be infinite)
             walk_read_frags<D, B>(buf + (int64_t)f * (D * D), wave, lane, t[u]);
         }
         walk_all_requested();
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
-            const float keep = f0 + u < f_hi ? 1.f : 0.f;
+            if (f0 + u >= f_hi) continue;
 #pragma unroll
             for (int i = 0; i < B::SLOTS; ++i)
                 if (B::valid(wave, i)) {
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) st[i][v] += keep * t[u][i][v];
+                    for (int v = 0; v < 16; ++v) st[i][v] += t[u][i][v];
                 }
         }
     }
@@ -1081,7 +1081,7 @@ __device__ __forceinline__ void walk_sum_two(const float *a, const float *b, int
         f32x16 ta[GROUP][W::NBW], tb[GROUP][W::NBW];
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
-            // (past the range: the last state once more, not added)
+            // (past the range: the last state once more, not added -- nor times zero: it may be infinite)
             const int f = f0 + u < f_hi ? f0 + u : f_hi - 1;
             walk_read_frags<D, B>(a + (int64_t)f * E, wave, lane, ta[u]);
             walk_read_frags<D, B>(b + (int64_t)f * E, wave, lane, tb[u]);
@@ -1089,12 +1089,12 @@ __device__ __forceinline__ void walk_sum_two(const float *a, const float *b, int
         walk_all_requested();
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
-            const float keep = f0 + u < f_hi ? 1.f : 0.f;
+            if (f0 + u >= f_hi) continue;
 #pragma unroll
             for (int i = 0; i < B::SLOTS; ++i)
                 if (B::valid(wave, i)) {
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) st_a[i][v] += keep * ta[u][i][v], st_b[i][v] += keep * tb[u][i][v];
+                    for (int v = 0; v < 16; ++v) st_a[i][v] += ta[u][i][v], st_b[i][v] += tb[u][i][v];
                 }
         }
     }

@@ -69,3 +69,22 @@ def test_a_state_buffer_and_no_workspace(h, n, accepted, gpu_device):
     if accepted:
         assert valid.value == 1
         assert_close("O", out, want.float())
+
+
+# numbers of segments whose sums leave part of a group over
+@pytest.mark.parametrize("h,n,dqk,dv", [(12, 20 * 64, 128, 128), (12, 40 * 128, 64, 64), (36, 7 * 64, 256, 64), (6, 20 * 64, 256, 256)])
+def test_an_infinite_value_stays_infinite(h, n, dqk, dv, gpu_device):
+    """With q, k > 0 a value (an upstream gradient) of +inf gives +inf in its column of every row after (before) it, not NaN, and
+    nothing in the other columns."""
+    q, k, v, do = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, dqk, dv, torch.bfloat16, seed=n + dqk))
+    want, state = linear_attention_chunked_fwd(q, k, v, want_state=True)
+    want_dv = linear_attention_chunked_bwd(do, q, k, v, state)[2]
+    v_inf, do_inf = v.clone(), do.clone()
+    v_inf[:, :, 3, 1], do_inf[:, :, n - 2, 1] = float("inf"), float("inf")
+    # (a row's own chunk, of up to 128 rows, multiplies masked scores of zero by it)
+    got, after, before = linear_attention_chunked_fwd(q, k, v_inf, want_state=False), slice(128, n), slice(0, n - 128)
+    got_dv = linear_attention_chunked_bwd(do_inf, q, k, v, state)[2]
+    for x, x_want, rows in ((got, want, after), (got_dv, want_dv, before)):
+        assert bool((x[:, :, rows, 1] == float("inf")).all())
+        x[:, :, :, 1] = x_want[:, :, :, 1] = 0
+        assert torch.equal(x, x_want)
