@@ -1015,10 +1015,11 @@ __device__ __forceinline__ void walk_load_state(const float *init, bool transpos
 //     the totals kernel and the walk, whose launch costs more than it computes on plans this small
 //     (B H = 16, N = 1024, D = 64, forward + backward: 40.7 -> 32.8 us, bound by its six -> four launches).  D = 64, scan
 //     against sums on load: 32 segments B H 16 N 4096 84.7 / 77.1 us, N 32768 232.8 / 227.6, B H 12 N 8192 81.9 / 75.0, forward
-//     alone B H 12 N 4096 24.2 / 21.5, B H 10 N 8192 25.2 / 25.7; 64 segments (B H 8 N 8192) forward alone 23.3 / 24.9;
+//     alone B H 12 N 4096 24.2 / 21.5, B H 10 N 8192 25.2 / 25.7; 64 segments (B H 8 N 8192) forward alone 23.3 / 24.9; beyond 32 forward alone B H 12 N 19200
+//     (40 columns) 40.8 / 44.3.  D = 32, whose scan is a quarter of that: 32 segments B H 16 N 8503 forward alone 26.2 / 28.3;
 //   * more segments: the slots hold the entry states themselves (walk_scan_kernel).
 // (At D = 128 a forward walk then writes the entry states it formed, for backward.)
-__host__ __device__ constexpr int walk_sum_on_load_max(int D) { return D <= 64 ? 40 : 0; }
+__host__ __device__ constexpr int walk_sum_on_load_max(int D) { return D <= 32 ? 16 : D <= 64 ? 32 : 0; }
 __host__ __device__ constexpr bool walk_entries_are_totals(int D, int n_seg) {
     return n_seg >= 3 && n_seg <= walk_sum_on_load_max(D);
 }

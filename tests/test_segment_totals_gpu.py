@@ -1,5 +1,5 @@
 """Plans whose walks add up the segments' totals as they start, around the numbers of segments where a scan takes over (20 at
-128 columns and with both sides above 128, 7 with a wide q / k alone, 40 up to 64): both passes, with forward's state and
+128 columns and with both sides above 128, 7 with a wide q / k alone, 32 at 64, 16 at 32): both passes, with forward's state and
 without, against the fp32 oracle (``-m gpu``)."""
 
 import ctypes
@@ -23,6 +23,7 @@ pytestmark = pytest.mark.gpu
     (64, 1003, 96, 96, torch.float16), (50, 5 * 64 - 1, 128, 128, torch.bfloat16), (12, 1270, 128, 64, torch.bfloat16),
     (6, 20 * 64 - 3, 256, 256, torch.bfloat16), (6, 21 * 64 - 3, 160, 256, torch.bfloat16), (32, 5 * 64, 256, 160, torch.float16),
     (36, 7 * 64 - 7, 256, 64, torch.bfloat16), (32, 8 * 64 - 7, 256, 64, torch.bfloat16), (16, 900, 192, 128, torch.float16),
+    (16, 32 * 128 - 9, 64, 64, torch.bfloat16), (15, 33 * 128 - 9, 64, 64, torch.bfloat16), (30, 17 * 128 - 9, 32, 32, torch.bfloat16),
     (12, 40 * 128 - 9, 64, 64, torch.bfloat16), (12, 41 * 128 - 9, 64, 64, torch.float16), (51, 9 * 128 + 1, 32, 32, torch.bfloat16),
 ])
 def test_both_passes(h, n, dqk, dv, dtype, gpu_device):
@@ -72,7 +73,7 @@ def test_a_state_buffer_and_no_workspace(h, n, accepted, gpu_device):
 
 
 # numbers of segments whose sums leave part of a group over
-@pytest.mark.parametrize("h,n,dqk,dv", [(12, 20 * 64, 128, 128), (12, 40 * 128, 64, 64), (36, 7 * 64, 256, 64), (6, 20 * 64, 256, 256)])
+@pytest.mark.parametrize("h,n,dqk,dv", [(12, 20 * 64, 128, 128), (12, 40 * 128, 64, 64), (16, 32 * 128, 64, 64), (36, 7 * 64, 256, 64), (6, 20 * 64, 256, 256)])
 def test_an_infinite_value_stays_infinite(h, n, dqk, dv, gpu_device):
     """With q, k > 0 a value (an upstream gradient) of +inf gives +inf in its column of every row after (before) it, not NaN, and
     nothing in the other columns."""
