@@ -36,6 +36,20 @@ def test_both_passes(h, n, dqk, dv, dtype, gpu_device):
             assert_close(name, got, want)
 
 
+# one chunk of 128 (D = 128: 64) rows a segment, and groups of eight states (six at 128 over 64 columns) that are full, begun and left over
+@pytest.mark.parametrize("segments", [3, 6, 7, 8, 9, 11, 13, 16])
+@pytest.mark.parametrize("dqk,dv", [(32, 32), (64, 64), (128, 64)])
+def test_groups_of_states(segments, dqk, dv, gpu_device):
+    rows, resident = (128, 512) if dqk <= 64 else (64, 256)
+    h, n = resident // segments, segments * rows - 5
+    q, k, v, do = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, dqk, dv, torch.bfloat16, seed=n + dqk))
+    want_o, want_g = gpu_fp32_reference(q, k, v, do, True)
+    out, state = linear_attention_chunked_fwd(q, k, v, want_state=True)
+    assert_close("O", out, want_o)
+    for name, got, want in zip(("dQ", "dK", "dV"), linear_attention_chunked_bwd(do, q, k, v, state), want_g):
+        assert_close(name, got, want)
+
+
 @pytest.mark.parametrize("h,n,dqk,dv", [(24, 1500, 80, 80), (36, 7 * 64, 256, 64), (36, 448, 153, 64), (32, 512, 256, 128)])
 def test_operators_that_keep_dq_causal(h, n, dqk, dv, gpu_device):
     q, k, v, do = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, dqk, dv, torch.bfloat16, seed=n + dqk))
