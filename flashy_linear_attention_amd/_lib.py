@@ -54,6 +54,7 @@ SIGNATURES = {
                                         + [ctypes.c_int, ctypes.c_int, ctypes.c_int, _ptr, _ptr, _i64, _ptr], ctypes.c_int),
     "fla_linear_attn_chunked_fwd_static": ([_ptr] * 4 + [_i64] * 5 + [_strides] * 4 + [ctypes.c_int, _ptr], ctypes.c_int),
     "fla_linear_attn_chunked_fwd_workspace_bytes": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int64),
+    "fla_linear_attn_chunked_grads_f32": ([_i64] * 5 + [ctypes.c_int] * 2, ctypes.c_int),
     "fla_linear_attn_chunked_state_operands": ([_i64] * 5 + [ctypes.POINTER(ctypes.c_int64)] * 2, ctypes.c_int),
     "fla_linear_attn_chunked_bwd": ([_ptr] * 7 + [_i64] * 5 + [_strides] * 7 + [ctypes.c_int, _ptr, _ptr, _i64, _ptr],
                                     ctypes.c_int),

@@ -1089,18 +1089,23 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
     return FLA_OK;
 }
 
-// whether walks that can store their results in fp32 (FLA_GRADS_F32) take a backward; `plain`: without feature map and normaliser
+// whether walks that can store their results in fp32 (FLA_GRADS_F32) take a backward of these sizes; `plain`: without feature map and
+// normaliser
+bool wide_grads_sizes(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool plain, bool with_state) {
+    if (dqk % 8 || dv % 8 || dv > 128) return false;
+    if (dqk > 128) return plain && dv <= 64 && wide_plan(B, H, N, dqk, dv).ok;
+    const WalkPlan wp = walk_plan(B, H, N, dqk, dv, plain);
+    return wp.ok && (wp.split || with_state) && (states_shareable(dqk, dv, N) || pad_index(dqk) != pad_index(dv));
+}
+
+// ... and of these operands
 bool wide_grads_walk(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk, const View &dvv,
                      int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype, const void *state_in, bool plain) {
-    if (dtype != FLA_DTYPE_BF16) return false;
+    if (dtype != FLA_DTYPE_BF16 || !wide_grads_sizes(B, H, N, dqk, dv, plain, state_in != nullptr)) return false;
     // (a (b, h) of a result stays within the 1 GiB that a descriptor's offsets reach, as 16-bit operands do)
     for (const View *t : {&dq, &dk, &dvv})
         if (N * t->strides[2] * 4 > fla::kMaxFastExtent) return false;
-    if (dqk > 128)
-        return plain && dv <= 64 && wide_plan(B, H, N, dqk, dv).ok && wide_fast_path(q, k, v, go, B, H, N, dqk, dv) &&
-               wide_fast_path(dq, dk, dvv, dvv, B, H, N, dqk, dv);
-    const WalkPlan wp = walk_plan(B, H, N, dqk, dv, plain);
-    if (!wp.ok || !(wp.split || state_in) || (!states_shareable(dqk, dv, N) && pad_index(dqk) == pad_index(dv))) return false;
+    if (dqk > 128) return wide_fast_path(q, k, v, go, B, H, N, dqk, dv) && wide_fast_path(dq, dk, dvv, dvv, B, H, N, dqk, dv);
     return fla::fast_path_ok(make_params(go, v, k, dq, B, H, N, dv, dqk, 0)) &&
            fla::fast_path_ok(make_params(k, q, go, dvv, B, H, N, dqk, dv, 1)) &&
            fla::fast_path_ok(make_params(v, go, q, dk, B, H, N, dv, dqk, 1));
@@ -1479,7 +1484,7 @@ int plain_chunked_backward(const View &go, const View &q, const View &k, const V
     if (int rc = check_common(B, H, N, dtype)) return rc;
     if (dqk < 1 || dqk > 256) return FLA_ERR_HEAD_DIM;
     if (dv < 1 || dv > 256) return FLA_ERR_V_HEAD_DIM;
-    if (wide_out && (dv > 128 || dqk % 8 || dv % 8)) return FLA_ERR_UNSUPPORTED;
+    if (wide_out && (dv > 128 || dqk % 8 || dv % 8)) return FLA_ERR_UNSUPPORTED;  // (wide_grads_sizes: before any copy)
     // (causal, D_v above 128: product by product with the states of 256-row chunks in memory, each sum rounded once and no state
     // by subtraction, where the copies would run as column halves of v)
     if (const PackPlan p = pack_plan(B, H, N, dqk, dv); p.ok && !(causal && dv > 128))
@@ -2240,6 +2245,11 @@ int fla_linear_attn_chunked_state_operands(int64_t B, int64_t H, int64_t N, int6
         offsets[i] = copied ? p.inner_state + i * p.q_bytes : -1, pitches[i] = i < 2 ? p.wq : p.wv;
     }
     return 1;
+}
+
+int fla_linear_attn_chunked_grads_f32(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int plain, int with_state) {
+    if (B < 1 || H < 1 || N < 1 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
+    return wide_grads_sizes(B, H, N, D_qk, D_v, plain != 0, with_state != 0);
 }
 
 int fla_linear_attn_chunked_fwd(const void *q, const void *k, const void *v, void *o, int64_t B, int64_t H, int64_t N,

@@ -58,6 +58,7 @@ struct Call {
           dqk(q.size(3)), dv(v.size(3)), dtype(dtype_code(q.scalar_type())) {}
     Tensor rows(int64_t width) const { return at::empty({b, h, n, width}, like); }
     Tensor row_floats() const { return at::empty({b, h, n}, like.dtype(at::kFloat)); }
+    bool grads_f32(bool plain, bool state) const { return fla_linear_attn_chunked_grads_f32(b, h, n, dqk, dv, plain, state) != 0; }
     Tensor bytes(int64_t count) const { return count ? at::empty({count}, like.dtype(at::kByte)) : Tensor(); }
 };
 
@@ -121,10 +122,12 @@ struct Casts {
 };
 
 // A chunk-wise backward: allocates the gradients and makes `call(dq, dk, dv, dtype)`.  For inputs that all came in fp32
-// (`widened` == 7) the gradients are stored in fp32 where the library's kernels can do so.
+// (`widened` == 7) the gradients are stored in fp32 where the library's kernels can do so; `sizes`: they can for these sizes (what is
+// refused then is an operand's alignment, and asked for again in 16 bits.  To find out by a refusal for every shape cost the shapes
+// without such a kernel 2 us of the host, three allocations and a call: B 1 H 2 N 100 D 64 51.5 -> 53.9 us).
 template <typename Backward>
-variable_list chunked_gradients(const Call &c, int64_t widened, Backward &&call) {
-    for (bool wide = widened == 7 && c.dtype == FLA_DTYPE_BF16;; wide = false) {
+variable_list chunked_gradients(const Call &c, int64_t widened, bool sizes, Backward &&call) {
+    for (bool wide = widened == 7 && sizes && c.dtype == FLA_DTYPE_BF16;; wide = false) {
         const at::TensorOptions as = wide ? c.like.dtype(at::kFloat) : c.like;
         const Tensor dq = at::empty({c.b, c.h, c.n, c.dqk}, as), dk = at::empty({c.b, c.h, c.n, c.dqk}, as),
                      dv = at::empty({c.b, c.h, c.n, c.dv}, as);
@@ -193,9 +196,7 @@ variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_,
     const Call c(q, v);
     if (ev == kChunked || ev == kChosen) {
         const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        // (what is refused whatever the operands is not tried)
-        const bool may = c.dv <= (c.dqk <= 128 ? 128 : 64) && c.dqk % 8 == 0 && c.dv % 8 == 0;
-        return chunked_gradients(c, may ? widened : 0, [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
+        return chunked_gradients(c, widened, c.grads_f32(true, state.defined()), [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
             return (ev == kChosen ? fla_linear_attn_chunked_bwd_causal : fla_linear_attn_chunked_bwd)(
                 ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go), str(q), str(k),
                 str(v), str(dq), str(dk), str(dv), dtype, ptr(state), ptr(work), size_of(work), c.stream);
@@ -321,8 +322,7 @@ variable_list mapped_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, 
     const float *n = opt.normalise ? denom.data_ptr<float>() : nullptr;
     const Tensor work = c.bytes(opt.normalise ? fla_normalised_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv, opt.chunked)
                                               : fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-    // (not chunk-wise: FLA_GRADS_F32 is refused before anything is launched)
-    return chunked_gradients(c, opt.chunked || !opt.normalise ? widened : 0,
+    return chunked_gradients(c, widened, (opt.chunked || !opt.normalise) && c.grads_f32(false, state.defined()),
                              [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
         if (!opt.normalise)
             return fla_feature_attn_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv,
@@ -409,7 +409,7 @@ variable_list poly_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, co
     const int64_t *os = o.defined() ? str(o) : nullptr;
     if (state.defined()) {
         const Tensor work = c.bytes(fla_poly_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
-        return chunked_gradients(c, widened, [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
+        return chunked_gradients(c, widened, true, [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
             return fla_poly_attn_chunked_bwd(ptr(go), ptr(q), ptr(k), ptr(v), ptr(o), n, ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n,
                                              c.dqk, c.dv, str(go), str(q), str(k), str(v), os, str(dq), str(dk), str(dv), p.c,
                                              dtype, ptr(state), ptr(work), size_of(work), c.stream);

@@ -219,6 +219,10 @@ int64_t fla_linear_attn_chunked_fwd_workspace_bytes(int64_t B, int64_t H, int64_
  * go.  0: none. */
 int fla_linear_attn_chunked_state_operands(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int64_t *offsets,
                                            int64_t *pitches);
+/* 1 where backward stores its gradients in fp32 (FLA_GRADS_F32) for bf16 operands of these sizes whose rows are 16-byte aligned
+ * (and a (b, h) of a gradient no longer than 1 GiB), 0 where it refuses the flag.  `plain`: fla_linear_attn_chunked_bwd(_causal); 0:
+ * the normalised and feature-map operators' chunk-wise backward.  `with_state`: given forward's state. */
+int fla_linear_attn_chunked_grads_f32(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int plain, int with_state);
 int fla_linear_attn_chunked_fwd(const void *q, const void *k, const void *v, void *o,
                                 int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v,
                                 const int64_t *q_strides, const int64_t *k_strides,

@@ -102,8 +102,8 @@ class Tensor:
 
 
 def make_tensor(arena: Arena, name: str, b: int, h: int, n: int, w: int, layout: str = "contiguous",
-                misalign: int = 0) -> Tensor:
-    """(B, H, N, W) 16-bit tensor: contiguous, stored as (B, N, H, W) ("bnhd"), with padded rows
+                misalign: int = 0, size: int = 2) -> Tensor:
+    """(B, H, N, W) tensor of elements of `size` bytes: contiguous, stored as (B, N, H, W) ("bnhd"), with padded rows
     ("padded": row stride W + 8), with an odd row stride ("odd": W + 1, rows not 16-byte aligned), or
     expanded along the sequence ("expanded": one stored row per head, row stride 0)."""
     if layout == "contiguous":
@@ -119,7 +119,7 @@ def make_tensor(arena: Arena, name: str, b: int, h: int, n: int, w: int, layout:
     else:
         raise ValueError(layout)
     last = (b - 1) * st[0] + (h - 1) * st[1] + (n - 1) * st[2] + w if min(b, h, n) > 0 else 0
-    ptr = arena.alloc(name, 2 * last, misalign)
+    ptr = arena.alloc(name, size * last, misalign)
     return Tensor(ptr, st, (b, h, n, w))
 
 

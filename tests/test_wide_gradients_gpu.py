@@ -78,3 +78,26 @@ def test_what_the_flag_is_taken_for(dtype, n, d, causal, status, gpu_device):
     assert got == status
     torch.cuda.synchronize()
     assert all(bool((t == 7.0).all()) == (status != 0) for t in grads)
+
+
+@pytest.mark.parametrize("op,b,h,n,dqk,dv,stored", [
+    ("chunked", 1, 2, 100, 64, 64, False), ("auto", 1, 8, 249, 32, 32, False), ("normalised", 1, 2, 300, 256, 64, False),
+    ("feature", 1, 2, 100, 64, 64, False), ("feature_normalised", 1, 2, 200, 128, 128, False), ("chunked", 1, 3, 700, 256, 128, False),
+    ("chunked", 1, 2, 300, 64, 64, True), ("normalised", 1, 5, 700, 64, 64, True), ("feature", 1, 3, 400, 128, 128, True),
+    ("feature_normalised", 1, 3, 515, 48, 48, True), ("smallv", 1, 8, 4096, 256, 64, True), ("poly", 1, 3, 515, 16, 40, True),
+])
+def test_gradients_are_allocated_once(op, b, h, n, dqk, dv, stored, gpu_device):
+    """Beside what a 16-bit backward allocates, one of fp32 operands allocates nothing where the kernels store fp32, and the
+    three converted gradients elsewhere -- no second set for a call that is refused."""
+    def allocations(cast):
+        ins = [torch.rand(b, h, n, d, device=gpu_device) for d in (dqk, dqk, dv)]
+        ins = [(t if cast else t.bfloat16()).requires_grad_(True) for t in ins]
+        do = torch.rand(b, h, n, dv, device=gpu_device).bfloat16()
+        with torch.autocast("cuda", dtype=torch.bfloat16, enabled=cast):
+            out = OPS[op](*ins)
+        before = torch.cuda.memory_stats(gpu_device)["allocation.all.allocated"]
+        grads = torch.autograd.grad(out, ins, do)
+        assert all(g.dtype == t.dtype for g, t in zip(grads, ins))
+        return torch.cuda.memory_stats(gpu_device)["allocation.all.allocated"] - before
+    allocations(False), allocations(True)
+    assert allocations(True) - allocations(False) == (0 if stored else 3)
