@@ -53,6 +53,10 @@ FLA_FIELD(vec_q) FLA_FIELD(vec_k) FLA_FIELD(vec_a) FLA_FIELD(vec_b) FLA_FIELD(ve
 FLA_FIELD(vec_dk) FLA_FIELD(eps) FLA_FIELD(fmap) FLA_FIELD(only_dk)
 FLA_FIELDS_END
 
+FLA_FIELDS_BEGIN(WalkRowsOut)
+FLA_FIELD(ptr) FLA_FIELD(s_b) FLA_FIELD(s_h) FLA_FIELD(s_n) FLA_FIELD(width)
+FLA_FIELDS_END
+
 FLA_FIELDS_BEGIN(WalkParams)
 FLA_FIELD(q) FLA_FIELD(k) FLA_FIELD(v) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(dq) FLA_FIELD(dk) FLA_FIELD(dv)
 FLA_FIELD(qs_b) FLA_FIELD(qs_h) FLA_FIELD(qs_n) FLA_FIELD(ks_b) FLA_FIELD(ks_h) FLA_FIELD(ks_n)
@@ -66,6 +70,10 @@ FLA_FIELD(denom) FLA_FIELD(eps) FLA_FIELD(zc) FLA_FIELD(dn) FLA_FIELD(rc) FLA_FI
 FLA_FIELD(xtotal) FLA_FIELD(accumulate)
     FLA_FIELD(wqk2) FLA_FIELD(init2) FLA_FIELD(total_out2) FLA_FIELD(xinit2) FLA_FIELD(xtotal2)
     FLA_FIELD(init_is_totals) FLA_FIELD(entry_out) FLA_FIELD(entry_out2) FLA_FIELD(quad) FLA_FIELD(wv2) FLA_FIELD(vsum) FLA_FIELD(zc_out)
+FLA_FIELD(wide_out) FLA_FIELD(any_rows) FLA_FIELD(r_q) FLA_FIELD(rs_b) FLA_FIELD(rs_h) FLA_FIELD(rs_n) FLA_FIELD(r_frags)
+FLA_FIELD(r_totals)
+    trace_fields(r, arg, pre + "rows_o.", p.rows_o), trace_fields(r, arg, pre + "rows_dq.", p.rows_dq);
+    trace_fields(r, arg, pre + "rows_dk.", p.rows_dk), trace_fields(r, arg, pre + "rows_dv.", p.rows_dv);
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(WalkTotalsParams)
@@ -73,7 +81,7 @@ FLA_FIELD(y) FLA_FIELD(z) FLA_FIELD(ys_b) FLA_FIELD(ys_h) FLA_FIELD(ys_n) FLA_FI
 FLA_FIELD(zs_n) FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(dy) FLA_FIELD(dz) FLA_FIELD(n_chunks)
 FLA_FIELD(seg_chunks) FLA_FIELD(n_seg) FLA_FIELD(seg_lo) FLA_FIELD(seg_hi) FLA_FIELD(totals) FLA_FIELD(direct)
 FLA_FIELD(map_y) FLA_FIELD(ymap_out) FLA_FIELD(yo_b) FLA_FIELD(yo_h) FLA_FIELD(yo_n) FLA_FIELD(y2) FLA_FIELD(dy2)
-FLA_FIELD(totals2) FLA_FIELD(dz2) FLA_FIELD(z_narrow) FLA_FIELD(vsum)
+FLA_FIELD(totals2) FLA_FIELD(dz2) FLA_FIELD(z_narrow) FLA_FIELD(vsum) FLA_FIELD(frags)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(WalkVecParams)
@@ -85,7 +93,7 @@ FLA_FIELDS_BEGIN(WalkGradParams)
 FLA_FIELD(q) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(qs_b) FLA_FIELD(qs_h) FLA_FIELD(qs_n) FLA_FIELD(gs_b) FLA_FIELD(gs_h)
 FLA_FIELD(gs_n) FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n) FLA_FIELD(denom) FLA_FIELD(dout) FLA_FIELD(dn) FLA_FIELD(H)
 FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(wqk) FLA_FIELD(wv) FLA_FIELD(vec) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks)
-FLA_FIELD(n_seg) FLA_FIELD(totals) FLA_FIELD(rsum)
+FLA_FIELD(n_seg) FLA_FIELD(totals) FLA_FIELD(rsum) FLA_FIELD(frags)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(ChunkStateParams)
@@ -102,7 +110,11 @@ FLA_FIELDS_END
 FLA_FIELDS_BEGIN(PolyWalkParams)
 FLA_FIELD(q) FLA_FIELD(k) FLA_FIELD(v) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(out) FLA_FIELD(dq) FLA_FIELD(dk) FLA_FIELD(dv)
 FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(r) FLA_FIELD(wv) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks) FLA_FIELD(n_seg)
-FLA_FIELD(denom) FLA_FIELD(totals) FLA_FIELD(sum_entries) FLA_FIELD(entries)
+FLA_FIELD(denom) FLA_FIELD(totals) FLA_FIELD(sum_entries) FLA_FIELD(entries) FLA_FIELD(wide_out)
+FLA_FIELD(qs_b) FLA_FIELD(qs_h) FLA_FIELD(qs_n) FLA_FIELD(ks_b) FLA_FIELD(ks_h) FLA_FIELD(ks_n) FLA_FIELD(vs_b) FLA_FIELD(vs_h)
+FLA_FIELD(vs_n) FLA_FIELD(gs_b) FLA_FIELD(gs_h) FLA_FIELD(gs_n) FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n) FLA_FIELD(us_b)
+FLA_FIELD(us_h) FLA_FIELD(us_n) FLA_FIELD(dqs_b) FLA_FIELD(dqs_h) FLA_FIELD(dqs_n) FLA_FIELD(dks_b) FLA_FIELD(dks_h)
+FLA_FIELD(dks_n) FLA_FIELD(dvs_b) FLA_FIELD(dvs_h) FLA_FIELD(dvs_n)
 FLA_FIELDS_END
 
 #undef FLA_FIELDS_BEGIN

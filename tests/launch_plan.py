@@ -232,17 +232,19 @@ def check_launch_limits(l: Launch) -> None:
     gx, gy, gz = l.grid
     assert 1 <= gx <= 0x7fffffff, f"{l.kernel}: grid.x = {gx}"
     assert 1 <= gy <= 65535 and 1 <= gz <= 65535, f"{l.kernel}: grid.y, z = {gy}, {gz}"
-    assert l.block == 256, f"{l.kernel}: block = {l.block}"
+    eight_waves = l.kernel == "poly_totals_kernel" or l.kernel.startswith("poly_walk_")
+    assert l.block == (512 if eight_waves else 256), f"{l.kernel}: block = {l.block}"
     assert l.lds <= LDS_PER_CU, f"{l.kernel}: {l.lds} bytes of LDS"
     assert l.lds <= l.lds_limit, f"{l.kernel}: {l.lds} bytes of dynamic LDS, limit raised to {l.lds_limit} only"
 
 
-def tensor_extent(p: Dict, ptr: str, sb: str, sh: str, sn: str, H: int, BH: int, N: int, width: int) -> Tuple[int, int]:
-    """Byte range of a (B, H, N, width) tensor given by pointer and element strides in struct p."""
+def tensor_extent(p: Dict, ptr: str, sb: str, sh: str, sn: str, H: int, BH: int, N: int, width: int,
+                  size: int = 2) -> Tuple[int, int]:
+    """Byte range of a (B, H, N, width) tensor of elements of `size` bytes given by pointer and element strides in struct p."""
     B = BH // H
     lo = p[ptr]
     last = (B - 1) * p[sb] + (H - 1) * p[sh] + (N - 1) * p[sn] + width
-    return lo, lo + 2 * last
+    return lo, lo + size * last
 
 
 # ---------------------------------------------------------------------------------------------
@@ -320,6 +322,7 @@ class Stats:
     workgroups: int = 0
     lane_accesses: int = 0
     kernels: Dict[str, int] = field(default_factory=dict)
+    results: List[Tuple[int, int]] = field(default_factory=list)  # byte ranges that walks and copies write results to
 
 
 def _buffer_check(what: str, offsets, meant, num_records: int, size: int = 16) -> None:
@@ -759,15 +762,25 @@ def model_walk(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats) -> None:
     assert l.grid[0] == 8 * ((BH + 7) // 8) * n_seg
     resident = 256 if D > 64 else 512
     assert BH * n_seg <= max(resident, BH), f"{l.kernel}: {BH * n_seg} workgroups for {resident} resident"
-    for nm, ptr, sb, sh, sn, w in (("q", "q", "qs_b", "qs_h", "qs_n", p["wqk"]), ("k", "k", "ks_b", "ks_h", "ks_n", p["wqk"]),
-                                   ("v", "v", "vs_b", "vs_h", "vs_n", p["wv"]), ("go", "go", "gs_b", "gs_h", "gs_n", p["wv"]),
-                                   ("o", "o", "os_b", "os_h", "os_n", p["wv"]), ("dq", "dq", "dqs_b", "dqs_h", "dqs_n", p["wqk"]),
-                                   ("dk", "dk", "dks_b", "dks_h", "dks_n", p["wqk"]), ("dv", "dv", "dvs_b", "dvs_h", "dvs_n", p["wv"])):
+    # (pairs of column halves, grid y: a q / k of 128 + wqk2 columns, a v of 128 + wv2)
+    wqk = p["wqk"] + (p["wqk2"] if p["quad"] and l.kernel == "walk_bwd_rev_kernel" else 0)
+    wv = p["wv"] + (p["wv2"] if p["quad"] else 0)
+    for nm, ptr, sb, sh, sn, w in (("q", "q", "qs_b", "qs_h", "qs_n", wqk), ("k", "k", "ks_b", "ks_h", "ks_n", wqk),
+                                   ("v", "v", "vs_b", "vs_h", "vs_n", wv), ("go", "go", "gs_b", "gs_h", "gs_n", wv)):
         if p[ptr]:
             lo, hi = tensor_extent(p, ptr, sb, sh, sn, H, BH, N, w)
             arena.require(f"{l.kernel} {nm}", lo, hi)
             assert p[ptr] % 16 == 0 and w % 8 == 0 and p[sn] % 8 == 0
             assert N * p[sn] * 2 <= 0x3fffffff
+    model_walk_results(arena, l, p, wqk, wv, stats)
+    if p["r_totals"]:  # (dQ's walk adds up its segments' totals of Q^T dO: q's rows as wide as the result's)
+        assert l.kernel == "walk_fwd_kernel" and D == 128 and n_seg >= 3 and p["r_q"] % 16 == 0 and p["rs_n"] % 8 == 0
+        arena.require("q of the reverse walk's totals", *tensor_extent(p, "r_q", "rs_b", "rs_h", "rs_n", H, BH, N, p["wv"]))
+        assert N * p["rs_n"] * 2 <= 0x3fffffff
+        arena.require("the reverse walk's totals", p["r_totals"], p["r_totals"] + BH * n_seg * D * D * 4)
+        assert l.lds == 8 * 64 * 256 + 128 * 256, f"{l.kernel}: {l.lds} bytes of LDS for two sets of four tiles and a state"
+    else:
+        assert not p["r_q"]
     E = D * D * 4
     if p["init"]:
         arena.require("entry states", p["init"], p["init"] + BH * n_seg * E)
@@ -787,13 +800,48 @@ def model_walk(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats) -> None:
         arena.require("final states", p["total_out"], p["total_out"] + BH * E)
     if p["saved"]:
         arena.require("per-chunk states", p["saved"], p["saved"] + BH * n_chunks * D * D * 2)
-    for nm in ("zc", "rc"):
+    for nm, count in (("zc", n_chunks), ("zc_out", n_chunks), ("rc", n_seg), ("vsum", n_seg)):
         if p[nm]:
-            arena.require(nm, p[nm], p[nm] + BH * n_chunks * D * 4)
+            arena.require(nm, p[nm], p[nm] + BH * count * D * 4)
     for nm in ("denom", "dn"):
         if p[nm]:
-            arena.require(nm, p[nm], p[nm] + BH * N * 4)
+            # (the walk for dK and dV reads dn in whole groups of four rows)
+            past = -N % 4 if l.kernel == "walk_dkdv_kernel" else 0
+            arena.require(nm, p[nm], p[nm] + (BH * N + past) * 4)
     stats.workgroups += BH * n_seg
+
+
+# what each walk writes; dq of the wide reverse walk may be another walk's
+WALK_RESULTS = {"walk_fwd_kernel": ("o",), "walk_fwd_wide_kernel": ("o",), "walk_bwd_kernel": ("dq", "dk", "dv"),
+                "walk_dkdv_kernel": ("dk", "dv"), "walk_bwd_rev_kernel": ("dq", "dk", "dv"),
+                "walk_bwd_rev_wide_kernel": ("dk", "dv")}
+
+
+def model_walk_results(arena: Arena, l: Launch, p: Dict, wqk: int, wv: int, stats: Stats) -> None:
+    """Every result of a walk has a place, in one of two forms: 16-byte aligned rows of 16-bit elements (of floats, with
+    wide_out), bounded by a buffer descriptor of 32-bit offsets; or, with any_rows, rows of any alignment that are stored to
+    through plain pointers."""
+    H, BH, N = p["H"], p["BH"], p["N"]
+    size = 4 if p["wide_out"] else 2
+    for nm in ("o", "dq", "dk", "dv"):
+        w = wv if nm in ("o", "dv") else wqk
+        place, rows = p[nm], p["any_rows"] and p[f"rows_{nm}.ptr"]
+        assert not (place and rows), f"{l.kernel}: two places for {nm}"
+        if nm in WALK_RESULTS[l.kernel]:
+            assert place or rows, f"{l.kernel}: no place for {nm}"
+        if rows:
+            width = p[f"rows_{nm}.width"]
+            assert 1 <= width <= w and not p["wide_out"] and rows % 2 == 0
+            lo, hi = tensor_extent(p, *(f"rows_{nm}.{f}" for f in ("ptr", "s_b", "s_h", "s_n")), H, BH, N, width)
+        elif place:
+            pre = {"o": "os", "dq": "dqs", "dk": "dks", "dv": "dvs"}[nm]
+            lo, hi = tensor_extent(p, nm, f"{pre}_b", f"{pre}_h", f"{pre}_n", H, BH, N, w, size)
+            assert place % 16 == 0 and w % 8 == 0 and p[f"{pre}_n"] % 8 == 0
+            assert N * p[f"{pre}_n"] * size <= 0x3fffffff
+        else:
+            continue
+        arena.require(f"{l.kernel} {nm}", lo, hi)
+        stats.results.append((lo, hi))
 
 
 def model_walk_wide(arena: Arena, l: Launch, p: Dict, stats: Stats) -> None:
@@ -803,7 +851,7 @@ def model_walk_wide(arena: Arena, l: Launch, p: Dict, stats: Stats) -> None:
     assert p["wqk"] == 128 and 1 <= p["wqk2"] <= 128 and p["wqk2"] % 8 == 0 and not p["accumulate"]
     assert not p["init_transposed"] and not p["fmap"] and not p["denom"] and not p["dn"] and not p["saved"]
     if p["init_is_totals"]:  # (the walk adds up the segments' totals itself; what it forms goes to entry_out)
-        assert 3 <= p["n_seg"] <= 7 and p["init"]
+        assert p["n_seg"] >= 3 and p["init"] and p["init2"]
         if p["entry_out"]:
             assert l.kernel == "walk_fwd_wide_kernel"
             arena.require("entry_out", p["entry_out"], p["entry_out"] + p["BH"] * p["n_seg"] * E)
@@ -850,8 +898,109 @@ def model_walk_totals(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats, bo
     stats.workgroups += BH * n_seg
 
 
+def model_walk_grad_totals(arena: Arena, l: Launch, p: Dict, D: int, vec: bool, stats: Stats) -> None:
+    """The normalised backward's first pass: dO and dn from g, out and n, the segments' totals of Q^T dO and of dn_i q_i."""
+    rows = 128 if D <= 64 else 64
+    N, BH, H, wqk, wv = p["N"], p["BH"], p["H"], p["wqk"], p["wv"]
+    n_chunks, seg_chunks, n_seg = p["n_chunks"], p["seg_chunks"], p["n_seg"]
+    assert n_chunks == -(-N // rows) and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks
+    assert l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
+    assert l.lds == ((2 if D == 128 else 1) + 3) * rows * 2 * D + 2 * rows * 4, f"{l.kernel}: {l.lds} bytes of LDS"
+    assert 1 <= wqk <= D and 1 <= wv <= D and wqk % 8 == 0 and wv % 8 == 0
+    assert p["q"] % 16 == 0 and p["qs_n"] % 8 == 0 and p["dout"] % 16 == 0 and N * p["qs_n"] * 2 <= 0x3fffffff
+    for nm, pre, w in (("q", "qs", wqk), ("go", "gs", wv), ("o", "os", wv)):
+        arena.require(f"{l.kernel} {nm}", *tensor_extent(p, nm, f"{pre}_b", f"{pre}_h", f"{pre}_n", H, BH, N, w))
+    assert vec == bool(p["vec"])
+    if vec:
+        assert all(p[x] % 16 == 0 for x in ("go", "o")) and all(p[f"{t}_{d}"] % 8 == 0 for t in ("gs", "os") for d in "bhn")
+    ranges = [(nm, p[nm], p[nm] + nbytes) for nm, nbytes in (("denom", BH * N * 4), ("dn", BH * N * 4), ("dout", BH * N * wv * 2))]
+    if n_seg > 1:
+        ranges += [("totals", p["totals"], p["totals"] + BH * n_seg * D * D * 4), ("rsum", p["rsum"], p["rsum"] + BH * n_seg * D * 4)]
+    else:
+        assert not p["totals"] and not p["rsum"]
+    for nm, lo, hi in ranges:
+        arena.require(f"{l.kernel} {nm}", lo, hi)
+    ranges.sort(key=lambda r: r[1])
+    for (a, _, hi), (b, lo, _) in zip(ranges, ranges[1:]):
+        assert hi <= lo, f"{l.kernel}: {a} and {b} overlap"
+    stats.workgroups += BH * n_seg
+
+
+POLY_STATE, POLY_ROOM = 160 * 65, 224 * 65  # floats of a polynomial state; of its place in a state buffer
+
+
+def model_poly(arena: Arena, l: Launch, p: Dict, backward: bool, stats: Stats) -> None:
+    """The polynomial map's kernels: every operand, result and state that the kernel touches."""
+    H, BH, N, n_seg = p["H"], p["BH"], p["N"], p["n_seg"]
+    assert p["n_chunks"] == -(-N // 128) and l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
+    assert (n_seg - 1) * p["seg_chunks"] < p["n_chunks"] <= n_seg * p["seg_chunks"]
+    widths = {"q": p["r"], "k": p["r"], "v": p["wv"], "go": p["wv"], "o": p["wv"], "out": p["wv"], "dq": p["r"], "dk": p["r"],
+              "dv": p["wv"]}
+    strides = {"go": "gs", "out": "us"}
+    results = {"poly_walk_fwd_kernel": ("out",), "poly_walk_dq_kernel": ("dq",), "poly_walk_dkdv_kernel": ("dk", "dv")}
+    for nm, w in widths.items():
+        size = 4 if nm in ("dq", "dk", "dv") and p["wide_out"] else 2
+        is_result = nm in results.get(l.kernel, ())
+        assert p[nm] or not (is_result or nm in ("q", "k", "v") or (backward and nm == "go")), f"{l.kernel}: no {nm}"
+        if not p[nm]:
+            continue
+        pre = strides.get(nm, nm + "s")
+        lo, hi = tensor_extent(p, nm, f"{pre}_b", f"{pre}_h", f"{pre}_n", H, BH, N, w, size)
+        arena.require(f"{l.kernel} {nm}", lo, hi)
+        assert p[nm] % 16 == 0 and w % 8 == 0 and all(p[f"{pre}_{d}"] % 8 == 0 for d in "bhn")
+        if is_result:
+            stats.results.append((lo, hi))
+    if p["denom"]:
+        arena.require("denom", p["denom"], p["denom"] + BH * N * 4)
+    assert n_seg == 1 or p["totals"]
+    if p["totals"]:
+        arena.require("polynomial totals", p["totals"], p["totals"] + BH * n_seg * POLY_STATE * 4)
+    if p["entries"]:
+        arena.require("polynomial entry states", p["entries"], p["entries"] + BH * n_seg * POLY_ROOM * 4)
+    stats.workgroups += BH * n_seg
+
+
+def model_pack(arena: Arena, l: Launch, p: Dict, stats: Stats) -> None:
+    """Copies of rows: `width` columns of the source to rows of `wp`, zeros behind them."""
+    H, N, rows = p["H"], p["N"], p["rows"]
+    for i in range(l.grid[1]):
+        t = {k[len(f"t{i}."):]: v for k, v in p.items() if k.startswith(f"t{i}.")}
+        for nm, pre, w in (("src", "ss", t["width"]), ("dst", "ds", t["wp"])):
+            lo, hi = tensor_extent(t, nm, f"{pre}_b", f"{pre}_h", f"{pre}_n", H, rows // N, N, w)
+            arena.require(f"{l.kernel} {nm}{i}", lo, hi)
+        stats.results.append((lo, hi))
+
+
+class StateForms:
+    """In which of its two forms a buffer of states was written last -- row by row, or by fragments -- held against the form
+    in which the next kernel reads it: a walk that adds up totals reads fragments, everything else rows."""
+
+    def __init__(self):
+        self.frags: Dict[int, bool] = {}
+
+    def wrote(self, ptr: int, frags) -> None:
+        if ptr:
+            self.frags[ptr] = bool(frags)
+
+    def reads(self, l: Launch, what: str, ptr: int, frags) -> None:
+        if ptr in self.frags:
+            assert self.frags[ptr] == bool(frags), \
+                f"{l.kernel}: {what} were written {'by fragments' if self.frags[ptr] else 'row by row'} and are read otherwise"
+
+    def walk(self, l: Launch, p: Dict, D: int) -> None:
+        by_count = D <= 64 and 3 <= p["n_seg"] <= (16 if D <= 32 else 32)
+        for nm in ("init", "init2"):
+            if p[nm]:
+                self.reads(l, nm, p[nm], p["init_is_totals"] or by_count)
+        for nm in ("xinit", "xinit2"):
+            if p[nm]:
+                self.reads(l, nm, p[nm], by_count)
+        self.wrote(p["entry_out"], False), self.wrote(p["entry_out2"], False), self.wrote(p["r_totals"], p["r_frags"])
+
+
 def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
     """Every launch of a call: the general limits, then the kernel's model."""
+    forms = StateForms()
     for l in launches:
         stats.launches += 1
         stats.kernels[l.kernel] = stats.kernels.get(l.kernel, 0) + 1
@@ -900,8 +1049,10 @@ def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
                 arena.require("wsum", wsum, wsum + BH * chunks * DP * 4)
         elif k in ("walk_fwd_kernel", "walk_bwd_kernel", "walk_dkdv_kernel", "walk_bwd_rev_kernel"):
             model_walk(arena, l, l.struct("a0"), t[1], stats)
+            forms.walk(l, l.struct("a0"), t[1])
         elif k in ("walk_fwd_wide_kernel", "walk_bwd_rev_wide_kernel"):
             model_walk_wide(arena, l, l.struct("a0"), stats)
+            forms.walk(l, l.struct("a0"), 128)
         elif k == "walk_scan_kernel":
             totals, entry, n_seg, E, total2 = (l.args[f"a{i}"] for i in range(5))
             totals_b, entry_b = l.args["a8"], l.args["a9"]
@@ -910,8 +1061,30 @@ def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
             for t_, e_ in ((totals, entry),) + (((totals_b, entry_b),) if totals_b else ()):
                 arena.require("segment totals", t_, t_ + BH * n_seg * E * 4)
                 arena.require("entry states", e_, e_ + BH * n_seg * E * 4)
+                forms.reads(l, "totals", t_, False), forms.wrote(e_, False)
         elif k == "walk_totals_kernel":
-            model_walk_totals(arena, l, l.struct("a0"), t[1], stats, both=len(t) > 4 and bool(t[4]))
+            p = l.struct("a0")
+            model_walk_totals(arena, l, p, t[1], stats, both=len(t) > 4 and bool(t[4]))
+            forms.wrote(p["totals"], p["frags"]), forms.wrote(p["totals2"], p["frags"])
+        elif k == "walk_totals_quad_kernel":
+            p = l.struct("a0")
+            for nm, w in (("y", p["dy"] + p["dy2"]), ("z", p["dz"] + p["dz2"])):
+                arena.require(f"totals {nm}", *tensor_extent(p, nm, f"{nm}s_b", f"{nm}s_h", f"{nm}s_n", p["H"], p["BH"], p["N"], w))
+            # (a z of two halves: the states of the four pairs one after the other, y's second half at totals2)
+            states = p["BH"] * p["n_seg"] * 128 * 128 * 4
+            assert not p["dz2"] or p["totals2"] == p["totals"] + states
+            for base in [p["totals"] + i * states for i in range(4)] if p["dz2"] else [p["totals"], p["totals2"]]:
+                arena.require("segment totals", base, base + states)
+                forms.wrote(base, p["frags"])
+        elif k == "walk_grad_totals_kernel":
+            model_walk_grad_totals(arena, l, l.struct("a0"), t[1], t[2], stats)
+            forms.wrote(l.args["a0.totals"], l.args["a0.frags"])
+        elif k == "poly_totals_kernel" or k.startswith("poly_walk_"):
+            model_poly(arena, l, l.struct("a0"), t[2] if k == "poly_totals_kernel" else "_d" in k, stats)
+        elif k == "poly_scan_kernel":
+            arena.require("polynomial totals", l.args["a0"], l.args["a0"] + l.args["a1"] * l.args["a2"] * 4)
+        elif k == "pack_rows_kernel":
+            model_pack(arena, l, l.struct("a0"), stats)
         else:
             # remaining kernels (scans, vector sums, element-wise passes, chunk states): limits above,
             # and every pointer argument inside a tensor or the workspace
