@@ -76,6 +76,21 @@ def _check_no_scratch(report: str, kernel: str) -> None:
         raise RuntimeError(f"no resource report for {kernel}: the spill check did not run")
 
 
+def _check_waves(report: str, kernel: str, waves: int) -> None:
+    """Fail the build if an instantiation of `kernel` (a part of the mangled name) leaves room for fewer than `waves` wavefronts on a
+    SIMD: with many small workgroups the kernel's rate goes by how many of them are resident."""
+    name, seen = None, 0
+    for line in report.splitlines():
+        if "Function Name:" in line:
+            name = line.split("Function Name:")[1].split()[0]
+        elif "Occupancy [waves/SIMD]:" in line and name and kernel in name:
+            seen += 1
+            if int(line.split("Occupancy [waves/SIMD]:")[1].split()[0]) < waves:
+                raise RuntimeError(f"{name} uses registers for fewer than {waves} wavefronts per SIMD")
+    if seen == 0:
+        raise RuntimeError(f"no resource report for {kernel}: the occupancy check did not run")
+
+
 def _compile_inst(args) -> str:
     dtype, dc, do = args
     obj = os.path.join(OBJ_DIR, f"inst_t{dtype}_c{dc}_o{do}.o")
@@ -92,6 +107,8 @@ def _compile_walk(args) -> str:
     if part == 1:
         _check_no_scratch(report, "walk_bwd_rev_kernel")
         _check_no_scratch(report, "walk_bwd_rev_wide_kernel")
+    else:  # (the plain forward walk at D = 32)
+        _check_waves(report, f"walk_fwd_kernelI{('DF16b', 'DF16_')[dtype]}Li32ELb0ELi0ELb0", 4)
     return obj
 
 

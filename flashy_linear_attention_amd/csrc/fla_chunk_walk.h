@@ -1038,11 +1038,14 @@ __device__ __forceinline__ void walk_all_requested() {
 // plan of eleven segments then read 1.75 times the states they need, from L2 -- backward walk, D = 64, B H 40, N 5184, 41.1 us, this way
 // 38.3; forward, D = 32, B H 128, N 1536, four segments 11.1 / 10.2; 128 over 64 columns, B H 64, N 1024, reverse walk 24.8 / 23.5.
 // With four blocks per wave, in groups of three, it stays so: the branches take registers that walk_bwd_rev_wide_kernel does not have)
+// At D = 32, where one wave has the state's one block and there are at most 16 segments, groups of four: eight take 148 registers in
+// place of 110 and leave three wavefronts to a SIMD in place of four, where many heads have more workgroups than that (the build checks
+// it).  Forward, B H 2048, N 300 32.0 us with eight, this way 30.7; forward + backward, B H 32, N 2048, 16 segments 31.5 / 28.7.
 template <int D, typename B>
 __device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int f_hi, int wave, int lane,
                                                 f32x16 (&st)[WalkCfg<D>::NBW]) {
     using W = WalkCfg<D>;
-    constexpr int GROUP = B::SLOTS > 2 ? 3 : B::SLOTS > 1 ? 6 : 8;  // (GROUP x SLOTS x 16 registers beside the sum)
+    constexpr int GROUP = B::SLOTS > 2 ? 3 : B::SLOTS > 1 ? 6 : D == 32 ? 4 : 8;  // (GROUP x SLOTS x 16 registers beside the sum)
 #pragma unroll
     for (int i = 0; i < W::NBW; ++i)
 #pragma unroll
