@@ -1076,7 +1076,9 @@ __device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int 
 }
 
 // st_a, st_b = this wave's blocks of the sums of the states a[f_lo .. f_hi - 1], b[f_lo .. f_hi - 1], the loads of
-// up to three states of each in flight together (a chain of dependent loads costs a memory latency per state)
+// up to three states of each in flight together (a chain of dependent loads costs a memory latency per state).  Past the range
+// nothing is requested, as above (forward + backward with the last state once more in its place -> this: 256 / 64, B H 64,
+// N 1024 90.8 -> 89.3 us; 153 / 64, B H 80, N 640 98.7 -> 96.9)
 template <int D, typename B>
 __device__ __forceinline__ void walk_sum_two(const float *a, const float *b, int f_lo, int f_hi, int wave, int lane,
                                              f32x16 (&st_a)[WalkCfg<D>::NBW], f32x16 (&st_b)[WalkCfg<D>::NBW]) {
@@ -1092,10 +1094,9 @@ __device__ __forceinline__ void walk_sum_two(const float *a, const float *b, int
         f32x16 ta[GROUP][W::NBW], tb[GROUP][W::NBW];
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
-            // (past the range: the last state once more, not added -- nor times zero: it may be infinite)
-            const int f = f0 + u < f_hi ? f0 + u : f_hi - 1;
-            walk_read_frags<D, B>(a + (int64_t)f * E, wave, lane, ta[u]);
-            walk_read_frags<D, B>(b + (int64_t)f * E, wave, lane, tb[u]);
+            if (f0 + u >= f_hi) continue;
+            walk_read_frags<D, B>(a + (int64_t)(f0 + u) * E, wave, lane, ta[u]);
+            walk_read_frags<D, B>(b + (int64_t)(f0 + u) * E, wave, lane, tb[u]);
         }
         walk_all_requested();
 #pragma unroll
