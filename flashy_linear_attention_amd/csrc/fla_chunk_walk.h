@@ -1041,7 +1041,10 @@ __device__ __forceinline__ void walk_all_requested() {
 // At D = 32, where one wave has the state's one block and there are at most 16 segments, groups of four: eight take 148 registers in
 // place of 110 and leave three wavefronts to a SIMD in place of four, where many heads have more workgroups than that (the build checks
 // it).  Forward, B H 2048, N 300 32.0 us with eight, this way 30.7; forward + backward, B H 32, N 2048, 16 segments 31.5 / 28.7.
-template <int D, typename B>
+// TOGETHER: the group's loads stay ahead of its additions (walk_all_requested).  Not in walk_fwd_wide_kernel with a v above 64 columns:
+// its loop over the chunks then holds more in accumulation registers than it has to, 300 moves in place of 221 (forward, 192 / 128, B H
+// 128, N 2048 106.6 us, this way 105.2; forward + backward, 256 / 128, B H 42, N 1536, six segments 207.7 / 202.6)
+template <int D, typename B, bool TOGETHER = true>
 __device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int f_hi, int wave, int lane,
                                                 f32x16 (&st)[WalkCfg<D>::NBW]) {
     using W = WalkCfg<D>;
@@ -1061,7 +1064,7 @@ __device__ __forceinline__ void walk_sum_states(const float *buf, int f_lo, int 
                 if (f0 + u < f_hi) walk_read_frags<D, B>(buf + (int64_t)(f0 + u) * (D * D), wave, lane, t[u]);
             }
         }
-        walk_all_requested();
+        if constexpr (TOGETHER) walk_all_requested();
 #pragma unroll
         for (int u = 0; u < GROUP; ++u) {
             if (f0 + u >= f_hi) continue;
@@ -1501,8 +1504,8 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
         if constexpr (NV == 2) {  // (both halves' loads in flight together; with four blocks per wave and state, one half's)
             walk_sum_two<D, B>(p.init + at, p.init2 + at, 0, sl.seg, wave, lane, st0, st1);
         } else {
-            walk_sum_states<D, B>(p.init + at, 0, sl.seg, wave, lane, st0);
-            walk_sum_states<D, B>(p.init2 + at, 0, sl.seg, wave, lane, st1);
+            walk_sum_states<D, B, false>(p.init + at, 0, sl.seg, wave, lane, st0);
+            walk_sum_states<D, B, false>(p.init2 + at, 0, sl.seg, wave, lane, st1);
         }
         if (p.entry_out && sl.seg > 0) {  // (the first segment's entry state, zero, is read by nobody)
             walk_write_state<D, B>(p.entry_out + at + (int64_t)sl.seg * (D * D), wave, lane, st0);
