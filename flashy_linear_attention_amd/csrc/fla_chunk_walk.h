@@ -1245,8 +1245,24 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     f32x16 st[W::NBW];
     walk_load_init<D, B>(p, sl, wave, lane, st, false);
     if constexpr (DOUBLE && NORM <= 1) {  // (the entry state this walk formed from the segments' totals, for backward)
-        if (p.init_is_totals && p.entry_out && sl.seg > 0)
-            walk_write_state<D, B>(p.entry_out + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D), wave, lane, st);
+        // (Through a descriptor.  By walk_write_state, with a scalar address per store, scalar registers ran out: the loop below held the
+        // result's descriptor in vector registers, with a loop over the lanes around each of its stores -- in every plan, entry states
+        // or not.  Forward that way -> this: normalised, B H 300, N 600 66.9 -> 64.1 us (two rounds of one segment), B H 100, N 1000 45.3 -> 43.6
+        // (two), B H 16, N 20000 110.9 -> 107.5; plain, B H 300, N 600 51.7 -> 49.1)
+        if (p.init_is_totals && p.entry_out && sl.seg > 0) {
+            const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                p.entry_out + ((int64_t)sl.bh * p.n_seg + sl.seg) * (D * D), 0, D * D * 4, 0x00020000);
+#pragma unroll
+            for (int i = 0; i < B::SLOTS; ++i)
+                if (B::valid(wave, i)) {
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const float x = st[i][v];  // (of an element itself the cast takes the vector's first)
+                        const int at = (32 * B::dbk(wave, i) + 8 * (v / 4) + 4 * g + (v % 4)) * D + 32 * B::eb(wave) + l32;
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), rs, (uint32_t)(at * 4), 0, 0);
+                    }
+                }
+        }
     }
     // the state's copy in LDS for the next chunk (SCALED: every wave has passed a barrier since its walk_state_max)
     float sback = 1.f, *smax = reinterpret_cast<float *>(xv);
