@@ -402,8 +402,13 @@ struct WalkPlan {
 //   (22) 101.9 / 105.7; B H 10, N 16384 (24) 248 / 251; B H 8, N 8192 (32) 91.4 / 99.4.  Four pairs of column
 //   halves at a time (256 / 256) the same: B H 8, N 4096 (16) 154.4 / 141.7; B H 6, N 8192 (19) 313 / 304; B H 5, N 4096 (22)
 //   182.9 / 190.1.
-//   A wide q / k against a v of up to 128: two states to add up, and the walks are held to seven.  256 / 64, B H 64, N 4096 (4)
-//   320 / 313 (kernels); it would pay up to fifteen: B H 32, N 2048 (8) 104.0 / 95.5, B H 20, N 4096 (11) 162.8 / 155.4.
+//   A wide q / k against a v of up to 128: two states to add up.  256 / 64, B H 64, N 4096 (4) 320 / 313 (kernels).  Nothing in the
+//   walks holds them to seven: B H 32, N 2048 (8) 104.0 / 95.5, B H 20, N 4096 (11) 162.8 / 155.4, and fifteen still gained.  The line
+//   lies at seven because only these sizes over a v of 64 columns were timed above it, none over a v of up to 128, whose
+//   sums hold four blocks per wave in groups of three.
+//   kSumOnLoadWorkspace: a plain forward with a state buffer and no workspace is refused up to this many segments and taken beyond,
+//   by a scan in the state buffer.  The scan could do the fewer segments as well; twelve is where the walks' sums ended before the
+//   loads of several states were in flight together, and it stays so that every call keeps its answer.
 //   The polynomial map, 41 KiB a state, forward + backward (forward alone): B H 20, N 4096 (11 segments) 136.1 / 129.9 us (47.1 /
 //   43.7); B H 16, N 4096 (16) 84.1 / 83.3 (32.5 / 27.2); B H 10, N 2000 (16) 59.2 / 53.4; B H 8, N 8192 (32) 83.8 / 94.6.
 constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 7, kSumOnLoadPoly = 20, kSumOnLoadWorkspace = 12;
@@ -807,7 +812,9 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
     const bool rev_sums_on_load = sums_on_load(wp, kSumOnLoadWide);
     // dQ's walks add up their halves' totals of Q^T dO on their way (WalkParams::r_totals).  A totals kernel in front -> this: 256 / 64,
     // B H 32, N 2048 104.5 -> 101.0 us, B H 64, N 4096 293 -> 288.  With a v above 64 columns a walk holds two full states: 256 / 128 eight
-    // segments or more 159.8 -> 155.5 (B H 32, N 2048), four 399 -> 403 (B H 64, N 4096), ten short ones 130.6 -> 130.4
+    // segments or more 159.8 -> 155.5 (B H 32, N 2048), four 399 -> 403 (B H 64, N 4096), ten short ones 130.6 -> 130.4; and there
+    // only with more than 64 columns in q / k's second half too: a v above 64 columns against a half of at most 64 has no such variant
+    // of the walk.  bf16 alone: two sets of four tiles and the state are all of the LDS, and an fp16 walk's scale needs a place there
     const bool dq_walk_sums = !one_walk && (dv <= 64 || (dqk > 192 && wp.n_seg >= 8)) && wp.n_seg > 2 && dtype == FLA_DTYPE_BF16;
     if (wp.n_seg > 1) {
         float *const none[2] = {nullptr, nullptr};
@@ -1017,7 +1024,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         // D = 128, a few segments more than two: the totals go to the workspace, the walk adds them up itself as it starts
         // and writes the entry states it formed to state_out -- no scan launch
         // (a caller may have brought a state buffer and no workspace: then a scan in the former -- but for the plain operator up to
-        // kSumOnLoadWorkspace segments, which asks for its workspace)
+        // kSumOnLoadWorkspace segments, which is refused without its workspace: the reason stands there)
         const bool has_work = workspace && reinterpret_cast<uintptr_t>(workspace) % 16 == 0 && workspace_bytes >= wp.work_bytes;
         const bool sum_on_load = wp.split && sums_on_load(wp) && (!in_state || has_work || (!fmap && !nx && wp.n_seg <= kSumOnLoadWorkspace));
         if (need_totals && (!in_state || sum_on_load) && !has_work) return FLA_ERR_WORKSPACE;
@@ -1212,7 +1219,8 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
         const bool rev_sums_on_load = (one_walk || causal || nx) && sums_on_load(wp);
         float *const rcv = nx ? reinterpret_cast<float *>(static_cast<char *>(nx->vec) + walk_vec_bytes(B, H, N, dqk, dv)) : nullptr;
-        // dQ's walk adds up the segments' totals of Q^T dO on its way (WalkParams::r_totals, figures there)
+        // dQ's walk adds up the segments' totals of Q^T dO on its way (WalkParams::r_totals, figures there; bf16 alone: an fp16 walk's
+        // scale has no place in the LDS beside two sets of four tiles and the state)
         const bool dq_walk_sums = !one_walk && !nx && !fmap && wp.n_seg > 2 && dtype == FLA_DTYPE_BF16 && dqk > 64;
         if (wp.n_seg > 1) {
             if (!state_in) {

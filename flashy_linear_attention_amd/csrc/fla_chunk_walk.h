@@ -1599,7 +1599,7 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
 // forward then wrote element by element, spilled 64 bytes a lane: B H 64, N 4096, D 64 71 us, this way 59.)
 // (Obtained backwards instead -- from the state at the segment's end, subtracting every chunk's K^T V when the walk reaches
 // it -- one late row that is infinite, NaN or merely huge spoiled the dQ of every chunk before it.  Forward + backward
-// at B H 16, N 32768, D 64 that way 222 us, this way 234.)
+// at B H 16, N 32768, D 64 that way 222 us, this way 234 at the time, 222 with totals added up by fragments.)
 template <typename T, int D, bool NORM, bool WIDE = false>
 __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -1786,7 +1786,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         walk_load_tile<D>(rv, base + 2 * W::TILE, row0, vs2, p.wv, wave, lane);
         walk_load_tile<D>(rg, base + 3 * W::TILE, row0, gs2, p.wv, wave, lane);
     };
-    static_assert(!NORM || W::C == 64, "one dn value per lane covers a chunk of 64 rows");
+    static_assert(!NORM || W::C == 64, "eight groups of four dn values are a chunk of 64 rows");
     // Ordinary loads, requested a chunk ahead (once the tiles of the chunk before have been awaited) and
     // read at the top of their chunk, BEFORE the next tile loads go out: the wait the compiler puts
     // in front of the first use is one for every outstanding load and store (it cannot count past

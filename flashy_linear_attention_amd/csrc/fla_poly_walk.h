@@ -70,7 +70,8 @@ struct PolyFeatures {
     static constexpr int kHalves = kF / 16;                    // blocks of 16 features: the units in which waves own a state
     static constexpr int kV = 64;                              // value columns of a state
     static constexpr int kState = kF * kV + kF;                // [feature][value column], then the column of ones / dn
-    static constexpr int kStateRoom = 224 * 65;                // floats per segment of a state buffer (what callers set aside)
+    static constexpr int kStateRoom = 224 * 65;                // floats per segment of a state buffer: a state of 224 features,
+                                                               // by which the size query still answers; the rest is not touched
 };
 
 struct PolyLds {  // byte offsets

@@ -20,7 +20,7 @@ def test_widths_that_are_no_multiples_of_8(bh, dqk, dv, pair_from, forward_from)
 
 
 def test_polynomial_state_is_for_several_segments_alone():
-    """One state of 224 features over 64 columns, and their column of ones, per segment; nothing where a (b, h) is one segment
+    """Room for 224 features over 64 columns, and their column of ones, per segment (a state takes 160 of them); nothing where a (b, h) is one segment
     (256 workgroups at a time, 128 rows a chunk), however many heads there are."""
     nbytes = lambda *shape: _lib.query("fla_poly_attn_chunked_state_bytes", *shape)  # noqa: E731
     assert nbytes(16, 256, 128, 16, 64) == nbytes(4, 100, 4096, 16, 64) == nbytes(1, 1, 100, 8, 32) == 16
