@@ -74,10 +74,9 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkStateParams
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 5, lam = lane & 15, l32 = lane & 31, beta = (lane >> 4) & 1;
 
-    const int wg = blockIdx.x, xcd = wg & 7, slot = wg >> 3;
-    const int hl = slot / p.n_chunks, chunk = slot - hl * p.n_chunks;
-    const int bh = hl * 8 + xcd;
-    if (bh >= p.BH) return;
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_chunks, p.ys_h);
+    const int bh = item.bh, chunk = item.part;
+    if (bh < 0) return;
     const int b = bh / p.H, h = bh - b * p.H;
     const T *Y = static_cast<const T *>(p.y) + b * p.ys_b + h * p.ys_h;
     const T *Z = static_cast<const T *>(p.z) + b * p.zs_b + h * p.zs_h;

@@ -912,15 +912,14 @@ struct WalkSlice {
     bool valid;
 };
 
-// workgroup -> ((b, h), segment): heads of one XCD in sequence, as in the other kernels
+// workgroup -> ((b, h), segment)
 __device__ __forceinline__ WalkSlice walk_slice(const WalkParams &p) {
-    const int wg = blockIdx.x, xcd = wg & 7, slot = wg >> 3;
-    const int hl = slot / p.n_seg, seg = slot - hl * p.n_seg;
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.ks_h);
     WalkSlice s;
-    s.bh = hl * 8 + xcd, s.seg = seg;
-    s.c_lo = seg * p.seg_chunks;
+    s.bh = item.bh, s.seg = item.part;
+    s.c_lo = s.seg * p.seg_chunks;
     s.c_hi = s.c_lo + p.seg_chunks < p.n_chunks ? s.c_lo + p.seg_chunks : p.n_chunks;
-    s.valid = s.bh < p.BH && s.c_lo < p.n_chunks;
+    s.valid = s.bh >= 0 && s.c_lo < p.n_chunks;
     return s;
 }
 
@@ -2246,10 +2245,9 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wg = blockIdx.x, xcd = wg & 7, slot = wg >> 3;
-    const int hl = slot / p.n_seg, bh = hl * 8 + xcd;
-    int seg = slot - hl * p.n_seg;
-    if (bh >= p.BH) return;
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.ys_h);
+    const int bh = item.bh, seg = item.part;
+    if (bh < 0) return;
     const int dy = p.dy;
     int64_t out_at;
     int c_lo, c_hi;
@@ -2590,9 +2588,9 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void walk_grad_totals_kernel
     float *vd = reinterpret_cast<float *>(smem + (QT + 2) * W::TILE);  // QT tiles of Q, two of dO, two of dn
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wg = blockIdx.x, xcd = wg & 7, slot = wg >> 3;
-    const int hl = slot / p.n_seg, bh = hl * 8 + xcd, seg = slot - hl * p.n_seg;
-    if (bh >= p.BH) return;
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.qs_h);
+    const int bh = item.bh, seg = item.part;
+    if (bh < 0) return;
     // the chunks whose sums are wanted, [a_lo, a_hi), and those that are visited for dO and dn alone, from b_lo on.  Two
     // segments: both workgroups of a (b, h) take one half of either segment
     int a_lo = seg * p.seg_chunks, a_hi = a_lo + p.seg_chunks < p.n_chunks ? a_lo + p.seg_chunks : p.n_chunks;

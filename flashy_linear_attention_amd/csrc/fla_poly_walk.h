@@ -469,13 +469,12 @@ struct PolySlice {
     bool valid;
 };
 __device__ __forceinline__ PolySlice poly_slice(const PolyWalkParams &p) {  // (walk_slice's map)
-    const int wg = blockIdx.x, xcd = wg & 7, slot = wg >> 3;
-    const int hl = slot / p.n_seg, seg = slot - hl * p.n_seg;
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.ks_h);
     PolySlice s;
-    s.bh = hl * 8 + xcd, s.seg = seg;
-    s.c_lo = seg * p.seg_chunks;
+    s.bh = item.bh, s.seg = item.part;
+    s.c_lo = s.seg * p.seg_chunks;
     s.c_hi = s.c_lo + p.seg_chunks < p.n_chunks ? s.c_lo + p.seg_chunks : p.n_chunks;
-    s.valid = s.bh < p.BH && s.c_lo < p.n_chunks;
+    s.valid = s.bh >= 0 && s.c_lo < p.n_chunks;
     return s;
 }
 

@@ -66,6 +66,32 @@ __device__ __forceinline__ void dma_16B_per_lane(u32x4 rsrc, uint32_t lds_base, 
                  : "s"(lds_base), "v"(voffset), "s"(rsrc), "s"(soffset), "n"(LDS_IMM)
                  : "memory", "m0", "scc");
 }
+// Workgroup -> (head, part) of a launch of BH heads with `parts` equal parts each.  Workgroup ids go round the eight XCDs, so id % 8
+// is the XCD.  The parts of a head stay together, for the L2 that they share.
+//   * BH a multiple of 8: an XCD takes every eighth head -- or, where a head's rows end inside a 128-byte line (`stride_h`: elements
+//     of 16 bits from a head to the next), pairs of neighbours, which share those lines in (B, N, H, D) storage.  Forward + backward:
+//     32 columns, B 2 H 16 N 8192 76.4 -> 67.2 us; 96 columns, B 2 H 24 N 4096 153 -> 148.  (Pairs for every row: 64 columns, B 1 H 16
+//     N 32768 in that storage 241 -> 232 us, but with a feature map B 4 H 16 N 4096 144 -> 148, and (B, H, N, D) storage gains nothing.)
+//   * else an eighth of all parts, consecutive ones.  Whole heads per XCD left XCDs idle, and gave others two rounds: forward +
+//     backward, D = 128: B H 1 N 16384 241 -> 86 us, B H 4 153 -> 95, B H 12 278 -> 179, B H 20 N 8192 232 -> 152; D = 64: B H 12
+//     N 32768 218 -> 165, B H 20 N 16384 161 -> 138.
+// The grid may hold more workgroups than there are parts (8 ceil(BH / 8) parts of them): bh < 0 is none.
+struct XcdItem {
+    int bh, part;
+};
+__device__ __forceinline__ XcdItem xcd_item(int wg, int BH, int parts, int64_t stride_h) {
+    const int xcd = wg & 7, slot = wg >> 3;
+    if (BH % 8 == 0) {
+        const int hl = slot / parts;
+        const bool pairs = BH % 16 == 0 && stride_h % 64 != 0;
+        return {hl >= BH / 8 ? -1 : pairs ? (hl >> 1) * 16 + xcd * 2 + (hl & 1) : hl * 8 + xcd, slot - hl * parts};
+    }
+    const int total = BH * parts, share = (total + 7) >> 3, item = xcd * share + slot;
+    if (slot >= share || item >= total) return {-1, 0};
+    const int bh = item / parts;
+    return {bh, item - bh * parts};
+}
+
 // s_waitcnt vmcnt(N) only (expcnt and lgkmcnt fields left at their maxima): returns once at
 // most N of this wave's buffer loads, the most recently issued ones, are still in flight.
 // f(integral_constant<int, I>) for I = BEGIN .. END-1, unrolled at compile time
@@ -231,10 +257,11 @@ __device__ __forceinline__ void tri_fast_body(const TriParams &p, const int wg_i
     // same time).  Single tiles differ in work, so they are ordered heaviest first across all
     // heads: whatever CU frees up next takes the heaviest tile left.
     const int n_hl = (p.BH + 7) >> 3;
-    const int hl = (single && !chunked) ? slot % n_hl : slot / n_pairs;
-    const int rank = (single && !chunked) ? slot / n_hl : slot - hl * n_pairs;
-    const int bh = hl * 8 + xcd;
-    if (bh >= p.BH) return;
+    const XcdItem chunk = chunked ? xcd_item(wg, p.BH, p.n_tiles, p.ys_h) : XcdItem{0, 0};
+    const int hl = single ? slot % n_hl : slot / n_pairs;
+    const int rank = chunked ? chunk.part : single ? slot / n_hl : slot - hl * n_pairs;
+    const int bh = chunked ? chunk.bh : hl * 8 + xcd;
+    if (chunked ? bh < 0 : bh >= p.BH) return;
     const bool upper = p.upper != 0;
     const int b = bh / p.H, h = bh - b * p.H;
     const T *X = static_cast<const T *>(p.x) + b * p.xs_b + h * p.xs_h;
