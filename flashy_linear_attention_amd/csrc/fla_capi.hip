@@ -2075,9 +2075,16 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
         return d <= 32 ? N > 512 : d <= 64 ? N >= 256 : d <= 128 ? N >= 128 : 1;
     }
     // (padded widths that differ: the quadratic side is the small-V operator, whose wide products are two launches)
-    if (wp.ok && !backward) return wp.D <= 32 ? N >= 4096 || w >= 5e9 : N >= 2048 || w >= 1.2e10;
-    if (wp.ok && pad_index(D_qk) != pad_index(D_v)) return N >= 1024 || w >= (wp.D <= 64 ? 1e9 : 5e8);
-    if (wp.ok) return N >= (wp.D <= 32 ? 4096 : 2048) || w >= (wp.D <= 64 ? 4e9 : 8e9);  // equal padded head dims up to 128
+    // Forward alone, B H 1 ... 520: 64 columns 1.10 to 1.4 at N = 768 (0.90 to 1.2 at 576), 32 and 128 columns 1.06 to 1.3 at 1024
+    // (0.94 to 1.2 at 768), 64 / 32, 128 / 64 and 128 / 32 1.06 to 1.5 at 1024; a single segment per head, which has no totals to
+    // wait for, 1.12 to 2.3 from N = 320 on.
+    const bool equal = pad_index(D_qk) == pad_index(D_v), one = wp.n_seg == 1 && N > 256;
+    if (wp.ok && !backward) return one || N >= (wp.D == 64 && equal ? 768 : 1024) || w >= (wp.D <= 32 ? 5e9 : 1.2e10);
+    if (wp.ok && !equal) return N >= 1024 || w >= (wp.D <= 64 ? 1e9 : 5e8);
+    // Equal padded head dims up to 128.  (Pairs gain earlier on the GPU -- 64 columns 1.2 to 1.5 from N = 768 on --, but there the
+    // host, 58 us for the quadratic pair's two launches and 72 for the chunk-wise one's four, takes longer than either.  Single
+    // segments of 128 columns: B H 130 N 448 74 / 64 us, B H 256 N 320 92 / 61.)
+    if (wp.ok) return N >= (wp.D <= 32 ? 4096 : 2048) || w >= (wp.D <= 64 ? 4e9 : one ? 3.2e9 : 8e9);
     // D_qk in (128, 256].  D_v <= 64: pairs 1.13 to 5 from N = 1024 or W = 1e9 on, forward alone 1.13 to 2.9 from N = 1024 (N = 512
     // 0.82 to 1.1).  D_v in (64, 128]: pairs 1.35 to 3.1 from N = 2048, 1.3 from W = 2.5e10 (1.0 at 1.7e10, N = 1024); forward
     // alone 1.14 to 1.55 from N = 4096, at N = 2048 1.1 to 1.4 with B H <= 4 and 0.93 with 16.
@@ -2424,7 +2431,19 @@ int fla_normalised_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int6
     const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v);
     if (!wp.ok) return 0;
     const double w = (double)B * (double)H * (double)N * (double)N * (double)wp.D;
-    return N >= 2048 || (N >= 1024 && wp.D <= 64) || w >= 1.2e10;
+    // (a single segment per head: 1.03 to 2.1 from N = 320 on, B H 130 ... 600)
+    return N >= 2048 || (N >= 1024 && wp.D <= 64) || w >= 1.2e10 || (wp.n_seg == 1 && N > 256);
+}
+// Pairs, GPU time of the quadratic evaluation over the chunk-wise one's, B H 1 ... 400: 1.13 to 1.8 at N = 320, 1.06 to 1.9 at 384,
+// 1.3 to 2.2 at 1024, 2.2 to 4.1 at 4096; 0.54 to 0.95 up to 256 (a single chunk of 256 rows with states in memory).  Both are four
+// launches, but the chunk-wise one has two buffers more to allocate, 47 against 43 us of the host through autograd, so the line lies
+// where the quadratic kernels take about that long: 128 columns from 257 rows on, 64 from 768, 32 from 1536, or many heads.  Errors
+// against fp64 (elu + 1 features): dQ 0.77 to 0.99 of the quadratic evaluation's, O, dK and dV 0.72 to 1.0.
+int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype) {
+    if (dtype != FLA_DTYPE_BF16 || D_qk < 1 || D_v < 1 || D_qk % 8 != 0 || D_v % 8 != 0) return 0;
+    const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v);
+    const double w = (double)B * (double)H * (double)N * (double)N * (double)wp.D;
+    return wp.ok && N > 256 && (wp.D == 128 || N >= (wp.D == 64 ? 768 : 1536) || w >= 1.2e9);
 }
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward) {
     if (dtype != FLA_DTYPE_BF16 || !poly_plan(B, H, N, R, D_v).ok) return 0;
