@@ -402,16 +402,16 @@ struct WalkPlan {
 //   (22) 101.9 / 105.7; B H 10, N 16384 (24) 248 / 251; B H 8, N 8192 (32) 91.4 / 99.4.  Four pairs of column
 //   halves at a time (256 / 256) the same: B H 8, N 4096 (16) 154.4 / 141.7; B H 6, N 8192 (19) 313 / 304; B H 5, N 4096 (22)
 //   182.9 / 190.1.
-//   A wide q / k against a v of up to 128: two states to add up.  256 / 64, B H 64, N 4096 (4) 320 / 313 (kernels).  Nothing in the
-//   walks holds them to seven: B H 32, N 2048 (8) 104.0 / 95.5, B H 20, N 4096 (11) 162.8 / 155.4, and fifteen still gained.  The line
-//   lies at seven because only these sizes over a v of 64 columns were timed above it, none over a v of up to 128, whose
-//   sums hold four blocks per wave in groups of three.
+//   A wide q / k against a v of up to 128: two states to add up.  256 / 64, B H 64, N 4096 (4) 320 / 313 (kernels); through the
+//   operator, v of 64: 153 / 64, B H 32, N 2048 (8) 121.6 / 117.0; 256 / 64, B H 32, N 2048 (8) 99.6 / 98.7, B H 24, N 8192 (10)
+//   226.0 / 219.9, B H 16, N 4096 (16) 103.6 / 104.8.  v of 128: 192 / 128, B H 32, N 2048 (8) 148 / 130, B H 24, N 4096 (10)
+//   191 / 176, 256 / 128, B H 16, N 4096 (16) 151.8 / 146.0, N 2048 111.2 / 108.6, forward alone 192 / 128, B H 16, N 4096 51.2 / 48.6.
 //   kSumOnLoadWorkspace: a plain forward with a state buffer and no workspace is refused up to this many segments and taken beyond,
 //   by a scan in the state buffer.  The scan could do the fewer segments as well; twelve is where the walks' sums ended before the
 //   loads of several states were in flight together, and it stays so that every call keeps its answer.
 //   The polynomial map, 41 KiB a state, forward + backward (forward alone): B H 20, N 4096 (11 segments) 136.1 / 129.9 us (47.1 /
 //   43.7); B H 16, N 4096 (16) 84.1 / 83.3 (32.5 / 27.2); B H 10, N 2000 (16) 59.2 / 53.4; B H 8, N 8192 (32) 83.8 / 94.6.
-constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 7, kSumOnLoadPoly = 20, kSumOnLoadWorkspace = 12;
+constexpr int kSumOnLoadMost = 20, kSumOnLoadWide = 15, kSumOnLoadPoly = 20, kSumOnLoadWorkspace = 12;
 
 // `parts`: workgroups per segment (a launch that does several column halves at a time).
 WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, bool mixed = false, int64_t parts = 1) {
@@ -768,7 +768,7 @@ int wide_forward(const WidePlan &wide, const View &q, const View &k, const View 
     // starts (three of each half in flight together) and writes the entry state it formed for backward
     // (B 4, H 16, N 4096, D_qk 256, D_v 64, four segments: 0.273 -> 0.267 ms per forward + backward, and 0.264 with
     // the reverse walk doing the same).
-    const bool sum_on_load = sums_on_load(wp, kSumOnLoadWide);
+    const bool sum_on_load = sums_on_load(wp, dv <= 64 ? kSumOnLoadWide : kSumOnLoadMost);
     float *keep[2] = {nullptr, nullptr};
     if (wp.n_seg > 1) {
         // (kept for backward when there is a state buffer: each half's entry states, its final state behind them;
@@ -809,7 +809,7 @@ int wide_backward(const WidePlan &wide, const View &go, const View &q, const Vie
     // at hand -- K_h^T V over the segments before
     const float *fwd_entries[2] = {nullptr, nullptr}, *entries[2] = {nullptr, nullptr};
     // (the reverse walk adds up the totals of the segments after its own itself, as forward does)
-    const bool rev_sums_on_load = sums_on_load(wp, kSumOnLoadWide);
+    const bool rev_sums_on_load = sums_on_load(wp, dv <= 64 ? kSumOnLoadWide : kSumOnLoadMost);
     // dQ's walks add up their halves' totals of Q^T dO on their way (WalkParams::r_totals).  A totals kernel in front -> this: 256 / 64,
     // B H 32, N 2048 104.5 -> 101.0 us, B H 64, N 4096 293 -> 288.  With a v above 64 columns a walk holds two full states: 256 / 128 eight
     // segments or more 159.8 -> 155.5 (B H 32, N 2048), four 399 -> 403 (B H 64, N 4096), ten short ones 130.6 -> 130.4; and there

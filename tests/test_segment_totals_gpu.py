@@ -1,5 +1,5 @@
 """Plans whose walks add up the segments' totals as they start, around the numbers of segments where a scan takes over (20 at
-128 columns and with both sides above 128, 7 with a wide q / k alone, 32 at 64, 16 at 32): both passes, with forward's state and
+128 columns and with both sides above 128, 20 or 15 with a wide q / k alone, 32 at 64, 16 at 32): both passes, with forward's state and
 without, against the fp32 oracle (``-m gpu``)."""
 
 import ctypes
@@ -103,3 +103,10 @@ def test_an_infinite_value_stays_infinite(h, n, dqk, dv, gpu_device):
         assert bool((x[:, :, rows, 1] == float("inf")).all())
         x[:, :, :, 1] = x_want[:, :, :, 1] = 0
         assert torch.equal(x, x_want)
+
+
+# a wide q / k alone: up to 15 segments over a v of 64 columns, 20 over a v of 128, a scan beyond (one chunk of 64 rows a segment)
+@pytest.mark.parametrize("segments,dqk,dv", [(9, 256, 64), (12, 153, 64), (15, 192, 64), (16, 256, 64), (9, 256, 128), (20, 192, 128),
+                                             (21, 256, 128)])
+def test_a_wide_q_k(segments, dqk, dv, gpu_device):
+    test_operators_that_keep_dq_causal(256 // segments, 64 * segments, dqk, dv, gpu_device)
