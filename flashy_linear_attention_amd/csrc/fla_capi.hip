@@ -2434,17 +2434,6 @@ int fla_normalised_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int6
     // (a single segment per head: 1.03 to 2.1 from N = 320 on, B H 130 ... 600)
     return N >= 2048 || (N >= 1024 && wp.D <= 64) || w >= 1.2e10 || (wp.n_seg == 1 && N > 256);
 }
-// Pairs, GPU time of the quadratic evaluation over the chunk-wise one's, B H 1 ... 400: 1.13 to 1.8 at N = 320, 1.06 to 1.9 at 384,
-// 1.3 to 2.2 at 1024, 2.2 to 4.1 at 4096; 0.54 to 0.95 up to 256 (a single chunk of 256 rows with states in memory).  Both are four
-// launches, but the chunk-wise one has two buffers more to allocate, 47 against 43 us of the host through autograd, so the line lies
-// where the quadratic kernels take about that long: 128 columns from 257 rows on, 64 from 768, 32 from 1536, or many heads.  Errors
-// against fp64 (elu + 1 features): dQ 0.77 to 0.99 of the quadratic evaluation's, O, dK and dV 0.72 to 1.0.
-int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype) {
-    if (dtype != FLA_DTYPE_BF16 || D_qk < 1 || D_v < 1 || D_qk % 8 != 0 || D_v % 8 != 0) return 0;
-    const WalkPlan wp = walk_plan(B, H, N, D_qk, D_v);
-    const double w = (double)B * (double)H * (double)N * (double)N * (double)wp.D;
-    return wp.ok && N > 256 && (wp.D == 128 || N >= (wp.D == 64 ? 768 : 1536) || w >= 1.2e9);
-}
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward) {
     if (dtype != FLA_DTYPE_BF16 || !poly_plan(B, H, N, R, D_v).ok) return 0;
     // Quadratic time over chunk-wise time, R 8 and 16, with and without the normaliser, B H 1 ... 1024, N 100 ... 4096.  Pairs,

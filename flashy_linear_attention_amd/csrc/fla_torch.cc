@@ -544,10 +544,10 @@ PyObject *py_mapped(PyObject *, PyObject *const *args, Py_ssize_t n) {
         PyErr_Clear();
         Py_RETURN_NONE;
     }
-    if (!opt.fmap && opt.normalise && !opt.chunked) {  // (normalised.py)
+    if (!opt.fmap && opt.normalise && !opt.chunked && !wants_grad(a.q, a.k, a.v)) {  // (normalised.py)
         const int dtype = a.cast ? FLA_DTYPE_BF16 : dtype_code(a.q.scalar_type());
-        opt.chunked = (wants_grad(a.q, a.k, a.v) ? fla_normalised_prefers_chunked : fla_normalised_forward_prefers_chunked)(
-                          a.q.size(0), a.q.size(1), a.q.size(2), a.q.size(3), a.v.size(3), dtype) != 0;
+        opt.chunked = fla_normalised_forward_prefers_chunked(a.q.size(0), a.q.size(1), a.q.size(2), a.q.size(3), a.v.size(3),
+                                                             dtype) != 0;
     }
     return released([&]() -> Tensor {
         if (wants_grad(a.q, a.k, a.v)) return Mapped::apply(a.q, a.k, a.v, opt.code(), opt.eps, a.cast);

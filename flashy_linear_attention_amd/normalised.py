@@ -4,8 +4,8 @@ normaliser to the caller, README.md:27-30 of the reference):
     out = LinearAttention.apply(q, k, v) / ((q * k.cumsum(-2)).sum(-1, keepdim=True) + eps)
 
 ``LinearAttentionNormalised.apply(q, k, v, eps, chunked=False)`` returns the same tensor
-(``chunked=True``: the product is evaluated chunk-wise, O(N), whatever the shape; by default
-where that is faster, ``fla_normalised_prefers_chunked``, for forward alone ``fla_normalised_forward_prefers_chunked``).  The product runs on the kernels of ``LinearAttention``;
+(``chunked=True``: the product is evaluated chunk-wise, O(N), whatever the shape; by default for
+forward alone where that is faster, ``fla_normalised_forward_prefers_chunked``).  The product runs on the kernels of ``LinearAttention``;
 the cumulative sum, the dot with q, eps and the division are one fused pass in fp32 (``fla_linear_attn_normalised_fwd``), and backward adds the
 normaliser's own gradient terms with two more fused passes instead of an autograd graph of
 elementwise kernels (``fla_linear_attn_normalised_bwd``).
@@ -35,15 +35,10 @@ def _state_buffer(lib, b: int, h: int, n: int, dqk: int, dv: int, want: bool, de
     return torch.empty(sbytes, dtype=torch.uint8, device=device) if sbytes else None
 
 
-def _prefers_chunked(q: torch.Tensor, v: torch.Tensor, grad: bool) -> bool:
+def _forward_prefers_chunked(q: torch.Tensor, v: torch.Tensor) -> bool:
     if q.dim() != 4 or v.dim() != 4 or not q.is_cuda or q.dtype != torch.bfloat16:
         return False  # (what is no call of the operator is refused by its forward)
-    name = "fla_normalised_prefers_chunked" if grad else "fla_normalised_forward_prefers_chunked"
-    return bool(_lib.query(name, *q.shape, v.shape[-1], dtype_code(q)))
-
-
-def _forward_prefers_chunked(q: torch.Tensor, v: torch.Tensor) -> bool:
-    return _prefers_chunked(q, v, False)
+    return bool(_lib.query("fla_normalised_forward_prefers_chunked", *q.shape, v.shape[-1], dtype_code(q)))
 
 
 def linear_attention_normalised_fwd(
@@ -125,7 +120,7 @@ class LinearAttentionNormalised(Function):
     def forward(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, eps: float = 1e-5,
                 chunked: bool = False) -> torch.Tensor:
         grad = any(ctx.needs_input_grad[:3])
-        chunked = bool(chunked) or _prefers_chunked(q, v, grad)
+        chunked = bool(chunked) or (not grad and _forward_prefers_chunked(q, v))
         want = chunked and grad
         out, denom, state = linear_attention_normalised_fwd(q, k, v, eps, chunked, want_state=True) if want else (
             *linear_attention_normalised_fwd(q, k, v, eps, chunked), None)

@@ -385,8 +385,6 @@ int fla_poly_attn_bwd(const void *grad_out, const void *xq, const void *xk, cons
 /* 1 where the chunk-wise evaluation (chunked != 0) of the normalised operator's forward alone is the faster one (host
  * arithmetic, measured thresholds), 0 elsewhere. */
 int fla_normalised_forward_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype);
-/* The same question for a forward + backward pair. */
-int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int dtype);
 
 /* The same operator evaluated chunk-wise (O(N): running sums of Taylor features formed inside the kernels, nothing
  * feature-wide in memory but the states at segment ends).  FLA_DTYPE_BF16 and R <= 16, D_v <= 64 only
