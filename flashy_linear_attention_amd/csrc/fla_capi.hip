@@ -451,6 +451,24 @@ WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, boo
 
 bool sums_on_load(const WalkPlan &w, int most = kSumOnLoadMost) { return w.n_seg >= 3 && w.n_seg <= most; }
 
+// Two workgroups per (b, h) on two column halves of O, on dV and dK (WalkParams::cols, roles), where they would be two segments: q and
+// k (q and dO) come from the L2 that both read through, and no totals of half of the sequence come before the walk.  `plain`: no
+// normaliser and no feature map.
+//   128 columns, two segments -> this.  Forward + backward: B H 128, N 1024 114 / 102 us, N 2048 219 / 204, N 4096 433 / 398, N 8192
+//   857 / 819; B H 112, N 4096 387 / 375; B H 104, N 3072 279 / 268; B H 96, N 1024 98 / 90, N 4096 355 / 350; 72 and 96 columns, B H 88
+//   and 96, N 2048 147 to 150 / 151 to 153; 80 columns, B H 128, N 4096 307 / 316, 96 columns, N 3008 251 / 246.  (dQ's walk as well: B H 128, N 4096 408 -> 422: it starts from what forward left and has no
+//   totals to save.)
+//   Forward alone: B H 88 ... 128, N 1024 31.4 to 36.0 / 27.6 to 29.8, N 2048 50.4 to 64.8 / 49.1 to 57.3, N 3072 77 to 96 / 83 to 98; N 4096
+//   B H 104 107 / 116, B H 120 124.4 / 123.6, B H 128 132 / 127; N 8192 B H 112 236 / 232, B H 128 261 / 247 (the two fall out of step on
+//   long sequences, and each then reads all of q and k from memory).
+bool walk_by_columns(const WalkPlan &w, int64_t bh, int64_t N, int64_t dqk, int64_t dv, bool plain) {
+    return plain && w.ok && w.split && dqk > 64 && dv > 64 && w.n_seg == 2 && (bh > 96 || N <= 1024) &&
+           (N <= 2048 || (dqk >= 96 && dv >= 96));
+}
+bool forward_by_columns(const WalkPlan &w, int64_t bh, int64_t N, int64_t dqk, int64_t dv, bool plain) {
+    return walk_by_columns(w, bh, N, dqk, dv, plain) && (N <= 2048 || (N >= 4096 && bh > 112));
+}
+
 // totals of Y^T Z over the walk's segments into `work`, then the segments' entry states: their sums
 // over the segments before (reverse == 0) or after (reverse != 0), written to `entry` (null: over
 // the totals in `work`).  Returns where the entry states are.
@@ -1016,6 +1034,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         (!fmap || fla::fast_path_ok(make_params(mapped[0], mapped[1], v, o, B, H, N, dqk, dv, 0)))) {
         // the segments' entry states; with a feature map the same kernel maps xk as it loads it and
         // writes phi(xk), which the walk then reads (so it runs for a single segment as well)
+        const bool by_columns = forward_by_columns(wp, B * H, N, dqk, dv, !fmap && !nx);
         const bool need_totals = wp.n_seg > 1 || fmap;
         // D = 128: the entry states (and the state after the last chunk) are what backward gets, so the scan writes
         // them to state_out (the totals themselves are computed there, and no workspace is used);
@@ -1031,7 +1050,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         if (state_out && reinterpret_cast<uintptr_t>(state_out) % 16 != 0) return FLA_ERR_WORKSPACE;
         hipStream_t s = static_cast<hipStream_t>(stream);
         const float *entry = nullptr;
-        if (need_totals)
+        if (need_totals && !by_columns)
             if (int rc = walk_entry_states(wp, k, v, B, H, N, dqk, dv, dtype, 0,
                                            in_state && !sum_on_load ? state_out : workspace,
                                            in_state && !sum_on_load ? static_cast<float *>(state_out) : nullptr, &entry, s,
@@ -1053,6 +1072,10 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = wp.n_seg > 1 ? entry : nullptr, w.saved = in_state ? nullptr : state_out;
         if (sum_on_load) w.init_is_totals = 1, w.entry_out = in_state ? static_cast<float *>(state_out) : nullptr;
+        if (by_columns) {  // (the state buffer is that of two segments all the same)
+            w.cols = 1, w.n_seg = 1, w.seg_chunks = w.n_chunks, w.init = nullptr;
+            w.mid_out = in_state ? static_cast<float *>(state_out) : nullptr, w.mid_chunk = (int32_t)wp.seg_chunks;
+        }
         if (any && wp.split) {
             w.any_rows = 1, w.rows_o = rows_out(*any->o, any->wv), w.o = nullptr, any->done = true;
         }
@@ -1222,6 +1245,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         // dQ's walk adds up the segments' totals of Q^T dO on its way (WalkParams::r_totals, figures there; bf16 alone: an fp16 walk's
         // scale has no place in the LDS beside two sets of four tiles and the state)
         const bool dq_walk_sums = !one_walk && !nx && !fmap && wp.n_seg > 2 && dtype == FLA_DTYPE_BF16 && dqk > 64;
+        const bool by_columns = !one_walk && walk_by_columns(wp, B * H, N, dqk, dv, !fmap && !nx);
         if (wp.n_seg > 1) {
             if (!state_in) {
                 const float *fwd_entry = nullptr;
@@ -1230,7 +1254,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                     return rc;
                 state_in = fwd_entry;
             }
-            if (!nx && !dq_walk_sums)
+            if (!nx && !dq_walk_sums && !by_columns)
                 if (int rc = walk_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, workspace, nullptr, &entry, s, 0, nullptr,
                                                nullptr, rev_sums_on_load))
                     return rc;
@@ -1297,6 +1321,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         r.n_chunks = (int32_t)wp.n_chunks, r.seg_chunks = (int32_t)wp.seg_chunks, r.n_seg = (int32_t)wp.n_seg;
         r.init = entry, r.fmap = fmap;  // (dK: the slope from phi(xk) in the K tile)
         r.init_is_totals = rev_sums_on_load, r.wide_out = wide_out;
+        if (by_columns) r.roles = 1, r.n_seg = 1, r.seg_chunks = r.n_chunks, r.init = nullptr;
         if (nx) r.dn = nx->dn, r.rc = wp.n_seg > 1 ? rcv : nullptr;  // dK's terms
         if (any) results_to_rows(r, *any);
         return fla::walk_dkdv(dtype, wp.D, r, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;

@@ -172,6 +172,13 @@ struct WalkParams {
     // q / k with half y (2) or half 1 - y (3) of v, so that the two parts of a launch write different columns.
     // The states of (q / k half i, v half j) are matrices (2 j + i) BH .. of every state buffer.
     int32_t quad, wv2;
+    // D = 128, plain, both sides above 64 columns, one segment per (b, h): two workgroups per (b, h) in place of two segments
+    // (grid y), so that no totals come before the walk.  cols (walk_fwd_kernel; kernels of their own: COLS): grid y takes columns
+    // 64 y .. of v and of the result; q and k are read by both, within one XCD, at the same time.  The state at the entry of chunk
+    // mid_chunk goes to mid_out (null: nowhere) in the form of two segments' partial sums, total_out as always.  roles
+    // (walk_dkdv_kernel, ROLES): dV is formed by grid y = 0, dK by 1, each with a copy of R; q and dO are read by both.
+    int32_t cols, roles, mid_chunk;
+    float *mid_out;
 };
 
 template <int D>
@@ -1194,7 +1201,7 @@ template <typename T, int NORM, bool FM>
 constexpr bool walk_fwd_scaled = std::is_same<T, _Float16>::value && NORM == 0 && !FM;
 
 template <typename T, int D, bool DOUBLE, int NORM, bool FM, int NQ = D / 32, int NV = D / 32, bool WIDE = false, bool ROWS = false,
-          bool RSUM = false>
+          bool RSUM = false, bool COLS = false>
 __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1204,6 +1211,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     static_assert(NORM == 0 || (NQ == W::DB && NV == W::DB), "the normaliser's variants are built for full widths");
     constexpr int SETS = DOUBLE ? 2 : 1, TPS = RSUM ? 4 : 3;  // (tiles per set)
     static_assert(!RSUM || (DOUBLE && NORM == 0 && !FM), "the plain dQ walk");
+    static_assert(!COLS || (DOUBLE && NORM == 0 && !FM && !RSUM && NQ == 4 && NV == 2), "64 of the columns of a plain walk");
     using RB = WalkExt<D, D / 32, NQ>;  // (RSUM: the total's blocks -- q's columns are v's here, dO's are q's)
     constexpr bool SCALED = walk_fwd_scaled<T, NORM, FM>;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -1221,13 +1229,15 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
     const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
     const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
-    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h;
+    const int col0 = COLS ? 64 * (int)blockIdx.y : 0;
+    const int wv = !COLS ? p.wv : p.wv - col0 < 64 ? p.wv - col0 : 64;
+    const T *V = static_cast<const T *>(p.v) + b * p.vs_b + h * p.vs_h + col0;
     const int qs2 = (int)p.qs_n * 2, ks2 = (int)p.ks_n * 2, vs2 = (int)p.vs_n * 2;
     const u32x4 rq = make_rsrc(Q, (uint32_t)((N - 1) * qs2 + p.wqk * 2));
     const u32x4 rk = make_rsrc(K, (uint32_t)((N - 1) * ks2 + p.wqk * 2));
-    const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + p.wv * 2));
-    const WalkResult ro(p.o, b * p.os_b + h * p.os_h, p.os_n, p.wv, N, WIDE);
-    const WalkAnyRows<T> ao(p.rows_o, b, h, 0, p.rows_o.width, N);
+    const u32x4 rv = make_rsrc(V, (uint32_t)((N - 1) * vs2 + wv * 2));
+    const WalkResult ro(p.o, b * p.os_b + h * p.os_h + col0, p.os_n, wv, N, WIDE);
+    const WalkAnyRows<T> ao(p.rows_o, b, h, col0, !COLS ? p.rows_o.width : p.rows_o.width - col0 < 64 ? p.rows_o.width - col0 : 64, N);
 
     // (RSUM: the first segment's total is under no sum of the reverse walk)
     const bool rsum = RSUM && sl.seg > 0;
@@ -1306,7 +1316,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         const uint32_t base = lds0 + buf * TPS * W::TILE;
         walk_load_tile<D>(rq, base, c * W::C, qs2, p.wqk, wave, lane);
         walk_load_tile<D>(rk, base + W::TILE, c * W::C, ks2, p.wqk, wave, lane);
-        walk_load_tile<D>(rv, base + 2 * W::TILE, c * W::C, vs2, p.wv, wave, lane);
+        walk_load_tile<D>(rv, base + 2 * W::TILE, c * W::C, vs2, wv, wave, lane);
         if constexpr (RSUM)
             if (rsum) walk_load_tile<D>(rr, base + 3 * W::TILE, c * W::C, rs2, p.wv, wave, lane);
         const uint32_t xbase = lds0 + SETS * 3 * W::TILE + W::STATE + buf * W::VEC;
@@ -1414,8 +1424,23 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         if constexpr (ROWS)
             ao.template store<D, OB::PER>(row, g, db0, acc);
         else
-            walk_store<T, D, OB::PER>(ro.rs, ro.stride, p.wv, row, g, db0, acc, 0, nullptr, 0, WIDE);
+            walk_store<T, D, OB::PER>(ro.rs, ro.stride, wv, row, g, db0, acc, 0, nullptr, 0, WIDE);
         walk_update<T, D, B>(tk, tv, wave, lane, st);
+        if constexpr (COLS) {
+            if (p.mid_out && c + 1 == p.mid_chunk) {  // (as the partial sums of two segments: this, and zeros)
+                const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+                    p.mid_out + (int64_t)sl.bh * 2 * (D * D), 0, 2 * D * D * 4, 0x00020000);
+#pragma unroll
+                for (int i = 0; i < B::SLOTS; ++i)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v) {
+                        const float x = st[i][v];
+                        const int at = (32 * B::dbk(wave, i) + 8 * (v / 4) + 4 * g + (v % 4)) * D + col0 + 32 * B::eb(wave) + l32;
+                        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, x), rs, (uint32_t)(at * 4), 0, 0);
+                        __builtin_amdgcn_raw_buffer_store_b32(0u, rs, (uint32_t)(at * 4), D * D * 4, 0);
+                    }
+            }
+        }
         if constexpr (RSUM)
             if (rsum) walk_update<T, D, RB>(tv + W::TILE, tq, wave, lane, rt);
         if constexpr (SCALED) walk_state_max<D, B>(smax, wave, lane, st);
@@ -1451,7 +1476,7 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
         return;
     }
     if (p.total_out && sl.c_hi == p.n_chunks) {  // the state after the last chunk, for the backward walks
-        float *out = p.total_out + (int64_t)sl.bh * (D * D);
+        float *out = p.total_out + (int64_t)sl.bh * (D * D) + col0;
 #pragma unroll
         for (int i = 0; i < B::SLOTS; ++i)
             if (B::valid(wave, i)) {
@@ -1742,7 +1767,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 // D = 128, so the chunk's dn comes as ordinary loads, a chunk ahead, in the order in which the scores' registers take it, and
 // rc is carried in registers: a wave adds up its own output columns, in the order of an MFMA's A rows, and one MFMA
 // per 32 columns adds rc to the result (walk_split3).
-template <typename T, int D, bool NORM, int NQ = D / 32, int NV = D / 32, bool WIDE = false, bool ROWS = false>
+template <typename T, int D, bool NORM, int NQ = D / 32, int NV = D / 32, bool WIDE = false, bool ROWS = false, bool ROLES = false>
 __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1757,8 +1782,11 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
     using OQ = WalkOut<D, NQ>;      // dK as q and k
     static_assert(!NORM || (NQ == W::DB && NV == W::DB), "the normaliser's variant is built for full widths");
     const int rb = W::NCH == 1 ? wave : wave % W::NRB, db0 = OQ::db0(wave);  // (db0: dK's, and rc's columns)
+    static_assert(!ROLES || !NORM, "one result of a plain walk");
     const WalkSlice sl = walk_slice(p);
     if (!sl.valid) return;
+    const bool with_dv = !ROLES || blockIdx.y == 0, with_dk = !ROLES || blockIdx.y != 0;
+    constexpr int n_tiles = ROLES ? 3 : 4;
     const int b = sl.bh / p.H, h = sl.bh - b * p.H, N = p.N;
     const T *Q = static_cast<const T *>(p.q) + b * p.qs_b + h * p.qs_h;
     const T *K = static_cast<const T *>(p.k) + b * p.ks_b + h * p.ks_h;
@@ -1781,8 +1809,8 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         const uint32_t base = lds0 + buf * 4 * W::TILE;
         const int row0 = c * W::C;
         walk_load_tile<D>(rq, base, row0, qs2, p.wqk, wave, lane);
-        walk_load_tile<D>(rk, base + W::TILE, row0, ks2, p.wqk, wave, lane);
-        walk_load_tile<D>(rv, base + 2 * W::TILE, row0, vs2, p.wv, wave, lane);
+        if (with_dv) walk_load_tile<D>(rk, base + W::TILE, row0, ks2, p.wqk, wave, lane);
+        if (with_dk) walk_load_tile<D>(rv, base + 2 * W::TILE, row0, vs2, p.wv, wave, lane);
         walk_load_tile<D>(rg, base + 3 * W::TILE, row0, gs2, p.wv, wave, lane);
     };
     static_assert(!NORM || W::C == 64, "eight groups of four dn values are a chunk of 64 rows");
@@ -1843,7 +1871,7 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         // this wave's loads of chunk c have landed when at most the loads issued after them are
         // outstanding (the stores of the previous chunk were issued before those)
         if (more)
-            wait_vm<4 * W::NI>();
+            wait_vm<n_tiles * W::NI>();
         else
             wait_vm<0>();
         if constexpr (NORM) {
@@ -1855,32 +1883,36 @@ __global__ __launch_bounds__(256, 1) void walk_dkdv_kernel(const WalkParams p) {
         const int row = c * W::C + 32 * rb + l32;
         const bool later = c + 1 < p.n_chunks;  // chunks after this one exist: R is not identically zero
         f32x16 acc[W::DBW];
-        // dV = upper(K Q^T) dO + K R: A operand R^T[v index][q/k index] = the LDS copy as it is
-        walk_product<T, D, true, 0, B::KQ, NV>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
-            return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
-        }, acc);
-        if constexpr (ROWS)
-            adv.template store<D, OV::PER>(row, g, OV::db0(wave), acc);
-        else
-            walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, p.wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
-        // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
-        if constexpr (NORM) {
-            walk_product<T, D, true, 3>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
-                return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
-            }, acc, nullptr, nullptr, [&](int s, int a4) -> f32x4 { return s == 0 ? dnv[a4] : dnv[4 + a4]; });
-            const Mma<__bf16>::V8 ones = walk_ones3(g);
-#pragma unroll
-            for (int i = 0; i < W::DBW; ++i)
-                acc[i] = Mma<__bf16>::mma(walk_split3(rrun[i] + __shfl_xor(rrun[i], 32, 64), g), ones, acc[i]);
-        } else {
-            walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
-                return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
+        if (with_dv) {
+            // dV = upper(K Q^T) dO + K R: A operand R^T[v index][q/k index] = the LDS copy as it is
+            walk_product<T, D, true, 0, B::KQ, NV>(tk, tq, tg, wave, lane, later, [&](int db, int kc) -> V8 {
+                return walk_row_frag<T, D>(tl, 32 * db + walk_e_lane(l32), kc, g);
             }, acc);
+            if constexpr (ROWS)
+                adv.template store<D, OV::PER>(row, g, OV::db0(wave), acc);
+            else
+                walk_store<T, D, OV::PER>(rdv.rs, rdv.stride, p.wv, row, g, OV::db0(wave), acc, 0, nullptr, 0, WIDE);
         }
-        if constexpr (ROWS)
-            adk.template store<D, OQ::PER>(row, g, db0, acc);
-        else
-            walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, p.wqk, row, g, db0, acc, p.fmap, tk, 32 * rb + l32, WIDE);
+        if (with_dk) {
+            // dK = upper(V dO^T) Q + V R^T: A operand R[q/k index][v index] = the LDS copy read transposed
+            if constexpr (NORM) {
+                walk_product<T, D, true, 3>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
+                    return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
+                }, acc, nullptr, nullptr, [&](int s, int a4) -> f32x4 { return s == 0 ? dnv[a4] : dnv[4 + a4]; });
+                const Mma<__bf16>::V8 ones = walk_ones3(g);
+#pragma unroll
+                for (int i = 0; i < W::DBW; ++i)
+                    acc[i] = Mma<__bf16>::mma(walk_split3(rrun[i] + __shfl_xor(rrun[i], 32, 64), g), ones, acc[i]);
+            } else {
+                walk_product<T, D, true, 0, B::KV, NQ>(tv, tg, tq, wave, lane, later, [&](int db, int kc) -> V8 {
+                    return walk_col_frag_perm<T, D>(tl, 16 * kc, db, lane, true);
+                }, acc);
+            }
+            if constexpr (ROWS)
+                adk.template store<D, OQ::PER>(row, g, db0, acc);
+            else
+                walk_store<T, D, OQ::PER>(rdk.rs, rdk.stride, p.wqk, row, g, db0, acc, p.fmap, tk, 32 * rb + l32, WIDE);
+        }
         walk_update<T, D, B>(tq, tg, wave, lane, st);
         if constexpr (NORM) {  // rc += this chunk's dn_i q_i
             static_for<0, W::C / 16>([&](auto j) {
@@ -2833,6 +2865,13 @@ hipError_t launch_walk_fwd(const WalkParams &p, hipStream_t stream) {
     }
     if constexpr (!ROWS)
         if (fm) return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, true, NB, NB, WIDE>>(grid, smem, p, stream);
+    if (p.cols) {
+        if constexpr (D == 128) {
+            if (p.denom || p.dn || fm || p.r_totals || p.n_seg != 1 || p.init || p.wqk <= 64 || p.wv <= 64) return hipErrorInvalidValue;
+            return launch_walk_kernel<walk_fwd_kernel<T, D, kDouble, 0, false, 4, 2, WIDE, ROWS, false, true>>(grid, smem, p, stream, 2);
+        }
+        return hipErrorNotSupported;
+    }
     if (p.r_totals) {
         if constexpr (D == 128 && std::is_same<T, __bf16>::value) {
             constexpr int smem_r = 8 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
@@ -2923,11 +2962,16 @@ hipError_t launch_walk_dkdv(const WalkParams &p, hipStream_t stream) {
         if (p.dn || p.fmap || !walk_rows_ok(p.rows_dk, p.wqk) || !walk_rows_ok(p.rows_dv, p.wv)) return hipErrorInvalidValue;
     } else if (p.dn) {
         if (p.n_seg > 1 && !p.rc) return hipErrorInvalidValue;
+        if (p.roles) return hipErrorInvalidValue;
         constexpr auto kern = walk_dkdv_kernel<T, D, true, NB, NB, WIDE>;
         if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;
         return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem, stream, p);
     }
     if constexpr (D == 128) {
+        if (p.roles) {
+            if (p.fmap || p.n_seg != 1 || p.init || p.wqk <= 64 || p.wv <= 64) return hipErrorInvalidValue;
+            return launch_walk_kernel<walk_dkdv_kernel<T, D, false, NB, NB, WIDE, ROWS, true>>(grid, smem, p, stream, 2);
+        }
         if (!p.fmap && p.wqk > 64 && p.wv <= 64) {
             constexpr auto kern = walk_dkdv_kernel<T, D, false, 4, 2, WIDE, ROWS>;
             if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;

@@ -71,7 +71,7 @@ FLA_FIELD(xtotal) FLA_FIELD(accumulate)
     FLA_FIELD(wqk2) FLA_FIELD(init2) FLA_FIELD(total_out2) FLA_FIELD(xinit2) FLA_FIELD(xtotal2)
     FLA_FIELD(init_is_totals) FLA_FIELD(entry_out) FLA_FIELD(entry_out2) FLA_FIELD(quad) FLA_FIELD(wv2) FLA_FIELD(vsum) FLA_FIELD(zc_out)
 FLA_FIELD(wide_out) FLA_FIELD(any_rows) FLA_FIELD(r_q) FLA_FIELD(rs_b) FLA_FIELD(rs_h) FLA_FIELD(rs_n) FLA_FIELD(r_frags)
-FLA_FIELD(r_totals)
+FLA_FIELD(r_totals) FLA_FIELD(cols) FLA_FIELD(roles) FLA_FIELD(mid_chunk) FLA_FIELD(mid_out)
     trace_fields(r, arg, pre + "rows_o.", p.rows_o), trace_fields(r, arg, pre + "rows_dq.", p.rows_dq);
     trace_fields(r, arg, pre + "rows_dk.", p.rows_dk), trace_fields(r, arg, pre + "rows_dv.", p.rows_dv);
 FLA_FIELDS_END

@@ -798,6 +798,12 @@ def model_walk(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats) -> None:
         arena.require("forward's final states", p["xtotal"], p["xtotal"] + BH * E)
     if p["total_out"]:
         arena.require("final states", p["total_out"], p["total_out"] + BH * E)
+    if p["cols"] or p["roles"]:  # (grid y: the column halves of one result, or one result each; one segment)
+        assert l.kernel == ("walk_fwd_kernel" if p["cols"] else "walk_dkdv_kernel") and D == 128 and n_seg == 1 and l.grid[1] == 2
+        assert p["wqk"] > 64 and p["wv"] > 64 and not p["init"] and not p["fmap"] and not p["denom"] and not p["dn"]
+    if p["mid_out"]:  # (in the form of two segments' partial sums)
+        assert p["cols"] and 0 < p["mid_chunk"] < n_chunks
+        arena.require("the state at the middle", p["mid_out"], p["mid_out"] + BH * 2 * E)
     if p["saved"]:
         arena.require("per-chunk states", p["saved"], p["saved"] + BH * n_chunks * D * D * 2)
     for nm, count in (("zc", n_chunks), ("zc_out", n_chunks), ("rc", n_seg), ("vsum", n_seg)):
