@@ -586,8 +586,9 @@ int walk_chunk_vectors(const WalkPlan &wp, const View &k, int64_t width, float *
 // segments).  Returns where the entry states are.
 int walk_grad_entry_states(const WalkPlan &w, const View &q, const View &dout, const WalkNorm &nx, int64_t B, int64_t H, int64_t N,
                            int64_t dqk, int64_t dv, int dtype, void *work, float *rc_totals, const float **where, bool totals_only,
-                           hipStream_t s) {
+                           hipStream_t s, bool keep_g = false) {
     fla::WalkGradParams gp{};
+    gp.keep_g = keep_g;
     gp.q = q.ptr, gp.qs_b = q.strides[0], gp.qs_h = q.strides[1], gp.qs_n = q.strides[2];
     gp.go = nx.go->ptr, gp.gs_b = nx.go->strides[0], gp.gs_h = nx.go->strides[1], gp.gs_n = nx.go->strides[2];
     gp.o = nx.out->ptr, gp.os_b = nx.out->strides[0], gp.os_h = nx.out->strides[1], gp.os_n = nx.out->strides[2];
@@ -1335,20 +1336,24 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         const float *entry = nullptr;
         if (wp.n_seg > 1 && !nx)
             if (int rc = walk_entry_states(wp, q, go, B, H, N, dqk, dv, dtype, 1, workspace, nullptr, &entry, s)) return rc;
+        const View *gv = &go;
         fla::WalkParams w{};
         if (nx) {
             float *const rcv = reinterpret_cast<float *>(static_cast<char *>(nx->vec) + walk_vec_bytes(B, H, N, dqk, dv));
-            if (int rc = walk_grad_entry_states(wp, q, go, *nx, B, H, N, dqk, dv, dtype, workspace, rcv, &entry, false, s)) return rc;
+            // (g as aligned rows, as the walk's tile loads ask for: dO is formed where it is used)
+            const bool keep_g = nx->vec16 && fla::fast_path_ok(make_params(q, k, *nx->go, dvv, B, H, N, dqk, dv, 0));
+            if (int rc = walk_grad_entry_states(wp, q, go, *nx, B, H, N, dqk, dv, dtype, workspace, rcv, &entry, false, s, keep_g)) return rc;
+            gv = keep_g ? nx->go : &go, w.gn = keep_g ? nx->n : nullptr;
             w.dn = nx->dn, w.zc = zc_saved, w.rc = wp.n_seg > 1 ? rcv : nullptr;
             nx->fused = true;
         }
         w.fmap = fmap;  // q, k hold phi(x): the slopes come from the LDS tiles
-        w.q = q.ptr, w.k = k.ptr, w.v = v.ptr, w.go = go.ptr;
+        w.q = q.ptr, w.k = k.ptr, w.v = v.ptr, w.go = gv->ptr;
         w.dq = const_cast<void *>(dq.ptr), w.dk = const_cast<void *>(dk.ptr), w.dv = const_cast<void *>(dvv.ptr);
         w.qs_b = q.strides[0], w.qs_h = q.strides[1], w.qs_n = q.strides[2];
         w.ks_b = k.strides[0], w.ks_h = k.strides[1], w.ks_n = k.strides[2];
         w.vs_b = v.strides[0], w.vs_h = v.strides[1], w.vs_n = v.strides[2];
-        w.gs_b = go.strides[0], w.gs_h = go.strides[1], w.gs_n = go.strides[2];
+        w.gs_b = gv->strides[0], w.gs_h = gv->strides[1], w.gs_n = gv->strides[2];
         w.dqs_b = dq.strides[0], w.dqs_h = dq.strides[1], w.dqs_n = dq.strides[2];
         w.dks_b = dk.strides[0], w.dks_h = dk.strides[1], w.dks_n = dk.strides[2];
         w.dvs_b = dvv.strides[0], w.dvs_h = dvv.strides[1], w.dvs_n = dvv.strides[2];

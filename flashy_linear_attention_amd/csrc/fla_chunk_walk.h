@@ -126,6 +126,10 @@ struct WalkParams {
     float *zc_out;      // as zc
     const float *dn;  // fp32 [BH][N]
     const float *rc;  // fp32 [BH][n_seg][D], slots as those of `init`
+    // walk_bwd_kernel: go holds g, and dO = g / n is formed in its tile as it lands (null: go holds dO).  An operand less for
+    // walk_grad_totals_kernel to write: B H 64, N 4096, D 64 that kernel 24.8 -> 19.4 us, the walk 57.3 to 59.9 (55.2 from 54.4 without a
+    // feature map); forward + backward with a feature map 151 -> 145, B H 128 283 -> 274, without one B H 512, N 1024 228 -> 221
+    const float *gn;  // n, fp32 [BH][N]
     // Forward, D = 128: where the state after the last chunk of every (b, h) goes, fp32 [BH][D][D]
     // ([q/k index][v index]), or null.  walk_bwd_rev_kernel: that buffer (xtotal) and forward's entry
     // states (xinit, the layout of `init`, not transposed; may be null with a single segment).
@@ -1695,12 +1699,31 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
         if constexpr (NORM) {  // the normaliser's terms: zc of this chunk and its rows of dn
             walk_load_vec<D>(p.zc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase, lane);
             walk_load_rows<D>(p.dn + (int64_t)sl.bh * N, row0, N, xbase + 2048, lane);
+            if (p.gn) walk_load_rows<D>(p.gn + (int64_t)sl.bh * N, row0, N, xbase + 2560, lane);
         }
         if (c > 0)
             walk_load_state_copy<D>(static_cast<const unsigned char *>(p.saved) + at * W::STATE, NORM ? lds0 + 4 * W::TILE : xbase, wave,
                                     lane);
         wait_vm<0>();
         __syncthreads();
+        if constexpr (NORM) {
+            if (p.gn) {  // dO = g / n, as walk_grad_totals_kernel rounds it
+                const float *vn = vd + 128;
+#pragma unroll
+                for (int v = 0; v < W::C * W::CR / 256; ++v) {
+                    const int u = tid + 256 * v, r = u / W::CR, pos = u % W::CR;
+                    if (row0 + r < N && (pos ^ walk_swizzle<W::CR>(r)) * 8 < p.wv) {
+                        u32x4 *ptr = reinterpret_cast<u32x4 *>(tg + r * W::RB + (pos << 4));
+                        V8 x = __builtin_bit_cast(V8, *ptr);
+                        const float inv = 1.0f / vn[r];
+#pragma unroll
+                        for (int e = 0; e < 8; ++e) x[e] = static_cast<T>(static_cast<float>(x[e]) * inv);
+                        *ptr = __builtin_bit_cast(u32x4, x);
+                    }
+                }
+                __syncthreads();
+            }
+        }
         const int row = row0 + 32 * wave + l32;
         const bool later = c + 1 < p.n_chunks;  // chunks after this one exist: R is not identically zero
         f32x16 acc[W::DBW];
@@ -2601,6 +2624,7 @@ struct WalkGradParams {
     float *totals, *rsum;      // [BH][n_seg] states and vectors in the slots the walks read (two segments: partial sums of the
                                // second one's in both; the first one's stay unwritten otherwise); null with a single segment
     int32_t frags;             // WalkTotalsParams::frags
+    int32_t keep_g;            // dO is formed again by the walk behind (WalkParams::gn) and not written
 };
 
 // Steps on their way: what a step needs is requested DEPTH steps ahead -- one where two workgroups share a CU, two at D = 128,
@@ -2711,7 +2735,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void walk_grad_totals_kernel
             *reinterpret_cast<u32x4 *>(tg + r * W::RB + (((tid % W::CR) ^ walk_swizzle<W::CR>(r)) << 4)) = w;
             if (tid % W::CR == 0) vdn[r] = ok ? -dot * inv : 0.f;
             if (ok) {
-                if (col < p.wv) *reinterpret_cast<u32x4 *>(dO + (int64_t)row * p.wv + col) = w;
+                if (col < p.wv && !p.keep_g) *reinterpret_cast<u32x4 *>(dO + (int64_t)row * p.wv + col) = w;
                 if (tid % W::CR == 0) dn[row] = -dot * inv;
             }
         }

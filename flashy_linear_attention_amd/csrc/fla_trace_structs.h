@@ -71,7 +71,7 @@ FLA_FIELD(xtotal) FLA_FIELD(accumulate)
     FLA_FIELD(wqk2) FLA_FIELD(init2) FLA_FIELD(total_out2) FLA_FIELD(xinit2) FLA_FIELD(xtotal2)
     FLA_FIELD(init_is_totals) FLA_FIELD(entry_out) FLA_FIELD(entry_out2) FLA_FIELD(quad) FLA_FIELD(wv2) FLA_FIELD(vsum) FLA_FIELD(zc_out)
 FLA_FIELD(wide_out) FLA_FIELD(any_rows) FLA_FIELD(r_q) FLA_FIELD(rs_b) FLA_FIELD(rs_h) FLA_FIELD(rs_n) FLA_FIELD(r_frags)
-FLA_FIELD(r_totals) FLA_FIELD(cols) FLA_FIELD(roles) FLA_FIELD(mid_chunk) FLA_FIELD(mid_out)
+FLA_FIELD(r_totals) FLA_FIELD(cols) FLA_FIELD(roles) FLA_FIELD(mid_chunk) FLA_FIELD(mid_out) FLA_FIELD(gn)
     trace_fields(r, arg, pre + "rows_o.", p.rows_o), trace_fields(r, arg, pre + "rows_dq.", p.rows_dq);
     trace_fields(r, arg, pre + "rows_dk.", p.rows_dk), trace_fields(r, arg, pre + "rows_dv.", p.rows_dv);
 FLA_FIELDS_END
@@ -93,7 +93,7 @@ FLA_FIELDS_BEGIN(WalkGradParams)
 FLA_FIELD(q) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(qs_b) FLA_FIELD(qs_h) FLA_FIELD(qs_n) FLA_FIELD(gs_b) FLA_FIELD(gs_h)
 FLA_FIELD(gs_n) FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n) FLA_FIELD(denom) FLA_FIELD(dout) FLA_FIELD(dn) FLA_FIELD(H)
 FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(wqk) FLA_FIELD(wv) FLA_FIELD(vec) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks)
-FLA_FIELD(n_seg) FLA_FIELD(totals) FLA_FIELD(rsum) FLA_FIELD(frags)
+FLA_FIELD(n_seg) FLA_FIELD(totals) FLA_FIELD(rsum) FLA_FIELD(frags) FLA_FIELD(keep_g)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(ChunkStateParams)
