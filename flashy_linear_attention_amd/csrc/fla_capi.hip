@@ -2076,7 +2076,12 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
     w.dv = const_cast<void *>(dvv.ptr), w.dvs_b = dvv.strides[0], w.dvs_h = dvv.strides[1], w.dvs_n = dvv.strides[2];
     w.denom = const_cast<float *>(denom), w.entries = pl.n_seg > 1 ? static_cast<float *>(const_cast<void *>(state_in)) : nullptr;
     hipStream_t s = static_cast<hipStream_t>(stream);
-    if (int rc = poly_entries(pl, w, true, workspace, s)) return rc;
+    // (with two segments half of the workgroups would have the totals' work beside dq)
+    if (pl.n_seg >= 3 && pl.n_seg <= kSumOnLoadPoly) {
+        w.totals = static_cast<float *>(workspace), w.sum_entries = w.u_totals = 1;
+    } else if (int rc = poly_entries(pl, w, true, workspace, s)) {
+        return rc;
+    }
     return fla::poly_walk(w, true, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
 }
 

@@ -29,8 +29,8 @@
 // into segments and the forms of their entry states are the walk kernels' (fla_chunk_walk.h).  Backward is a walk in
 // forward direction for dq, from the entry states forward formed, and one in reverse for dk and dv, so that nothing of a
 // row reaches the dq of the chunks before it.
-// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 208 us this way (kernels
-// under the profiler 21 totals, 53 forward, 29 totals, 53 dq, 74 dk and dv).  With the pairs taken by blocks of eight columns -- 209
+// Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 200 us this way (kernels
+// under the profiler 21 totals, 53 forward, 73 dq with the reverse walk's totals, 74 dk and dv).  With the pairs taken by blocks of eight columns -- 209
 // features in seven blocks of 32 -- and a barrier more per chunk 239 us.  With T for dq going backwards, by subtraction, in the reverse walk
 // 228 us, but a late row that is infinite, NaN or huge spoiled dq before it; with feature rows rounded to one bf16 number on
 // both sides as well, from tiles of them in LDS, 200 us, and errors up to 1.28 times the quadratic kernels'.
@@ -58,6 +58,11 @@ struct PolyWalkParams {
                          // T (forward) / U (backward); null with a single segment
     int32_t sum_entries;
     float *entries;      // T before every segment but the first: written by forward (null: nowhere), read by dq's walk
+    // dq's walk (sum_entries, three segments or more: a kernel of its own) adds up its segment's total of U beside dq and writes it to
+    // totals for the walk behind -- g and dn are in LDS already.  Forward + backward, a totals kernel in front -> this:
+    // B 4 H 16 N 4096 211 -> 200 us; B H 16, N 4096 83.7 -> 77.1, N 16384 219 -> 210; B H 80, N 4096 268 -> 258; 8 over 32 columns, B H 24,
+    // N 4096 112.9 -> 107.4
+    int32_t u_totals;
 };
 
 // Feature order: groups of eight.  Groups 0 .. 15: x_a x_b with a = 8h + j and b = (a + d) % 16 for d = 0 .. 7, h = 0, 1 (group
@@ -85,7 +90,7 @@ struct PolyLds {  // byte offsets
                          fSum = fZ + Z, fTotal = fSum + 2 * C * 4;
     // dq (the exchange: sixteen floats a row)
     static constexpr int qQ = 0, qK = qQ + XT, qKt = qK + XT, qV = qKt + XTR, qG = qV + VT, qS = qG + VT, qEx = qS + ST,
-                         qZ = qEx + C * 64, qDn = qZ + Z, qTotal = qDn + DN;
+                         qZ = qEx + C * 64, qDn = qZ + Z, qTotal = qDn + DN, qQt = qTotal, qTotalSums = qQt + XTR;
     // dk, dv
     static constexpr int kQ = 0, kQt = kQ + XT, kK = kQt + XTR, kV = kK + XT, kG = kV + VT, kU = kG + VT, kY = kU + ST,
                          kDn = kY + Z, kEx = kDn + DN, kTotal = kEx + EX;
@@ -289,6 +294,9 @@ struct PolyState {
     }
     // ten blocks on eight waves, two waves to a SIMD: the waves of the row blocks with the least other work take two
     __device__ __forceinline__ void clear_lower(int wave) { clear(wave, wave < 2 ? 8 + wave : -1); }
+    // (a second state beside one of clear_lower: on the other two SIMDs.  Waves 4 and 5, on the first two again: B 5 H 16 N 4096 270 us in
+    // place of 264)
+    __device__ __forceinline__ void clear_beside_lower(int wave) { clear(wave, wave == 2 || wave == 3 ? 6 + wave : -1); }
     __device__ __forceinline__ void clear_upper(int wave) {
         clear(wave < 4 ? 2 * wave : wave >= 6 ? wave + 2 : -1, wave < 4 ? 2 * wave + 1 : -1);
     }
@@ -910,7 +918,7 @@ __device__ __forceinline__ void poly_contract(const unsigned char *S, const floa
 
 // dq: chunks ascending, T += phi(k) [v, 1]^T as in forward.  Each of the two waves of a row block takes a part of the feature
 // blocks and every other score block.
-template <typename T, bool NORM>
+template <typename T, bool NORM, bool SUMS>
 __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkParams p) {
 #if defined(__gfx950__)
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
@@ -933,8 +941,11 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
     unsigned char *tq = smem + L::qQ, *tk = smem + L::qK, *tkt = smem + L::qKt, *tv = smem + L::qV, *tg = smem + L::qG,
                   *ts = smem + L::qS, *exch = smem + L::qEx;
     float *z = reinterpret_cast<float *>(smem + L::qZ), *dn = reinterpret_cast<float *>(smem + L::qDn);
-    PolyState s;
+    unsigned char *tqt = smem + L::qQt;
+    PolyState s, sums;
     s.clear_lower(wave);
+    if constexpr (SUMS) sums.clear_beside_lower(wave);
+    const bool with_sums = SUMS && sl.seg > 0;  // (the first segment's total is under no sum)
     if (sl.seg > 0) s.template add<NORM>(p.entries + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kStateRoom, tid0 & 63);
     u32x4 x;
     PolyTile<T> v;
@@ -951,7 +962,11 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
         const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
         // (every wave is past the barrier behind its last reads of the tiles and of the state's copy)
         poly_put_x(tid < 256 ? tq : tk, x, tid);
-        if (tid >= 256) poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
+        if (tid >= 256) {
+            poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
+        } else if (with_sums) {
+            poly_put_xt(tqt, x, tid), poly_put_ones<T>(tqt, c * L::C, N, tid);
+        }
         v.put(tv, tid);
         go.put(tg, dn, tid);
         s.template to_lds<T, NORM>(ts, z, lane);
@@ -1006,6 +1021,8 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
                 *reinterpret_cast<f32x4 *>(exch + (a * L::C + trow) * 16) = f32x4{f[4 * a], f[4 * a + 1], f[4 * a + 2], f[4 * a + 3]};
         }
         if (c + 1 < sl.c_hi) s.template update<NORM>(tkt, tv, nullptr, lane);
+        if constexpr (SUMS)
+            if (with_sums) sums.template update<NORM>(tqt, tg, dn, lane);
         __syncthreads();
         if (kh == 0 && g == 0) {
 #pragma unroll
@@ -1017,6 +1034,8 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
             if (row < N) poly_store16<T>(p.dq, dq_at + (int64_t)row * p.dqs_n, f, 0, p.r, p.wide_out);
         }
     }
+    if constexpr (SUMS)
+        if (with_sums) sums.template store<NORM>(p.totals + ((int64_t)sl.bh * p.n_seg + sl.seg) * PolyFeatures::kState, tid0 & 63);
 #else
     (void)p;
 #endif
@@ -1191,8 +1210,11 @@ template <typename T>
 hipError_t launch_poly_walk(const PolyWalkParams &p, bool bwd, hipStream_t stream) {
     if (bwd) {
         if (p.n_seg > 1 && !p.entries) return hipErrorInvalidValue;
-        if (hipError_t e = p.denom ? launch_poly_kernel<poly_walk_dq_kernel<T, true>>(p, PolyLds::qTotal, stream)
-                                   : launch_poly_kernel<poly_walk_dq_kernel<T, false>>(p, PolyLds::qTotal, stream))
+        if (p.u_totals && (!p.sum_entries || !p.totals || p.n_seg < 3)) return hipErrorInvalidValue;
+        if (hipError_t e = p.u_totals ? (p.denom ? launch_poly_kernel<poly_walk_dq_kernel<T, true, true>>(p, PolyLds::qTotalSums, stream)
+                                                 : launch_poly_kernel<poly_walk_dq_kernel<T, false, true>>(p, PolyLds::qTotalSums, stream))
+                           : p.denom ? launch_poly_kernel<poly_walk_dq_kernel<T, true, false>>(p, PolyLds::qTotal, stream)
+                                     : launch_poly_kernel<poly_walk_dq_kernel<T, false, false>>(p, PolyLds::qTotal, stream))
             return e;
         return p.denom ? launch_poly_kernel<poly_walk_dkdv_kernel<T, true>>(p, PolyLds::kTotal, stream)
                        : launch_poly_kernel<poly_walk_dkdv_kernel<T, false>>(p, PolyLds::kTotal, stream);
