@@ -18,7 +18,7 @@
 // the running sums once per chunk: errors against fp64 0.87 to 1.01 times the quadratic kernels', the normaliser's 1e-7.
 //
 // What bounds it: the matrix instructions and the VALU work that forms features together (an update's fragment of eight
-// features costs 48 VALU instructions and serves ten MFMAs of 16 x 16 x 32, one along the row 32 and four of 32 x 32 x 16): the VALU
+// features costs 32 VALU instructions and serves ten MFMAs of 16 x 16 x 32, one along the row 32 and four of 32 x 32 x 16): the VALU
 // issues two thirds of the walks' time, the matrix unit is busy a quarter; HBM is far away
 // (40 KiB per 128-row chunk).  Hence eight waves, two per SIMD, so that one wave's VALU work runs under the other's MFMAs: wave w owns
 // rows 32 (w % 4) .. of the chunk, and of their work one half: half of the features and of the score blocks (forward
@@ -30,7 +30,7 @@
 // forward direction for dq, from the entry states forward formed, and one in reverse for dk and dv, so that nothing of a
 // row reaches the dq of the chunks before it.
 // Measured, B 4 H 16 N 4096, 16 over 64 columns, normalised, forward + backward: 605 us quadratic, 200 us this way (kernels
-// under the profiler 21 totals, 53 forward, 73 dq with the reverse walk's totals, 74 dk and dv).  With the pairs taken by blocks of eight columns -- 209
+// under the profiler 20 totals, 52 forward, 71 dq with the reverse walk's totals, 77 dk and dv).  With the pairs taken by blocks of eight columns -- 209
 // features in seven blocks of 32 -- and a barrier more per chunk 239 us.  With T for dq going backwards, by subtraction, in the reverse walk
 // 228 us, but a late row that is infinite, NaN or huge spoiled dq before it; with feature rows rounded to one bf16 number on
 // both sides as well, from tiles of them in LDS, 200 us, and errors up to 1.28 times the quadratic kernels'.
@@ -80,8 +80,12 @@ struct PolyFeatures {
 };
 
 struct PolyLds {  // byte offsets
-    // XTR: an x tile transposed (rows of 272 bytes: the sixteen columns, a one per row of the sequence, zeros)
-    static constexpr int C = 128, XT = C * 32, VT = C * 128, ST = 2 * 64 * 256, XTR = 18 * 272, EX = 8 * 4096;
+    // XTR: an x tile transposed, in fp32 (rows of 528 bytes: the sixteen columns, a one per row of the sequence, zeros): the state's update
+    // multiplies two of its rows, and as 16-bit rows the unpacking was a third of its VALU instructions.  16-bit rows -> this, same
+    // bits: B H 64, N 4096 203.6 -> 200.6 us forward + backward, 67.0 -> 65.2 forward (totals 22.1 -> 20.4, walk 53.1 -> 51.9); B H 80
+    // 256.2 -> 253.6; B H 300, N 1024 291.8 -> 287.5.
+    // XTB: the sixteen columns as they are, operands of the chunk's own scores (poly_col_frag)
+    static constexpr int C = 128, XT = C * 32, VT = C * 128, ST = 2 * 64 * 256, XR = 528, XTR = 18 * XR, XTB = 16 * 272, EX = 8 * 4096;
     static constexpr int Z = PolyFeatures::kF * 4, DN = C * 4;
     // totals: two sets of the x tile transposed, the v tile, dn
     static constexpr int tX = 0, tV = tX + XTR, tDn = tV + VT, tSet = tDn + DN, tTotal = 2 * tSet;
@@ -89,12 +93,12 @@ struct PolyLds {  // byte offsets
     static constexpr int fQ = 0, fK = fQ + XT, fKt = fK + XT, fV = fKt + XTR, fS = fV + VT, fEx = fS + ST, fZ = fEx + EX,
                          fSum = fZ + Z, fTotal = fSum + 2 * C * 4;
     // dq (the exchange: sixteen floats a row)
-    static constexpr int qQ = 0, qK = qQ + XT, qKt = qK + XT, qV = qKt + XTR, qG = qV + VT, qS = qG + VT, qEx = qS + ST,
+    static constexpr int qQ = 0, qK = qQ + XT, qKt = qK + XT, qKb = qKt + XTR, qV = qKb + XTB, qG = qV + VT, qS = qG + VT, qEx = qS + ST,
                          qZ = qEx + C * 64, qDn = qZ + Z, qTotal = qDn + DN, qQt = qTotal, qTotalSums = qQt + XTR;
     // dk, dv
-    static constexpr int kQ = 0, kQt = kQ + XT, kK = kQt + XTR, kV = kK + XT, kG = kV + VT, kU = kG + VT, kY = kU + ST,
+    static constexpr int kQ = 0, kQt = kQ + XT, kQb = kQt + XTR, kK = kQb + XTB, kV = kK + XT, kG = kV + VT, kU = kG + VT, kY = kU + ST,
                          kDn = kY + Z, kEx = kDn + DN, kTotal = kEx + EX;
-    static_assert(XTR % 16 == 0 && tTotal >= 8 * 5 * 1024 && fTotal <= 160 * 1024 && qTotal <= 160 * 1024 && kTotal <= 160 * 1024, "a CU's LDS");
+    static_assert(XTR % 16 == 0 && tTotal >= 8 * 5 * 1024 && fTotal <= 160 * 1024 && qTotalSums <= 160 * 1024 && kTotal <= 160 * 1024, "a CU's LDS");
 };
 
 // (a select of two values: written between two elements of an array it would become one load with a computed index, and
@@ -130,10 +134,10 @@ __device__ __forceinline__ typename Mma<T>::V8 poly_row_frag(const unsigned char
 
 // column r of an x tile from its transposed copy, rows R0 + {4g .., 8 + 4g ..}: the k order of a rounded score
 template <typename T>
-__device__ __forceinline__ typename Mma<T>::V8 poly_col_frag(const unsigned char *xtr, int r, int R0, int g) {
+__device__ __forceinline__ typename Mma<T>::V8 poly_col_frag(const unsigned char *xtb, int r, int R0, int g) {
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    const u32x2 lo = *reinterpret_cast<const u32x2 *>(xtr + r * 272 + (R0 + 4 * g) * 2);
-    const u32x2 hi = *reinterpret_cast<const u32x2 *>(xtr + r * 272 + (R0 + 8 + 4 * g) * 2);
+    const u32x2 lo = *reinterpret_cast<const u32x2 *>(xtb + r * 272 + (R0 + 4 * g) * 2);
+    const u32x2 hi = *reinterpret_cast<const u32x2 *>(xtb + r * 272 + (R0 + 8 + 4 * g) * 2);
     return __builtin_bit_cast(typename Mma<T>::V8, u32x4{lo[0], lo[1], hi[0], hi[1]});
 }
 
@@ -274,7 +278,7 @@ __device__ __forceinline__ PolyFactors poly_factors(int f) {
     } else {  // the row itself; a one and zeros
         a = group < 19 ? 8 * (group - 17) + j : 16, b = group < 19 || j == 0 ? 16 : 17;
     }
-    return {(uint32_t)(a * 272), (uint32_t)(b * 272)};
+    return {(uint32_t)(a * PolyLds::XR), (uint32_t)(b * PolyLds::XR)};
 }
 
 // A state's blocks of this wave: up to two blocks of 16 features (`first`, `second`, < 0: none) over the four 16-column blocks of
@@ -387,7 +391,8 @@ struct PolyState {
     // What a step of 32 rows reads; requested a step ahead of its use, block after block (both blocks in one loop of
     // branches: the forward walk 53.6 us in place of 53.1, dk and dv 75.3 in place of 74.1).
     struct Rows {
-        u32x4 a, b, e[2];
+        f32x4 a[2], b[2];
+        u32x4 e[2];
         Mma<__bf16>::V8 z[4];
     };
     template <bool NORM>
@@ -395,7 +400,9 @@ struct PolyState {
                                             const float *extra) const {
 #pragma unroll
         for (int cb = 0; cb < 4; ++cb) r.z[cb] = poly_tr<__bf16>(zt, za, cb << 5);
-        r.a = *reinterpret_cast<const u32x4 *>(fa), r.b = *reinterpret_cast<const u32x4 *>(fb);
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            r.a[h] = *reinterpret_cast<const f32x4 *>(fa + 16 * h), r.b[h] = *reinterpret_cast<const f32x4 *>(fb + 16 * h);
         if constexpr (NORM)
             if (extra) r.e[0] = *reinterpret_cast<const u32x4 *>(extra), r.e[1] = *reinterpret_cast<const u32x4 *>(extra + 4);
     }
@@ -403,10 +410,7 @@ struct PolyState {
     __device__ __forceinline__ void add_rows(const Rows &r, bool ones, f32x4 (&acc)[4], f32x4 &e) {
         float f[8];
 #pragma unroll
-        for (int k = 0; k < 4; ++k) {
-            f[2 * k] = __builtin_bit_cast(float, r.a[k] << 16) * __builtin_bit_cast(float, r.b[k] << 16);
-            f[2 * k + 1] = __builtin_bit_cast(float, r.a[k] & 0xffff0000u) * __builtin_bit_cast(float, r.b[k] & 0xffff0000u);
-        }
+        for (int k = 0; k < 8; ++k) f[k] = r.a[k / 4][k % 4] * r.b[k / 4][k % 4];
         const PolyTwo y = poly_split8<true>(f);
         Mma<__bf16>::V8 ef;
         if constexpr (NORM) {
@@ -442,7 +446,7 @@ struct PolyState {
         auto block = [&](auto uc, auto steps, int first) {
             constexpr int U = decltype(uc)::value, NS = decltype(steps)::value;
             const PolyFactors at = poly_factors(16 * own[U] + l16);
-            const unsigned char *fa = xtr + 16 * kq + at.a + 64 * first, *fb = xtr + 16 * kq + at.b + 64 * first;
+            const unsigned char *fa = xtr + 32 * kq + at.a + 128 * first, *fb = xtr + 32 * kq + at.b + 128 * first;
             const unsigned char *z0 = zt + 32 * 128 * first;
             const float *e0 = extra ? ex_at + 32 * first : nullptr;
             Rows r[2];
@@ -450,7 +454,7 @@ struct PolyState {
             static_for<0, NS>([&](auto sc) {
                 constexpr int S = decltype(sc)::value;
                 if constexpr (S + 1 < NS)
-                    request<NORM>(r[(S + 1) & 1], fa + 64 * (S + 1), fb + 64 * (S + 1), z0 + 32 * 128 * (S + 1), za, extra ? e0 + 32 * (S + 1) : nullptr);
+                    request<NORM>(r[(S + 1) & 1], fa + 128 * (S + 1), fb + 128 * (S + 1), z0 + 32 * 128 * (S + 1), za, extra ? e0 + 32 * (S + 1) : nullptr);
                 __builtin_amdgcn_sched_barrier(0);
                 add_rows<NORM>(r[S & 1], !extra, st[U], ex[U]);
             });
@@ -498,17 +502,20 @@ __device__ __forceinline__ u32x4 poly_fetch_x(const T *base, int64_t stride, int
 __device__ __forceinline__ void poly_put_x(unsigned char *xt, u32x4 v, int tid) {
     *reinterpret_cast<u32x4 *>(xt + (tid & 127) * 32 + ((tid >> 7) & 1) * 16) = v;
 }
-__device__ __forceinline__ void poly_put_xt(unsigned char *xtr, u32x4 v, int tid) {  // the transposed copy
+// the transposed copy in fp32, with its rows of ones (zeros past the sequence's last row) and of zeros, by the same threads
+template <typename T>
+__device__ __forceinline__ void poly_put_xt(unsigned char *xtr, u32x4 v, int row0, int N, int tid) {
+    const int row = tid & 127, half = (tid >> 7) & 1;
+    const typename Mma<T>::V8 e = __builtin_bit_cast(typename Mma<T>::V8, v);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) *reinterpret_cast<float *>(xtr + (8 * half + j) * PolyLds::XR + row * 4) = static_cast<float>(e[j]);
+    *reinterpret_cast<float *>(xtr + (16 + half) * PolyLds::XR + row * 4) = half == 0 && row0 + row < N ? 1.f : 0.f;
+}
+__device__ __forceinline__ void poly_put_xb(unsigned char *xtb, u32x4 v, int tid) {  // the transposed copy in the storage type
     const int row = tid & 127, half = (tid >> 7) & 1;
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-        *reinterpret_cast<uint16_t *>(xtr + (8 * half + j) * 272 + row * 2) = (uint16_t)(v[j / 2] >> (16 * (j & 1)));
-}
-// ... its rows of ones (zeros past the sequence's last row) and of zeros, by the same threads
-template <typename T>
-__device__ __forceinline__ void poly_put_ones(unsigned char *xtr, int row0, int N, int tid) {
-    const int row = tid & 127, half = (tid >> 7) & 1;
-    *reinterpret_cast<T *>(xtr + (16 + half) * 272 + row * 2) = static_cast<T>(half == 0 && row0 + row < N ? 1.f : 0.f);
+        *reinterpret_cast<uint16_t *>(xtb + (8 * half + j) * 272 + row * 2) = (uint16_t)(v[j / 2] >> (16 * (j & 1)));
 }
 template <typename T>
 struct PolyTile {
@@ -650,7 +657,7 @@ __global__ __launch_bounds__(512, 2) void poly_totals_kernel(const PolyWalkParam
         unsigned char *tile = smem + S * L::tSet;
         float *dn = reinterpret_cast<float *>(tile + L::tDn);
         // (every wave has passed the barrier below a chunk ago, behind its reads of this set)
-        if (tid < 256) poly_put_xt(tile + L::tX, x[S], tid), poly_put_ones<T>(tile + L::tX, c * L::C, N, tid);
+        if (tid < 256) poly_put_xt<T>(tile + L::tX, x[S], c * L::C, N, tid);
         if constexpr (BWD)
             go[S].put(tile + L::tV, dn, tid);
         else
@@ -762,7 +769,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_fwd_kernel(const PolyWalkPar
         const int tid = poly_opaque(tid0), lane = tid & 63, l32 = lane & 31, g = lane >> 5;
         // (every wave is past the barrier behind its last reads of the tiles and of the state's copy)
         poly_put_x(tid < 256 ? tq : tk, x, tid);
-        if (tid >= 256) poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
+        if (tid >= 256) poly_put_xt<T>(tkt, x, c * L::C, N, tid);
         v.put(tv, tid);
         s.template to_lds<T, NORM>(ts, z, lane);
         if (c + 1 < sl.c_hi) fetch(c + 1, tid);
@@ -938,7 +945,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
     const float *den = NORM ? p.denom + (int64_t)sl.bh * N : nullptr;
     const int64_t dq_at = b * p.dqs_b + h * p.dqs_h;
     const float c1 = p.c1, c2 = p.c2;
-    unsigned char *tq = smem + L::qQ, *tk = smem + L::qK, *tkt = smem + L::qKt, *tv = smem + L::qV, *tg = smem + L::qG,
+    unsigned char *tq = smem + L::qQ, *tk = smem + L::qK, *tkt = smem + L::qKt, *tkb = smem + L::qKb, *tv = smem + L::qV, *tg = smem + L::qG,
                   *ts = smem + L::qS, *exch = smem + L::qEx;
     float *z = reinterpret_cast<float *>(smem + L::qZ), *dn = reinterpret_cast<float *>(smem + L::qDn);
     unsigned char *tqt = smem + L::qQt;
@@ -963,9 +970,9 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
         // (every wave is past the barrier behind its last reads of the tiles and of the state's copy)
         poly_put_x(tid < 256 ? tq : tk, x, tid);
         if (tid >= 256) {
-            poly_put_xt(tkt, x, tid), poly_put_ones<T>(tkt, c * L::C, N, tid);
+            poly_put_xt<T>(tkt, x, c * L::C, N, tid), poly_put_xb(tkb, x, tid);
         } else if (with_sums) {
-            poly_put_xt(tqt, x, tid), poly_put_ones<T>(tqt, c * L::C, N, tid);
+            poly_put_xt<T>(tqt, x, c * L::C, N, tid);
         }
         v.put(tv, tid);
         go.put(tg, dn, tid);
@@ -1010,7 +1017,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
             for (int i = 0; i < 16; ++i) d[i] = m[i] * (c1 + 2.f * c2 * u[i]);
             poly_round_masked<T, false>(d, all, l32, g, df);
 #pragma unroll
-            for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(tkt, rc, 32 * sb + 16 * t, g), df[t], dx);
+            for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(tkb, rc, 32 * sb + 16 * t, g), df[t], dx);
         }
         float f[16];  // (lanes of g = 0 hold the block's columns 0 .. 15)
 #pragma unroll
@@ -1062,7 +1069,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
     const float *den = NORM ? p.denom + (int64_t)sl.bh * N : nullptr;
     const int64_t dk_at = b * p.dks_b + h * p.dks_h, dv_at = b * p.dvs_b + h * p.dvs_h;
     const float c0 = p.c0, c1 = p.c1, c2 = p.c2;
-    unsigned char *tq = smem + L::kQ, *tqt = smem + L::kQt, *tk = smem + L::kK, *tv = smem + L::kV, *tg = smem + L::kG,
+    unsigned char *tq = smem + L::kQ, *tqt = smem + L::kQt, *tqb = smem + L::kQb, *tk = smem + L::kK, *tv = smem + L::kV, *tg = smem + L::kG,
                   *us = smem + L::kU, *exch = smem + L::kEx;
     float *y = reinterpret_cast<float *>(smem + L::kY), *dn = reinterpret_cast<float *>(smem + L::kDn);
     PolyState su;
@@ -1084,7 +1091,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
         const bool after = c + 1 < p.n_chunks;  // (U of this chunk holds anything)
         // (every wave is past the barrier behind its last reads of the tiles and of the state's copy)
         poly_put_x(tid < 256 ? tq : tk, x, tid);
-        if (tid < 256) poly_put_xt(tqt, x, tid), poly_put_ones<T>(tqt, c * L::C, N, tid);
+        if (tid < 256) poly_put_xt<T>(tqt, x, c * L::C, N, tid), poly_put_xb(tqb, x, tid);
         v.put(tv, tid);
         go.put(tg, dn, tid);
         if (after) su.template to_lds<T, NORM>(us, y, lane);
@@ -1156,7 +1163,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
                 poly_round_masked<T, true>(f, all, l32, g, pf);
 #pragma unroll
                 for (int t = 0; t < 2; ++t) {
-                    dx = M::mma(poly_col_frag<T>(tqt, rc, 32 * sb + 16 * t, g), df[t], dx);
+                    dx = M::mma(poly_col_frag<T>(tqb, rc, 32 * sb + 16 * t, g), df[t], dx);
 #pragma unroll
                     for (int e = 0; e < 2; ++e)
                         acc[e] = M::mma(poly_tr<T>(tg + 128 * (32 * sb + 16 * t), ga, e << 6), pf[t], acc[e]);
