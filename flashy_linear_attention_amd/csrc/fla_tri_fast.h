@@ -72,19 +72,26 @@ __device__ __forceinline__ void dma_16B_per_lane(u32x4 rsrc, uint32_t lds_base, 
 //     of 16 bits from a head to the next), pairs of neighbours, which share those lines in (B, N, H, D) storage.  Forward + backward:
 //     32 columns, B 2 H 16 N 8192 76.4 -> 67.2 us; 96 columns, B 2 H 24 N 4096 153 -> 148.  (Pairs for every row: 64 columns, B 1 H 16
 //     N 32768 in that storage 241 -> 232 us, but with a feature map B 4 H 16 N 4096 144 -> 148, and (B, H, N, D) storage gains nothing.)
+//   * no multiple of 8, but no XCD with more than kWholeHeadParts parts: whole heads all the same.  A part reads the totals that its
+//     head's other parts wrote, from that XCD's own L2, and half of an XCD's CUs are enough for them.  Forward alone, runs of parts ->
+//     whole heads (parts of the fullest XCD): 80 columns, B H 12 N 306 (10) 12.45 -> 12.02 us; 128 columns, B H 1 N 1024 (16) 17.8 ->
+//     16.3, B H 4 N 800 (13) 16.1 -> 15.1, B H 20 N 300 (15) 12.85 -> 12.46, B H 12 N 500 (16) 14.2 -> 14.2; above the line B H 12 N 620
+//     (20) 14.9 -> 14.8, N 750 (24) 16.5 -> 16.6, B H 3 N 1200 (19) 20.6 -> 18.5, but B H 4 and 1, N 1500 (24) 18.7 -> 22.5 and 14.3 -> 17.4.
 //   * else an eighth of all parts, consecutive ones.  Whole heads per XCD left XCDs idle, and gave others two rounds: forward +
 //     backward, D = 128: B H 1 N 16384 241 -> 86 us, B H 4 153 -> 95, B H 12 278 -> 179, B H 20 N 8192 232 -> 152; D = 64: B H 12
 //     N 32768 218 -> 165, B H 20 N 16384 161 -> 138.
 // The grid may hold more workgroups than there are parts (8 ceil(BH / 8) parts of them): bh < 0 is none.
+constexpr int kWholeHeadParts = 16;
 struct XcdItem {
     int bh, part;
 };
 __device__ __forceinline__ XcdItem xcd_item(int wg, int BH, int parts, int64_t stride_h) {
     const int xcd = wg & 7, slot = wg >> 3;
-    if (BH % 8 == 0) {
+    if (BH % 8 == 0 || ((BH + 7) >> 3) * parts <= kWholeHeadParts) {
         const int hl = slot / parts;
         const bool pairs = BH % 16 == 0 && stride_h % 64 != 0;
-        return {hl >= BH / 8 ? -1 : pairs ? (hl >> 1) * 16 + xcd * 2 + (hl & 1) : hl * 8 + xcd, slot - hl * parts};
+        const int bh = pairs ? (hl >> 1) * 16 + xcd * 2 + (hl & 1) : hl * 8 + xcd;
+        return {bh < BH ? bh : -1, slot - hl * parts};
     }
     const int total = BH * parts, share = (total + 7) >> 3, item = xcd * share + slot;
     if (slot >= share || item >= total) return {-1, 0};

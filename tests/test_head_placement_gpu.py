@@ -1,5 +1,5 @@
 """Which workgroup takes which part of which head (csrc/fla_tri_fast.h, xcd_item): a head count that is no multiple of 8 (runs of
-consecutive parts), a multiple of 8 (every eighth head) and, with rows that end inside a 128-byte line in (B, N, H, D) storage, a
+consecutive parts, or whole heads where no XCD gets more than 16 parts), a multiple of 8 (every eighth head) and, with rows that end inside a 128-byte line in (B, N, H, D) storage, a
 multiple of 16 (pairs of neighbours) -- in every kernel that goes by it, so that a part taken twice or not at all would show
 (``-m gpu``)."""
 
@@ -24,6 +24,19 @@ def _bnhd(t):
 def test_every_part_of_every_head(heads, width, gpu_device):
     n = 1000 if width <= 128 else 777
     q, k, v, dy = (_bnhd(t.to(gpu_device)) for t in reference_style_inputs(1, heads, n, width, width, torch.bfloat16, seed=heads))
+    want_o, want_g = gpu_fp32_reference(q, k, v, dy, True)
+    qg, kg, vg = (t.detach().requires_grad_(True) for t in (q, k, v))
+    out = LinearAttentionChunked.apply(qg, kg, vg)
+    out.backward(dy)
+    assert_close("O", out, want_o)
+    for name, got, want in zip(("dQ", "dK", "dV"), (qg.grad, kg.grad, vg.grad), want_g):
+        assert_close(name, got, want)
+
+
+# (128 columns, four heads: 16 parts each, the most that stay together, and 17)
+@pytest.mark.parametrize("n", [1024, 1025])
+def test_either_side_of_whole_heads(n, gpu_device):
+    q, k, v, dy = (_bnhd(t.to(gpu_device)) for t in reference_style_inputs(1, 4, n, 128, 128, torch.bfloat16, seed=n))
     want_o, want_g = gpu_fp32_reference(q, k, v, dy, True)
     qg, kg, vg = (t.detach().requires_grad_(True) for t in (q, k, v))
     out = LinearAttentionChunked.apply(qg, kg, vg)
