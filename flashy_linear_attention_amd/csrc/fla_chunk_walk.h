@@ -894,26 +894,36 @@ __device__ __forceinline__ void walk_load_state_copy(const void *src, uint32_t l
 }
 
 // fp16: the sums of a long sequence leave its range where results of the operator do not, so the state's 16-bit copy is
-// scaled by a power of two that puts its largest element at 2^14 (exact; what is 2^28 times smaller than that becomes
-// subnormal).  Every wave leaves its largest |element| in smax[wave]; behind a barrier walk_state_scale gives
-// the factor of the copy and, in `back`, its inverse for the product (1 for a zero or a non-finite state).
-template <int D, typename B>
-__device__ __forceinline__ void walk_state_max(float *smax, int wave, int lane, const f32x16 (&st)[WalkCfg<D>::NBW]) {
+// scaled by a power of two that puts its largest finite element at 2^14 (exact; what is 2^28 times smaller than that becomes
+// subnormal).  An infinite or NaN element, which stays what it is at any scale, has no say: the other columns' elements would leave
+// fp16's range.  Every wave leaves its largest finite |element| in smax[wave]; behind a barrier walk_state_scale gives the factor of
+// the copy and, in `back`, its inverse for the product (1 for a state of zeros).
+template <int D, typename B, bool FINITE = false>
+__device__ __forceinline__ float walk_state_largest(const f32x16 (&st)[WalkCfg<D>::NBW], int wave) {
     float m = 0.f;
 #pragma unroll
     for (int i = 0; i < B::SLOTS; ++i)
         if (B::valid(wave, i)) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) m = fmaxf(m, fabsf(st[i][v]));
+            for (int v = 0; v < 16; ++v) {
+                const float x = fabsf(st[i][v]);
+                m = fmaxf(m, FINITE && x == __builtin_inff() ? 0.f : x);  // (a NaN is never the larger one)
+            }
         }
 #pragma unroll
     for (int d = 1; d < 64; d <<= 1) m = fmaxf(m, __shfl_xor(m, d, 64));
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, m)));
+}
+template <int D, typename B>
+__device__ __forceinline__ void walk_state_max(float *smax, int wave, int lane, const f32x16 (&st)[WalkCfg<D>::NBW]) {
+    float m = walk_state_largest<D, B>(st, wave);
+    if (__builtin_expect(__builtin_bit_cast(uint32_t, m) == 0x7f800000u, 0)) m = walk_state_largest<D, B, true>(st, wave);
     if (lane == 0) smax[wave] = m;
 }
 __device__ __forceinline__ float walk_state_scale(const float *smax, float &back) {
     const float m = fmaxf(fmaxf(smax[0], smax[1]), fmaxf(smax[2], smax[3]));
     const int e = (int)(__builtin_bit_cast(uint32_t, m) >> 23);  // biased exponent: m < 2^(e - 126)
-    const int k = m > 0.f && e < 255 ? (e < 40 ? 40 : e) - 141 : 0;
+    const int k = m > 0.f ? (e < 40 ? 40 : e) - 141 : 0;
     back = __builtin_bit_cast(float, (uint32_t)(127 + k) << 23);
     return __builtin_bit_cast(float, (uint32_t)(127 - k) << 23);
 }

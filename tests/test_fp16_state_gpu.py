@@ -32,3 +32,21 @@ def test_state_beyond_the_range(b, h, n, dqk, dv, sq, sk, sv, gpu_device):
         with torch.no_grad():
             got = op.apply(q, k, v)
         assert_close("O, evaluation chosen by shape", torch.where(inside, got.float(), 0.0), torch.where(inside, want, 0.0))
+
+
+# an infinite or NaN value: the other columns' state elements, 1e5 and more beyond the range, keep their scale (widths up to 64: one
+# segment and several; 128: several)
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")], ids=["inf", "-inf", "nan"])
+@pytest.mark.parametrize("h,n,dqk,dv", [(3, 1024, 32, 32), (2, 1024, 64, 64), (300, 512, 64, 64), (2, 1024, 128, 128), (128, 1024, 96, 96), (2, 1024, 128, 64)])
+def test_a_non_finite_value_beside_a_state_beyond_the_range(h, n, dqk, dv, value, gpu_device):
+    gen = torch.Generator().manual_seed(n + dqk)
+    q, k = (torch.rand(1, h, n, dqk, generator=gen).add(0.5).mul(s).half().to(gpu_device) for s in (2.0**-14, 20.0))
+    v = torch.rand(1, h, n, dv, generator=gen).add(0.5).mul(20.0).half().to(gpu_device)
+    want, _ = gpu_fp32_reference(q, k, v, None, False)
+    v[:, :, 3, 1] = value
+    with torch.no_grad():
+        picked = (LinearAttention if dqk == dv else LinearAttentionSmallVHD).apply(q, k, v)
+    for out in (linear_attention_chunked_fwd(q, k, v), picked):
+        assert not bool(out[:, :, 3:, 1].isfinite().any())
+        keep = torch.arange(dv, device=gpu_device) != 1
+        assert_close("O", out[..., keep], want[..., keep])
