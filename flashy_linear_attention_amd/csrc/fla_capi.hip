@@ -2135,6 +2135,16 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
 
 extern "C" {
 
+#if defined(FLA_TRACE_LAUNCHES)
+// The kernels' map of workgroups to (head, part), for all of a grid: `items` receives both of every workgroup (head < 0: none).
+void fla_trace_xcd_items(int grid, int BH, int parts, int64_t stride_h, int32_t *items) {
+    for (int wg = 0; wg < grid; ++wg) {
+        const fla::XcdItem item = fla::xcd_item(wg, BH, parts, stride_h);
+        items[2 * wg] = item.bh, items[2 * wg + 1] = item.part;
+    }
+}
+#endif
+
 int fla_abi_version(void) { return FLA_ABI_VERSION; }
 
 int fla_convert(const void *const *src, void *const *dst, const int64_t *counts, int n, int widen, int dtype, void *stream) {

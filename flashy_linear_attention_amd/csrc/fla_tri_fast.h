@@ -85,7 +85,7 @@ constexpr int kWholeHeadParts = 16;
 struct XcdItem {
     int bh, part;
 };
-__device__ __forceinline__ XcdItem xcd_item(int wg, int BH, int parts, int64_t stride_h) {
+__host__ __device__ __forceinline__ XcdItem xcd_item(int wg, int BH, int parts, int64_t stride_h) {
     const int xcd = wg & 7, slot = wg >> 3;
     if (BH % 8 == 0 || ((BH + 7) >> 3) * parts <= kWholeHeadParts) {
         const int hl = slot / parts;

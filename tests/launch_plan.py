@@ -50,6 +50,8 @@ def trace_lib(rebuild: bool = False) -> ctypes.CDLL:
             fn.restype = restype
         lib.fla_trace_take.argtypes = [ctypes.c_char_p, ctypes.c_int64]
         lib.fla_trace_take.restype = ctypes.c_int64
+        lib.fla_trace_xcd_items.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_void_p]
+        lib.fla_trace_xcd_items.restype = None
         _trace_lib = lib
     return _trace_lib
 
@@ -248,6 +250,22 @@ def tensor_extent(p: Dict, ptr: str, sb: str, sh: str, sn: str, H: int, BH: int,
 
 
 # ---------------------------------------------------------------------------------------------
+# workgroups -> (head, part): csrc/fla_tri_fast.h, xcd_item
+
+def xcd_items(grid: int, BH: int, parts: int, stride_h: int) -> np.ndarray:
+    """(head, part) of every workgroup of a grid, by the kernels' own function; head -1: none.  Every part of every head is one
+    workgroup's and no other's."""
+    items = np.empty((grid, 2), dtype=np.int32)
+    trace_lib().fla_trace_xcd_items(grid, BH, parts, stride_h, items.ctypes.data)
+    used = items[items[:, 0] >= 0]
+    where = f"{BH} heads of {parts} parts, {stride_h} elements apart"
+    assert (used[:, 0] < BH).all() and (used[:, 1] >= 0).all() and (used[:, 1] < parts).all(), f"{where}: outside them"
+    times = np.bincount(used[:, 0].astype(np.int64) * parts + used[:, 1], minlength=BH * parts)
+    assert (times == 1).all(), f"{where}: {int((times > 1).sum())} taken twice, {int((times == 0).sum())} not at all"
+    return items
+
+
+# ---------------------------------------------------------------------------------------------
 # model of the fast masked-product kernels (csrc/fla_tri_fast.h), quadratic walk
 
 @dataclass
@@ -379,14 +397,15 @@ def model_tri_fast(arena: Arena, l: Launch, p: Dict, T: str, DC: int, DO: int, c
     # every workgroup index: its head and row tiles.  Heads differ in their base addresses only, so
     # the lane-level part runs for the first heads, the last one and every rank.
     sample_ranks = {0, 1, n_pairs // 2, n_pairs - 2, n_pairs - 1}
+    items = xcd_items(l.grid[0], BH, n_tiles, p["ys_h"]).tolist() if chunked else None
     for wg in range(l.grid[0]):
         xcd, slot = wg & 7, wg >> 3
-        if single and not chunked:
-            hl, rank = slot % n_hl, slot // n_hl
+        if chunked:
+            bh, rank = items[wg]
         else:
-            hl, rank = slot // n_pairs, slot - (slot // n_pairs) * n_pairs
-        bh = hl * 8 + xcd
-        if bh >= BH:
+            hl, rank = (slot % n_hl, slot // n_hl) if single else (slot // n_pairs, slot - (slot // n_pairs) * n_pairs)
+            bh = hl * 8 + xcd
+        if not 0 <= bh < BH:
             continue
         stats.workgroups += 1
         if chunked:
@@ -760,6 +779,7 @@ def model_walk(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats) -> None:
     assert seg_chunks >= 1 and n_seg >= 1 and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks, \
         f"{l.kernel}: {n_seg} segments of {seg_chunks} chunks do not tile {n_chunks} chunks"
     assert l.grid[0] == 8 * ((BH + 7) // 8) * n_seg
+    xcd_items(l.grid[0], BH, n_seg, p["ks_h"])
     resident = 256 if D > 64 else 512
     assert BH * n_seg <= max(resident, BH), f"{l.kernel}: {BH * n_seg} workgroups for {resident} resident"
     # (pairs of column halves, grid y: a q / k of 128 + wqk2 columns, a v of 128 + wv2)
@@ -809,6 +829,9 @@ def model_walk(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats) -> None:
     for nm, count in (("zc", n_chunks), ("zc_out", n_chunks), ("rc", n_seg), ("vsum", n_seg)):
         if p[nm]:
             arena.require(nm, p[nm], p[nm] + BH * count * D * 4)
+    if p["gn"]:  # (dO = g / n formed in the tile: n's rows of a chunk behind dn's, in the vectors' 3 KiB)
+        assert l.kernel == "walk_bwd_kernel" and p["dn"] and l.lds == (4 * rows + D) * 2 * D + 4096, f"{l.kernel}: {l.lds} bytes of LDS"
+        arena.require("n", p["gn"], p["gn"] + BH * N * 4)
     for nm in ("denom", "dn"):
         if p[nm]:
             # (the walk for dK and dV reads dn in whole groups of four rows)
@@ -887,6 +910,7 @@ def model_walk_totals(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats, bo
     assert n_chunks == -(-N // rows) and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks
     assert 0 <= p["seg_lo"] <= p["seg_hi"] <= n_seg
     assert l.grid[0] == 8 * ((BH + 7) // 8) * n_seg
+    xcd_items(l.grid[0], BH, n_seg, p["ys_h"])
     operands = [("y", "y", "ys_b", "ys_h", "ys_n", p["dy"]), ("z", "z", "zs_b", "zs_h", "zs_n", p["dz"])]
     if p["y2"]:  # a second Y operand (the other half of a wide q / k) in the same launch
         # (grid y picks the operand, or -- the kernel built for it -- every workgroup takes both: three sets of three tiles)
@@ -911,6 +935,7 @@ def model_walk_grad_totals(arena: Arena, l: Launch, p: Dict, D: int, vec: bool, 
     n_chunks, seg_chunks, n_seg = p["n_chunks"], p["seg_chunks"], p["n_seg"]
     assert n_chunks == -(-N // rows) and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks
     assert l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
+    xcd_items(l.grid[0], BH, n_seg, p["qs_h"])
     assert l.lds == ((2 if D == 128 else 1) + 3) * rows * 2 * D + 2 * rows * 4, f"{l.kernel}: {l.lds} bytes of LDS"
     assert 1 <= wqk <= D and 1 <= wv <= D and wqk % 8 == 0 and wv % 8 == 0
     assert p["q"] % 16 == 0 and p["qs_n"] % 8 == 0 and p["dout"] % 16 == 0 and N * p["qs_n"] * 2 <= 0x3fffffff
@@ -933,12 +958,16 @@ def model_walk_grad_totals(arena: Arena, l: Launch, p: Dict, D: int, vec: bool, 
 
 
 POLY_STATE, POLY_ROOM = 160 * 65, 224 * 65  # floats of a polynomial state; of its place in a state buffer
+# bytes of LDS of the walk for dq: tiles of q, k, v, g, the transposed k in fp32 and in 16 bits, the state's copy, the exchange, z, dn;
+# the transposed q in fp32 where it adds up totals
+POLY_DQ_LDS, POLY_QT_LDS = 2 * 4096 + 2 * 16384 + 18 * 528 + 16 * 272 + 32768 + 8192 + 640 + 512, 18 * 528
 
 
 def model_poly(arena: Arena, l: Launch, p: Dict, backward: bool, stats: Stats) -> None:
     """The polynomial map's kernels: every operand, result and state that the kernel touches."""
     H, BH, N, n_seg = p["H"], p["BH"], p["N"], p["n_seg"]
     assert p["n_chunks"] == -(-N // 128) and l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
+    xcd_items(l.grid[0], BH, n_seg, p["ks_h"])
     assert (n_seg - 1) * p["seg_chunks"] < p["n_chunks"] <= n_seg * p["seg_chunks"]
     widths = {"q": p["r"], "k": p["r"], "v": p["wv"], "go": p["wv"], "o": p["wv"], "out": p["wv"], "dq": p["r"], "dk": p["r"],
               "dv": p["wv"]}
@@ -959,6 +988,10 @@ def model_poly(arena: Arena, l: Launch, p: Dict, backward: bool, stats: Stats) -
     if p["denom"]:
         arena.require("denom", p["denom"], p["denom"] + BH * N * 4)
     assert n_seg == 1 or p["totals"]
+    if p["u_totals"]:  # (dq's walk adds up the totals that the walk for dk and dv then sums as it starts)
+        assert l.kernel in ("poly_walk_dq_kernel", "poly_walk_dkdv_kernel") and 3 <= n_seg <= 20 and p["sum_entries"]
+    if l.kernel == "poly_walk_dq_kernel":
+        assert l.targs[2] == bool(p["u_totals"]) and l.lds == POLY_DQ_LDS + (POLY_QT_LDS if p["u_totals"] else 0)
     if p["totals"]:
         arena.require("polynomial totals", p["totals"], p["totals"] + BH * n_seg * POLY_STATE * 4)
     if p["entries"]:
@@ -1007,6 +1040,8 @@ class StateForms:
 def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
     """Every launch of a call: the general limits, then the kernel's model."""
     forms = StateForms()
+    grads = None  # the normalised backward's first pass, ahead of the walk that reads what it left
+    poly_totals = {}  # by address: the kernel that wrote them last, and their direction
     for l in launches:
         stats.launches += 1
         stats.kernels[l.kernel] = stats.kernels.get(l.kernel, 0) + 1
@@ -1054,8 +1089,15 @@ def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
             if wsum:
                 arena.require("wsum", wsum, wsum + BH * chunks * DP * 4)
         elif k in ("walk_fwd_kernel", "walk_bwd_kernel", "walk_dkdv_kernel", "walk_bwd_rev_kernel"):
-            model_walk(arena, l, l.struct("a0"), t[1], stats)
-            forms.walk(l, l.struct("a0"), t[1])
+            p = l.struct("a0")
+            model_walk(arena, l, p, t[1], stats)
+            forms.walk(l, p, t[1])
+            if k == "walk_bwd_kernel" and grads:  # dO of its own, or g and n where it was not written
+                place = {"go": grads["go"], "gn": grads["denom"]} if grads["keep_g"] else {"go": grads["dout"], "gn": 0}
+                assert all(p[nm] == at for nm, at in place.items()), "the walk reads another dO than the pass ahead of it left"
+                assert not grads["keep_g"] or all(p[f"gs_{d}"] == grads[f"gs_{d}"] for d in "bhn")
+            else:
+                assert not p["gn"] and not (grads and grads["keep_g"]), f"{k}: dO is nowhere"
         elif k in ("walk_fwd_wide_kernel", "walk_bwd_rev_wide_kernel"):
             model_walk_wide(arena, l, l.struct("a0"), stats)
             forms.walk(l, l.struct("a0"), 128)
@@ -1084,9 +1126,20 @@ def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
                 forms.wrote(base, p["frags"])
         elif k == "walk_grad_totals_kernel":
             model_walk_grad_totals(arena, l, l.struct("a0"), t[1], t[2], stats)
+            grads = l.struct("a0")
             forms.wrote(l.args["a0.totals"], l.args["a0.frags"])
         elif k == "poly_totals_kernel" or k.startswith("poly_walk_"):
-            model_poly(arena, l, l.struct("a0"), t[2] if k == "poly_totals_kernel" else "_d" in k, stats)
+            p, backward = l.struct("a0"), t[2] if k == "poly_totals_kernel" else "_d" in k
+            model_poly(arena, l, p, backward, stats)
+            if k == "poly_walk_fwd_kernel" or k == "poly_walk_dkdv_kernel":
+                assert p["n_seg"] == 1 or poly_totals.get(p["totals"]) == backward, f"{k}: totals that nothing wrote"
+            elif k == "poly_totals_kernel" or p["u_totals"]:
+                poly_totals[p["totals"]] = backward
+        elif k == "chunk_state_kernel":
+            p = l.struct("a0")
+            xcd_items(l.grid[0], p["BH"], p["n_chunks"], p["ys_h"])
+            for nm in ("y", "z"):
+                assert arena.find(p[nm]) is not None, f"{k}: {nm} points nowhere"
         elif k == "poly_scan_kernel":
             arena.require("polynomial totals", l.args["a0"], l.args["a0"] + l.args["a1"] * l.args["a2"] * 4)
         elif k == "pack_rows_kernel":

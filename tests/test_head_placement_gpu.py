@@ -1,7 +1,8 @@
 """Which workgroup takes which part of which head (csrc/fla_tri_fast.h, xcd_item): a head count that is no multiple of 8 (runs of
-consecutive parts, or whole heads where no XCD gets more than 16 parts), a multiple of 8 (every eighth head) and, with rows that end inside a 128-byte line in (B, N, H, D) storage, a
-multiple of 16 (pairs of neighbours) -- in every kernel that goes by it, so that a part taken twice or not at all would show
-(``-m gpu``)."""
+consecutive parts, or whole heads where no XCD gets more than 16 parts), a multiple of 8 (every eighth head) and, with rows that end
+inside a 128-byte line in (B, N, H, D) storage, a multiple of 16 (pairs of neighbours) -- in every kernel that goes by it, so that a
+part that no workgroup takes would show (``-m gpu``; a part taken twice leaves the same results, and the launch-plan tests
+enumerate the map on the CPU)."""
 
 import pytest
 import torch

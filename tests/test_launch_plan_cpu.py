@@ -11,6 +11,7 @@ sweep's space: head-dim pairs x (batch, heads) x lengths x both evaluations.
 import ctypes
 import itertools
 
+import numpy as np
 import pytest
 
 import launch_plan as lp
@@ -38,12 +39,12 @@ def _workspace(arena, name, nbytes):
     return arena.alloc(name, max(int(nbytes), 16))
 
 
-def trace_normalised(lib, b, h, n, dqk, dv, chunked, dtype=0, layout="contiguous"):
+def trace_normalised(lib, b, h, n, dqk, dv, chunked, dtype=0, layout="contiguous", g_layout="contiguous"):
     """fla_linear_attn_normalised_fwd + _bwd as LinearAttentionNormalised calls them."""
     arena = lp.Arena()
     q, k = (lp.make_tensor(arena, nm, b, h, n, dqk, layout) for nm in ("q", "k"))
     v = lp.make_tensor(arena, "v", b, h, n, dv, layout)
-    o, g = (lp.make_tensor(arena, nm, b, h, n, dv) for nm in ("out", "grad_out"))
+    o, g = lp.make_tensor(arena, "out", b, h, n, dv), lp.make_tensor(arena, "grad_out", b, h, n, dv, g_layout)
     dq, dk = (lp.make_tensor(arena, nm, b, h, n, dqk) for nm in ("dq", "dk"))
     dvv = lp.make_tensor(arena, "dv", b, h, n, dv)
     denom = arena.alloc("denom", 4 * b * h * n)
@@ -195,6 +196,21 @@ def test_normalised_operator_over_the_sweep_space(lib, dims):
     assert cases > 25 and stats.launches > cases * 4
 
 
+@pytest.mark.parametrize("g_layout,kept", [("contiguous", True), ("odd", False)])
+def test_where_the_normalised_walk_takes_dO_from(lib, g_layout, kept):
+    """From g and n where g's rows are aligned, else from what the pass ahead wrote; another place is noticed."""
+    arena, launches = trace_normalised(lib, 1, 3, 1000, 64, 64, True, g_layout=g_layout)
+    ahead = next(l for l in launches if l.kernel == "walk_grad_totals_kernel")
+    walk = next(l for l in launches if l.kernel == "walk_bwd_kernel")
+    assert bool(ahead.args["a0.keep_g"]) == kept == bool(walk.args["a0.gn"])
+    lp.check_all(arena, launches, lp.Stats())
+    for nm, other in (("go", ahead.args["a0.dout" if kept else "a0.go"]), ("gn", 0 if kept else ahead.args["a0.denom"])):
+        right, walk.args[f"a0.{nm}"] = walk.args[f"a0.{nm}"], other
+        with pytest.raises(AssertionError):
+            lp.check_all(arena, launches, lp.Stats())
+        walk.args[f"a0.{nm}"] = right
+
+
 # (a v wider than 128 columns as two column halves, over the D = 128 walks and over the wide ones; padded widths that differ)
 @pytest.mark.parametrize("dims", DIMS + [(256, 256), (40, 40), (25, 25), (91, 91), (128, 32), (200, 200), (128, 256),
                                          (96, 200), (256, 136), (128, 64), (64, 128), (64, 32), (32, 64), (24, 128),
@@ -261,6 +277,19 @@ def test_benchmark_shapes(lib):
     assert stats.kernels["tri_xyt_z_fast_batch_kernel"] >= 4 and stats.kernels["walk_bwd_rev_kernel"] >= 1
     # (C4: one walk over both halves of q / k, forward and backward)
     assert stats.kernels["walk_fwd_wide_kernel"] >= 1 and stats.kernels["walk_bwd_rev_wide_kernel"] >= 1
+
+
+@pytest.mark.parametrize("stride_h", [64, 40], ids=["whole lines", "part of a line"])
+def test_every_part_of_every_head_is_one_workgroups(lib, stride_h):
+    """The walks' map over the grid that their launchers take: 16 parts per XCD and 17, and counts off every line."""
+    for bh in [*range(1, 70), 72, 80, 96, 100, 112, 127, 128, 129, 191, 192, 255, 256, 257, 300]:
+        for parts in [*range(1, 21), 31, 32, 33, 63, 64]:
+            items = lp.xcd_items(8 * ((bh + 7) // 8) * parts, bh, parts, stride_h)
+            per_xcd = [int((items[x::8, 0] >= 0).sum()) for x in range(8)]
+            if bh % 8 == 0 or (bh + 7) // 8 * parts <= 16:  # whole heads
+                assert all(len(set(np.flatnonzero(items[:, 0] == head) % 8)) == 1 for head in {0, bh // 2, bh - 1})
+            else:  # an eighth of the parts each
+                assert max(per_xcd) == -(-bh * parts // 8)
 
 
 def test_empty_problems_make_no_launch(lib):

@@ -129,4 +129,10 @@ def test_polynomial_map(lib, h, n, r, dv, flag, normalised):
     assert lib.fla_poly_attn_chunked_bwd(g.ptr, q.ptr, k.ptr, v.ptr, o.ptr if normalised else None, denom, dq.ptr, dk.ptr, dvv.ptr, 1, h,
                                          n, r, dv, *st, coef, flag, state, arena.alloc("backward workspace", max(wbytes, 16)), wbytes,
                                          None) == 0
-    checked(arena, lp.take_launches(lib), ("dq", "dk", "dv"))
+    launches = lp.take_launches(lib)
+    checked(arena, launches, ("dq", "dk", "dv"))
+    own_totals = [l.args["a0.u_totals"] for l in launches if l.kernel == "poly_walk_dq_kernel"] == [1]
+    assert own_totals == (3 <= launches[-1].args["a0.n_seg"] <= 20)
+    if own_totals:  # (without the walk for dq, nothing has written the totals)
+        with pytest.raises(AssertionError, match="totals that nothing wrote"):
+            lp.check_all(arena, [l for l in launches if l.kernel != "poly_walk_dq_kernel"], lp.Stats())
