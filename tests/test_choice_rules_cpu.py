@@ -1,6 +1,6 @@
-"""Which evaluation the library names (host arithmetic, no GPU) for widths that are no multiples of 8 and for the polynomial
-map: the chunk-wise one where it was measured to be the faster one, later for forward alone than for a pair; and the
-polynomial map's state."""
+"""Which evaluation the library names (host arithmetic, no GPU): the chunk-wise one where it was measured to be the faster one.
+Widths up to 128 that are multiples of 8, forward alone and pairs of 128 columns, and the normalised forward; widths that are no
+multiples of 8 and the polynomial map, later for forward alone than for a pair; and the polynomial map's state."""
 
 import pytest
 
@@ -17,6 +17,30 @@ def test_widths_that_are_no_multiples_of_8(bh, dqk, dv, pair_from, forward_from)
             assert _lib.query(name, 1, bh, first - 1, dqk, dv) == 0
         assert _lib.query(name, 1, bh, first, dqk, dv) == 1
         assert _lib.query(name, 1, bh, 4096, dqk, dv) == 1
+
+
+# (129 heads of 128 columns and 257 of 64 are a single segment each, 128 and 256 are two: W = B H N^2 D from 1.2e10 on)
+@pytest.mark.parametrize("bh,dqk,dv,first", [
+    (1, 64, 64, 768), (1, 32, 32, 1024), (1, 128, 128, 1024), (1, 64, 32, 1024), (1, 128, 64, 1024), (1, 128, 32, 1024),
+    (129, 128, 128, 257), (257, 64, 64, 257), (128, 128, 128, 856), (256, 64, 64, 768),
+])
+def test_forward_alone(bh, dqk, dv, first):
+    for n, want in ((first - 1, 0), (first, 1)):
+        assert _lib.query("fla_linear_attn_forward_prefers_chunked", 1, bh, n, dqk, dv) == want
+
+
+@pytest.mark.parametrize("bh,first", [(130, 439), (128, 699), (1, 2048)])
+def test_pairs_of_128_columns(bh, first):
+    """From W = B H N^2 128 = 3.2e9 on with a single segment per head, else from 8e9 or 2048 rows."""
+    for n, want in ((first - 1, 0), (first, 1)):
+        assert _lib.query("fla_linear_attn_prefers_chunked", 1, bh, n, 128, 128) == want
+
+
+@pytest.mark.parametrize("bh,d,first", [(1, 64, 1024), (1, 32, 1024), (1, 128, 2048), (129, 128, 257), (257, 64, 257), (128, 128, 856)])
+def test_normalised_forward(bh, d, first):
+    for n, want in ((first - 1, 0), (first, 1)):
+        assert _lib.query("fla_normalised_forward_prefers_chunked", 1, bh, n, d, d, 0) == want
+        assert _lib.query("fla_normalised_forward_prefers_chunked", 1, bh, n, d, d, 1) == 0  # fp16
 
 
 def test_polynomial_state_is_for_several_segments_alone():

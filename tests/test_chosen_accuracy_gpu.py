@@ -49,6 +49,25 @@ def test_no_larger_than_the_quadratic_kernels(h, n, dqk, dv, positive, gpu_devic
     _compare(chosen, other, _exact(q, k, v, do))
 
 
+# from the first lengths that forward alone takes chunk-wise: a single segment per head (257 and 129 heads), several
+@pytest.mark.parametrize("positive", [False, True], ids=["signed", "positive"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("h,n,dqk,dv", [
+    (257, 320, 64, 64), (129, 320, 128, 128), (520, 257, 32, 32), (2, 768, 64, 64), (4, 1024, 32, 32), (2, 1024, 128, 128), (4, 1024, 128, 64),
+])
+def test_forward_alone_no_larger_than_the_quadratic_kernels(h, n, dqk, dv, dtype, positive, gpu_device):
+    gen = torch.Generator().manual_seed(n + dqk + dv)
+    q, k, v = (torch.randn(1, h, n, d, generator=gen) for d in (dqk, dqk, dv))
+    # (in fp16 the results, up to 2e5 at 1024 rows of 128 positive columns, would leave its range)
+    q, k, v = ((t.abs() if positive else t).mul(s).to(dtype).to(gpu_device) for t, s in ((q, dqk**-0.5), (k, 1.0), (v, 1.0)))
+    with torch.no_grad():
+        chosen = (LinearAttention if dqk == dv else LinearAttentionSmallVHD).apply(q, k, v)
+    other = (kernels.linear_flash_wrapper_fwd if dqk == dv else kernels.linear_flash_wrapper_fwd_smallv_hd)(q, k, v)
+    assert not torch.equal(chosen, other)  # (chunk-wise, at these sizes)
+    want = torch.matmul(torch.matmul(q.double(), k.double().transpose(-2, -1).contiguous()).tril(), v.double())
+    _compare((chosen,), (other,), (want,))
+
+
 # (0.1 and 0.3 are no bf16 numbers; the second-order part alone; a leading constant)
 @pytest.mark.parametrize("normalise", [False, True], ids=["plain", "normalised"])
 @pytest.mark.parametrize("coef", [(1.0, 1.0, 0.5), (0.0, 0.0, 0.5), (0.1, 0.3, 0.7)], ids=str)

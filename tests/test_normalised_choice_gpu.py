@@ -19,10 +19,11 @@ def _recipe(q, k, v, g):
     return (out, *torch.autograd.grad(out, (q, k, v), g.double()))
 
 
-# (B, H, N, D, chunk-wise without gradients): below and from each threshold, ragged lengths
+# (B, H, N, D, chunk-wise without gradients): below and from each threshold, ragged lengths, a single segment per head
 @pytest.mark.parametrize("b,h,n,d,chunked", [
     (1, 2, 1023, 64, False), (1, 2, 1024, 64, True), (1, 1, 1500, 128, False), (1, 1, 2049, 72, True), (2, 2, 4096, 32, True),
     (1, 30, 1500, 64, True), (1, 2, 257, 128, False), (1, 8, 2900, 128, True), (1, 1, 2100, 100, False),
+    (2, 65, 320, 128, True), (1, 128, 320, 128, False), (1, 260, 257, 64, True),
 ])
 def test_choice_and_results(b, h, n, d, chunked, gpu_device):
     gen = torch.Generator().manual_seed(n + d)
