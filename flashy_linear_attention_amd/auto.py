@@ -5,7 +5,8 @@
 returns the same ``tril(Q K^T) V``; it runs the quadratic kernels where they are faster (short
 sequences, few heads) and the chunk-wise ones elsewhere, by the library's table of measured
 thresholds (``fla_linear_attn_prefers_chunked``) and where that narrows no range
-(:func:`chunked_keeps_range`) -- the reference lists autotuning as a to-do (README.md:68).  The
+(:func:`chunked_keeps_range`; an infinite value is infinite or NaN in its column of the results either way, which of the
+two goes by the evaluation) -- the reference lists autotuning as a to-do (README.md:68).  The
 two reference-named Functions choose the same way within the reference's limits on shapes;
 ``kernels.linear_flash_wrapper_*`` are the quadratic kernels whatever the shape.
 """

@@ -19,10 +19,19 @@
  *     the second product, so a single score q_i . k_j above 65504 becomes inf there (and inf * 0
  *     is NaN): keep |q_i . k_j| below that, e.g. by the usual 1/sqrt(D) scaling.  The chunk-wise
  *     entry points also round the running state (sums of k_j v_j^T over the rows before a chunk)
- *     to the storage type, so there the state's elements must fit as well.  The normalised
+ *     to the storage type, so there the state's elements must fit as well (not in the plain forward
+ *     at head dims up to 128 that are multiples of 8, from 257 rows on: it scales that copy of its
+ *     state by the largest finite element).  The normalised
  *     entry points divide in fp32 before the one rounding: their outputs are averages of v and
  *     do not grow with N.  FLA_DTYPE_BF16 has fp32's exponent range and no such limit (the
  *     reference computes in bf16 only, flashlinear/kernels/linear_attn_kernels.py:82,98).
+ *   - Infinite and NaN operands: a forward result that depends on one is infinite or NaN, the others
+ *     are what they would be without it.  An element of v reaches its own column, from its row on
+ *     and in the rows before it of the same 32 (a masked score is multiplied by it too).  Whether
+ *     +inf, -inf or NaN comes out goes by the evaluation: with q and k of either sign one infinite
+ *     v_j leaves a column of the chunk-wise running state with both infinities, and the rows of
+ *     later chunks are NaN in that column, where the quadratic kernels give +inf or -inf by the
+ *     sign of the score.
  *   - `stream` is a hipStream_t (NULL = the null stream).  Calls only enqueue
  *     work; they never synchronise, allocate or free.  Outputs must not alias
  *     inputs or each other: the byte range each tensor spans (first to last

@@ -42,6 +42,25 @@ def test_late_rows_do_not_reach_earlier_ones(op, b, h, n, dqk, dv, late, gpu_dev
         assert torch.equal(a[:, :, :rows], w[:, :, :rows]), name
 
 
+# (forward alone at lengths and head counts that take either evaluation: a single segment per head and several, two column halves)
+@pytest.mark.parametrize("value", [float("inf"), float("-inf"), float("nan")], ids=["inf", "-inf", "nan"])
+@pytest.mark.parametrize("op,h,n,dqk,dv", [
+    ("linear", 2, 512, 64, 64), ("linear", 3, 1024, 64, 64), ("linear", 300, 384, 64, 64), ("linear", 4, 1088, 32, 32),
+    ("linear", 130, 320, 128, 128), ("linear", 100, 640, 128, 128), ("smallv", 3, 1024, 128, 64), ("smallv", 2, 2048, 256, 64),
+])
+def test_a_non_finite_value_keeps_to_its_column(op, h, n, dqk, dv, value, gpu_device):
+    gen = torch.Generator().manual_seed(n + dqk + dv)
+    q, k, v = (torch.randn(1, h, n, d, generator=gen).bfloat16().to(gpu_device) for d in (dqk, dqk, dv))
+    want = OPERATORS[op].apply(q, k, v)
+    row, column = 70, dv - 3
+    v[:, :, row, column] = value
+    got = OPERATORS[op].apply(q, k, v)
+    assert not bool(got[:, :, row:, column].isfinite().any())
+    assert torch.equal(got[:, :, : row // 32 * 32], want[:, :, : row // 32 * 32])
+    others = torch.arange(dv, device=gpu_device) != column
+    assert torch.equal(got[..., others], want[..., others])
+
+
 @pytest.mark.parametrize("normalise", [False, True], ids=["plain", "normalised"])
 @pytest.mark.parametrize("late", [float("nan"), float("inf"), 1e9], ids=["nan", "inf", "huge"])
 @pytest.mark.parametrize("b,h,n,r,dv", [(4, 70, 512, 16, 64), (4, 32, 1024, 8, 32), (1, 6, 1700, 16, 64), (1, 1, 4096, 16, 48)])
