@@ -451,22 +451,30 @@ WalkPlan walk_plan(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, boo
 
 bool sums_on_load(const WalkPlan &w, int most = kSumOnLoadMost) { return w.n_seg >= 3 && w.n_seg <= most; }
 
-// Two workgroups per (b, h) on two column halves of O, on dV and dK (WalkParams::cols, roles), where they would be two segments: q and
-// k (q and dO) come from the L2 that both read through, and no totals of half of the sequence come before the walk.  `plain`: no
-// normaliser and no feature map.
-//   128 columns, two segments -> this.  Forward + backward: B H 128, N 1024 114 / 102 us, N 2048 219 / 204, N 4096 433 / 398, N 8192
-//   857 / 819; B H 112, N 4096 387 / 375; B H 104, N 3072 279 / 268; B H 96, N 1024 98 / 90, N 4096 355 / 350; 72 and 96 columns, B H 88
-//   and 96, N 2048 147 to 150 / 151 to 153; 80 columns, B H 128, N 4096 307 / 316, 96 columns, N 3008 251 / 246.  (dQ's walk as well: B H 128, N 4096 408 -> 422: it starts from what forward left and has no
-//   totals to save.)
-//   Forward alone: B H 88 ... 128, N 1024 31.4 to 36.0 / 27.6 to 29.8, N 2048 50.4 to 64.8 / 49.1 to 57.3, N 3072 77 to 96 / 83 to 98; N 4096
-//   B H 104 107 / 116, B H 120 124.4 / 123.6, B H 128 132 / 127; N 8192 B H 112 236 / 232, B H 128 261 / 247 (the two fall out of step on
-//   long sequences, and each then reads all of q and k from memory).
+// Two workgroups per (b, h) on two column halves of O, on dV and dK (WalkParams::cols, roles), where they would be two segments: no
+// totals of half of the sequence come before the walk.  q and k (q and dO) are read by both, within one XCD: its L2 serves the second
+// read, at B H 128 and N 2048 to 8192 both kernels fetch every operand once (FETCH_SIZE, 403 and 537 MB at N 4096).  A workgroup
+// then walks the whole sequence, at 1.8 to 1.9 us a chunk of 128 columns however many heads there are, where the segments' time
+// grows with the bytes of all heads: hence lines by the head count.  `plain`: no normaliser and no feature map.
+//   Backward, 128 columns, two segments -> this, forward + backward: B H 128, N 1024 114 / 102 us, N 2048 219 / 204, N 8192 857 / 819; B H
+//   112, N 4096 387 / 375; B H 104, N 3072 279 / 268; B H 96, N 1024 98 / 90, N 4096 355 / 350; 72 and 96 columns, B H 88 and 96, N 2048 147
+//   to 150 / 151 to 153; 80 columns, B H 128, N 4096 307 / 316, 96 columns, N 3008 251 / 246.  (dQ's walk as well: B H 128, N 4096
+//   408 -> 422: it starts from what forward left and has no totals to save.)
+//   Forward alone in bf16, inputs that change from pass to pass (with the same ones again and again the Infinity Cache hides the
+//   segments' second read of k and v, up to N 4096): 128 columns, N 2048 B H 97 59.0 / 57.9, B H 128 68.8 / 63.0; N 3072 B H 97 85.0 /
+//   85.1, B H 112 93.9 / 89.0, B H 128 105 / 95; N 4096 B H 104 116 / 114, B H 116 129 / 118, B H 128 136 / 124 (with backward 422 / 411);
+//   N 8192 B H 97 210 / 221, B H 104 222 / 223, B H 112 235 / 230, B H 128 263 / 246; N 16384 B H 116 474 / 469; 96 and 112 columns, B H
+//   105 to 128, N 2560 to 8192 0.99 to 1.11.
+//   In fp16, where a chunk takes 2.1 us (the state's scale), forward alone: N 1024 B H 100 39.2 / 37.9, B H 128 48.0 / 39.8; N 2048 B H 100
+//   65.8 / 68.0, B H 112 69.6 / 68.8, B H 128 77.4 / 74.1; N 3072 B H 112 102 / 106; N 4096 B H 120 139 / 142, B H 128 145 / 145; N 8192 B H
+//   128 276 / 288.
 bool walk_by_columns(const WalkPlan &w, int64_t bh, int64_t N, int64_t dqk, int64_t dv, bool plain) {
     return plain && w.ok && w.split && dqk > 64 && dv > 64 && w.n_seg == 2 && (bh > 96 || N <= 1024) &&
            (N <= 2048 || (dqk >= 96 && dv >= 96));
 }
-bool forward_by_columns(const WalkPlan &w, int64_t bh, int64_t N, int64_t dqk, int64_t dv, bool plain) {
-    return walk_by_columns(w, bh, N, dqk, dv, plain) && (N <= 2048 || (N >= 4096 && bh > 112));
+bool forward_by_columns(const WalkPlan &w, int64_t bh, int64_t N, int64_t dqk, int64_t dv, int dtype, bool plain) {
+    return walk_by_columns(w, bh, N, dqk, dv, plain) &&
+           (dtype == FLA_DTYPE_F16 ? N <= 1024 || (N <= 2048 && bh > 104) : N <= 2048 || bh > 104);
 }
 
 // totals of Y^T Z over the walk's segments into `work`, then the segments' entry states: their sums
@@ -1035,7 +1043,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         (!fmap || fla::fast_path_ok(make_params(mapped[0], mapped[1], v, o, B, H, N, dqk, dv, 0)))) {
         // the segments' entry states; with a feature map the same kernel maps xk as it loads it and
         // writes phi(xk), which the walk then reads (so it runs for a single segment as well)
-        const bool by_columns = forward_by_columns(wp, B * H, N, dqk, dv, !fmap && !nx);
+        const bool by_columns = forward_by_columns(wp, B * H, N, dqk, dv, dtype, !fmap && !nx);
         const bool need_totals = wp.n_seg > 1 || fmap;
         // D = 128: the entry states (and the state after the last chunk) are what backward gets, so the scan writes
         // them to state_out (the totals themselves are computed there, and no workspace is used);

@@ -14,11 +14,12 @@ pytestmark = pytest.mark.gpu
 
 
 # (heads, N, D_qk, D_v): the fewest chunks, an odd number of them, a ragged last one; a second half of 8, 32, 36 and 64 columns;
-# forward by columns and backward not (B H 90), the reverse (N 2049), neither (N 2049, 72 columns)
+# both passes so above 2048 rows (B H 105, and 113 with a long sequence), backward alone (B H 100, N 2049; fp16), neither (B H 90; 72
+# columns above 2048 rows)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
 @pytest.mark.parametrize("h,n,dqk,dv", [
     (128, 257, 128, 128), (97, 320, 72, 128), (100, 451, 96, 96), (128, 1000, 100, 100), (86, 600, 128, 72), (90, 1100, 128, 128),
-    (100, 2049, 104, 96), (100, 2049, 72, 72),
+    (100, 2049, 104, 96), (100, 2049, 72, 72), (105, 2300, 96, 128), (113, 4099, 128, 128),
 ])
 def test_both_passes(h, n, dqk, dv, dtype, gpu_device):
     q, k, v, do = (t.to(gpu_device) for t in reference_style_inputs(1, h, n, dqk, dv, dtype, seed=n + dqk))

@@ -279,6 +279,20 @@ def test_benchmark_shapes(lib):
     assert stats.kernels["walk_fwd_wide_kernel"] >= 1 and stats.kernels["walk_bwd_rev_wide_kernel"] >= 1
 
 
+# (heads, N, width, dtype 0 bf16 / 1 fp16): two column halves in place of two segments, from each line on
+@pytest.mark.parametrize("bh,n,d,dtype,columns", [
+    (86, 1024, 128, 0, True), (96, 1025, 128, 0, False), (97, 2048, 80, 0, True), (104, 2049, 128, 0, False), (105, 2049, 128, 0, True),
+    (128, 3000, 96, 0, True), (128, 3000, 88, 0, False), (113, 4099, 128, 0, True), (85, 1024, 128, 0, False), (129, 2048, 128, 0, False),
+    (86, 1024, 128, 1, True), (104, 1025, 128, 1, False), (105, 2048, 128, 1, True), (128, 2049, 128, 1, False),
+])
+def test_forward_by_columns(lib, bh, n, d, dtype, columns):
+    arena, launches = trace_plain(lib, 1, bh, n, d, d, True, dtype)
+    lp.check_all(arena, launches, lp.Stats())
+    first = next(l for l in launches if l.kernel == "walk_fwd_kernel")
+    assert bool(first.args["a0.cols"]) == columns and bool(first.args["a0.mid_out"]) == columns
+    assert (launches[0].kernel == "walk_totals_kernel") == (not columns and bh < 129)
+
+
 @pytest.mark.parametrize("stride_h", [64, 40], ids=["whole lines", "part of a line"])
 def test_every_part_of_every_head_is_one_workgroups(lib, stride_h):
     """The walks' map over the grid that their launchers take: 16 parts per XCD and 17, and counts off every line."""
