@@ -91,6 +91,24 @@ def _check_waves(report: str, kernel: str, waves: int) -> None:
         raise RuntimeError(f"no resource report for {kernel}: the occupancy check did not run")
 
 
+def _check_scalar_spills(report: str, kernel: str, most: int) -> None:
+    """Fail the build if an instantiation of `kernel` (a part of the mangled name) spills more than `most` scalar registers: each is a
+    v_writelane or v_readlane, in the loop over the chunks where the allocator puts it there.  The map of workgroups to parts
+    (xcd_item) with a division on either side of a branch cost the normalised forward walk 14 (64 columns) and 24 (32) of them and 3 to
+    8 % of its time."""
+    name, seen = None, 0
+    for line in report.splitlines():
+        if "Function Name:" in line:
+            name = line.split("Function Name:")[1].split()[0]
+        elif "SGPRs Spill:" in line and name and kernel in name:
+            seen += 1
+            spills = int(line.split("SGPRs Spill:")[1].split()[0])
+            if spills > most:
+                raise RuntimeError(f"{name} spills {spills} scalar registers, at most {most} so far")
+    if seen == 0:
+        raise RuntimeError(f"no resource report for {kernel}: the check of scalar spills did not run")
+
+
 def _compile_inst(args) -> str:
     dtype, dc, do = args
     obj = os.path.join(OBJ_DIR, f"inst_t{dtype}_c{dc}_o{do}.o")
@@ -107,8 +125,11 @@ def _compile_walk(args) -> str:
     if part == 1:
         _check_no_scratch(report, "walk_bwd_rev_kernel")
         _check_no_scratch(report, "walk_bwd_rev_wide_kernel")
-    else:  # (the plain forward walk at D = 32)
-        _check_waves(report, f"walk_fwd_kernelI{('DF16b', 'DF16_')[dtype]}Li32ELb0ELi0ELb0", 4)
+    else:  # (the plain forward walk at D = 32; the forward walks without a feature map up to 64 columns, the normalised one among them)
+        walk = f"walk_fwd_kernelI{('DF16b', 'DF16_')[dtype]}"
+        _check_waves(report, walk + "Li32ELb0ELi0ELb0", 4)
+        for width, norm, most in ((32, 0, 0), (64, 0, 0), (32, 1, 4), (64, 1, 0), (32, 2, 0), (64, 2, 0)):
+            _check_scalar_spills(report, f"{walk}Li{width}ELb0ELi{norm}ELb0", most)
     return obj
 
 

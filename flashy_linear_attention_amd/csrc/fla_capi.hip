@@ -2144,10 +2144,13 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
 extern "C" {
 
 #if defined(FLA_TRACE_LAUNCHES)
-// The kernels' map of workgroups to (head, part), for all of a grid: `items` receives both of every workgroup (head < 0: none).
-void fla_trace_xcd_items(int grid, int BH, int parts, int64_t stride_h, int32_t *items) {
+// The launchers' choice of a map of workgroups to (head, part), and the kernels' map, for all of a grid: `items` receives both of every
+// workgroup (head < 0: none).
+int fla_trace_xcd_place(int BH, int parts, int64_t stride_h) { return fla::xcd_place(BH, parts, stride_h); }
+uint32_t fla_trace_xcd_inverse(int parts) { return fla::xcd_inverse(parts); }
+void fla_trace_xcd_items(int grid, int BH, int parts, int place, uint32_t inverse, int32_t *items) {  // (inverse 1: the kernel divides)
     for (int wg = 0; wg < grid; ++wg) {
-        const fla::XcdItem item = fla::xcd_item(wg, BH, parts, stride_h);
+        const fla::XcdItem item = inverse == 1 ? fla::xcd_item(wg, BH, parts, place) : fla::xcd_item(wg, BH, parts, place, inverse);
         items[2 * wg] = item.bh, items[2 * wg + 1] = item.part;
     }
 }

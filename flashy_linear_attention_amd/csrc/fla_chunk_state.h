@@ -32,6 +32,7 @@ struct ChunkStateParams {
     int32_t H, N, BH;
     int32_t dc, dout;
     int32_t n_chunks;
+    int32_t place;  // which workgroup takes which chunk (xcd_place), filled by the launcher
     // Feature map on load (fla_feature.h): map_y != 0 replaces every element of Y by phi(element) as
     // the tiles arrive, and writes the mapped rows to `ymap_out` (Y's shape, element strides yo_*) so
     // that the passes after this one read phi(y) instead of mapping again.
@@ -74,7 +75,7 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const ChunkStateParams
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int g = lane >> 5, lam = lane & 15, l32 = lane & 31, beta = (lane >> 4) & 1;
 
-    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_chunks, p.ys_h);
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_chunks, p.place);
     const int bh = item.bh, chunk = item.part;
     if (bh < 0) return;
     const int b = bh / p.H, h = bh - b * p.H;
@@ -271,6 +272,7 @@ hipError_t launch_chunk_state(ChunkStateParams p, hipStream_t stream) {
     } else {
         const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_chunks;
         if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
+        p.place = xcd_place(p.BH, p.n_chunks, p.ys_h);
         constexpr auto kern = chunk_state_kernel<T, DC, DO>;
         constexpr int smem = ChunkStateLds<DC, DO>::kBytes;
         if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;

@@ -90,6 +90,8 @@ struct WalkParams {
     int32_t H, N, BH, wqk, wv;   // true widths of q/k and of v (<= D)
     int32_t n_chunks;            // ceil(N / rows per chunk)
     int32_t seg_chunks, n_seg;   // chunks per segment, segments per (b, h)
+    int32_t place;               // which workgroup takes which segment (walk_place) and xcd_item's factor for n_seg, both filled on the way
+    uint32_t n_seg_inv;          // to the launcher; here and below
     // entry state of every segment, fp32 [BH][n_seg][D (q/k index)][D (v index)]: sum of K^T V over
     // the segments before (forward) / of Q^T dO over the segments after (backward); null when
     // there is a single segment (entry state zero).  init_transposed: the buffer holds the
@@ -935,7 +937,7 @@ struct WalkSlice {
 
 // workgroup -> ((b, h), segment)
 __device__ __forceinline__ WalkSlice walk_slice(const WalkParams &p) {
-    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.ks_h);
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.place, p.n_seg_inv);
     WalkSlice s;
     s.bh = item.bh, s.seg = item.part;
     s.c_lo = s.seg * p.seg_chunks;
@@ -2266,7 +2268,8 @@ struct WalkTotalsParams {
     const void *y, *z;
     int64_t ys_b, ys_h, ys_n, zs_b, zs_h, zs_n;
     int32_t H, N, BH, dy, dz;
-    int32_t n_chunks, seg_chunks, n_seg;
+    int32_t n_chunks, seg_chunks, n_seg, place;
+    uint32_t n_seg_inv;
     int32_t seg_lo, seg_hi;  // only segments seg_lo .. seg_hi - 1 are needed (the others' totals stay unwritten)
     float *totals;
     // two segments: only the total of segment seg_lo is needed, as the other segment's entry state.
@@ -2310,7 +2313,7 @@ __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) unsigned char *)smem;
     const int tid = threadIdx.x, lane = tid & 63, l32 = lane & 31, g = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.ys_h);
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.place, p.n_seg_inv);
     const int bh = item.bh, seg = item.part;
     if (bh < 0) return;
     const int dy = p.dy;
@@ -2630,7 +2633,8 @@ struct WalkGradParams {
     float *dn;                 // fp32 [BH][N]
     int32_t H, N, BH, wqk, wv;
     int32_t vec;               // g and out allow 16-byte loads
-    int32_t n_chunks, seg_chunks, n_seg;
+    int32_t n_chunks, seg_chunks, n_seg, place;
+    uint32_t n_seg_inv;
     float *totals, *rsum;      // [BH][n_seg] states and vectors in the slots the walks read (two segments: partial sums of the
                                // second one's in both; the first one's stay unwritten otherwise); null with a single segment
     int32_t frags;             // WalkTotalsParams::frags
@@ -2654,7 +2658,7 @@ __global__ __launch_bounds__(256, D == 128 ? 1 : 2) void walk_grad_totals_kernel
     float *vd = reinterpret_cast<float *>(smem + (QT + 2) * W::TILE);  // QT tiles of Q, two of dO, two of dn
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.qs_h);
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.place, p.n_seg_inv);
     const int bh = item.bh, seg = item.part;
     if (bh < 0) return;
     // the chunks whose sums are wanted, [a_lo, a_hi), and those that are visited for dO and dn alone, from b_lo on.  Two
@@ -3090,5 +3094,13 @@ hipError_t launch_walk_bwd_rev_wide(const WalkParams &p, hipStream_t stream) {
     else
         return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 4, false>>(grid, smem, p, stream);
 }
+
+template <typename P>
+void walk_place(P &p, int64_t stride_h) {
+    p.place = xcd_place(p.BH, p.n_seg, stride_h), p.n_seg_inv = xcd_inverse(p.n_seg);
+}
+inline void walk_place(int, WalkParams &p) { walk_place(p, p.ks_h); }
+inline void walk_place(int, WalkTotalsParams &p) { walk_place(p, p.ys_h); }
+inline void walk_place(int, WalkGradParams &p) { walk_place(p, p.qs_h); }
 
 }  // namespace fla

@@ -55,13 +55,15 @@ FLA_DECLARE_PAIR(32) FLA_DECLARE_PAIR(64) FLA_DECLARE_PAIR(128)
 #define FLA_DECLARE_WALK_D(fn, P)                                                                    \
     hipError_t FLA_WALK_NAME(fn, 0)(int D, const P &p, hipStream_t stream);                          \
     hipError_t FLA_WALK_NAME(fn, 1)(int D, const P &p, hipStream_t stream);                          \
-    inline hipError_t fn(int dtype, int D, const P &p, hipStream_t stream) {                         \
+    inline hipError_t fn(int dtype, int D, P p, hipStream_t stream) {                                \
+        walk_place(D, p);                                                                            \
         return dtype == 0 ? FLA_WALK_NAME(fn, 0)(D, p, stream) : FLA_WALK_NAME(fn, 1)(D, p, stream); \
     }
 #define FLA_DECLARE_WALK_WIDE(fn)                                                                    \
     hipError_t FLA_WALK_NAME(fn, 0)(const WalkParams &p, hipStream_t stream);                        \
     hipError_t FLA_WALK_NAME(fn, 1)(const WalkParams &p, hipStream_t stream);                        \
-    inline hipError_t fn(int dtype, const WalkParams &p, hipStream_t stream) {                       \
+    inline hipError_t fn(int dtype, WalkParams p, hipStream_t stream) {                              \
+        walk_place(128, p);                                                                          \
         return dtype == 0 ? FLA_WALK_NAME(fn, 0)(p, stream) : FLA_WALK_NAME(fn, 1)(p, stream);       \
     }
 FLA_DECLARE_WALK_D(walk_totals, WalkTotalsParams)

@@ -50,6 +50,8 @@ struct PolyWalkParams {
     int64_t us_b, us_h, us_n;  // out
     int64_t dqs_b, dqs_h, dqs_n, dks_b, dks_h, dks_n, dvs_b, dvs_h, dvs_n;
     int32_t H, N, BH, r, wv, n_chunks, seg_chunks, n_seg;
+    int32_t place;  // which workgroup takes which segment (xcd_place) and xcd_item's factor for n_seg, filled by the launcher
+    uint32_t n_seg_inv;
     float c0, c1, c2, eps;
     int32_t wide_out;  // dq, dk, dv are floats (and receive the bf16-rounded values)
     float *denom;  // fp32 [BH][N], or null: not normalised.  Forward writes it, backward reads it
@@ -481,7 +483,7 @@ struct PolySlice {
     bool valid;
 };
 __device__ __forceinline__ PolySlice poly_slice(const PolyWalkParams &p) {  // (walk_slice's map)
-    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.ks_h);
+    const XcdItem item = xcd_item(blockIdx.x, p.BH, p.n_seg, p.place, p.n_seg_inv);
     PolySlice s;
     s.bh = item.bh, s.seg = item.part;
     s.c_lo = s.seg * p.seg_chunks;
@@ -1197,7 +1199,8 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
 }
 
 template <auto kern>
-hipError_t launch_poly_kernel(const PolyWalkParams &p, int smem, hipStream_t stream) {
+hipError_t launch_poly_kernel(PolyWalkParams p, int smem, hipStream_t stream) {
+    p.place = xcd_place(p.BH, p.n_seg, p.ks_h), p.n_seg_inv = xcd_inverse(p.n_seg);
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;

@@ -26,7 +26,7 @@ FLA_FIELDS_BEGIN(TriParams)
 FLA_FIELD(x) FLA_FIELD(y) FLA_FIELD(z) FLA_FIELD(out)
 FLA_FIELD(xs_b) FLA_FIELD(xs_h) FLA_FIELD(xs_n) FLA_FIELD(ys_b) FLA_FIELD(ys_h) FLA_FIELD(ys_n)
 FLA_FIELD(zs_b) FLA_FIELD(zs_h) FLA_FIELD(zs_n) FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n)
-FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(dc) FLA_FIELD(dout) FLA_FIELD(upper) FLA_FIELD(n_tiles)
+FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(dc) FLA_FIELD(dout) FLA_FIELD(upper) FLA_FIELD(place) FLA_FIELD(n_tiles)
 FLA_FIELD(single) FLA_FIELD(vec_x) FLA_FIELD(vec_y) FLA_FIELD(vec_z) FLA_FIELD(vec_out) FLA_FIELD(state)
 FLA_FIELD(state_transposed) FLA_FIELD(denom) FLA_FIELD(eps) FLA_FIELD(poly_on) FLA_FIELD(map_x) FLA_FIELD(map_out)
 FLA_FIELD(xmap_out) FLA_FIELD(xo_b) FLA_FIELD(xo_h) FLA_FIELD(xo_n) FLA_FIELD(omap) FLA_FIELD(ms_b) FLA_FIELD(ms_h)
@@ -64,7 +64,7 @@ FLA_FIELD(vs_b) FLA_FIELD(vs_h) FLA_FIELD(vs_n) FLA_FIELD(gs_b) FLA_FIELD(gs_h) 
 FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n) FLA_FIELD(dqs_b) FLA_FIELD(dqs_h) FLA_FIELD(dqs_n)
 FLA_FIELD(dks_b) FLA_FIELD(dks_h) FLA_FIELD(dks_n) FLA_FIELD(dvs_b) FLA_FIELD(dvs_h) FLA_FIELD(dvs_n)
 FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(wqk) FLA_FIELD(wv) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks)
-FLA_FIELD(n_seg) FLA_FIELD(init) FLA_FIELD(init_transposed) FLA_FIELD(saved) FLA_FIELD(fmap) FLA_FIELD(qmap_out)
+FLA_FIELD(n_seg) FLA_FIELD(place) FLA_FIELD(n_seg_inv) FLA_FIELD(init) FLA_FIELD(init_transposed) FLA_FIELD(saved) FLA_FIELD(fmap) FLA_FIELD(qmap_out)
 FLA_FIELD(qo_b) FLA_FIELD(qo_h) FLA_FIELD(qo_n) FLA_FIELD(slope_y) FLA_FIELD(sy_b) FLA_FIELD(sy_h) FLA_FIELD(sy_n)
 FLA_FIELD(denom) FLA_FIELD(eps) FLA_FIELD(zc) FLA_FIELD(dn) FLA_FIELD(rc) FLA_FIELD(total_out) FLA_FIELD(xinit)
 FLA_FIELD(xtotal) FLA_FIELD(accumulate)
@@ -79,7 +79,7 @@ FLA_FIELDS_END
 FLA_FIELDS_BEGIN(WalkTotalsParams)
 FLA_FIELD(y) FLA_FIELD(z) FLA_FIELD(ys_b) FLA_FIELD(ys_h) FLA_FIELD(ys_n) FLA_FIELD(zs_b) FLA_FIELD(zs_h)
 FLA_FIELD(zs_n) FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(dy) FLA_FIELD(dz) FLA_FIELD(n_chunks)
-FLA_FIELD(seg_chunks) FLA_FIELD(n_seg) FLA_FIELD(seg_lo) FLA_FIELD(seg_hi) FLA_FIELD(totals) FLA_FIELD(direct)
+FLA_FIELD(seg_chunks) FLA_FIELD(n_seg) FLA_FIELD(place) FLA_FIELD(n_seg_inv) FLA_FIELD(seg_lo) FLA_FIELD(seg_hi) FLA_FIELD(totals) FLA_FIELD(direct)
 FLA_FIELD(map_y) FLA_FIELD(ymap_out) FLA_FIELD(yo_b) FLA_FIELD(yo_h) FLA_FIELD(yo_n) FLA_FIELD(y2) FLA_FIELD(dy2)
 FLA_FIELD(totals2) FLA_FIELD(dz2) FLA_FIELD(z_narrow) FLA_FIELD(vsum) FLA_FIELD(frags)
 FLA_FIELDS_END
@@ -93,13 +93,13 @@ FLA_FIELDS_BEGIN(WalkGradParams)
 FLA_FIELD(q) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(qs_b) FLA_FIELD(qs_h) FLA_FIELD(qs_n) FLA_FIELD(gs_b) FLA_FIELD(gs_h)
 FLA_FIELD(gs_n) FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n) FLA_FIELD(denom) FLA_FIELD(dout) FLA_FIELD(dn) FLA_FIELD(H)
 FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(wqk) FLA_FIELD(wv) FLA_FIELD(vec) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks)
-FLA_FIELD(n_seg) FLA_FIELD(totals) FLA_FIELD(rsum) FLA_FIELD(frags) FLA_FIELD(keep_g)
+FLA_FIELD(n_seg) FLA_FIELD(place) FLA_FIELD(n_seg_inv) FLA_FIELD(totals) FLA_FIELD(rsum) FLA_FIELD(frags) FLA_FIELD(keep_g)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(ChunkStateParams)
 FLA_FIELD(y) FLA_FIELD(z) FLA_FIELD(w) FLA_FIELD(ys_b) FLA_FIELD(ys_h) FLA_FIELD(ys_n) FLA_FIELD(zs_b) FLA_FIELD(zs_h)
 FLA_FIELD(zs_n) FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(dc) FLA_FIELD(dout) FLA_FIELD(n_chunks)
-FLA_FIELD(map_y) FLA_FIELD(ymap_out) FLA_FIELD(yo_b) FLA_FIELD(yo_h) FLA_FIELD(yo_n)
+FLA_FIELD(place) FLA_FIELD(map_y) FLA_FIELD(ymap_out) FLA_FIELD(yo_b) FLA_FIELD(yo_h) FLA_FIELD(yo_n)
 FLA_FIELDS_END
 
 FLA_FIELDS_BEGIN(PackItem)
@@ -110,7 +110,7 @@ FLA_FIELDS_END
 FLA_FIELDS_BEGIN(PolyWalkParams)
 FLA_FIELD(q) FLA_FIELD(k) FLA_FIELD(v) FLA_FIELD(go) FLA_FIELD(o) FLA_FIELD(out) FLA_FIELD(dq) FLA_FIELD(dk) FLA_FIELD(dv)
 FLA_FIELD(H) FLA_FIELD(N) FLA_FIELD(BH) FLA_FIELD(r) FLA_FIELD(wv) FLA_FIELD(n_chunks) FLA_FIELD(seg_chunks) FLA_FIELD(n_seg)
-FLA_FIELD(denom) FLA_FIELD(totals) FLA_FIELD(sum_entries) FLA_FIELD(u_totals) FLA_FIELD(entries) FLA_FIELD(wide_out)
+FLA_FIELD(place) FLA_FIELD(n_seg_inv) FLA_FIELD(denom) FLA_FIELD(totals) FLA_FIELD(sum_entries) FLA_FIELD(u_totals) FLA_FIELD(entries) FLA_FIELD(wide_out)
 FLA_FIELD(qs_b) FLA_FIELD(qs_h) FLA_FIELD(qs_n) FLA_FIELD(ks_b) FLA_FIELD(ks_h) FLA_FIELD(ks_n) FLA_FIELD(vs_b) FLA_FIELD(vs_h)
 FLA_FIELD(vs_n) FLA_FIELD(gs_b) FLA_FIELD(gs_h) FLA_FIELD(gs_n) FLA_FIELD(os_b) FLA_FIELD(os_h) FLA_FIELD(os_n) FLA_FIELD(us_b)
 FLA_FIELD(us_h) FLA_FIELD(us_n) FLA_FIELD(dqs_b) FLA_FIELD(dqs_h) FLA_FIELD(dqs_n) FLA_FIELD(dks_b) FLA_FIELD(dks_h)

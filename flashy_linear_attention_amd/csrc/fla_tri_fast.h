@@ -85,18 +85,30 @@ constexpr int kWholeHeadParts = 16;
 struct XcdItem {
     int bh, part;
 };
-__host__ __device__ __forceinline__ XcdItem xcd_item(int wg, int BH, int parts, int64_t stride_h) {
-    const int xcd = wg & 7, slot = wg >> 3;
-    if (BH % 8 == 0 || ((BH + 7) >> 3) * parts <= kWholeHeadParts) {
-        const int hl = slot / parts;
-        const bool pairs = BH % 16 == 0 && stride_h % 64 != 0;
-        const int bh = pairs ? (hl >> 1) * 16 + xcd * 2 + (hl & 1) : hl * 8 + xcd;
-        return {bh < BH ? bh : -1, slot - hl * parts};
-    }
-    const int total = BH * parts, share = (total + 7) >> 3, item = xcd * share + slot;
-    if (slot >= share || item >= total) return {-1, 0};
-    const int bh = item / parts;
-    return {bh, item - bh * parts};
+// The map as one number, by the launcher (the kernels' `place`): 0 whole heads, every eighth; -1 whole heads, pairs of neighbours; else
+// runs, so many parts per XCD.
+inline int32_t xcd_place(int64_t BH, int64_t parts, int64_t stride_h) {
+    if (BH % 8 == 0) return BH % 16 == 0 && stride_h % 64 != 0 ? -1 : 0;
+    return (BH + 7) / 8 * parts <= kWholeHeadParts ? 0 : (int32_t)((BH * parts + 7) / 8);
+}
+// 2^32 / parts, rounded up: with it floor(item / parts) is the upper half of a product, exact while item parts < 2^32 (walks: 512
+// workgroups at a time or one part per head).  0: of one part.
+inline uint32_t xcd_inverse(int parts) { return parts > 1 ? (uint32_t)(((1ull << 32) + parts - 1) / parts) : 0; }
+// (The choice of the map and a division on either side of it, made in the kernels, cost every launch 0.07 us, and the normalised forward
+// walk spilled 14 (64 columns) and 24 (32) scalar registers into its chunk loop: B H 64, N 2048 23.3 -> 22.6 us, N 1443 20.1 -> 19.5, 32
+// columns 13.3 -> 12.5 without)
+__host__ __device__ __forceinline__ XcdItem xcd_item_at(uint32_t xcd, uint32_t slot, uint32_t item, uint32_t head, int BH, int parts, int place) {
+    const uint32_t p2 = place < 0, whole = ((head >> p2) << (3 + p2)) + (xcd << p2) + (head & p2);  // (pairs of heads, or single ones)
+    const uint32_t bh = place > 0 ? head : whole, end = place > 0 ? (uint32_t)place : ~0u;
+    return {bh < (uint32_t)BH && slot < end ? (int)bh : -1, (int)(item - head * parts)};
+}
+__host__ __device__ __forceinline__ XcdItem xcd_item(int wg, int BH, int parts, int place, uint32_t inverse) {
+    const uint32_t xcd = wg & 7, slot = wg >> 3, item = (place > 0 ? xcd * place : 0) + slot;
+    return xcd_item_at(xcd, slot, item, (uint32_t)(((uint64_t)item * inverse) >> 32) + (inverse ? 0 : item), BH, parts, place);
+}
+__host__ __device__ __forceinline__ XcdItem xcd_item(int wg, int BH, int parts, int place) {  // (any number of parts)
+    const uint32_t xcd = wg & 7, slot = wg >> 3, item = (place > 0 ? xcd * place : 0) + slot;
+    return xcd_item_at(xcd, slot, item, item / (uint32_t)parts, BH, parts, place);
 }
 
 // s_waitcnt vmcnt(N) only (expcnt and lgkmcnt fields left at their maxima): returns once at
@@ -264,7 +276,7 @@ __device__ __forceinline__ void tri_fast_body(const TriParams &p, const int wg_i
     // same time).  Single tiles differ in work, so they are ordered heaviest first across all
     // heads: whatever CU frees up next takes the heaviest tile left.
     const int n_hl = (p.BH + 7) >> 3;
-    const XcdItem chunk = chunked ? xcd_item(wg, p.BH, p.n_tiles, p.ys_h) : XcdItem{0, 0};
+    const XcdItem chunk = chunked ? xcd_item(wg, p.BH, p.n_tiles, p.place) : XcdItem{0, 0};
     const int hl = single ? slot % n_hl : slot / n_pairs;
     const int rank = chunked ? chunk.part : single ? slot / n_hl : slot - hl * n_pairs;
     const int bh = chunked ? chunk.bh : hl * 8 + xcd;
@@ -1104,7 +1116,7 @@ hipError_t launch_tri_fast_variant(TriParams p, hipStream_t stream) {
         return hipErrorNotSupported;
     } else {
         if (CHUNKED && p.state_transposed && !Cfg::kStateTransposable) return hipErrorNotSupported;
-        p.n_tiles = (p.N + Cfg::BM - 1) / Cfg::BM;
+        p.n_tiles = (p.N + Cfg::BM - 1) / Cfg::BM, p.place = xcd_place(p.BH, p.n_tiles, p.ys_h);
         p.single = (!CHUNKED && run_single_tiles((int64_t)p.BH * ((p.n_tiles + 1) / 2), Cfg::kMinWavesPerSimd)) ? 1 : 0;
         const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * ((CHUNKED || p.single) ? p.n_tiles : (p.n_tiles + 1) / 2);
         if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
@@ -1144,7 +1156,7 @@ hipError_t launch_tri_fast_chunked_batch(TriBatch b, int count, hipStream_t stre
         const int n_tiles = (b.p[0].N + Cfg::BM - 1) / Cfg::BM;
         for (int i = 0; i < count; ++i) {
             if (!b.p[i].state || (b.p[i].state_transposed && !Cfg::kStateTransposable)) return hipErrorNotSupported;
-            b.p[i].n_tiles = n_tiles, b.p[i].single = 0;
+            b.p[i].n_tiles = n_tiles, b.p[i].single = 0, b.p[i].place = xcd_place(b.p[i].BH, n_tiles, b.p[i].ys_h);
         }
         const int64_t grid = (int64_t)8 * ((b.p[0].BH + 7) / 8) * n_tiles;
         if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;

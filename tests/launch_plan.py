@@ -50,7 +50,9 @@ def trace_lib(rebuild: bool = False) -> ctypes.CDLL:
             fn.restype = restype
         lib.fla_trace_take.argtypes = [ctypes.c_char_p, ctypes.c_int64]
         lib.fla_trace_take.restype = ctypes.c_int64
-        lib.fla_trace_xcd_items.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_void_p]
+        lib.fla_trace_xcd_place.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64]
+        lib.fla_trace_xcd_items.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_uint32, ctypes.c_void_p]
+        lib.fla_trace_xcd_inverse.restype = ctypes.c_uint32
         lib.fla_trace_xcd_items.restype = None
         _trace_lib = lib
     return _trace_lib
@@ -252,17 +254,24 @@ def tensor_extent(p: Dict, ptr: str, sb: str, sh: str, sn: str, H: int, BH: int,
 # ---------------------------------------------------------------------------------------------
 # workgroups -> (head, part): csrc/fla_tri_fast.h, xcd_item
 
-def xcd_items(grid: int, BH: int, parts: int, stride_h: int) -> np.ndarray:
+def xcd_items(grid: int, BH: int, parts: int, place: int, inverse: Optional[int] = None) -> np.ndarray:
     """(head, part) of every workgroup of a grid, by the kernels' own function; head -1: none.  Every part of every head is one
-    workgroup's and no other's."""
+    workgroup's and no other's.  `inverse`: the factor that the launch brings for its number of parts (None: the kernel divides)."""
     items = np.empty((grid, 2), dtype=np.int32)
-    trace_lib().fla_trace_xcd_items(grid, BH, parts, stride_h, items.ctypes.data)
+    trace_lib().fla_trace_xcd_items(grid, BH, parts, place, 1 if inverse is None else inverse, items.ctypes.data)
     used = items[items[:, 0] >= 0]
-    where = f"{BH} heads of {parts} parts, {stride_h} elements apart"
+    where = f"{BH} heads of {parts} parts, place {place}"
     assert (used[:, 0] < BH).all() and (used[:, 1] >= 0).all() and (used[:, 1] < parts).all(), f"{where}: outside them"
     times = np.bincount(used[:, 0].astype(np.int64) * parts + used[:, 1], minlength=BH * parts)
     assert (times == 1).all(), f"{where}: {int((times > 1).sum())} taken twice, {int((times == 0).sum())} not at all"
     return items
+
+
+def check_place(l: "Launch", p: Dict, parts: int, stride_h: int) -> None:
+    """The launch's map is the one that its heads and parts ask for."""
+    want = trace_lib().fla_trace_xcd_place(p["BH"], parts, stride_h)
+    assert p["place"] == want, f"{l.kernel}: place {p['place']}, not {want}"
+    xcd_items(l.grid[0], p["BH"], parts, p["place"], p.get("n_seg_inv"))
 
 
 # ---------------------------------------------------------------------------------------------
@@ -397,7 +406,9 @@ def model_tri_fast(arena: Arena, l: Launch, p: Dict, T: str, DC: int, DO: int, c
     # every workgroup index: its head and row tiles.  Heads differ in their base addresses only, so
     # the lane-level part runs for the first heads, the last one and every rank.
     sample_ranks = {0, 1, n_pairs // 2, n_pairs - 2, n_pairs - 1}
-    items = xcd_items(l.grid[0], BH, n_tiles, p["ys_h"]).tolist() if chunked else None
+    if chunked:
+        check_place(l, p, n_tiles, p["ys_h"])
+        items = xcd_items(l.grid[0], BH, n_tiles, p["place"]).tolist()
     for wg in range(l.grid[0]):
         xcd, slot = wg & 7, wg >> 3
         if chunked:
@@ -779,7 +790,7 @@ def model_walk(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats) -> None:
     assert seg_chunks >= 1 and n_seg >= 1 and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks, \
         f"{l.kernel}: {n_seg} segments of {seg_chunks} chunks do not tile {n_chunks} chunks"
     assert l.grid[0] == 8 * ((BH + 7) // 8) * n_seg
-    xcd_items(l.grid[0], BH, n_seg, p["ks_h"])
+    check_place(l, p, n_seg, p["ks_h"])
     resident = 256 if D > 64 else 512
     assert BH * n_seg <= max(resident, BH), f"{l.kernel}: {BH * n_seg} workgroups for {resident} resident"
     # (pairs of column halves, grid y: a q / k of 128 + wqk2 columns, a v of 128 + wv2)
@@ -910,7 +921,7 @@ def model_walk_totals(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats, bo
     assert n_chunks == -(-N // rows) and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks
     assert 0 <= p["seg_lo"] <= p["seg_hi"] <= n_seg
     assert l.grid[0] == 8 * ((BH + 7) // 8) * n_seg
-    xcd_items(l.grid[0], BH, n_seg, p["ys_h"])
+    check_place(l, p, n_seg, p["ys_h"])
     operands = [("y", "y", "ys_b", "ys_h", "ys_n", p["dy"]), ("z", "z", "zs_b", "zs_h", "zs_n", p["dz"])]
     if p["y2"]:  # a second Y operand (the other half of a wide q / k) in the same launch
         # (grid y picks the operand, or -- the kernel built for it -- every workgroup takes both: three sets of three tiles)
@@ -935,7 +946,7 @@ def model_walk_grad_totals(arena: Arena, l: Launch, p: Dict, D: int, vec: bool, 
     n_chunks, seg_chunks, n_seg = p["n_chunks"], p["seg_chunks"], p["n_seg"]
     assert n_chunks == -(-N // rows) and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks
     assert l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
-    xcd_items(l.grid[0], BH, n_seg, p["qs_h"])
+    check_place(l, p, n_seg, p["qs_h"])
     assert l.lds == ((2 if D == 128 else 1) + 3) * rows * 2 * D + 2 * rows * 4, f"{l.kernel}: {l.lds} bytes of LDS"
     assert 1 <= wqk <= D and 1 <= wv <= D and wqk % 8 == 0 and wv % 8 == 0
     assert p["q"] % 16 == 0 and p["qs_n"] % 8 == 0 and p["dout"] % 16 == 0 and N * p["qs_n"] * 2 <= 0x3fffffff
@@ -967,7 +978,7 @@ def model_poly(arena: Arena, l: Launch, p: Dict, backward: bool, stats: Stats) -
     """The polynomial map's kernels: every operand, result and state that the kernel touches."""
     H, BH, N, n_seg = p["H"], p["BH"], p["N"], p["n_seg"]
     assert p["n_chunks"] == -(-N // 128) and l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
-    xcd_items(l.grid[0], BH, n_seg, p["ks_h"])
+    check_place(l, p, n_seg, p["ks_h"])
     assert (n_seg - 1) * p["seg_chunks"] < p["n_chunks"] <= n_seg * p["seg_chunks"]
     widths = {"q": p["r"], "k": p["r"], "v": p["wv"], "go": p["wv"], "o": p["wv"], "out": p["wv"], "dq": p["r"], "dk": p["r"],
               "dv": p["wv"]}
@@ -1040,6 +1051,7 @@ class StateForms:
 def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
     """Every launch of a call: the general limits, then the kernel's model."""
     forms = StateForms()
+    last_totals = None  # the last totals kernel's parameters
     grads = None  # the normalised backward's first pass, ahead of the walk that reads what it left
     poly_totals = {}  # by address: the kernel that wrote them last, and their direction
     for l in launches:
@@ -1092,6 +1104,8 @@ def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
             p = l.struct("a0")
             model_walk(arena, l, p, t[1], stats)
             forms.walk(l, p, t[1])
+            if last_totals and p["init"] and p["init"] == last_totals["totals"] and p["BH"] % 8:  # (from the L2 that they were written through)
+                assert p["place"] == last_totals["place"], f"{k}: placed otherwise than its totals"
             if k == "walk_bwd_kernel" and grads:  # dO of its own, or g and n where it was not written
                 place = {"go": grads["go"], "gn": grads["denom"]} if grads["keep_g"] else {"go": grads["dout"], "gn": 0}
                 assert all(p[nm] == at for nm, at in place.items()), "the walk reads another dO than the pass ahead of it left"
@@ -1113,6 +1127,7 @@ def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
         elif k == "walk_totals_kernel":
             p = l.struct("a0")
             model_walk_totals(arena, l, p, t[1], stats, both=len(t) > 4 and bool(t[4]))
+            last_totals = p
             forms.wrote(p["totals"], p["frags"]), forms.wrote(p["totals2"], p["frags"])
         elif k == "walk_totals_quad_kernel":
             p = l.struct("a0")
@@ -1137,7 +1152,7 @@ def check_all(arena: Arena, launches: List[Launch], stats: Stats) -> None:
                 poly_totals[p["totals"]] = backward
         elif k == "chunk_state_kernel":
             p = l.struct("a0")
-            xcd_items(l.grid[0], p["BH"], p["n_chunks"], p["ys_h"])
+            check_place(l, p, p["n_chunks"], p["ys_h"])
             for nm in ("y", "z"):
                 assert arena.find(p[nm]) is not None, f"{k}: {nm} points nowhere"
         elif k == "poly_scan_kernel":

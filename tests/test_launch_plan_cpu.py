@@ -295,15 +295,27 @@ def test_forward_by_columns(lib, bh, n, d, dtype, columns):
 
 @pytest.mark.parametrize("stride_h", [64, 40], ids=["whole lines", "part of a line"])
 def test_every_part_of_every_head_is_one_workgroups(lib, stride_h):
-    """The walks' map over the grid that their launchers take: 16 parts per XCD and 17, and counts off every line."""
+    """The walks' map over the grid that their launchers take: the last number of parts that keeps heads whole, the next, and counts
+    off every line."""
     for bh in [*range(1, 70), 72, 80, 96, 100, 112, 127, 128, 129, 191, 192, 255, 256, 257, 300]:
         for parts in [*range(1, 21), 31, 32, 33, 63, 64]:
-            items = lp.xcd_items(8 * ((bh + 7) // 8) * parts, bh, parts, stride_h)
-            per_xcd = [int((items[x::8, 0] >= 0).sum()) for x in range(8)]
+            place = lib.fla_trace_xcd_place(bh, parts, stride_h)
+            items = lp.xcd_items(8 * ((bh + 7) // 8) * parts, bh, parts, place, lib.fla_trace_xcd_inverse(parts))
+            if parts in (1, 7, 64):
+                assert (items == lp.xcd_items(8 * ((bh + 7) // 8) * parts, bh, parts, place)).all()
             if bh % 8 == 0 or (bh + 7) // 8 * parts <= 16:  # whole heads
+                assert place == (-1 if bh % 16 == 0 and stride_h == 40 else 0)
                 assert all(len(set(np.flatnonzero(items[:, 0] == head) % 8)) == 1 for head in {0, bh // 2, bh - 1})
             else:  # an eighth of the parts each
-                assert max(per_xcd) == -(-bh * parts // 8)
+                assert place == -(-bh * parts // 8)
+
+
+@pytest.mark.parametrize("parts", [2, 3, 5, 7, 17, 31, 33, 127, 255, 511, 512])
+def test_the_factor_in_place_of_a_division(lib, parts):
+    """Exact for every item of a walk: 512 workgroups at a time or one part per head."""
+    items = np.arange(0, 512 * 8 * 512, 1 if parts < 10 else 13, dtype=np.uint64)
+    assert ((items * np.uint64(lib.fla_trace_xcd_inverse(parts))) >> np.uint64(32) == items // np.uint64(parts)).all()
+    assert lib.fla_trace_xcd_inverse(1) == 0
 
 
 def test_empty_problems_make_no_launch(lib):
