@@ -493,9 +493,9 @@ struct EntryHalf {
 int walk_entry_states(const WalkPlan &w, const View &y, const View &z, int64_t B, int64_t H, int64_t N, int64_t dy,
                       int64_t dz, int dtype, int reverse, void *work, float *entry, const float **where, hipStream_t s,
                       int map_y = 0, const View *ymap_out = nullptr, const EntryHalf *second = nullptr,
-                      bool totals_only = false, bool z_narrow = false, float *vsum = nullptr) {
+                      bool totals_only = false, bool z_narrow = false, float *vsum = nullptr, bool alone = false) {
     fla::WalkTotalsParams tp{};
-    tp.vsum = vsum;
+    tp.vsum = vsum, tp.alone = alone;
     tp.z_narrow = z_narrow;
     if (map_y) {
         tp.map_y = map_y, tp.ymap_out = const_cast<void *>(ymap_out->ptr);
@@ -1064,7 +1064,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
                                            in_state && !sum_on_load ? state_out : workspace,
                                            in_state && !sum_on_load ? static_cast<float *>(state_out) : nullptr, &entry, s,
                                            fmap, fmap ? &mapped[1] : nullptr, nullptr, sum_on_load, false,
-                                           nx ? static_cast<float *>(nx->vec) : nullptr))
+                                           nx ? static_cast<float *>(nx->vec) : nullptr, !state_out))
                 return rc;
         const View &kk = fmap ? mapped[1] : k;
         fla::WalkParams w{};
@@ -2146,7 +2146,7 @@ extern "C" {
 #if defined(FLA_TRACE_LAUNCHES)
 // The launchers' choice of a map of workgroups to (head, part), and the kernels' map, for all of a grid: `items` receives both of every
 // workgroup (head < 0: none).
-int fla_trace_xcd_place(int BH, int parts, int64_t stride_h) { return fla::xcd_place(BH, parts, stride_h); }
+int fla_trace_xcd_place(int BH, int parts, int64_t stride_h, int most, int resident) { return fla::xcd_place(BH, parts, stride_h, most, resident); }
 uint32_t fla_trace_xcd_inverse(int parts) { return fla::xcd_inverse(parts); }
 void fla_trace_xcd_items(int grid, int BH, int parts, int place, uint32_t inverse, int32_t *items) {  // (inverse 1: the kernel divides)
     for (int wg = 0; wg < grid; ++wg) {

@@ -2294,6 +2294,7 @@ struct WalkTotalsParams {
     float *vsum;
     // the totals are written by fragments (walk_write_frags): the walks add them up as they start
     int32_t frags;
+    int32_t alone;  // of a forward that hands no states over (walk_whole_parts)
     // nobody reads the totals' columns 64 .. (every walk behind them leaves a narrow z's padding out): they may stay
     // unwritten for a narrow y as well
     int32_t z_narrow;
@@ -3095,12 +3096,27 @@ hipError_t launch_walk_bwd_rev_wide(const WalkParams &p, hipStream_t stream) {
         return launch_walk_kernel<walk_bwd_rev_wide_kernel<T, 4, false>>(grid, smem, p, stream);
 }
 
-template <typename P>
-void walk_place(P &p, int64_t stride_h) {
-    p.place = xcd_place(p.BH, p.n_seg, stride_h), p.n_seg_inv = xcd_inverse(p.n_seg);
+// xcd_place's line for a launch of walks or of their totals, D <= 64: whole heads up to twice as many parts, as many as an XCD has CUs (two
+// workgroups share a CU), for the normalised operator and where a forward walk without a backward adds up its head's totals as it
+// starts; at D = 32 in both passes.  Passes that hand states over go by the same line: a plain forward with whole heads in front of
+// a backward in runs, D = 64, took up to 10 % longer than both in runs (B H 15 N 2048 29.4 us, 26.8; both with whole heads 26.8).
+// Runs -> whole heads, 17 to 32 parts on the fullest XCD, N 1100 to 4083, device time: normalised forward B H 1 N 4083 15.6 -> 13.7,
+// B H 7 N 3500 16.1 -> 13.8, B H 9 N 2048 12.9 -> 11.8, D = 32 B H 9 N 2048 10.1 -> 9.1; with backward B H 15 N 2048 38.0 -> 33.8, D = 32
+// 27.1 -> 23.4.  Plain forward B H 7 N 4083 13.9 -> 12.7, B H 12 N 2048 10.7 -> 10.8, D = 32 B H 9 N 2048 8.6 -> 8.0; D = 32 from 17 segments
+// on, whose totals another kernel adds up, B H 4 N 4083 11.2 -> 11.8.  Plain, with backward: B H 4 N 4083 27.7 -> 30.4, B H 7 N 3000 27.9
+// -> 27.0, B H 12 N 2048 25.0 -> 26.4, but D = 32 B H 9 N 1500 17.2 -> 16.5, B H 12 N 2048 18.5 -> 18.8.
+inline int walk_whole_parts(int D, int n_seg, bool norm, bool alone) {
+    return D <= 64 && (norm || (n_seg <= walk_sum_on_load_max(D) && (alone || D == 32))) ? 2 * kWholeHeadParts : kWholeHeadParts;
 }
-inline void walk_place(int, WalkParams &p) { walk_place(p, p.ks_h); }
-inline void walk_place(int, WalkTotalsParams &p) { walk_place(p, p.ys_h); }
-inline void walk_place(int, WalkGradParams &p) { walk_place(p, p.qs_h); }
+// ... and the workgroups that an XCD holds, where the totals are added up as the walks start (D = 128: kSumOnLoadMost)
+inline int walk_resident(int D, int n_seg) { return n_seg > (D <= 64 ? walk_sum_on_load_max(D) : 20) ? 0 : D <= 64 ? 64 : 32; }
+template <typename P>
+void walk_place(int D, P &p, int64_t stride_h, bool norm, bool alone) {
+    p.place = xcd_place(p.BH, p.n_seg, stride_h, walk_whole_parts(D, p.n_seg, norm, alone), walk_resident(D, p.n_seg));
+    p.n_seg_inv = xcd_inverse(p.n_seg);
+}
+inline void walk_place(int D, WalkParams &p) { walk_place(D, p, p.ks_h, p.denom || p.dn, !p.saved); }
+inline void walk_place(int D, WalkTotalsParams &p) { walk_place(D, p, p.ys_h, p.vsum != nullptr, p.alone); }
+inline void walk_place(int D, WalkGradParams &p) { walk_place(D, p, p.qs_h, true, false); }
 
 }  // namespace fla

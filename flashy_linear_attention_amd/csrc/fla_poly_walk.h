@@ -1200,7 +1200,7 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
 
 template <auto kern>
 hipError_t launch_poly_kernel(PolyWalkParams p, int smem, hipStream_t stream) {
-    p.place = xcd_place(p.BH, p.n_seg, p.ks_h), p.n_seg_inv = xcd_inverse(p.n_seg);
+    p.place = xcd_place(p.BH, p.n_seg, p.ks_h, kWholeHeadParts, p.n_seg <= 20 ? 32 : 0), p.n_seg_inv = xcd_inverse(p.n_seg);  // (kSumOnLoadPoly)
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     if (hipError_t e = ensure_dynamic_lds<kern>(smem)) return e;

@@ -72,11 +72,18 @@ __device__ __forceinline__ void dma_16B_per_lane(u32x4 rsrc, uint32_t lds_base, 
 //     of 16 bits from a head to the next), pairs of neighbours, which share those lines in (B, N, H, D) storage.  Forward + backward:
 //     32 columns, B 2 H 16 N 8192 76.4 -> 67.2 us; 96 columns, B 2 H 24 N 4096 153 -> 148.  (Pairs for every row: 64 columns, B 1 H 16
 //     N 32768 in that storage 241 -> 232 us, but with a feature map B 4 H 16 N 4096 144 -> 148, and (B, H, N, D) storage gains nothing.)
-//   * no multiple of 8, but no XCD with more than kWholeHeadParts parts: whole heads all the same.  A part reads the totals that its
-//     head's other parts wrote, from that XCD's own L2, and half of an XCD's CUs are enough for them.  Forward alone, runs of parts ->
-//     whole heads (parts of the fullest XCD): 80 columns, B H 12 N 306 (10) 12.45 -> 12.02 us; 128 columns, B H 1 N 1024 (16) 17.8 ->
-//     16.3, B H 4 N 800 (13) 16.1 -> 15.1, B H 20 N 300 (15) 12.85 -> 12.46, B H 12 N 500 (16) 14.2 -> 14.2; above the line B H 12 N 620
-//     (20) 14.9 -> 14.8, N 750 (24) 16.5 -> 16.6, B H 3 N 1200 (19) 20.6 -> 18.5, but B H 4 and 1, N 1500 (24) 18.7 -> 22.5 and 14.3 -> 17.4.
+//   * no multiple of 8, but no XCD with more than `most` parts, kWholeHeadParts unless a caller says why: whole heads all the same.  A
+//     part reads the totals that its head's other parts wrote, from that XCD's own L2, and half of an XCD's CUs are enough for them.
+//     Forward alone, runs of parts -> whole heads (parts of the fullest XCD): 80 columns, B H 12 N 306 (10) 12.45 -> 12.02 us; 128
+//     columns, B H 1 N 1024 (16) 17.8 -> 16.3, B H 4 N 800 (13) 16.1 -> 15.1, B H 20 N 300 (15) 12.85 -> 12.46, B H 12 N 500 (16) 14.2 ->
+//     14.2; above the line B H 12 N 620 (20) 14.9 -> 14.8, N 750 (24) 16.5 -> 16.6, but B H 4 and 1, N 1500 (24) 18.7 -> 22.5 and 14.3 ->
+//     17.4.
+//   * nor where the XCDs are nearly as full anyway, all but an eighth of their places for heads, up to four each, and the fullest one holds
+//     its parts at a time (`resident`; 0: the parts add up no totals).  Device time, runs -> whole heads, forward alone (with backward):
+//     B H 7, 128 columns N 2500 25.9 -> 22.2 (59.3 -> 58.8), normalised 30.1 -> 25.5 (76.9 -> 73.7), 64 columns N 2500 10.4 -> 10.4 (25.7
+//     -> 25.1), N 4083 12.4 -> 12.4 (32.3 -> 30.8); B H 15, 128 columns N 1500 21.5 -> 20.2 (53.2 -> 52.6), 64 columns N 2500 14.1 -> 13.2
+//     (34.8 -> 33.7); B H 14 and 22 0.98 to 1.02; B H 31, 32 columns N 1500 9.0 -> 8.6 (20.4 -> 20.5).  More heads: B H 61, 64 columns, N 4083
+//     33.5 -> 34.3.  Entry states from a kernel in between: 128 columns, B H 7 N 4083 26.0 -> 26.8 (62.4 -> 64.6).
 //   * else an eighth of all parts, consecutive ones.  Whole heads per XCD left XCDs idle, and gave others two rounds: forward +
 //     backward, D = 128: B H 1 N 16384 241 -> 86 us, B H 4 153 -> 95, B H 12 278 -> 179, B H 20 N 8192 232 -> 152; D = 64: B H 12
 //     N 32768 218 -> 165, B H 20 N 16384 161 -> 138.
@@ -87,9 +94,11 @@ struct XcdItem {
 };
 // The map as one number, by the launcher (the kernels' `place`): 0 whole heads, every eighth; -1 whole heads, pairs of neighbours; else
 // runs, so many parts per XCD.
-inline int32_t xcd_place(int64_t BH, int64_t parts, int64_t stride_h) {
+inline int32_t xcd_place(int64_t BH, int64_t parts, int64_t stride_h, int most = kWholeHeadParts, int resident = 0) {
     if (BH % 8 == 0) return BH % 16 == 0 && stride_h % 64 != 0 ? -1 : 0;
-    return (BH + 7) / 8 * parts <= kWholeHeadParts ? 0 : (int32_t)((BH * parts + 7) / 8);
+    const int64_t heads = (BH + 7) / 8;  // (of the fullest XCD)
+    if (heads * parts <= most || (heads <= 4 && 8 * heads - BH <= heads && heads * parts <= resident)) return 0;
+    return (int32_t)((BH * parts + 7) / 8);
 }
 // 2^32 / parts, rounded up: with it floor(item / parts) is the upper half of a product, exact while item parts < 2^32 (walks: 512
 // workgroups at a time or one part per head).  0: of one part.

@@ -50,7 +50,7 @@ def trace_lib(rebuild: bool = False) -> ctypes.CDLL:
             fn.restype = restype
         lib.fla_trace_take.argtypes = [ctypes.c_char_p, ctypes.c_int64]
         lib.fla_trace_take.restype = ctypes.c_int64
-        lib.fla_trace_xcd_place.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64]
+        lib.fla_trace_xcd_place.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int64, ctypes.c_int, ctypes.c_int]
         lib.fla_trace_xcd_items.argtypes = [ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_int, ctypes.c_uint32, ctypes.c_void_p]
         lib.fla_trace_xcd_inverse.restype = ctypes.c_uint32
         lib.fla_trace_xcd_items.restype = None
@@ -267,11 +267,19 @@ def xcd_items(grid: int, BH: int, parts: int, place: int, inverse: Optional[int]
     return items
 
 
-def check_place(l: "Launch", p: Dict, parts: int, stride_h: int) -> None:
-    """The launch's map is the one that its heads and parts ask for."""
-    want = trace_lib().fla_trace_xcd_place(p["BH"], parts, stride_h)
+def check_place(l: "Launch", p: Dict, parts: int, stride_h: int, whole: int = 16, resident: int = 0) -> None:
+    """The launch's map: heads stay whole up to `whole` parts on an XCD, and up to `resident` of them if nearly every XCD has as many."""
+    want = trace_lib().fla_trace_xcd_place(p["BH"], parts, stride_h, whole, resident)
     assert p["place"] == want, f"{l.kernel}: place {p['place']}, not {want}"
     xcd_items(l.grid[0], p["BH"], parts, p["place"], p.get("n_seg_inv"))
+
+
+def check_walk_place(l: "Launch", p: Dict, D: int, stride_h: int, norm, alone) -> None:
+    """Up to 64 columns whole heads up to 32 parts in the normalised operator and where a plain forward adds up its head's totals as
+    it starts (or has two segments); nearly full XCDs count where totals are added up so."""
+    sums = p["n_seg"] <= {32: 16, 64: 32, 128: 20}[D]
+    check_place(l, p, p["n_seg"], stride_h, 32 if D <= 64 and (norm or (sums and (alone or D == 32))) else 16,
+                (64 if D <= 64 else 32) if sums else 0)
 
 
 # ---------------------------------------------------------------------------------------------
@@ -790,7 +798,7 @@ def model_walk(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats) -> None:
     assert seg_chunks >= 1 and n_seg >= 1 and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks, \
         f"{l.kernel}: {n_seg} segments of {seg_chunks} chunks do not tile {n_chunks} chunks"
     assert l.grid[0] == 8 * ((BH + 7) // 8) * n_seg
-    check_place(l, p, n_seg, p["ks_h"])
+    check_walk_place(l, p, D, p["ks_h"], p["denom"] or p["dn"], not p["saved"])
     resident = 256 if D > 64 else 512
     assert BH * n_seg <= max(resident, BH), f"{l.kernel}: {BH * n_seg} workgroups for {resident} resident"
     # (pairs of column halves, grid y: a q / k of 128 + wqk2 columns, a v of 128 + wv2)
@@ -921,7 +929,7 @@ def model_walk_totals(arena: Arena, l: Launch, p: Dict, D: int, stats: Stats, bo
     assert n_chunks == -(-N // rows) and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks
     assert 0 <= p["seg_lo"] <= p["seg_hi"] <= n_seg
     assert l.grid[0] == 8 * ((BH + 7) // 8) * n_seg
-    check_place(l, p, n_seg, p["ys_h"])
+    check_walk_place(l, p, D, p["ys_h"], p["vsum"], p["alone"])
     operands = [("y", "y", "ys_b", "ys_h", "ys_n", p["dy"]), ("z", "z", "zs_b", "zs_h", "zs_n", p["dz"])]
     if p["y2"]:  # a second Y operand (the other half of a wide q / k) in the same launch
         # (grid y picks the operand, or -- the kernel built for it -- every workgroup takes both: three sets of three tiles)
@@ -946,7 +954,7 @@ def model_walk_grad_totals(arena: Arena, l: Launch, p: Dict, D: int, vec: bool, 
     n_chunks, seg_chunks, n_seg = p["n_chunks"], p["seg_chunks"], p["n_seg"]
     assert n_chunks == -(-N // rows) and (n_seg - 1) * seg_chunks < n_chunks <= n_seg * seg_chunks
     assert l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
-    check_place(l, p, n_seg, p["qs_h"])
+    check_walk_place(l, p, D, p["qs_h"], True, False)
     assert l.lds == ((2 if D == 128 else 1) + 3) * rows * 2 * D + 2 * rows * 4, f"{l.kernel}: {l.lds} bytes of LDS"
     assert 1 <= wqk <= D and 1 <= wv <= D and wqk % 8 == 0 and wv % 8 == 0
     assert p["q"] % 16 == 0 and p["qs_n"] % 8 == 0 and p["dout"] % 16 == 0 and N * p["qs_n"] * 2 <= 0x3fffffff
@@ -978,7 +986,7 @@ def model_poly(arena: Arena, l: Launch, p: Dict, backward: bool, stats: Stats) -
     """The polynomial map's kernels: every operand, result and state that the kernel touches."""
     H, BH, N, n_seg = p["H"], p["BH"], p["N"], p["n_seg"]
     assert p["n_chunks"] == -(-N // 128) and l.grid == (8 * ((BH + 7) // 8) * n_seg, 1, 1)
-    check_place(l, p, n_seg, p["ks_h"])
+    check_place(l, p, n_seg, p["ks_h"], 16, 32 if n_seg <= 20 else 0)
     assert (n_seg - 1) * p["seg_chunks"] < p["n_chunks"] <= n_seg * p["seg_chunks"]
     widths = {"q": p["r"], "k": p["r"], "v": p["wv"], "go": p["wv"], "o": p["wv"], "out": p["wv"], "dq": p["r"], "dk": p["r"],
               "dv": p["wv"]}

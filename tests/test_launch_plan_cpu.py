@@ -294,16 +294,18 @@ def test_forward_by_columns(lib, bh, n, d, dtype, columns):
 
 
 @pytest.mark.parametrize("stride_h", [64, 40], ids=["whole lines", "part of a line"])
-def test_every_part_of_every_head_is_one_workgroups(lib, stride_h):
+@pytest.mark.parametrize("whole,resident", [(16, 0), (16, 32), (32, 64)])
+def test_every_part_of_every_head_is_one_workgroups(lib, whole, resident, stride_h):
     """The walks' map over the grid that their launchers take: the last number of parts that keeps heads whole, the next, and counts
     off every line."""
     for bh in [*range(1, 70), 72, 80, 96, 100, 112, 127, 128, 129, 191, 192, 255, 256, 257, 300]:
         for parts in [*range(1, 21), 31, 32, 33, 63, 64]:
-            place = lib.fla_trace_xcd_place(bh, parts, stride_h)
+            place = lib.fla_trace_xcd_place(bh, parts, stride_h, whole, resident)
             items = lp.xcd_items(8 * ((bh + 7) // 8) * parts, bh, parts, place, lib.fla_trace_xcd_inverse(parts))
             if parts in (1, 7, 64):
                 assert (items == lp.xcd_items(8 * ((bh + 7) // 8) * parts, bh, parts, place)).all()
-            if bh % 8 == 0 or (bh + 7) // 8 * parts <= 16:  # whole heads
+            fullest = (bh + 7) // 8 * parts
+            if bh % 8 == 0 or fullest <= whole or (bh in (7, 14, 15, 21, 22, 23, 28, 29, 30, 31) and fullest <= resident):  # whole heads
                 assert place == (-1 if bh % 16 == 0 and stride_h == 40 else 0)
                 assert all(len(set(np.flatnonzero(items[:, 0] == head) % 8)) == 1 for head in {0, bh // 2, bh - 1})
             else:  # an eighth of the parts each
