@@ -1348,8 +1348,10 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         fla::WalkParams w{};
         if (nx) {
             float *const rcv = reinterpret_cast<float *>(static_cast<char *>(nx->vec) + walk_vec_bytes(B, H, N, dqk, dv));
-            // (g as aligned rows, as the walk's tile loads ask for: dO is formed where it is used)
-            const bool keep_g = nx->vec16 && fla::fast_path_ok(make_params(q, k, *nx->go, dvv, B, H, N, dqk, dv, 0));
+            // (g as aligned rows, as the walk's tile loads ask for, and not from the caches at a few heads: dO is formed where it is
+            // used.  A dO written and read -> this, forward + backward, MB of dO, D = 64: 0.13 to 2.1 25.2 -> 25.8 us, 32.2 -> 32.6; 8.4
+            // 45.8 -> 46.1, 50.5 -> 50.1, 64.0 -> 63.6; 12.6 57.6 -> 57.2; 16.8 71.8 -> 70.3; 33.6 130 -> 127)
+            const bool keep_g = nx->vec16 && B * H * N * dv * 2 > (10 << 20) && fla::fast_path_ok(make_params(q, k, *nx->go, dvv, B, H, N, dqk, dv, 0));
             if (int rc = walk_grad_entry_states(wp, q, go, *nx, B, H, N, dqk, dv, dtype, workspace, rcv, &entry, false, s, keep_g)) return rc;
             gv = keep_g ? nx->go : &go, w.gn = keep_g ? nx->n : nullptr;
             w.dn = nx->dn, w.zc = zc_saved, w.rc = wp.n_seg > 1 ? rcv : nullptr;

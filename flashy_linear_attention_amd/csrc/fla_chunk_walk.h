@@ -1640,7 +1640,7 @@ __global__ __launch_bounds__(256, 1) void walk_fwd_wide_kernel(const WalkParams 
 // (Obtained backwards instead -- from the state at the segment's end, subtracting every chunk's K^T V when the walk reaches
 // it -- one late row that is infinite, NaN or merely huge spoiled the dQ of every chunk before it.  Forward + backward
 // at B H 16, N 32768, D 64 that way 222 us, this way 234 at the time, 222 with totals added up by fragments.)
-template <typename T, int D, bool NORM, bool WIDE = false>
+template <typename T, int D, bool NORM, bool WIDE = false, bool GN = false>
 __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
     using W = WalkCfg<D>;
@@ -1711,7 +1711,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
         if constexpr (NORM) {  // the normaliser's terms: zc of this chunk and its rows of dn
             walk_load_vec<D>(p.zc + ((int64_t)sl.bh * p.n_chunks + c) * D, xbase, lane);
             walk_load_rows<D>(p.dn + (int64_t)sl.bh * N, row0, N, xbase + 2048, lane);
-            if (p.gn) walk_load_rows<D>(p.gn + (int64_t)sl.bh * N, row0, N, xbase + 2560, lane);
+            if constexpr (GN) walk_load_rows<D>(p.gn + (int64_t)sl.bh * N, row0, N, xbase + 2560, lane);
         }
         if (c > 0)
             walk_load_state_copy<D>(static_cast<const unsigned char *>(p.saved) + at * W::STATE, NORM ? lds0 + 4 * W::TILE : xbase, wave,
@@ -1719,7 +1719,7 @@ __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
         wait_vm<0>();
         __syncthreads();
         if constexpr (NORM) {
-            if (p.gn) {  // dO = g / n, as walk_grad_totals_kernel rounds it
+            if constexpr (GN) {  // dO = g / n, as walk_grad_totals_kernel rounds it
                 const float *vn = vd + 128;
 #pragma unroll
                 for (int v = 0; v < W::C * W::CR / 256; ++v) {
@@ -2964,12 +2964,12 @@ hipError_t launch_walk_bwd(const WalkParams &p, hipStream_t stream) {
     const int64_t grid = (int64_t)8 * ((p.BH + 7) / 8) * p.n_seg;
     if (grid > 0x7fffffffLL) return hipErrorInvalidConfiguration;
     constexpr int smem = 4 * WalkCfg<D>::TILE + WalkCfg<D>::STATE;
+    if (p.gn && !p.dn) return hipErrorInvalidValue;
     if (p.dn) {
         if (!p.zc || !p.saved || (p.n_seg > 1 && !p.rc)) return hipErrorInvalidValue;
-        constexpr auto kern = walk_bwd_kernel<T, D, true, WIDE>;
         constexpr int smem_n = smem + WalkCfg<D>::VEC + 1024;
-        if (hipError_t e = ensure_dynamic_lds<kern>(smem_n)) return e;
-        return launch_kernel<kern>(dim3((unsigned)grid), dim3(256), smem_n, stream, p);
+        return p.gn ? launch_walk_kernel<walk_bwd_kernel<T, D, true, WIDE, true>>(grid, smem_n, p, stream)
+                    : launch_walk_kernel<walk_bwd_kernel<T, D, true, WIDE>>(grid, smem_n, p, stream);
     }
     if (!p.saved) return hipErrorInvalidValue;
     constexpr auto kern = walk_bwd_kernel<T, D, false, WIDE>;

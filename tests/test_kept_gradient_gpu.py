@@ -1,5 +1,5 @@
-"""The normalised chunk-wise backward up to 64 columns forms dO = g / n where it is used when g's rows are aligned, and ahead of the
-walk when they are not (csrc/fla_chunk_walk.h, WalkParams::gn): the same bits either way (``-m gpu``)."""
+"""The normalised chunk-wise backward up to 64 columns forms dO = g / n where it is used when g's rows are aligned and dO is of more
+than 10 MiB, and ahead of the walk otherwise (csrc/fla_chunk_walk.h, WalkParams::gn): the same bits either way (``-m gpu``)."""
 
 import pytest
 import torch
@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
-@pytest.mark.parametrize("h,n,d", [(1, 257, 64), (3, 1000, 40), (24, 900, 32), (300, 384, 64), (2, 4100, 24)])
+@pytest.mark.parametrize("h,n,d", [(1, 257, 64), (3, 1000, 40), (24, 900, 32), (300, 384, 64), (2, 4100, 24), (170, 1000, 40), (700, 384, 32), (500, 520, 24)])
 @pytest.mark.parametrize("mapped", [False, True], ids=["plain", "elu1"])
 def test_aligned_and_unaligned_rows_of_g(mapped, h, n, d, dtype, gpu_device):
     gen = torch.Generator().manual_seed(n + d)

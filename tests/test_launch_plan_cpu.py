@@ -196,10 +196,11 @@ def test_normalised_operator_over_the_sweep_space(lib, dims):
     assert cases > 25 and stats.launches > cases * 4
 
 
-@pytest.mark.parametrize("g_layout,kept", [("contiguous", True), ("odd", False)])
-def test_where_the_normalised_walk_takes_dO_from(lib, g_layout, kept):
-    """From g and n where g's rows are aligned, else from what the pass ahead wrote; another place is noticed."""
-    arena, launches = trace_normalised(lib, 1, 3, 1000, 64, 64, True, g_layout=g_layout)
+@pytest.mark.parametrize("h,g_layout,kept", [(100, "contiguous", True), (100, "odd", False), (3, "contiguous", False)])
+def test_where_the_normalised_walk_takes_dO_from(lib, h, g_layout, kept):
+    """From g and n where g's rows are aligned and dO is of more than 10 MiB, else from what the pass ahead wrote; another place is
+    noticed."""
+    arena, launches = trace_normalised(lib, 1, h, 1000, 64, 64, True, g_layout=g_layout)
     ahead = next(l for l in launches if l.kernel == "walk_grad_totals_kernel")
     walk = next(l for l in launches if l.kernel == "walk_bwd_kernel")
     assert bool(ahead.args["a0.keep_g"]) == kept == bool(walk.args["a0.gn"])
