@@ -2101,8 +2101,8 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
 // 192, N 256 ... 8192.  Forward + backward (dQ by its own walk, see chunked_backward), equal widths: from W = B H N^2 D = 4e9
 // (8e9 at 128) 1.17 to 4.8 with few heads or many (0.90 at 32 columns, B H 16, N 3072); few heads and long: N = 4096 1.5 to
 // 3.1, N = 2048 1.42 to 2.0 at 64 and 128 columns, 0.88 to 1.19 at 32; N = 1024 0.67 to 1.2.  Widths that differ (small-V
-// operator): N = 1024 1.38 to 2.1, from W = 5e8 (1e9 below 128) 1.08 to 1.6.  Forward alone: N = 2048 1.17 to 1.9 (0.92 to
-// 0.99 at 32 columns), W from 1.2e10 1.1 to 2; N = 512 and 1024 below that 0.65 to 1.15.
+// operator): N = 1024 1.38 to 2.1, from W = 5e8 (1e9 below 128) 1.08 to 1.6.  Forward alone, at its line below: W from 1.2e10
+// (5e9 at 32 columns) 1.1 to 2, N = 2048 1.17 to 1.9, and earlier by width.
 int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, bool backward) {
     if (B < 1 || H < 1 || N < 1 || D_qk < 1 || D_qk > 256 || D_v < 1 || D_v > 256) return 0;
     const double w = (double)B * (double)H * (double)N * (double)N * (double)padded(D_qk > D_v ? D_qk : D_v);

@@ -3,7 +3,7 @@
 //     kernel=<function with template arguments>;grid=x,y,z;block=n;lds=bytes;a0=...;a1.field=...
 // Scalars and pointers are written as they are; parameter structs field by field (the overloads
 // of trace_describe in fla_trace_structs.h).  The records of a thread are kept until taken with
-// fla_trace_take (declared at the bottom; defined in fla_capi.hip).
+// fla_trace_take (fla_trace.cc).
 #pragma once
 
 #include <stdint.h>
