@@ -90,8 +90,6 @@ struct WalkParams {
     int32_t H, N, BH, wqk, wv;   // true widths of q/k and of v (<= D)
     int32_t n_chunks;            // ceil(N / rows per chunk)
     int32_t seg_chunks, n_seg;   // chunks per segment, segments per (b, h)
-    int32_t place;               // which workgroup takes which segment (walk_place) and xcd_item's factor for n_seg, both filled on the way
-    uint32_t n_seg_inv;          // to the launcher; here and below
     // entry state of every segment, fp32 [BH][n_seg][D (q/k index)][D (v index)]: sum of K^T V over
     // the segments before (forward) / of Q^T dO over the segments after (backward); null when
     // there is a single segment (entry state zero).  init_transposed: the buffer holds the
@@ -185,6 +183,8 @@ struct WalkParams {
     // (walk_dkdv_kernel, ROLES): dV is formed by grid y = 0, dK by 1, each with a copy of R; q and dO are read by both.
     int32_t cols, roles, mid_chunk;
     float *mid_out;
+    int32_t place;       // which workgroup takes which segment (walk_place) and xcd_item's factor for n_seg, both filled on the way to the
+    uint32_t n_seg_inv;  // launcher; here and below
 };
 
 template <int D>
@@ -2268,8 +2268,7 @@ struct WalkTotalsParams {
     const void *y, *z;
     int64_t ys_b, ys_h, ys_n, zs_b, zs_h, zs_n;
     int32_t H, N, BH, dy, dz;
-    int32_t n_chunks, seg_chunks, n_seg, place;
-    uint32_t n_seg_inv;
+    int32_t n_chunks, seg_chunks, n_seg;
     int32_t seg_lo, seg_hi;  // only segments seg_lo .. seg_hi - 1 are needed (the others' totals stay unwritten)
     float *totals;
     // two segments: only the total of segment seg_lo is needed, as the other segment's entry state.
@@ -2298,6 +2297,8 @@ struct WalkTotalsParams {
     // nobody reads the totals' columns 64 .. (every walk behind them leaves a narrow z's padding out): they may stay
     // unwritten for a narrow y as well
     int32_t z_narrow;
+    int32_t place;  // (as in WalkParams; at the far end, where they bring in the rest of the parameters' lines together with n_seg)
+    uint32_t n_seg_inv;
 };
 
 constexpr int walk_totals_sets(int D) { return D == 128 ? 4 : 2; }  // sets of (Y, Z) tiles in LDS
@@ -2634,12 +2635,13 @@ struct WalkGradParams {
     float *dn;                 // fp32 [BH][N]
     int32_t H, N, BH, wqk, wv;
     int32_t vec;               // g and out allow 16-byte loads
-    int32_t n_chunks, seg_chunks, n_seg, place;
-    uint32_t n_seg_inv;
+    int32_t n_chunks, seg_chunks, n_seg;
     float *totals, *rsum;      // [BH][n_seg] states and vectors in the slots the walks read (two segments: partial sums of the
                                // second one's in both; the first one's stay unwritten otherwise); null with a single segment
     int32_t frags;             // WalkTotalsParams::frags
     int32_t keep_g;            // dO is formed again by the walk behind (WalkParams::gn) and not written
+    int32_t place;             // (as in WalkTotalsParams)
+    uint32_t n_seg_inv;
 };
 
 // Steps on their way: what a step needs is requested DEPTH steps ahead -- one where two workgroups share a CU, two at D = 128,

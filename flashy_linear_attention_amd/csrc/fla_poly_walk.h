@@ -50,8 +50,6 @@ struct PolyWalkParams {
     int64_t us_b, us_h, us_n;  // out
     int64_t dqs_b, dqs_h, dqs_n, dks_b, dks_h, dks_n, dvs_b, dvs_h, dvs_n;
     int32_t H, N, BH, r, wv, n_chunks, seg_chunks, n_seg;
-    int32_t place;  // which workgroup takes which segment (xcd_place) and xcd_item's factor for n_seg, filled by the launcher
-    uint32_t n_seg_inv;
     float c0, c1, c2, eps;
     int32_t wide_out;  // dq, dk, dv are floats (and receive the bf16-rounded values)
     float *denom;  // fp32 [BH][N], or null: not normalised.  Forward writes it, backward reads it
@@ -65,6 +63,8 @@ struct PolyWalkParams {
     // B 4 H 16 N 4096 211 -> 200 us; B H 16, N 4096 83.7 -> 77.1, N 16384 219 -> 210; B H 80, N 4096 268 -> 258; 8 over 32 columns, B H 24,
     // N 4096 112.9 -> 107.4
     int32_t u_totals;
+    int32_t place;  // which workgroup takes which segment (xcd_place) and xcd_item's factor for n_seg, filled by the launcher
+    uint32_t n_seg_inv;
 };
 
 // Feature order: groups of eight.  Groups 0 .. 15: x_a x_b with a = 8h + j and b = (a + d) % 16 for d = 0 .. 7, h = 0, 1 (group

@@ -48,7 +48,6 @@ struct TriParams {
     int32_t dc, dout;  // actual widths (<= DC, DO of the instantiation)
     int32_t upper;     // 0: keep row >= col, 1: keep row <= col
     int32_t n_tiles;   // ceil(N / BM), filled by the launcher
-    int32_t place;     // chunk-wise: which workgroup takes which tile (xcd_place), filled by the launcher
     int32_t single;    // fast path: one row tile per workgroup instead of a balanced pair (launcher's choice)
     int32_t vec_x, vec_y, vec_z;  // 1: rows are 16-byte aligned and width % 8 == 0
     int32_t vec_out;              // same for the output
@@ -82,6 +81,7 @@ struct TriParams {
     // multiplied by phi'(x) computed from y, map_out naming phi -- the chain rule of a gradient with
     // respect to the argument of phi.
     int32_t map_x, map_out;
+    int32_t place;  // (chunk-wise) which workgroup takes which tile (xcd_place), filled by the launcher
     void *xmap_out;
     int64_t xo_b, xo_h, xo_n;
     const void *omap;

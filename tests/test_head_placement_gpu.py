@@ -47,6 +47,20 @@ def test_either_side_of_whole_heads(n, gpu_device):
         assert_close(name, got, want)
 
 
+# (7 heads, nearly one per XCD: up to 20 parts of 128 columns whole, whose totals the walks add up, and 21 in runs; 9 heads over 64
+# columns: a forward alone whole up to 2 x 16 parts on an XCD, and 2 x 17; 15 heads, nearly two per XCD)
+@pytest.mark.parametrize("heads,n,width", [(7, 1280, 128), (7, 1281, 128), (9, 2048, 64), (9, 2049, 64), (15, 2500, 64)])
+def test_either_side_of_more_parts(heads, n, width, gpu_device):
+    q, k, v, dy = (_bnhd(t.to(gpu_device)) for t in reference_style_inputs(1, heads, n, width, width, torch.bfloat16, seed=n))
+    want_o, want_g = gpu_fp32_reference(q, k, v, dy, True)
+    assert_close("O alone", LinearAttentionChunked.apply(q, k, v), want_o)
+    leaves = [t.detach().requires_grad_(True) for t in (q, k, v)]
+    out = LinearAttentionChunked.apply(*leaves)
+    assert_close("O", out, want_o)
+    for name, got, want in zip(("dQ", "dK", "dV"), torch.autograd.grad(out, leaves, dy), want_g):
+        assert_close(name, got, want)
+
+
 @pytest.mark.parametrize("heads", [3, 16, 20])
 def test_the_normalised_backward_and_the_polynomial_map(heads, gpu_device):
     q, k, v, dy = (_bnhd(t.to(gpu_device)) for t in reference_style_inputs(1, heads, 900, 32, 32, torch.bfloat16, seed=7))
