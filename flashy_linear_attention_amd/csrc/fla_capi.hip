@@ -710,8 +710,9 @@ int64_t shared_state_bytes(int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t
     return core ? core + walk_vec_bytes(B, H, N, dqk, dv) : 0;
 }
 
-// fp16, plain, up to 64 columns: the saved copies' scales, a float per chunk, lie in that room (null where there is none: widths whose
-// paddings differ)
+// fp16 without the normaliser, up to 64 columns: the saved copies' scales, a float per chunk, lie in that room (null where there is none:
+// widths whose paddings differ).  Every such forward leaves them and every such backward reads them, whatever evaluated either: a feature
+// map's forward runs the plain walk where the operands' rows keep the map out of it, and its backward maps all the same.
 float *saved_scales(const void *state, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv) {
     if (!walk_vec_bytes(B, H, N, dqk, dv)) return nullptr;
     return reinterpret_cast<float *>(static_cast<char *>(const_cast<void *>(state)) + state_core_bytes(B, H, N, dqk, dv));
@@ -996,7 +997,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
 int chunked_backward(const View &go, const View &q, const View &k, const View &v, const View &dq, const View &dk,
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                      const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap, WalkNorm *nx,
-                     bool causal, bool wide_out, AnyRows *any, bool plain_state);
+                     bool causal, bool wide_out, AnyRows *any, bool scaled_state);
 
 // fmap != 0 (feature_forward below): q and k hold the arguments xq, xk of the feature map phi, and
 // `mapped` = {phi(xq), phi(xk)} are outputs: the state kernel maps xk as it loads it and writes
@@ -1092,7 +1093,7 @@ int chunked_forward(const View &q, const View &k, const View &v, const View &o, 
         w.H = (int32_t)H, w.N = (int32_t)N, w.BH = (int32_t)(B * H), w.wqk = (int32_t)dqk, w.wv = (int32_t)dv;
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = wp.n_seg > 1 ? entry : nullptr, w.saved = in_state ? nullptr : state_out;
-        if (w.saved && dtype == FLA_DTYPE_F16 && !fmap && !nx) w.saved_scale = saved_scales(state_out, B, H, N, dqk, dv);
+        if (w.saved && dtype == FLA_DTYPE_F16 && !nx) w.saved_scale = saved_scales(state_out, B, H, N, dqk, dv);
         if (sum_on_load) w.init_is_totals = 1, w.entry_out = in_state ? static_cast<float *>(state_out) : nullptr;
         if (by_columns) {  // (the state buffer is that of two segments all the same)
             w.cols = 1, w.n_seg = 1, w.seg_chunks = w.n_chunks, w.init = nullptr;
@@ -1180,7 +1181,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
                      const View &dvv, int64_t B, int64_t H, int64_t N, int64_t dqk, int64_t dv, int dtype,
                      const void *state_in, void *workspace, int64_t workspace_bytes, void *stream, int fmap = 0,
                      WalkNorm *nx = nullptr, bool causal = false, bool wide_out = false, AnyRows *any = nullptr,
-                     bool plain_state = true) {  // (the state is from a plain forward: saved_scales)
+                     bool scaled_state = true) {  // (the state is not a normalised forward's: saved_scales)
     if (nx) nx->fused = nx->dk_pending = false;
     const View all[] = {go, q, k, v, dq, dk, dvv};
     for (const View &t : all)
@@ -1385,7 +1386,7 @@ int chunked_backward(const View &go, const View &q, const View &k, const View &v
         w.n_chunks = (int32_t)wp.n_chunks, w.seg_chunks = (int32_t)wp.seg_chunks, w.n_seg = (int32_t)wp.n_seg;
         w.init = entry;
         w.saved = const_cast<void *>(state_in);
-        if (dtype == FLA_DTYPE_F16 && !fmap && !nx && plain_state) w.saved_scale = saved_scales(state_in, B, H, N, dqk, dv);
+        if (dtype == FLA_DTYPE_F16 && !nx && scaled_state) w.saved_scale = saved_scales(state_in, B, H, N, dqk, dv);
         w.wide_out = wide_out;
         return fla::walk_bwd(dtype, wp.D, w, s) == hipSuccess ? FLA_OK : FLA_ERR_LAUNCH;
     }

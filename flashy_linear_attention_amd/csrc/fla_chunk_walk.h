@@ -124,7 +124,8 @@ struct WalkParams {
     float *zc_out;      // as zc
     const float *dn;  // fp32 [BH][N]
     const float *rc;  // fp32 [BH][n_seg][D], slots as those of `init`
-    // fp16, plain, up to 64 columns: what each of the saved copies is to be multiplied by, [BH][n_chunks] (walk_state_scale; null: they were multiplied by it)
+    // fp16 without the normaliser, up to 64 columns: what each of the saved copies is to be multiplied by, [BH][n_chunks] (walk_state_scale, 1
+    // with a feature map on load; null: they were multiplied by it)
     float *saved_scale;
     // walk_bwd_kernel: go holds g, and dO = g / n is formed in its tile as it lands (null: go holds dO).  An operand less for
     // walk_grad_totals_kernel to write: B H 64, N 4096, D 64 that kernel 24.8 -> 19.4 us, the walk 57.3 to 59.9 (55.2 from 54.4 without a
@@ -1401,7 +1402,8 @@ __global__ __launch_bounds__(256, DOUBLE ? 1 : 2) void walk_fwd_kernel(const Wal
                     }
                     *reinterpret_cast<u32x4 *>(sv + i) = __builtin_bit_cast(u32x4, copy);
                 }
-                if (SCALED && p.saved_scale && tid == 0) p.saved_scale[(int64_t)sl.bh * p.n_chunks + c] = sback;
+                if constexpr (std::is_same<T, _Float16>::value && NORM == 0)  // (1 where the copy is not scaled)
+                    if (p.saved_scale && tid == 0) p.saved_scale[(int64_t)sl.bh * p.n_chunks + c] = sback;
             }
         }
         f32x16 acc[W::DBW];
