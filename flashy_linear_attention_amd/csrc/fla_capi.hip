@@ -2250,16 +2250,23 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
     // (0.94 to 1.2 at 768), 64 / 32, 128 / 64 and 128 / 32 1.06 to 1.5 at 1024; a single segment per head, which has no totals to
     // wait for, 1.12 to 2.3 from N = 320 on.
     const bool equal = pad_index(D_qk) == pad_index(D_v), one = wp.n_seg == 1 && N > 256;
+    // Up to 256 rows above 64 columns (widths that differ: one segment of two to four chunks).  Pairs, 128 / 64 and 128 / 32: B H 300 ... 1024
+    // 1.22 to 1.42 from N = 128 on (the quadratic products' second round of workgroups); up to 256 heads 1.04 to 1.30 from W = 1.7e9 on, 0.93 to
+    // 1.09 below it, where two launches wait for the host for 36 us and three for 38.  Forward alone, B H 2000, N 256 1.21 and 1.27.
+    if (wp.ok && N < 128 && wp.split) return 0;
     if (wp.ok && !backward) return one || N >= (wp.D == 64 && equal ? 768 : 1024) || w >= (wp.D <= 32 ? 5e9 : 1.2e10);
+    if (wp.ok && !equal && wp.split && N <= 256) return B * H > 256 || w >= 1.7e9;
     if (wp.ok && !equal) return N >= 1024 || w >= (wp.D <= 64 ? 1e9 : 5e8);
     // Equal padded head dims up to 128.  (Pairs gain earlier on the GPU -- 64 columns 1.2 to 1.5 from N = 768 on --, but there the
     // host, 58 us for the quadratic pair's two launches and 72 for the chunk-wise one's four, takes longer than either.  Single
     // segments of 128 columns: B H 130 N 448 74 / 64 us, B H 256 N 320 92 / 61.)
     if (wp.ok) return N >= (wp.D <= 32 ? 4096 : 2048) || w >= (wp.D <= 64 ? 4e9 : one ? 3.2e9 : 8e9);
-    // D_qk in (128, 256].  D_v <= 64: pairs 1.13 to 5 from N = 1024 or W = 1e9 on, forward alone 1.13 to 2.9 from N = 1024 (N = 512
-    // 0.82 to 1.1).  D_v in (64, 128]: pairs 1.35 to 3.1 from N = 2048, 1.3 from W = 2.5e10 (1.0 at 1.7e10, N = 1024); forward
-    // alone 1.14 to 1.55 from N = 4096, at N = 2048 1.1 to 1.4 with B H <= 4 and 0.93 with 16.
+    // D_qk in (128, 256].  D_v <= 64: pairs 1.13 to 5 from N = 1024 or W = 1e9 on (192 / 64 and 256 / 64, N 128 ... 256, B H 60 ... 1024 1.15 to
+    // 1.51), forward alone 1.13 to 2.9 from N = 1024 (N = 512 0.82 to 1.1).  D_v in (64, 128]: pairs 1.35 to 3.1 from N = 2048, 1.3 from
+    // W = 2.5e10 (1.0 at 1.7e10, N = 1024; at N = 256 0.99 to 1.07); forward alone 1.14 to 1.55 from N = 4096, at N = 2048 1.1 to 1.4 with
+    // B H <= 4 and 0.93 with 16.
     if (wide_plan(B, H, N, D_qk, D_v).ok) {
+        if (N < 128 || (D_v > 64 && N <= 256)) return 0;
         if (D_v <= 64) return N >= 1024 || (backward && w >= 1e9);
         return backward ? N >= 2048 || w >= 2.5e10 : N >= 4096 || (N >= 2048 && B * H <= 4) || w >= 5e10;
     }
@@ -2268,9 +2275,10 @@ int prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, 
 }
 
 // The operators' choice: the table above, whose answers callers of the C ABI go by, and earlier with both widths in (128, 256], where the
-// gradients are summed in fp32 over both halves and rounded once.  Those from N = 320 on, B H 1 ... 400, widths 160, 192 and 256: pairs 1.13 to 2.1 up
-// to N = 700, 1.5 to 2.4 at N = 1024, 2.2 to 4 at 2048, 4.2 to 25 beyond; forward alone 1.0 to 4.7, but 0.81 to 0.96 below N = 640 with two
-// segments per head (33 to 64 heads).
+// gradients are summed in fp32 over both halves and rounded once.  Those, widths 160, 192 and 256, B H 1 ... 300 (400 from N = 320 on): at N 128, 192 and
+// 256 (one segment per head) pairs 1.04 to 1.84, forward alone 1.13 to 1.8; from N = 320 on pairs 1.13 to 2.1 up to N = 700, 1.5 to 2.4 at N = 1024,
+// 2.2 to 4 at 2048, 4.2 to 25 beyond; forward alone 0.97 to 4.7, but 0.81 to 0.96 below N = 640 with two segments per head (33 to 64 heads).
+// Errors over the quadratic kernels', N 128 ... 1024, 192 heads each: dQ and dK 0.997 to 1.004, O and dV 0.69 to 1.002.
 int operators_prefer_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, bool backward) {
     if (const WalkPlan quad = quad_plan(B, H, N, D_qk, D_v); quad.ok && D_qk % 8 == 0 && D_v % 8 == 0)
         return N >= 128 && (backward || quad.n_seg != 2 || N >= 640);

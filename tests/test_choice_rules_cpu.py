@@ -89,3 +89,16 @@ def test_half_precision_pairs(bh, dqk, dv, first):
         assert _lib.query(name, 1, bh, n, dqk, dv) == want
     for widths in ((64, 32), (136, 128), (100, 100), (256, 64)):
         assert _lib.query(name, 1, bh, 16384, *widths) == 0
+
+
+# (what takes 128 to 256 rows in one segment: padded widths that differ, q and k above 128 columns)
+@pytest.mark.parametrize("dqk,dv,bh,n,pair,forward", [
+    (128, 64, 256, 128, 0, 0), (128, 64, 257, 128, 1, 0), (128, 32, 5000, 127, 0, 0), (64, 128, 202, 256, 0, 0), (72, 40, 203, 256, 1, 0),
+    (128, 32, 1430, 256, 1, 0), (128, 32, 1431, 256, 1, 1), (256, 64, 256, 127, 0, 0), (256, 64, 239, 128, 1, 0), (192, 40, 238, 128, 0, 0),
+    (192, 64, 60, 256, 1, 0), (160, 128, 5000, 256, 0, 0), (256, 72, 1600, 257, 1, 0),
+])
+def test_up_to_256_rows(dqk, dv, bh, n, pair, forward):
+    for name, want in (("fla_linear_attn_prefers_chunked", pair), ("fla_linear_attn_forward_prefers_chunked", forward)):
+        assert _lib.query(name, 1, bh, n, dqk, dv) == want
+    for backward, want in ((1, pair), (0, forward)):
+        assert _lib.query("fla_linear_attn_operator_prefers_chunked", 1, bh, n, dqk, dv, backward) == want
