@@ -98,6 +98,8 @@ def _copies_bwd(grad_output: torch.Tensor, q: torch.Tensor, k: torch.Tensor, v: 
 def evaluate_fwd(ctx: Any, q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, chunked: bool, equal: bool) -> torch.Tensor:
     """Forward of an autograd Function by the evaluation `chunked` names; keeps what :func:`evaluate_bwd` needs."""
     ctx.chunked, ctx.equal = chunked, equal
+    # (an fp16 pair that is chunk-wise because the walks keep the range)
+    ctx.walks = chunked and q.dtype == torch.float16 and any(ctx.needs_input_grad[:3]) and chunked_keeps_range(q, k, v, True)
     state = None
     if chunked:
         if any(ctx.needs_input_grad[:3]):
@@ -119,7 +121,7 @@ def evaluate_bwd(ctx: Any, grad_output: torch.Tensor) -> Tuple[torch.Tensor, tor
     else:
         (q, k, v), state = ctx.saved_tensors, None
     if ctx.chunked:
-        if q.dtype == torch.float16:  # (the walks alone keep the quadratic evaluation's range)
+        if ctx.walks:  # (a gradient whose rows they do not take is copied)
             grad_output, q, k, v = (t if rows_for_walks(t) else t.clone(memory_format=torch.contiguous_format)
                                     for t in prepare(grad_output, q, k, v))
         # (what later rows hold must not reach dQ, as in the quadratic evaluation)

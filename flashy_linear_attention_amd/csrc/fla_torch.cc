@@ -177,8 +177,9 @@ bool wants_grad(const Tensor &q, const Tensor &k, const Tensor &v) {
 
 // ---- tril(Q K^T) V
 
-// (kChosen: chunk-wise because the shape says so, with the quadratic evaluation's causality of dQ)
-enum Evaluation { kEqual = 0, kSmallV = 1, kChunked = 2, kChosen = 3 };
+// (kChosen: chunk-wise because the shape says so, with the quadratic evaluation's causality of dQ; kWalks: and, an fp16 pair, by the walks,
+// which alone keep the quadratic evaluation's range)
+enum Evaluation { kEqual = 0, kSmallV = 1, kChunked = 2, kChosen = 3, kWalks = 4 };
 
 std::tuple<Tensor, Tensor> product_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, int ev, bool want_state) {
     at::AutoDispatchBelowADInplaceOrView below;
@@ -209,17 +210,17 @@ std::tuple<Tensor, Tensor> product_fwd(const Tensor &q_, const Tensor &k_, const
 variable_list product_bwd(const Tensor &go_, const Tensor &q_, const Tensor &k_, const Tensor &v_, const Tensor &state, int ev,
                           int64_t widened) {
     at::AutoDispatchBelowADInplaceOrView below;
-    // (fp16, chosen: the walks alone keep the quadratic evaluation's range)
+    // (kWalks: a gradient whose rows their loads do not take is copied; other calls, widths off the eights among them, go as they come)
     auto rows = [&](const Tensor &t) {
         const Tensor d = dense(t);
-        return ev != kChosen || d.scalar_type() != at::kHalf || rows_for_walks(d) ? d : d.clone(at::MemoryFormat::Contiguous);
+        return ev != kWalks || rows_for_walks(d) ? d : d.clone(at::MemoryFormat::Contiguous);
     };
     const Tensor go = rows(go_), q = rows(q_), k = rows(k_), v = rows(v_);
     const Call c(q, v);
-    if (ev == kChunked || ev == kChosen) {
+    if (ev == kChunked || ev == kChosen || ev == kWalks) {
         const Tensor work = c.bytes(fla_linear_attn_chunked_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
         return chunked_gradients(c, widened, c.grads_f32(true, state.defined()), [&](const Tensor &dq, const Tensor &dk, const Tensor &dv, int dtype) {
-            return (ev == kChosen ? fla_linear_attn_chunked_bwd_causal : fla_linear_attn_chunked_bwd)(
+            return (ev == kChunked ? fla_linear_attn_chunked_bwd : fla_linear_attn_chunked_bwd_causal)(
                 ptr(go), ptr(q), ptr(k), ptr(v), ptr(dq), ptr(dk), ptr(dv), c.b, c.h, c.n, c.dqk, c.dv, str(go), str(q), str(k),
                 str(v), str(dq), str(dk), str(dv), dtype, ptr(state), ptr(work), size_of(work), c.stream);
         });
@@ -541,15 +542,16 @@ PyObject *py_product(PyObject *, PyObject *const *args, Py_ssize_t n) {
                                             rows_for_walks(a.q) && rows_for_walks(a.k) && rows_for_walks(a.v));
     // (a v above 128 columns: chunk-wise where every sum is rounded once, beside a q / k above 128 too)
     const bool once = dv <= 128 || (dqk > 128 && dqk % 8 == 0 && dv % 8 == 0);
+    const int chosen = !bf16 && grad && range ? kWalks : kChosen;
     int ev = equal ? kEqual : kSmallV;
     if (kind == 0) {  // (the shapes its forward takes, and its choice: linear_attn.py)
         if (!equal || rows % (dqk > 128 ? 32 : 64) != 0) Py_RETURN_NONE;
-        if (range && once && prefers()) ev = kChosen;
+        if (range && once && prefers()) ev = chosen;
     } else if (kind == 1) {  // (linear_attn_smallv_hd.py)
         if (!pow2(dv) || dv > next_pow2(dqk) || rows % 64 != 0) Py_RETURN_NONE;
-        ev = range && once && prefers() ? kChosen : kSmallV;
+        ev = range && once && prefers() ? chosen : kSmallV;
     } else if (kind == 2) {  // (auto.py)
-        if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || (range && prefers())) ev = kChosen;
+        if (rows % 64 != 0 || (!equal && (dv > dqk || !pow2(dv))) || (range && prefers())) ev = chosen;
     } else {
         ev = kChunked;
     }
