@@ -76,6 +76,7 @@ SIGNATURES = {
     "fla_poly_attn_prefers_chunked": ([_i64] * 5 + [ctypes.c_int] * 2, ctypes.c_int),
     "fla_poly_attn_chunked_state_bytes": ([_i64] * 5, ctypes.c_int64),
     "fla_poly_attn_chunked_workspace_bytes": ([_i64] * 5, ctypes.c_int64),
+    "fla_poly_attn_chunked_fwd_workspace_bytes": ([_i64] * 5, ctypes.c_int64),
     "fla_poly_attn_chunked_fwd": ([_ptr] * 5 + [_i64] * 5 + [_strides] * 4
                                   + [ctypes.POINTER(ctypes.c_float), ctypes.c_float, ctypes.c_int, _ptr, _ptr, _i64, _ptr],
                                   ctypes.c_int),

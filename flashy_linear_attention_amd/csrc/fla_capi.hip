@@ -2086,7 +2086,7 @@ struct PolyPlan {
     int64_t halves, part_bytes;  // halves of v's columns, each planned as a head; room behind the totals for one of dq_part, dk_part
     // more than 16 columns of q and k: three parts with states of their own, and their sums behind the totals (PolyWalkParams::part)
     bool parts;
-    int64_t sums_bytes, total_bytes, state_at[4];
+    int64_t sums_bytes, total_bytes, fwd_bytes, state_at[4];  // (fwd_bytes: work_bytes of forward)
 };
 
 PolyPlan poly_plan(int64_t B, int64_t H, int64_t N, int64_t r, int64_t dv) {
@@ -2105,10 +2105,11 @@ PolyPlan poly_plan(int64_t B, int64_t H, int64_t N, int64_t r, int64_t dv) {
     p.parts = r > 16;
     const int64_t slots = heads * p.n_seg * 4, cross = fla::PolyFeatures::kCross * 65;
     p.part_bytes = p.halves == 2 ? heads * N * (p.parts ? 32 : 16) * 4 : 0;
-    // (O or dV, dq, dk; forward's n in the place of dq)
+    // (backward: dV, dq, dk; forward: O and n)
     p.sums_bytes = p.parts ? heads * N * (64 + 32 + 32) * 4 : 0;
     p.total_bytes = p.n_seg > 1 ? slots * (p.parts ? cross : fla::PolyFeatures::kState) : 0;
     p.work_bytes = p.total_bytes + p.sums_bytes + 2 * p.part_bytes;
+    p.fwd_bytes = p.total_bytes + (p.parts ? heads * N * (64 + 1) * 4 : 0);
     // (a single segment per (b, h) hands nothing over: a token)
     p.state_bytes = p.n_seg == 1 ? 16 : slots * (p.parts ? 2 * fla::PolyFeatures::kState + cross : fla::PolyFeatures::kStateRoom);
     p.state_at[fla::kPolySecond] = p.parts ? slots * fla::PolyFeatures::kState : 0;
@@ -2116,10 +2117,9 @@ PolyPlan poly_plan(int64_t B, int64_t H, int64_t N, int64_t r, int64_t dv) {
     return p;
 }
 
-int check_poly_chunked(const PolyPlan &pl, int dtype, int64_t workspace_bytes, const void *workspace, const void *state) {
+int check_poly_chunked(const PolyPlan &pl, int dtype, int64_t need, int64_t workspace_bytes, const void *workspace, const void *state) {
     if (!pl.ok || dtype != FLA_DTYPE_BF16) return FLA_ERR_UNSUPPORTED;
-    if (pl.work_bytes && (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < pl.work_bytes))
-        return FLA_ERR_WORKSPACE;
+    if (need && (!workspace || reinterpret_cast<uintptr_t>(workspace) % 16 != 0 || workspace_bytes < need)) return FLA_ERR_WORKSPACE;
     return reinterpret_cast<uintptr_t>(state) % 16 != 0 ? FLA_ERR_WORKSPACE : FLA_OK;
 }
 
@@ -2139,7 +2139,11 @@ int poly_run(const PolyPlan &pl, fla::PolyWalkParams &w, bool bwd, const void *s
     char *const at = static_cast<char *>(workspace) + pl.total_bytes;
     if (pl.parts) {
         w.acc = reinterpret_cast<float *>(at);
-        w.acc_q = w.acc_n = w.acc + (int64_t)w.BH * w.N * 64, w.acc_k = w.acc_q + (int64_t)w.BH * w.N * 32;
+        float *const next = w.acc + (int64_t)w.BH * w.N * 64;
+        if (bwd)
+            w.acc_q = next, w.acc_k = next + (int64_t)w.BH * w.N * 32;
+        else
+            w.acc_n = next;
     }
     for (int i = 0; i < (pl.parts ? 3 : 1); ++i) {
         w.part = pl.parts ? parts[i] : fla::kPolyWhole;
@@ -2176,7 +2180,7 @@ int poly_chunked_forward(const View &xq, const View &xk, const View &v, const Vi
     if (int rc = check_alias_fwd(xq, xk, v, o, B, H, N, r, dv)) return rc;
     if (B == 0 || H == 0 || N == 0) return FLA_OK;
     const PolyPlan pl = poly_plan(B, H, N, r, dv);
-    if (int rc = check_poly_chunked(pl, dtype, workspace_bytes, workspace, state_out)) return rc;
+    if (int rc = check_poly_chunked(pl, dtype, pl.fwd_bytes, workspace_bytes, workspace, state_out)) return rc;
     if (!vec_ok(xq, r) || !vec_ok(xk, r) || !vec_ok(v, dv) || !vec_ok(o, dv)) return FLA_ERR_UNSUPPORTED;
     fla::PolyWalkParams w{};
     poly_common(w, pl, xq, xk, v, B, H, N, r, dv, coef);
@@ -2200,7 +2204,7 @@ int poly_chunked_backward(const View &go, const View &xq, const View &xk, const 
     if (B == 0 || H == 0 || N == 0) return FLA_OK;
     if (!state_in) return FLA_ERR_NULL_POINTER;
     const PolyPlan pl = poly_plan(B, H, N, r, dv);
-    if (int rc = check_poly_chunked(pl, dtype, workspace_bytes, workspace, state_in)) return rc;
+    if (int rc = check_poly_chunked(pl, dtype, pl.work_bytes, workspace_bytes, workspace, state_in)) return rc;
     if (!vec_ok(go, dv) || !vec_ok(xq, r) || !vec_ok(xk, r) || !vec_ok(v, dv) || !vec_ok(dxq, r) || !vec_ok(dxk, r) ||
         !vec_ok(dvv, dv) || (o && !vec_ok(*o, dv)))
         return FLA_ERR_UNSUPPORTED;
@@ -2727,6 +2731,9 @@ int64_t fla_poly_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64
 
 int64_t fla_poly_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v) {
     return poly_plan(B, H, N, R, D_v).work_bytes;
+}
+int64_t fla_poly_attn_chunked_fwd_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v) {
+    return poly_plan(B, H, N, R, D_v).fwd_bytes;
 }
 
 int fla_poly_attn_chunked_fwd(const void *xq, const void *xk, const void *v, void *o, float *denom, int64_t B, int64_t H,

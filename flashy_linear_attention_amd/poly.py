@@ -111,7 +111,7 @@ def poly_attention_chunked_fwd(
     lib = _lib.load()
     with device_guard(xq.device):
         state = torch.empty(_lib.query("fla_poly_attn_chunked_state_bytes", b, h, n, r, dv), dtype=torch.uint8, device=xq.device)
-        nbytes = _lib.query("fla_poly_attn_chunked_workspace_bytes", b, h, n, r, dv)
+        nbytes = _lib.query("fla_poly_attn_chunked_fwd_workspace_bytes", b, h, n, r, dv)
         work = torch.empty(max(nbytes, 16), dtype=torch.uint8, device=xq.device)
         _lib.check(
             "fla_poly_attn_chunked_fwd",
