@@ -66,9 +66,11 @@ struct PolyWalkParams {
     int32_t u_totals;
     // 1: v of 65 to 128 columns.  BH counts halves of its columns, a (b, h)'s two next to each other, each a head of its own with states of
     // its own: O, dV and the sums are column by column, dq and dk (and dn, a sum over columns) are the halves' added up.  The halves write
-    // theirs in fp32 to dq_part / dk_part [BH][N][16] (32 over 16 columns), poly_add_halves_kernel adds and rounds once.  Forward + backward, 16 over 128 columns,
-    // normalised, quadratic -> this: B H 16, N 4096 415 -> 120 us, B H 2, N 16384 1546 -> 95, B H 64, N 4096 1014 -> 402 (a v of 64
-    // columns there: 200; both halves form every feature).
+    // theirs in fp32 to dq_part / dk_part [BH][N][16] (32 over 16 columns), poly_add_halves_kernel adds and rounds once.  So are the scores'
+    // gradients below them, which a half keeps as two bf16 numbers (rounded to one, as the quadratic kernels round the whole, dq and dk were 0.97 to 1.07 of those
+    // kernels' errors with few rows, single heads up to 1.2; this way 0.70 to 0.72 up to 128 rows, 0.80 to 0.99 beyond, for 2 to 4 % of a pair's time).  Forward +
+    // backward, 16 over 128 columns, normalised, quadratic -> this: B H 16, N 4096 415 -> 126 us, B H 2, N 16384 1546 -> 100, B H 64, N 4096
+    // 1014 -> 417 (a v of 64 columns there: 192; both halves form every feature).
     int32_t vhalf;
     float *dq_part, *dk_part;
     // Rows of 17 to 32 columns, as two halves a and b: the features are those of a, those of b and the 256 products of a column of each, and a walk is
@@ -237,6 +239,15 @@ __device__ __forceinline__ void poly_round_masked(const float (&d)[16], uint32_t
         }
         out[t] = __builtin_bit_cast(typename Mma<T>::V8, w);
     }
+}
+
+// ... what that left of the values (the masked ones whole: to be masked again)
+template <typename T>
+__device__ __forceinline__ void poly_left_over(float (&d)[16], const typename Mma<T>::V8 (&rounded)[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) d[8 * t + j] -= static_cast<float>(rounded[t][j]);
 }
 
 // Eight fp32 numbers as sums of two bf16 ones each: the upper half of the bits, and what is left, rounded (EXACT: of a
@@ -562,6 +573,8 @@ template <int PART>
 struct PolyPartOf {
     static constexpr bool PARTS = PART >= kPolyFirst && PART <= kPolyCross, HALVES = PART != kPolyWhole;
     static constexpr bool CROSS = PART == kPolyCross, TWO = PART == kPolyFirst || CROSS, SCORES = !PARTS || PART == kPolyFirst;
+    // over half of v's columns (vhalf) a score's gradient is a partial sum: it is kept as two bf16 numbers
+    static constexpr bool TWO_TERMS = PART == kPolyHalves || PART == kPolyFirst;
     static constexpr bool ADDS = PART == kPolyFirst || PART == kPolySecond;  // to what the parts before it left
     static constexpr int F = CROSS ? PolyFeatures::kCross : PolyFeatures::kF, kOff = PART == kPolySecond ? 16 : 0;
     static constexpr int kRoom = PARTS ? F * 65 : PolyFeatures::kStateRoom;  // floats per segment of a state buffer
@@ -1250,6 +1263,13 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dq_kernel(const PolyWalkPara
                 poly_round_masked<T, false>(d, all, l32, g, df);
 #pragma unroll
                 for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(kb, rc, 32 * sb + 16 * t, g), df[t], dx);
+                if constexpr (P::TWO_TERMS)
+                    if (p.vhalf) {
+                        poly_left_over<T>(d, df);
+                        poly_round_masked<T, false>(d, all, l32, g, df);
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(kb, rc, 32 * sb + 16 * t, g), df[t], dx);
+                    }
             }
         }
         float f[16];  // (lanes of g = 0 hold the block's columns 0 .. 15)
@@ -1461,6 +1481,13 @@ __global__ __launch_bounds__(512, 2) void poly_walk_dkdv_kernel(const PolyWalkPa
                     for (int e = 0; e < 2; ++e)
                         acc[e] = M::mma(poly_tr<T>(tg + 128 * (32 * sb + 16 * t), ga, e << 6), pf[t], acc[e]);
                 }
+                if constexpr (P::TWO_TERMS)
+                    if (p.vhalf) {
+                        poly_left_over<T>(d, df);
+                        poly_round_masked<T, true>(d, all, l32, g, df);
+#pragma unroll
+                        for (int t = 0; t < 2; ++t) dx = M::mma(poly_col_frag<T>(qb, rc, 32 * sb + 16 * t, g), df[t], dx);
+                    }
             }
             if constexpr (PART == kPolyFirst) poly_get_sums(acck_at, row < N, had_k);  // (earlier: 16 registers spilled)
             float f[16];
