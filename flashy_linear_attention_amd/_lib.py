@@ -74,6 +74,7 @@ SIGNATURES = {
     "fla_normalised_forward_prefers_chunked": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int),
     "fla_normalised_prefers_chunked": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int),
     "fla_poly_attn_prefers_chunked": ([_i64] * 5 + [ctypes.c_int] * 2, ctypes.c_int),
+    "fla_poly_attn_operator_prefers_chunked": ([_i64] * 5 + [ctypes.c_int] * 3, ctypes.c_int),
     "fla_poly_attn_chunked_state_bytes": ([_i64] * 5, ctypes.c_int64),
     "fla_poly_attn_chunked_workspace_bytes": ([_i64] * 5, ctypes.c_int64),
     "fla_poly_attn_chunked_fwd_workspace_bytes": ([_i64] * 5, ctypes.c_int64),

@@ -2289,6 +2289,36 @@ int operators_prefer_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk, int6
     return prefers_chunked(B, H, N, D_qk, D_v, backward);
 }
 
+// Quadratic time over chunk-wise time of the polynomial map.  R 8 and 16, with and without the normaliser, B H 1 ... 1024, N 100 ... 4096.  Pairs,
+// D_v 64: 1.0 to 4.8 (0.91 to 0.99 at a few N of 200).  D_v 32, up to 256 heads: 0.94 to 4.2 (0.88 at B H 128, N 512); 512
+// and 1024 heads: N 128 1.07 to 1.6, N 200 to 512 0.59 to 1.06, N 1024 0.85 to 1.18, N 2048 1.34 to 1.7.  Forward
+// alone: N 4096 1.07 to 2.6; N 2048 1.1 to 1.5 with at most four heads, 0.62 to 1.09 with more; below 0.36 to 1.0.
+// D_v above 64, two halves.  Pairs, one chunk (N up to 128): 0.95 to 1.15 (normalised 1.0 to 1.36 at 128), N 64 with 800 and 1024 heads 0.83
+// to 0.93.  Beyond, 120 and 128 columns, plain and normalised at 120: N 160 to 512 0.60 to 1.08, N 700 0.92 to 1.2, N 1000 0.97 to 1.5, N 2048 1.0 to 2.4,
+// 4096 1.8 to 5.5; normalised at 128: N 160 and 200 0.97 to 1.09 up to 128 heads and 0.75 to 1.02 above, N 256 0.92 to 1.18, N 384 0.99 to 1.32, N 700 1.15 to
+// 1.4.  72 and 104 columns, whose second half is half padding or more: up to 33 heads N 512 0.96 to 1.02, N 700 0.95 to 1.21, N 1000 1.2 to 1.5; 48 heads
+// N 1000 to 2048 0.91 to 1.09, 4096 1.7 to 2.1; more heads N 2048 1.04 to 1.6.  Forward alone: up to 16 heads 1.3 to 2.2 from N 1024 on, 4096 1.5 to 4.
+// R above 16, three launches a walk, 24 and 32 columns over 32 to 128: pairs at N 8192 with 16 heads and more 1.02 to 1.7 (72 columns normalised 0.92 to
+// 1.02; N 9216 1.24 to 1.9), with up to 8 1.35 to 4, N 4096 up to 8 heads 1.08 to 2.4, N 16384 1.7 to 6; forward alone N 16384 1.2 to 2.9, N 8192 up to 4 heads 0.94 to 1.9 (32
+// columns of v 0.88 and 0.95 with 4 heads, 1.12 to 1.4 with up to 2).
+bool poly_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, bool backward, bool normalised) {
+    if (dtype != FLA_DTYPE_BF16 || !poly_plan(B, H, N, R, D_v).ok) return false;
+    const int64_t heads = B * H;
+    if (R > 16) {
+        if (!backward) return N >= 16384 || (N >= 8192 && heads <= (D_v > 32 ? 4 : 2));
+        return N >= (heads <= 8 ? 4096 : D_v > 64 && D_v <= 96 ? 9216 : 8192);
+    }
+    if (D_v > 64) {
+        if (!backward) return N >= 4096 || (N >= 1024 && heads <= 16);
+        if (N <= 128) return (D_v > 112 || heads <= 48) && (N > 64 || heads <= 512);
+        if (D_v > 120 && normalised) return N >= 256 || heads <= 128;
+        if (D_v > 112 || heads <= 33) return N >= 768;
+        return N >= (heads <= 48 ? 3072 : 2048);
+    }
+    if (backward) return D_v > 32 || heads <= 256 || N <= 128 || N >= 2048;
+    return N >= 4096 || (N >= 2048 && heads <= 4);
+}
+
 }  // namespace
 
 extern "C" {
@@ -2704,25 +2734,10 @@ int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk
     return N >= (wp.D <= 32 ? 4096 : 3072) || w >= 6e9 || (one && w >= 2e9);
 }
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward) {
-    if (dtype != FLA_DTYPE_BF16 || !poly_plan(B, H, N, R, D_v).ok) return 0;
-    // Quadratic time over chunk-wise time, R 8 and 16, with and without the normaliser, B H 1 ... 1024, N 100 ... 4096.  Pairs,
-    // D_v 64: 1.0 to 4.8 (0.91 to 0.99 at a few N of 200).  D_v 32, up to 256 heads: 0.94 to 4.2 (0.88 at B H 128, N 512); 512
-    // and 1024 heads: N 128 1.07 to 1.6, N 200 to 512 0.59 to 1.06, N 1024 0.85 to 1.18, N 2048 1.34 to 1.7.  Forward
-    // alone: N 4096 1.07 to 2.6; N 2048 1.1 to 1.5 with at most four heads, 0.62 to 1.09 with more; below 0.36 to 1.0.
-    // D_v above 64, two halves, 72 to 128 columns, B H 1 ... 1024: pairs at 128 1.05 to 16 (B H 2, N 4096 389 / 58 us, B H 16, N 8192
-    // 870 / 206, B H 64, N 4096 1014 / 402, B H 512, N 256 178 / 166); at 72 to 104, whose second half is half padding or more, up to 33
-    // heads 1.1 to 12, above 0.8 to 1.2 below N 2048 and 1.1 to 1.8 from there on.  Forward alone: up to 16 heads 1.2 to 9 from
-    // N 1024 on, above 0.5 to 1.2 up to N 2048, 1.4 to 1.5 at 4096.
-    // R above 16, three launches a walk, 24 and 32 columns over 32 to 128, B H 1 ... 300: pairs at N 8192 1.15 to 3.2, at 4096 0.74 to 1.0 with 16 heads and
-    // more, 1.3 to 2.1 with up to 8 (N 16384 2.4 to 4.9: B H 2 1062 / 258 us, B H 16 2154 / 747); forward alone, 16384 1.4 to 2.7, 8192 0.65 to 0.95, with up to 2 1.1 to 1.55.
-    if (R > 16) return backward ? N >= 8192 || (N >= 4096 && B * H <= 8) : N >= 16384 || (N >= 8192 && B * H <= 4);
-    if (D_v > 64) {
-        if (backward) return D_v > 112 || B * H <= 48 || N >= 2048;
-        return N >= 4096 || (N >= 1024 && B * H <= 16);
-    }
-    const bool few = B * H <= 256;
-    if (backward) return D_v > 32 || few || N <= 128 || N >= 2048;
-    return N >= 4096 || (N >= 2048 && B * H <= 4);
+    return poly_prefers_chunked(B, H, N, R, D_v, dtype, backward != 0, false);
+}
+int fla_poly_attn_operator_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward, int normalised) {
+    return poly_prefers_chunked(B, H, N, R, D_v, dtype, backward != 0, normalised != 0);
 }
 
 int64_t fla_poly_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v) {

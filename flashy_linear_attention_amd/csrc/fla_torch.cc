@@ -416,7 +416,7 @@ PolyResult poly_fwd(const Tensor &q_, const Tensor &k_, const Tensor &v_, const 
     r.o = c.rows(c.dv);
     if (p.normalise) r.denom = c.row_floats();
     float *n = static_cast<float *>(ptr(r.denom));
-    if (fla_poly_attn_prefers_chunked(c.b, c.h, c.n, c.dqk, c.dv, c.dtype, want_state)) {
+    if (fla_poly_attn_operator_prefers_chunked(c.b, c.h, c.n, c.dqk, c.dv, c.dtype, want_state, p.normalise)) {
         if (want_state) r.state = c.bytes(fla_poly_attn_chunked_state_bytes(c.b, c.h, c.n, c.dqk, c.dv));
         const Tensor work = c.bytes(fla_poly_attn_chunked_fwd_workspace_bytes(c.b, c.h, c.n, c.dqk, c.dv));
         must(fla_poly_attn_chunked_fwd(ptr(q), ptr(k), ptr(v), ptr(r.o), n, c.b, c.h, c.n, c.dqk, c.dv, str(q), str(k), str(v),

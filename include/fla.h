@@ -426,13 +426,15 @@ int fla_normalised_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t D_qk
  * feature-wide in memory but the states at segment ends).  FLA_DTYPE_BF16 only
  * (FLA_ERR_UNSUPPORTED otherwise, as for operands that are not 16-byte aligned).  fla_poly_attn_prefers_chunked(): 1 where
  * it is the faster evaluation (of a forward + backward pair, or with backward == 0 of forward alone; host arithmetic,
- * measured thresholds), 0 elsewhere and where it does not exist.
+ * measured thresholds), 0 elsewhere and where it does not exist; fla_poly_attn_operator_prefers_chunked(), which the operator goes by, answers
+ * for the normalised call apart (the one above holds for either).
  * `workspace`: fla_poly_attn_chunked_workspace_bytes() bytes, of which the forward call needs fla_poly_attn_chunked_fwd_workspace_bytes()
  * (R > 16: sums go on in fp32 from launch to launch, per row and half of v 260 bytes in forward and 512 in backward; D_v > 64, backward:
  * 128 bytes per row and half, 256 with R > 16, for the halves' dXq and dXk); `state_out` / `state_in`:
  * fla_poly_attn_chunked_state_bytes() bytes (58 KiB per segment, 146 for R > 16, and per half of a v of more than 64 columns; a single segment per (b, h) needs none: 16),
  * written by forward (NULL: no backward will follow) and read by backward; both 16-byte aligned. */
 int fla_poly_attn_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward);
+int fla_poly_attn_operator_prefers_chunked(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v, int dtype, int backward, int normalised);
 int64_t fla_poly_attn_chunked_state_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v);
 int64_t fla_poly_attn_chunked_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v);
 int64_t fla_poly_attn_chunked_fwd_workspace_bytes(int64_t B, int64_t H, int64_t N, int64_t R, int64_t D_v);

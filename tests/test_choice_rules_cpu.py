@@ -102,3 +102,22 @@ def test_up_to_256_rows(dqk, dv, bh, n, pair, forward):
         assert _lib.query(name, 1, bh, n, dqk, dv) == want
     for backward, want in ((1, pair), (0, forward)):
         assert _lib.query("fla_linear_attn_operator_prefers_chunked", 1, bh, n, dqk, dv, backward) == want
+
+
+# (pairs over two halves of v: one chunk, the lines beyond it, the normalised call over a full second half; above 16 columns of q and k)
+@pytest.mark.parametrize("bh,n,r,dv,plain,normalised", [
+    (512, 64, 16, 128, 1, 1), (513, 64, 16, 128, 0, 0), (1024, 128, 8, 120, 1, 1), (49, 128, 16, 72, 0, 0),
+    (1, 129, 16, 128, 0, 1), (128, 255, 16, 128, 0, 1), (129, 255, 16, 128, 0, 0), (129, 256, 8, 128, 0, 1),
+    (300, 767, 16, 120, 0, 0), (300, 768, 16, 120, 1, 1), (33, 767, 16, 72, 0, 0), (33, 768, 8, 104, 1, 1), (48, 3071, 16, 96, 0, 0),
+    (48, 3072, 16, 96, 1, 1), (9, 8192, 32, 72, 0, 0), (9, 9216, 24, 96, 1, 1), (9, 8192, 32, 104, 1, 1), (8, 4096, 24, 72, 1, 1),
+])
+def test_polynomial_pairs_over_two_halves(bh, n, r, dv, plain, normalised):
+    for flag, want in ((0, plain), (1, normalised)):
+        assert _lib.query("fla_poly_attn_operator_prefers_chunked", 1, bh, n, r, dv, 0, 1, flag) == want
+    assert _lib.query("fla_poly_attn_prefers_chunked", 1, bh, n, r, dv, 0, 1) == plain
+    assert _lib.query("fla_poly_attn_operator_prefers_chunked", 1, bh, n, r, dv, 1, 1, 1) == 0  # fp16
+
+
+@pytest.mark.parametrize("bh,dv,want", [(2, 32, 1), (3, 32, 0), (4, 40, 1), (5, 40, 0)])
+def test_polynomial_forward_above_sixteen_columns(bh, dv, want):
+    assert _lib.query("fla_poly_attn_operator_prefers_chunked", 1, bh, 8192, 24, dv, 0, 0, 1) == want
