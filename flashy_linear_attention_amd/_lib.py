@@ -56,6 +56,7 @@ SIGNATURES = {
     "fla_linear_attn_chunked_fwd_static": ([_ptr] * 4 + [_i64] * 5 + [_strides] * 4 + [ctypes.c_int, _ptr], ctypes.c_int),
     "fla_linear_attn_f16_pair_prefers_chunked": ([_i64] * 5, ctypes.c_int),
     "fla_linear_attn_prefers_copies": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int),
+    "fla_linear_attn_operator_prefers_copies": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int),
     "fla_linear_attn_copies_bytes": ([_i64] * 5 + [ctypes.c_int], ctypes.c_int64),
     "fla_linear_attn_copies_fwd": ([_ptr] * 4 + [_i64] * 5 + [_strides] * 4 + [ctypes.c_int, _ptr, _i64, _ptr], ctypes.c_int),
     "fla_linear_attn_copies_bwd": ([_ptr] * 7 + [_i64] * 5 + [_strides] * 7 + [ctypes.c_int, _ptr, _i64, _ptr], ctypes.c_int),

@@ -68,7 +68,7 @@ def rounded_once(q: torch.Tensor, v: torch.Tensor) -> bool:
 def _copies_bytes(q: torch.Tensor, v: torch.Tensor, backward: int) -> int:
     """Workspace of the quadratic evaluation on copies with aligned rows (widths that are no multiples of 8), 0 where it is not taken."""
     shape = (*q.shape, v.shape[-1], backward)
-    if not _lib.query("fla_linear_attn_prefers_copies", *shape):
+    if not _lib.query("fla_linear_attn_operator_prefers_copies", *shape):
         return 0
     return _lib.query("fla_linear_attn_copies_bytes", *shape)
 

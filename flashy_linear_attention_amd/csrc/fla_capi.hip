@@ -2430,6 +2430,17 @@ int fla_linear_attn_prefers_copies(int64_t B, int64_t H, int64_t N, int64_t D_qk
     return widest > 64 || N >= (widest > 32 ? 512 : 1024);
 }
 
+// Through the operators the host weighs in, which the two copy launches keep for 4 us of the 65 to 80 of a pair.  fp16 pairs, B H 1 ... 300,
+// bounds-checked time over the copies': 20 columns N 256 0.95 to 1.01, 512 1.19 to 1.34; 36 and 60 N 64 0.92 to 0.96, 128 0.91 to 1.05, 256 1.29 to 1.5; 100 and
+// 153 / 64 N 64 0.90 to 0.95 and with 300 heads 1.6 to 1.8, 128 1.24 to 2.1; 250 N 64 2.2 to 3.4.  Forward alone, 91 / 64, N 64 1.24 to 1.38 up to 128 heads, 0.90
+// with 300.
+int fla_linear_attn_operator_prefers_copies(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int backward) {
+    if (!fla_linear_attn_prefers_copies(B, H, N, D_qk, D_v, backward)) return 0;
+    const int64_t heads = B * H, widest = D_qk > D_v ? D_qk : D_v;
+    if (!backward) return N > 64 || D_v > 64 || D_qk > 128 || heads <= 128;
+    return N >= (widest <= 32 ? 512 : widest <= 64 ? 256 : 128) || (D_qk > 128 && D_v > 128) || (widest > 64 && heads > 256);
+}
+
 int fla_linear_attn_copies_fwd(const void *q, const void *k, const void *v, void *o, int64_t B, int64_t H, int64_t N, int64_t D_qk,
                                int64_t D_v, const int64_t *q_strides, const int64_t *k_strides, const int64_t *v_strides,
                                const int64_t *o_strides, int dtype, void *workspace, int64_t workspace_bytes, void *stream) {

@@ -62,7 +62,7 @@ struct Call {
     // (a quadratic product of widths off the eights: the workspace of fla_linear_attn_copies_fwd / _bwd, 0 where those are not taken)
     int64_t copies(bool backward) const {
         if (dqk % 8 == 0 && dv % 8 == 0) return 0;
-        return fla_linear_attn_prefers_copies(b, h, n, dqk, dv, backward) ? fla_linear_attn_copies_bytes(b, h, n, dqk, dv, backward) : 0;
+        return fla_linear_attn_operator_prefers_copies(b, h, n, dqk, dv, backward) ? fla_linear_attn_copies_bytes(b, h, n, dqk, dv, backward) : 0;
     }
     Tensor bytes(int64_t count) const { return count ? at::empty({count}, like.dtype(at::kByte)) : Tensor(); }
 };

@@ -136,8 +136,10 @@ int fla_linear_attn_smallv_bwd(const void *grad_out, const void *q, const void *
 /* fla_linear_attn_fwd / _bwd and the small-V pair for widths that are no multiples of 8 (one of D_qk, D_v at least;
  * FLA_ERR_UNSUPPORTED otherwise), on copies with 16-byte aligned rows in `workspace` (fla_linear_attn_copies_bytes() bytes, 16-byte
  * aligned; 0: multiples of 8): the fast kernels in place of the bounds-checked one.  fla_linear_attn_prefers_copies(): 1 where that is the
- * faster way (host arithmetic, measured thresholds). */
+ * faster way by the kernels' time, fla_linear_attn_operator_prefers_copies(): for the operators of the Python package, whose host waits for the
+ * launches of short calls (host arithmetic, measured thresholds). */
 int fla_linear_attn_prefers_copies(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int backward);
+int fla_linear_attn_operator_prefers_copies(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int backward);
 int64_t fla_linear_attn_copies_bytes(int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v, int backward);
 int fla_linear_attn_copies_fwd(const void *q, const void *k, const void *v, void *o,
                                int64_t B, int64_t H, int64_t N, int64_t D_qk, int64_t D_v,

@@ -121,3 +121,13 @@ def test_polynomial_pairs_over_two_halves(bh, n, r, dv, plain, normalised):
 @pytest.mark.parametrize("bh,dv,want", [(2, 32, 1), (3, 32, 0), (4, 40, 1), (5, 40, 0)])
 def test_polynomial_forward_above_sixteen_columns(bh, dv, want):
     assert _lib.query("fla_poly_attn_operator_prefers_chunked", 1, bh, 8192, 24, dv, 0, 0, 1) == want
+
+
+@pytest.mark.parametrize("bh,n,dqk,dv,forward,backward", [
+    (4, 511, 20, 20, 0, 0), (4, 512, 20, 20, 0, 1), (300, 255, 36, 60, 0, 0), (1, 256, 36, 36, 0, 1), (256, 127, 100, 100, 1, 0),
+    (257, 64, 100, 100, 1, 1), (1, 128, 153, 64, 1, 1), (4, 64, 153, 64, 1, 0), (1, 64, 250, 250, 1, 1), (128, 64, 91, 64, 1, 0),
+    (129, 64, 91, 64, 0, 0), (129, 128, 91, 64, 1, 1), (4, 4096, 64, 64, 0, 0),
+])
+def test_copies_through_the_operators(bh, n, dqk, dv, forward, backward):
+    for back, want in ((0, forward), (1, backward)):
+        assert _lib.query("fla_linear_attn_operator_prefers_copies", 1, bh, n, dqk, dv, back) == want
