@@ -27,7 +27,8 @@
  *     reference computes in bf16 only, flashlinear/kernels/linear_attn_kernels.py:82,98).
  *   - Infinite and NaN operands: a forward result that depends on one is infinite or NaN, the others
  *     are what they would be without it.  An element of v reaches its own column, from its row on
- *     and in the rows before it of the same 32 (a masked score is multiplied by it too).  Whether
+ *     and in the rows before it of the same 32 (a masked score is multiplied by it too; of the same
+ *     128 or 256 where rows that are not 16-byte aligned run on the bounds-checked kernel).  Whether
  *     +inf, -inf or NaN comes out goes by the evaluation: with q and k of either sign one infinite
  *     v_j leaves a column of the chunk-wise running state with both infinities, and the rows of
  *     later chunks are NaN in that column, where the quadratic kernels give +inf or -inf by the
