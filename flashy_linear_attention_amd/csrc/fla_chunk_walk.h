@@ -1587,6 +1587,8 @@ __device__ __forceinline__ void walk_wide_body(const WalkParams &p) {
             walk_sum_states<D, B2, false>(init2 + at, f_lo, f_hi, wave, lane, st1);
         }
         if constexpr (REV) {
+            // (dK's totals are [q/k][v] too: a second half of v that is narrow is so in their columns, and in rows once they are turned.  One
+            // map of blocks to waves for both, as B2 would be, leaves rows unsummed and turns what the LDS held there)
             static_assert(NV == 4 && N2 == 4, "whole states are turned");
             if (dk) {
                 float *const turn = reinterpret_cast<float *>(smem);
@@ -1702,7 +1704,9 @@ __global__ __launch_bounds__(256, 1) void walk_rev_wide_kernel(const WalkParams 
 // it -- one late row that is infinite, NaN or merely huge spoiled the dQ of every chunk before it.  Forward + backward
 // at B H 16, N 32768, D 64 that way 222 us, this way 234 at the time, 222 with totals added up by fragments.)
 // fp16, plain: R's copy is scaled, as forward's (walk_state_scale); the waves exchange their largest elements through a tile that has been
-// multiplied, between two barriers more per chunk -- tiles and states fill half of a CU's LDS.
+// multiplied, between two barriers more per chunk -- tiles and states fill half of a CU's LDS.  fp16 calls that took this walk unscaled before
+// (LinearAttentionChunked, feature maps) pay 2 to 3 % at 64 columns: B H 64, N 4000 100 -> 102 us, with a feature map 119 -> 122; 32 columns and those
+// of walk_dkdv_kernel 0 to 1 %.
 template <typename T, int D, bool NORM, bool WIDE = false, bool GN = false>
 __global__ __launch_bounds__(256, 2) void walk_bwd_kernel(const WalkParams p) {
 #if defined(__HIP_DEVICE_COMPILE__)
@@ -2395,7 +2399,8 @@ template <typename T, int D, int NQ, int NV, bool BOTH, bool PAIRS = false>
 __device__ __forceinline__ void walk_totals_body(const WalkTotalsParams &p) {
     using W = WalkCfg<D>;
     static_assert(!BOTH || D == 128, "halves of 128 columns");
-    // (the halves of Z and of Y: walk_totals_quad_kernel, walk_totals_pairs_kernel)
+    // (the halves of Z and of Y: walk_totals_quad_kernel, walk_totals_pairs_kernel -- grid y there is 2 (half of Y) + half of Z; elsewhere & ~0, no
+    // instruction)
     const int zh = (BOTH || PAIRS) && p.dz2 ? (int)blockIdx.y & (PAIRS ? 1 : ~0) : 0, dz = zh ? p.dz2 : p.dz;
     const bool yh = PAIRS && blockIdx.y >= 2;
     extern __shared__ __attribute__((aligned(16))) unsigned char smem[];
